@@ -113,63 +113,82 @@ inline unsigned grid_for(int64_t n_threads, int block, int64_t cap) {
 
 struct FwdPlan {
   int vec;
-  int ntiles;
-  int64_t n_items;
+  int lpr;  // lanes per row piece
+  int64_t n_row_blocks;
+  int64_t n_items;   // (tile, row block)
+  int64_t xcd_span;  // items per XCD, or 0: items in order
+  unsigned grid;
 };
 
 FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target, const void *bias,
                  const float *resid) {
   const size_t es = dtype_size(s->weight_dtype);
-  int vec = pick_vec(s->D, es, weight, 4);  // 256-column tiles measured faster than 512
+  int vec = pick_vec(s->D, es, weight, 8);
   // resid is stored with fp32 vectors of the same width, target/bias are read with the
   // weight's vector type when they share its dtype
   if (s->target_dtype == s->weight_dtype && !aligned(target, vec * es)) vec = 1;
   if (s->bias_dtype == s->weight_dtype && !aligned(bias, vec * es)) vec = 1;
-  if (!aligned(resid, vec * 4)) vec = 1;
-  // a tile of 64*vec columns that is mostly padding wastes lanes: narrow it for small D
-  while (vec > 1 && s->D < static_cast<int64_t>(kWave) * vec && s->D % (vec / 2) == 0) vec >>= 1;
+  if (!aligned(resid, 16)) vec = 1;
   FwdPlan p;
   p.vec = vec;
-  p.ntiles = static_cast<int>(ceil_div(s->D, static_cast<int64_t>(kWave) * vec));
-  p.n_items = s->B * p.ntiles;
+  // Bytes of a row piece, and whether every L2 works on a tile of its own.  Measured (us; uniform / skewed
+  // indices; B=4096, K=64, D=2304 bf16):
+  //   F            128 B per L2    256 B per L2    512 B, all L2s on one tile
+  //   16384          68 / 62         72 / 59         135 / 63
+  //   32768          93 / 64        114 / 61         152 / 66
+  //   49152         124 / 66        133 / 62         166 / 69
+  //   65536         139 / 72        145 / 67         162 / 72
+  //   131072        168 / 87        161 / 82         167 / 83
+  //   196608        175 / 93        179 / 87         173 / 87
+  // (from 65536 on the narrow pieces gain less on uniform indices than they lose on skewed ones) and fp32
+  // (B=2048, K=64, D=1024): 256 B beats 128 B from 32768 rows on (65536: 65 / 31 against 73 / 32, 131072:
+  // 73 / 32 against 83 / 34; 512 B 78 / 37) and equals it below.  Eight-byte lanes gain 5 % on uniform
+  // indices around 65536 rows and lose 25 % on skewed ones: 16 bytes per lane wherever rows allow it.
+  const bool by_xcd = s->F <= 131072;
+  const size_t piece_bytes = !by_xcd ? 512 : (es == 2 && s->F <= 49152) ? 128 : 256;
+  p.lpr = static_cast<int>(piece_bytes / (static_cast<size_t>(vec) * es));
+  if (p.lpr > kWave) p.lpr = kWave;
+  const int64_t rows = (kWave / p.lpr) * static_cast<int64_t>(kWavesPerBlock);
+  p.n_row_blocks = ceil_div(s->B, rows);
+  p.n_items = ceil_div(s->D, static_cast<int64_t>(p.lpr) * vec) * p.n_row_blocks;
+  p.xcd_span = by_xcd ? ceil_div(p.n_items, 8) : 0;
+  p.grid = static_cast<unsigned>(by_xcd ? p.xcd_span * 8 : p.n_items);
   return p;
 }
 
-template <typename WT, int VEC, bool HIER>
-void launch_fwd_t(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices,
-                  const void *weight, const void *vals, const void *bias, const void *target,
-                  float *resid, float *partial, int *status_flag, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>(ceil_div(p.n_items, kWavesPerBlock));
-  hipLaunchKernelGGL((sae_fwd_kernel<WT, VEC, HIER, FLEXSAE_FWD_U>), dim3(grid), dim3(kBlock), 0, st, indices,
-                     weight, vals, s->vals_dtype, bias, s->bias_dtype, target, s->target_dtype,
-                     resid, partial, status_flag, p.n_items, p.ntiles, static_cast<int>(s->K),
-                     s->F, static_cast<int>(s->D));
-}
-
 template <typename WT, bool HIER>
-void launch_fwd_v(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices,
-                  const void *weight, const void *vals, const void *bias, const void *target,
-                  float *resid, float *partial, int *status_flag, hipStream_t st) {
-  switch (p.vec) {
-    case 8:
-      if constexpr (sizeof(typename Traits<WT>::store_t) == 2) {
-        launch_fwd_t<WT, 8, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                  status_flag, st);
-        break;
-      }
-      [[fallthrough]];
-    case 4:
-      launch_fwd_t<WT, 4, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                status_flag, st);
-      break;
-    case 2:
-      launch_fwd_t<WT, 2, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                status_flag, st);
-      break;
-    default:
-      launch_fwd_t<WT, 1, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                status_flag, st);
+void launch_fwd(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices,
+                const void *weight, const void *vals, const void *bias, const void *target,
+                float *resid, float *partial, int *status_flag, hipStream_t st) {
+#define FLEXSAE_LAUNCH_FWD(VEC, LPR)                                                                       \
+  hipLaunchKernelGGL((sae_fwd_kernel<WT, VEC, LPR, HIER, FLEXSAE_FWD_U>), dim3(p.grid), dim3(kBlock), 0, st, \
+                     indices, weight, vals, s->vals_dtype, bias, s->bias_dtype, target, s->target_dtype,   \
+                     resid, partial, status_flag, s->B, p.n_row_blocks, p.n_items, p.xcd_span,             \
+                     static_cast<int>(s->K), s->F, static_cast<int>(s->D))
+  constexpr int E = static_cast<int>(sizeof(typename Traits<WT>::store_t));
+  constexpr int V16 = 16 / E, V8 = 8 / E, V4 = 4 / E;  // columns per lane
+  constexpr bool kNarrow = E == 2;  // 128-byte pieces: 16-bit weights only
+#define FLEXSAE_LAUNCH_FWD_V(VEC, LPR128, LPR256, LPR512)  \
+  do {                                                     \
+    if (kNarrow && p.lpr == LPR128) {                      \
+      FLEXSAE_LAUNCH_FWD(VEC, (kNarrow ? LPR128 : LPR256)); \
+    } else if (p.lpr == LPR256) {                          \
+      FLEXSAE_LAUNCH_FWD(VEC, LPR256);                     \
+    } else {                                               \
+      FLEXSAE_LAUNCH_FWD(VEC, LPR512);                     \
+    }                                                      \
+  } while (0)
+  if (p.vec == V16) {
+    FLEXSAE_LAUNCH_FWD_V(V16, 8, 16, 32);
+  } else if (p.vec == V8) {
+    FLEXSAE_LAUNCH_FWD_V(V8, 16, 32, 64);
+  } else if (p.vec == V4) {
+    FLEXSAE_LAUNCH_FWD_V(V4, 32, 64, 64);
+  } else if constexpr (kNarrow) {
+    FLEXSAE_LAUNCH_FWD_V(1, 64, 64, 64);
   }
+#undef FLEXSAE_LAUNCH_FWD_V
+#undef FLEXSAE_LAUNCH_FWD
 }
 
 template <bool HIER>
@@ -191,15 +210,15 @@ int forward(const flexsae_shape *s, const int64_t *indices, const void *weight, 
   float *partial = static_cast<float *>(workspace);
   switch (s->weight_dtype) {
     case FLEXSAE_F32:
-      launch_fwd_v<float, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+      launch_fwd<float, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
                                 status_flag, st);
       break;
     case FLEXSAE_BF16:
-      launch_fwd_v<bf16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+      launch_fwd<bf16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
                                  status_flag, st);
       break;
     default:
-      launch_fwd_v<f16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+      launch_fwd<f16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
                                 status_flag, st);
   }
   rc = launch_status();

@@ -7,91 +7,160 @@
 
 namespace flexsae {
 
-// Work decomposition: one wavefront per (row b, D-tile) item.  A tile is 64*VEC
-// consecutive columns, lane l owning columns [l*VEC, (l+1)*VEC) of the tile, so one
-// gathered row piece is a single vector load per lane and 64*VEC*sizeof(W) contiguous
-// bytes per wavefront.  The row's indices/vals are fetched 64 at a time with one
-// coalesced load (lane j holds step k0+j) and handed out with v_readlane, which puts
-// the row number in a scalar register: the gather address is scalar-base + lane offset.
-// U independent gathers are issued before the first one is consumed.
+// Work decomposition: a block of four wavefronts walks 4 * R rows of one narrow column tile.  LPR lanes
+// serve a row piece of LPR * VEC columns, so a wavefront has R = 64 / LPR rows and one vector load
+// fetches R row pieces.  Every step's row number and val are read from the LDS, where the
+// wavefront has put those of kFwdChunk steps of its R rows with coalesced loads (a broadcast read:
+// all lanes of a piece read the same entry).  U independent gathers are issued before the first one
+// is consumed.
 //
-// Per item the wavefront writes resid[b, tile] = r_{b,K-1} - target_b (fp32) and one
-// fp32 partial sum of squares into partial[item]; loss_finalize_kernel adds the
-// partials in a fixed order, so the loss is bit-reproducible from run to run.
-template <typename WT, int VEC, bool HIER, int U>
+// What bounds it: the gathered bytes.  The weight matrix is read once per pair, and how fast depends on
+// which cache answers.  Two orders of the (tile, row block) items, picked by plan_fwd:
+//   xcd_span > 0   the items, tiles outermost, are cut into eight equal runs, one per L2 (blocks
+//                  go round the eight XCDs): an L2 sees F pieces of one narrow tile at a time instead of
+//                  whole rows.  65536 pieces of 128 bytes are 8.4 MB against 4 MB of L2: about half of the
+//                  gathers hit.  128 bytes is the L2's line; 64-byte pieces fetch the whole line anyway
+//                  (twice as slow).
+//   xcd_span == 0  items in order, tiles outermost, wide tiles: all XCDs gather from the same column
+//                  tile, which the memory-side cache (256 MB) holds where the L2s cannot help.
+// Against one wavefront per (row, 256 columns) in row order, which no cache but the memory-side one served:
+// B=4096, K=128, F=65536, D=2304 bf16 (2.42 GB gathered) 328 -> 275 us (8.8 TB/s), K=64 172 -> 143 us; B=2048,
+// K=256, F=131072, D=1024 fp32 292 -> 273 us; B=16384, K=128, F=524288, D=8192 bf16 6.3 -> 4.8 ms (7.2 TB/s).
+// Where the L2s serve nearly all of it (skewed indices, few latents) it runs at their 18 TB/s.  Streaming hints
+// on the index loads cost 5-10 % (the eight XCDs share those lines in the memory-side cache); 32-bit
+// offsets through a buffer descriptor change nothing.
+//
+// Per item the block writes resid[b, tile] = r_{b,K-1} - target_b (fp32) and one fp32 partial sum of
+// squares; loss_finalize_kernel adds the partials in a fixed order, so the loss is bit-reproducible from
+// run to run.
+constexpr int kFwdChunk = 64;  // steps per LDS fill
+
+template <typename WT, int VEC, int LPR, bool HIER, int U>
 __global__ __launch_bounds__(256) void sae_fwd_kernel(
     const int64_t *__restrict__ indices, const void *__restrict__ weight,
     const void *__restrict__ vals, int vals_dtype, const void *__restrict__ bias, int bias_dtype,
     const void *__restrict__ target, int target_dtype, float *__restrict__ resid,
-    float *__restrict__ partial, int *status_flag, int64_t n_items, int ntiles, int K, int64_t F,
-    int D) {
+    float *__restrict__ partial, int *status_flag, int64_t B, int64_t n_row_blocks, int64_t n_items,
+    int64_t xcd_span, int K, int64_t F, int D) {
+  constexpr int R = kWave / LPR;  // rows per wavefront
+  constexpr int kWaves = 256 / kWave;
+  static_assert(kFwdChunk == kWave && kFwdChunk % U == 0, "one lane per step of a chunk");
+  __shared__ vec_t<uint32_t, 2> steps[kWaves][R][kFwdChunk];  // (row of the weight matrix, val bits)
+  __shared__ float wave_loss[kWaves];
   const int lane = lane_id();
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
-  if (item >= n_items) return;  // uniform per wavefront
-  const int64_t b = item / ntiles;
-  const int tile = static_cast<int>(item - b * ntiles);
-  const int d0 = tile * (kWave * VEC) + lane * VEC;
-  const bool active = d0 < D;  // D % VEC == 0 is checked on the host
-  const int dsafe = active ? d0 : 0;
+  const int wv = wave_in_block();
+  int64_t item = blockIdx.x;
+  if (xcd_span > 0) {
+    const int64_t i = item >> 3;
+    item = (item & 7) * xcd_span + i;
+    if (i >= xcd_span) return;  // uniform per block
+  }
+  if (item >= n_items) return;  // uniform per block
+  const int64_t tile = item / n_row_blocks;
+  const int64_t b0 = ((item - tile * n_row_blocks) * kWaves + wv) * R;  // first row of the wavefront
+  const int64_t b = b0 + lane / LPR;
+  const int d0 = static_cast<int>(tile) * (LPR * VEC) + (lane % LPR) * VEC;
+  const bool active = d0 < D && b < B;  // D % VEC == 0 is checked on the host
+  const int dsafe = d0 < D ? d0 : 0;
+  const int64_t bsafe = b < B ? b : B - 1;
 
-  float r[VEC], t[VEC], acc[VEC];
-  load_vec_dyn<WT, VEC>(bias, bias_dtype, dsafe, r);
-  load_vec_dyn<WT, VEC>(target, target_dtype, b * D + dsafe, t);
+  // e = reconstruction error, starting from bias - target
+  float e[VEC], acc[VEC];
+  {
+    float t[VEC];
+    load_vec_dyn<WT, VEC>(bias, bias_dtype, dsafe, e);
+    load_vec_dyn<WT, VEC>(target, target_dtype, bsafe * D + dsafe, t);
 #pragma unroll
-  for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-
-  const int64_t pair0 = b * K;
-  for (int k0 = 0; k0 < K; k0 += kWave) {
-    const int kk = k0 + lane;
-    int64_t my_idx = 0;
-    float my_val = 0.f;
-    if (kk < K) {
-      my_idx = indices[pair0 + kk];
-      my_val = load_scalar(vals, vals_dtype, pair0 + kk);
+    for (int i = 0; i < VEC; ++i) {
+      e[i] -= t[i];
+      acc[i] = 0.f;
     }
-    if (static_cast<uint64_t>(my_idx) >= static_cast<uint64_t>(F)) {
-      if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);
-      my_idx = 0;
-      my_val = 0.f;
-    }
-    const int my_row = static_cast<int>(my_idx);
-    const int n = (K - k0) < kWave ? (K - k0) : kWave;  // uniform
+  }
+  using S = typename Traits<WT>::store_t;
+  const S *__restrict__ wbase = static_cast<const S *>(weight) + dsafe;
+  const uint32_t d_elems = static_cast<uint32_t>(D);
+  const vec_t<uint32_t, 2> *my_steps = &steps[wv][lane / LPR][0];
 
-    auto consume = [&](const float(&w)[VEC], float v) {
+  auto consume = [&](const raw_vec_t<WT, VEC> &raw, float v) {
+    float w[VEC];
+    unpack_raw<WT, VEC>(raw, w);
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        r[i] = fmaf(w[i], v, r[i]);
-        if constexpr (HIER) {
-          const float diff = r[i] - t[i];
-          acc[i] = fmaf(diff, diff, acc[i]);
-        }
+    for (int i = 0; i < VEC; ++i) {
+      e[i] = fmaf(w[i], v, e[i]);
+      if constexpr (HIER) acc[i] = fmaf(e[i], e[i], acc[i]);
+    }
+  };
+  auto gather = [&](uint32_t row) {
+    return *reinterpret_cast<const raw_vec_t<WT, VEC> *>(wbase + static_cast<uint64_t>(row) * d_elems);
+  };
+
+  for (int k0 = 0; k0 < K; k0 += kFwdChunk) {
+    const int n = (K - k0) < kFwdChunk ? (K - k0) : kFwdChunk;  // uniform
+    // lane j: step k0 + j of every row of the wavefront
+    {
+      int64_t idx[R];
+      uint32_t vbits[R];
+      const int kk = k0 + (lane < n ? lane : 0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int64_t p = (b0 + r < B ? b0 + r : B - 1) * K + kk;
+        idx[r] = indices[p];
+        vbits[r] = load_scalar_bits(vals, vals_dtype, p);
       }
-    };
-
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float v = scalar_from_bits(vbits[r], vals_dtype);
+        if (static_cast<uint64_t>(idx[r]) >= static_cast<uint64_t>(F)) {
+          if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);
+          idx[r] = 0;
+          v = 0.f;
+        }
+        vec_t<uint32_t, 2> s;
+        s[0] = static_cast<uint32_t>(idx[r]);
+        s[1] = __float_as_uint(v);
+        steps[wv][r][lane] = s;
+      }
+      // (the wavefront's own LDS accesses are served in order; this keeps the compiler from moving them)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
     int j = 0;
     for (; j + U <= n; j += U) {
-      float w[U][VEC];
+      raw_vec_t<WT, VEC> raw[U];
+      float v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int64_t row = bcast_i32(my_row, j + u);
-        load_vec<WT, VEC>(weight, row * D + dsafe, w[u]);
+        const vec_t<uint32_t, 2> s = my_steps[j + u];
+        v[u] = __uint_as_float(s[1]);
+        raw[u] = gather(s[0]);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) consume(w[u], bcast_f32(my_val, j + u));
+      for (int u = 0; u < U; ++u) consume(raw[u], v[u]);
+    }
+    for (; j + 4 <= n; j += 4) {
+      raw_vec_t<WT, VEC> raw[4];
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const vec_t<uint32_t, 2> s = my_steps[j + u];
+        v[u] = __uint_as_float(s[1]);
+        raw[u] = gather(s[0]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) consume(raw[u], v[u]);
     }
     for (; j < n; ++j) {
-      float w[VEC];
-      const int64_t row = bcast_i32(my_row, j);
-      load_vec<WT, VEC>(weight, row * D + dsafe, w);
-      consume(w, bcast_f32(my_val, j));
+      const vec_t<uint32_t, 2> s = my_steps[j];
+      consume(gather(s[0]), __uint_as_float(s[1]));
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 
   float lsum = 0.f;
-  float e[VEC];
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
-    e[i] = r[i] - t[i];
     if constexpr (HIER) {
       lsum += acc[i];
     } else {
@@ -104,7 +173,14 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     lsum = 0.f;
   }
   lsum = wave_sum_lane63(lsum);
-  if (lane == kWave - 1) partial[item] = lsum;
+  if (lane == kWave - 1) wave_loss[wv] = lsum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += wave_loss[w];
+    partial[item] = s;
+  }
 }
 
 // loss[0] = inv_count * sum(partial[0..n)), one block, fixed summation order, double

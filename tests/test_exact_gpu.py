@@ -196,3 +196,31 @@ def test_rows_beyond_four_gib_are_addressed_exactly():
     assert rc == 0, _lib.status_string(rc)
     assert torch.equal(dv.double().cpu(), dv_x)
     assert torch.equal(db.double().cpu(), db_x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 1, 49152, 8), (33, 65, 49152, 72), (34, 7, 49153, 136), (63, 130, 131072, 68),
+                                   (17, 63, 131073, 264), (9, 64, 131073, 520), (66, 8, 300, 2), (3, 73, 40, 1),
+                                   (40, 12, 131073, 6)])
+@pytest.mark.parametrize("mode", ["topk", "hier"])
+def test_forward_tilings_are_exact(mode, shape, dtype):
+    """Forward kernel on either side of the sizes where its tiling changes (49152 and 131072 latents), with
+    ragged row blocks, last tiles and step counts, for every vector width the row length allows: integer
+    weights, vals of one, so that every error is an exact integer (all partial sums of squares stay below
+    2^24 units) and the residual shows which rows were read."""
+    B, K, F, D = shape
+    _announce("exact forward", mode, shape, dtype)
+    g = torch.Generator().manual_seed(B * K + D)
+    idx = torch.randint(0, F, (B, K), generator=g)
+    W = torch.randint(-1, 2, (F, D), generator=g).float()
+    bias = torch.randint(-2, 3, (D,), generator=g).float()
+    target = torch.randint(-2, 3, (B, D), generator=g).float()
+    e = W[idx].cumsum(1) + (bias - target).unsqueeze(1)
+    sq = e.square().sum() if mode == "hier" else e[:, -1].square().sum()
+    rc, loss, resid = abi.forward(mode, idx.to(DEV), *(x.to(dtype).to(DEV) for x in (W, torch.ones(B, K), bias, target)))
+    torch.cuda.synchronize()
+    assert rc == 0, _lib.status_string(rc)
+    assert torch.equal(resid.cpu(), e[:, -1])
+    # (a wavefront's fp32 sum is exact below 2^24; the total is one rounding away)
+    want = float(sq.double()) / (B * D * (K if mode == "hier" else 1))
+    assert abs(loss.item() - want) <= 2.0 ** -23 * want
