@@ -51,6 +51,7 @@ constexpr size_t kAlign = 256;
 constexpr int kBwdSgdUpdate = 1 << 20;  // internal flag of the slice loop: dW is the weight matrix, updated in place
 constexpr int kBwdHot = 1 << 21;        // internal flag of the slice loop: hot latents are accumulated in the LDS
 constexpr unsigned kLongBlocks = 1024;    // leading blocks of a reduction launch that serve hot latents
+constexpr int64_t kListBlocks = 8192;     // blocks of a reduction launch that work from the lists of latents
 
 inline bool valid_dtype(int d) { return d == FLEXSAE_F32 || d == FLEXSAE_BF16 || d == FLEXSAE_F16; }
 inline size_t dtype_size(int d) { return d == FLEXSAE_F32 ? 4 : 2; }
@@ -115,8 +116,8 @@ struct FwdPlan {
   int vec;
   int lpr;  // lanes per row piece
   int64_t n_row_blocks;
-  int64_t n_items;   // (tile, row block)
-  int64_t xcd_span;  // items per XCD, or 0: items in order
+  int64_t n_items;   // blocks with work, each leaves one loss partial
+  int64_t xcd_span;  // items per XCD; 0: items in order; -n_tiles: wavefronts in row order
   unsigned grid;
 };
 
@@ -144,14 +145,21 @@ FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target,
   // (B=2048, K=64, D=1024): 256 B beats 128 B from 32768 rows on (65536: 65 / 31 against 73 / 32, 131072:
   // 73 / 32 against 83 / 34; 512 B 78 / 37) and equals it below.  Eight-byte lanes gain 5 % on uniform
   // indices around 65536 rows and lose 25 % on skewed ones: 16 bytes per lane wherever rows allow it.
-  const bool by_xcd = s->F <= 131072;
-  const size_t piece_bytes = !by_xcd ? 512 : (es == 2 && s->F <= 49152) ? 128 : 256;
+  // Rows that do not start on a line (D=1538 bf16, F=65536: row order 133 / 70, 256 B per L2 154 / 62; D=1452,
+  // F=262144, K=128: 239, 512 B with all L2s on one tile 274; D=8184, F=524288: 834 against 775) keep the row
+  // order from 24576 latents up to 4 GiB of weights.
+  const bool lines = static_cast<size_t>(s->D) * es % 128 == 0;
+  const uint64_t w_bytes = static_cast<uint64_t>(s->F) * static_cast<uint64_t>(s->D) * es;
+  const bool by_row = !lines && s->F > 24576 && w_bytes < (uint64_t{1} << 32);
+  const bool by_xcd = !by_row && s->F <= 131072;
+  const size_t piece_bytes = by_row ? 1024 : !by_xcd ? 512 : (es == 2 && s->F <= 49152 && lines) ? 128 : 256;
   p.lpr = static_cast<int>(piece_bytes / (static_cast<size_t>(vec) * es));
   if (p.lpr > kWave) p.lpr = kWave;
-  const int64_t rows = (kWave / p.lpr) * static_cast<int64_t>(kWavesPerBlock);
-  p.n_row_blocks = ceil_div(s->B, rows);
-  p.n_items = ceil_div(s->D, static_cast<int64_t>(p.lpr) * vec) * p.n_row_blocks;
-  p.xcd_span = by_xcd ? ceil_div(p.n_items, 8) : 0;
+  const int64_t rows = kWave / p.lpr;
+  const int64_t n_tiles = ceil_div(s->D, static_cast<int64_t>(p.lpr) * vec);
+  p.n_row_blocks = ceil_div(s->B, rows * kWavesPerBlock);
+  p.n_items = by_row ? ceil_div(n_tiles * ceil_div(s->B, rows), static_cast<int64_t>(kWavesPerBlock)) : n_tiles * p.n_row_blocks;
+  p.xcd_span = by_xcd ? ceil_div(p.n_items, 8) : by_row ? -n_tiles : 0;
   p.grid = static_cast<unsigned>(by_xcd ? p.xcd_span * 8 : p.n_items);
   return p;
 }
@@ -174,8 +182,10 @@ void launch_fwd(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices
       FLEXSAE_LAUNCH_FWD(VEC, (kNarrow ? LPR128 : LPR256)); \
     } else if (p.lpr == LPR256) {                          \
       FLEXSAE_LAUNCH_FWD(VEC, LPR256);                     \
-    } else {                                               \
+    } else if (p.lpr == LPR512) {                          \
       FLEXSAE_LAUNCH_FWD(VEC, LPR512);                     \
+    } else {                                               \
+      FLEXSAE_LAUNCH_FWD(VEC, 64);                         \
     }                                                      \
   } while (0)
   if (p.vec == V16) {

@@ -15,7 +15,7 @@ namespace flexsae {
 // is consumed.
 //
 // What bounds it: the gathered bytes.  The weight matrix is read once per pair, and how fast depends on
-// which cache answers.  Two orders of the (tile, row block) items, picked by plan_fwd:
+// which cache answers.  Three orders of the (tile, row block) items, picked by plan_fwd:
 //   xcd_span > 0   the items, tiles outermost, are cut into eight equal runs, one per L2 (blocks
 //                  go round the eight XCDs): an L2 sees F pieces of one narrow tile at a time instead of
 //                  whole rows.  65536 pieces of 128 bytes are 8.4 MB against 4 MB of L2: about half of the
@@ -23,6 +23,9 @@ namespace flexsae {
 //                  (twice as slow).
 //   xcd_span == 0  items in order, tiles outermost, wide tiles: all XCDs gather from the same column
 //                  tile, which the memory-side cache (256 MB) holds where the L2s cannot help.
+//   xcd_span < 0   wavefronts in order, the -xcd_span tiles of a row next to each other: where rows do not
+//                  start on a 128-byte line, neighbouring pieces share lines, and only this order has them
+//                  read together.
 // Against one wavefront per (row, 256 columns) in row order, which no cache but the memory-side one served:
 // B=4096, K=128, F=65536, D=2304 bf16 (2.42 GB gathered) 328 -> 275 us (8.8 TB/s), K=64 172 -> 143 us; B=2048,
 // K=256, F=131072, D=1024 fp32 292 -> 273 us; B=16384, K=128, F=524288, D=8192 bf16 6.3 -> 4.8 ms (7.2 TB/s).
@@ -56,11 +59,23 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     if (i >= xcd_span) return;  // uniform per block
   }
   if (item >= n_items) return;  // uniform per block
-  const int64_t tile = item / n_row_blocks;
-  const int64_t b0 = ((item - tile * n_row_blocks) * kWaves + wv) * R;  // first row of the wavefront
+  int64_t tile, b0;  // of the wavefront: its tile, its first row
+  bool idle = false;
+  if (xcd_span >= 0) {
+    tile = item / n_row_blocks;
+    b0 = ((item - tile * n_row_blocks) * kWaves + wv) * R;
+  } else {
+    const int64_t n_tiles = -xcd_span;
+    const int64_t at = item * kWaves + wv;
+    b0 = at / n_tiles;
+    tile = at - b0 * n_tiles;
+    b0 *= R;
+    idle = b0 >= B;  // uniform per wavefront
+    if (idle) b0 = 0;
+  }
   const int64_t b = b0 + lane / LPR;
   const int d0 = static_cast<int>(tile) * (LPR * VEC) + (lane % LPR) * VEC;
-  const bool active = d0 < D && b < B;  // D % VEC == 0 is checked on the host
+  const bool active = d0 < D && b < B && !idle;  // D % VEC == 0 is checked on the host
   const int dsafe = d0 < D ? d0 : 0;
   const int64_t bsafe = b < B ? b : B - 1;
 
@@ -94,7 +109,7 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     return *reinterpret_cast<const raw_vec_t<WT, VEC> *>(wbase + static_cast<uint64_t>(row) * d_elems);
   };
 
-  for (int k0 = 0; k0 < K; k0 += kFwdChunk) {
+  for (int k0 = idle ? K : 0; k0 < K; k0 += kFwdChunk) {
     const int n = (K - k0) < kFwdChunk ? (K - k0) : kFwdChunk;  // uniform
     // lane j: step k0 + j of every row of the wavefront
     {
