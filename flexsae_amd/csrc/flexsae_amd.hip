@@ -270,47 +270,49 @@ void zero_f32(float *p, int64_t n, hipStream_t st) {
 }
 
 // How a pair list is built for a given problem size.  The bucketed construction serves every
-// size whose bucket count fits the LDS counters of its kernels; beyond that (more than
+// size whose bucket count fits the LDS cursors of its chunk kernel; beyond that (more than
 // kBucketMaxBuckets * kSortMaxLatents latents) the list is built with one memory atomic per pair.
 struct CsrPlan {
   bool bucketed;
   int shift;           // a bucket is 2^shift consecutive latents
   uint32_t n_buckets;
-  int64_t chunk;       // consecutive pairs counted by one block
+  int n_bits;          // bits of a bucket number
+  int64_t chunk;       // consecutive pairs ordered by one block
   uint32_t n_chunks;
-  size_t table_len;    // n_buckets * n_chunks (+1 entry for the total)
+  size_t table_len;    // (n_buckets + 1) * n_chunks
 };
 
 CsrPlan plan_csr(int64_t n_pairs, int64_t F) {
   CsrPlan p;
   // latents per bucket: about 2048 pairs per bucket on average, a power of two
   int shift = 0;
-  while (shift < 12 && (static_cast<int64_t>(2) << shift) * n_pairs <= 2048 * F) ++shift;
-  static_assert((1 << 12) == kSortMaxLatents, "shift limit follows the LDS counters of the sort kernel");
-  while (shift < 12 && ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketMaxBuckets) ++shift;
+  while (shift < kSortMaxShift && (static_cast<int64_t>(2) << shift) * n_pairs <= 2048 * F) ++shift;
+  while (shift < kSortMaxShift && ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketMaxBuckets) ++shift;
   p.shift = shift;
   const int64_t n_buckets = ceil_div(F, static_cast<int64_t>(1) << shift);
   p.bucketed = n_buckets <= kBucketMaxBuckets;
   p.n_buckets = static_cast<uint32_t>(p.bucketed ? n_buckets : 0);
+  p.n_bits = 0;
+  while (p.bucketed && (static_cast<int64_t>(1) << p.n_bits) < n_buckets) ++p.n_bits;
   p.chunk = 2048;
-  while (p.bucketed && ceil_div(n_pairs, p.chunk) * n_buckets > (static_cast<int64_t>(1) << 22)) p.chunk *= 2;
+  while (p.bucketed && p.chunk < kMaxChunk && ceil_div(n_pairs, p.chunk) * n_buckets > (static_cast<int64_t>(1) << 22))
+    p.chunk *= 2;
   p.n_chunks = static_cast<uint32_t>(ceil_div(n_pairs, p.chunk));
-  p.table_len = p.bucketed ? static_cast<size_t>(n_buckets) * p.n_chunks : 0;
+  p.table_len = p.bucketed ? static_cast<size_t>(n_buckets + 1) * p.n_chunks : 0;
   return p;
 }
 
 // Scratch of the pair-list construction, carved out of one workspace:
-//   bucketed: tmp[B*K] u64 | table[table_len + 1] | scan block sums | long_count (one aligned
-//             slot) | long_list[B*K/65 + 1]
-//   atomic:   rank[B*K] u32 | scan block sums[ceil(F/kScanBlockElems)] | long_count | long_list
+//   bucketed: tmp[B*K] u32 | table[table_len] | ctrl (kCtrlWords) | long_list[B*K/65 + 1]
+//   atomic:   rank[B*K] u32 | scan block sums[ceil(F/kScanBlockElems)] | ctrl | long_list
+// The lists besides long_list (chunk_begin, empty_list, cls_list) belong to the caller's workspace.
 struct CsrScratch {
   CsrPlan plan;
-  uint64_t *tmp;
+  uint32_t *tmp;
   uint32_t *table;
   uint32_t *rank;
   uint32_t *block_sums;
-  uint32_t *long_count;
-  uint32_t *long_list;
+  PairLists lists;
 };
 
 size_t csr_scan_sums_bytes(int64_t n) {
@@ -318,31 +320,25 @@ size_t csr_scan_sums_bytes(int64_t n) {
 }
 
 size_t csr_scratch_bytes(int64_t n_pairs, int64_t F, CsrScratch *sc, uint8_t *ws) {
-  const CsrPlan pl = plan_csr(n_pairs, F);
+  CsrScratch local = {};
+  CsrScratch &c = sc ? *sc : local;
+  c = CsrScratch{};
+  c.plan = plan_csr(n_pairs, F);
   size_t off = 0;
-  if (sc) {
-    sc->plan = pl;
-    sc->tmp = nullptr;
-    sc->table = nullptr;
-    sc->rank = nullptr;
-  }
-  if (pl.bucketed) {
-    if (sc) sc->tmp = reinterpret_cast<uint64_t *>(ws + off);
-    off += round_up(static_cast<size_t>(n_pairs) * 8, kAlign);
-    if (sc) sc->table = reinterpret_cast<uint32_t *>(ws + off);
-    off += round_up((pl.table_len + 1) * 4, kAlign);
-    if (sc) sc->block_sums = reinterpret_cast<uint32_t *>(ws + off);
-    off += csr_scan_sums_bytes(static_cast<int64_t>(pl.table_len));
+  auto take = [&](auto *&ptr, size_t bytes) {
+    ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(ws + off);
+    off += round_up(bytes, kAlign);
+  };
+  if (c.plan.bucketed) {
+    take(c.tmp, static_cast<size_t>(n_pairs) * 4);
+    take(c.table, c.plan.table_len * 4);
   } else {
-    if (sc) sc->rank = reinterpret_cast<uint32_t *>(ws + off);
-    off += round_up(static_cast<size_t>(n_pairs) * 4, kAlign);
-    if (sc) sc->block_sums = reinterpret_cast<uint32_t *>(ws + off);
-    off += csr_scan_sums_bytes(F);
+    take(c.rank, static_cast<size_t>(n_pairs) * 4);
+    take(c.block_sums, csr_scan_sums_bytes(F));
   }
-  if (sc) sc->long_count = reinterpret_cast<uint32_t *>(ws + off);
-  off += kAlign;
-  if (sc) sc->long_list = reinterpret_cast<uint32_t *>(ws + off);
-  off += round_up((static_cast<size_t>(n_pairs) / 65 + 1) * 4, kAlign);
+  static_assert(kCtrlWords * 4 <= kAlign, "the control words are one aligned slot");
+  take(c.lists.ctrl, kCtrlWords * 4);
+  take(c.lists.long_list, (static_cast<size_t>(n_pairs) / 65 + 1) * 4);
   return off;
 }
 
@@ -352,32 +348,30 @@ CsrScratch carve_csr_scratch(void *workspace, int64_t F, int64_t n_pairs) {
   return sc;
 }
 
-// begin[F+1], map[B*K] and, when `slot` is given, its inverse slot[B*K]; leaves the list of
-// latents with more than 64 pairs in sc.long_list / sc.long_count.
+void launch_pair_lists(const uint32_t *begin, int64_t F, const PairLists &lists, hipStream_t st) {
+  hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, lists.ctrl, static_cast<int64_t>(kCtrlWords), 0u);
+  hipLaunchKernelGGL(pair_lists_kernel, dim3(static_cast<unsigned>(ceil_div(F, kListLatents))), dim3(1024), 0, st, begin,
+                     F, lists);
+}
+
+// begin[F+1], map[B*K] and, when `slot` is given, its inverse slot[B*K] (and a second copy of it in
+// `hslot`); fills the lists of sc.lists.
 void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, uint32_t *begin,
-                      uint32_t *map, uint32_t *slot, const CsrScratch &sc, int *status_flag, hipStream_t st) {
+                      uint32_t *map, uint32_t *slot, uint32_t *hslot, const CsrScratch &sc, int *status_flag,
+                      hipStream_t st) {
   const int64_t n_pairs = B * K;
   const CsrPlan &pl = sc.plan;
   if (pl.bucketed) {
-    hipLaunchKernelGGL(csr_bucket_count_kernel, dim3(pl.n_chunks), dim3(kBucketThreads), 0, st, indices, n_pairs,
-                       F, pl.shift, pl.n_buckets, pl.chunk, pl.n_chunks, sc.table, sc.long_count, status_flag);
-    const int64_t len = static_cast<int64_t>(pl.table_len);
-    const unsigned scan_blocks = static_cast<unsigned>(ceil_div(len, kScanBlockElems));
-    hipLaunchKernelGGL(csr_scan_sums_kernel, dim3(scan_blocks), dim3(kScanThreads), 0, st, sc.table, len,
-                       sc.block_sums);
-    hipLaunchKernelGGL(csr_scan_apply_kernel, dim3(scan_blocks), dim3(kScanThreads), 0, st, sc.table, len,
-                       sc.block_sums);
-    hipLaunchKernelGGL(csr_bucket_scatter_kernel, dim3(pl.n_chunks), dim3(kBucketThreads), 0, st, indices,
-                       n_pairs, F, pl.shift, pl.n_buckets, pl.chunk, pl.n_chunks, sc.table, sc.tmp);
+    const size_t lds = (static_cast<size_t>(pl.n_buckets) * kChunkWaves + kChunkWaves) * 4;
+    hipLaunchKernelGGL(csr_chunk_sort_kernel, dim3(pl.n_chunks), dim3(kChunkThreads), lds, st, indices, n_pairs, F,
+                       pl.shift, pl.n_buckets, pl.n_bits, pl.chunk, pl.n_chunks, sc.table, sc.tmp, sc.lists.ctrl,
+                       status_flag);
     hipLaunchKernelGGL(csr_bucket_sort_kernel, dim3(pl.n_buckets), dim3(kSortThreads), 0, st, sc.tmp, sc.table,
-                       pl.n_chunks, pl.shift, F, begin, map, slot, sc.long_count, sc.long_list);
-    hipLaunchKernelGGL(csr_sort_long_kernel, dim3(1024), dim3(1024), 0, st, begin, map, sc.long_count,
-                       sc.long_list, slot, static_cast<uint32_t>(B < (1LL << 31) ? B : 0xffffffffLL),
-                       static_cast<uint32_t>(K));
+                       pl.n_chunks, pl.chunk, pl.shift, F, begin, map, slot, hslot, sc.lists);
     return;
   }
   hipLaunchKernelGGL(csr_init_kernel, dim3(grid_for(F + 1, 256, 4096)), dim3(256), 0, st, begin, F + 1,
-                     sc.long_count);
+                     sc.lists.ctrl);
   hipLaunchKernelGGL(csr_count_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st,
                      indices, n_pairs, F, begin, sc.rank, status_flag);
   const unsigned scan_blocks = static_cast<unsigned>(ceil_div(F, kScanBlockElems));
@@ -389,13 +383,33 @@ void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
                      n_pairs, F, begin, sc.rank, map);
   hipLaunchKernelGGL(csr_sort_short_kernel,
                      dim3(static_cast<unsigned>(ceil_div(F, kWavesPerBlock))), dim3(kBlock), 0, st,
-                     begin, map, F, sc.long_count, sc.long_list);
-  hipLaunchKernelGGL(csr_sort_long_kernel, dim3(1024), dim3(1024), 0, st, begin, map, sc.long_count,
-                     sc.long_list, static_cast<uint32_t *>(nullptr), static_cast<uint32_t>(B < (1LL << 31) ? B : 0xffffffffLL),
+                     begin, map, F, sc.lists.ctrl + kLongCount, sc.lists.long_list);
+  hipLaunchKernelGGL(csr_sort_long_kernel, dim3(1024), dim3(1024), 0, st, begin, map, sc.lists.ctrl + kLongCount,
+                     sc.lists.long_list, static_cast<uint32_t>(B < (1LL << 31) ? B : 0xffffffffLL),
                      static_cast<uint32_t>(K));
   if (slot)
     hipLaunchKernelGGL(csr_inverse_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, map, n_pairs,
-                       slot);
+                       slot, hslot);
+  if (sc.lists.chunk_begin) launch_pair_lists(begin, F, sc.lists, st);
+}
+
+// The lists of a pair list that belong to the caller's workspace (everything but ctrl and long_list): their bytes, and
+// their places in `base` if that is given.
+size_t carve_pair_lists(size_t n_pairs, size_t F, void *base, PairLists *ls) {
+  size_t off = 0;
+  auto take = [&](uint32_t *&ptr, size_t entries) {
+    if (base) ptr = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(base) + off);
+    off += round_up(entries * 4, kAlign);
+  };
+  PairLists none = {};
+  PairLists &l = ls ? *ls : none;
+  take(l.chunk_begin, n_pairs / 65 + 1);
+  take(l.empty_list, F);
+  for (int i = 0; i < kClasses; ++i) {
+    const size_t most = n_pairs / ((size_t{1} << i) / 2 + 1);
+    take(l.cls_list[i], (most < F ? most : F) + 1);
+  }
+  return off;
 }
 
 // Columns per tile of the training-step kernel: one register per gathered row piece, so 16-bit
@@ -406,11 +420,8 @@ inline int64_t train_tile_cols(const flexsae_shape *s) {
 
 // ---- two-phase hierarchical backward: workspace plan -----------------------------------
 
-constexpr int kClsStride = 80;  // slots per counter array of the class list
-static_assert(kSegClasses + 1 <= kClsStride, "a counter array holds one slot per class and the total");
-
-// Most latents without a pair, the rest with few: the reduction by pieces then works from the list
-// of latents ordered by row count and the rows of latents without pairs are zeroed in one pass.
+// Most latents without a pair, the rest with few: the reduction by pieces then works from the lists
+// of latents by row count and the rows of latents without pairs are zeroed in one pass.
 // Whether that pays depends on how many latents really are without a pair: with two pairs per latent
 // on average it does for skewed indices (two thirds of the latents empty: the step a sixth faster) and
 // does not for uniform ones (an eighth of them empty: the step 8 % slower).  Only the caller can know,
@@ -427,7 +438,7 @@ struct HierBwdPlan {
   size_t n_pairs;          // B * K
   size_t n_rows;           // B
   size_t n_partial_rows;   // upper bound on the number of 64-pair chunks of long latents
-  size_t off_begin, off_map, off_slot, off_csr, off_chunk, off_cls, off_cls_list, off_sfinal, off_colsum, off_loss, off_dvpart, off_partial;  // per-slice buffers follow
+  size_t off_begin, off_map, off_slot, off_csr, off_lists, off_sfinal, off_colsum, off_loss, off_dvpart, off_partial;  // per-slice buffers follow
   size_t n_loss_partials;  // training-step kernel: one per (tile of 64 or 128 columns, row)
   size_t fixed_bytes;      // everything that does not depend on the slice width
   // hot-latent tables (only with `hot`): slots with the hot pairs marked, control words, the hot
@@ -463,14 +474,8 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false) {
   off += round_up(p.n_pairs * 4, kAlign);
   p.off_csr = off;
   off += flexsae_csr_workspace_bytes(s->B, s->K, s->F);
-  p.off_chunk = off;
-  off += round_up((p.n_pairs / 65 + 2) * 4, kAlign);
-  // latents ordered by row count (sparse shapes, see seg_class_scatter_kernel): three counter
-  // arrays of kClsStride slots (histogram, cursors, first entry of every class) and the list
-  p.off_cls = off;
-  off += round_up(3 * static_cast<size_t>(kClsStride) * 4, kAlign);
-  p.off_cls_list = off;
-  off += round_up(static_cast<size_t>(s->F) * 4, kAlign);
+  p.off_lists = off;
+  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), nullptr, nullptr);
   p.off_sfinal = off;  // S_{b,0} of every row, [B, d_pad] fp32: dbias is its column sum
   off += round_up(p.n_rows * static_cast<size_t>(p.d_pad) * 4, kAlign);
   p.off_colsum = off;  // partial column sums, [ceil(B/64), D] fp32
@@ -507,6 +512,13 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false) {
   p.off_partial = off;
   p.fixed_bytes = off;
   return p;
+}
+
+// The pair-list scratch and lists of a hierarchical workspace.
+CsrScratch carve_hier_lists(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws) {
+  CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
+  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), ws + pl.off_lists, &sc.lists);
+  return sc;
 }
 
 // Slice granule (columns) of the training step.  The training-step kernel works on tiles of
@@ -678,15 +690,14 @@ size_t hier_bwd_bytes(const HierBwdPlan &p, int64_t slice_w) {
 // tiles, twice the wavefronts): faster once a latent has about four rows or more, slower for
 // shorter groups.
 template <typename PT, typename GT, int VEC>
-void launch_seg_reduce(bool narrow, const uint32_t *begin, const CsrScratch &sc, const uint32_t *chunk_begin,
+void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, const PairLists &ls,
                        const void *P, float *partial, void *dW, const float *dw_scale, int64_t F, int tps,
                        int col0, int sw, int D, hipStream_t st, int piece_cols = 0, int64_t cols = 0, int64_t n_pairs = 0,
-                       int update = 0, const uint32_t *cls_begin = nullptr, const uint32_t *cls_list = nullptr,
-                       HotFinalize *defer = nullptr) {
+                       int update = 0, bool by_count = false, HotFinalize *defer = nullptr) {
   // the second step of the hot latents: launched here, or handed back through `defer` for the next
   // training-step launch to carry
   auto finalize = [&](int mode, int units) {
-    HotFinalize h = {sc.long_count, sc.long_list, chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, 256u};
+    HotFinalize h = {ll.ctrl, ll.list, ll.chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, 256u};
     if (defer) {
       h.n_blocks = 64u;  // riding along with a long launch: few blocks, so that they cost little where there is nothing to do
       *defer = h;
@@ -699,22 +710,22 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const CsrScratch &sc,
     int pps_shift = -1;  // log2(pps) when pps is a power of two
     for (int sh = 0; sh < 16; ++sh)
       if (pps == (1 << sh)) pps_shift = sh;
-    // latents per group of lanes: four, taken from the list ordered by row count, where most latents
+    // latents per group of lanes: four, taken from the lists by row count, where most latents
     // have no or few rows (with four rows per latent on average the bookkeeping already costs more
-    // than the shorter launch saves); the list holds at most min(F, pairs) latents with rows
-#define FLEXSAE_PIECE_REDUCE(G, N_ITEMS, CLS_LIST, CLS_BEGIN)                                                      \
+    // than the shorter launch saves); the lists hold at most min(F, pairs) latents with rows
+#define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS)                                                                          \
   hipLaunchKernelGGL((seg_reduce_piece_kernel<PT, GT, FLEXSAE_PIECE_U, G>),                                        \
-                     dim3(kLongBlocks +                                                                            \
-                          static_cast<unsigned>(ceil_div((N_ITEMS) * pps, kBlock / kPieceLanes))),             \
-                     dim3(kBlock), 0, st, begin, sc.long_count, sc.long_list, chunk_begin, P, partial, dW, dw_scale, \
-                     F, kLongBlocks, pps, pps_shift, col0, sw, D, update, CLS_LIST, CLS_BEGIN)
-    if (cls_list) {
-      // work items of the list: one per latent with kSegBigRows rows or more, one per four others
+                     dim3(kLongBlocks + static_cast<unsigned>(N_BLOCKS)), dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, \
+                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, ls)
+    constexpr int64_t kGroups = kBlock / kPieceLanes;
+    if (by_count) {
+      // work items: one per latent with nine rows or more, one per four others of a class
       const int64_t n_listed_max = F < n_pairs ? F : n_pairs;
-      const int64_t n_items_max = n_pairs / kSegBigRows + ceil_div(n_listed_max, 4) + 1;
-      FLEXSAE_PIECE_REDUCE(4, n_items_max, cls_list, cls_begin);
+      const int64_t n_items_max = (n_pairs / 9 + ceil_div(n_listed_max, 4) + kClasses) * pps;
+      const int64_t n_blocks = ceil_div(n_items_max, kGroups);
+      FLEXSAE_PIECE_REDUCE(4, (n_blocks < kListBlocks ? n_blocks : kListBlocks));
     } else {
-      FLEXSAE_PIECE_REDUCE(1, F, static_cast<const uint32_t *>(nullptr), static_cast<const uint32_t *>(nullptr));
+      FLEXSAE_PIECE_REDUCE(1, ceil_div(F * pps, kGroups));
     }
 #undef FLEXSAE_PIECE_REDUCE
     // the chunk partials of hot latents are combined per 64-column piece
@@ -727,7 +738,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const CsrScratch &sc,
     const int rtps = tps * (VEC / RV);
     const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * rtps, kWavesPerBlock));
     hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, RV, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
-                       dim3(kBlock), 0, st, begin, sc.long_count, sc.long_list, chunk_begin, P, partial, dW, dw_scale,
+                       dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale,
                        F, kLongBlocks, rtps, col0, sw, D);
     static_assert(RV == 2 || !kCanNarrow, "the narrow reduction works on tiles of 128 columns");
     finalize(3, rtps);
@@ -735,13 +746,13 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const CsrScratch &sc,
   }
   const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * tps, kWavesPerBlock));
   hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, VEC, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
-                     dim3(kBlock), 0, st, begin, sc.long_count, sc.long_list, chunk_begin, P, partial, dW, dw_scale, F,
+                     dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale, F,
                      kLongBlocks, tps, col0, sw, D);
   if constexpr (VEC == 4) {
     finalize(2, tps);
   } else {
-    hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st, sc.long_count,
-                       sc.long_list, chunk_begin, partial, dW, dw_scale, tps, col0, sw, D);
+    hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st, ll.ctrl,
+                       ll.list, ll.chunk_begin, partial, dW, dw_scale, tps, col0, sw, D);
   }
 }
 
@@ -758,8 +769,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   const float *dw_scale = (flags & (FLEXSAE_BWD_SCALE_BY_GRAD_OUT | kBwdSgdUpdate)) ? grad_out : nullptr;
   const uint32_t *begin = reinterpret_cast<const uint32_t *>(ws + pl.off_begin);
   const uint32_t *slot = reinterpret_cast<const uint32_t *>(ws + pl.off_slot);
-  const CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
-  uint32_t *chunk_begin = reinterpret_cast<uint32_t *>(ws + pl.off_chunk);
+  const CsrScratch sc = carve_hier_lists(s, pl, ws);
   float *s_final = reinterpret_cast<float *>(ws + pl.off_sfinal);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   float *colsum_part = reinterpret_cast<float *>(ws + pl.off_colsum);
@@ -777,14 +787,14 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   uint32_t *hot_ctrl = hot ? reinterpret_cast<uint32_t *>(ws + pl.off_hot_ctrl) : nullptr;
   const uint32_t *hot_list = hot ? reinterpret_cast<const uint32_t *>(ws + pl.off_hot_list) : nullptr;
   float *hot_partial[2] = {nullptr, nullptr};
-  CsrScratch sc_cold = sc;  // the long latents the reduction serves
+  // the long latents the reduction serves
+  LongList reduce_long = {sc.lists.ctrl, sc.lists.long_list, sc.lists.chunk_begin};
   if (hot) {
     uint8_t *base = static_cast<uint8_t *>(P) + hier_p_bytes(pl, slice_w);
     hot_partial[0] = reinterpret_cast<float *>(base);
     hot_partial[1] = reinterpret_cast<float *>(base + hier_hot_partial_bytes(pl, slice_w));
-    sc_cold.long_count = hot_ctrl + kHotLong2Count;
-    sc_cold.long_list = reinterpret_cast<uint32_t *>(ws + pl.off_long2);
-    chunk_begin = reinterpret_cast<uint32_t *>(ws + pl.off_chunk2);
+    reduce_long = {hot_ctrl + kHotLong2, reinterpret_cast<uint32_t *>(ws + pl.off_long2),
+                   reinterpret_cast<uint32_t *>(ws + pl.off_chunk2)};
   }
   const int hot_headroom = (flags & FLEXSAE_BWD_HOT_NO_HEADROOM) ? -6 : 2;
   // columns that are worked on: whole reduction tiles, or, with the piece reduction, whole training
@@ -796,14 +806,13 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   int sweep_vec = VEC;
   const int min_sweep_vec = static_cast<int>((pl.tile < train_tile_cols(s) ? pl.tile : train_tile_cols(s)) / kWave);
   while (sweep_vec > 1 && sweep_vec > min_sweep_vec && s->B * (slice_w / (kWave * sweep_vec)) < 6144) sweep_vec >>= 1;
-  // Sparse shapes reduce every slice by pieces from the list of latents ordered by row count; the
+  // Sparse shapes reduce every slice by pieces from the lists of latents by row count; the
   // rows of latents without pairs are zeroed here, whole rows in one pass (the in-place update leaves
   // them alone).
   const bool sparse = piece != 0 && sparse_latents(s, flags);
-  const uint32_t *cls_begin = reinterpret_cast<const uint32_t *>(ws + pl.off_cls) + 2 * kClsStride;
-  const uint32_t *cls_list = reinterpret_cast<const uint32_t *>(ws + pl.off_cls_list);
   if (sparse && do_reduce && !update)
-    hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, cls_begin, cls_list, dW, D);
+    hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, sc.lists.ctrl,
+                       sc.lists.empty_list, dW, D);
   // In the training step the second step of a slice's hot latents travels with the next slice's
   // training-step launch (a gradient of the weight's own dtype only: that is what that kernel writes);
   // the last slice's gets a launch of its own.
@@ -852,9 +861,9 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     const bool cache_sized = static_cast<size_t>(s->B * s->K) * static_cast<size_t>(sw) * pl.p_size <= (size_t{384} << 20);
     const bool by_pieces =
         piece != 0 && (update || cols % pl.tile != 0 || sparse_latents(s, flags) || cache_sized);
-    launch_seg_reduce<PT, GT, VEC>(narrow_reduce, begin, sc_cold, chunk_begin, P, partial, dW, dw_scale, s->F, tps,
+    launch_seg_reduce<PT, GT, VEC>(narrow_reduce, begin, reduce_long, sc.lists, P, partial, dW, dw_scale, s->F, tps,
                                    static_cast<int>(col0), sw, D, st, by_pieces ? piece : 0, cols, s->B * s->K, update,
-                                   sparse ? cls_begin : nullptr, sparse ? cls_list : nullptr, fold ? &pending : nullptr);
+                                   sparse, fold ? &pending : nullptr);
     if (hot) {
       // the block partials of the slice's hot latents are added up by the next training-step launch
       // (they live in the buffer that launch does not write), or here
@@ -937,26 +946,11 @@ void launch_hier_slices_w(const flexsae_shape *s, const HierBwdPlan &pl, int64_t
   }
 }
 
-// What follows the pair list in a hierarchical workspace: the chunk table of the hot latents and, for
-// sparse shapes, the list of latents ordered by row count.
-void finish_pair_list(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws, const uint32_t *begin,
-                      const CsrScratch &sc, hipStream_t st, int flags = 0) {
-  uint32_t *cls = reinterpret_cast<uint32_t *>(ws + pl.off_cls);
-  const bool sparse = sparse_latents(s, flags);
-  hipLaunchKernelGGL(seg_chunk_table_kernel, dim3(1), dim3(1024), 0, st, begin, sc.long_count, sc.long_list,
-                     reinterpret_cast<uint32_t *>(ws + pl.off_chunk), sparse ? cls : static_cast<uint32_t *>(nullptr),
-                     2 * kClsStride);
-  if (!sparse) return;
-  // few blocks: every block ends with one memory atomic per class it met, all on the same counters
-  hipLaunchKernelGGL(seg_class_hist_kernel, dim3(grid_for(s->F, 256, 128)), dim3(256), 0, st, begin, s->F, cls);
-  hipLaunchKernelGGL(seg_class_scatter_kernel, dim3(static_cast<unsigned>(ceil_div(s->F, 256 * kClassPerThread))),
-                     dim3(256), 0, st, begin, s->F, cls, cls + kClsStride, cls + 2 * kClsStride,
-                     reinterpret_cast<uint32_t *>(ws + pl.off_cls_list));
-}
-
 // Hot-latent tables of a workspace whose pair list is complete: the slots with the hot pairs marked,
-// the hot latents, the long latents that stayed cold and their chunk table.
-void build_hot_tables(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws, const CsrScratch &sc, hipStream_t st) {
+// the hot latents, the long latents that stayed cold and their chunk table.  have_hslot: hslot[] already
+// holds a copy of slot[].
+void build_hot_tables(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws, const CsrScratch &sc, bool have_hslot,
+                      hipStream_t st) {
   const uint32_t *begin = reinterpret_cast<const uint32_t *>(ws + pl.off_begin);
   const uint32_t *map = reinterpret_cast<const uint32_t *>(ws + pl.off_map);
   uint32_t *hslot = reinterpret_cast<uint32_t *>(ws + pl.off_hslot);
@@ -966,17 +960,17 @@ void build_hot_tables(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws
   uint32_t *cand_state = reinterpret_cast<uint32_t *>(ws + pl.off_cand_state);
   uint32_t *long_cand = reinterpret_cast<uint32_t *>(ws + pl.off_long_cand);
   uint32_t *long2 = reinterpret_cast<uint32_t *>(ws + pl.off_long2);
-  const int64_t n_pairs = s->B * s->K;
-  hipLaunchKernelGGL(copy_u32_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, hslot,
-                     reinterpret_cast<const uint32_t *>(ws + pl.off_slot), n_pairs);
-  hipLaunchKernelGGL(hot_select_kernel, dim3(1), dim3(1024), 0, st, begin, sc.long_count, sc.long_list, ctrl,
+  if (!have_hslot) {
+    const int64_t n_pairs = s->B * s->K;
+    hipLaunchKernelGGL(copy_u32_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, hslot,
+                       reinterpret_cast<const uint32_t *>(ws + pl.off_slot), n_pairs);
+  }
+  hipLaunchKernelGGL(hot_select_kernel, dim3(1), dim3(1024), 0, st, begin, sc.lists.ctrl, sc.lists.long_list, ctrl,
                      cand_list, long_cand, static_cast<uint32_t>(kHotMax));
   hipLaunchKernelGGL(hot_mark_kernel, dim3(kHotMax), dim3(1024), 0, st, begin, map, ctrl, cand_list, cand_state,
                      hot_list, hslot, static_cast<uint32_t>(s->K));
-  hipLaunchKernelGGL(hot_cold_long_kernel, dim3(64), dim3(256), 0, st, sc.long_count, sc.long_list, long_cand,
-                     cand_state, ctrl, long2);
-  hipLaunchKernelGGL(seg_chunk_table_kernel, dim3(1), dim3(1024), 0, st, begin, ctrl + kHotLong2Count, long2,
-                     reinterpret_cast<uint32_t *>(ws + pl.off_chunk2), static_cast<uint32_t *>(nullptr), 0);
+  hipLaunchKernelGGL(hot_cold_long_kernel, dim3(64), dim3(256), 0, st, begin, sc.lists.ctrl, sc.lists.long_list,
+                     long_cand, cand_state, ctrl, long2, reinterpret_cast<uint32_t *>(ws + pl.off_chunk2));
 }
 
 // ---- TopK backward: workspace plan and slice loop ---------------------------------------
@@ -985,7 +979,7 @@ struct TopkBwdPlan {
   int vec, tile;
   int64_t d_pad;
   size_t n_pairs, n_partial_rows;
-  size_t off_colsum, off_long_count, off_long_list, off_chunk, off_resid16, off_dvpart, off_slotbv, off_partial, fixed_bytes;
+  size_t off_colsum, off_ctrl, off_long_list, off_lists, off_resid16, off_dvpart, off_slotbv, off_partial, fixed_bytes;
   bool resid16;  // gather a bf16 copy of the residual (bf16 weights): half the cache footprint
 };
 
@@ -1006,12 +1000,12 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   size_t off = 0;
   p.off_colsum = off;
   off += round_up(static_cast<size_t>(ceil_div(s->B, kColsumRows)) * static_cast<size_t>(s->D) * 4, kAlign);
-  p.off_long_count = off;
-  off += kAlign;
+  p.off_ctrl = off;
+  off += round_up(kCtrlWords * 4, kAlign);
   p.off_long_list = off;
   off += round_up((p.n_pairs / 65 + 1) * 4, kAlign);
-  p.off_chunk = off;
-  off += round_up((p.n_pairs / 65 + 2) * 4, kAlign);
+  p.off_lists = off;
+  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), nullptr, nullptr);
   p.off_resid16 = off;
   if (p.resid16) off += round_up(static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 2, kAlign);
   p.off_dvpart = off;  // per-tile shares of dvals: [d_pad / tile, B*K] fp32
@@ -1023,6 +1017,14 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   return p;
 }
 
+PairLists carve_topk_lists(const flexsae_shape *s, const TopkBwdPlan &pl, uint8_t *ws) {
+  PairLists ls = {};
+  ls.ctrl = reinterpret_cast<uint32_t *>(ws + pl.off_ctrl);
+  ls.long_list = reinterpret_cast<uint32_t *>(ws + pl.off_long_list);
+  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), ws + pl.off_lists, &ls);
+  return ls;
+}
+
 size_t topk_bwd_bytes(const TopkBwdPlan &p, int64_t slice_w) {
   return p.fixed_bytes + round_up(p.n_partial_rows * static_cast<size_t>(slice_w) * 4, kAlign);
 }
@@ -1032,9 +1034,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
                         const uint32_t *begin, const uint32_t *map, const void *weight,
                         const void *vals, const void *resid, const float *grad_out, float coef,
                         void *dW, float *dvals, uint8_t *ws, hipStream_t st) {
-  const uint32_t *long_count = reinterpret_cast<const uint32_t *>(ws + pl.off_long_count);
-  const uint32_t *long_list = reinterpret_cast<const uint32_t *>(ws + pl.off_long_list);
-  const uint32_t *chunk_begin = reinterpret_cast<const uint32_t *>(ws + pl.off_chunk);
+  const PairLists ls = carve_topk_lists(s, pl, ws);
+  const uint32_t *long_ctrl = ls.ctrl, *long_list = ls.long_list, *chunk_begin = ls.chunk_begin;
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   const int64_t n_pairs = static_cast<int64_t>(pl.n_pairs);
@@ -1047,12 +1048,12 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
         static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * sizeof(typename Traits<RT>::store_t);
     hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC>),
                        dim3(kLongBlocks + static_cast<unsigned>(n_short_blocks), static_cast<unsigned>(tps)),
-                       dim3(kBlock), 0, st, begin, map, long_count, long_list, chunk_begin,
+                       dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
                        s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, kLongBlocks, tps,
                        static_cast<int>(col0), sw, s->F, K, D, static_cast<uint32_t>(resid_bytes));
     hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st,
-                       long_count, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps,
+                       long_ctrl, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps,
                        static_cast<int>(col0), sw, D);
   }
 }
@@ -1240,10 +1241,8 @@ int flexsae_hier_pair_stats(const flexsae_shape *s, const void *workspace, uint3
   if (!aligned(workspace, kAlign) || !aligned(stats, 4)) return FLEXSAE_ERR_ALIGNMENT;
   const HierBwdPlan pl = plan_hier_bwd(s);  // the part of the layout every hierarchical workspace shares
   uint8_t *ws = static_cast<uint8_t *>(const_cast<void *>(workspace));
-  const CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
-  hipLaunchKernelGGL(pair_stats_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream),
-                     reinterpret_cast<const uint32_t *>(ws + pl.off_begin), s->F, sc.long_count,
-                     reinterpret_cast<const uint32_t *>(ws + pl.off_chunk), stats);
+  const CsrScratch sc = carve_hier_lists(s, pl, ws);
+  hipLaunchKernelGGL(pair_stats_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), sc.lists.ctrl, stats);
   return launch_status();
 }
 
@@ -1295,12 +1294,9 @@ int flexsae_hier_bwd(const flexsae_shape *s, const int64_t *indices, const void 
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   uint32_t *begin = reinterpret_cast<uint32_t *>(ws + pl.off_begin);
   uint32_t *map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
-  const CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
-  if (!(flags & FLEXSAE_BWD_REUSE_PAIR_LIST)) {
-    csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot), sc,
-                     status_flag, st);
-    finish_pair_list(s, pl, ws, begin, sc, st, flags);
-  }
+  if (!(flags & FLEXSAE_BWD_REUSE_PAIR_LIST))
+    csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot), nullptr,
+                     carve_hier_lists(s, pl, ws), status_flag, st);
   const float coef = static_cast<float>(
       2.0 / (static_cast<double>(s->B) * static_cast<double>(s->K) * static_cast<double>(s->D)));
   if (pl.vec == 4) {
@@ -1339,7 +1335,6 @@ int flexsae_hier_import_pair_list(const flexsae_shape *s, const uint32_t *begin,
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   uint32_t *ws_begin = reinterpret_cast<uint32_t *>(ws + pl.off_begin);
   uint32_t *ws_map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
-  const CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
   const int64_t n_pairs = s->B * s->K;
   if (ws_begin != begin)
     hipLaunchKernelGGL(copy_u32_kernel, dim3(grid_for(s->F + 1, 256, 4096)), dim3(256), 0, st, ws_begin, begin,
@@ -1347,11 +1342,8 @@ int flexsae_hier_import_pair_list(const flexsae_shape *s, const uint32_t *begin,
   if (ws_map != map)
     hipLaunchKernelGGL(copy_u32_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, ws_map, map, n_pairs);
   hipLaunchKernelGGL(csr_inverse_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, ws_map, n_pairs,
-                     reinterpret_cast<uint32_t *>(ws + pl.off_slot));
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, sc.long_count, static_cast<int64_t>(1), 0u);
-  hipLaunchKernelGGL(seg_find_long_kernel, dim3(grid_for(s->F, 256, 2048)), dim3(256), 0, st, ws_begin, s->F,
-                     sc.long_count, sc.long_list);
-  finish_pair_list(s, pl, ws, ws_begin, sc, st);
+                     reinterpret_cast<uint32_t *>(ws + pl.off_slot), static_cast<uint32_t *>(nullptr));
+  launch_pair_lists(ws_begin, s->F, carve_hier_lists(s, pl, ws).lists, st);
   return launch_status();
 }
 
@@ -1409,14 +1401,13 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   uint32_t *begin = reinterpret_cast<uint32_t *>(ws + pl.off_begin);
   uint32_t *map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
-  const CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
-  if (!(flags & FLEXSAE_BWD_REUSE_PAIR_LIST)) {
-    csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot), sc,
-                     status_flag, st);
-    finish_pair_list(s, pl, ws, begin, sc, st, flags);
-  }
+  const CsrScratch sc = carve_hier_lists(s, pl, ws);
+  const bool build = !(flags & FLEXSAE_BWD_REUSE_PAIR_LIST);
+  if (build)
+    csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot),
+                     hot ? reinterpret_cast<uint32_t *>(ws + pl.off_hslot) : nullptr, sc, status_flag, st);
   if (hot && !((flags & FLEXSAE_BWD_REUSE_PAIR_LIST) && (flags & FLEXSAE_BWD_REUSE_HOT_TABLES)))
-    build_hot_tables(s, pl, ws, sc, st);
+    build_hot_tables(s, pl, ws, sc, build, st);
   const double count = static_cast<double>(s->B) * static_cast<double>(s->K) * static_cast<double>(s->D);
   const float coef = static_cast<float>(2.0 / count);
   const TrainArgs ta = {bias, target, loss, s->B * (hier_cols_used(s, pl, true, piece) / train_tile_cols(s)),
@@ -1491,7 +1482,7 @@ int flexsae_csr_build(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
       !aligned(workspace, kAlign))
     return FLEXSAE_ERR_WORKSPACE;
   const CsrScratch sc = carve_csr_scratch(workspace, F, B * K);
-  csr_build_launch(indices, B, K, F, begin, map, nullptr, sc, status_flag, static_cast<hipStream_t>(stream));
+  csr_build_launch(indices, B, K, F, begin, map, nullptr, nullptr, sc, status_flag, static_cast<hipStream_t>(stream));
   return launch_status();
 }
 
@@ -1537,14 +1528,8 @@ int flexsae_topk_bwd(const flexsae_shape *s, const uint32_t *begin, const uint32
   hipStream_t st = static_cast<hipStream_t>(stream);
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   // (every output element is written exactly once: nothing needs a zero-fill, whatever `flags` says)
-  // latents with more than 64 pairs and their chunk table
-  uint32_t *long_count = reinterpret_cast<uint32_t *>(ws + pl.off_long_count);
-  uint32_t *long_list = reinterpret_cast<uint32_t *>(ws + pl.off_long_list);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, long_count, static_cast<int64_t>(1), 0u);
-  hipLaunchKernelGGL(seg_find_long_kernel, dim3(grid_for(s->F, 256, 2048)), dim3(256), 0, st, begin, s->F,
-                     long_count, long_list);
-  hipLaunchKernelGGL(seg_chunk_table_kernel, dim3(1), dim3(1024), 0, st, begin, long_count, long_list,
-                     reinterpret_cast<uint32_t *>(ws + pl.off_chunk), static_cast<uint32_t *>(nullptr), 0);
+  const PairLists lists = carve_topk_lists(s, pl, ws);
+  launch_pair_lists(begin, s->F, lists, st);
   const float coef =
       static_cast<float>(2.0 / (static_cast<double>(s->B) * static_cast<double>(s->D)));
   // per-pair records and, for bf16 weights, the bf16 copy of the residual: one launch

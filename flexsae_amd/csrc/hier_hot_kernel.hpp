@@ -42,7 +42,9 @@ constexpr uint32_t kHotNone = 0xffffffffu;
 constexpr int kHotExpMin = -96;         // exponents are clamped to [kHotExpMin, 127]: 2^(22 - E) stays a normal float
 
 // Control words of the hot-latent tables (one uint32 each).
-enum { kHotNHot = 0, kHotNCand = 1, kHotLong2Count = 2, kHotThreshold = 3, kHotDeferred = 4, kHotCtrlWords = 64 };
+// From kHotLong2 on the same two words as a pair list's control words begin with: chunks and number of
+// the long latents that stayed cold.
+enum { kHotNHot = 0, kHotNCand = 1, kHotLong2Count = 2, kHotThreshold = 3, kHotDeferred = 4, kHotLong2 = 6, kHotCtrlWords = 64 };
 
 __device__ __forceinline__ float wave_max_bcast(float v) {
   v = fmaxf(v, dpp_move<0xB1>(v));       // lanes whose source does not exist receive 0: the values are >= 0
@@ -61,7 +63,7 @@ __device__ __forceinline__ float wave_max_bcast(float v) {
 // the order of that list.  Single block.  cand_list[c] = latent, long_cand[i] = candidate number of
 // long_list[i] or kHotNone; clears the counters that the kernels after it advance.
 __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__restrict__ begin,
-                                                          const uint32_t *__restrict__ long_count,
+                                                          const uint32_t *__restrict__ long_ctrl,
                                                           const uint32_t *__restrict__ long_list,
                                                           uint32_t *__restrict__ ctrl,
                                                           uint32_t *__restrict__ cand_list,
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__rest
   __shared__ uint32_t sel_prefix, sel_k, sel_prefix_next, sel_k_next, n_cand_s;
   __shared__ uint32_t wave_tot[4];
   const int tid = threadIdx.x;
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   for (uint32_t i = tid; i < n_long && i < kCached; i += 1024) {
     const uint32_t f = long_list[i];
     cnt_lds[i] = begin[f + 1] - begin[f];
@@ -136,6 +138,8 @@ __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__rest
     n_cand_s = 0;
     ctrl[kHotNHot] = 0;
     ctrl[kHotLong2Count] = 0;
+    ctrl[kHotLong2 + kLongChunks] = 0;
+    ctrl[kHotLong2 + kLongCount] = 0;
     ctrl[kHotThreshold] = T;
     ctrl[kHotDeferred] = 0;
   }
@@ -185,45 +189,37 @@ __global__ __launch_bounds__(1024) void hot_mark_kernel(const uint32_t *__restri
   for (uint32_t i = s0 + threadIdx.x; i < s1; i += blockDim.x) hslot[map[i]] = kHotSlotBit | h;
 }
 
-// long2_list = the latents with more than kSegChunk pairs that did not become hot (any order):
-// what the chunked part of the segment reduction still serves.
-__global__ void hot_cold_long_kernel(const uint32_t *__restrict__ long_count,
+// long2_list = the latents with more than kSegChunk pairs that did not become hot (any order), with
+// their chunk table: what the chunked part of the segment reduction still serves.
+__global__ void hot_cold_long_kernel(const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
                                      const uint32_t *__restrict__ long_list,
                                      const uint32_t *__restrict__ long_cand,
                                      const uint32_t *__restrict__ cand_state, uint32_t *__restrict__ ctrl,
-                                     uint32_t *__restrict__ long2_list) {
-  const uint32_t n_long = *long_count;
+                                     uint32_t *__restrict__ long2_list, uint32_t *__restrict__ chunk2_begin) {
+  const uint32_t n_long = long_ctrl[kLongCount];
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_long; i += stride) {
     const uint32_t c = long_cand[i];
     const bool hot = c != kHotNone && cand_state[c] != kHotNone;
-    if (!hot) long2_list[atomicAdd(&ctrl[kHotLong2Count], 1u)] = long_list[i];
+    if (hot) continue;
+    const uint32_t f = long_list[i];
+    const uint32_t chunks = (begin[f + 1] - begin[f] + kSegChunk - 1) / kSegChunk;
+    const unsigned long long at =
+        atomicAdd(reinterpret_cast<unsigned long long *>(ctrl + kHotLong2), (1ull << 32) | chunks);
+    long2_list[at >> 32] = f;
+    chunk2_begin[at >> 32] = static_cast<uint32_t>(at);
+    atomicAdd(&ctrl[kHotLong2Count], 1u);  // a statistic
   }
 }
 
-// out[0] = latents with more than kSegChunk pairs, out[1] = their pairs in chunks of kSegChunk,
-// out[2] = latents without a pair.  One block (the pair list's segment starts are read once:
-// 4 bytes per latent); `out` may be pinned host memory.
-__global__ __launch_bounds__(1024) void pair_stats_kernel(const uint32_t *__restrict__ begin, int64_t F,
-                                                          const uint32_t *__restrict__ long_count,
-                                                          const uint32_t *__restrict__ chunk_begin,
-                                                          uint32_t *__restrict__ out) {
-  __shared__ uint32_t wave_tot[1024 / kWave];
-  uint32_t mine = 0;  // per lane, so that the loads of several rounds are in flight together
-#pragma unroll 8
-  for (int64_t f = threadIdx.x; f < F; f += 1024) mine += begin[f + 1] == begin[f] ? 1u : 0u;
-  uint32_t empty = mine;
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) empty += static_cast<uint32_t>(__shfl_xor(static_cast<int>(empty), off, kWave));
-  if (lane_id() == 0) wave_tot[threadIdx.x >> 6] = empty;
-  __syncthreads();
+// What a pair list's control words say about the indices: out[0] = latents with more than kSegChunk
+// pairs, out[1] = their pairs in chunks of kSegChunk, out[2] = latents without a pair.  `out` may be
+// pinned host memory.
+__global__ void pair_stats_kernel(const uint32_t *__restrict__ ctrl, uint32_t *__restrict__ out) {
   if (threadIdx.x == 0) {
-    uint32_t total = 0;
-    for (int w = 0; w < 1024 / kWave; ++w) total += wave_tot[w];
-    const uint32_t n_long = *long_count;
-    out[0] = n_long;
-    out[1] = chunk_begin[n_long];
-    out[2] = total;
+    out[0] = ctrl[kLongCount];
+    out[1] = ctrl[kLongChunks];
+    out[2] = ctrl[kEmptyCount];
   }
 }
 

@@ -6,6 +6,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "csr_kernels.hpp"
 
 #ifndef FLEXSAE_REDUCE_NT
 #define FLEXSAE_REDUCE_NT true
@@ -14,8 +15,7 @@
 namespace flexsae {
 
 constexpr int kSegChunk = 64;  // rows per chunk; groups longer than this count as "long"
-constexpr int kSegClasses = kSegChunk + 1;  // row counts 0..kSegChunk of the list ordered by row count (below)
-constexpr int kSegBigRows = 9;  // latents with at least this many rows get a group of lanes to themselves there
+static_assert(kSegChunk == static_cast<int>(kListLong), "the long latents of a pair list are the ones reduced in chunks");
 
 // acc += sum of rows [r0, r0+n) of X (row stride `ld` elements) over the lane's VEC columns at pc.
 // Rows are fetched up to U at a time; n is uniform over the wavefront, so the tests around the
@@ -73,6 +73,14 @@ __device__ __forceinline__ void accumulate_rows_by4(const void *__restrict__ X, 
   for (int i = 0; i < VEC; ++i) acc[i] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
 }
 
+// The long latents a reduction serves: a pair list's (see PairLists), or those of them that the
+// hot-latent accumulators have not taken.
+struct LongList {
+  const uint32_t *ctrl;  // [kLongChunks], [kLongCount]
+  const uint32_t *list;
+  const uint32_t *chunk_begin;
+};
+
 // Decode work item `chunk` of the long-latent work list: which latent, which rows.
 struct LongChunk {
   uint32_t long_slot;
@@ -107,7 +115,7 @@ __device__ __forceinline__ LongChunk seg_decode_chunk(const uint32_t *__restrict
 // without rows get zeros; latents with more than kSegChunk rows are skipped.
 template <typename PT, typename GT, int VEC, int U>
 __global__ __launch_bounds__(256) void seg_reduce_kernel(
-    const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_count,
+    const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int tps, int col0,
@@ -136,9 +144,9 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
     if (d0 < D) store_vec<GT, VEC, FLEXSAE_REDUCE_NT>(out, f * D + d0, acc);
     return;
   }
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   if (n_long == 0) return;
-  const int64_t total = static_cast<int64_t>(chunk_begin[n_long]) * tps;
+  const int64_t total = static_cast<int64_t>(long_ctrl[kLongChunks]) * tps;
   const int64_t n_waves = static_cast<int64_t>(n_long_blocks) * (blockDim.x >> 6);
   for (int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block(); w < total;
        w += n_waves) {
@@ -161,20 +169,20 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
 // and this one.  The four latents (or pieces) of a wavefront have different row counts: the loop
 // runs to the longest, loads beyond a group's own count are masked off.  Work order: pieces of a
 // latent adjacent, latents ascending, so the launch still reads P front to back.  G > 1: a group
-// serves G latents taken from the list ordered by row count (cls_list / cls_begin, see
-// seg_class_scatter_kernel; chosen by the caller where most latents have no or few rows), and
-// latents without rows are not written here.
+// serves G latents taken from the lists of latents by row count (chosen by the caller where most
+// latents have no or few rows), and latents without rows are not written here.
+__device__ __forceinline__ int64_t ceil_div_u32(uint32_t a, int b) { return (static_cast<int64_t>(a) + b - 1) / b; }
+
 constexpr int kPieceLanes = 16;
 constexpr int kPieceBytes = kPieceLanes * 16;
 
 template <typename PT, typename GT, int U, int G>
 __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
-    const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_count,
+    const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int pps, int pps_shift, int col0,
-    int slice_w, int D, int update, const uint32_t *__restrict__ cls_list,
-    const uint32_t *__restrict__ cls_begin) {
+    int slice_w, int D, int update, PairLists lists) {
   using S = typename Traits<PT>::store_t;
   constexpr int EV = 16 / static_cast<int>(sizeof(S));  // columns per lane
   constexpr int kGroupsPerBlock = 256 / kPieceLanes;
@@ -220,121 +228,135 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
   };
 
   if (blockIdx.x >= n_long_blocks) {
-    // (latent block, piece) of this group of lanes; a latent block is G consecutive latents.  The
-    // block's first item is split with one wave-uniform division; the sixteen groups then only
+    // (latent block, piece) of this group of lanes; a latent block is G consecutive latents.  How many
+    // there are is only known on the device where they come from the lists: a bounded number of blocks strides
+    // over them (a block for every group there could be is four times as many, most of them empty: 69 instead of
+    // 64 us for 75 750 latents of 1 to 8 and 4 252 of 9 to 64 rows of 512 columns).  A block's first item is split with one wave-uniform division; the sixteen groups then only
     // divide a number below pps + 16 (a 64-bit division per lane would cost more instructions than
     // the rest of a short item)
-    const int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock;
-    int64_t fb;
-    int t;
-    if (pps_shift >= 0) {  // pps is a power of two (the usual slice widths): shifts only
-      const int64_t item = item0 + group;
-      fb = item >> pps_shift;
-      t = static_cast<int>(item & ((1 << pps_shift) - 1));
-    } else {
-      const int64_t f_first = item0 / pps;
-      const uint32_t rem = static_cast<uint32_t>(item0 - f_first * pps) + static_cast<uint32_t>(group);
-      const uint32_t q = rem / static_cast<uint32_t>(pps);
-      fb = f_first + q;
-      t = static_cast<int>(rem - q * static_cast<uint32_t>(pps));
+    int64_t n_groups = F;
+    if constexpr (G > 1) {
+      n_groups = 0;
+#pragma unroll
+      for (int i = 0; i < kClasses; ++i) n_groups += ceil_div_u32(lists.ctrl[kClassCount + i], i < kClassSolo ? G : 1);
     }
-    const int pc = t * (kPieceLanes * EV) + sub * EV;
-    const int d0 = col0 + pc;
-    const float g = scale ? scale[0] : 1.0f;  // the rows were produced for a unit upstream gradient
-    float acc[EV];
-#pragma unroll
-    for (int i = 0; i < EV; ++i) acc[i] = 0.f;
-    if constexpr (G == 1) {
-      const int64_t f = fb;
-      uint32_t s0 = 0, n = 0;
-      if (f < F) {
-        s0 = begin[f];
-        n = begin[f + 1] - s0;
-      }
-      const bool mine = f < F && n <= static_cast<uint32_t>(kSegChunk);  // longer ones: chunked below
-      accumulate(s0, mine ? static_cast<int>(n) : 0, 1, pc, acc);
-      if (scale) {
-#pragma unroll
-        for (int i = 0; i < EV; ++i) acc[i] *= g;
-      }
-      if (mine && !(update && n == 0)) emit(f, d0, acc);
-    } else {
-      // Few rows per latent and most latents without any: the latents come from the list that
-      // seg_class_scatter_kernel wrote, ordered by row count (those without rows first: they are
-      // zeroed by seg_zero_rows_kernel and skipped here; those with more than kSegChunk rows are not
-      // in it).  A group serves G consecutive entries, i.e. G latents of (nearly always) the same row
-      // count, so the four groups of a wavefront finish together; their rows are fetched U at a time
-      // regardless of where one latent ends and the next begins, and a latent's sum is stored when
-      // its last row has been added.  The order of the additions of a latent is the same as with G = 1.
-      // Work items: first the latents with kSegBigRows rows or more, one per group and the heaviest
-      // first (a group that had four of them would still be running long after the rest of the launch),
-      // then the others, G per group.
-      const uint32_t lo = cls_begin[1], mid = cls_begin[kSegBigRows], hi = cls_begin[kSegChunk + 1];
-      const int64_t n_big = static_cast<int64_t>(hi - mid);
-      int64_t first;  // first entry of this group
-      int count;      // entries it serves
-      if (fb < n_big) {
-        first = static_cast<int64_t>(hi) - 1 - fb;
-        count = 1;
+    const int64_t n_items = n_groups * pps;
+    const int64_t item_stride = static_cast<int64_t>(gridDim.x - n_long_blocks) * kGroupsPerBlock;
+    for (int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock; item0 < n_items;
+         item0 += item_stride) {
+      int64_t fb;
+      int t;
+      if (pps_shift >= 0) {  // pps is a power of two (the usual slice widths): shifts only
+        const int64_t item = item0 + group;
+        fb = item >> pps_shift;
+        t = static_cast<int>(item & ((1 << pps_shift) - 1));
       } else {
-        first = static_cast<int64_t>(lo) + (fb - n_big) * G;
-        const int64_t left = static_cast<int64_t>(mid) - first;
-        count = left < G ? (left > 0 ? static_cast<int>(left) : 0) : G;
+        const int64_t f_first = item0 / pps;
+        const uint32_t rem = static_cast<uint32_t>(item0 - f_first * pps) + static_cast<uint32_t>(group);
+        const uint32_t q = rem / static_cast<uint32_t>(pps);
+        fb = f_first + q;
+        t = static_cast<int>(rem - q * static_cast<uint32_t>(pps));
       }
-      uint32_t fv = 0, b0v = 0, b1v = 0;  // lane j < count of the group: entry j, its latent and rows
-      if (sub < count) {
-        fv = cls_list[first + sub];
-        b0v = begin[fv];
-        b1v = begin[fv + 1];
-      }
-      uint32_t c[G + 1], off[G], fid[G];  // row i of the group's list, c[j] <= i < c[j+1], is row i + off[j] of P
-      c[0] = 0;
+      const int pc = t * (kPieceLanes * EV) + sub * EV;
+      const int d0 = col0 + pc;
+      const float g = scale ? scale[0] : 1.0f;  // the rows were produced for a unit upstream gradient
+      float acc[EV];
 #pragma unroll
-      for (int j = 0; j < G; ++j) {
-        const uint32_t b0 = static_cast<uint32_t>(__shfl(static_cast<int>(b0v), j, kPieceLanes));
-        const uint32_t b1 = static_cast<uint32_t>(__shfl(static_cast<int>(b1v), j, kPieceLanes));
-        fid[j] = static_cast<uint32_t>(__shfl(static_cast<int>(fv), j, kPieceLanes));
-        c[j + 1] = c[j] + (b1 - b0);  // nothing for entries beyond the list
-        off[j] = b0 - c[j];
-      }
-      const uint32_t total = c[G];
-      for (uint32_t i0 = 0; __any(i0 < total); i0 += U) {
-        raw_vec_t<PT, EV> raw[U];
-        uint32_t whose[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t i = i0 + u;
-          raw[u] = raw_vec_t<PT, EV>{};
-          whose[u] = fid[0];
-          uint32_t o = off[0];
-#pragma unroll
-          for (int j = 1; j < G; ++j)
-            if (i >= c[j]) {
-              whose[u] = fid[j];
-              o = off[j];
-            }
-          if (i < total)
-            raw[u] = __builtin_nontemporal_load(reinterpret_cast<const raw_vec_t<PT, EV> *>(
-                Pp + static_cast<int64_t>(i + o) * slice_w + pc));
+      for (int i = 0; i < EV; ++i) acc[i] = 0.f;
+      if constexpr (G == 1) {
+        const int64_t f = fb;
+        uint32_t s0 = 0, n = 0;
+        if (f < F) {
+          s0 = begin[f];
+          n = begin[f + 1] - s0;
         }
+        const bool mine = f < F && n <= static_cast<uint32_t>(kSegChunk);  // longer ones: chunked below
+        accumulate(s0, mine ? static_cast<int>(n) : 0, 1, pc, acc);
+        if (scale) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t i = i0 + u;
-          float x[EV];
-          unpack_raw<PT, EV>(raw[u], x);
+          for (int i = 0; i < EV; ++i) acc[i] *= g;
+        }
+        if (mine && !(update && n == 0)) emit(f, d0, acc);
+      } else {
+        // Few rows per latent and most latents without any: the latents come from the lists of the pair
+        // list (those without rows are zeroed by seg_zero_rows_kernel and skipped here; those with more
+        // than kSegChunk rows are in neither list).  A group serves G consecutive entries, i.e. G latents
+        // of nearly always the same row count, so the four groups of a wavefront finish together; their
+        // rows are fetched U at a time regardless of where one latent ends and the next begins, and a
+        // latent's sum is stored when its last row has been added.  The order of the additions of a
+        // latent is the same as with G = 1.  Work items: the classes in descending order, so that the heaviest
+        // groups start first, those of kClassSolo on one latent per group (a group that had four of them
+        // would still be running long after the rest of the launch), the others G per group.
+        const uint32_t *list = nullptr;  // first entry of this group
+        int count = 0;                   // entries it serves
+        int64_t at = fb;
 #pragma unroll
-          for (int k = 0; k < EV; ++k) acc[k] += x[k];  // masked-off loads left zeros
-          bool last = false;  // the last row of its latent
+        for (int i = kClasses - 1; i >= 0; --i) {
+          const int64_t n_cls = static_cast<int64_t>(lists.ctrl[kClassCount + i]);
+          const int per = i < kClassSolo ? G : 1;
+          const int64_t groups = ceil_div_u32(lists.ctrl[kClassCount + i], per);
+          if (at >= 0 && at < groups) {
+            list = lists.cls_list[i] + at * per;
+            const int64_t left = n_cls - at * per;
+            count = left < per ? static_cast<int>(left) : per;
+          }
+          at -= groups;
+        }
+        uint32_t fv = 0, b0v = 0, b1v = 0;  // lane j < count of the group: entry j, its latent and rows
+        if (sub < count) {
+          fv = list[sub];
+          b0v = begin[fv];
+          b1v = begin[fv + 1];
+        }
+        uint32_t c[G + 1], off[G], fid[G];  // row i of the group's list, c[j] <= i < c[j+1], is row i + off[j] of P
+        c[0] = 0;
 #pragma unroll
-          for (int j = 1; j <= G; ++j) last |= i + 1 == c[j];
-          if (i < total && last) {
-            if (scale) {
+        for (int j = 0; j < G; ++j) {
+          const uint32_t b0 = static_cast<uint32_t>(__shfl(static_cast<int>(b0v), j, kPieceLanes));
+          const uint32_t b1 = static_cast<uint32_t>(__shfl(static_cast<int>(b1v), j, kPieceLanes));
+          fid[j] = static_cast<uint32_t>(__shfl(static_cast<int>(fv), j, kPieceLanes));
+          c[j + 1] = c[j] + (b1 - b0);  // nothing for entries beyond the list
+          off[j] = b0 - c[j];
+        }
+        const uint32_t total = c[G];
+        for (uint32_t i0 = 0; __any(i0 < total); i0 += U) {
+          raw_vec_t<PT, EV> raw[U];
+          uint32_t whose[U];
 #pragma unroll
-              for (int k = 0; k < EV; ++k) acc[k] *= g;
+          for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + u;
+            raw[u] = raw_vec_t<PT, EV>{};
+            whose[u] = fid[0];
+            uint32_t o = off[0];
+#pragma unroll
+            for (int j = 1; j < G; ++j)
+              if (i >= c[j]) {
+                whose[u] = fid[j];
+                o = off[j];
+              }
+            if (i < total)
+              raw[u] = __builtin_nontemporal_load(reinterpret_cast<const raw_vec_t<PT, EV> *>(
+                  Pp + static_cast<int64_t>(i + o) * slice_w + pc));
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + u;
+            float x[EV];
+            unpack_raw<PT, EV>(raw[u], x);
+#pragma unroll
+            for (int k = 0; k < EV; ++k) acc[k] += x[k];  // masked-off loads left zeros
+            bool last = false;  // the last row of its latent
+#pragma unroll
+            for (int j = 1; j <= G; ++j) last |= i + 1 == c[j];
+            if (i < total && last) {
+              if (scale) {
+#pragma unroll
+                for (int k = 0; k < EV; ++k) acc[k] *= g;
+              }
+              emit(static_cast<int64_t>(whose[u]), d0, acc);
+#pragma unroll
+              for (int k = 0; k < EV; ++k) acc[k] = 0.f;
             }
-            emit(static_cast<int64_t>(whose[u]), d0, acc);
-#pragma unroll
-            for (int k = 0; k < EV; ++k) acc[k] = 0.f;
           }
         }
       }
@@ -344,10 +366,10 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
   // Long latents: one wavefront per (64-row chunk, piece); its four groups take every fourth row
   // (sixteen rows in flight per wavefront) and their sums are added across the groups in a fixed
   // order.  A hot latent's chunks are spread over many wavefronts.
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   if (n_long == 0) return;
   constexpr int kGroups = kWave / kPieceLanes;
-  const int64_t total = static_cast<int64_t>(chunk_begin[n_long]) * pps;
+  const int64_t total = static_cast<int64_t>(long_ctrl[kLongChunks]) * pps;
   const int64_t n_waves = static_cast<int64_t>(n_long_blocks) * (blockDim.x >> 6);
   const int g = (static_cast<int>(threadIdx.x) & (kWave - 1)) / kPieceLanes;
   for (int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block(); w < total; w += n_waves) {
@@ -373,14 +395,14 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
 // the next slice's training-step launch).
 template <typename GT>
 __device__ __forceinline__ void seg_piece_finalize_body(
-    const uint32_t *__restrict__ long_count, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial,
     void *__restrict__ out, const float *__restrict__ scale, int pieces, int col0, int slice_w, int D,
     int update, unsigned block, unsigned n_blocks) {
   constexpr int EV = 4, U = 4, kGroups = kWave / kPieceLanes;
   const int lane = lane_id();
   const int sub = lane & (kPieceLanes - 1), g = lane / kPieceLanes;
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   const int64_t total = static_cast<int64_t>(n_long) * pieces;
   const int64_t n_waves = static_cast<int64_t>(n_blocks) * (blockDim.x >> 6);
   for (int64_t w = static_cast<int64_t>(block) * (blockDim.x >> 6) + wave_in_block(); w < total; w += n_waves) {
@@ -388,7 +410,7 @@ __device__ __forceinline__ void seg_piece_finalize_body(
     const int t = static_cast<int>(w - static_cast<int64_t>(i) * pieces);
     const int pc = t * (kPieceLanes * EV) + sub * EV;
     const int d0 = col0 + pc;
-    const uint32_t c0 = chunk_begin[i], c1 = chunk_begin[i + 1];
+    const uint32_t c0 = chunk_begin[i], c1 = i + 1 < n_long ? chunk_begin[i + 1] : long_ctrl[kLongChunks];
     const int n = (static_cast<int>(c1 - c0) - g + kGroups - 1) / kGroups;
     const float *row = partial + (static_cast<int64_t>(c0) + g) * slice_w + pc;
     const int64_t stride = static_cast<int64_t>(kGroups) * slice_w;
@@ -427,11 +449,11 @@ __device__ __forceinline__ void seg_piece_finalize_body(
 
 template <typename GT>
 __global__ __launch_bounds__(256) void seg_reduce_piece_finalize_kernel(
-    const uint32_t *__restrict__ long_count, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial,
     void *__restrict__ out, const float *__restrict__ scale, int pieces, int col0, int slice_w, int D,
     int update) {
-  seg_piece_finalize_body<GT>(long_count, long_list, chunk_begin, partial, out, scale, pieces, col0, slice_w, D, update,
+  seg_piece_finalize_body<GT>(long_ctrl, long_list, chunk_begin, partial, out, scale, pieces, col0, slice_w, D, update,
                               blockIdx.x, gridDim.x);
 }
 
@@ -439,12 +461,12 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_finalize_kernel(
 // partials, in chunk order.
 template <typename GT, int VEC, int U>
 __device__ __forceinline__ void seg_long_finalize_body(
-    const uint32_t *__restrict__ long_count, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial,
     void *__restrict__ out, const float *__restrict__ scale, int tps, int col0, int slice_w, int D,
     unsigned block, unsigned n_blocks) {
   const int lane = lane_id();
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   const int64_t total = static_cast<int64_t>(n_long) * tps;
   const int64_t n_waves = static_cast<int64_t>(n_blocks) * (blockDim.x >> 6);
   for (int64_t w = static_cast<int64_t>(block) * (blockDim.x >> 6) + wave_in_block(); w < total;
@@ -453,7 +475,7 @@ __device__ __forceinline__ void seg_long_finalize_body(
     const int t = static_cast<int>(w - static_cast<int64_t>(i) * tps);
     const int pc = t * (kWave * VEC) + lane * VEC;
     const int d0 = col0 + pc;
-    const uint32_t c0 = chunk_begin[i], c1 = chunk_begin[i + 1];
+    const uint32_t c0 = chunk_begin[i], c1 = i + 1 < n_long ? chunk_begin[i + 1] : long_ctrl[kLongChunks];
     float acc[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) acc[k] = 0.f;
@@ -469,10 +491,10 @@ __device__ __forceinline__ void seg_long_finalize_body(
 
 template <typename GT, int VEC, int U>
 __global__ __launch_bounds__(256) void seg_reduce_long_finalize_kernel(
-    const uint32_t *__restrict__ long_count, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial,
     void *__restrict__ out, const float *__restrict__ scale, int tps, int col0, int slice_w, int D) {
-  seg_long_finalize_body<GT, VEC, U>(long_count, long_list, chunk_begin, partial, out, scale, tps, col0, slice_w, D,
+  seg_long_finalize_body<GT, VEC, U>(long_ctrl, long_list, chunk_begin, partial, out, scale, tps, col0, slice_w, D,
                                      blockIdx.x, gridDim.x);
 }
 
@@ -481,7 +503,7 @@ __global__ __launch_bounds__(256) void seg_reduce_long_finalize_kernel(
 // contributions nor the partial sums, and the reduction that overwrites the partial sums comes after
 // it in the stream), which saves a launch per slice.
 struct HotFinalize {
-  const uint32_t *long_count;
+  const uint32_t *long_ctrl;
   const uint32_t *long_list;
   const uint32_t *chunk_begin;
   const float *partial;
@@ -496,13 +518,13 @@ struct HotFinalize {
 template <typename GT>
 __device__ __forceinline__ void hot_finalize_run(const HotFinalize &h, unsigned block) {
   if (h.mode == 1)
-    seg_piece_finalize_body<GT>(h.long_count, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units, h.col0,
+    seg_piece_finalize_body<GT>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units, h.col0,
                                 h.slice_w, h.D, h.update, block, h.n_blocks);
   else if (h.mode == 2)
-    seg_long_finalize_body<GT, 4, 8>(h.long_count, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units,
+    seg_long_finalize_body<GT, 4, 8>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units,
                                      h.col0, h.slice_w, h.D, block, h.n_blocks);
   else if (h.mode == 3)
-    seg_long_finalize_body<GT, 2, 8>(h.long_count, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units,
+    seg_long_finalize_body<GT, 2, 8>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units,
                                      h.col0, h.slice_w, h.D, block, h.n_blocks);
 }
 
@@ -511,140 +533,15 @@ __global__ __launch_bounds__(256) void hot_finalize_kernel(HotFinalize h) {
   hot_finalize_run<GT>(h, blockIdx.x);
 }
 
-// long_list[0..*long_count) = latents with more than kSegChunk pairs (any order);
-// *long_count must be zero on entry.
-__global__ void seg_find_long_kernel(const uint32_t *__restrict__ begin, int64_t F,
-                                     uint32_t *__restrict__ long_count,
-                                     uint32_t *__restrict__ long_list) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t f = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; f < F; f += stride)
-    if (begin[f + 1] - begin[f] > static_cast<uint32_t>(kSegChunk))
-      long_list[atomicAdd(long_count, 1u)] = static_cast<uint32_t>(f);
-}
-
-// chunk_begin[i] = number of chunks of the long latents before long_list[i]
-// (chunk_begin[n_long] = total); single block.  Also clears zero_me[0..n_zero) when given (n_zero <= 1024).
-__global__ __launch_bounds__(1024) void seg_chunk_table_kernel(const uint32_t *__restrict__ begin,
-                                                               const uint32_t *__restrict__ long_count,
-                                                               const uint32_t *__restrict__ long_list,
-                                                               uint32_t *__restrict__ chunk_begin,
-                                                               uint32_t *__restrict__ zero_me, int n_zero) {
-  __shared__ uint32_t wave_tot[1024 / kWave];
-  __shared__ uint32_t carry_s;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid >> 6;
-  // counters of the kernels that follow in the stream (the class histogram and cursors below)
-  if (zero_me && tid < n_zero) zero_me[tid] = 0u;
-  const uint32_t n_long = *long_count;
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (uint32_t base = 0; base < n_long; base += 1024) {
-    const uint32_t i = base + tid;
-    uint32_t c = 0;
-    if (i < n_long) {
-      const uint32_t f = long_list[i];
-      c = (begin[f + 1] - begin[f] + kSegChunk - 1) / kSegChunk;
-    }
-    uint32_t inc = c;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint32_t y = __shfl_up(inc, off, kWave);
-      if (lane >= off) inc += y;
-    }
-    if (lane == kWave - 1) wave_tot[wv] = inc;
-    __syncthreads();
-    uint32_t wave_off = 0;
-    for (int w = 0; w < wv; ++w) wave_off += wave_tot[w];
-    const uint32_t excl = carry_s + wave_off + inc - c;
-    if (i < n_long) chunk_begin[i] = excl;
-    __syncthreads();
-    if (tid == 1023) carry_s = excl + c;
-    __syncthreads();
-  }
-  if (tid == 0) chunk_begin[n_long] = carry_s;
-}
-
-// ---- latents ordered by row count ----------------------------------------------------------
-// Where most latents have no pair at all and the rest one or a few (B*K <= 2F, skewed indices), the
-// reduction by pieces works from a list of the latents ordered by their number of rows:
-//   cls_list[cls_begin[n] .. cls_begin[n+1]) = the latents with exactly n rows, 0 <= n <= kSegChunk
-// (any order inside a class; latents with more rows are not listed: they go through the chunked
-// path).  Class 0 is zeroed in one pass over whole rows of the output (seg_zero_rows_kernel); the
-// groups of lanes of the reduction take four consecutive entries of the classes 1..kSegChunk, which
-// nearly always have the same row count, so no load slot is wasted on unequal groups.
-// Two launches: a histogram over the classes, then the placement (a counting sort whose cursors
-// are advanced once per block and class).  hist, cursor: kSegClasses counters each, zero on entry.
-constexpr int kClassPerThread = 8;  // latents per thread of the placement kernel
-
-__global__ __launch_bounds__(256) void seg_class_hist_kernel(const uint32_t *__restrict__ begin, int64_t F,
-                                                             uint32_t *__restrict__ hist) {
-  __shared__ uint32_t h[kSegClasses];
-  for (int t = threadIdx.x; t < kSegClasses; t += 256) h[t] = 0u;
-  __syncthreads();
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t f0 = static_cast<int64_t>(blockIdx.x) * blockDim.x; f0 < F; f0 += stride) {  // uniform per block
-    const int64_t f = f0 + threadIdx.x;
-    uint32_t n = kSegClasses;  // not counted
-    if (f < F) n = begin[f + 1] - begin[f];
-    // the empty class is the common one: counted per wavefront, not per lane
-    const unsigned long long empties = __ballot(n == 0u);
-    if (lane_id() == 0 && empties) atomicAdd(&h[0], static_cast<uint32_t>(__popcll(empties)));
-    if (n != 0u && n < static_cast<uint32_t>(kSegClasses)) atomicAdd(&h[n], 1u);
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < kSegClasses; t += 256)
-    if (h[t]) atomicAdd(&hist[t], h[t]);
-}
-
-__global__ __launch_bounds__(256) void seg_class_scatter_kernel(const uint32_t *__restrict__ begin, int64_t F,
-                                                                const uint32_t *__restrict__ hist,
-                                                                uint32_t *__restrict__ cursor,
-                                                                uint32_t *__restrict__ cls_begin,
-                                                                uint32_t *__restrict__ cls_list) {
-  __shared__ uint32_t base[kSegClasses + 1];  // first entry of every class
-  __shared__ uint32_t cnt[kSegClasses];       // this block's latents per class, then where they start in the class
-  const int tid = threadIdx.x;
-  if (tid <= kSegClasses) {
-    uint32_t s = 0;
-    for (int k = 0; k < tid; ++k) s += hist[k];
-    base[tid] = s;
-    if (blockIdx.x == 0) cls_begin[tid] = s;
-  }
-  if (tid < kSegClasses) cnt[tid] = 0u;
-  __syncthreads();
-  const int64_t f_block = static_cast<int64_t>(blockIdx.x) * (256 * kClassPerThread);
-  uint32_t cls[kClassPerThread], rank[kClassPerThread];
-#pragma unroll
-  for (int i = 0; i < kClassPerThread; ++i) {
-    const int64_t f = f_block + i * 256 + tid;
-    cls[i] = kSegClasses;  // not listed
-    rank[i] = 0u;
-    if (f < F) {
-      const uint32_t n = begin[f + 1] - begin[f];
-      if (n < static_cast<uint32_t>(kSegClasses)) cls[i] = n;
-    }
-    if (cls[i] < static_cast<uint32_t>(kSegClasses)) rank[i] = atomicAdd(&cnt[cls[i]], 1u);
-  }
-  __syncthreads();
-  if (tid < kSegClasses) {
-    const uint32_t c = cnt[tid];
-    cnt[tid] = c ? atomicAdd(&cursor[tid], c) : 0u;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kClassPerThread; ++i)
-    if (cls[i] < static_cast<uint32_t>(kSegClasses))
-      cls_list[base[cls[i]] + cnt[cls[i]] + rank[i]] = static_cast<uint32_t>(f_block + i * 256 + tid);
-}
-
-// out[f, 0..D) = 0 for the latents without rows (class 0 of the list): one wavefront per row, EV
+// out[f, 0..D) = 0 for the latents without rows: one wavefront per row, EV
 // columns per lane like the reduction by pieces (D is a multiple of EV and rows are 16-byte aligned
 // wherever that reduction runs).
 template <typename PT, typename GT>
-__global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__restrict__ cls_begin,
+__global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__restrict__ ctrl,
                                                             const uint32_t *__restrict__ cls_list,
                                                             void *__restrict__ out, int D) {
   constexpr int EV = 16 / static_cast<int>(sizeof(typename Traits<PT>::store_t));
-  const uint32_t n = cls_begin[1];
+  const uint32_t n = ctrl[kEmptyCount];
   const int lane = lane_id();
   float zero[EV];
 #pragma unroll

@@ -226,7 +226,7 @@ __device__ __forceinline__ void topk_short_latent(
 template <typename WT, typename GT, typename RT, int VEC>
 __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const uint32_t *__restrict__ begin, const uint32_t *__restrict__ map,
-    const uint32_t *__restrict__ long_count, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const vec_t<uint32_t, 2> *__restrict__ slot_bv,
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
@@ -255,9 +255,9 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
         dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f, b0, static_cast<int>(n), d0, D);
     return;
   }
-  const uint32_t n_long = *long_count;
+  const uint32_t n_long = long_ctrl[kLongCount];
   if (n_long == 0) return;
-  const uint32_t n_chunks = chunk_begin[n_long];
+  const uint32_t n_chunks = long_ctrl[kLongChunks];
   const int64_t total = static_cast<int64_t>(n_chunks) * tps;
   const int64_t n_waves = static_cast<int64_t>(n_long_blocks) * gridDim.y * (blockDim.x >> 6);
   for (int64_t wk = (static_cast<int64_t>(blockIdx.y) * n_long_blocks + blockIdx.x) * (blockDim.x >> 6) +

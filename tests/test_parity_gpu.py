@@ -7,6 +7,8 @@ and, on the reference's own shape x dtype matrix, also torch.testing.assert_clos
 reference's per-dtype atol/rtol (reference tests/test_setup.py:35-39).  Integer outputs (the
 latent-major pair list) and gather addressing are compared bit for bit.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -1061,3 +1063,40 @@ def _graph_capture_body(mode, fn, idx, W, v, b, t):
         ref = _run_op(mode, new, 1.0)  # eager work between the replays
         for a, c in zip(got, ref):
             assert torch.equal(a, c), (mode, trial)
+
+
+@pytest.mark.parametrize("shape", [(16384, 140, 5000, 0.0), (9000, 250, 300000, 0.1), (2049, 1, 7, 0.0), (4100, 64, 64, 0.0),
+                                   (700, 47, 40000, 0.9)])
+def test_pair_list_pieces_and_lists(shape):
+    """Pair list where the bucket kernel collects its pieces from more chunks than one window holds, chunks
+    with a ragged end, buckets that consist of long groups only, and a bucket with one group far larger than the
+    LDS; and the counters that come with it (latents with more than 64 pairs, their 64-pair chunks, latents
+    without pairs) as flexsae_hier_pair_stats hands them out after a step."""
+    B, K, F, hot = shape
+    _announce("csr pieces", shape)
+    g = torch.Generator().manual_seed(B + K)
+    idx = torch.randint(0, F, (B, K), generator=g)
+    if hot:
+        idx = torch.where(torch.rand(B, K, generator=g) < hot, torch.tensor(F // 3), idx)
+    rbegin, rmap = oracle.csr(idx, F)
+    for _ in range(2):
+        rc, begin, mp = abi.csr_build(idx.to(DEV), F)
+        torch.cuda.synchronize()
+        assert rc == 0
+        np.testing.assert_array_equal(abi.widen_u32(begin).cpu().numpy(), rbegin.astype(np.int64))
+        np.testing.assert_array_equal(abi.widen_u32(mp).cpu().numpy(), rmap.astype(np.int64))
+    lib = _lib.load()
+    D = 8
+    W, v, b, t = (torch.zeros(n, device=DEV) for n in ((F, D), (B, K), (D,), (B, D)))
+    sh = abi.shape_of(idx, W, v)
+    nbytes = lib.flexsae_hier_fwd_bwd_workspace_bytes(ctypes.byref(sh), 0)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    loss, dv, db, dW = (torch.empty(n, device=DEV) for n in (1, (B, K), (D,), (F, D)))
+    p = abi.ptr
+    assert lib.flexsae_hier_fwd_bwd(ctypes.byref(sh), p(idx.to(DEV)), p(W), p(v), p(b), p(t), p(loss), p(dW), _lib.F32, p(dv),
+                                    p(db), p(ws), nbytes, 0, None, abi.stream()) == 0
+    stats = torch.zeros(3, dtype=torch.int32, device=DEV)
+    assert lib.flexsae_hier_pair_stats(ctypes.byref(sh), p(ws), p(stats), abi.stream()) == 0
+    n = np.bincount(idx.flatten().numpy(), minlength=F)
+    long = n[n > 64]
+    assert stats.tolist() == [len(long), int(((long + 63) // 64).sum()), int((n == 0).sum())]
