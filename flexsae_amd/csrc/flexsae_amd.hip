@@ -814,11 +814,11 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, sc.lists.ctrl,
                        sc.lists.empty_list, dW, D);
   // In the training step the second step of a slice's hot latents travels with the next slice's
-  // training-step launch (a gradient of the weight's own dtype only: that is what that kernel writes);
-  // the last slice's gets a launch of its own.
+  // training-step launch (a gradient of CarriedGrad's type only: that is what that kernel writes; a launch
+  // of its own costs 4.7 us a slice); the last slice's gets one.
   HotFinalize pending = {};
   HotBlockFinalize pending_hot = {};
-  const bool fold = std::is_same<GT, WT>::value && train != nullptr && do_sweep && do_reduce;
+  const bool fold = std::is_same<GT, typename CarriedGrad<WT>::type>::value && train != nullptr && do_sweep && do_reduce;
   int slice_no = 0;
   for (int64_t col0 = 0; col0 < s->D; col0 += slice_w, ++slice_no) {
     const int64_t cols = (d_used - col0) < slice_w ? (d_used - col0) : slice_w;

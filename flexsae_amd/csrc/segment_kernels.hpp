@@ -242,8 +242,9 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     }
     const int64_t n_items = n_groups * pps;
     const int64_t item_stride = static_cast<int64_t>(gridDim.x - n_long_blocks) * kGroupsPerBlock;
-    for (int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock; item0 < n_items;
-         item0 += item_stride) {
+    int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock;
+    if (item0 >= n_items) return;
+    do {
       int64_t fb;
       int t;
       if (pps_shift >= 0) {  // pps is a power of two (the usual slice widths): shifts only
@@ -360,7 +361,11 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
           }
         }
       }
-    }
+      // (without the lists the grid covers every item: no loop around the short body, whose loads would wait for
+      // the loop's bookkeeping; 131072 latents of 64 fp32 columns, four rows each: 27.6 us looped, 26.8 not)
+      if constexpr (G == 1) return;
+      item0 += item_stride;
+    } while (item0 < n_items);
     return;
   }
   // Long latents: one wavefront per (64-row chunk, piece); its four groups take every fourth row
@@ -527,6 +532,17 @@ __device__ __forceinline__ void hot_finalize_run(const HotFinalize &h, unsigned 
     seg_long_finalize_body<GT, 2, 8>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units,
                                      h.col0, h.slice_w, h.D, block, h.n_blocks);
 }
+
+// Gradient type of the finalize work that a training-step launch carries: the type the package asks for, the
+// weight's own, or fp32 for fp16 weights (whose unit gradient would underflow).
+template <typename WT>
+struct CarriedGrad {
+  using type = WT;
+};
+template <>
+struct CarriedGrad<f16_t> {
+  using type = float;
+};
 
 template <typename GT>
 __global__ __launch_bounds__(256) void hot_finalize_kernel(HotFinalize h) {
