@@ -312,15 +312,14 @@ def main():
     hot = bool(fused and not staged and flex.ops._use_hot_latents(B, K, F, D, dtype, dev))
     # ... and whether shapes with few pairs per latent reduce without the row-count list
     dense = bool(fused and not staged and flex.ops._use_dense_latents(B, K, F, D, dtype, dev))
-    HOTF = (_lib.BWD_HOT_LATENTS if hot else 0) | (_lib.BWD_DENSE_LATENTS if dense else 0)
+    HOTF = (flex.ops._hot_flags(B, D, dev) if hot else 0) | (_lib.BWD_DENSE_LATENTS if dense else 0)
     if hot:
         slice_cols = flex.ops._hot_slice_cols(B, slice_cols, dev)
     tile = 64 * (4 if D % 4 == 0 else 2 if D % 2 == 0 else 1)
     d_pad = -(-D // tile) * tile
     if fused:
         # slices are whole training tiles when the reduction can work on 256-byte pieces
-        bws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(sh), slice_cols,
-                                                                   _lib.BWD_HOT_LATENTS if hot else 0)
+        bws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(sh), slice_cols, HOTF)
         train_tile = 64 if (dtype == torch.float32 and K > 64) else 128
         granule = train_tile if D % (16 // p_size) == 0 else tile
     else:

@@ -37,6 +37,8 @@ BWD_HOT_LATENTS = 128
 BWD_HOT_NO_HEADROOM = 512
 BWD_REUSE_HOT_TABLES = 1024
 BWD_DENSE_LATENTS = 2048
+BWD_HOT_BLOCKS_64 = 4096
+BWD_HOT_BLOCKS_32 = 8192
 TOPK_BWD_FP32_RESIDUAL = 256
 
 

@@ -446,7 +446,8 @@ struct HierBwdPlan {
   // chunk table
   bool hot;
   size_t off_hslot, off_hot_ctrl, off_hot_list, off_cand_list, off_cand_state, off_long_cand, off_long2, off_chunk2;
-  size_t n_row_blocks;     // blocks of kHotRowsPerBlock rows
+  int hot_rows;            // rows per block of the accumulator kernel
+  size_t n_row_blocks;     // blocks of that many rows
 };
 
 // Hot-latent accumulators: 16-bit weights of at most 64 steps (one register per row piece, four
@@ -456,7 +457,7 @@ inline bool hot_supported(const flexsae_shape *s) {
          s->D % (s->weight_dtype == FLEXSAE_BF16 ? 8 : 4) == 0 && s->B * s->K < (1LL << 31);
 }
 
-HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false) {
+HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 0) {
   HierBwdPlan p;
   p.vec = (s->D % 4 == 0) ? 4 : (s->D % 2 == 0) ? 2 : 1;
   p.tile = kWave * p.vec;
@@ -479,7 +480,9 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false) {
   p.off_sfinal = off;  // S_{b,0} of every row, [B, d_pad] fp32: dbias is its column sum
   off += round_up(p.n_rows * static_cast<size_t>(p.d_pad) * 4, kAlign);
   p.off_colsum = off;  // partial column sums, [ceil(B/64), D] fp32
-  off += round_up(static_cast<size_t>(ceil_div(s->B, kColsumRows)) * static_cast<size_t>(s->D) * 4, kAlign);
+  // (with hot latents one per row block, however small the flags make those)
+  off += round_up(static_cast<size_t>(ceil_div(s->B, hot ? kHotMinRowsPerBlock : kColsumRows)) * static_cast<size_t>(s->D) * 4,
+                  kAlign);
   p.off_loss = off;
   p.n_loss_partials = p.n_rows * static_cast<size_t>(p.d_pad / 64 + 1);
   off += round_up(p.n_loss_partials * 4, kAlign);
@@ -489,7 +492,8 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false) {
   const int64_t tt = train_tile_cols(s);
   off += round_up(static_cast<size_t>(p.d_pad / (p.tile < tt ? p.tile : tt)) * p.n_pairs * 4, kAlign);
   p.hot = hot;
-  p.n_row_blocks = static_cast<size_t>(ceil_div(s->B, kHotRowsPerBlock));
+  p.hot_rows = kHotRowsPerBlock >> hot_halvings(flags);
+  p.n_row_blocks = static_cast<size_t>(ceil_div(s->B, p.hot_rows));
   if (hot) {
     const size_t n_long_max = p.n_pairs / 65 + 2;
     p.off_hslot = off;
@@ -634,7 +638,7 @@ void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const 
                              float *dvals, float *colsum_part, float *loss_partial, int *status_flag,
                              int64_t cols, int col0, int slice_w, hipStream_t st, HotFinalize fin,
                              const HotBlockFinalize &hfin, uint32_t *ctrl, float *hot_partial,
-                             int n_row_blocks, int headroom) {
+                             int hot_rows, int n_row_blocks, int headroom) {
   if constexpr (sizeof(typename Traits<WT>::store_t) == 2) {
     const int n_tiles = static_cast<int>(cols / kHotCols);
     const unsigned grid = static_cast<unsigned>(n_tiles) * static_cast<unsigned>(n_row_blocks);
@@ -652,7 +656,7 @@ void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const 
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHotThreads), 0, st, indices, weight, vals, s->vals_dtype, ta.bias, \
                        s->bias_dtype, ta.target, s->target_dtype, coef, hslot, P, dvals, colsum_part,           \
                        loss_partial, status_flag, s->B, n_tiles, n_row_blocks, col0, slice_w,                   \
-                       static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, fin, hfin); \
+                       static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, hot_rows / kHotWaves, fin, hfin); \
   } while (0)
     if (s->K <= 16) {
       FLEXSAE_TRAIN_HOT(16);
@@ -828,7 +832,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                                       reinterpret_cast<const uint32_t *>(ws + pl.off_hslot), P, dv_part, colsum_part,
                                       reinterpret_cast<float *>(ws + pl.off_loss), status_flag, cols,
                                       static_cast<int>(col0), sw, st, pending, pending_hot, hot_ctrl,
-                                      hot_partial[slice_no & 1], static_cast<int>(pl.n_row_blocks), hot_headroom);
+                                      hot_partial[slice_no & 1], pl.hot_rows, static_cast<int>(pl.n_row_blocks), hot_headroom);
       pending = HotFinalize{};
       pending_hot = HotBlockFinalize{};
     } else if (train && do_sweep) {
@@ -898,7 +902,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                        static_cast<int64_t>(d_pad), D, colsum_part, n_colsum_blocks, dv_part,
                        static_cast<int>(d_used / (train ? train_tile_cols(s) : kWave * sweep_vec)), s->B * s->K, dvals);
   }
-  // (one partial per block of kHotRowsPerBlock rows from the hot-latent step, else per chunk of kColsumRows)
+  // (one partial per row block of the hot-latent step, else per chunk of kColsumRows)
   hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(D, 256))), dim3(256), 0, st,
                      colsum_part, hot ? static_cast<int>(pl.n_row_blocks) : n_chunks, D,
                      static_cast<const float *>(nullptr), 1.0f, dbias);
@@ -1219,7 +1223,7 @@ size_t flexsae_hier_bwd_workspace_bytes(const flexsae_shape *s, int64_t slice_co
 size_t flexsae_hier_fwd_bwd_workspace_bytes_flags(const flexsae_shape *s, int64_t slice_cols, int flags) {
   if (check_shape(s) != FLEXSAE_OK || !train_supported(s)) return 0;
   const bool hot = (flags & FLEXSAE_BWD_HOT_LATENTS) && hot_supported(s);
-  const HierBwdPlan pl = plan_hier_bwd(s, hot);
+  const HierBwdPlan pl = plan_hier_bwd(s, hot, flags);
   const int64_t granule = piece_reduce_ok(s, pl, nullptr, s->weight_dtype) ? train_tile_cols(s) : pl.tile;
   int64_t sw = slice_cols <= 0 ? granule : ceil_div(slice_cols, granule) * granule;
   if (sw > pl.d_pad) sw = pl.d_pad;
@@ -1379,7 +1383,7 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   // call and every pointer is aligned for the piece reduction (the workspace layout depends on it)
   const bool hot = (flags & FLEXSAE_BWD_HOT_LATENTS) && hot_supported(s) && !defer_reduce &&
                    piece_reduce_ok(s, plan_hier_bwd(s), (defer_reduce || no_dw) ? nullptr : dW, dW_dtype);
-  const HierBwdPlan pl = plan_hier_bwd(s, hot);  // D % 4 == 0 here, so tiles are 256 columns
+  const HierBwdPlan pl = plan_hier_bwd(s, hot, flags);  // D % 4 == 0 here, so tiles are 256 columns
   if (!aligned(indices, 8) || !aligned(weight, 4 * dtype_size(s->weight_dtype)) ||
       !aligned(vals, dtype_size(s->vals_dtype)) || !aligned(bias, 2 * dtype_size(s->bias_dtype)) ||
       !aligned(target, 2 * dtype_size(s->target_dtype)) || !aligned(loss, 4) ||
@@ -1442,7 +1446,8 @@ int flexsae_hier_sgd_step(const flexsae_shape *s, const int64_t *indices, void *
   return hier_fwd_bwd_impl(s, indices, weight, vals, bias, target, loss, weight, s->weight_dtype, dvals, dbias,
                            workspace, workspace_bytes,
                            flags & (FLEXSAE_BWD_REUSE_PAIR_LIST | FLEXSAE_BWD_HOT_LATENTS | FLEXSAE_BWD_REUSE_HOT_TABLES |
-                                    FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS),
+                                    FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS | FLEXSAE_BWD_HOT_BLOCKS_64 |
+                                    FLEXSAE_BWD_HOT_BLOCKS_32),
                            status_flag, stream, step);
 }
 

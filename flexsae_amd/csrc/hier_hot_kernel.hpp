@@ -3,9 +3,9 @@
 // A latent that many batch rows select (skewed indices: a few latents in most rows) receives one
 // contribution per selecting row; staged like the others, each of them is written to memory and
 // read back.  Here the kHotMax most frequent latents of the batch get accumulators in the LDS
-// instead: a block walks kHotRowsPerBlock rows of one 128-column tile, adds the contributions of
+// instead: a block walks up to kHotRowsPerBlock rows of one 128-column tile, adds the contributions of
 // marked pairs into its accumulators, and writes one partial sum per (block, hot latent) at the
-// end -- kHotRowsPerBlock times fewer bytes through the memory fabric for those pairs.
+// end -- that many times fewer bytes through the memory fabric for those pairs.
 //
 // The accumulators are 32-bit integers (fixed point with one exponent per block), added with LDS
 // atomics: integer addition is associative, so the sums do not depend on the order in which the
@@ -33,10 +33,16 @@ constexpr int kHotMax = 288;            // accumulator rows in the LDS: 288 * 12
 constexpr int kHotCols = 128;           // columns per tile (two per lane)
 constexpr int kHotThreads = 1024;       // one block per compute unit: its LDS holds the accumulators
 constexpr int kHotWaves = kHotThreads / kWave;
-constexpr int kHotRowsPerBlock = 128;   // fixed: the grouping of the sums must not depend on the slice width
+// Rows per block: at most 128 (eight per wavefront), halved up to three times by the caller's flags for
+// batches whose blocks of 128 rows leave compute units without a block.  Never by the slice width: the
+// grouping of the sums must not depend on it.
+// (B = 1024, D = 1024, K = 64, Zipf indices: 64 blocks of 128 rows 118 us, 256 blocks of 32 rows 46 us.)
+constexpr int kHotRowsPerBlock = 128;
 constexpr int kHotRowsPerWave = kHotRowsPerBlock / kHotWaves;
-constexpr int kHotRowsLog2 = 7;
-static_assert((1 << kHotRowsLog2) == kHotRowsPerBlock, "log2 of the rows per block");
+constexpr int kHotMinRowsPerBlock = kHotWaves;
+static_assert(FLEXSAE_BWD_HOT_BLOCKS_64 == 1 << 12 && FLEXSAE_BWD_HOT_BLOCKS_32 == 1 << 13 && kHotRowsPerWave >> 3 == 1,
+              "the two flags count the halvings");
+constexpr int hot_halvings(int flags) { return (flags >> 12) & 3; }
 constexpr uint32_t kHotSlotBit = 0x80000000u;  // marks a pair of a hot latent in hslot[]; the low bits are its accumulator row
 constexpr uint32_t kHotNone = 0xffffffffu;
 constexpr int kHotExpMin = -96;         // exponents are clamped to [kHotExpMin, 127]: 2^(22 - E) stays a normal float
@@ -295,9 +301,9 @@ __global__ __launch_bounds__(256) void hot_block_finalize_kernel(HotBlockFinaliz
 }
 
 // ---- the training-step kernel with hot-latent accumulators ---------------------------------
-// One block of kHotThreads per (row block of kHotRowsPerBlock rows, 128-column tile of the slice):
+// One block of kHotThreads per (row block of 16 * rows_per_wave rows, 128-column tile of the slice):
 // blockIdx = row block * n_tiles + tile, so that with the usual round-robin placement the blocks
-// of one tile share an L2.  Wavefront w walks rows row block * 128 + i * 16 + w, i = 0..7, each
+// of one tile share an L2.  Wavefront w walks rows (row block * rows_per_wave + i) * 16 + w, each
 // exactly like hier_train_kernel (all K gathers at once, forward walk, reverse walk), except that
 // a pair whose hslot has the hot bit adds its contribution to the block's accumulator row instead
 // of storing it.  The leading work of every block is its share of the previous slice's second
@@ -317,7 +323,7 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
     const uint32_t *__restrict__ hslot, void *__restrict__ P, float *__restrict__ dv_part,
     float *__restrict__ colsum_part, float *__restrict__ loss_partial,
     int *status_flag, int64_t B, int n_tiles, int n_row_blocks, int col0, int slice_w, int K, int64_t F, int D,
-    uint32_t *__restrict__ ctrl, float *__restrict__ hot_partial, int headroom, HotFinalize fin,
+    uint32_t *__restrict__ ctrl, float *__restrict__ hot_partial, int headroom, int rows_per_wave, HotFinalize fin,
     HotBlockFinalize hfin) {
   constexpr int VEC = 2;
   using Piece = RowPiece<WT, VEC>;
@@ -371,13 +377,13 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
 
 #pragma unroll 1
   for (int pass = 0; pass < 2; ++pass) {
-    uint32_t todo = pass == 0 ? (1u << kHotRowsPerWave) - 1u : deferred;
+    uint32_t todo = pass == 0 ? (1u << rows_per_wave) - 1u : deferred;
     bool calibrate = pass == 0;
 #pragma unroll 1
     while (todo != 0) {  // uniform
       const int i = __builtin_ctz(todo);
       todo &= todo - 1;
-      const int64_t b = static_cast<int64_t>(rb) * kHotRowsPerBlock + i * kHotWaves + wv;
+      const int64_t b = (static_cast<int64_t>(rb) * rows_per_wave + i) * kHotWaves + wv;
       const bool valid = b < B;  // uniform
       const int64_t pair0 = b * K;
 

@@ -93,6 +93,10 @@ enum {
                                      /* (flexsae_hier_pair_stats counts them).  A pair list     */
                                      /* built under this flag has no such list: REUSE_PAIR_LIST */
                                      /* on it needs the flag again                              */
+  FLEXSAE_BWD_HOT_BLOCKS_64 = 4096,  /* with HOT_LATENTS: blocks of 64 batch rows instead of 128, */
+  FLEXSAE_BWD_HOT_BLOCKS_32 = 8192,  /* of 32, or with both flags of 16: for batches whose blocks */
+                                     /* of 128 rows are fewer than the compute units.  The same */
+                                     /* flags in the workspace query and in every call on it    */
   FLEXSAE_BWD_HOT_NO_HEADROOM = 512, /* NOT PART OF THE STABLE ABI (a test aid): the block      */
                                      /* exponent of the hot-latent accumulators is set 8 bits   */
                                      /* lower than usual, so that most rows take the deferred   */
@@ -245,7 +249,8 @@ size_t flexsae_hier_fwd_bwd_workspace_bytes(const flexsae_shape *shape, int64_t 
  * honoured for `shape`, `_workspace_bytes_flags` is the workspace query for a call with `flags`
  * (the accumulators' block partials take (slice columns / 128) x ceil(B / 128) x 147456 bytes, twice).
  * Slices are best chosen so that (slice columns / 128) x ceil(B / 128) is a multiple of the number
- * of compute units (one block each).
+ * of compute units (one block each); where all of D is too few of them, FLEXSAE_BWD_HOT_BLOCKS_*
+ * make the blocks shorter (their sums are then grouped differently: equal up to rounding).
  */
 int flexsae_hier_hot_latents_supported(const flexsae_shape *shape);
 size_t flexsae_hier_fwd_bwd_workspace_bytes_flags(const flexsae_shape *shape, int64_t slice_cols, int flags);

@@ -88,6 +88,31 @@ def test_hot_latents_match_the_oracle(shape, dtype, zipf):
     assert e_hot <= (4e-3 if dtype == torch.bfloat16 else 2e-5), (e_hot, e_plain)
 
 
+@pytest.mark.parametrize("flags", [_lib.BWD_HOT_BLOCKS_64, _lib.BWD_HOT_BLOCKS_32,
+                                   _lib.BWD_HOT_BLOCKS_64 | _lib.BWD_HOT_BLOCKS_32])
+@pytest.mark.parametrize("B", [16, 300])  # one block of 16 rows; a last block of 12, 12 and 44 rows
+def test_blocks_of_fewer_rows(B, flags):
+    """Blocks of 64, 32 and 16 rows: loss and dvals are the plain step's bits, dW and dbias the oracle's and the
+    same bits for every slice width."""
+    print("[case] hot blocks", B, flags, flush=True)
+    cpu_args = make_inputs(B, 64, 2000 if B > 64 else 90, 384, torch.bfloat16, seed=37, zipf_s=1.1 if B > 64 else None,
+                           w_std=0.3)
+    args = _dev(cpu_args)
+    rc0, loss0, dW0, dv0, db0 = abi.hier_train(*args, dw_dtype=torch.bfloat16, slice_cols=128)
+    outs = []
+    for cols in (128, 384):
+        rc, loss, dW, dv, db, ws = abi.hier_train(*args, dw_dtype=torch.bfloat16, slice_cols=cols, flags=HOT | flags,
+                                                  keep_workspace=True)
+        assert rc0 == 0 and rc == 0
+        assert torch.equal(loss, loss0) and torch.equal(dv, dv0)
+        assert rel_err(db.cpu(), db0.cpu()) <= 2e-6
+        if B > 64:
+            assert abi.hot_stats(*args, ws)[0] > 0 and not torch.equal(dW, dW0)
+        outs.append((dW, db))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    _check_vs_oracle(cpu_args, outs[0][0], dv, outs[0][1], loss, 1e-2)
+
+
 def test_repeated_rows_keep_a_latent_cold():
     """randint indices on few latents: every latent is frequent and nearly every one is repeated
     inside some row, so none may be summed in the accumulators: dW is the plain step's, bit for bit."""
