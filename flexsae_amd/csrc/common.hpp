@@ -426,6 +426,11 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(x, y, acc, false);
 }
 
+// Marks in slot[] the only pair of its latent (problems of fewer than 2^30 pairs; the bits below are the slot).
+// Its contribution is the latent's whole gradient: where it is stored in the gradient's own type, the training step
+// writes it to the gradient itself, and the reductions leave latents of one pair out.
+constexpr uint32_t kSoloSlotBit = 0x40000000u;
+
 // Wave index inside the block as a scalar (uniform) value, so that everything
 // derived from it is addressed through scalar registers.
 __device__ __forceinline__ int wave_in_block() {

@@ -535,7 +535,8 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
   if (have) atomicAdd(&counter[at], 1u);
 }
 
-// One block per bucket.  hslot: a second copy of slot[] (null: none).
+// One block per bucket.  hslot: a second copy of slot[] (null: none).  solo_bit: marks in both the only pair of
+// its latent (0: no marks).
 // Groups of more than kListLong pairs (frequent latents) are placed by walking the bucket's pairs in order:
 // every wavefront takes a run of them, counts its pairs of every such latent, and places them behind those
 // of the wavefronts before it.  The others are gathered in the LDS in any order, and every pair counts
@@ -543,7 +544,7 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
 __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
     const uint32_t *__restrict__ tmp, const uint32_t *__restrict__ table, uint32_t n_chunks, int64_t chunk, int shift,
     int64_t F, uint32_t *__restrict__ begin, uint32_t *__restrict__ map, uint32_t *__restrict__ slot,
-    uint32_t *__restrict__ hslot, PairLists ls) {
+    uint32_t *__restrict__ hslot, uint32_t solo_bit, PairLists ls) {
   constexpr int kWaves = kSortThreads / kWave;
   constexpr int PER = kSortMaxLatents / kSortThreads;
   constexpr uint32_t kRunLatents = kSortCap / kWaves;  // frequent latents counted per wavefront at a time
@@ -740,10 +741,10 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
   }
   append_latents(ls, f0, nlat, [&](uint32_t k) { return cnt[k + 1] - cnt[k]; }, sh);
 
-  auto put = [&](uint32_t place, uint32_t id) {
+  auto put = [&](uint32_t place, uint32_t id, uint32_t mark) {
     map[place] = id;
-    if (slot) slot[id] = place;
-    if (hslot) hslot[id] = place;
+    if (slot) slot[id] = place | mark;
+    if (hslot) hslot[id] = place | mark;
   };
   // frequent latents, kRunLatents of them at a time; where the bucket's list did not fit the LDS but its other
   // pairs do, those are listed on the way
@@ -819,7 +820,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
                                                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0u));
           if (have) {
             const uint32_t place = mine[l] + rank;
-            put(place, id[u]);
+            put(place, id[u], 0u);
             if (rank == 0) mine[l] = place + static_cast<uint32_t>(__popcll(same));
           }
           __builtin_amdgcn_wave_barrier();
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
         for (int u = 0; u < 8; ++u) rank += (x[u] < id) ? 1u : 0u;
       }
       for (; j < len; ++j) rank += (group[j] < id) ? 1u : 0u;
-      put(base + cnt[key] + rank, id);
+      put(base + cnt[key] + rank, id, len == 1 ? solo_bit : 0u);
     });
     k0 = k1;
   }

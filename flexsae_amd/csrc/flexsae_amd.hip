@@ -49,6 +49,7 @@ constexpr int kBlock = 256;              // threads per block of the wave-per-it
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr size_t kAlign = 256;
 constexpr int kBwdSgdUpdate = 1 << 20;  // internal flag of the slice loop: dW is the weight matrix, updated in place
+constexpr int kBwdSolo = 1 << 22;       // internal flag of the slice loop: slot[] marks the only pairs of their latents
 constexpr int kBwdHot = 1 << 21;        // internal flag of the slice loop: hot latents are accumulated in the LDS
 constexpr unsigned kLongBlocks = 1024;    // leading blocks of a reduction launch that serve hot latents
 constexpr int64_t kListBlocks = 8192;     // blocks of a reduction launch that work from the lists of latents
@@ -358,7 +359,7 @@ void launch_pair_lists(const uint32_t *begin, int64_t F, const PairLists &lists,
 // `hslot`); fills the lists of sc.lists.
 void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, uint32_t *begin,
                       uint32_t *map, uint32_t *slot, uint32_t *hslot, const CsrScratch &sc, int *status_flag,
-                      hipStream_t st) {
+                      hipStream_t st, uint32_t solo_bit = 0u) {
   const int64_t n_pairs = B * K;
   const CsrPlan &pl = sc.plan;
   if (pl.bucketed) {
@@ -367,7 +368,7 @@ void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
                        pl.shift, pl.n_buckets, pl.n_bits, pl.chunk, pl.n_chunks, sc.table, sc.tmp, sc.lists.ctrl,
                        status_flag);
     hipLaunchKernelGGL(csr_bucket_sort_kernel, dim3(pl.n_buckets), dim3(kSortThreads), 0, st, sc.tmp, sc.table,
-                       pl.n_chunks, pl.chunk, pl.shift, F, begin, map, slot, hslot, sc.lists);
+                       pl.n_chunks, pl.chunk, pl.shift, F, begin, map, slot, hslot, solo_bit, sc.lists);
     return;
   }
   hipLaunchKernelGGL(csr_init_kernel, dim3(grid_for(F + 1, 256, 4096)), dim3(256), 0, st, begin, F + 1,
@@ -554,6 +555,10 @@ struct TrainArgs {
   double inv_count;         // 1 / (B*K*D)
 };
 
+// what of slot[] is the slot: all of it, or all but the mark of a latent's only pair
+inline bool solo_marks(const flexsae_shape *s) { return s->B * s->K < (1LL << 30); }
+inline uint32_t slot_mask(const flexsae_shape *s) { return solo_marks(s) ? kSoloSlotBit - 1u : 0xffffffffu; }
+
 // largest K the training-step kernel holds in registers
 inline bool train_supported(const flexsae_shape *s) { return s->D % 4 == 0 && s->K <= 256; }
 
@@ -581,7 +586,7 @@ template <typename WT, typename PT, int KMAX, int VEC = 2>
 void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int64_t *indices,
                          const void *weight, const void *vals, float coef, const uint32_t *slot, void *P,
                          float *dvals, float *s_final, int d_pad, float *loss_partial, int *status_flag,
-                         int64_t cols, int col0, int slice_w, hipStream_t st, const HotFinalize &fin) {
+                         int64_t cols, int col0, int slice_w, hipStream_t st, const HotFinalize &fin, void *dW_solo) {
   constexpr int LDSROWS = train_lds_rows<WT, KMAX, VEC>();
   const int64_t n_items = s->B * (cols / (kWave * VEC));
   // K == KMAX (the usual powers of two) runs the variant without per-step bound tests, part of its
@@ -595,7 +600,7 @@ void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int6
   hipLaunchKernelGGL(kernel, dim3(fin.n_blocks + static_cast<unsigned>(ceil_div(n_items, kWavesPerBlock))), dim3(kBlock),
                      0, st, indices, weight, vals, s->vals_dtype, ta.bias, s->bias_dtype, ta.target, s->target_dtype,
                      coef, slot, P, dvals, s_final, d_pad, loss_partial, status_flag, n_items, s->B, col0,
-                     slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), fin);
+                     slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), slot_mask(s), dW_solo, fin);
 }
 
 template <typename WT, typename PT>
@@ -603,10 +608,10 @@ void launch_train_kernel_k(const flexsae_shape *s, const TrainArgs &ta, const in
                            const void *weight, const void *vals, float coef, const uint32_t *slot, void *P,
                            float *dvals, float *s_final, int d_pad, float *loss_partial,
                            int *status_flag, int64_t cols, int col0, int slice_w, hipStream_t st,
-                           const HotFinalize &fin) {
+                           const HotFinalize &fin, void *dW_solo) {
 #define FLEXSAE_TRAIN(KM)                                                                              \
   launch_train_kernel<WT, PT, KM>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,  \
-                                  loss_partial, status_flag, cols, col0, slice_w, st, fin)
+                                  loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo)
   // (the fp32 16-step instantiation allocates registers badly; 32 covers it)
   if (s->K <= 16 && sizeof(typename Traits<WT>::store_t) == 2) {
     FLEXSAE_TRAIN(16);
@@ -622,10 +627,10 @@ void launch_train_kernel_k(const flexsae_shape *s, const TrainArgs &ta, const in
     }
   } else if (s->K <= 128) {  // fp32 rows of 65..128 steps: one column per lane
     launch_train_kernel<WT, PT, 128, 1>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,
-                                        loss_partial, status_flag, cols, col0, slice_w, st, fin);
+                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo);
   } else {
     launch_train_kernel<WT, PT, 256, 1>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,
-                                        loss_partial, status_flag, cols, col0, slice_w, st, fin);
+                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo);
   }
 #undef FLEXSAE_TRAIN
 }
@@ -638,7 +643,7 @@ void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const 
                              float *dvals, float *colsum_part, float *loss_partial, int *status_flag,
                              int64_t cols, int col0, int slice_w, hipStream_t st, HotFinalize fin,
                              const HotBlockFinalize &hfin, uint32_t *ctrl, float *hot_partial,
-                             int hot_rows, int n_row_blocks, int headroom) {
+                             int hot_rows, int n_row_blocks, int headroom, void *dW_solo) {
   if constexpr (sizeof(typename Traits<WT>::store_t) == 2) {
     const int n_tiles = static_cast<int>(cols / kHotCols);
     const unsigned grid = static_cast<unsigned>(n_tiles) * static_cast<unsigned>(n_row_blocks);
@@ -656,7 +661,8 @@ void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const 
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHotThreads), 0, st, indices, weight, vals, s->vals_dtype, ta.bias, \
                        s->bias_dtype, ta.target, s->target_dtype, coef, hslot, P, dvals, colsum_part,           \
                        loss_partial, status_flag, s->B, n_tiles, n_row_blocks, col0, slice_w,                   \
-                       static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, hot_rows / kHotWaves, fin, hfin); \
+                       static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, hot_rows / kHotWaves, slot_mask(s), \
+                       dW_solo, fin, hfin); \
   } while (0)
     if (s->K <= 16) {
       FLEXSAE_TRAIN_HOT(16);
@@ -697,7 +703,7 @@ template <typename PT, typename GT, int VEC>
 void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, const PairLists &ls,
                        const void *P, float *partial, void *dW, const float *dw_scale, int64_t F, int tps,
                        int col0, int sw, int D, hipStream_t st, int piece_cols = 0, int64_t cols = 0, int64_t n_pairs = 0,
-                       int update = 0, bool by_count = false, HotFinalize *defer = nullptr) {
+                       int update = 0, bool by_count = false, HotFinalize *defer = nullptr, int skip_solo = 0) {
   // the second step of the hot latents: launched here, or handed back through `defer` for the next
   // training-step launch to carry
   auto finalize = [&](int mode, int units) {
@@ -720,7 +726,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
 #define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS)                                                                          \
   hipLaunchKernelGGL((seg_reduce_piece_kernel<PT, GT, FLEXSAE_PIECE_U, G>),                                        \
                      dim3(kLongBlocks + static_cast<unsigned>(N_BLOCKS)), dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, \
-                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, ls)
+                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, skip_solo, ls)
     constexpr int64_t kGroups = kBlock / kPieceLanes;
     if (by_count) {
       // work items: one per latent with nine rows or more, one per four others of a class
@@ -743,7 +749,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
     const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * rtps, kWavesPerBlock));
     hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, RV, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
                        dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale,
-                       F, kLongBlocks, rtps, col0, sw, D);
+                       F, kLongBlocks, rtps, col0, sw, D, skip_solo);
     static_assert(RV == 2 || !kCanNarrow, "the narrow reduction works on tiles of 128 columns");
     finalize(3, rtps);
     return;
@@ -751,7 +757,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
   const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * tps, kWavesPerBlock));
   hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, VEC, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
                      dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale, F,
-                     kLongBlocks, tps, col0, sw, D);
+                     kLongBlocks, tps, col0, sw, D, skip_solo);
   if constexpr (VEC == 4) {
     finalize(2, tps);
   } else {
@@ -823,6 +829,11 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   HotFinalize pending = {};
   HotBlockFinalize pending_hot = {};
   const bool fold = std::is_same<GT, typename CarriedGrad<WT>::type>::value && train != nullptr && do_sweep && do_reduce;
+  // Only pairs of their latents write dW themselves where its type is the contributions' own.
+  void *const dW_solo = (flags & kBwdSolo) && std::is_same<GT, PT>::value && train != nullptr && do_sweep && do_reduce &&
+                                !update && !dw_scale
+                            ? dW
+                            : nullptr;
   int slice_no = 0;
   for (int64_t col0 = 0; col0 < s->D; col0 += slice_w, ++slice_no) {
     const int64_t cols = (d_used - col0) < slice_w ? (d_used - col0) : slice_w;
@@ -832,13 +843,14 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                                       reinterpret_cast<const uint32_t *>(ws + pl.off_hslot), P, dv_part, colsum_part,
                                       reinterpret_cast<float *>(ws + pl.off_loss), status_flag, cols,
                                       static_cast<int>(col0), sw, st, pending, pending_hot, hot_ctrl,
-                                      hot_partial[slice_no & 1], pl.hot_rows, static_cast<int>(pl.n_row_blocks), hot_headroom);
+                                      hot_partial[slice_no & 1], pl.hot_rows, static_cast<int>(pl.n_row_blocks), hot_headroom,
+                                      dW_solo);
       pending = HotFinalize{};
       pending_hot = HotBlockFinalize{};
     } else if (train && do_sweep) {
       launch_train_kernel_k<WT, PT>(s, *train, indices, weight, vals, coef, slot, P, dv_part, s_final, d_pad,
                                     reinterpret_cast<float *>(ws + pl.off_loss), status_flag, cols,
-                                    static_cast<int>(col0), sw, st, pending);
+                                    static_cast<int>(col0), sw, st, pending, dW_solo);
       pending = HotFinalize{};
     } else if (do_sweep) {
 #define FLEXSAE_SWEEP(SV)                                                                                      \
@@ -846,7 +858,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                      dim3(static_cast<unsigned>(ceil_div(s->B * (cols / (kWave * SV)), kWavesPerBlock))),      \
                      dim3(kBlock), 0, st, indices, weight, vals, s->vals_dtype, resid, grad_out, coef, slot, P, \
                      dv_part, s_final, d_pad, status_flag, s->B * (cols / (kWave * SV)), s->B,                 \
-                     static_cast<int>(col0), sw, K, s->F, D)
+                     static_cast<int>(col0), sw, K, s->F, D, slot_mask(s))
       if (sweep_vec == VEC) {
         FLEXSAE_SWEEP(VEC);
       } else if (sweep_vec == (VEC >= 2 ? VEC / 2 : 1)) {
@@ -867,7 +879,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
         piece != 0 && (update || cols % pl.tile != 0 || sparse_latents(s, flags) || cache_sized);
     launch_seg_reduce<PT, GT, VEC>(narrow_reduce, begin, reduce_long, sc.lists, P, partial, dW, dw_scale, s->F, tps,
                                    static_cast<int>(col0), sw, D, st, by_pieces ? piece : 0, cols, s->B * s->K, update,
-                                   sparse, fold ? &pending : nullptr);
+                                   sparse, fold ? &pending : nullptr, dW_solo != nullptr);
     if (hot) {
       // the block partials of the slice's hot latents are added up by the next training-step launch
       // (they live in the buffer that launch does not write), or here
@@ -1407,9 +1419,13 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   uint32_t *map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
   const CsrScratch sc = carve_hier_lists(s, pl, ws);
   const bool build = !(flags & FLEXSAE_BWD_REUSE_PAIR_LIST);
+  // Latents of one pair: their contribution is their gradient (kSoloSlotBit), where this call builds the list that
+  // marks them.  (Whatever the number of pairs per latent: see hier_train_kernel.)
+  const bool solo = build && !defer_reduce && !no_dw && !sgd_step && solo_marks(s) && sc.plan.bucketed;
   if (build)
     csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot),
-                     hot ? reinterpret_cast<uint32_t *>(ws + pl.off_hslot) : nullptr, sc, status_flag, st);
+                     hot ? reinterpret_cast<uint32_t *>(ws + pl.off_hslot) : nullptr, sc, status_flag, st,
+                     solo ? kSoloSlotBit : 0u);
   if (hot && !((flags & FLEXSAE_BWD_REUSE_PAIR_LIST) && (flags & FLEXSAE_BWD_REUSE_HOT_TABLES)))
     build_hot_tables(s, pl, ws, sc, build, st);
   const double count = static_cast<double>(s->B) * static_cast<double>(s->K) * static_cast<double>(s->D);
@@ -1421,7 +1437,8 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
                           no_dw ? s->weight_dtype : dW_dtype, dvals, dbias, ws,
                           (flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE |
                                     FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS)) |
-                              (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : 0) | (hot ? kBwdHot : 0),
+                              (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : 0) | (hot ? kBwdHot : 0) |
+                              (solo ? kBwdSolo : 0),
                           status_flag, st, &ta, piece ? static_cast<int>(piece_cols(pl)) : 0);
   return launch_status();
 }
@@ -1435,7 +1452,7 @@ int flexsae_hier_fwd_bwd(const flexsae_shape *s, const int64_t *indices, const v
                          void *dW, int dW_dtype, float *dvals, float *dbias, void *workspace,
                          size_t workspace_bytes, int flags, int *status_flag, void *stream) {
   return hier_fwd_bwd_impl(s, indices, weight, vals, bias, target, loss, dW, dW_dtype, dvals, dbias, workspace,
-                           workspace_bytes, flags & ~(kBwdSgdUpdate | kBwdHot), status_flag, stream, nullptr);
+                           workspace_bytes, flags & ~(kBwdSgdUpdate | kBwdHot | kBwdSolo), status_flag, stream, nullptr);
 }
 
 int flexsae_hier_sgd_step(const flexsae_shape *s, const int64_t *indices, void *weight, const void *vals,

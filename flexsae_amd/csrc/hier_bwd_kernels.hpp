@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
     const float *__restrict__ grad_out, float coef, const uint32_t *__restrict__ slot,
     void *__restrict__ P, float *__restrict__ dv_part, float *__restrict__ s_final, int s_final_ld,
     int *status_flag, int64_t n_items, int64_t B, int col0, int slice_w, int K, int64_t F,
-    int D) {
+    int D, uint32_t slot_mask) {
   const int lane = lane_id();
   const int64_t item = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
   if (item >= n_items) return;  // uniform per wavefront
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
     if (kk < K) {
       my_idx = indices[pair0 + kk];
       my_val = load_scalar(vals, vals_dtype, pair0 + kk);
-      my_slot = static_cast<int>(slot[pair0 + kk]);
+      my_slot = static_cast<int>(slot[pair0 + kk] & slot_mask);  // (without the mark of a latent's only pair)
     }
     if (static_cast<uint64_t>(my_idx) >= static_cast<uint64_t>(F)) {
       if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);

@@ -74,6 +74,13 @@ struct RowPiece<f16_t, 2> {
 // when all of P is written before any of it is read back (it is far larger than the caches);
 // when P is one slice that the reduction reads right after this launch, plain stores leave part
 // of it in the memory-side cache and the pair of launches is faster.
+// dW (of PT's type, or null): the contribution of a pair that is its latent's only one (kSoloSlotBit in slot[])
+// goes to the latent's row of dW and not to P, and the reduction leaves those latents out: at two pairs per
+// latent, uniform, 13.5 % of the contributions are neither written nor read back (B=4096, K=32, F=65536, D=2304
+// bf16: the step 428 -> 410 us, fp16 812 -> 772; Zipf indices, B=8192, K=64, F=262144, D=4096: 2253 -> 2149).
+// The lanes form the destination of every step (lane k: step k) as a 64-bit address: a store costs two lane reads and
+// no address arithmetic, which is no slower than one lane read and a scalar multiplication where no latent has
+// a single pair (K=256 of 65536 latents, D=1024: 1192 -> 1172 us).
 template <typename WT, typename PT, int KMAX, bool FULL, bool STREAM, int VEC, int LDSROWS = 0>
 __global__ __launch_bounds__(256) void hier_train_kernel(
     const int64_t *__restrict__ indices, const void *__restrict__ weight,
@@ -81,7 +88,8 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
     const void *__restrict__ target, int target_dtype, float coef,
     const uint32_t *__restrict__ slot, void *__restrict__ P, float *__restrict__ dv_part,
     float *__restrict__ s_final, int s_final_ld, float *__restrict__ loss_partial,
-    int *status_flag, int64_t n_items, int64_t B, int col0, int slice_w, int K, int64_t F, int D, HotFinalize fin) {
+    int *status_flag, int64_t n_items, int64_t B, int col0, int slice_w, int K, int64_t F, int D, uint32_t slot_mask,
+    void *__restrict__ dW, HotFinalize fin) {
   using Piece = RowPiece<WT, VEC>;
   using raw_t = typename Piece::raw_t;
   using S_t = typename Traits<WT>::store_t;
@@ -161,6 +169,21 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
       my_val[c] = 0.f;
     }
     my_row[c] = static_cast<int>(idx);
+  }
+  // where the step's contribution goes, the first column of the slice
+  uint32_t dst_lo[KC], dst_hi[KC];
+  {
+    constexpr uint32_t kElem = sizeof(typename Traits<PT>::store_t);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const uint32_t sl = static_cast<uint32_t>(my_slot[c]);
+      const bool solo = dW && (sl & ~slot_mask) != 0;
+      const uint64_t base = solo ? reinterpret_cast<uint64_t>(dW) + static_cast<uint64_t>(col0) * kElem : reinterpret_cast<uint64_t>(P);
+      const uint64_t at = base + static_cast<uint64_t>(solo ? static_cast<uint32_t>(my_row[c]) : sl & slot_mask) *
+                                     ((solo ? static_cast<uint32_t>(D) : static_cast<uint32_t>(slice_w)) * kElem);
+      dst_lo[c] = static_cast<uint32_t>(at);
+      dst_hi[c] = static_cast<uint32_t>(at >> 32);
+    }
   }
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
@@ -247,7 +270,8 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
 #pragma unroll
   for (int i = 0; i < VEC; ++i) S[i] = 0.f;
   const int kb_rev = k_bound();
-  const uint32_t p_row_bytes = static_cast<uint32_t>(slice_w) * sizeof(typename Traits<PT>::store_t);
+  // (a row of dW ends at column D; a row of P may end there too, its padding columns are read by nobody)
+  const uint32_t dst_row_bytes = static_cast<uint32_t>(slice_w < D - col0 ? slice_w : D - col0) * sizeof(typename Traits<PT>::store_t);
   const uint32_t p_lane_bytes = static_cast<uint32_t>(pc) * sizeof(typename Traits<PT>::store_t);
 #pragma unroll
   for (int k8 = KMAX - 8; k8 >= 0; k8 -= 8) {
@@ -269,7 +293,6 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
         dots[u] = 0.f;
         if (FULL || k < kb_rev) {  // uniform
           const float v = bcast_f32(my_val[k / kWave], k % kWave);
-          const uint32_t prow = static_cast<uint32_t>(bcast_i32(my_slot[k / kWave], k % kWave));
           // Without this the compiler reuses the unpacked values of the forward walk, which
           // doubles the registers held across the two walks; re-unpacking costs one op per value.
           raw_t rk;
@@ -302,7 +325,11 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
 #pragma unroll
             for (int i = 0; i < VEC; ++i) packed[i] = __float_as_uint(contrib[i]);
           }
-          descriptor_store<sizeof(packed), STREAM>(row_descriptor(P, prow, p_row_bytes), p_lane_bytes, packed);
+          const uint32_t lo = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_lo[k / kWave]), k % kWave));
+          const uint32_t hi = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_hi[k / kWave]), k % kWave));
+          void *const dst = reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo);
+          descriptor_store<sizeof(packed), STREAM>(
+              __builtin_amdgcn_make_buffer_rsrc(dst, 0, static_cast<int>(dst_row_bytes), 0x00020000), p_lane_bytes, packed);
           dots[u] = dot;  // zero where the lane is beyond column D: its w is zero
         }
       }

@@ -112,14 +112,15 @@ __device__ __forceinline__ LongChunk seg_decode_chunk(const uint32_t *__restrict
 // combines the partials in chunk order.  These blocks come first so that hot latents start
 // at once and overlap with the bulk of the work.
 // Remaining blocks: one wavefront per (latent, tile of 64*VEC columns of the slice); latents
-// without rows get zeros; latents with more than kSegChunk rows are skipped.
+// without rows get zeros; latents with more than kSegChunk rows are skipped, and with skip_solo those of
+// one row (the training step has written them: see kSoloSlotBit).
 template <typename PT, typename GT, int VEC, int U>
 __global__ __launch_bounds__(256) void seg_reduce_kernel(
     const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int tps, int col0,
-    int slice_w, int D) {
+    int slice_w, int D, int skip_solo) {
   const int lane = lane_id();
   if (blockIdx.x >= n_long_blocks) {
     // one wavefront per (latent, tile), tiles of a latent adjacent: the launch reads P front to back
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
     const int t = static_cast<int>(item - f * tps);
     const uint32_t s0 = begin[f];
     const uint32_t n = begin[f + 1] - s0;
-    if (n > static_cast<uint32_t>(kSegChunk)) return;
+    if (n > static_cast<uint32_t>(kSegChunk) || (skip_solo && n == 1)) return;
     const int pc = t * (kWave * VEC) + lane * VEC;
     const int d0 = col0 + pc;
     float acc[VEC];
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int pps, int pps_shift, int col0,
-    int slice_w, int D, int update, PairLists lists) {
+    int slice_w, int D, int update, int skip_solo, PairLists lists) {
   using S = typename Traits<PT>::store_t;
   constexpr int EV = 16 / static_cast<int>(sizeof(S));  // columns per lane
   constexpr int kGroupsPerBlock = 256 / kPieceLanes;
@@ -238,7 +239,8 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     if constexpr (G > 1) {
       n_groups = 0;
 #pragma unroll
-      for (int i = 0; i < kClasses; ++i) n_groups += ceil_div_u32(lists.ctrl[kClassCount + i], i < kClassSolo ? G : 1);
+      for (int i = 0; i < kClasses; ++i)
+        n_groups += i == 0 && skip_solo ? 0 : ceil_div_u32(lists.ctrl[kClassCount + i], i < kClassSolo ? G : 1);
     }
     const int64_t n_items = n_groups * pps;
     const int64_t item_stride = static_cast<int64_t>(gridDim.x - n_long_blocks) * kGroupsPerBlock;
@@ -271,7 +273,8 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
           s0 = begin[f];
           n = begin[f + 1] - s0;
         }
-        const bool mine = f < F && n <= static_cast<uint32_t>(kSegChunk);  // longer ones: chunked below
+        // longer ones: chunked below
+        const bool mine = f < F && n <= static_cast<uint32_t>(kSegChunk) && !(skip_solo && n == 1);
         accumulate(s0, mine ? static_cast<int>(n) : 0, 1, pc, acc);
         if (scale) {
 #pragma unroll
@@ -296,7 +299,7 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
           const int64_t n_cls = static_cast<int64_t>(lists.ctrl[kClassCount + i]);
           const int per = i < kClassSolo ? G : 1;
           const int64_t groups = ceil_div_u32(lists.ctrl[kClassCount + i], per);
-          if (at >= 0 && at < groups) {
+          if (at >= 0 && at < groups && !(i == 0 && skip_solo)) {
             list = lists.cls_list[i] + at * per;
             const int64_t left = n_cls - at * per;
             count = left < per ? static_cast<int>(left) : per;

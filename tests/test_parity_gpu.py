@@ -1100,3 +1100,54 @@ def test_pair_list_pieces_and_lists(shape):
     n = np.bincount(idx.flatten().numpy(), minlength=F)
     long = n[n > 64]
     assert stats.tolist() == [len(long), int(((long + 63) // 64).sum()), int((n == 0).sum())]
+
+
+ONLY_PAIR_SHAPES = [
+    (torch.bfloat16, (70, 64, 3000, 264)),   # K of the full kernel, a ragged last tile
+    (torch.bfloat16, (77, 50, 2800, 520)),   # K below the kernel's bound
+    (torch.bfloat16, (40, 128, 6000, 256)),
+    (torch.bfloat16, (19, 200, 3000, 128)),
+    (torch.bfloat16, (70, 16, 9000, 136)),   # most latents without a pair
+    (torch.float16, (70, 32, 1500, 132)),    # fp32 contributions and gradient
+    (torch.float32, (70, 32, 1500, 132)),
+    (torch.float32, (20, 100, 2000, 68)),    # one column per lane
+    (torch.float32, (9, 256, 900, 192)),
+]
+
+
+@pytest.mark.parametrize("dtype,shape,hot", [(d, s, h) for d, s in ONLY_PAIR_SHAPES for h in (False, True)
+                                             if not h or (d != torch.float32 and s[1] <= 64)])
+def test_only_pairs_written_by_the_walk(dtype, shape, hot):
+    """Contributions that are their latent's whole gradient go to dW without being staged where the call
+    builds its pair list, and are staged where it reuses one: the same bits either way, for several slice widths,
+    with repeated and out-of-range indices among them; and the oracle's."""
+    B, K, F, D = shape
+    _announce("only pairs", dtype, shape, hot)
+    cpu = list(make_inputs(B, K, F, D, dtype, seed=51, w_std=0.3))
+    if hot:
+        cpu[0][:, 0] = 5  # a latent in every row
+        assert B > 64
+    cpu[0][1, 1] = cpu[0][1, 2] = F - 1  # twice in a row
+    args = _to_dev(cpu)
+    dw_dtype = torch.float32 if dtype == torch.float16 else dtype
+    flags = _lib.BWD_HOT_LATENTS if hot else 0
+    for cols in (128, 1024):
+        for dense in (0, _lib.BWD_DENSE_LATENTS):
+            rc, *got, ws = abi.hier_train(*args, dw_dtype=dw_dtype, slice_cols=cols, flags=flags | dense, keep_workspace=True)
+            assert rc == 0
+            rc, *again = abi.hier_train(*args, dw_dtype=dw_dtype, slice_cols=cols, workspace=ws,
+                                        flags=flags | dense | _lib.BWD_REUSE_PAIR_LIST)
+            assert rc == 0
+            for a, c in zip(got, again):
+                assert torch.equal(a, c)
+    _, rW, rv, _ = oracle.loss_grads(oracle.HIER, *cpu)
+    check_gradient("dW", got[1], rW, dw_dtype, 1e-2 if dtype == torch.bfloat16 else 1e-4)
+    check_gradient("dvals", got[2], rv, torch.float32, 1e-2 if dtype == torch.bfloat16 else 1e-4)
+    # an index out of range is flagged and adds nothing, wherever latent 0's gradient is formed
+    bad = args[0].clone()
+    bad[0, 0] = F
+    bad[bad == 0] = 1
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    rc, _, dW, _, _ = abi.hier_train(bad, *args[1:], dw_dtype=dw_dtype, flag=flag, flags=flags)
+    assert rc == 0 and int(flag) == _lib.FLAG_INDEX_RANGE
+    assert not dW[0].any()
