@@ -123,6 +123,35 @@ __device__ __forceinline__ void store_vec(void *base, int64_t off, const float (
   }
 }
 
+// The same where rows may end inside the vector and start anywhere: the first `left` elements are stored.  dwords
+// (uniform): every row starts at a multiple of four bytes, which is all that a vector access to memory asks for.
+template <typename T, int VEC, bool NT = false>
+__device__ __forceinline__ void store_vec_upto(void *base, int64_t off, const float (&x)[VEC], int left, bool dwords) {
+  using S = typename Traits<T>::store_t;
+  constexpr int kWords = VEC * static_cast<int>(sizeof(S)) / 4;
+  static_assert(kWords * 4 == VEC * static_cast<int>(sizeof(S)), "whole dwords");
+  S *p = static_cast<S *>(base) + off;
+  if (dwords && left >= VEC) {
+    typedef uint32_t words_t __attribute__((ext_vector_type(kWords), aligned(4)));
+    words_t v;
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) {
+      if constexpr (Traits<T>::dtype == FLEXSAE_F32)
+        v[i] = __float_as_uint(x[i]);
+      else if constexpr (Traits<T>::dtype == FLEXSAE_BF16)
+        v[i] = f32x2_to_bf16x2_bits(x[2 * i], x[2 * i + 1]);
+      else
+        v[i] = static_cast<uint32_t>(f32_to_f16_bits(x[2 * i])) | (static_cast<uint32_t>(f32_to_f16_bits(x[2 * i + 1])) << 16);
+    }
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<words_t *>(p));
+    else *reinterpret_cast<words_t *>(p) = v;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    if (i < left) p[i] = Traits<T>::down(x[i]);
+}
+
 // One element of a tensor whose dtype is only known at run time (vals, bias, target:
 // small tensors next to the gathered weight rows).
 __device__ __forceinline__ float load_scalar(const void *base, int dtype, int64_t i) {

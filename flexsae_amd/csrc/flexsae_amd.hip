@@ -695,6 +695,9 @@ size_t hier_bwd_bytes(const HierBwdPlan &p, int64_t slice_w) {
          (p.hot ? 2 * hier_hot_partial_bytes(p, slice_w) : 0);
 }
 
+// every row starts at a multiple of four bytes
+inline int rows_on_dwords(const void *rows, int64_t D, size_t elem) { return aligned(rows, 4) && D * elem % 4 == 0; }
+
 // Segment reduction of one slice plus the finalize step of its hot latents.  fp32 contributions
 // are read 16 bytes per lane (256-column tiles), or, when `narrow`, 8 bytes per lane (128-column
 // tiles, twice the wavefronts): faster once a latent has about four rows or more, slower for
@@ -704,10 +707,11 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
                        const void *P, float *partial, void *dW, const float *dw_scale, int64_t F, int tps,
                        int col0, int sw, int D, hipStream_t st, int piece_cols = 0, int64_t cols = 0, int64_t n_pairs = 0,
                        int update = 0, bool by_count = false, HotFinalize *defer = nullptr, int skip_solo = 0) {
+  const int dwords = rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t));
   // the second step of the hot latents: launched here, or handed back through `defer` for the next
   // training-step launch to carry
   auto finalize = [&](int mode, int units) {
-    HotFinalize h = {ll.ctrl, ll.list, ll.chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, 256u};
+    HotFinalize h = {ll.ctrl, ll.list, ll.chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, dwords, 256u};
     if (defer) {
       h.n_blocks = 64u;  // riding along with a long launch: few blocks, so that they cost little where there is nothing to do
       *defer = h;
@@ -716,7 +720,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
       hipLaunchKernelGGL((hot_finalize_kernel<GT>), dim3(h.n_blocks), dim3(kBlock), 0, st, h);
   };
   if (piece_cols > 0) {  // 256-byte pieces, sixteen lanes each
-    const int pps = static_cast<int>(cols / piece_cols);
+    const int pps = static_cast<int>(ceil_div(cols, piece_cols));
     int pps_shift = -1;  // log2(pps) when pps is a power of two
     for (int sh = 0; sh < 16; ++sh)
       if (pps == (1 << sh)) pps_shift = sh;
@@ -726,7 +730,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
 #define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS)                                                                          \
   hipLaunchKernelGGL((seg_reduce_piece_kernel<PT, GT, FLEXSAE_PIECE_U, G>),                                        \
                      dim3(kLongBlocks + static_cast<unsigned>(N_BLOCKS)), dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, \
-                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, skip_solo, ls)
+                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, skip_solo, dwords, ls)
     constexpr int64_t kGroups = kBlock / kPieceLanes;
     if (by_count) {
       // work items: one per latent with nine rows or more, one per four others of a class
@@ -822,13 +826,15 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   const bool sparse = piece != 0 && sparse_latents(s, flags);
   if (sparse && do_reduce && !update)
     hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, sc.lists.ctrl,
-                       sc.lists.empty_list, dW, D);
+                       sc.lists.empty_list, dW, D, rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t)));
   // In the training step the second step of a slice's hot latents travels with the next slice's
   // training-step launch (a gradient of CarriedGrad's type only: that is what that kernel writes; a launch
   // of its own costs 4.7 us a slice); the last slice's gets one.
   HotFinalize pending = {};
   HotBlockFinalize pending_hot = {};
-  const bool fold = std::is_same<GT, typename CarriedGrad<WT>::type>::value && train != nullptr && do_sweep && do_reduce;
+  // (the sweep of the plain backward carries it for a gradient of the weight's type)
+  const bool fold = (train ? std::is_same<GT, typename CarriedGrad<WT>::type>::value : std::is_same<GT, WT>::value) &&
+                    do_sweep && do_reduce;
   // Only pairs of their latents write dW themselves where its type is the contributions' own.
   void *const dW_solo = (flags & kBwdSolo) && std::is_same<GT, PT>::value && train != nullptr && do_sweep && do_reduce &&
                                 !update && !dw_scale
@@ -855,10 +861,11 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     } else if (do_sweep) {
 #define FLEXSAE_SWEEP(SV)                                                                                      \
   hipLaunchKernelGGL((hier_sweep_kernel<WT, PT, SV, FLEXSAE_SWEEP_U>),                                         \
-                     dim3(static_cast<unsigned>(ceil_div(s->B * (cols / (kWave * SV)), kWavesPerBlock))),      \
+                     dim3(pending.n_blocks +                                                                   \
+                          static_cast<unsigned>(ceil_div(s->B * (cols / (kWave * SV)), kWavesPerBlock))),      \
                      dim3(kBlock), 0, st, indices, weight, vals, s->vals_dtype, resid, grad_out, coef, slot, P, \
                      dv_part, s_final, d_pad, status_flag, s->B * (cols / (kWave * SV)), s->B,                 \
-                     static_cast<int>(col0), sw, K, s->F, D, slot_mask(s))
+                     static_cast<int>(col0), sw, K, s->F, D, slot_mask(s), pending)
       if (sweep_vec == VEC) {
         FLEXSAE_SWEEP(VEC);
       } else if (sweep_vec == (VEC >= 2 ? VEC / 2 : 1)) {
@@ -867,16 +874,18 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
         FLEXSAE_SWEEP(1);
       }
 #undef FLEXSAE_SWEEP
+      pending = HotFinalize{};
     }
     if (!do_reduce) continue;
-    // Pieces where the slice is not made of whole reduction tiles, where most latents are empty
+    // Pieces where rows allow no 8- or 16-byte access of their own elements (a piece of contributions is read 16
+    // bytes per lane whatever D is), where the slice is not made of whole reduction tiles, where most latents are empty
     // (four latents per group of lanes), for the in-place update, and where a slice of
     // contributions is about the size of the memory-side cache (measured 1 % faster there); else one
     // wavefront per (latent, reduction tile), which wastes no load slots on the unequal row counts
     // of the four latents a wavefront would otherwise share (4 % faster on slices read from HBM).
     const bool cache_sized = static_cast<size_t>(s->B * s->K) * static_cast<size_t>(sw) * pl.p_size <= (size_t{384} << 20);
     const bool by_pieces =
-        piece != 0 && (update || cols % pl.tile != 0 || sparse_latents(s, flags) || cache_sized);
+        piece != 0 && (update || pl.vec < 4 || cols % pl.tile != 0 || sparse_latents(s, flags) || cache_sized);
     launch_seg_reduce<PT, GT, VEC>(narrow_reduce, begin, reduce_long, sc.lists, P, partial, dW, dw_scale, s->F, tps,
                                    static_cast<int>(col0), sw, D, st, by_pieces ? piece : 0, cols, s->B * s->K, update,
                                    sparse, fold ? &pending : nullptr, dW_solo != nullptr);
@@ -1318,12 +1327,16 @@ int flexsae_hier_bwd(const flexsae_shape *s, const int64_t *indices, const void 
   if (pl.vec == 4) {
     launch_hier_slices_w<4>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
                             dvals, dbias, ws, flags, status_flag, st);
-  } else if (pl.vec == 2) {
-    launch_hier_slices_w<2>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
-                            dvals, dbias, ws, flags, status_flag, st);
   } else {
-    launch_hier_slices_w<1>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
-                            dvals, dbias, ws, flags, status_flag, st);
+    // rows that allow no more than 8 bytes of their own elements at a time are reduced by pieces where a slice is
+    // whole pieces
+    const int piece = slice_w % piece_cols(pl) == 0 ? static_cast<int>(piece_cols(pl)) : 0;
+    if (pl.vec == 2)
+      launch_hier_slices_w<2>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
+                              dvals, dbias, ws, flags, status_flag, st, nullptr, piece);
+    else
+      launch_hier_slices_w<1>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
+                              dvals, dbias, ws, flags, status_flag, st, nullptr, piece);
   }
   return launch_status();
 }

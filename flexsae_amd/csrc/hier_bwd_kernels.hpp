@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "segment_kernels.hpp"
 #include "csr_kernels.hpp"
 #include "fwd_kernels.hpp"
 
@@ -125,6 +126,8 @@ namespace flexsae {
 // moment gather from the same 64*VEC-column slice of W, which is small enough to stay in the
 // on-chip caches while it is being reused by every row.  Lane l owns VEC consecutive columns,
 // so the gathered weight piece and the stored contribution are one vector access per lane.
+// U = 16 gathers in flight: 64 of them at one register each are 3-5 % slower for the step (B=4096, K=64, F=65536,
+// D=2306 and 2305 bf16: 1061 and 1307 us against 1027 and 1243), the wavefronts they cost hide more.
 template <typename WT, typename PT, int VEC, int U>
 __global__ __launch_bounds__(256) void hier_sweep_kernel(
     const int64_t *__restrict__ indices, const void *__restrict__ weight,
@@ -132,9 +135,14 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
     const float *__restrict__ grad_out, float coef, const uint32_t *__restrict__ slot,
     void *__restrict__ P, float *__restrict__ dv_part, float *__restrict__ s_final, int s_final_ld,
     int *status_flag, int64_t n_items, int64_t B, int col0, int slice_w, int K, int64_t F,
-    int D, uint32_t slot_mask) {
+    int D, uint32_t slot_mask, HotFinalize fin) {
   const int lane = lane_id();
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
+  // the leading blocks finish the hot latents of the previous slice (a gradient of the weight's type)
+  if (blockIdx.x < fin.n_blocks) {
+    hot_finalize_run<WT>(fin, blockIdx.x);
+    return;
+  }
+  const int64_t item = static_cast<int64_t>(blockIdx.x - fin.n_blocks) * (blockDim.x >> 6) + wave_in_block();
   if (item >= n_items) return;  // uniform per wavefront
   const int t = static_cast<int>(item / B);
   const int64_t b = item - static_cast<int64_t>(t) * B;
@@ -153,14 +161,17 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
   static_assert(U % 8 == 0, "the prefetch depth counts blocks of eight steps");
   const int64_t pair0 = b * K;
   for (int k0 = ((K - 1) / kWave) * kWave; k0 >= 0; k0 -= kWave) {
+    // all that the steps need requested at once and waited for once (the conversion branches on a run-time type)
     const int kk = k0 + lane;
-    int64_t my_idx = 0;
-    float my_val = 0.f;
-    int my_slot = 0;
-    if (kk < K) {
-      my_idx = indices[pair0 + kk];
-      my_val = load_scalar(vals, vals_dtype, pair0 + kk);
-      my_slot = static_cast<int>(slot[pair0 + kk] & slot_mask);  // (without the mark of a latent's only pair)
+    const int64_t mine = pair0 + (kk < K ? kk : 0);
+    int64_t my_idx = indices[mine];
+    const uint32_t val_bits = load_scalar_bits(vals, vals_dtype, mine);
+    int my_slot = static_cast<int>(slot[mine] & slot_mask);  // (without the mark of a latent's only pair)
+    float my_val = scalar_from_bits(val_bits, vals_dtype);
+    if (kk >= K) {
+      my_idx = 0;
+      my_val = 0.f;
+      my_slot = 0;
     }
     if (static_cast<uint64_t>(my_idx) >= static_cast<uint64_t>(F)) {
       if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);

@@ -1151,3 +1151,45 @@ def test_only_pairs_written_by_the_walk(dtype, shape, hot):
     rc, _, dW, _, _ = abi.hier_train(bad, *args[1:], dw_dtype=dw_dtype, flag=flag, flags=flags)
     assert rc == 0 and int(flag) == _lib.FLAG_INDEX_RANGE
     assert not dW[0].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shape", [
+    (40, 66, 900, 258),    # 66 steps: more than one chunk; last slice of two columns
+    (33, 64, 3000, 131),   # odd rows: no two of them start on the same alignment
+    (70, 9, 4000, 390),    # most latents without a pair
+    (150, 70, 60, 1),      # one column, frequent latents only
+    (90, 130, 100, 262),   # frequent latents, their second step in the next sweep
+    (40, 12, 300, 127),
+])
+def test_backward_of_rows_that_start_anywhere(dtype, shape):
+    """Plain backward where D is no multiple of four: dW rows start and end inside the vectors that it is
+    written with.  Against the oracle, the same bits for every slice width, and nothing beyond the last row."""
+    B, K, F, D = shape
+    _announce("rows anywhere", dtype, shape)
+    cpu = make_inputs(B, K, F, D, dtype, seed=61, w_std=0.3)
+    idx, W, v, b, t = _to_dev(cpu)
+    rc, loss, resid = abi.forward("hier", idx, W, v, b, t)
+    assert rc == 0
+    g = torch.tensor([2.0], device=DEV)
+    lib, p = _lib.load(), abi.ptr
+    sh = abi.shape_of(idx, W, v)
+    outs = []
+    dw_dtype = torch.float32 if dtype == torch.float16 else dtype
+    for cols in (0, 256, 4096):
+        nbytes = lib.flexsae_hier_bwd_workspace_bytes(ctypes.byref(sh), cols)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        guarded = torch.full((F * D + 64,), 7.0, dtype=dw_dtype, device=DEV)
+        dv, db = torch.empty((B, K), device=DEV), torch.empty((D,), device=DEV)
+        assert lib.flexsae_hier_bwd(ctypes.byref(sh), p(idx), p(W), p(v), p(resid), p(g), p(guarded), abi.DT[dw_dtype], p(dv),
+                                    p(db), p(ws), nbytes, 0, None, abi.stream()) == 0
+        assert bool((guarded[F * D:] == 7.0).all())
+        outs.append((guarded[:F * D].view(F, D), dv, db))
+    for o in outs[1:]:
+        assert torch.equal(o[0], outs[0][0]) and torch.equal(o[2], outs[0][2])
+        assert rel_err(o[1].cpu(), outs[0][1].cpu()) <= 1e-6
+    _, rW, rv, rb = oracle.loss_grads(oracle.HIER, *cpu)
+    tol = 1e-2 if dtype == torch.bfloat16 else 1e-4
+    check_gradient("dW", outs[0][0], 2 * rW, dw_dtype, tol)
+    check_gradient("dvals", outs[0][1], 2 * rv, torch.float32, tol)
+    check_gradient("dbias", outs[0][2], 2 * rb, torch.float32, tol)
