@@ -916,18 +916,10 @@ __device__ __forceinline__ void colsum_partial_one(const float *__restrict__ x, 
   partial[chunk * cols + c] = s;
 }
 
-__global__ __launch_bounds__(256) void colsum_partial_kernel(const float *__restrict__ x, int64_t rows,
-                                                             int64_t ld, int cols,
-                                                             float *__restrict__ partial) {
-  colsum_partial_one(x, rows, ld, cols, partial, static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x),
-                     static_cast<int64_t>(blockIdx.y));
-}
-
-__global__ __launch_bounds__(256) void colsum_final_kernel(const float *__restrict__ partial,
-                                                           int n_chunks, int cols,
-                                                           const float *__restrict__ grad_out, float coef,
-                                                           float *__restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// stage 2 for column c
+__device__ __forceinline__ void colsum_final_one(const float *__restrict__ partial, int n_chunks, int cols,
+                                                 const float *__restrict__ grad_out, float coef,
+                                                 float *__restrict__ out, int c) {
   if (c >= cols) return;
   float s = 0.f;
   int k = 0;
@@ -940,6 +932,13 @@ __global__ __launch_bounds__(256) void colsum_final_kernel(const float *__restri
   }
   for (; k < n_chunks; ++k) s += partial[static_cast<int64_t>(k) * cols + c];
   out[c] = s * coef * (grad_out ? grad_out[0] : 1.f);
+}
+
+__global__ __launch_bounds__(256) void colsum_final_kernel(const float *__restrict__ partial,
+                                                           int n_chunks, int cols,
+                                                           const float *__restrict__ grad_out, float coef,
+                                                           float *__restrict__ out) {
+  colsum_final_one(partial, n_chunks, cols, grad_out, coef, out, static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
 __global__ void fill_f32_kernel(float *__restrict__ p, int64_t n) {

@@ -349,8 +349,10 @@ CsrScratch carve_csr_scratch(void *workspace, int64_t F, int64_t n_pairs) {
   return sc;
 }
 
-void launch_pair_lists(const uint32_t *begin, int64_t F, const PairLists &lists, hipStream_t st) {
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, lists.ctrl, static_cast<int64_t>(kCtrlWords), 0u);
+// cleared: the control words are zero already
+void launch_pair_lists(const uint32_t *begin, int64_t F, const PairLists &lists, hipStream_t st, bool cleared = false) {
+  if (!cleared)
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, lists.ctrl, static_cast<int64_t>(kCtrlWords), 0u);
   hipLaunchKernelGGL(pair_lists_kernel, dim3(static_cast<unsigned>(ceil_div(F, kListLatents))), dim3(1024), 0, st, begin,
                      F, lists);
 }
@@ -1058,7 +1060,7 @@ template <typename WT, typename GT, typename RT, int VEC>
 void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                         const uint32_t *begin, const uint32_t *map, const void *weight,
                         const void *vals, const void *resid, const float *grad_out, float coef,
-                        void *dW, float *dvals, uint8_t *ws, hipStream_t st) {
+                        void *dW, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
   const PairLists ls = carve_topk_lists(s, pl, ws);
   const uint32_t *long_ctrl = ls.ctrl, *long_list = ls.long_list, *chunk_begin = ls.chunk_begin;
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
@@ -1077,9 +1079,20 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
                        s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, kLongBlocks, tps,
                        static_cast<int>(col0), sw, s->F, K, D, static_cast<uint32_t>(resid_bytes));
-    hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st,
-                       long_ctrl, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps,
-                       static_cast<int>(col0), sw, D);
+    if (col0 + slice_w < s->D) {
+      hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st,
+                         long_ctrl, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps,
+                         static_cast<int>(col0), sw, D);
+      continue;
+    }
+    constexpr unsigned n_long_blocks = 256;
+    const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(D, kBlock));
+    hipLaunchKernelGGL((topk_epilogue_kernel<GT, VEC>),
+                       dim3(n_long_blocks + n_col_blocks + grid_for(n_pairs, kBlock, 8192)), dim3(kBlock), 0, st, long_ctrl,
+                       long_list, chunk_begin, partial, dW, tps, static_cast<int>(col0), sw, D, n_long_blocks,
+                       reinterpret_cast<const float *>(ws + pl.off_colsum), static_cast<int>(ceil_div(s->B, kColsumRows)),
+                       grad_out, coef, dbias, n_col_blocks, map, dv_part, static_cast<int>(pl.d_pad / pl.tile), n_pairs,
+                       dvals);
   }
 }
 
@@ -1087,19 +1100,19 @@ template <typename WT, typename RT, int VEC>
 void launch_topk_slices_g(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                           const uint32_t *begin, const uint32_t *map, const void *weight,
                           const void *vals, const void *resid, const float *grad_out, float coef,
-                          void *dW, int dW_dtype, float *dvals, uint8_t *ws, hipStream_t st) {
+                          void *dW, int dW_dtype, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
   switch (dW_dtype) {
     case FLEXSAE_F32:
       launch_topk_slices<WT, float, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                             coef, dW, dvals, ws, st);
+                                             coef, dW, dvals, dbias, ws, st);
       break;
     case FLEXSAE_BF16:
       launch_topk_slices<WT, bf16_t, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dvals, ws, st);
+                                              coef, dW, dvals, dbias, ws, st);
       break;
     default:
       launch_topk_slices<WT, f16_t, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                             coef, dW, dvals, ws, st);
+                                             coef, dW, dvals, dbias, ws, st);
   }
 }
 
@@ -1108,23 +1121,23 @@ template <int VEC>
 void launch_topk_slices_w(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                           const uint32_t *begin, const uint32_t *map, const void *weight,
                           const void *vals, const void *resid, const float *grad_out, float coef,
-                          void *dW, int dW_dtype, float *dvals, uint8_t *ws, hipStream_t st) {
+                          void *dW, int dW_dtype, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
   switch (s->weight_dtype) {
     case FLEXSAE_F32:
       launch_topk_slices_g<float, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dW_dtype, dvals, ws, st);
+                                              coef, dW, dW_dtype, dvals, dbias, ws, st);
       break;
     case FLEXSAE_BF16:
       if (pl.resid16)
         launch_topk_slices_g<bf16_t, bf16_t, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                                  coef, dW, dW_dtype, dvals, ws, st);
+                                                  coef, dW, dW_dtype, dvals, dbias, ws, st);
       else
         launch_topk_slices_g<bf16_t, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                                 coef, dW, dW_dtype, dvals, ws, st);
+                                                 coef, dW, dW_dtype, dvals, dbias, ws, st);
       break;
     default:
       launch_topk_slices_g<f16_t, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dW_dtype, dvals, ws, st);
+                                              coef, dW, dW_dtype, dvals, dbias, ws, st);
   }
 }
 
@@ -1564,46 +1577,34 @@ int flexsae_topk_bwd(const flexsae_shape *s, const uint32_t *begin, const uint32
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   // (every output element is written exactly once: nothing needs a zero-fill, whatever `flags` says)
   const PairLists lists = carve_topk_lists(s, pl, ws);
-  launch_pair_lists(begin, s->F, lists, st);
   const float coef =
       static_cast<float>(2.0 / (static_cast<double>(s->B) * static_cast<double>(s->D)));
-  // per-pair records and, for bf16 weights, the bf16 copy of the residual: one launch
+  // per-pair records, for bf16 weights the bf16 copy of the residual, and stage 1 of dbias: one launch
   const void *gather_src = pl.resid16 ? static_cast<const void *>(ws + pl.off_resid16) : resid;
   {
     const int64_t n_resid = pl.resid16 ? s->B * s->D : 0;
     const int64_t work = s->B * s->K > ceil_div(n_resid, 4) ? s->B * s->K : ceil_div(n_resid, 4);
-    hipLaunchKernelGGL(topk_prepare_kernel, dim3(grid_for(work, 256, 1 << 16)), dim3(256), 0, st, map, indices,
+    const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(s->D, 256) * ceil_div(s->B, kColsumRows));
+    hipLaunchKernelGGL(topk_prepare_kernel, dim3(n_col_blocks + grid_for(work, 256, 1 << 16)), dim3(256), 0, st, map, indices,
                        s->F, vals, s->vals_dtype, s->B * s->K, static_cast<int>(s->K),
                        reinterpret_cast<vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), resid, n_resid,
-                       pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr);
+                       pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr, lists.ctrl, s->B,
+                       static_cast<int>(s->D), reinterpret_cast<float *>(ws + pl.off_colsum), n_col_blocks);
   }
+  launch_pair_lists(begin, s->F, lists, st, true);
   if (pl.vec == 8) {
     launch_topk_slices_g<bf16_t, bf16_t, 8>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef,
-                                            dW, dW_dtype, dvals, ws, st);
+                                            dW, dW_dtype, dvals, dbias, ws, st);
   } else if (pl.vec == 4) {
     launch_topk_slices_w<4>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, ws, st);
+                            dW_dtype, dvals, dbias, ws, st);
   } else if (pl.vec == 2) {
     launch_topk_slices_w<2>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, ws, st);
+                            dW_dtype, dvals, dbias, ws, st);
   } else {
     launch_topk_slices_w<1>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, ws, st);
+                            dW_dtype, dvals, dbias, ws, st);
   }
-  hipLaunchKernelGGL(topk_dvals_finalize_kernel, dim3(grid_for(s->B * s->K, 256, 8192)), dim3(256), 0, st, map,
-                     reinterpret_cast<const float *>(ws + pl.off_dvpart), static_cast<int>(pl.d_pad / pl.tile),
-                     s->B * s->K, dvals);
-  rc = launch_status();
-  if (rc != FLEXSAE_OK) return rc;
-  // dbias = coef * grad_out * column sums of resid, in a fixed order
-  float *colsum_part = reinterpret_cast<float *>(ws + pl.off_colsum);
-  const int n_chunks = static_cast<int>(ceil_div(s->B, kColsumRows));
-  const int D = static_cast<int>(s->D);
-  hipLaunchKernelGGL(colsum_partial_kernel,
-                     dim3(static_cast<unsigned>(ceil_div(D, 256)), static_cast<unsigned>(n_chunks)), dim3(256),
-                     0, st, resid, s->B, s->D, D, colsum_part);
-  hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(D, 256))), dim3(256), 0, st,
-                     colsum_part, n_chunks, D, grad_out, coef, dbias);
   return launch_status();
 }
 

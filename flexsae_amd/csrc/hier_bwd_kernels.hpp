@@ -257,7 +257,7 @@ __global__ void hier_dvals_finalize_kernel(const float *__restrict__ dv_part, in
 // parts are independent; each computes what its own kernel computes, bit for bit):
 //   block 0                 the loss from the per-(tile, row) partials (loss_finalize_kernel), when
 //                           loss_partial is given;
-//   the next n_colsum_blocks stage 1 of the column sums of s_final (colsum_partial_kernel): a block
+//   the next n_colsum_blocks stage 1 of the column sums of s_final (colsum_partial_one): a block
 //                           takes 256 columns of four consecutive row chunks;
 //   the rest                dvals from its per-tile shares (hier_dvals_finalize_kernel).
 __global__ __launch_bounds__(1024) void hier_epilogue_kernel(

@@ -22,7 +22,7 @@ namespace flexsae {
 //   acc      += vals[p] * scale * resid[b_p]          (dW contribution)
 //   dv_tile[slot] = scale * <resid[b_p], W[f]>        (this tile's share of dvals[p]; the lane that
 //                                                      owns the slot stores it, so stores coalesce;
-//                                                      topk_dvals_finalize_kernel adds the tiles up)
+//                                                      topk_epilogue_kernel adds the tiles up)
 // resid rows (element type RT) are read through the caches: the waves in flight share one
 // B x tile slice of the [B,D] matrix, which has to stay in the 4 MB L2 of every XCD.
 template <typename RT, int VEC>
@@ -284,13 +284,34 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
   }
 }
 
-// dvals[map[slot]] = sum over the column tiles of dv_part[tile, slot], in tile order
-// (every pair sits in exactly one slot, so dvals is written once and needs no zero-fill).
-__global__ void topk_dvals_finalize_kernel(const uint32_t *__restrict__ map,
-                                           const float *__restrict__ dv_part, int n_tiles,
-                                           int64_t n_pairs, float *__restrict__ dvals) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t s = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < n_pairs; s += stride) {
+// What follows the (last) slice of a TopK backward, in one launch of 256-thread blocks; the parts are independent:
+//   the first n_long_blocks  second step of the slice's long latents (seg_long_finalize_body);
+//   the next n_col_blocks    dbias = coef * grad_out * column sums of resid: stage 2 (colsum_final_one);
+//   the rest                 dvals[map[slot]] = sum over the column tiles of dv_part[tile, slot], in tile order (every
+//                            pair sits in exactly one slot, so dvals is written once and needs no zero-fill).
+// A launch costs 4-5 us in a busy stream: with the preparation (below) four launches instead of eight around the pair
+// list and the backward: B=4096, K=128, F=65536, D=2304 bf16 618 -> 610 us, B=64, K=32, F=4096, D=256 250 -> 239.
+template <typename GT, int VEC>
+__global__ __launch_bounds__(256) void topk_epilogue_kernel(
+    const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
+    const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial, void *__restrict__ dW, int tps, int col0,
+    int slice_w, int D, unsigned n_long_blocks, const float *__restrict__ colsum_part, int n_chunks,
+    const float *__restrict__ grad_out, float coef, float *__restrict__ dbias, unsigned n_col_blocks,
+    const uint32_t *__restrict__ map, const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs,
+    float *__restrict__ dvals) {
+  if (blockIdx.x < n_long_blocks) {
+    seg_long_finalize_body<GT, VEC, 8>(long_ctrl, long_list, chunk_begin, partial, dW, nullptr, tps, col0, slice_w, D,
+                                       blockIdx.x, n_long_blocks);
+    return;
+  }
+  unsigned blk = blockIdx.x - n_long_blocks;
+  if (blk < n_col_blocks) {
+    colsum_final_one(colsum_part, n_chunks, D, grad_out, coef, dbias, static_cast<int>(blk * blockDim.x + threadIdx.x));
+    return;
+  }
+  blk -= n_col_blocks;
+  const int64_t stride = static_cast<int64_t>(gridDim.x - n_long_blocks - n_col_blocks) * blockDim.x;
+  for (int64_t s = static_cast<int64_t>(blk) * blockDim.x + threadIdx.x; s < n_pairs; s += stride) {
     float acc = 0.f;
     for (int t = 0; t < n_tiles; ++t) acc += dv_part[t * n_pairs + s];
     dvals[map[s]] = acc;
@@ -302,14 +323,24 @@ __global__ void topk_dvals_finalize_kernel(const uint32_t *__restrict__ map,
 //     the backward reads per pair, contiguous per latent instead of scattered over vals; a pair
 //     whose index lies outside [0, F) gets a val of zero, as in the forward (the pair list files it
 //     under latent 0), so that it adds nothing to dW (`indices` may be null: every val is kept);
-//   resid16[i] = bf16(resid[i]) for i < n_resid (n_resid = 0: no copy wanted).
-__global__ void topk_prepare_kernel(const uint32_t *__restrict__ map, const int64_t *__restrict__ indices,
+//   resid16[i] = bf16(resid[i]) for i < n_resid (n_resid = 0: no copy wanted);
+//   ctrl[] = 0: the control words of the lists that the next launch fills;
+//   in the first n_col_blocks blocks, stage 1 of the column sums of resid (for dbias).
+__global__ __launch_bounds__(256) void topk_prepare_kernel(const uint32_t *__restrict__ map, const int64_t *__restrict__ indices,
                                     int64_t F, const void *__restrict__ vals,
                                     int vals_dtype, int64_t n_pairs, int K,
                                     vec_t<uint32_t, 2> *__restrict__ slot_bv, const float *__restrict__ resid,
-                                    int64_t n_resid, void *__restrict__ resid16) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+                                    int64_t n_resid, void *__restrict__ resid16, uint32_t *__restrict__ ctrl,
+                                    int64_t rows, int cols, float *__restrict__ colsum_part, unsigned n_col_blocks) {
+  if (blockIdx.x < n_col_blocks) {
+    const unsigned across = static_cast<unsigned>((cols + 255) / 256);
+    colsum_partial_one(resid, rows, cols, cols, colsum_part, static_cast<int>(blockIdx.x % across * 256 + threadIdx.x),
+                       static_cast<int64_t>(blockIdx.x / across));
+    return;
+  }
+  if (blockIdx.x == n_col_blocks && threadIdx.x < kCtrlWords) ctrl[threadIdx.x] = 0u;
+  const int64_t stride = static_cast<int64_t>(gridDim.x - n_col_blocks) * blockDim.x;
+  const int64_t tid = static_cast<int64_t>(blockIdx.x - n_col_blocks) * blockDim.x + threadIdx.x;
   for (int64_t s = tid; s < n_pairs; s += stride) {
     const uint32_t p = map[s];
     vec_t<uint32_t, 2> r;
