@@ -117,12 +117,30 @@ def _prep(t: Tensor) -> Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
-def _ptr(t: Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: Tensor) -> int:
+    return t.data_ptr()  # (the library's argument types make it a pointer)
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+# The current device and the current stream's handle without the Stream object and the checks around it, where this
+# torch has them: an entry asks once or twice, 3 us each time.
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream() -> int:
+    if _raw_stream is None or _get_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_get_device())
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on_device(dev: torch.device):
+    """Context in which `dev` (a tensor's device) is the current one: nothing to do where it already is."""
+    if _get_device is not None and torch.cuda.is_initialized() and _get_device() == dev.index:
+        return _SAME_DEVICE
+    return torch.cuda.device(dev)
 
 
 def _forward(entry: str, indices, weight, vals, bias, target) -> Tuple[Tensor, Tensor]:
@@ -130,7 +148,7 @@ def _forward(entry: str, indices, weight, vals, bias, target) -> Tuple[Tensor, T
     lib = _lib.load()
     indices, weight, vals, bias, target = (_prep(t) for t in (indices, weight, vals, bias, target))
     dev = weight.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         ws_bytes = lib.flexsae_fwd_workspace_bytes(ctypes.byref(shape))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
@@ -349,14 +367,14 @@ def _hot_measure(lib, shape, workspace: Tensor, B, K, F, D, weight_dtype) -> Non
     st = _hot_auto.get(key)
     if st is None:
         st = _hot_auto[key] = {"hot": False, "dense": False,
-                               "pinned": torch.zeros(3, dtype=torch.int32, pin_memory=True), "event": None}
+                               "pinned": torch.zeros(3, dtype=torch.int32, pin_memory=True), "event": None,
+                               "spare": torch.cuda.Event()}
     if st["event"] is not None:
         return  # a measurement is still on its way
     rc = lib.flexsae_hier_pair_stats(ctypes.byref(shape), _ptr(workspace), _ptr(st["pinned"]), _stream())
     _lib.check(rc, "flexsae_hier_pair_stats")
-    ev = torch.cuda.Event()
-    ev.record()
-    st["event"] = ev
+    st["spare"].record()
+    st["event"] = st["spare"]
 
 
 def _hot_slice_cols(B: int, cols: int, device) -> int:
@@ -473,7 +491,7 @@ def hier_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
     F, D = weight.shape
     dev = weight.device
     indices, weight, vals, resid = (_prep(t) for t in (indices, weight, vals, resid))
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         shape = _shape(B, K, F, D, weight, vals, torch.float32, torch.float32)
         dvals = torch.empty((B, K), dtype=torch.float32, device=dev)
@@ -531,7 +549,7 @@ def topk_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
     F, D = weight.shape
     dev = weight.device
     indices, weight, vals, resid = (_prep(t) for t in (indices, weight, vals, resid))
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         shape = _shape(B, K, F, D, weight, vals, torch.float32, torch.float32)
         cached = _pair_lookup(indices, F)
@@ -640,7 +658,7 @@ def hier_train(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, targ
     dev = weight.device
     if stage.dtype != torch.uint8 or stage.device != dev or not stage.is_contiguous():
         raise ValueError("stage must be a contiguous uint8 tensor on the weight's device (see hier_train_stage)")
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         loss = torch.empty((), dtype=torch.float32, device=dev)
         dvals = torch.empty((B, K), dtype=torch.float32, device=dev)
@@ -675,7 +693,7 @@ def hier_finish(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
     B, K = indices.shape
     F, D = weight.shape
     dev = weight.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         shape = _shape(B, K, F, D, weight, vals, torch.float32, torch.float32)
         dW = torch.empty((F, D), dtype=weight.dtype, device=dev)
@@ -731,7 +749,7 @@ def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tenso
     lib = _lib.load()
     indices, weight, vals, bias, target = (_prep(t) for t in (indices, weight, vals, bias, target))
     dev = weight.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype)
         hot_flag = _hot_flags(B, D, dev) if (hot and need_dw) else 0
@@ -802,7 +820,7 @@ def hier_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, t
     lib = _lib.load()
     indices, vals, bias, target = (_prep(t) for t in (indices, vals, bias, target))
     dev = weight.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype)
         # hot-latent accumulators: the same decision as the loss takes (set_hot_latents)
@@ -862,7 +880,7 @@ def scale_by(x: Tensor, grad_out: Tensor) -> Tensor:
     ``dW.mul_(grad)`` (hierarchical_kernels.py:294-297) after a unit-gradient pass."""
     lib = _lib.load()
     dev = x.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         x = _prep(x)
         out = torch.empty_like(x)
@@ -885,7 +903,7 @@ def scale_to(x: Tensor, grad_out: Tensor, dtype: torch.dtype) -> Tensor:
         raise TypeError("scale_to expects a float32 tensor")
     lib = _lib.load()
     dev = x.device
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         x = _prep(x)
         out = torch.empty(x.shape, dtype=dtype, device=dev)
@@ -906,7 +924,7 @@ def scale_(x: Tensor, grad_out: Tensor) -> None:
     dev = x.device
     if not x.is_contiguous():
         raise ValueError("scale_ needs a contiguous tensor")
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         rc = lib.flexsae_scale(_ptr(x), _ptr(x), _DTYPES[x.dtype], x.numel(), _ptr(g), _stream())
         _lib.check(rc, "flexsae_scale")
