@@ -220,11 +220,19 @@ __device__ __forceinline__ float dpp_move(float v) {
       __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
 }
 
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
 __device__ __forceinline__ int lane_id() { return static_cast<int>(threadIdx.x) & (kWave - 1); }
 
 // Sum over the 64 lanes of the wavefront using DPP moves only (no LDS traffic).
 // The total is valid in lane 63; use wave_sum_bcast() to have it in every lane.
-__device__ __forceinline__ float wave_sum_lane63(float v) {
+template <typename T>  // float or double
+__device__ __forceinline__ T wave_sum_lane63(T v) {
   v += dpp_move<0xB1>(v);         // quad_perm [1,0,3,2]: lane ^ 1
   v += dpp_move<0x4E>(v);         // quad_perm [2,3,0,1]: lane ^ 2
   v += dpp_move<0x141>(v);        // row_half_mirror: the other quad of each 8

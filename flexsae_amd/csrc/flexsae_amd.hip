@@ -151,7 +151,8 @@ FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target,
   // order from 24576 latents up to 4 GiB of weights.
   const bool lines = static_cast<size_t>(s->D) * es % 128 == 0;
   const uint64_t w_bytes = static_cast<uint64_t>(s->F) * static_cast<uint64_t>(s->D) * es;
-  const bool by_row = !lines && s->F > 24576 && w_bytes < (uint64_t{1} << 32);
+  // (A single row: a block per narrow tile would leave more partials than the workspace has room for, see forward().)
+  const bool by_row = s->B == 1 || (!lines && s->F > 24576 && w_bytes < (uint64_t{1} << 32));
   const bool by_xcd = !by_row && s->F <= 131072;
   const size_t piece_bytes = by_row ? 1024 : !by_xcd ? 512 : (es == 2 && s->F <= 49152 && lines) ? 128 : 256;
   p.lpr = static_cast<int>(piece_bytes / (static_cast<size_t>(vec) * es));
@@ -168,7 +169,7 @@ FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target,
 template <typename WT, bool HIER>
 void launch_fwd(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices,
                 const void *weight, const void *vals, const void *bias, const void *target,
-                float *resid, float *partial, int *status_flag, hipStream_t st) {
+                float *resid, double *partial, int *status_flag, hipStream_t st) {
 #define FLEXSAE_LAUNCH_FWD(VEC, LPR)                                                                       \
   hipLaunchKernelGGL((sae_fwd_kernel<WT, VEC, LPR, HIER, FLEXSAE_FWD_U>), dim3(p.grid), dim3(kBlock), 0, st, \
                      indices, weight, vals, s->vals_dtype, bias, s->bias_dtype, target, s->target_dtype,   \
@@ -218,7 +219,11 @@ int forward(const flexsae_shape *s, const int64_t *indices, const void *weight, 
     return FLEXSAE_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const FwdPlan p = plan_fwd(s, weight, target, bias, resid);
-  float *partial = static_cast<float *>(workspace);
+  // One double per block.  A tile has at least 64 columns and a block four rows (two or more rows are at least twice as
+  // many as blocks of them; a single row goes by row, four tiles to a block): no more than the workspace's four bytes
+  // per row and 64 columns, to which it is rounded up.
+  if (static_cast<size_t>(p.n_items) * sizeof(double) > workspace_bytes) return FLEXSAE_ERR_WORKSPACE;
+  double *partial = static_cast<double *>(workspace);
   switch (s->weight_dtype) {
     case FLEXSAE_F32:
       launch_fwd<float, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,

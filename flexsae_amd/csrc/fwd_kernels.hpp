@@ -33,9 +33,9 @@ namespace flexsae {
 // on the index loads cost 5-10 % (the eight XCDs share those lines in the memory-side cache); 32-bit
 // offsets through a buffer descriptor change nothing.
 //
-// Per item the block writes resid[b, tile] = r_{b,K-1} - target_b (fp32) and one fp32 partial sum of
-// squares; loss_finalize_kernel adds the partials in a fixed order, so the loss is bit-reproducible from
-// run to run.
+// Per item the block writes resid[b, tile] = r_{b,K-1} - target_b (fp32) and one partial sum of squares;
+// loss_finalize_kernel adds the partials in a fixed order, so the loss is bit-reproducible from
+// run to run.  Everything beyond a lane's own column of a row is added in double.
 constexpr int kFwdChunk = 64;  // steps per LDS fill
 
 template <typename WT, int VEC, int LPR, bool HIER, int U>
@@ -43,13 +43,13 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     const int64_t *__restrict__ indices, const void *__restrict__ weight,
     const void *__restrict__ vals, int vals_dtype, const void *__restrict__ bias, int bias_dtype,
     const void *__restrict__ target, int target_dtype, float *__restrict__ resid,
-    float *__restrict__ partial, int *status_flag, int64_t B, int64_t n_row_blocks, int64_t n_items,
+    double *__restrict__ partial, int *status_flag, int64_t B, int64_t n_row_blocks, int64_t n_items,
     int64_t xcd_span, int K, int64_t F, int D) {
   constexpr int R = kWave / LPR;  // rows per wavefront
   constexpr int kWaves = 256 / kWave;
   static_assert(kFwdChunk == kWave && kFwdChunk % U == 0, "one lane per step of a chunk");
   __shared__ vec_t<uint32_t, 2> steps[kWaves][R][kFwdChunk];  // (row of the weight matrix, val bits)
-  __shared__ float wave_loss[kWaves];
+  __shared__ double wave_loss[kWaves];
   const int lane = lane_id();
   const int wv = wave_in_block();
   int64_t item = blockIdx.x;
@@ -173,25 +173,25 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     __builtin_amdgcn_wave_barrier();
   }
 
-  float lsum = 0.f;
+  double lsum = 0.0;
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
     if constexpr (HIER) {
-      lsum += acc[i];
+      lsum += static_cast<double>(acc[i]);
     } else {
-      lsum = fmaf(e[i], e[i], lsum);
+      lsum = fma(static_cast<double>(e[i]), static_cast<double>(e[i]), lsum);
     }
   }
   if (active) {
     store_vec<float, VEC>(resid, b * D + d0, e);
   } else {
-    lsum = 0.f;
+    lsum = 0.0;
   }
   lsum = wave_sum_lane63(lsum);
   if (lane == kWave - 1) wave_loss[wv] = lsum;
   __syncthreads();
   if (threadIdx.x == 0) {
-    float s = 0.f;
+    double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) s += wave_loss[w];
     partial[item] = s;
@@ -199,14 +199,15 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
 }
 
 // loss[0] = inv_count * sum(partial[0..n)), one block, fixed summation order, double
-// accumulation (n is B * ntiles, up to a few million).
-// (the body, for a block of 1024 threads; `red` is 1024 doubles of LDS)
-__device__ __forceinline__ void loss_finalize_block(const float *__restrict__ partial, int64_t n, double inv_count,
+// accumulation (n up to a few million).
+// (the body, for a block of 1024 threads; `red` is 1024 doubles of LDS; PT: float or double partials)
+template <typename PT>
+__device__ __forceinline__ void loss_finalize_block(const PT *__restrict__ partial, int64_t n, double inv_count,
                                                     float *__restrict__ loss, double *red) {
   double s = 0.0;
   int64_t i = threadIdx.x;
   for (; i + 7 * 1024 < n; i += 8 * 1024) {  // eight independent loads in flight
-    float x[8];
+    PT x[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) x[u] = partial[i + u * 1024];
 #pragma unroll
@@ -222,7 +223,7 @@ __device__ __forceinline__ void loss_finalize_block(const float *__restrict__ pa
   if (threadIdx.x == 0) loss[0] = static_cast<float>(red[0] * inv_count);
 }
 
-__global__ __launch_bounds__(1024) void loss_finalize_kernel(const float *__restrict__ partial,
+__global__ __launch_bounds__(1024) void loss_finalize_kernel(const double *__restrict__ partial,
                                                              int64_t n, double inv_count,
                                                              float *__restrict__ loss) {
   __shared__ double red[1024];

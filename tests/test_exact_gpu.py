@@ -224,3 +224,31 @@ def test_forward_tilings_are_exact(mode, shape, dtype):
     # (a wavefront's fp32 sum is exact below 2^24; the total is one rounding away)
     want = float(sq.double()) / (B * D * (K if mode == "hier" else 1))
     assert abs(loss.item() - want) <= 2.0 ** -23 * want
+
+
+@pytest.mark.parametrize("shape", [(512, 128, 100), (512, 128, 131073), (510, 70, 30000), (1, 8192, 64), (1, 6150, 200000),
+                                   (2, 8192, 100), (3, 4160, 100)])
+@pytest.mark.parametrize("mode", ["topk", "hier"])
+def test_forward_loss_keeps_small_rows_beside_large_ones(mode, shape):
+    """Beyond a row's own columns the squared errors are added in double.  One row in four has an error of 4096, the
+    others of one, with the rows 1, 2, 4, 8 or 32 apart (the rows of a wavefront, of a block): a sum of
+    2^24 and three ones in fp32 loses them, whichever way the rows are grouped.  The loss is the float next to the
+    exact one.  With one to three rows, the most partials per byte of the workspace, the columns take the rows' part."""
+    B, D, F = shape
+    _announce("exact loss", mode, shape)
+    W = torch.zeros(F, D, dtype=torch.bfloat16, device=DEV)
+    idx = torch.zeros(B, 1, dtype=torch.long, device=DEV)
+    vals, bias = torch.ones(B, 1, device=DEV), torch.zeros(D, dtype=torch.bfloat16, device=DEV)
+    for apart in (1, 2, 4, 8, 32):
+        at = torch.arange(B * D // 64 if B < 4 else B)
+        err = torch.where(at % (4 * apart) == 0, 4096.0, torch.where(at % apart == 0, 1.0, 0.0))
+        target = torch.zeros(B, D)
+        if B < 4:  # one entry in each run of 64 columns
+            target.view(-1)[at * 64] = err
+        else:
+            target[:, 0] = err
+        rc, loss, _ = abi.forward(mode, idx, W, vals, bias, target.bfloat16().to(DEV))
+        torch.cuda.synchronize()
+        assert rc == 0, _lib.status_string(rc)
+        want = target.double().square().sum() / (B * D)
+        assert loss.item() == want.float().item(), (apart, loss.item(), want.item())
