@@ -402,8 +402,8 @@ void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
 }
 
 // The lists of a pair list that belong to the caller's workspace (everything but ctrl and long_list): their bytes, and
-// their places in `base` if that is given.
-size_t carve_pair_lists(size_t n_pairs, size_t F, void *base, PairLists *ls) {
+// their places in `base` if that is given.  classes: the lists by number of pairs too.
+size_t carve_pair_lists(size_t n_pairs, size_t F, bool classes, void *base, PairLists *ls) {
   size_t off = 0;
   auto take = [&](uint32_t *&ptr, size_t entries) {
     if (base) ptr = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(base) + off);
@@ -412,6 +412,7 @@ size_t carve_pair_lists(size_t n_pairs, size_t F, void *base, PairLists *ls) {
   PairLists none = {};
   PairLists &l = ls ? *ls : none;
   take(l.chunk_begin, n_pairs / 65 + 1);
+  if (!classes) return off;
   take(l.empty_list, F);
   for (int i = 0; i < kClasses; ++i) {
     const size_t most = n_pairs / ((size_t{1} << i) / 2 + 1);
@@ -484,7 +485,7 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 
   p.off_csr = off;
   off += flexsae_csr_workspace_bytes(s->B, s->K, s->F);
   p.off_lists = off;
-  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), nullptr, nullptr);
+  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), sparse_latents(s), nullptr, nullptr);
   p.off_sfinal = off;  // S_{b,0} of every row, [B, d_pad] fp32: dbias is its column sum
   off += round_up(p.n_rows * static_cast<size_t>(p.d_pad) * 4, kAlign);
   p.off_colsum = off;  // partial column sums, [ceil(B/64), D] fp32
@@ -526,10 +527,11 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 
   return p;
 }
 
-// The pair-list scratch and lists of a hierarchical workspace.
-CsrScratch carve_hier_lists(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws) {
+// The pair-list scratch and lists of a hierarchical workspace, the lists by number of pairs only where a call with
+// these flags reduces from them.
+CsrScratch carve_hier_lists(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws, int flags = 0) {
   CsrScratch sc = carve_csr_scratch(ws + pl.off_csr, s->F, s->B * s->K);
-  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), ws + pl.off_lists, &sc.lists);
+  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), sparse_latents(s, flags), ws + pl.off_lists, &sc.lists);
   return sc;
 }
 
@@ -1037,7 +1039,7 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   p.off_long_list = off;
   off += round_up((p.n_pairs / 65 + 1) * 4, kAlign);
   p.off_lists = off;
-  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), nullptr, nullptr);
+  off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), false, nullptr, nullptr);
   p.off_resid16 = off;
   if (p.resid16) off += round_up(static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 2, kAlign);
   p.off_dvpart = off;  // per-tile shares of dvals: [d_pad / tile, B*K] fp32
@@ -1053,7 +1055,7 @@ PairLists carve_topk_lists(const flexsae_shape *s, const TopkBwdPlan &pl, uint8_
   PairLists ls = {};
   ls.ctrl = reinterpret_cast<uint32_t *>(ws + pl.off_ctrl);
   ls.long_list = reinterpret_cast<uint32_t *>(ws + pl.off_long_list);
-  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), ws + pl.off_lists, &ls);
+  carve_pair_lists(pl.n_pairs, static_cast<size_t>(s->F), false, ws + pl.off_lists, &ls);
   return ls;
 }
 
@@ -1339,7 +1341,7 @@ int flexsae_hier_bwd(const flexsae_shape *s, const int64_t *indices, const void 
   uint32_t *map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
   if (!(flags & FLEXSAE_BWD_REUSE_PAIR_LIST))
     csr_build_launch(indices, s->B, s->K, s->F, begin, map, reinterpret_cast<uint32_t *>(ws + pl.off_slot), nullptr,
-                     carve_hier_lists(s, pl, ws), status_flag, st);
+                     carve_hier_lists(s, pl, ws, flags), status_flag, st);
   const float coef = static_cast<float>(
       2.0 / (static_cast<double>(s->B) * static_cast<double>(s->K) * static_cast<double>(s->D)));
   if (pl.vec == 4) {
@@ -1448,7 +1450,7 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   uint32_t *begin = reinterpret_cast<uint32_t *>(ws + pl.off_begin);
   uint32_t *map = reinterpret_cast<uint32_t *>(ws + pl.off_map);
-  const CsrScratch sc = carve_hier_lists(s, pl, ws);
+  const CsrScratch sc = carve_hier_lists(s, pl, ws, flags);
   const bool build = !(flags & FLEXSAE_BWD_REUSE_PAIR_LIST);
   // Latents of one pair: their contribution is their gradient (kSoloSlotBit), where this call builds the list that
   // marks them.  (Whatever the number of pairs per latent: see hier_train_kernel.)

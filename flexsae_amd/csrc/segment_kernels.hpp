@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__re
                                                             const uint32_t *__restrict__ cls_list,
                                                             void *__restrict__ out, int D, int dwords) {
   constexpr int EV = 16 / static_cast<int>(sizeof(typename Traits<PT>::store_t));
-  const uint32_t n = ctrl[kEmptyCount];
+  const uint32_t n = ctrl[kListed] ? ctrl[kEmptyCount] : 0u;
   const int lane = lane_id();
   float zero[EV];
 #pragma unroll

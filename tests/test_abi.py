@@ -147,3 +147,19 @@ def test_static_forward_rejects_bad_arguments_before_touching_the_gpu():
     assert fn(ctypes.byref(_shape(B=70000, K=1, D=4096)), *args, NULL, NULL) == _lib.ERR_SCRATCH_LIMIT
     m = re.search(r"FLEXSAE_STATIC_SCRATCH_BYTES\s*\((\d+)u\s*<<\s*(\d+)\)", open(HEADER).read())
     assert m and (int(m.group(1)) << int(m.group(2))) == 16 << 20
+
+
+@pytest.mark.parametrize("B,K,D,wdt", [(64, 16, 256, 0), (4096, 128, 2304, 1), (31, 3, 70, 2)])
+def test_workspaces_hold_the_lists_by_number_of_pairs_only_where_they_are_read(B, K, D, wdt):
+    """The TopK backward reads a list of the long latents only, so its workspace does not depend on the size of the
+    dictionary; a hierarchical one with more than two pairs per latent grows with it by the pair list itself."""
+    lib = _lib.load()
+    at = lambda fn, F: getattr(lib, fn)(ctypes.byref(_shape(B=B, K=K, F=F, D=D, wd=wdt)), 0)
+    assert at("flexsae_topk_bwd_workspace_bytes", 1 << 20) == at("flexsae_topk_bwd_workspace_bytes", 256)
+    f0, f1 = B * K // 8, B * K // 2 - 1
+    list_bytes = lambda F: (4 * (F + 1) + 255) // 256 * 256 + lib.flexsae_csr_workspace_bytes(B, K, F)
+    grown = at("flexsae_hier_bwd_workspace_bytes", f1) - at("flexsae_hier_bwd_workspace_bytes", f0)
+    assert grown == list_bytes(f1) - list_bytes(f0)
+    # at two pairs per latent the reduction may work from the lists: four bytes per latent and more
+    grown = at("flexsae_hier_bwd_workspace_bytes", 1 << 20) - at("flexsae_hier_bwd_workspace_bytes", f0)
+    assert grown >= list_bytes(1 << 20) - list_bytes(f0) + (4 << 20)
