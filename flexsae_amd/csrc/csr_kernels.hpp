@@ -440,34 +440,36 @@ __global__ __launch_bounds__(1024) void csr_sort_long_kernel(const uint32_t *__r
 //                           buckets, so no scan over the table is needed in between.  Per-latent counts
 //                           -> begin[], the lists, and map[] ascending inside every latent.
 // Bound by latency (a few dependent passes over a megabyte) and by launches, which cost 4-5 us each in a
-// busy stream.  B*K = 524288 over 65536 latents: 8 + 15 us; 524288 Zipf pairs over 262144 latents: 9 + 56 us
-// (count, two scan launches, scatter, bucket sort, long-group sort, chunk table and, for sparse shapes, two
-// launches for the lists before: 41 and 115 us).
+// busy stream; where frequent latents share a bucket, by the instructions of that bucket's one block.
 // ---------------------------------------------------------------------------------
 constexpr int kChunkThreads = 256;
 constexpr int kChunkWaves = kChunkThreads / kWave;
 constexpr int kBucketMaxBuckets = 8192;  // LDS cursors of the chunk kernel: 4 bytes per wavefront and bucket
 constexpr int kSortThreads = kListThreads;
-constexpr int kSortMaxShift = 11;
+constexpr int kSortMaxShift = 12;
 constexpr int kSortMaxLatents = 1 << kSortMaxShift;  // latents per bucket at most
-constexpr int kSortCap = 4096;                       // pairs of a bucket that are kept in the LDS
-constexpr int kSortWindow = 1024;                    // chunks whose pieces are collected together
-constexpr int kPackShift = 32 - kSortMaxShift;       // a pair inside its chunk: latent within bucket | place in the chunk
-constexpr int64_t kMaxChunk = int64_t{1} << kPackShift;
+constexpr int kSortCap = 4096;                       // pairs of a bucket that its block keeps in registers
+constexpr int kSortChunks = 2048;                    // chunks at most
+constexpr int kRunLatents = 512;                     // latents of a larger bucket that are placed together
 static_assert((kBucketMaxBuckets * kChunkWaves + kChunkWaves) * 4 <= 160 * 1024, "LDS of csr_chunk_sort_kernel");
-// (the bucket kernel's arrays come to 71 KB: two blocks per compute unit)
+constexpr int64_t kBucketBlocks = 512;  // blocks of the bucket kernel on the chip at once (77 KB of LDS: two per compute unit)
 
-// Dynamic LDS: kChunkWaves * n_buckets + kChunkWaves words.  n_bits: bits of a bucket number.
+// A pair inside its chunk is one word: latent within its bucket << pack_shift | place in the chunk.
+inline int csr_pack_shift(int shift) { return 32 - (shift > 11 ? shift : 11); }
+
+// Dynamic LDS: (n_buckets rounded up to four + 1) * kChunkWaves words.  n_bits: bits of a bucket number.
 __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
-    const int64_t *__restrict__ indices, int64_t n_pairs, int64_t F, int shift, uint32_t n_buckets, int n_bits,
+    const int64_t *__restrict__ indices, int64_t n_pairs, int64_t F, int shift, int pack_shift, uint32_t n_buckets, int n_bits,
     int64_t chunk, uint32_t n_chunks, uint32_t *__restrict__ table, uint32_t *__restrict__ tmp,
     uint32_t *__restrict__ ctrl, int *status_flag) {
-  extern __shared__ uint32_t chunk_lds[];
+  extern __shared__ __align__(16) uint32_t chunk_lds[];
+  using four_t = vec_t<uint32_t, 4>;
+  const uint32_t n_cursors = (n_buckets + 3u) & ~3u;
   uint32_t *const cursor = chunk_lds;                            // [wavefront][bucket]
-  uint32_t *const wave_tot = chunk_lds + kChunkWaves * n_buckets;
+  uint32_t *const wave_tot = chunk_lds + kChunkWaves * n_cursors;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = wave_in_block();
   if (blockIdx.x == 0 && tid < kCtrlWords) ctrl[tid] = 0u;
-  for (uint32_t q = tid; q < kChunkWaves * n_buckets; q += kChunkThreads) cursor[q] = 0u;
+  for (uint32_t q = tid; q < kChunkWaves * n_cursors / 4; q += kChunkThreads) reinterpret_cast<four_t *>(cursor)[q] = four_t{};
   __syncthreads();
   const int64_t p0 = static_cast<int64_t>(blockIdx.x) * chunk;
   const int64_t n = (n_pairs - p0) < chunk ? (n_pairs - p0) : chunk;
@@ -488,7 +490,7 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
         f[u] = 0;
       }
   };
-  uint32_t *const mine = cursor + wv * n_buckets;
+  uint32_t *const mine = cursor + wv * n_cursors;
   for (int64_t at = r0; at < r1; at += U * kWave) {
     int64_t f[U];
     load(at, f, true);
@@ -497,13 +499,18 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
       if (at + u * kWave + lane < r1) atomicAdd(&mine[f[u] >> shift], 1u);
   }
   __syncthreads();
-  {  // exclusive scan over (bucket, wavefront): every thread owns `per` consecutive buckets
-    const uint32_t per = (n_buckets + kChunkThreads - 1) / kChunkThreads;
-    const uint32_t q0 = tid * per, q1 = (q0 + per) < n_buckets ? (q0 + per) : n_buckets;
+  // exclusive scan over (bucket, wavefront), four buckets per thread and round
+  uint32_t earlier = 0;  // pairs of the buckets of earlier rounds
+  for (uint32_t q0 = 0; q0 < n_buckets; q0 += 4 * kChunkThreads) {
+    const uint32_t q = q0 + 4 * tid;
+    four_t c[kChunkWaves];
     uint32_t sum = 0;
-    for (uint32_t q = q0; q < q1; ++q)
 #pragma unroll
-      for (int w = 0; w < kChunkWaves; ++w) sum += cursor[w * n_buckets + q];
+    for (int w = 0; w < kChunkWaves; ++w) {
+      c[w] = four_t{};
+      if (q < n_buckets) c[w] = *reinterpret_cast<const four_t *>(cursor + w * n_cursors + q);
+      sum += c[w][0] + c[w][1] + c[w][2] + c[w][3];
+    }
     uint32_t inc = sum;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {
@@ -512,20 +519,29 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
     }
     if (lane == kWave - 1) wave_tot[wv] = inc;
     __syncthreads();
-    uint32_t at = inc - sum;
-    for (int w = 0; w < wv; ++w) at += wave_tot[w];
-    for (uint32_t q = q0; q < q1; ++q) {
-      table[static_cast<size_t>(q) * n_chunks + blockIdx.x] = at;
+    uint32_t at = earlier + inc - sum;
+#pragma unroll
+    for (int w = 0; w < kChunkWaves; ++w) {
+      if (w < wv) at += wave_tot[w];
+      earlier += wave_tot[w];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (q + i < n_buckets) table[static_cast<size_t>(q + i) * n_chunks + blockIdx.x] = at;
 #pragma unroll
       for (int w = 0; w < kChunkWaves; ++w) {
-        const uint32_t c = cursor[w * n_buckets + q];
-        cursor[w * n_buckets + q] = at;
-        at += c;
+        const uint32_t mine_c = c[w][i];
+        c[w][i] = at;
+        at += mine_c;
       }
     }
-    if (tid == 0) table[static_cast<size_t>(n_buckets) * n_chunks + blockIdx.x] = static_cast<uint32_t>(n);
+    if (q < n_buckets) {
+#pragma unroll
+      for (int w = 0; w < kChunkWaves; ++w) *reinterpret_cast<four_t *>(cursor + w * n_cursors + q) = c[w];
+    }
+    __syncthreads();
   }
-  __syncthreads();
+  if (tid == 0) table[static_cast<size_t>(n_buckets) * n_chunks + blockIdx.x] = static_cast<uint32_t>(n);
   const int64_t mask = (static_cast<int64_t>(1) << shift) - 1;
   for (int64_t at = r0; at < r1; at += U * kWave) {
     int64_t f[U];
@@ -545,7 +561,7 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0u));
       if (have) {
         const uint32_t place = mine[q] + rank;
-        tmp[p0 + place] = (static_cast<uint32_t>(f[u] & mask) << kPackShift) | static_cast<uint32_t>(i);
+        tmp[p0 + place] = (static_cast<uint32_t>(f[u] & mask) << pack_shift) | static_cast<uint32_t>(i);
         // (LDS accesses of a wavefront are served in order: all lanes have read the cursor)
         if (rank == 0) mine[q] = place + static_cast<uint32_t>(__popcll(same));
       }
@@ -555,11 +571,12 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
 }
 
 // counter[at] += 1 for every lane with `have`, in the LDS.  The lanes that agree with the first one add up
-// beforehand (twice over): adds to one address are served one lane after the other, and a frequent latent
+// beforehand (ROUNDS times over): adds to one address are served one lane after the other, and a frequent latent
 // is most of its bucket.
+template <int ROUNDS>
 __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, bool have) {
 #pragma unroll
-  for (int round = 0; round < 2; ++round) {
+  for (int round = 0; round < ROUNDS; ++round) {
     const unsigned long long left = __ballot(have);
     if (left == 0) return;  // uniform
     const int leader = __builtin_ctzll(left);
@@ -574,346 +591,373 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
 
 // One block per bucket.  hslot: a second copy of slot[] (null: none).  solo_bit: marks in both the only pair of
 // its latent (0: no marks).
-// Groups of more than kListLong pairs (frequent latents) are placed by walking the bucket's pairs in order:
-// every wavefront takes a run of them, counts its pairs of every such latent, and places them behind those
-// of the wavefronts before it.  The others are gathered in the LDS in any order, and every pair counts
-// the smaller ids of its group.
+// The pieces of a bucket, one from every chunk, hold its pairs in pair order: pair i of the bucket is found by a search
+// for its chunk in first[].
+//   Up to kSortCap pairs: four to a thread, kept in registers.  Groups of up to kListLong pairs are gathered in the LDS in
+//     any order, and every pair counts the smaller ids of its group.  Pairs of longer groups (frequent latents) are placed
+//     by wavefront: a round of a wavefront is 64 consecutive pairs, and goes behind the rounds before it.
+//   More pairs (frequent latents among them): every wavefront walks a run of the bucket's pairs twice, kRunLatents
+//     latents at a time; first it counts its pairs of every latent, then it places them behind those of the wavefronts
+//     before it.  Nothing is searched for within a piece of 64 pairs or more.  The blocks of a bucket (gridDim.y) share
+//     the batches of latents, where there is room for more blocks than buckets.  What bounds it are the instructions of
+//     one compute unit (and a line per pair of the stores, where every pair goes to another group).
+// Pair list, us; in brackets with every pair searched for, separate passes for long and short groups and the latter in
+// batches that fit the LDS: 524288 pairs of 65536 latents, uniform: 21 (24); 262144 of 262144, skewed, latents in any
+// order: 75 (96), latents by frequency: 298 (3336), half of the pairs on the first 32 latents: 144 (317); 64 latents in
+// every one of 16384 rows: 1329 (2584).
 __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
     const uint32_t *__restrict__ tmp, const uint32_t *__restrict__ table, uint32_t n_chunks, int64_t chunk, int shift,
-    int64_t F, uint32_t *__restrict__ begin, uint32_t *__restrict__ map, uint32_t *__restrict__ slot,
+    int pack_shift, int64_t F, uint32_t *__restrict__ begin, uint32_t *__restrict__ map, uint32_t *__restrict__ slot,
     uint32_t *__restrict__ hslot, uint32_t solo_bit, PairLists ls) {
   constexpr int kWaves = kSortThreads / kWave;
-  constexpr int PER = kSortMaxLatents / kSortThreads;
-  constexpr uint32_t kRunLatents = kSortCap / kWaves;  // frequent latents counted per wavefront at a time
-  constexpr uint32_t kShort = 0xffffu;
-  __shared__ uint32_t cnt[kSortMaxLatents + 1];    // pairs per latent, then their exclusive scan
-  __shared__ uint32_t shorts[kSortMaxLatents + 1]; // the same over the groups of up to kListLong pairs
-  __shared__ uint16_t lid[kSortMaxLatents];        // number of a frequent latent, or kShort
-  __shared__ uint32_t ids[kSortCap];               // cursors [wavefront][frequent latent], then short groups' pair ids
-  __shared__ uint32_t list_id[kSortCap];           // the bucket's pairs in pair order, where they fit
-  __shared__ uint16_t list_key[kSortCap];          //   and their latents
-  __shared__ uint32_t first[kSortWindow + 1];      // window of chunks: first place of each chunk's piece in the list
-  __shared__ uint32_t from[kSortWindow + 1];       //   and its place inside the chunk
+  constexpr int PER = kSortMaxLatents / kSortThreads;  // latents per thread
+  constexpr int kPairs = kSortCap / kSortThreads;      // pairs per thread
+  constexpr int CPER = kSortChunks / kSortThreads;     // chunks per thread
+  __shared__ __align__(16) uint32_t cnt[kSortMaxLatents + 4];  // pairs per latent, then their exclusive scan
+  __shared__ uint8_t lid[kSortMaxLatents];        // number of a frequent latent
+  // up to kSortCap pairs: first half cursors [frequent latent][round], then the pair ids of short groups; second half
+  // the next place of every latent.  More: cursors [wavefront][latent of the batch]
+  __shared__ __align__(16) uint32_t ids[kWaves * kRunLatents];
+  __shared__ uint32_t first[kSortChunks + 1];     // first pair of each chunk's piece; the number of pairs beyond the last
+  __shared__ uint32_t from[kSortChunks];          // what to add to the number of a pair of that piece for its place in tmp[]
   __shared__ uint32_t wave_tot[kWaves], wave_tot2[kWaves];
-  __shared__ uint32_t n_long_s, n_short_s;
+  __shared__ unsigned long long agree[kWaves][kWave];
+  __shared__ uint32_t n_long_s;
   __shared__ AppendScratch sh;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = wave_in_block();
+  static_assert(kWaves * kRunLatents >= kSortCap + kSortMaxLatents, "ids and next places");
+  constexpr uint32_t kRounds = kSortCap / kWave;
+  static_assert(kRounds == kWave && (kSortCap / (kListLong + 1)) * kRounds <= kSortCap && kSortCap / (kListLong + 1) <= 64,
+                "a lane per round, cursors of all frequent latents, six bits for the number of one");
+  uint32_t *const next_place = ids + kSortCap;
+  using latents_t = vec_t<uint32_t, PER>;
+  const int tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
   const uint32_t q = blockIdx.x;
   const uint32_t lpb = 1u << shift;
   const int64_t f0 = static_cast<int64_t>(q) << shift;
   const uint32_t nlat = (F - f0) < static_cast<int64_t>(lpb) ? static_cast<uint32_t>(F - f0) : lpb;
-  const uint32_t *const row0 = table + static_cast<size_t>(q) * n_chunks;
-  const uint32_t *const row1 = row0 + n_chunks;
+  const uint32_t place_mask = (1u << pack_shift) - 1u;
+  const uint32_t chunk_w = static_cast<uint32_t>(chunk);
+  const uint32_t my_k = static_cast<uint32_t>(tid) * PER;
 
-  // base = pairs in earlier buckets, n = pairs in this one
+  // base = pairs in earlier buckets, n = pairs in this one; the table of the pieces
   uint32_t base = 0, n = 0;
   {
-    uint32_t s0 = 0, s1 = 0;
-    for (uint32_t c = tid; c < n_chunks; c += kSortThreads) {
-      s0 += row0[c];
-      s1 += row1[c];
-    }
+    const uint32_t *const row0 = table + static_cast<size_t>(q) * n_chunks;
+    uint32_t at[CPER], len[CPER], s0 = 0, s1 = 0;
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      s0 += static_cast<uint32_t>(__shfl_xor(static_cast<int>(s0), off, kWave));
-      s1 += static_cast<uint32_t>(__shfl_xor(static_cast<int>(s1), off, kWave));
+    for (int j = 0; j < CPER; ++j) {
+      const uint32_t c = static_cast<uint32_t>(tid) * CPER + j;
+      at[j] = len[j] = 0;
+      if (c < n_chunks) {
+        at[j] = row0[c];
+        len[j] = row0[n_chunks + c] - at[j];
+      }
+      s0 += at[j];
+      s1 += len[j];
     }
-    if (lane == 0) {
-      wave_tot[wv] = s0;
-      wave_tot2[wv] = s1;
-    }
-    for (uint32_t k = tid; k <= lpb; k += kSortThreads) cnt[k] = 0u;
-    if (tid == 0) n_long_s = n_short_s = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      base += wave_tot[w];
-      n += wave_tot2[w];
-    }
-    n -= base;
-  }
-  const bool listed = n <= static_cast<uint32_t>(kSortCap) && n_chunks <= static_cast<uint32_t>(kSortWindow);
-
-  // The pieces of the window of chunks that begins at c0: fills first[] and from[], returns the number of pairs.
-  auto open_window = [&](uint32_t c0) {
-    static_assert(kSortWindow == kSortThreads, "one chunk per thread");
-    const uint32_t c = c0 + tid;
-    uint32_t len = 0, at = 0;
-    if (c < n_chunks) {
-      at = row0[c];
-      len = row1[c] - at;
-    }
-    uint32_t inc = len;
+    uint32_t inc = s1;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {
       const uint32_t y = __shfl_up(inc, off, kWave);
       if (lane >= off) inc += y;
     }
-    __syncthreads();  // the window before has been read by everybody
-    if (lane == kWave - 1) wave_tot[wv] = inc;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) s0 += static_cast<uint32_t>(__shfl_xor(static_cast<int>(s0), off, kWave));
+    if (lane == kWave - 1) {
+      wave_tot[wv] = inc;
+      wave_tot2[wv] = s0;
+    }
+    for (uint32_t k = my_k; k <= lpb; k += kSortThreads * PER) *reinterpret_cast<latents_t *>(cnt + k) = latents_t{};
+    agree[wv][lane] = 0ull;
+    if (tid == 0) n_long_s = 0u;
     __syncthreads();
-    uint32_t start = inc - len, m = 0;
+    uint32_t start = inc - s1;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
+      base += wave_tot2[w];
       if (w < wv) start += wave_tot[w];
-      m += wave_tot[w];
+      n += wave_tot[w];
     }
-    first[tid] = start;
-    from[tid] = at;
+#pragma unroll
+    for (int j = 0; j < CPER; ++j) {
+      const uint32_t c = static_cast<uint32_t>(tid) * CPER + j;
+      first[c] = start;
+      from[c] = c * chunk_w + at[j] - start;  // (modulo 2^32, as the sum with a pair's number: fewer than 2^32 pairs)
+      start += len[j];
+    }
+    if (tid == 0) first[kSortChunks] = n;
     __syncthreads();
-    return m;
-  };
-  // U pairs of that window at once, from the chunks or from the list where there is one: i[u], any pair where i[u] >= m
-  uint32_t probes = 1;  // a power of two, at least the number of chunks in a window
-  while (probes < n_chunks && probes < static_cast<uint32_t>(kSortWindow)) probes <<= 1;
-  auto fetch = [&](uint32_t c0, uint32_t m, bool from_list, const auto &i, auto &key, auto &id) {
-    constexpr int U = sizeof(i) / sizeof(i[0]);
-    if (from_list) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t at = i[u] < m ? i[u] : 0u;
-        key[u] = list_key[at];
-        id[u] = list_id[at];
-      }
-      return;
-    }
-    uint32_t at[U], c[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      at[u] = i[u] < m ? i[u] : 0u;
-      c[u] = 0;
-    }
-    // largest chunk with first[chunk] <= i (an empty chunk repeats its successor's place; past the last one: m)
-    for (uint32_t step = probes >> 1; step > 0; step >>= 1)
-#pragma unroll
-      for (int u = 0; u < U; ++u) c[u] += first[c[u] + step] <= at[u] ? step : 0u;
-    uint32_t v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      v[u] = tmp[static_cast<int64_t>(c0 + c[u]) * chunk + from[c[u]] + (at[u] - first[c[u]])];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      key[u] = v[u] >> kPackShift;
-      id[u] = static_cast<uint32_t>(static_cast<int64_t>(c0 + c[u]) * chunk) + (v[u] & static_cast<uint32_t>(kMaxChunk - 1));
-    }
-  };
-  // body(i, key, id, valid) for the pairs begin, begin + stride, ... of the window, U of them requested together; called
-  // by all lanes of a wavefront alike, valid: below end
-  auto for_pairs = [&](uint32_t c0, uint32_t m, bool from_list, uint32_t begin_i, uint32_t end_i, uint32_t stride, auto body) {
-    constexpr int U = 4;
-    for (uint32_t i0 = begin_i; __any(i0 < end_i); i0 += U * stride) {
-      uint32_t i[U], key[U], id[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) i[u] = i0 + u * stride;
-      fetch(c0, m, from_list, i, key, id);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        body(i[u], key[u], id[u], i[u] < end_i);
-    }
-  };
-  // body(c0, m) for every window of chunks; a single window stays open
-  uint32_t open_m = 0;
-  const bool one_window = n_chunks <= static_cast<uint32_t>(kSortWindow);
-  if (one_window) open_m = open_window(0);
-  auto for_windows = [&](auto body) {
-    for (uint32_t c0 = 0; c0 < n_chunks; c0 += kSortWindow) body(c0, one_window ? open_m : open_window(c0));
-  };
-
-  for_windows([&](uint32_t c0, uint32_t m) {
-    for_pairs(c0, m, false, tid, m, kSortThreads, [&](uint32_t i, uint32_t key, uint32_t id, bool valid) {
-      if (listed && valid) {
-        list_id[i] = id;
-        list_key[i] = static_cast<uint16_t>(key);
-      }
-      count_in_lds(cnt, key, valid);
-    });
-  });
-  __syncthreads();
-  uint32_t x[PER];  // pairs of the thread's latents
-  {  // exclusive scans of all groups and of the short ones
-    uint32_t y[PER], xs = 0, ys = 0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const uint32_t k = static_cast<uint32_t>(tid) * PER + i;
-      x[i] = (k < lpb) ? cnt[k] : 0u;
-      y[i] = x[i] > kListLong ? 0u : x[i];
-      if (k < lpb) lid[k] = static_cast<uint16_t>(x[i] > kListLong ? atomicAdd(&n_long_s, 1u) : kShort);
-      xs += x[i];
-      ys += y[i];
-    }
-    uint32_t xi = xs, yi = ys;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint32_t a = __shfl_up(xi, off, kWave), b = __shfl_up(yi, off, kWave);
-      if (lane >= off) {
-        xi += a;
-        yi += b;
-      }
-    }
-    if (lane == kWave - 1) {
-      wave_tot[wv] = xi;
-      wave_tot2[wv] = yi;
-    }
-    __syncthreads();
-    uint32_t xr = xi - xs, yr = yi - ys;
-    for (int w = 0; w < wv; ++w) {
-      xr += wave_tot[w];
-      yr += wave_tot2[w];
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const uint32_t k = static_cast<uint32_t>(tid) * PER + i;
-      if (k < nlat) begin[f0 + k] = base + xr;
-      if (k < lpb) {
-        cnt[k] = xr;
-        shorts[k] = yr;
-      }
-      xr += x[i];
-      yr += y[i];
-    }
-    if (tid == kSortThreads - 1) {
-      cnt[lpb] = xr;
-      shorts[lpb] = yr;
-      if (q == gridDim.x - 1) begin[F] = base + n;
-    }
   }
-  if (ls.chunk_begin) {  // uniform
-    const uint32_t k = static_cast<uint32_t>(tid) * PER;
-    append_latents(ls, f0 + k, nlat >= k + PER ? PER : nlat > k ? static_cast<int>(nlat - k) : 0, x, sh);
-  }
-  __syncthreads();
-
+  uint32_t probes = 1;  // a power of two, at least the number of chunks
+  while (probes < n_chunks) probes <<= 1;
+  // largest chunk with first[chunk] <= i (an empty piece repeats its successor's place)
+  auto chunk_of = [&](uint32_t i) {
+    uint32_t c = 0;
+    for (uint32_t step = probes >> 1; step > 0; step >>= 1) c += first[c + step] <= i ? step : 0u;
+    return c;
+  };
   auto put = [&](uint32_t place, uint32_t id, uint32_t mark) {
     map[place] = id;
     if (slot) slot[id] = place | mark;
     if (hslot) hslot[id] = place | mark;
   };
-  // frequent latents, kRunLatents of them at a time; where the bucket's list did not fit the LDS but its other
-  // pairs do, those are listed on the way
-  const uint32_t n_long = n_long_s;
-  const bool collect = !listed && n_long != 0 && shorts[nlat] <= static_cast<uint32_t>(kSortCap);
-  for (uint32_t l0 = 0; l0 < n_long; l0 += kRunLatents) {
-    const uint32_t nl = (n_long - l0) < kRunLatents ? (n_long - l0) : kRunLatents;
-    uint32_t bits = 0;
-    while ((1u << bits) < nl) ++bits;
-    uint32_t *const mine = ids + wv * kRunLatents;
-    bool opened = false;
-    for_windows([&](uint32_t c0, uint32_t m) {
-      uint32_t run = (m + kWaves - 1) / kWaves;
-      run = (run + kWave - 1) / kWave * kWave;
-      const uint32_t r0 = wv * run, r1 = (r0 + run) < m ? (r0 + run) : m;
-      // wavefront 0's cursors go on from the window before; the others' hold counts until the scan below
-      for (uint32_t l = lane; l < nl; l += kWave)
-        if (wv != 0 || !opened) mine[l] = 0u;
-      __syncthreads();
-      if (!opened)
-        for (uint32_t k = tid; k < nlat; k += kSortThreads) {
-          const uint32_t l = lid[k] - l0;
-          if (lid[k] != kShort && l < nl) ids[l] = base + cnt[k];
-        }
-      opened = true;
-      __syncthreads();
-      // wavefront w counts into the cursors of wavefront w + 1
-      if (wv + 1 < kWaves) {
-        for_pairs(c0, m, listed, r0 + lane, r1, kWave, [&](uint32_t, uint32_t key, uint32_t, bool valid) {
-          const uint32_t l = lid[key] - l0;
-          count_in_lds(mine + kRunLatents, l, valid && lid[key] != kShort && l < nl);
-        });
-      }
-      __syncthreads();
-      for (uint32_t l = tid; l < nl; l += kSortThreads) {
-        uint32_t at = ids[l];
-        for (int w = 1; w < kWaves; ++w) {
-          at += ids[w * kRunLatents + l];
-          ids[w * kRunLatents + l] = at;
-        }
-      }
-      __syncthreads();
-      constexpr int U = 4;
-      for (uint32_t i0 = r0; i0 < r1; i0 += U * kWave) {
-        uint32_t i[U], key[U], id[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) i[u] = i0 + u * kWave + lane;
-        fetch(c0, m, listed, i, key, id);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t l = lid[key[u]] - l0;
-          const bool have = i[u] < r1 && lid[key[u]] != kShort && l < nl;
-          if (collect && l0 == 0) {  // uniform
-            const bool is_short = i[u] < r1 && lid[key[u]] == kShort;
-            const unsigned long long with = __ballot(is_short);
-            uint32_t at = 0;
-            if (lane == 0 && with) at = atomicAdd(&n_short_s, static_cast<uint32_t>(__popcll(with)));
-            at = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
-            if (is_short) {
-              at += __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(with >> 32),
-                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(with), 0u));
-              list_id[at] = id[u];
-              list_key[at] = static_cast<uint16_t>(key[u]);
-            }
-          }
-          unsigned long long same = __ballot(have);
-          if (same == 0) continue;
-          for (uint32_t b = 0; b < bits; ++b) {
-            const unsigned long long ones = __ballot((l >> b) & 1u);
-            same &= ((l >> b) & 1u) ? ones : ~ones;
-          }
-          const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(same >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0u));
-          if (have) {
-            const uint32_t place = mine[l] + rank;
-            put(place, id[u], 0u);
-            if (rank == 0) mine[l] = place + static_cast<uint32_t>(__popcll(same));
-          }
-          __builtin_amdgcn_wave_barrier();
-        }
-      }
-      __syncthreads();
-      // the last wavefront's cursors are where the next window goes on
-      for (uint32_t l = tid; l < nl; l += kSortThreads) ids[l] = ids[(kWaves - 1) * kRunLatents + l];
-      __syncthreads();
-    });
-  }
-
-  // short groups, as many consecutive latents at a time as the LDS holds the pairs of (usually all)
-  auto for_shorts = [&](auto body) {
-    if (collect) for_pairs(0, n_short_s, true, tid, n_short_s, kSortThreads, body);
-    else for_windows([&](uint32_t c0, uint32_t m) { for_pairs(c0, m, listed, tid, m, kSortThreads, body); });
-  };
-  for (uint32_t k0 = 0; k0 < nlat;) {  // uniform
-    const uint32_t s0 = shorts[k0];
-    uint32_t k1 = nlat;
-    if (shorts[nlat] - s0 > static_cast<uint32_t>(kSortCap)) {
-      uint32_t lo = k0 + 1, hi = nlat;  // largest k1 with shorts[k1] - s0 <= kSortCap
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (shorts[mid] - s0 <= static_cast<uint32_t>(kSortCap)) lo = mid; else hi = mid - 1;
-      }
-      k1 = lo;
+  // the lanes (of those with `have`, at least one) that agree with this one in the low `bits` bits of key: the first
+  // lane's followers by a ballot (a frequent latent), the others by their marks in the LDS under the key's low six bits
+  // and a ballot for each bit above.  Seven vector operations for each of nine bits cost the walk below a fifth more.
+  auto agreeing = [&](uint32_t key, bool have, uint32_t bits) {
+    const int leader = __builtin_ctzll(__ballot(have));
+    const bool led = have && key == static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), leader));
+    unsigned long long same = __ballot(led);
+    if (have && !led) {
+      // (LDS accesses of a wavefront are served in order)
+      unsigned long long *const mark = &agree[wv][key & (kWave - 1)];
+      atomicOr(mark, 1ull << lane);
+      same = *mark;
+      *mark = 0ull;
     }
-    __syncthreads();  // everybody has read shorts[] and is done with ids[]
-    // placed in the order of the atomics, which leave shorts[k] at the end of group k
-    for_shorts([&](uint32_t, uint32_t key, uint32_t id, bool valid) {
-      if (valid && key >= k0 && key < k1 && lid[key] == kShort) ids[atomicAdd(&shorts[key], 1u) - s0] = id;
-    });
+    for (uint32_t b = 6; b < bits; ++b) {
+      const unsigned long long ones = __ballot((key >> b) & 1u);
+      if (!led) same &= ((key >> b) & 1u) ? ones : ~ones;
+    }
+    return same;
+  };
+  auto lanes_before = [](unsigned long long with) {
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(with >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(with), 0u));
+  };
+
+  if (n <= static_cast<uint32_t>(kSortCap)) {  // uniform
+    if (blockIdx.y != 0) return;
+    uint32_t x[PER] = {};  // pairs of the thread's latents
+    const int my_n = nlat >= my_k + PER ? PER : nlat > my_k ? static_cast<int>(nlat - my_k) : 0;
+    if (n == 0) {
+      for (uint32_t k = tid; k < nlat; k += kSortThreads) begin[f0 + k] = base;
+      if (tid == 0 && q == gridDim.x - 1) begin[F] = base;
+      if (ls.chunk_begin) append_latents(ls, f0 + my_k, my_n, x, sh);
+      return;
+    }
+    uint32_t key[kPairs], id[kPairs];
+    const int rounds = static_cast<int>((n + kSortThreads - 1) / kSortThreads);
+    {
+      uint32_t c[kPairs], v[kPairs];
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u) {
+        if (u < rounds) {  // uniform
+          const uint32_t i = static_cast<uint32_t>(tid) + u * kSortThreads;
+          const uint32_t at = i < n ? i : 0u;
+          c[u] = chunk_of(at);
+          v[u] = tmp[from[c[u]] + at];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u) {
+        key[u] = id[u] = 0;
+        if (u < rounds) {
+          key[u] = v[u] >> pack_shift;
+          id[u] = c[u] * chunk_w + (v[u] & place_mask);
+          count_in_lds<2>(cnt, key[u], static_cast<uint32_t>(tid) + u * kSortThreads < n);
+        }
+      }
+    }
     __syncthreads();
-    for_shorts([&](uint32_t, uint32_t key, uint32_t id, bool valid) {
-      if (!valid || key < k0 || key >= k1 || lid[key] != kShort) return;
-      const uint32_t len = cnt[key + 1] - cnt[key];
-      const uint32_t *const group = ids + (shorts[key] - len - s0);
+    {  // exclusive scan over the latents
+      uint32_t xs = 0;
+      latents_t own = {};
+      if (my_k < lpb) own = *reinterpret_cast<const latents_t *>(cnt + my_k);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        x[i] = my_k + i < lpb ? own[i] : 0u;
+        if (x[i] > kListLong) lid[my_k + i] = static_cast<uint8_t>(atomicAdd(&n_long_s, 1u));
+        xs += x[i];
+      }
+      uint32_t xi = xs;
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t y = __shfl_up(xi, off, kWave);
+        if (lane >= off) xi += y;
+      }
+      if (lane == kWave - 1) wave_tot[wv] = xi;
+      __syncthreads();
+      uint32_t run = xi - xs;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w)
+        if (w < wv) run += wave_tot[w];
+      latents_t at;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        at[i] = run;
+        run += x[i];
+      }
+      if (my_k <= lpb) *reinterpret_cast<latents_t *>(cnt + my_k) = at;  // (n beyond the last latent)
+      if (my_k < lpb) *reinterpret_cast<latents_t *>(next_place + my_k) = at;
+      if (lpb == kSortMaxLatents && tid == 0) cnt[lpb] = n;
+    }
+    __syncthreads();
+    for (uint32_t k = tid; k < nlat; k += kSortThreads) begin[f0 + k] = base + cnt[k];
+    const uint32_t n_long = n_long_s;
+    if (n_long != 0) {  // uniform
+      uint32_t bits = 0;
+      while ((1u << bits) < n_long) ++bits;
+      for (uint32_t l = tid; l < n_long * kRounds; l += kSortThreads) ids[l] = 0u;
+      __syncthreads();
+      auto is_long = [&](int u) {
+        return static_cast<uint32_t>(tid) + u * kSortThreads < n && cnt[key[u] + 1] - cnt[key[u]] > kListLong;
+      };
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u)
+        if (u < rounds) {
+          const bool have = is_long(u);
+          count_in_lds<2>(ids, have ? lid[key[u]] * kRounds + u * kWaves + wv : 0u, have);
+        }
+      __syncthreads();
+      for (uint32_t l = wv; l < n_long; l += kWaves) {  // a wavefront per latent, a lane per round
+        const uint32_t own = ids[l * kRounds + lane];
+        uint32_t inc = own;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+          const uint32_t y = __shfl_up(inc, off, kWave);
+          if (lane >= off) inc += y;
+        }
+        ids[l * kRounds + lane] = inc - own;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u)
+        if (u < rounds) {
+          const bool have = is_long(u);
+          if (!__any(have)) continue;
+          const uint32_t l = have ? lid[key[u]] : 0u;
+          const unsigned long long same = agreeing(l, have, bits);
+          if (have) put(base + cnt[key[u]] + ids[l * kRounds + u * kWaves + wv] + lanes_before(same), id[u], 0u);
+        }
+      __syncthreads();
+    }
+    // short groups: placed in the order of the atomics, then ranked
+#pragma unroll
+    for (int u = 0; u < kPairs; ++u)
+      if (static_cast<uint32_t>(tid) + u * kSortThreads < n && cnt[key[u] + 1] - cnt[key[u]] <= kListLong)
+        ids[atomicAdd(&next_place[key[u]], 1u)] = id[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPairs; ++u) {
+      if (static_cast<uint32_t>(tid) + u * kSortThreads >= n) continue;
+      const uint32_t start = cnt[key[u]], len = cnt[key[u] + 1] - start;
+      if (len > kListLong) continue;
+      const uint32_t *const group = ids + start;
       uint32_t rank = 0, j = 0;
       for (; j + 8 <= len; j += 8) {
-        uint32_t x[8];
+        uint32_t y[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = group[j + u];
+        for (int w = 0; w < 8; ++w) y[w] = group[j + w];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) rank += (x[u] < id) ? 1u : 0u;
+        for (int w = 0; w < 8; ++w) rank += (y[w] < id[u]) ? 1u : 0u;
       }
-      for (; j < len; ++j) rank += (group[j] < id) ? 1u : 0u;
-      put(base + cnt[key] + rank, id, len == 1 ? solo_bit : 0u);
-    });
-    k0 = k1;
+      for (; j < len; ++j) rank += (group[j] < id[u]) ? 1u : 0u;
+      put(base + start + rank, id[u], len == 1 ? solo_bit : 0u);
+    }
+    if (ls.chunk_begin) append_latents(ls, f0 + my_k, my_n, x, sh);
+  } else {
+    uint32_t run = (n + kWaves - 1) / kWaves;
+    run = (run + kWave - 1) / kWave * kWave;
+    const uint32_t r0 = wv * run, r1 = (r0 + run) < n ? (r0 + run) : n;
+    // body(key, id, valid) for the wavefront's pairs in order, 64 at a time
+    auto walk = [&](auto body) {
+      constexpr int U = 8;
+      uint32_t hi = 0, off = 0, id0 = 0;  // pairs from the last one looked at to hi lie in one piece
+      for (uint32_t i0 = r0; i0 < r1; i0 += U * kWave) {
+        uint32_t v[U], idb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t at = i0 + u * kWave;  // uniform
+          v[u] = idb[u] = 0;
+          if (at >= r1) continue;
+          const uint32_t i = at + lane < n ? at + lane : n - 1;
+          if (at + kWave <= hi) {
+            v[u] = tmp[off + i];
+            idb[u] = id0;
+          } else {
+            const uint32_t c = chunk_of(i);
+            v[u] = tmp[from[c] + i];
+            idb[u] = c * chunk_w;
+            const uint32_t last = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(c), kWave - 1));
+            hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(first[last + 1])));
+            off = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(from[last])));
+            id0 = last * chunk_w;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t at = i0 + u * kWave;
+          if (at < r1) body(v[u] >> pack_shift, idb[u] + (v[u] & place_mask), at + lane < r1);
+        }
+      }
+    };
+    uint32_t *const mine = ids + wv * kRunLatents;
+    const uint32_t batch = lpb < static_cast<uint32_t>(kRunLatents) ? lpb : static_cast<uint32_t>(kRunLatents);
+    uint32_t bits = 0;
+    while ((1u << bits) < batch) ++bits;
+    for (uint32_t k0 = blockIdx.y * batch; k0 < nlat; k0 += gridDim.y * batch) {  // uniform
+      for (uint32_t l = tid; l < kWaves * kRunLatents; l += kSortThreads) ids[l] = 0u;
+      __syncthreads();
+      uint32_t before = 0;  // this lane's pairs of the latents before the batch
+      walk([&](uint32_t key, uint32_t, bool valid) {
+        before += valid && key < k0 ? 1u : 0u;
+        count_in_lds<1>(mine, key - k0, valid && key - k0 < batch);
+      });
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) before += static_cast<uint32_t>(__shfl_xor(static_cast<int>(before), off, kWave));
+      if (lane == 0) wave_tot2[wv] = before;
+      __syncthreads();
+      uint32_t total[1] = {0};  // of latent k0 + tid
+      if (static_cast<uint32_t>(tid) < batch) {
+        uint32_t c[kWaves];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) c[w] = ids[w * kRunLatents + tid];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          ids[w * kRunLatents + tid] = total[0];
+          total[0] += c[w];
+        }
+      }
+      uint32_t inc = total[0];
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t y = __shfl_up(inc, off, kWave);
+        if (lane >= off) inc += y;
+      }
+      if (lane == kWave - 1) wave_tot[wv] = inc;
+      __syncthreads();
+      uint32_t start = inc - total[0];
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        start += wave_tot2[w];
+        if (w < wv) start += wave_tot[w];
+      }
+      const bool mine_too = static_cast<uint32_t>(tid) < batch && k0 + tid < nlat;
+      if (static_cast<uint32_t>(tid) < batch) cnt[tid] = start;
+      if (tid == static_cast<int>(batch) - 1) cnt[batch] = start + total[0];
+      if (mine_too) begin[f0 + k0 + tid] = base + start;
+      if (ls.chunk_begin) append_latents(ls, f0 + k0 + tid, mine_too ? 1 : 0, total, sh);
+      __syncthreads();
+      walk([&](uint32_t key, uint32_t id, bool valid) {
+        const uint32_t l = key - k0;
+        const bool have = valid && l < batch;
+        if (!__any(have)) return;
+        const unsigned long long same = agreeing(l, have, bits);
+        const uint32_t rank = lanes_before(same);
+        if (have) {
+          const uint32_t place = mine[l] + rank, at = cnt[l];
+          put(base + at + place, id, cnt[l + 1] - at == 1u ? solo_bit : 0u);
+          // (LDS accesses of a wavefront are served in order: all lanes have read the cursor)
+          if (rank == 0) mine[l] = place + static_cast<uint32_t>(__popcll(same));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      });
+      __syncthreads();
+    }
   }
+  if (tid == 0 && blockIdx.y == 0 && q == gridDim.x - 1) begin[F] = base + n;
 }
 
 __global__ void copy_u32_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src, int64_t n) {

@@ -281,6 +281,8 @@ void zero_f32(float *p, int64_t n, hipStream_t st) {
 struct CsrPlan {
   bool bucketed;
   int shift;           // a bucket is 2^shift consecutive latents
+  int pack_shift;
+  uint32_t n_batches;  // blocks per bucket, which share the batches of latents of a large one
   uint32_t n_buckets;
   int n_bits;          // bits of a bucket number
   int64_t chunk;       // consecutive pairs ordered by one block
@@ -290,20 +292,29 @@ struct CsrPlan {
 
 CsrPlan plan_csr(int64_t n_pairs, int64_t F) {
   CsrPlan p;
-  // latents per bucket: about 2048 pairs per bucket on average, a power of two
+  // latents per bucket: about 2048 pairs per bucket on average, a power of two; more than 2048 latents only where buckets
+  // of 2048 are more than the chip holds at once (2097152 latents, 262144 pairs: 29 us that way and 21 with 4096 latents;
+  // 1048576 latents fit and are as fast either way)
   int shift = 0;
-  while (shift < kSortMaxShift && (static_cast<int64_t>(2) << shift) * n_pairs <= 2048 * F) ++shift;
+  while (shift < kSortMaxShift && (static_cast<int64_t>(2) << shift) * n_pairs <= 2048 * F &&
+         (shift < 11 || ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketBlocks))
+    ++shift;
   while (shift < kSortMaxShift && ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketMaxBuckets) ++shift;
   p.shift = shift;
+  p.pack_shift = csr_pack_shift(shift);
   const int64_t n_buckets = ceil_div(F, static_cast<int64_t>(1) << shift);
+  p.n_batches = 1;
+  while ((p.n_batches * kRunLatents) >> shift == 0 && 2 * p.n_batches * n_buckets <= kBucketBlocks) p.n_batches *= 2;
   p.bucketed = n_buckets <= kBucketMaxBuckets;
-  p.n_buckets = static_cast<uint32_t>(p.bucketed ? n_buckets : 0);
   p.n_bits = 0;
   while (p.bucketed && (static_cast<int64_t>(1) << p.n_bits) < n_buckets) ++p.n_bits;
   p.chunk = 2048;
-  while (p.bucketed && p.chunk < kMaxChunk && ceil_div(n_pairs, p.chunk) * n_buckets > (static_cast<int64_t>(1) << 22))
+  while (p.bucketed && p.chunk < (int64_t{1} << p.pack_shift) &&
+         (ceil_div(n_pairs, p.chunk) > kSortChunks || ceil_div(n_pairs, p.chunk) * n_buckets > (static_cast<int64_t>(1) << 22)))
     p.chunk *= 2;
   p.n_chunks = static_cast<uint32_t>(ceil_div(n_pairs, p.chunk));
+  if (p.n_chunks > static_cast<uint32_t>(kSortChunks)) p.bucketed = false;  // (more than 2^31 pairs over more than 2^24 latents)
+  p.n_buckets = static_cast<uint32_t>(p.bucketed ? n_buckets : 0);
   p.table_len = p.bucketed ? static_cast<size_t>(n_buckets + 1) * p.n_chunks : 0;
   return p;
 }
@@ -370,12 +381,12 @@ void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
   const int64_t n_pairs = B * K;
   const CsrPlan &pl = sc.plan;
   if (pl.bucketed) {
-    const size_t lds = (static_cast<size_t>(pl.n_buckets) * kChunkWaves + kChunkWaves) * 4;
+    const size_t lds = (round_up(pl.n_buckets, 4) + 1) * kChunkWaves * 4;
     hipLaunchKernelGGL(csr_chunk_sort_kernel, dim3(pl.n_chunks), dim3(kChunkThreads), lds, st, indices, n_pairs, F,
-                       pl.shift, pl.n_buckets, pl.n_bits, pl.chunk, pl.n_chunks, sc.table, sc.tmp, sc.lists.ctrl,
+                       pl.shift, pl.pack_shift, pl.n_buckets, pl.n_bits, pl.chunk, pl.n_chunks, sc.table, sc.tmp, sc.lists.ctrl,
                        status_flag);
-    hipLaunchKernelGGL(csr_bucket_sort_kernel, dim3(pl.n_buckets), dim3(kSortThreads), 0, st, sc.tmp, sc.table,
-                       pl.n_chunks, pl.chunk, pl.shift, F, begin, map, slot, hslot, solo_bit, sc.lists);
+    hipLaunchKernelGGL(csr_bucket_sort_kernel, dim3(pl.n_buckets, pl.n_batches), dim3(kSortThreads), 0, st, sc.tmp, sc.table,
+                       pl.n_chunks, pl.chunk, pl.shift, pl.pack_shift, F, begin, map, slot, hslot, solo_bit, sc.lists);
     return;
   }
   hipLaunchKernelGGL(csr_init_kernel, dim3(grid_for(F + 1, 256, 4096)), dim3(256), 0, st, begin, F + 1,

@@ -387,11 +387,13 @@ def test_gather_addressing_is_exact(mode, dtype):
 
 @pytest.mark.parametrize("shape", [(4, 8, 16), (37, 16, 5), (64, 32, 4096), (192, 256, 512), (300, 70, 3),
                                    (128, 64, 100000), (2048, 33, 1), (4096, 128, 65536), (1000, 100, 700),
-                                   (64, 16, (1 << 25)), (64, 16, (1 << 25) + 7), (3000, 40, 9000, "skew")])
+                                   (64, 16, (1 << 25)), (64, 16, (1 << 25) + 7), (65536, 128, 65536),
+                                   (3000, 40, 9000, "skew")])
 def test_pair_list_bit_exact(shape):
     """begin/map equal the stable counting sort (oracle = numpy argsort(kind='stable')).  The shapes cover
     one bucket and many, buckets sorted in the LDS and buckets too large for it, latents with more than 64
-    pairs, the largest bucket count, and (F above 2^25) the construction with memory atomics."""
+    pairs, the largest bucket count (F = 2^25: 8192 buckets, 128 KiB of dynamic LDS), half of it through the number
+    of pairs (64 KiB), and (F above 2^25) the construction with memory atomics."""
     B, K, F = shape[:3]
     _announce("csr", shape)
     g = torch.Generator().manual_seed(B + K + F)
@@ -1100,6 +1102,54 @@ def test_pair_list_pieces_and_lists(shape):
     n = np.bincount(idx.flatten().numpy(), minlength=F)
     long = n[n > 64]
     assert stats.tolist() == [len(long), int(((long + 63) // 64).sum()), int((n == 0).sum())]
+
+
+def _side_by_side(kind, B, K, F, g):
+    if kind == "same":  # the same latents in every row
+        return torch.arange(K).repeat(B, 1) % F
+    if kind == "half":  # half of a row's pairs on adjacent latents
+        idx = torch.randint(0, F, (B, K), generator=g)
+        idx[:, : K // 2] = (torch.arange(K // 2) + F // 3) % F
+        return idx
+    p = torch.arange(1, F + 1, dtype=torch.float64) ** -1.1  # latents by frequency
+    return torch.searchsorted(p.cumsum(0) / p.sum(), torch.rand(B * K, generator=g, dtype=torch.float64)).clamp_(
+        max=F - 1).view(B, K)
+
+
+@pytest.mark.parametrize("kind", ["same", "half", "ranked"])
+@pytest.mark.parametrize("shape", [(4096, 64, 262144), (512, 64, 3 << 20), (2000, 100, 70000), (4096, 128, 65536), (300, 100, 3),
+                                   (1500, 3, 1 << 20), (16400, 130, 20000)])
+def test_pair_list_frequent_latents_side_by_side(kind, shape):
+    """A bucket with most of the batch's pairs: latents of one batch and of several, shared by several blocks and
+    not, pieces longer and shorter than a wavefront, more than 1024 chunks.  Equal to the stable counting sort."""
+    B, K, F = shape
+    _announce("csr side by side", kind, shape)
+    idx = _side_by_side(kind, B, K, F, torch.Generator().manual_seed(B + K + F))
+    rbegin, rmap = oracle.csr(idx, F)
+    rc, begin, mp = abi.csr_build(idx.to(DEV), F)
+    torch.cuda.synchronize()
+    assert rc == 0
+    np.testing.assert_array_equal(abi.widen_u32(begin).cpu().numpy(), rbegin.astype(np.int64))
+    np.testing.assert_array_equal(abi.widen_u32(mp).cpu().numpy(), rmap.astype(np.int64))
+
+
+@pytest.mark.parametrize("hot", [False, True])
+@pytest.mark.parametrize("F", [4096, 700, 9000])
+def test_step_with_frequent_latents_side_by_side(F, hot):
+    """The slots, the marks of only pairs and the lists by number of pairs that come with such a bucket: a training step
+    equals the oracle, with every row of dW written."""
+    B, K, D = 700, 16, 64
+    _announce("step side by side", F, hot)
+    cpu = list(make_inputs(B, K, F, D, torch.bfloat16, seed=61, w_std=0.3))
+    cpu[0] = _side_by_side("half", B, K, F, torch.Generator().manual_seed(F))
+    flags = _lib.BWD_HOT_LATENTS if hot else 0
+    _, rW, rv, rb = oracle.loss_grads(oracle.HIER, *cpu)
+    for dense in (0, _lib.BWD_DENSE_LATENTS):
+        rc, _, dW, dv, db = abi.hier_train(*_to_dev(cpu), dw_dtype=torch.bfloat16, flags=flags | dense)
+        torch.cuda.synchronize()
+        assert rc == 0 and not torch.isnan(dW).any()
+        check_gradient("dW", dW, rW, torch.bfloat16, 1e-2)
+        check_gradient("dvals", dv, rv, torch.float32, 1e-2)
 
 
 ONLY_PAIR_SHAPES = [
