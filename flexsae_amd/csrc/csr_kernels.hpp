@@ -114,24 +114,27 @@ __device__ __forceinline__ void append_latents(const PairLists &ls, int64_t f, i
   }
   if (!places) return;
   __syncthreads();
+  // (the wavefront's empty latents in ascending order: their rows are cleared in the order of the list)
   uint32_t empty_at = sh.empty[wv];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const bool have = i < n;
+    const unsigned long long with = __ballot(i < n && count[i] == 0u);
+    empty_at += __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(with >> 32),
+                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(with), 0u));
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    if (i >= n) continue;
     const uint32_t at_f = static_cast<uint32_t>(f + i);
-    const unsigned long long with = __ballot(have && count[i] == 0u);
-    if (!have) continue;
     if (count[i] > kListLong) {
       const unsigned long long at = atomicAdd(&sh.long_at, long_step(count[i]));
       ls.long_list[at >> 32] = at_f;
       ls.chunk_begin[at >> 32] = static_cast<uint32_t>(at);
     } else if (classes && count[i] == 0u) {
-      ls.empty_list[empty_at + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(with >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(with), 0u))] = at_f;
+      ls.empty_list[empty_at++] = at_f;
     } else if (classes) {
       ls.cls_list[class_of(count[i])][atomicAdd(&sh.cursor[count[i]], 1u)] = at_f;
     }
-    empty_at += static_cast<uint32_t>(__popcll(with));
   }
 }
 
