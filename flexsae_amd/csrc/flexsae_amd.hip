@@ -740,6 +740,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
       hipLaunchKernelGGL((hot_finalize_kernel<GT>), dim3(h.n_blocks), dim3(kBlock), 0, st, h);
   };
   if (piece_cols > 0) {  // 256-byte pieces, sixteen lanes each
+    const int how = (update ? kReduceUpdate : 0) | (skip_solo ? kReduceSkipSolo : 0) | (dwords ? kReduceDwords : 0);
     const int pps = static_cast<int>(ceil_div(cols, piece_cols));
     int pps_shift = -1;  // log2(pps) when pps is a power of two
     for (int sh = 0; sh < 16; ++sh)
@@ -750,7 +751,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
 #define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS)                                                                          \
   hipLaunchKernelGGL((seg_reduce_piece_kernel<PT, GT, FLEXSAE_PIECE_U, G>),                                        \
                      dim3(kLongBlocks + static_cast<unsigned>(N_BLOCKS)), dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, \
-                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, update, skip_solo, dwords, ls)
+                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, how, ls)
     constexpr int64_t kGroups = kBlock / kPieceLanes;
     if (by_count) {
       // work items: one per latent with nine rows or more, one per four others of a class
@@ -773,7 +774,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
     const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * rtps, kWavesPerBlock));
     hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, RV, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
                        dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale,
-                       F, kLongBlocks, rtps, col0, sw, D, skip_solo);
+                       F, kLongBlocks, rtps << 1 | skip_solo, col0, sw, D);
     static_assert(RV == 2 || !kCanNarrow, "the narrow reduction works on tiles of 128 columns");
     finalize(3, rtps);
     return;
@@ -781,7 +782,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
   const unsigned n_short_blocks = static_cast<unsigned>(ceil_div(F * tps, kWavesPerBlock));
   hipLaunchKernelGGL((seg_reduce_kernel<PT, GT, VEC, FLEXSAE_REDUCE_U>), dim3(kLongBlocks + n_short_blocks),
                      dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, ll.chunk_begin, P, partial, dW, dw_scale, F,
-                     kLongBlocks, tps, col0, sw, D, skip_solo);
+                     kLongBlocks, tps << 1 | skip_solo, col0, sw, D);
   if constexpr (VEC == 4) {
     finalize(2, tps);
   } else {

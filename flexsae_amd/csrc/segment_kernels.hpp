@@ -119,8 +119,12 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
     const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
-    const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int tps, int col0,
-    int slice_w, int D, int skip_solo) {
+    const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int tps_and_solo, int col0,
+    int slice_w, int D) {
+  // tiles per slice << 1 | skip_solo: one word, loaded with the first arguments, so that a latent without rows waits
+  // for no further one
+  const int tps = tps_and_solo >> 1;
+  const bool skip_solo = (tps_and_solo & 1) != 0;
   const int lane = lane_id();
   if (blockIdx.x >= n_long_blocks) {
     // one wavefront per (latent, tile), tiles of a latent adjacent: the launch reads P front to back
@@ -136,7 +140,11 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
     float acc[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-    accumulate_rows<PT, VEC, U, FLEXSAE_REDUCE_NT>(P, s0, static_cast<int>(n), slice_w, pc, acc);
+    if (n != 0) {  // (first of all: a launch over mostly empty latents is bound by its scalar instructions)
+      if (n > static_cast<uint32_t>(kSegChunk)) return;
+      if (n == 1 && skip_solo) return;
+      accumulate_rows<PT, VEC, U, FLEXSAE_REDUCE_NT>(P, s0, static_cast<int>(n), slice_w, pc, acc);
+    }
     if (scale) {  // the rows were produced for a unit upstream gradient
       const float g = scale[0];
 #pragma unroll
@@ -178,6 +186,10 @@ __device__ __forceinline__ int64_t ceil_div_u32(uint32_t a, int b) { return (sta
 
 constexpr int kPieceLanes = 16;
 constexpr int kPieceBytes = kPieceLanes * 16;
+// What a reduction by pieces is told in one word: the blocks of a launch over mostly empty latents are so short that
+// every further load of an argument shows (387930 latents of 2240 fp32 columns: the step 592 us with a word each and a test
+// against the number of items, 557 without).
+enum { kReduceUpdate = 1, kReduceSkipSolo = 2, kReduceDwords = 4 };
 
 template <typename PT, typename GT, int U, int G>
 __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
@@ -185,7 +197,8 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int pps, int pps_shift, int col0,
-    int slice_w, int D, int update, int skip_solo, int dwords, PairLists lists) {
+    int slice_w, int D, int how, PairLists lists) {
+  const bool update = (how & kReduceUpdate) != 0, skip_solo = (how & kReduceSkipSolo) != 0, dwords = (how & kReduceDwords) != 0;
   using S = typename Traits<PT>::store_t;
   constexpr int EV = 16 / static_cast<int>(sizeof(S));  // columns per lane
   constexpr int kGroupsPerBlock = 256 / kPieceLanes;
@@ -237,17 +250,16 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     // 64 us for 75 750 latents of 1 to 8 and 4 252 of 9 to 64 rows of 512 columns).  A block's first item is split with one wave-uniform division; the sixteen groups then only
     // divide a number below pps + 16 (a 64-bit division per lane would cost more instructions than
     // the rest of a short item)
-    int64_t n_groups = F;
+    int64_t n_items = 0;
+    int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock;
     if constexpr (G > 1) {
-      n_groups = 0;
 #pragma unroll
       for (int i = 0; i < kClasses; ++i)
-        n_groups += i == 0 && skip_solo ? 0 : ceil_div_u32(lists.ctrl[kClassCount + i], i < kClassSolo ? G : 1);
+        n_items += i == 0 && skip_solo ? 0 : ceil_div_u32(lists.ctrl[kClassCount + i], i < kClassSolo ? G : 1);
+      n_items *= pps;
+      if (item0 >= n_items) return;
     }
-    const int64_t n_items = n_groups * pps;
     const int64_t item_stride = static_cast<int64_t>(gridDim.x - n_long_blocks) * kGroupsPerBlock;
-    int64_t item0 = static_cast<int64_t>(blockIdx.x - n_long_blocks) * kGroupsPerBlock;
-    if (item0 >= n_items) return;
     do {
       int64_t fb;
       int t;
