@@ -849,12 +849,12 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, sc.lists.ctrl,
                        sc.lists.empty_list, dW, D, rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t)));
   // In the training step the second step of a slice's hot latents travels with the next slice's
-  // training-step launch (a gradient of CarriedGrad's type only: that is what that kernel writes; a launch
-  // of its own costs 4.7 us a slice); the last slice's gets one.
+  // training-step launch (a gradient of CarriedGrad's type or the in-place update only: that is what that kernel
+  // writes; a launch of its own costs 4.7 us a slice); the last slice's gets one.
   HotFinalize pending = {};
   HotBlockFinalize pending_hot = {};
   // (the sweep of the plain backward carries it for a gradient of the weight's type)
-  const bool fold = (train ? std::is_same<GT, typename CarriedGrad<WT>::type>::value : std::is_same<GT, WT>::value) &&
+  const bool fold = (train && !update ? std::is_same<GT, typename CarriedGrad<WT>::type>::value : std::is_same<GT, WT>::value) &&
                     do_sweep && do_reduce;
   // Only pairs of their latents write dW themselves where its type is the contributions' own.
   void *const dW_solo = (flags & kBwdSolo) && std::is_same<GT, PT>::value && train != nullptr && do_sweep && do_reduce &&

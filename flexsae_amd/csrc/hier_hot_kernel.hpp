@@ -345,8 +345,13 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
   const int wv = wave_in_block();
 
   // this block's share of the previous slice's second steps
-  hot_finalize_run<typename CarriedGrad<WT>::type>(fin, blockIdx.x);
-  hot_block_finalize_run<typename CarriedGrad<WT>::type>(hfin, blockIdx.x, gridDim.x);
+  hot_finalize_carried<WT>(fin, blockIdx.x);
+  if constexpr (!std::is_same<WT, typename CarriedGrad<WT>::type>::value) {
+    if (hfin.update) hot_block_finalize_run<WT>(hfin, blockIdx.x, gridDim.x);
+    else hot_block_finalize_run<typename CarriedGrad<WT>::type>(hfin, blockIdx.x, gridDim.x);
+  } else {
+    hot_block_finalize_run<WT>(hfin, blockIdx.x, gridDim.x);
+  }
 
   const int t = static_cast<int>(blockIdx.x % static_cast<unsigned>(n_tiles));
   const int rb = static_cast<int>(blockIdx.x / static_cast<unsigned>(n_tiles));

@@ -69,7 +69,7 @@ struct RowPiece<f16_t, 2> {
 // counter retires in order, so anything issued after them can only be waited for together with
 // all of them, and the forward walk could not start while rows are still arriving.
 // fin: the second step of the previous slice's hot latents (see HotFinalize), run by the leading blocks
-// of the launch into a gradient of CarriedGrad's type.
+// of the launch into a gradient of CarriedGrad's type, or into the weights.
 // STREAM: the contributions are stored with the non-temporal hint.  That is the faster choice
 // when all of P is written before any of it is read back (it is far larger than the caches);
 // when P is one slice that the reduction reads right after this launch, plain stores leave part
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
   const int lane = lane_id();
   // the leading blocks finish the hot latents of the previous slice (fin.n_blocks of them; none at the first slice)
   if (blockIdx.x < fin.n_blocks) {
-    hot_finalize_run<typename CarriedGrad<WT>::type>(fin, blockIdx.x);
+    hot_finalize_carried<WT>(fin, blockIdx.x);
     return;
   }
   const int64_t item = static_cast<int64_t>(blockIdx.x - fin.n_blocks) * (blockDim.x >> 6) + wave_in_block();

@@ -5,6 +5,8 @@
 // spread over many wavefronts and the summation order stays fixed (deterministic).
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "csr_kernels.hpp"
 
@@ -542,7 +544,7 @@ __device__ __forceinline__ void hot_finalize_run(const HotFinalize &h, unsigned 
 }
 
 // Gradient type of the finalize work that a training-step launch carries: the type the package asks for, the
-// weight's own, or fp32 for fp16 weights (whose unit gradient would underflow).
+// weight's own, or fp32 for fp16 weights (whose unit gradient would underflow).  The in-place update writes the weights.
 template <typename WT>
 struct CarriedGrad {
   using type = WT;
@@ -551,6 +553,20 @@ template <>
 struct CarriedGrad<f16_t> {
   using type = float;
 };
+
+template <typename WT>
+__device__ __forceinline__ void hot_finalize_carried(const HotFinalize &h, unsigned block) {
+  if constexpr (!std::is_same<WT, typename CarriedGrad<WT>::type>::value) {
+    if (h.update) {
+      // (by pieces, the only reduction that updates in place)
+      if (h.mode == 1)
+        seg_piece_finalize_body<WT>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units, h.col0,
+                                    h.slice_w, h.D, 1, h.dwords, block, h.n_blocks);
+      return;
+    }
+  }
+  hot_finalize_run<typename CarriedGrad<WT>::type>(h, block);
+}
 
 template <typename GT>
 __global__ __launch_bounds__(256) void hot_finalize_kernel(HotFinalize h) {
