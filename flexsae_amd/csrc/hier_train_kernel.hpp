@@ -277,6 +277,15 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
   for (int k8 = KMAX - 8; k8 >= 0; k8 -= 8) {
     if (FULL || k8 < kb_rev) {  // uniform
       float dots[8];
+      // the block's destinations, read together ahead of their use (a lane read needs five cycles until a store
+      // can use it)
+      uint32_t to_lo[8], to_hi[8];
+#pragma unroll
+      for (int u = 7; u >= 0; --u) {
+        const int k = k8 + u;
+        to_lo[u] = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_lo[k / kWave]), k % kWave));
+        to_hi[u] = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_hi[k / kWave]), k % kWave));
+      }
       raw_t from_lds[8];  // the block's LDS rows, fetched together ahead of their use
       if constexpr (LDSROWS > 0) {
         if (k8 < LDSROWS) {
@@ -325,9 +334,7 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
 #pragma unroll
             for (int i = 0; i < VEC; ++i) packed[i] = __float_as_uint(contrib[i]);
           }
-          const uint32_t lo = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_lo[k / kWave]), k % kWave));
-          const uint32_t hi = static_cast<uint32_t>(bcast_i32(static_cast<int>(dst_hi[k / kWave]), k % kWave));
-          void *const dst = reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo);
+          void *const dst = reinterpret_cast<void *>((static_cast<uint64_t>(to_hi[u]) << 32) | to_lo[u]);
           descriptor_store<sizeof(packed), STREAM>(
               __builtin_amdgcn_make_buffer_rsrc(dst, 0, static_cast<int>(dst_row_bytes), 0x00020000), p_lane_bytes, packed);
           dots[u] = dot;  // zero where the lane is beyond column D: its w is zero

@@ -136,7 +136,6 @@ __global__ __launch_bounds__(256) void seg_reduce_kernel(
     const int t = static_cast<int>(item - f * tps);
     const uint32_t s0 = begin[f];
     const uint32_t n = begin[f + 1] - s0;
-    if (n > static_cast<uint32_t>(kSegChunk) || (skip_solo && n == 1)) return;
     const int pc = t * (kWave * VEC) + lane * VEC;
     const int d0 = col0 + pc;
     float acc[VEC];
