@@ -846,7 +846,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   // them alone).
   const bool sparse = piece != 0 && sparse_latents(s, flags);
   if (sparse && do_reduce && !update)
-    hipLaunchKernelGGL((seg_zero_rows_kernel<PT, GT>), dim3(2048), dim3(kBlock), 0, st, sc.lists.ctrl,
+    hipLaunchKernelGGL((seg_zero_rows_kernel<GT>), dim3(static_cast<unsigned>(ceil_div(s->F, kZeroRows * kWavesPerBlock))), dim3(kBlock), 0, st, sc.lists.ctrl,
                        sc.lists.empty_list, dW, D, rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t)));
   // In the training step the second step of a slice's hot latents travels with the next slice's
   // training-step launch (a gradient of CarriedGrad's type or the in-place update only: that is what that kernel
