@@ -312,7 +312,7 @@ def main():
     hot = bool(fused and not staged and flex.ops._use_hot_latents(B, K, F, D, dtype, dev))
     # ... and whether shapes with few pairs per latent reduce without the row-count list
     dense = bool(fused and not staged and flex.ops._use_dense_latents(B, K, F, D, dtype, dev))
-    HOTF = (flex.ops._hot_flags(B, D, dev) if hot else 0) | (_lib.BWD_DENSE_LATENTS if dense else 0)
+    HOTF = (flex.ops._hot_flags(B, K, D, dev) if hot else 0) | (_lib.BWD_DENSE_LATENTS if dense else 0)
     if hot:
         slice_cols = flex.ops._hot_slice_cols(B, slice_cols, dev)
     tile = 64 * (4 if D % 4 == 0 else 2 if D % 2 == 0 else 1)

@@ -388,16 +388,27 @@ def _hot_slice_cols(B: int, cols: int, device) -> int:
     return want if cols <= want else (cols // want) * want
 
 
-def _hot_flags(B: int, D: int, device) -> int:
-    """Flags of a step with hot-latent accumulators: where all of D makes half a round of blocks or less,
-    blocks of half as many rows, as long as they stay within one round (B = 1024, D = 1024, K = 64, Zipf
-    indices: 64 blocks of 128 rows 118 us, 256 of 32 rows 46 us)."""
-    n_cu = torch.cuda.get_device_properties(device).multi_processor_count
+def _hot_halvings(B: int, K: int, D: int, n_cu: int) -> int:
+    """How often a block's rows are halved: where all of D makes half a round of blocks or less, as long as the blocks
+    stay within one round (B = 1024, D = 1024, K = 64, Zipf indices: 64 blocks of 128 rows 118 us, 256 of 32 rows
+    46 us), and as long as a walk of K steps gains more than the second step loses, which adds up one partial sum per
+    row block (the step in us with 128, 64, 32, 16 rows, B = 4096, D = 128: K = 4 96, 92, 99, 120; K = 16 122, 110,
+    114, 137; K = 64 277, 221, 205, 212)."""
     tiles = -(-D // 128)
     halvings = 0
-    while halvings < 3 and -(-B // (_HOT_ROWS_PER_BLOCK >> (halvings + 1))) * tiles <= n_cu:
+    while halvings < 3:
+        row_blocks = -(-B // (_HOT_ROWS_PER_BLOCK >> (halvings + 1)))
+        if row_blocks * tiles > n_cu or row_blocks > max(64, 2 * K):
+            break
         halvings += 1
-    return _lib.BWD_HOT_LATENTS | halvings * _lib.BWD_HOT_BLOCKS_64  # (the two flag bits count the halvings)
+    return halvings
+
+
+def _hot_flags(B: int, K: int, D: int, device) -> int:
+    """Flags of a step with hot-latent accumulators."""
+    n_cu = torch.cuda.get_device_properties(device).multi_processor_count
+    # (the two flag bits count the halvings)
+    return _lib.BWD_HOT_LATENTS | _hot_halvings(B, K, D, n_cu) * _lib.BWD_HOT_BLOCKS_64
 
 
 # Memory the fused training step may hold between forward and backward: all B*K*D per-pair
@@ -752,7 +763,7 @@ def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tenso
     with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype)
-        hot_flag = _hot_flags(B, D, dev) if (hot and need_dw) else 0
+        hot_flag = _hot_flags(B, K, D, dev) if (hot and need_dw) else 0
         if hot_flag:
             slice_cols = _hot_slice_cols(B, slice_cols, dev)
         ws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(shape), slice_cols, hot_flag)
@@ -824,7 +835,7 @@ def hier_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, t
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
         slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype)
         # hot-latent accumulators: the same decision as the loss takes (set_hot_latents)
-        hot_flag = _hot_flags(B, D, dev) if _use_hot_latents(B, K, F, D, weight.dtype, dev, _is_traced(weight)) else 0
+        hot_flag = _hot_flags(B, K, D, dev) if _use_hot_latents(B, K, F, D, weight.dtype, dev, _is_traced(weight)) else 0
         dense_flag = (_lib.BWD_DENSE_LATENTS
                       if _use_dense_latents(B, K, F, D, weight.dtype, dev, _is_traced(weight)) else 0)
         if hot_flag:

@@ -77,3 +77,14 @@ def test_package_never_imports_the_oracle():
                 text = open(os.path.join(dirpath, f)).read()
                 assert not re.search(r"^\s*(from|import)\s+oracle\b", text, flags=re.M), f
                 assert "sae_oracle" not in text, f
+
+
+@pytest.mark.parametrize("B,K,D,want", [
+    (3866, 4, 120, 1), (4096, 4, 128, 1), (4096, 16, 128, 1), (4096, 64, 128, 2),  # many row blocks: their sums count
+    (1024, 64, 1024, 2), (1024, 4, 128, 3), (256, 64, 2304, 2), (64, 16, 128, 3),    # within one round of blocks
+    (4096, 64, 512, 1), (4096, 64, 1024, 0), (8192, 64, 4096, 0)])
+def test_rows_per_block_of_the_hot_latent_step(B, K, D, want):
+    got = ops._hot_halvings(B, K, D, 256)
+    assert got == want
+    blocks = -(-B // (128 >> got)) * -(-D // 128)
+    assert got == 0 or blocks <= 256
