@@ -748,19 +748,19 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
     // latents per group of lanes: four, taken from the lists by row count, where most latents
     // have no or few rows (with four rows per latent on average the bookkeeping already costs more
     // than the shorter launch saves); the lists hold at most min(F, pairs) latents with rows
-#define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS)                                                                          \
+#define FLEXSAE_PIECE_REDUCE(G, N_BLOCKS, LISTS)                                                                       \
   hipLaunchKernelGGL((seg_reduce_piece_kernel<PT, GT, FLEXSAE_PIECE_U, G>),                                        \
                      dim3(kLongBlocks + static_cast<unsigned>(N_BLOCKS)), dim3(kBlock), 0, st, begin, ll.ctrl, ll.list, \
-                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, how, ls)
+                     ll.chunk_begin, P, partial, dW, dw_scale, F, kLongBlocks, pps, pps_shift, col0, sw, D, how, LISTS)
     constexpr int64_t kGroups = kBlock / kPieceLanes;
     if (by_count) {
       // work items: one per latent with nine rows or more, one per four others of a class
       const int64_t n_listed_max = F < n_pairs ? F : n_pairs;
       const int64_t n_items_max = (n_pairs / 9 + ceil_div(n_listed_max, 4) + kClasses) * pps;
       const int64_t n_blocks = ceil_div(n_items_max, kGroups);
-      FLEXSAE_PIECE_REDUCE(4, (n_blocks < kListBlocks ? n_blocks : kListBlocks));
+      FLEXSAE_PIECE_REDUCE(4, (n_blocks < kListBlocks ? n_blocks : kListBlocks), ls);
     } else {
-      FLEXSAE_PIECE_REDUCE(1, ceil_div(F * pps, kGroups));
+      FLEXSAE_PIECE_REDUCE(1, ceil_div(F * pps, kGroups), NoLists{});
     }
 #undef FLEXSAE_PIECE_REDUCE
     // the chunk partials of hot latents are combined per 64-column piece

@@ -191,6 +191,10 @@ constexpr int kPieceBytes = kPieceLanes * 16;
 // every further load of an argument shows (387930 latents of 2240 fp32 columns: the step 592 us with a word each and a test
 // against the number of items, 557 without).
 enum { kReduceUpdate = 1, kReduceSkipSolo = 2, kReduceDwords = 4 };
+// The lists of a reduction that works from them; a launch that does not is not handed their addresses.
+struct NoLists {};
+template <int G>
+using PieceLists = std::conditional_t<(G > 1), PairLists, NoLists>;
 
 template <typename PT, typename GT, int U, int G>
 __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(256) void seg_reduce_piece_kernel(
     const uint32_t *__restrict__ long_list, const uint32_t *__restrict__ chunk_begin,
     const void *__restrict__ P, float *__restrict__ partial, void *__restrict__ out,
     const float *__restrict__ scale, int64_t F, unsigned n_long_blocks, int pps, int pps_shift, int col0,
-    int slice_w, int D, int how, PairLists lists) {
+    int slice_w, int D, int how, PieceLists<G> lists) {
   const bool update = (how & kReduceUpdate) != 0, skip_solo = (how & kReduceSkipSolo) != 0, dwords = (how & kReduceDwords) != 0;
   using S = typename Traits<PT>::store_t;
   constexpr int EV = 16 / static_cast<int>(sizeof(S));  // columns per lane
