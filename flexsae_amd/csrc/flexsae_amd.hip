@@ -471,10 +471,11 @@ struct HierBwdPlan {
 };
 
 // Hot-latent accumulators: 16-bit weights of at most 64 steps (one register per row piece, four
-// wavefronts per SIMD next to 144 KiB of accumulators) whose slices the piece reduction serves.
+// wavefronts per SIMD next to 144 KiB of accumulators) whose slices the piece reduction serves, and
+// pair numbers below the walk's mark of a latent's only pair (kSoloSlotBit).
 inline bool hot_supported(const flexsae_shape *s) {
   return s->D % 4 == 0 && s->K <= 64 && s->weight_dtype != FLEXSAE_F32 &&
-         s->D % (s->weight_dtype == FLEXSAE_BF16 ? 8 : 4) == 0 && s->B * s->K < (1LL << 31);
+         s->D % (s->weight_dtype == FLEXSAE_BF16 ? 8 : 4) == 0 && s->B * s->K < (1LL << 30);
 }
 
 HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 0) {

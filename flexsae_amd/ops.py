@@ -312,8 +312,8 @@ def set_dense_latents(mode) -> None:
 
 def _hot_latents_supported(B: int, K: int, F: int, D: int, weight_dtype) -> bool:
     """flexsae_hier_hot_latents_supported() of the library, restated so that a compiler trace can
-    follow it: 16-bit weights, at most 64 steps, rows the piece reduction can serve."""
-    if weight_dtype not in (torch.bfloat16, torch.float16) or K > 64 or B * K >= 2 ** 31:
+    follow it: 16-bit weights, at most 64 steps, fewer than 2^30 pairs, rows the piece reduction can serve."""
+    if weight_dtype not in (torch.bfloat16, torch.float16) or K > 64 or B * K >= 2 ** 30:
         return False
     return D % (8 if weight_dtype == torch.bfloat16 else 4) == 0
 

@@ -245,7 +245,7 @@ size_t flexsae_hier_fwd_bwd_workspace_bytes(const flexsae_shape *shape, int64_t 
  * by blocks of 128 batch rows instead of being staged pair by pair, in 32-bit fixed point with one
  * exponent per block (integer sums do not depend on the order of the additions: results stay
  * bit-reproducible, and identical for every slice width).  Supported for 16-bit weights with
- * K <= 64 and D a multiple of 8 (bf16) or 4 (fp16); `_supported` says whether the flag would be
+ * K <= 64, B*K < 2^30 and D a multiple of 8 (bf16) or 4 (fp16); `_supported` says whether the flag would be
  * honoured for `shape`, `_workspace_bytes_flags` is the workspace query for a call with `flags`
  * (the accumulators' block partials take (slice columns / 128) x ceil(B / 128) x 147456 bytes, twice).
  * Slices are best chosen so that (slice columns / 128) x ceil(B / 128) is a multiple of the number

@@ -5,6 +5,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from flexsae_amd import _lib
 
@@ -163,3 +164,14 @@ def test_workspaces_hold_the_lists_by_number_of_pairs_only_where_they_are_read(B
     # at two pairs per latent the reduction may work from the lists: four bytes per latent and more
     grown = at("flexsae_hier_bwd_workspace_bytes", 1 << 20) - at("flexsae_hier_bwd_workspace_bytes", f0)
     assert grown >= list_bytes(1 << 20) - list_bytes(f0) + (4 << 20)
+
+
+@pytest.mark.parametrize("B,K", [((1 << 24) - 1, 64), (1 << 24, 64), (1 << 25, 63)])
+def test_hot_latents_stay_below_the_mark_of_an_only_pair(B, K):
+    """The accumulator walk takes bit 30 of a pair's place for the mark of a latent's only pair, so the hint is
+    honoured for fewer than 2^30 pairs, by the library and by the package's restatement alike."""
+    from flexsae_amd import ops
+    sh = _shape(B=B, K=K, F=1 << 20, D=256, wd=1)
+    want = B * K < 1 << 30
+    assert _lib.load().flexsae_hier_hot_latents_supported(ctypes.byref(sh)) == int(want)
+    assert ops._hot_latents_supported(B, K, 1 << 20, 256, torch.bfloat16) is want
