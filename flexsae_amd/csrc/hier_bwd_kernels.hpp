@@ -120,7 +120,7 @@ namespace flexsae {
 // segment reduction (segment_kernels.hpp) can stream them.  Only the columns
 // [col0, col0 + tps*64*VEC) of the problem (one "slice") are handled per launch, so P needs
 // B*K*slice_width elements.  Every tile leaves its share of the dvals dot products in dv_part;
-// hier_dvals_finalize_kernel adds the shares in tile order (deterministic).
+// hier_epilogue_kernel adds the shares in tile order (deterministic).
 //
 // One wavefront per (tile of the slice, row b), tile-major: the wavefronts in flight at any
 // moment gather from the same 64*VEC-column slice of W, which is small enough to stay in the
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
         }
       }
     }
-    // this tile's share of dvals; hier_dvals_finalize_kernel adds the tiles up in order
+    // this tile's share of dvals; hier_epilogue_kernel adds the tiles up in order
     if (kk < K) dv_part[(static_cast<int64_t>(col0 / (kWave * VEC)) + t) * (B * K) + pair0 + kk] = my_dval;
   }
   // the row's total S_{b,0} (its share of dbias) goes to s_final[b, column]; a column sum over
@@ -242,24 +242,14 @@ __global__ __launch_bounds__(256) void hier_sweep_kernel(
   store_vec<float, VEC>(s_final, b * s_final_ld + col0 + pc, S);
 }
 
-// dvals[p] = sum over the column tiles of dv_part[tile, p], in tile order (deterministic).
-__global__ void hier_dvals_finalize_kernel(const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs,
-                                           float *__restrict__ dvals) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; p < n_pairs; p += stride) {
-    float acc = 0.f;
-    for (int t = 0; t < n_tiles; ++t) acc += dv_part[t * n_pairs + p];
-    dvals[p] = acc;
-  }
-}
-
 // What follows the slices of a hierarchical step, in one launch of 1024-thread blocks (the three
-// parts are independent; each computes what its own kernel computes, bit for bit):
+// parts are independent):
 //   block 0                 the loss from the per-(tile, row) partials (loss_finalize_kernel), when
 //                           loss_partial is given;
 //   the next n_colsum_blocks stage 1 of the column sums of s_final (colsum_partial_one): a block
 //                           takes 256 columns of four consecutive row chunks;
-//   the rest                dvals from its per-tile shares (hier_dvals_finalize_kernel).
+//   the rest                dvals[p] = sum over the column tiles of dv_part[tile, p], in tile order
+//                           (deterministic).
 __global__ __launch_bounds__(1024) void hier_epilogue_kernel(
     const float *__restrict__ loss_partial, int64_t n_loss_partials, double inv_count, float *__restrict__ loss,
     const float *__restrict__ s_final, int64_t rows, int64_t ld, int cols, float *__restrict__ colsum_part,

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
 #pragma unroll
   for (int c = 0; c < KC; ++c) {
     const int kk = c * kWave + lane;
-    // this tile's share of dvals; hier_dvals_finalize_kernel adds the tiles up in order
+    // this tile's share of dvals; hier_epilogue_kernel adds the tiles up in order
     if (kk < K) dv_part[(static_cast<int64_t>(col0 / (kWave * VEC)) + t) * (B * K) + pair0 + kk] = my_dval[c];
   }
   if (!active) {
