@@ -242,15 +242,17 @@ size_t flexsae_hier_fwd_bwd_workspace_bytes(const flexsae_shape *shape, int64_t 
  * selected by most batch rows, and the reference's backward piles its atomic adds up on their rows
  * of dW (hierarchical_kernels.py:155-161).  With the flag, the (up to 288) latents with the most
  * pairs -- more than 64 and no batch row holding the latent twice -- are summed in LDS accumulators
- * by blocks of 128 batch rows instead of being staged pair by pair, in 32-bit fixed point with one
+ * by blocks of 128 batch rows (64, 32 or 16 with FLEXSAE_BWD_HOT_BLOCKS_*) instead of being staged
+ * pair by pair, in 32-bit fixed point with one
  * exponent per block (integer sums do not depend on the order of the additions: results stay
  * bit-reproducible, and identical for every slice width).  Supported for 16-bit weights with
  * K <= 64, B*K < 2^30 and D a multiple of 8 (bf16) or 4 (fp16); `_supported` says whether the flag would be
  * honoured for `shape`, `_workspace_bytes_flags` is the workspace query for a call with `flags`
- * (the accumulators' block partials take (slice columns / 128) x ceil(B / 128) x 147456 bytes, twice).
- * Slices are best chosen so that (slice columns / 128) x ceil(B / 128) is a multiple of the number
- * of compute units (one block each); where all of D is too few of them, FLEXSAE_BWD_HOT_BLOCKS_*
- * make the blocks shorter (their sums are then grouped differently: equal up to rounding).
+ * (the accumulators' block partials take (slice columns / 128) x ceil(B / rows) x 147456 bytes, twice,
+ * where `rows` is the 128, 64, 32 or 16 rows of a block that the flags select).  Slices are best chosen
+ * so that (slice columns / 128) x ceil(B / rows) is a multiple of the number of compute units (one block
+ * each); where all of D is too few of them with 128 rows, FLEXSAE_BWD_HOT_BLOCKS_* make the blocks
+ * shorter (their sums are then grouped differently: equal up to rounding).
  */
 int flexsae_hier_hot_latents_supported(const flexsae_shape *shape);
 size_t flexsae_hier_fwd_bwd_workspace_bytes_flags(const flexsae_shape *shape, int64_t slice_cols, int flags);
@@ -294,8 +296,8 @@ int flexsae_hier_fwd_bwd(const flexsae_shape *shape, const int64_t *indices, con
  * 16 bytes for fp32, 8 for fp16); otherwise FLEXSAE_ERR_UNSUPPORTED.  Workspace as for
  * flexsae_hier_fwd_bwd (for FLEXSAE_BWD_HOT_LATENTS from the _flags query); the flags accepted are
  * FLEXSAE_BWD_REUSE_PAIR_LIST, FLEXSAE_BWD_HOT_LATENTS (the accumulators' sums update the weight rows
- * of the hot latents the same way), FLEXSAE_BWD_REUSE_HOT_TABLES and FLEXSAE_BWD_DENSE_LATENTS; others
- * are ignored.
+ * of the hot latents the same way) with FLEXSAE_BWD_HOT_BLOCKS_64 / _32 and FLEXSAE_BWD_REUSE_HOT_TABLES,
+ * and FLEXSAE_BWD_DENSE_LATENTS; others are ignored.
  * replaces: the dense dW of the backward (hierarchical_kernels.py:241-243, 294-297) together with
  *           the optimizer pass that consumes it in a training loop written like reference
  *           example.py:76-77 with torch.optim.SGD (no momentum, no weight decay: for those the
