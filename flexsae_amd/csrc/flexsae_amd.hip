@@ -131,6 +131,13 @@ FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target,
   if (s->target_dtype == s->weight_dtype && !aligned(target, vec * es)) vec = 1;
   if (s->bias_dtype == s->weight_dtype && !aligned(bias, vec * es)) vec = 1;
   if (!aligned(resid, 16)) vec = 1;
+  const uint64_t row_bytes = static_cast<uint64_t>(s->D) * es;
+  // Eight bytes per lane where sixteen leave fewer than five wavefronts for every four SIMDs.  us with sixteen / eight (K=64,
+  // bf16; uniform, skewed indices): 512 wavefronts (B=512, D=512, F=65536) 14.4 / 10.4, 10.0 / 8.6; 1024 (B=451, D=1160,
+  // F=16384) 18.0 / 15.4, 14.1 / 12.4; 1152 (B=256, D=2304, F=16384) 16.8 / 14.1, 12.8 / 12.7; above it depends on the
+  // shape: 1536 (B=768, D=1024, F=65536) 18.2 / 17.1, 14.0 / 12.7, (B=677, D=1160, F=65536) 21.2 / 24.5, 16.0 / 15.3; from
+  // 2048 on the wider ones (B=1024, D=1024, F=65536) 21.2 / 21.7, 15.2 / 16.1.
+  if (vec == 8 && static_cast<uint64_t>(s->B) * row_bytes < 1280 * 1024) vec = 4;
   FwdPlan p;
   p.vec = vec;
   // Bytes of a row piece, and whether every L2 works on a tile of its own.  Measured (us; uniform / skewed
@@ -146,15 +153,37 @@ FwdPlan plan_fwd(const flexsae_shape *s, const void *weight, const void *target,
   // (B=2048, K=64, D=1024): 256 B beats 128 B from 32768 rows on (65536: 65 / 31 against 73 / 32, 131072:
   // 73 / 32 against 83 / 34; 512 B 78 / 37) and equals it below.  Eight-byte lanes gain 5 % on uniform
   // indices around 65536 rows and lose 25 % on skewed ones: 16 bytes per lane wherever rows allow it.
-  // Rows that do not start on a line (D=1538 bf16, F=65536: row order 133 / 70, 256 B per L2 154 / 62; D=1452,
-  // F=262144, K=128: 239, 512 B with all L2s on one tile 274; D=8184, F=524288: 834 against 775) keep the row
-  // order from 24576 latents up to 4 GiB of weights.
-  const bool lines = static_cast<size_t>(s->D) * es % 128 == 0;
-  const uint64_t w_bytes = static_cast<uint64_t>(s->F) * static_cast<uint64_t>(s->D) * es;
+  // The narrow pieces want the blocks of one tile (B / 32) to be about as many as an XCD runs at a time; with fewer it
+  // works on several tiles at once (F=32768, D=2304, 128 B against 256 B: B=1024 45.0 / 25.4 against 41.4 / 22.0, B=2048
+  // 64.4 / 39.3 against 70.9 / 36.4; F=16384, D=8192: B=256 43.9 / 20.8 against 40.5 / 19.6).
+  //
+  // Rows that do not start on a line: a piece reaches into one line more than its own, which the L2 has to hold and to
+  // fetch; in row order the pieces of a row share them.  The tiles pay while an L2 (4 MB) holds about two fifths of one
+  // tile's lines (F * 384 B = 10 MB); latents up to which they are the faster ones on uniform indices (B=4096, K=64; on
+  // skewed ones the two orders are within 6 %): D=1538 bf16 31000, 1540 29700, 2305 33000, 3004 32500, 4100 32500, fp32
+  // (B=2048) D=1002 27500, 1700 26800.  Rows of a few pieces are close together in row order too and lose the most to a
+  // last piece that is nearly empty: D=264 bf16 15000, 520 fp16 18500, 772 bf16 20000, 300 fp32 19000.
+  //
+  // Tiles that all L2s walk together pay where latents repeat within the batch.  Pairs per latent, then the time with
+  // tiles and in row order (K=64, bf16):
+  //   1/8   F=262144, D=4096  46.6 / 23.8    45.3 / 21.8      F=524288, D=8192  216.9 / 92.8   212.7 / 83.2
+  //   1/4   F=262144, D=4096  102.7 / 42.9   98.3 / 39.8      F=524288, D=2304  114.7 / 43.5   112.0 / 45.5
+  //   1/2   F=262144, D=4096  183.9 / 79.8   194.2 / 73.1     F=524288, D=2304  208.7 / 85.9   220.4 / 91.4
+  //   1     F=262144, D=4096  325.9 / 157.8  384.4 / 150.4    F=262144, D=8184  1464 / 654     1673 / 649
+  // (the last one two pairs per latent).  Where rows do not start on a line: only for weights of 4 GiB and more (D=3004,
+  // F=262144, one pair per latent: 281 / 144 against 281 / 142), not where one tile's lines are far more than the
+  // memory-side cache holds (B=16384, D=3004, F=800000: 1211 / 611 against 1238 / 587; D=1004, F=2000000: 491 / 205
+  // against 427 / 195), and not where a lane's four bytes halve the pieces (B=1346, K=256, F=524288, D=4966: 737
+  // against 640, uniform).
+  const bool lines = row_bytes % 128 == 0;
+  const uint64_t F = static_cast<uint64_t>(s->F);
+  const uint64_t n_256 = (row_bytes + 255) / 256;
+  const bool by_xcd = s->B > 1 && (lines ? F <= 131072 : n_256 < 8 ? F * n_256 * 256 <= 24576 * row_bytes : F <= 26624);
+  const bool repeats = 8 * static_cast<uint64_t>(s->B) * static_cast<uint64_t>(s->K) > 3 * F;
   // (A single row: a block per narrow tile would leave more partials than the workspace has room for, see forward().)
-  const bool by_row = s->B == 1 || (!lines && s->F > 24576 && w_bytes < (uint64_t{1} << 32));
-  const bool by_xcd = !by_row && s->F <= 131072;
-  const size_t piece_bytes = by_row ? 1024 : !by_xcd ? 512 : (es == 2 && s->F <= 49152 && lines) ? 128 : 256;
+  const bool by_row = !by_xcd && (s->B == 1 || !repeats ||
+                                  (!lines && (F * row_bytes < (uint64_t{1} << 32) || F > (uint64_t{1} << 20) || vec * es < 8)));
+  const size_t piece_bytes = by_row ? 1024 : !by_xcd ? 512 : (es == 2 && F <= 49152 && lines && s->B >= 2048) ? 128 : 256;
   p.lpr = static_cast<int>(piece_bytes / (static_cast<size_t>(vec) * es));
   if (p.lpr > kWave) p.lpr = kWave;
   const int64_t rows = kWave / p.lpr;

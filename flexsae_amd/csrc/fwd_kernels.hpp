@@ -23,9 +23,9 @@ namespace flexsae {
 //                  (twice as slow).
 //   xcd_span == 0  items in order, tiles outermost, wide tiles: all XCDs gather from the same column
 //                  tile, which the memory-side cache (256 MB) holds where the L2s cannot help.
-//   xcd_span < 0   wavefronts in order, the -xcd_span tiles of a row next to each other: where rows do not
-//                  start on a 128-byte line, neighbouring pieces share lines, and only this order has them
-//                  read together.
+//   xcd_span < 0   wavefronts in order, the -xcd_span tiles of a row next to each other: where no cache
+//                  holds a tile long enough for its pieces to be asked for again, and where rows do not
+//                  start on a 128-byte line and neighbouring pieces share lines.
 // Against one wavefront per (row, 256 columns) in row order, which no cache but the memory-side one served:
 // B=4096, K=128, F=65536, D=2304 bf16 (2.42 GB gathered) 328 -> 275 us (8.8 TB/s), K=64 172 -> 143 us; B=2048,
 // K=256, F=131072, D=1024 fp32 292 -> 273 us; B=16384, K=128, F=524288, D=8192 bf16 6.3 -> 4.8 ms (7.2 TB/s).
@@ -206,6 +206,19 @@ __device__ __forceinline__ void loss_finalize_block(const PT *__restrict__ parti
                                                     float *__restrict__ loss, double *red) {
   double s = 0.0;
   int64_t i = threadIdx.x;
+  if constexpr (sizeof(PT) == 8) {  // two at a time (partial starts at a multiple of 16 bytes)
+    const auto *const two = reinterpret_cast<const vec_t<PT, 2> *>(partial);
+    const int64_t n2 = n / 2;
+    for (; i + 7 * 1024 < n2; i += 8 * 1024) {
+      vec_t<PT, 2> x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = two[i + u * 1024];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += x[u][0] + x[u][1];
+    }
+    for (; i < n2; i += 1024) s += two[i][0] + two[i][1];
+    i = n2 * 2 + threadIdx.x;  // the last one of an odd number
+  }
   for (; i + 7 * 1024 < n; i += 8 * 1024) {  // eight independent loads in flight
     PT x[8];
 #pragma unroll

@@ -201,10 +201,16 @@ def test_rows_beyond_four_gib_are_addressed_exactly():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("shape", [(1, 1, 49152, 8), (33, 65, 49152, 72), (34, 7, 49153, 136), (63, 130, 131072, 68),
                                    (17, 63, 131073, 264), (9, 64, 131073, 520), (66, 8, 300, 2), (3, 73, 40, 1),
-                                   (40, 12, 131073, 6)])
+                                   (40, 12, 131073, 6),
+                                   # lanes of 8 bytes and of 16 (from 1280 wavefronts on), pieces of 128 bytes (from 2048 rows on)
+                                   (1279, 9, 1000, 512), (1280, 9, 1000, 512), (2047, 9, 1000, 512), (2048, 9, 1000, 512),
+                                   # three pairs for eight latents and fewer
+                                   (453, 109, 131671, 64), (453, 109, 131672, 64),
+                                   # rows that start anywhere: the bounds for rows of eight pieces and of fewer
+                                   (67, 5, 26624, 1026), (67, 5, 26625, 1026), (130, 7, 16896, 264), (130, 7, 16897, 264)])
 @pytest.mark.parametrize("mode", ["topk", "hier"])
 def test_forward_tilings_are_exact(mode, shape, dtype):
-    """Forward kernel on either side of the sizes where its tiling changes (49152 and 131072 latents), with
+    """Forward kernel on either side of the sizes where its tiling changes, with
     ragged row blocks, last tiles and step counts, for every vector width the row length allows: integer
     weights, vals of one, so that every error is an exact integer (all partial sums of squares stay below
     2^24 units) and the residual shows which rows were read."""
@@ -216,7 +222,7 @@ def test_forward_tilings_are_exact(mode, shape, dtype):
     bias = torch.randint(-2, 3, (D,), generator=g).float()
     target = torch.randint(-2, 3, (B, D), generator=g).float()
     e = W[idx].cumsum(1) + (bias - target).unsqueeze(1)
-    sq = e.square().sum() if mode == "hier" else e[:, -1].square().sum()
+    sq = e.square().double().sum() if mode == "hier" else e[:, -1].square().double().sum()
     rc, loss, resid = abi.forward(mode, idx.to(DEV), *(x.to(dtype).to(DEV) for x in (W, torch.ones(B, K), bias, target)))
     torch.cuda.synchronize()
     assert rc == 0, _lib.status_string(rc)
