@@ -614,9 +614,9 @@ inline bool train_supported(const flexsae_shape *s) { return s->D % 4 == 0 && s-
 
 // Row pieces the training-step kernel keeps in the LDS instead of registers (one dword per lane
 // and row: 16-bit weights with two columns per lane, fp32 with one), chosen so that one more
-// wavefront fits each SIMD: 256 steps 216 instead of 276 registers (two wavefronts instead of one,
-// 16 KB of LDS each), 128 steps 120 instead of 152 (four instead of three, 8 KB each), 64 steps 72
-// instead of 88.
+// wavefront fits each SIMD: 256 steps 222-224 registers, two wavefronts (280-284 and one with all pieces in
+// registers; 16 KB of LDS each), 128 steps 120-122, four (146-150, three; 8 KB each), 64 steps 63, eight
+// (80, six).
 #ifndef FLEXSAE_LDS_256
 #define FLEXSAE_LDS_256 64
 #endif
