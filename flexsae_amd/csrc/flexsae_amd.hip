@@ -232,6 +232,121 @@ void launch_fwd(const flexsae_shape *s, const FwdPlan &p, const int64_t *indices
 #undef FLEXSAE_LAUNCH_FWD
 }
 
+// ---- TopK forward in latent order ---------------------------------------------------------
+// Rows of at most 512 pairs.  `waves` wavefronts per block, lpr lanes per row piece; waves == 0: not in latent order.
+struct OrderedPlan {
+  int waves, lpr;
+  int64_t n_row_blocks, n_items, xcd_span;
+  size_t steps_bytes;  // (row, val) of every pair, after the loss partials
+};
+
+// By sizes alone; forward_ordered() also asks for rows of whole 16-byte vectors and room for the steps.
+// us without / with the ordering, uniform and skewed (Zipf 1.1) indices:
+//   bf16, K=128  B=4096, D=2304: F=65536 286 / 188, 150 / 149; F=131072 323 / 229, 168 / 164;  B=1024, D=2048, F=32768
+//                63 / 36, 33 / 33;   K=256  B=1024, D=1024, F=65536 65 / 48, 40 / 43;  B=512, D=4096 148 / 114, 73 / 69
+//   bf16, K=64   B=4096, D=2304: F=32768 96 / 76, 68 / 71; F=65536 151 / 116, 70 / 76;  B=16384, D=768 192 / 133, 89 / 96
+//   bf16, K=32   B=4096, D=2304, F=65536 84 / 77, 41 / 48;  B=16384, D=768 107 / 94, 51 / 63
+//   fp32, K=128  B=4096, D=2304, F=65536 553 / 338, 301 / 275;  K=64 286 / 219, 161 / 156;  K=32 156 / 153, 84 / 91;
+//                K=64, B=1024, D=1024, F=65536 36 / 33, 19 / 21;   K=256, B=2048, D=1024, F=131072 275 / 181, 144 / 133
+// So: rows of 64 pairs and more (with fewer, the latents at one position of two rows are too far apart); where the pieces of
+// one tile do not fit an L2 (4 MB; B=4096, K=64, D=2304, F=16384 72 / 71); gathers of a quarter of a GiB and more, half a
+// GiB below 128 steps (the ordering is a launch of 5-6 us); and, like the tiles per XCD that it walks, rows that start on a
+// line and at most 131072 latents (262144: B=8192, K=64, D=4096 614 / 658) and 512 batch rows or more (B=300, K=200,
+// F=40000, D=4096 72 / 65, 38 / 45; B=128, K=256, F=65536, D=2048 25 / 49).
+// 128-byte pieces (16-bit weights, eight rows per wavefront) beat 256-byte ones from more than 2048 rows on (B=4096, K=64,
+// D=2304, F=131072 149 / 161; at B=2048, K=256, D=1024 96 / 87, at B=512 143 / 114).  As many wavefronts per block as
+// leave 32 blocks, one per compute unit of an XCD, for a tile: fp32, K=256, D=4096, F=65536, B=512 blocks of 16 / 8 / 4
+// wavefronts 236 / 237 / 228, B=1024 (D=1024) 85 / 76 / 88, B=2048 181 / 210 / 235; 16-bit pieces of 128 bytes always
+// eight (they leave a last round of blocks that is not full otherwise).
+OrderedPlan plan_ordered(const flexsae_shape *s) {
+  OrderedPlan p = {};
+  const size_t es = dtype_size(s->weight_dtype);
+  const uint64_t row_bytes = static_cast<uint64_t>(s->D) * es;
+  const uint64_t F = static_cast<uint64_t>(s->F);
+  if (s->K < 64 || s->K > 512 || s->B < 512 || F > 131072 || row_bytes % 128 != 0) return p;
+  if (static_cast<uint64_t>(s->B) * s->K * row_bytes < (s->K < 128 ? uint64_t{512} << 20 : uint64_t{128} << 20)) return p;
+  const bool narrow = es == 2 && s->B > 2048;
+  const uint64_t piece_bytes = narrow ? 128 : 256;
+  if (F * piece_bytes < (uint64_t{4} << 20)) return p;
+  p.lpr = static_cast<int>(piece_bytes / 16);
+  const int64_t rows = kWave / p.lpr;
+  p.waves = narrow ? 8 : s->B >= 2048 ? 16 : s->B >= 1024 ? 8 : 4;
+  if (es == 2 && p.waves == 16) p.waves = 8;
+  p.n_row_blocks = ceil_div(s->B, rows * p.waves);
+  p.n_items = ceil_div(static_cast<int64_t>(row_bytes), static_cast<int64_t>(piece_bytes)) * p.n_row_blocks;
+  p.xcd_span = ceil_div(p.n_items, 8);
+  p.steps_bytes = round_up(static_cast<size_t>(s->B) * static_cast<size_t>(s->K) * 8, kAlign);
+  return p;
+}
+
+void launch_order(const flexsae_shape *s, const int64_t *indices, const void *vals, vec_t<uint32_t, 2> *steps,
+                  int *status_flag, hipStream_t st) {
+  const int K = static_cast<int>(s->K);
+  const int C = K <= 64 ? 1 : K <= 128 ? 2 : K <= 256 ? 4 : 8;
+  // latents that share a key, so that the keys stay below the one of the elements past a row's end
+  int shift = 0;
+  while ((static_cast<uint64_t>(s->F - 1) >> shift) + 1 >= (uint64_t{1} << (32 - order_pos_bits(C)))) ++shift;
+  const dim3 grid(static_cast<unsigned>(ceil_div(s->B, kWavesPerBlock)));
+  const auto kernel = C == 1 ? topk_order_kernel<1> : C == 2 ? topk_order_kernel<2> : C == 4 ? topk_order_kernel<4> : topk_order_kernel<8>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, indices, vals, s->vals_dtype, s->B, K, s->F, shift, steps, status_flag);
+}
+
+template <typename WT>
+void launch_ordered_fwd(const flexsae_shape *s, const OrderedPlan &p, const vec_t<uint32_t, 2> *steps, const void *weight,
+                        const void *bias, const void *target, float *resid, double *partial, hipStream_t st) {
+  constexpr int VEC = 16 / static_cast<int>(sizeof(typename Traits<WT>::store_t));
+#define FLEXSAE_ORDERED(LPR, U, NW)                                                                                          \
+  hipLaunchKernelGGL((topk_ordered_fwd_kernel<WT, VEC, LPR, U, NW>), dim3(static_cast<unsigned>(p.xcd_span * 8)),            \
+                     dim3(NW * kWave), 0, st, steps, weight, bias, s->bias_dtype, target, s->target_dtype, resid, partial, \
+                     s->B, p.n_row_blocks, p.n_items, p.xcd_span, static_cast<int>(s->K), static_cast<int>(s->D))
+  if constexpr (VEC == 8) {
+    if (p.lpr == 8) {
+      FLEXSAE_ORDERED(8, 8, 8);
+    } else if (p.waves == 8) {
+      FLEXSAE_ORDERED(16, 16, 8);
+    } else {
+      FLEXSAE_ORDERED(16, 16, 4);
+    }
+  } else {
+    if (p.waves == 16) {
+      FLEXSAE_ORDERED(16, 16, 16);
+    } else if (p.waves == 8) {
+      FLEXSAE_ORDERED(16, 16, 8);
+    } else {
+      FLEXSAE_ORDERED(16, 16, 4);
+    }
+  }
+#undef FLEXSAE_ORDERED
+}
+
+// The TopK forward in latent order, where it pays, the rows allow it and the workspace has room behind the partials
+// (flexsae_topk_fwd_workspace_bytes).  Returns the number of loss partials, 0 if nothing was launched.
+int64_t forward_ordered(const flexsae_shape *s, const int64_t *indices, const void *weight, const void *vals,
+                        const void *bias, const void *target, float *resid, void *workspace, size_t workspace_bytes,
+                        int *status_flag, hipStream_t st) {
+  const OrderedPlan p = plan_ordered(s);
+  const size_t base = flexsae_fwd_workspace_bytes(s);
+  if (p.waves == 0 || workspace_bytes < base + p.steps_bytes || !aligned(weight, 16) ||
+      static_cast<size_t>(p.n_items) * sizeof(double) > base)
+    return 0;
+  if ((s->target_dtype == s->weight_dtype && !aligned(target, 16)) || (s->bias_dtype == s->weight_dtype && !aligned(bias, 16)))
+    return 0;
+  auto *const steps = reinterpret_cast<vec_t<uint32_t, 2> *>(static_cast<uint8_t *>(workspace) + base);
+  double *const partial = static_cast<double *>(workspace);
+  launch_order(s, indices, vals, steps, status_flag, st);
+  switch (s->weight_dtype) {
+    case FLEXSAE_F32:
+      launch_ordered_fwd<float>(s, p, steps, weight, bias, target, resid, partial, st);
+      break;
+    case FLEXSAE_BF16:
+      launch_ordered_fwd<bf16_t>(s, p, steps, weight, bias, target, resid, partial, st);
+      break;
+    default:
+      launch_ordered_fwd<f16_t>(s, p, steps, weight, bias, target, resid, partial, st);
+  }
+  return p.n_items;
+}
+
 template <bool HIER>
 int forward(const flexsae_shape *s, const int64_t *indices, const void *weight, const void *vals,
             const void *bias, const void *target, float *loss, float *resid, void *workspace,
@@ -247,30 +362,36 @@ int forward(const flexsae_shape *s, const int64_t *indices, const void *weight, 
   if (!workspace || workspace_bytes < flexsae_fwd_workspace_bytes(s) || !aligned(workspace, kAlign))
     return FLEXSAE_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const FwdPlan p = plan_fwd(s, weight, target, bias, resid);
-  // One double per block.  A tile has at least 64 columns and a block four rows (two or more rows are at least twice as
-  // many as blocks of them; a single row goes by row, four tiles to a block): no more than the workspace's four bytes
-  // per row and 64 columns, to which it is rounded up.
-  if (static_cast<size_t>(p.n_items) * sizeof(double) > workspace_bytes) return FLEXSAE_ERR_WORKSPACE;
+  int64_t n_partials = 0;
+  if constexpr (!HIER)
+    n_partials = forward_ordered(s, indices, weight, vals, bias, target, resid, workspace, workspace_bytes, status_flag, st);
   double *partial = static_cast<double *>(workspace);
-  switch (s->weight_dtype) {
-    case FLEXSAE_F32:
-      launch_fwd<float, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                status_flag, st);
-      break;
-    case FLEXSAE_BF16:
-      launch_fwd<bf16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                 status_flag, st);
-      break;
-    default:
-      launch_fwd<f16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
-                                status_flag, st);
+  if (n_partials == 0) {
+    const FwdPlan p = plan_fwd(s, weight, target, bias, resid);
+    // One double per block.  A tile has at least 64 columns and a block four rows (two or more rows are at least twice as
+    // many as blocks of them; a single row goes by row, four tiles to a block): no more than the workspace's four bytes
+    // per row and 64 columns, to which it is rounded up.
+    if (static_cast<size_t>(p.n_items) * sizeof(double) > workspace_bytes) return FLEXSAE_ERR_WORKSPACE;
+    switch (s->weight_dtype) {
+      case FLEXSAE_F32:
+        launch_fwd<float, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+                                  status_flag, st);
+        break;
+      case FLEXSAE_BF16:
+        launch_fwd<bf16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+                                   status_flag, st);
+        break;
+      default:
+        launch_fwd<f16_t, HIER>(s, p, indices, weight, vals, bias, target, resid, partial,
+                                  status_flag, st);
+    }
+    n_partials = p.n_items;
   }
   rc = launch_status();
   if (rc != FLEXSAE_OK) return rc;
   const double count = static_cast<double>(s->B) * static_cast<double>(s->D) *
                        (HIER ? static_cast<double>(s->K) : 1.0);
-  hipLaunchKernelGGL(loss_finalize_kernel, dim3(1), dim3(1024), 0, st, partial, p.n_items,
+  hipLaunchKernelGGL(loss_finalize_kernel, dim3(1), dim3(1024), 0, st, partial, n_partials,
                      1.0 / count, loss);
   return launch_status();
 }
@@ -1226,6 +1347,11 @@ size_t flexsae_fwd_workspace_bytes(const flexsae_shape *s) {
   if (check_shape(s) != FLEXSAE_OK) return 0;
   // one fp32 partial per (row, tile); the narrowest tile is 64 columns
   return round_up(static_cast<size_t>(s->B) * static_cast<size_t>(ceil_div(s->D, kWave)) * 4, kAlign);
+}
+
+size_t flexsae_topk_fwd_workspace_bytes(const flexsae_shape *s) {
+  const size_t base = flexsae_fwd_workspace_bytes(s);
+  return base == 0 ? 0 : base + plan_ordered(s).steps_bytes;
 }
 
 int flexsae_hier_fwd(const flexsae_shape *shape, const int64_t *indices, const void *weight,

@@ -38,6 +38,9 @@ namespace flexsae {
 // run to run.  Everything beyond a lane's own column of a row is added in double.
 constexpr int kFwdChunk = 64;  // steps per LDS fill
 
+// Bits of a pair's position in a row of at most 64 * C pairs (topk_order_kernel).
+constexpr int order_pos_bits(int C) { return C == 1 ? 6 : C == 2 ? 7 : C == 4 ? 8 : 9; }
+
 template <typename WT, int VEC, int LPR, bool HIER, int U>
 __global__ __launch_bounds__(256) void sae_fwd_kernel(
     const int64_t *__restrict__ indices, const void *__restrict__ weight,
@@ -194,6 +197,175 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) s += wave_loss[w];
+    partial[item] = s;
+  }
+}
+
+// ---- TopK forward in latent order ---------------------------------------------------------
+// The TopK loss adds a row's pairs up in any order, so every row can walk them by ascending latent.  The wavefronts that
+// an XCD runs at a time then sweep the latents of their column tile together, and a row piece that one of them gathers is
+// still in the L2 when the others ask for it: where one tile's pieces are several times the L2, the misses fall to about
+// the weights once (B=4096, K=128, F=65536, D=2304 bf16: 16.3 -> 6.3 million lines, 2.1 -> 0.8 GB; the least is 2.4).
+
+// (row of the weight matrix, val bits) of every pair, each row's pairs by ascending latent (and by position where two are
+// equal: the order, and so every sum, is the same on every run).  One wavefront per row of at most 64 * C pairs: a bitonic
+// sort of one key per pair, the latent's upper bits over the pair's position.  `shift` latent bits are left out where both
+// do not fit a dword, which costs locality within that few latents and nothing else.  An index outside [0, F) becomes
+// latent 0 with a val of zero, as in the kernels that read indices themselves.  5-6 us for half a million pairs, most of it
+// the launch (ranks by counting, a comparison per pair of pairs: 9 us at K=128, 19 at K=256).
+template <int C>
+__global__ __launch_bounds__(256) void topk_order_kernel(const int64_t *__restrict__ indices, const void *__restrict__ vals,
+                                                         int vals_dtype, int64_t B, int K, int64_t F, int shift,
+                                                         vec_t<uint32_t, 2> *__restrict__ steps, int *status_flag) {
+  constexpr int N = kWave * C;
+  constexpr int kPosBits = order_pos_bits(C);
+  static_assert(N == 1 << kPosBits, "a key holds the position of a pair in its row");
+  __shared__ vec_t<uint32_t, 2> rows[256 / kWave][N];
+  const int lane = lane_id();
+  vec_t<uint32_t, 2> *const mine = rows[wave_in_block()];
+  const int64_t b = static_cast<int64_t>(blockIdx.x) * (256 / kWave) + wave_in_block();
+  if (b >= B) return;  // uniform per wavefront
+  // element e = lane * C + c of the row
+  uint32_t key[C], vbits[C];
+  int64_t idx[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int k = lane * C + c;
+    const int64_t p = b * K + (k < K ? k : 0);
+    idx[c] = indices[p];
+    vbits[c] = load_scalar_bits(vals, vals_dtype, p);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int k = lane * C + c;
+    float v = scalar_from_bits(vbits[c], vals_dtype);
+    if (static_cast<uint64_t>(idx[c]) >= static_cast<uint64_t>(F)) {
+      if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);
+      idx[c] = 0;
+      v = 0.f;
+    }
+    vec_t<uint32_t, 2> s;
+    s[0] = static_cast<uint32_t>(idx[c]);
+    s[1] = __float_as_uint(v);
+    mine[k] = s;
+    // elements past the row's end sort behind all others (the host leaves the largest key free)
+    key[c] = k < K ? (static_cast<uint32_t>(idx[c]) >> shift) << kPosBits | static_cast<uint32_t>(k) : 0xffffffffu;
+  }
+#pragma unroll
+  for (int size = 2; size <= N; size *= 2) {
+#pragma unroll
+    for (int stride = size / 2; stride > 0; stride /= 2) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const bool up = size == N || ((lane * C + c) & size) == 0;  // this run ascends
+        if (stride >= C) {
+          const uint32_t other = __shfl_xor(key[c], stride / C);
+          const bool low = (lane & (stride / C)) == 0;
+          key[c] = (low == up) == (key[c] < other) ? key[c] : other;
+        } else if ((c & stride) == 0) {
+          const uint32_t a = key[c], z = key[c | stride];
+          key[c] = up == (a < z) ? a : z;
+          key[c | stride] = up == (a < z) ? z : a;
+        }
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int e = lane * C + c;
+    if (e < K) steps[b * K + e] = mine[key[c] & (N - 1)];
+  }
+}
+
+// sae_fwd_kernel for rows in latent order: NW wavefronts per block, the tiles cut into runs, one per XCD.
+// At most four wavefronts per SIMD and eight gathers in flight (16-byte lanes): with more of either the wavefronts of a
+// tile drift further apart than the L2 covers, and those of the next tile join them.  What bounds it: the L2s, at 13-14 of
+// the 18 TB/s they give to row gathers, and the misses beside them (5-6 TB/s).  Ordering included: B=4096, K=128, F=65536,
+// D=2304 bf16 286 -> 188 us (128-byte pieces), B=2048, K=256, F=131072, D=1024 fp32 275 -> 181 us (256-byte pieces).
+template <typename WT, int VEC, int LPR, int U, int NW>
+__global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(1, 4))) void topk_ordered_fwd_kernel(
+    const vec_t<uint32_t, 2> *__restrict__ ordered, const void *__restrict__ weight, const void *__restrict__ bias,
+    int bias_dtype, const void *__restrict__ target, int target_dtype, float *__restrict__ resid,
+    double *__restrict__ partial, int64_t B, int64_t n_row_blocks, int64_t n_items, int64_t xcd_span, int K, int D) {
+  constexpr int R = kWave / LPR;  // rows per wavefront
+  static_assert(kFwdChunk == kWave, "one lane per step of a chunk");
+  __shared__ vec_t<uint32_t, 2> steps[NW][R][kFwdChunk];
+  __shared__ double wave_loss[NW];
+  const int lane = lane_id();
+  const int wv = wave_in_block();
+  const int64_t i = blockIdx.x >> 3;
+  const int64_t item = (blockIdx.x & 7) * xcd_span + i;
+  if (i >= xcd_span || item >= n_items) return;  // uniform per block
+  const int64_t tile = item / n_row_blocks;
+  const int64_t b0 = ((item - tile * n_row_blocks) * NW + wv) * R;
+  const int64_t b = b0 + lane / LPR;
+  const int d0 = static_cast<int>(tile) * (LPR * VEC) + (lane % LPR) * VEC;
+  const bool active = d0 < D && b < B;  // D % VEC == 0 is checked on the host
+  const int dsafe = d0 < D ? d0 : 0;
+  const int64_t bsafe = b < B ? b : B - 1;
+  float e[VEC];
+  {
+    float t[VEC];
+    load_vec_dyn<WT, VEC>(bias, bias_dtype, dsafe, e);
+    load_vec_dyn<WT, VEC>(target, target_dtype, bsafe * D + dsafe, t);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) e[k] -= t[k];
+  }
+  using S = typename Traits<WT>::store_t;
+  const S *__restrict__ wbase = static_cast<const S *>(weight) + dsafe;
+  const uint32_t d_elems = static_cast<uint32_t>(D);
+  const vec_t<uint32_t, 2> *my_steps = &steps[wv][lane / LPR][0];
+  for (int k0 = 0; k0 < K; k0 += kFwdChunk) {
+    const int n = (K - k0) < kFwdChunk ? (K - k0) : kFwdChunk;  // uniform
+    {
+      vec_t<uint32_t, 2> s[R];
+      const int kk = k0 + (lane < n ? lane : 0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] = ordered[(b0 + r < B ? b0 + r : B - 1) * K + kk];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int r = 0; r < R; ++r) steps[wv][r][lane] = s[r];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    for (int j = 0; j < n; j += U) {
+      raw_vec_t<WT, VEC> raw[U];
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // past the end: the last step once more, not consumed
+        const vec_t<uint32_t, 2> s = my_steps[j + u < n ? j + u : n - 1];
+        v[u] = __uint_as_float(s[1]);
+        raw[u] = *reinterpret_cast<const raw_vec_t<WT, VEC> *>(wbase + static_cast<uint64_t>(s[0]) * d_elems);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (j + u < n) {  // uniform
+          float w[VEC];
+          unpack_raw<WT, VEC>(raw[u], w);
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) e[k] = fmaf(w[k], v[u], e[k]);
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  double lsum = 0.0;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) lsum = fma(static_cast<double>(e[k]), static_cast<double>(e[k]), lsum);
+  if (active)
+    store_vec<float, VEC>(resid, b * D + d0, e);
+  else
+    lsum = 0.0;
+  lsum = wave_sum_lane63(lsum);
+  if (lane == kWave - 1) wave_loss[wv] = lsum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) s += wave_loss[w];
     partial[item] = s;
   }
 }
