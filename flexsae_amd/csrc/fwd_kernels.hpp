@@ -3,6 +3,8 @@
 // every prefix), without ever materialising the [B,K,D] reconstruction.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace flexsae {
@@ -330,25 +332,31 @@ __global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(1, 4)
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
     }
-    for (int j = 0; j < n; j += U) {
-      raw_vec_t<WT, VEC> raw[U];
-      float v[U];
+    auto group = [&](auto count, int j) {
+      constexpr int N = decltype(count)::value;
+      raw_vec_t<WT, VEC> raw[N];
+      float v[N];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {  // past the end: the last step once more, not consumed
-        const vec_t<uint32_t, 2> s = my_steps[j + u < n ? j + u : n - 1];
+      for (int u = 0; u < N; ++u) {
+        const vec_t<uint32_t, 2> s = my_steps[j + u];
         v[u] = __uint_as_float(s[1]);
         raw[u] = *reinterpret_cast<const raw_vec_t<WT, VEC> *>(wbase + static_cast<uint64_t>(s[0]) * d_elems);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (j + u < n) {  // uniform
-          float w[VEC];
-          unpack_raw<WT, VEC>(raw[u], w);
+      for (int u = 0; u < N; ++u) {
+        float w[VEC];
+        unpack_raw<WT, VEC>(raw[u], w);
 #pragma unroll
-          for (int k = 0; k < VEC; ++k) e[k] = fmaf(w[k], v[u], e[k]);
-        }
+        for (int k = 0; k < VEC; ++k) e[k] = fmaf(w[k], v[u], e[k]);
       }
-    }
+    };
+    int j = 0;
+#pragma unroll 1
+    for (; j + U <= n; j += U) group(std::integral_constant<int, U>{}, j);
+#pragma unroll 1
+    for (; j + 4 <= n; j += 4) group(std::integral_constant<int, 4>{}, j);
+#pragma unroll 1
+    for (; j < n; ++j) group(std::integral_constant<int, 1>{}, j);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
