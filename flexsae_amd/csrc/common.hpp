@@ -320,23 +320,25 @@ __device__ __forceinline__ GatherSource make_gather_source(const void *base, uin
   g.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, static_cast<int>(bytes), 0x00020000);
   return g;
 }
-template <typename T, int VEC>
+// NT: non-temporal (streaming) load
+template <typename T, int VEC, bool NT = false>
 __device__ __forceinline__ raw_vec_t<T, VEC> gather_raw(const GatherSource &g, uint32_t lane_bytes,
                                                         uint32_t row_bytes_offset) {
+  constexpr int kAux = NT ? 2 : 0;  // cache-policy bits of the instruction: bit 1 = nt
   constexpr int kBytes = VEC * static_cast<int>(sizeof(typename Traits<T>::store_t));
   raw_vec_t<T, VEC> out;
   if constexpr (kBytes == 2) {
-    const uint16_t v = __builtin_amdgcn_raw_buffer_load_b16(g.rsrc, lane_bytes, row_bytes_offset, 0);
+    const uint16_t v = __builtin_amdgcn_raw_buffer_load_b16(g.rsrc, lane_bytes, row_bytes_offset, kAux);
     __builtin_memcpy(&out, &v, 2);
   } else if constexpr (kBytes == 4) {
-    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(g.rsrc, lane_bytes, row_bytes_offset, 0);
+    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(g.rsrc, lane_bytes, row_bytes_offset, kAux);
     __builtin_memcpy(&out, &v, 4);
   } else if constexpr (kBytes == 8) {
-    const vec_t<uint32_t, 2> v = __builtin_amdgcn_raw_buffer_load_b64(g.rsrc, lane_bytes, row_bytes_offset, 0);
+    const vec_t<uint32_t, 2> v = __builtin_amdgcn_raw_buffer_load_b64(g.rsrc, lane_bytes, row_bytes_offset, kAux);
     __builtin_memcpy(&out, &v, 8);
   } else {
     static_assert(kBytes == 16, "gathers are 2 to 16 bytes per lane");
-    const vec_t<uint32_t, 4> v = __builtin_amdgcn_raw_buffer_load_b128(g.rsrc, lane_bytes, row_bytes_offset, 0);
+    const vec_t<uint32_t, 4> v = __builtin_amdgcn_raw_buffer_load_b128(g.rsrc, lane_bytes, row_bytes_offset, kAux);
     __builtin_memcpy(&out, &v, 16);
   }
   return out;

@@ -1236,18 +1236,23 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   const int64_t n_pairs = static_cast<int64_t>(pl.n_pairs);
+  const int64_t n_groups = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock) * topk_group<WT, GT, VEC>());
+  // a launch holds fewer than 2^32 threads, 2^24 blocks: narrower slices where all tiles would be more
+  const int64_t most_tiles = (int64_t{1} << 23) / (n_groups + kLongBlocks);
+  if (slice_w / pl.tile > most_tiles) slice_w = (most_tiles < 1 ? 1 : most_tiles) * pl.tile;
   const int K = static_cast<int>(s->K), D = static_cast<int>(s->D), sw = static_cast<int>(slice_w);
   for (int64_t col0 = 0; col0 < s->D; col0 += slice_w) {
     const int64_t cols = (pl.d_pad - col0) < slice_w ? (pl.d_pad - col0) : slice_w;
     const int tps = static_cast<int>(cols / pl.tile);
-    const int64_t n_short_blocks = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock));
+    const int64_t xcd_span = ceil_div(n_groups * tps, 8);
+    const unsigned n_long = kLongBlocks * static_cast<unsigned>(tps);
     const size_t resid_bytes =
         static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * sizeof(typename Traits<RT>::store_t);
     hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC>),
-                       dim3(kLongBlocks + static_cast<unsigned>(n_short_blocks), static_cast<unsigned>(tps)),
+                       dim3(n_long + static_cast<unsigned>(xcd_span * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
-                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, kLongBlocks, tps,
+                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, tps,
                        static_cast<int>(col0), sw, s->F, K, D, static_cast<uint32_t>(resid_bytes));
     if (col0 + slice_w < s->D) {
       hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st,

@@ -5,13 +5,6 @@
 #include "common.hpp"
 #include "segment_kernels.hpp"
 
-#ifndef FLEXSAE_TOPK_ONE_GROUP
-#define FLEXSAE_TOPK_ONE_GROUP 1
-#endif
-// rows of a group of eight that share one uniform "are there rows left" test
-#ifndef FLEXSAE_TOPK_ROWS_PER_TEST
-#define FLEXSAE_TOPK_ROWS_PER_TEST 2
-#endif
 #ifndef FLEXSAE_TOPK_NT
 #define FLEXSAE_TOPK_NT true
 #endif
@@ -81,146 +74,222 @@ __device__ __forceinline__ void topk_accumulate_slots(
   }
 }
 
-// One short latent (1 to kSegChunk pairs) for one tile: the pair records of the latent are one
-// contiguous load, the residual rows are gathered through a buffer descriptor (no vector ALU work
-// for addresses) eight at a time (with the next eight already requested when registers allow),
-// and each group of eight shares one transposed wave reduction for the dvals dot products.  Inside a
-// group, rows are requested and consumed two at a time under one uniform test, so a latent with
-// nine pairs costs ten rows, not sixteen (a test per row costs more than it saves; the odd slot
-// past the end re-reads the last row, a cache hit, with a val of zero).  With bf16 weights and a
-// bf16 residual copy the products run on packed pairs (dot2) without unpacking.
-template <typename WT, typename GT, typename RT, int VEC>
-__device__ __forceinline__ void topk_short_latent(
-    const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight, int vals_dtype,
-    const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
-    float *__restrict__ dv_tile, int64_t f, uint32_t b0, int n, int d0, int D) {
+// A wavefront's W pieces, one per latent of its group, and in their places the finished pieces of dW.
+template <typename WT, typename GT, int VEC>
+union LatentPiece {
+  raw_vec_t<WT, VEC> w;
+  raw_vec_t<GT, VEC> g;
+};
+// Latents per wavefront: eight; four where a piece takes more than 16 bytes of LDS per lane (32 KB per block either way).
+template <typename WT, typename GT, int VEC>
+constexpr int topk_group() {
+  return sizeof(LatentPiece<WT, GT, VEC>) > 16 ? 4 : 8;
+}
+
+// The short latents (at most kSegChunk pairs) of a group of L neighbours, one tile: their pairs are one run of slots but for
+// the long latents among them, so a wavefront walks them as one stream.  The chain of trips to memory at the head of a
+// latent (its bounds, its records and W row, the first residual rows) is paid once per group, and the batches of eight rows
+// are full whatever the latents' counts.  The W pieces wait in the LDS, each finished piece of dW takes the place of its W
+// piece, and all of them are stored at the end: the memory counter retires in order, so a store among the gathers would be
+// waited for by the batch behind it.  Residual rows are gathered through a buffer descriptor (no vector ALU work for
+// addresses), each batch requested while other wavefronts work on theirs, and its dot products share one transposed wave
+// reduction.  With bf16 weights and a bf16 residual copy the products run on packed pairs (dot2) without unpacking.
+// What bounds it: the L2s' row gathers (14 of 18 TB/s at B=4096, K=128, F=65536, D=2304 bf16, W and dW beside them), for fp32
+// the W and dW streams.  Against one latent per wavefront (us; the kernel there 265 -> 245) the whole backward: K=128 340 ->
+// 320, K=64 247 -> 224, K=32 214 -> 180; F=262144, K=64 650 -> 463; B=2048, K=64, F=131072, D=1024 fp32 241 -> 192; two or four
+// latents, or two batches in flight (fewer wavefronts per SIMD): 2-20 % slower.
+template <typename WT, typename GT, typename RT, int VEC, int L>
+__device__ __forceinline__ void topk_short_latents(
+    const uint32_t *__restrict__ begin, const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight,
+    int vals_dtype, const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
+    float *__restrict__ dv_tile, int64_t f0, int64_t F, int d0, int D, LatentPiece<WT, GT, VEC> *__restrict__ pieces) {
   using S = typename Traits<RT>::store_t;
+  using S_w = typename Traits<WT>::store_t;
+  static_assert(L <= 8, "the counts of a wavefront's latents are scanned inside eight lanes");
   const int lane = lane_id();
   const bool active = d0 < D;
-  const uint32_t lane_off = static_cast<uint32_t>(active ? d0 : 0) * sizeof(S);
+  const int dsafe = active ? d0 : 0;
+  const uint32_t lane_off = static_cast<uint32_t>(dsafe) * sizeof(S);
   constexpr bool kDot2 = Traits<WT>::dtype == FLEXSAE_BF16 && Traits<RT>::dtype == FLEXSAE_BF16 && VEC % 2 == 0;
   const bool late_scale = kDot2 && vals_dtype == FLEXSAE_BF16;  // vals enter the dot2 as they are
 
-  const raw_vec_t<WT, VEC> wraw = load_raw<WT, VEC, FLEXSAE_TOPK_NT>(weight, f * D + (active ? d0 : 0));
-  // lanes past the end hold row 0 and a val of zero
-  const vec_t<uint32_t, 2> bv = lane < n ? __builtin_nontemporal_load(slot_bv + b0 + lane) : vec_t<uint32_t, 2>{0u, 0u};
-  const int my_b = static_cast<int>(bv[0]);
-  const uint32_t vbits = bv[1];
+  // lane l: first slot of latent f0 + l (of the one after the last for l = L, and wherever F cuts the group short)
+  const int64_t fl = f0 + (lane < L ? lane : L);
+  const uint32_t first = begin[fl < F ? fl : F];
+  const uint32_t past = static_cast<uint32_t>(__shfl_down(static_cast<int>(first), 1));  // (of all lanes: lane L is read)
+  const uint32_t n_all = lane < L ? past - first : 0u;
+  const bool is_long = n_all > static_cast<uint32_t>(kSegChunk);  // chunk role
+  const uint32_t n_mine = is_long ? 0u : n_all;
+  uint32_t upto = n_mine;  // pairs of latents f0 .. f0 + lane
+#pragma unroll
+  for (int d = 1; d < L; d *= 2) {
+    const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(upto), d));
+    if (lane >= d) upto += o;
+  }
+  const int M = bcast_i32(static_cast<int>(upto), L - 1);
+  const uint32_t s0 = static_cast<uint32_t>(bcast_i32(static_cast<int>(first), 0));
+  const uint64_t any_long = __ballot(is_long);
 
-  // two groups of eight rows in flight, or one when a group alone takes 32 registers: the
-  // kernel gains more from another wavefront per SIMD than from the deeper prefetch
-  constexpr bool kTwoGroups = sizeof(raw_vec_t<RT, VEC>) * 8 <= 64 || !FLEXSAE_TOPK_ONE_GROUP;
-  raw_vec_t<RT, VEC> buf_a[8], buf_b[kTwoGroups ? 8 : 1];
-  auto issue = [&](raw_vec_t<RT, VEC>(&buf)[8], int j) {
+  int at = -1, end = 0;  // the latent being summed and the place in the stream where its pairs end
+  vec_t<uint32_t, 2> bv{0u, 0u};
+  auto slot_of = [&](int p) {
+    uint32_t slot = s0 + static_cast<uint32_t>(p);
+    if (any_long) {
 #pragma unroll
-    for (int h = 0; h < 8; h += FLEXSAE_TOPK_ROWS_PER_TEST) {
-      if (h == 0 || j + h < n) {  // uniform: the second half of a group only when it has rows
-#pragma unroll
-        for (int u = h; u < h + FLEXSAE_TOPK_ROWS_PER_TEST; ++u) {
-          const int jj = (j + u) < n ? (j + u) : (n - 1);
-          buf[u] = gather_raw<RT, VEC>(rows_src, lane_off, static_cast<uint32_t>(bcast_i32(my_b, jj)) * row_stride);
-        }
-      }
+      for (int l = 0; l < L; ++l)
+        if (any_long >> l & 1)
+          slot += p >= bcast_i32(static_cast<int>(upto), l) ? static_cast<uint32_t>(bcast_i32(static_cast<int>(n_all), l)) : 0u;
     }
+    return slot;
   };
-  issue(buf_a, 0);
-  if constexpr (kTwoGroups) {
-    if (n > 8) issue(buf_b, 8);
+  uint32_t slot = slot_of(lane);
+  // W rows: for a latent without pairs here a descriptor of no bytes, which reads zeros and no memory (so do lanes beyond D)
+  raw_vec_t<WT, VEC> wraw[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const uint32_t bytes = bcast_i32(static_cast<int>(n_mine), l) != 0 ? static_cast<uint32_t>(D) * sizeof(S_w) : 0u;
+    const GatherSource row = make_gather_source(static_cast<const S_w *>(weight) + (f0 + l) * D, bytes);
+    wraw[l] = gather_raw<WT, VEC, FLEXSAE_TOPK_NT>(row, static_cast<uint32_t>(d0) * sizeof(S_w), 0u);
   }
+  if (lane < M) bv = __builtin_nontemporal_load(slot_bv + slot);
+#pragma unroll
+  for (int l = 0; l < L; ++l) pieces[l * kWave + lane].w = wraw[l];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 
-  float w[VEC], acc[VEC];
-  unpack_raw<WT, VEC>(wraw, w);
+  float w[kDot2 ? 1 : VEC], acc[VEC];
+  uint32_t ww[(VEC + 1) / 2];  // the W piece as packed pairs (dot2 path)
+  auto next_latent = [&]() {
+    do {
+      ++at;
+      end = bcast_i32(static_cast<int>(upto), at);
+    } while (bcast_i32(static_cast<int>(n_mine), at) == 0 && at < L - 1);
+    const raw_vec_t<WT, VEC> x = pieces[at * kWave + lane].w;
+    if constexpr (kDot2) __builtin_memcpy(ww, &x, sizeof(x));
+    else unpack_raw<WT, VEC>(x, w);
 #pragma unroll
-  for (int i = 0; i < VEC; ++i) {
-    acc[i] = 0.f;
-    if (!active) w[i] = 0.f;
-  }
-  uint32_t ww[(VEC + 1) / 2] = {};  // the W piece as packed pairs (dot2 path)
-  if constexpr (kDot2) {
-    __builtin_memcpy(ww, &wraw, sizeof(raw_vec_t<WT, VEC>));
+    for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
+  };
+  auto flush = [&]() {
+    if (late_scale) {
 #pragma unroll
-    for (int i = 0; i < VEC / 2; ++i)
-      if (!active) ww[i] = 0u;
-  }
-  const float v = __uint_as_float(vbits) * (late_scale ? 1.f : scale);
-  float my_dot = 0.f;
-  auto consume = [&](const raw_vec_t<RT, VEC>(&rows)[8], int j) {  // slots j .. j+7 of the latent
-    float dots[8];
+      for (int i = 0; i < VEC; ++i) acc[i] *= scale;
+    }
+    raw_vec_t<GT, VEC> x;
+    store_vec<GT, VEC>(&x, 0, acc);
+    pieces[at * kWave + lane].g = x;
+  };
+  if (M > 0) next_latent();
+  // late: vals are bf16 and enter the dot2 as they are (kDot2 only)
+  auto walk = [&](auto late) {
+    constexpr bool kLate = decltype(late)::value;
+#pragma unroll 1
+    for (int p0 = 0; p0 < M; p0 += kWave) {
+      const int n = M - p0 < kWave ? M - p0 : kWave;  // uniform
+      if (p0 > 0) {
+        slot = slot_of(p0 + lane);
+        bv = vec_t<uint32_t, 2>{0u, 0u};
+        if (lane < n) bv = __builtin_nontemporal_load(slot_bv + slot);
+      }
+      const uint32_t my_off = bv[0] * row_stride;
+      const uint32_t vbits = kLate ? bv[1] : __float_as_uint(__uint_as_float(bv[1]) * scale);
+      float my_dot = 0.f;
+      raw_vec_t<RT, VEC> rows[8];
+      auto issue = [&](int j) {  // past the end: the last row once more, not consumed
 #pragma unroll
-    for (int u = 0; u < 8; ++u) dots[u] = 0.f;
+        for (int u = 0; u < 8; ++u) {
+          const int jj = (j + u) < n ? (j + u) : (n - 1);
+          rows[u] = gather_raw<RT, VEC>(rows_src, lane_off, static_cast<uint32_t>(bcast_i32(static_cast<int>(my_off), jj)));
+        }
+      };
+      auto consume = [&](auto full, int j) {
+        constexpr bool kFull = decltype(full)::value;
+        float dots[8];
 #pragma unroll
-    for (int h = 0; h < 8; h += FLEXSAE_TOPK_ROWS_PER_TEST) {
-      if (h != 0 && j + h >= n) continue;  // uniform
+        for (int u = 0; u < 8; ++u) {
+          dots[u] = 0.f;
+          if (!kFull && j + u >= n) continue;  // uniform
+          if (p0 + j + u == end) {
+            flush();
+            next_latent();
+          }
+          const uint32_t vj = static_cast<uint32_t>(bcast_i32(static_cast<int>(vbits), j + u));
+          float dot = 0.f;
+          if constexpr (kDot2) {
+            uint32_t xw[VEC / 2];
+            __builtin_memcpy(xw, &rows[u], sizeof(xw));
 #pragma unroll
-      for (int u = h; u < h + FLEXSAE_TOPK_ROWS_PER_TEST; ++u) {
-        float dot = 0.f;
-        if constexpr (kDot2) {
-          uint32_t xw[VEC / 2];
-          __builtin_memcpy(xw, &rows[u], sizeof(xw));
+            for (int i = 0; i < VEC / 2; ++i) dot = dot2_bf16(xw[i], ww[i], dot);
+            if constexpr (kLate) {
+              // a bf16 val widened to fp32 keeps its 16 bits in the upper half
+              const uint32_t v_lo = vj >> 16;
 #pragma unroll
-          for (int i = 0; i < VEC / 2; ++i) dot = dot2_bf16(xw[i], ww[i], dot);
-          if (late_scale) {  // uniform
-            // a bf16 val widened to fp32 keeps its 16 bits in the upper half
-            const uint32_t v_hi = static_cast<uint32_t>(bcast_i32(static_cast<int>(vbits), j + u));
-            const uint32_t v_lo = v_hi >> 16;
+              for (int i = 0; i < VEC / 2; ++i) {
+                acc[2 * i] = dot2_bf16(xw[i], v_lo, acc[2 * i]);
+                acc[2 * i + 1] = dot2_bf16(xw[i], vj, acc[2 * i + 1]);
+              }
+            } else {
+              float x[VEC];
+              unpack_raw<RT, VEC>(rows[u], x);
 #pragma unroll
-            for (int i = 0; i < VEC / 2; ++i) {
-              acc[2 * i] = dot2_bf16(xw[i], v_lo, acc[2 * i]);
-              acc[2 * i + 1] = dot2_bf16(xw[i], v_hi, acc[2 * i + 1]);
+              for (int i = 0; i < VEC; ++i) acc[i] = fmaf(__uint_as_float(vj), x[i], acc[i]);
             }
           } else {
             float x[VEC];
             unpack_raw<RT, VEC>(rows[u], x);
-            const float vj = bcast_f32(v, j + u);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] = fmaf(vj, x[i], acc[i]);
+            for (int i = 0; i < VEC; ++i) {
+              acc[i] = fmaf(__uint_as_float(vj), x[i], acc[i]);
+              dot = fmaf(x[i], w[i], dot);
+            }
           }
-        } else {
-          float x[VEC];
-          unpack_raw<RT, VEC>(rows[u], x);
-          const float vj = bcast_f32(v, j + u);
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            acc[i] = fmaf(vj, x[i], acc[i]);
-            dot = fmaf(x[i], w[i], dot);
-          }
+          dots[u] = dot;
         }
-        dots[u] = dot;
+        const float tot = wave_sum8_transposed(dots);  // lane L: total of place j + (L & 7)
+        if ((lane >> 3) == (j >> 3)) my_dot = tot;
+      };
+      issue(0);
+#pragma unroll 1
+      for (int j = 0; j < n; j += 8) {
+        if (j + 8 <= n) consume(std::true_type{}, j);
+        else consume(std::false_type{}, j);
+        if (j + 8 < n) issue(j + 8);
       }
+      if (lane < n) dv_tile[slot] = my_dot * scale;
     }
-    const float tot = wave_sum8_transposed(dots);  // lane L: total of slot j + (L & 7)
-    if ((lane >> 3) == (j >> 3)) my_dot = tot;
   };
-  if constexpr (kTwoGroups) {
-    for (int j = 0; j < n; j += 16) {
-      consume(buf_a, j);
-      if (j + 16 < n) issue(buf_a, j + 16);
-      if (j + 8 < n) {
-        consume(buf_b, j + 8);
-        if (j + 24 < n) issue(buf_b, j + 24);
+  if constexpr (kDot2) {
+    if (late_scale) walk(std::true_type{});
+    else walk(std::false_type{});
+  } else {
+    walk(std::false_type{});
+  }
+  if (M > 0) flush();
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const uint32_t n = static_cast<uint32_t>(bcast_i32(static_cast<int>(n_all), l));
+    if (f0 + l < F && n <= static_cast<uint32_t>(kSegChunk)) {  // uniform
+      using G = typename Traits<GT>::store_t;
+      raw_vec_t<GT, VEC> x = pieces[l * kWave + lane].g;
+      if (n == 0) x = raw_vec_t<GT, VEC>{};
+      if (active) {
+        auto *const to = reinterpret_cast<raw_vec_t<GT, VEC> *>(static_cast<G *>(dW) + (f0 + l) * D + d0);
+        if constexpr (FLEXSAE_TOPK_NT) __builtin_nontemporal_store(x, to);
+        else *to = x;
       }
     }
-  } else {
-    for (int j = 0; j < n; j += 8) {
-      consume(buf_a, j);
-      if (j + 8 < n) issue(buf_a, j + 8);
-    }
   }
-  if (late_scale) {
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] *= scale;
-  }
-  if (active) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f * D + d0, acc);
-  if (lane < n) dv_tile[b0 + lane] = my_dot * scale;
 }
 
 // TopK backward of one slice.  scale = grad_out * 2/(B*D).
-// Blocks [0, n_long_blocks): long latents, one wavefront per (64-pair chunk, tile): stores its
+// Blocks [0, n_long_blocks), a multiple of eight: long latents, one wavefront per (64-pair chunk, tile): stores its
 // dvals shares, leaves its dW contribution in partial[chunk, slice column] (fp32) for
 // seg_reduce_long_finalize_kernel (next launch).  They come first so hot latents start at once.
-// Remaining blocks: one wavefront per (tile of the slice = blockIdx.y, latent f); blocks are
-// handed out x first, i.e. tile-major, so that at any moment the waves in flight share one
-// B x tile slice of resid (L2-sized); see topk_short_latent.  tile = 64*VEC columns, lane l owning VEC consecutive columns.
+// Remaining blocks: one wavefront per (tile of the slice, group of latents), see topk_short_latents; tile = 64*VEC columns,
+// lane l owning VEC consecutive columns.  The n_groups blocks of each of the tps tiles, tiles outermost, are cut into eight runs of
+// xcd_span, one per XCD (blocks go round the XCDs): an L2 holds the B x tile slice of resid that its own wavefronts
+// gather from, instead of every L2 fetching every slice (B=2048, K=256, F=131072, D=1024 fp32 327 -> 301 us for the whole
+// backward, K=64 249 -> 192; bf16 the same either way).
 // dW[f, tile] is written exactly once, in the gradient's final dtype; latents without pairs
 // get zeros.
 template <typename WT, typename GT, typename RT, int VEC>
@@ -231,37 +300,32 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
-    unsigned n_long_blocks, int tps, int col0, int slice_w, int64_t F, int K, int D,
+    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int tps, int col0, int slice_w, int64_t F, int K, int D,
     uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
+  constexpr int L = topk_group<WT, GT, VEC>();
+  __shared__ LatentPiece<WT, GT, VEC> pieces[256 / kWave][L * kWave];
   if (blockIdx.x >= n_long_blocks) {
-    // blockIdx.y = tile of the slice, blockIdx.x - n_long_blocks = group of latents
-    const int64_t f = static_cast<int64_t>(blockIdx.x - n_long_blocks) * (blockDim.x >> 6) + wave_in_block();
-    if (f >= F) return;  // uniform per wavefront
-    const int t = static_cast<int>(blockIdx.y);
-    const uint32_t b0 = begin[f];
-    const uint32_t n = begin[f + 1] - b0;
-    if (n > static_cast<uint32_t>(kSegChunk)) return;  // chunk role
-    const int d0 = col0 + t * (kWave * VEC) + lane * VEC;
-    if (n == 0) {  // unused latent: zeros
-      const float zero[VEC] = {};
-      if (d0 < D) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f * D + d0, zero);
-      return;
-    }
+    const int64_t i = (blockIdx.x - n_long_blocks) >> 3;
+    const int64_t item = (blockIdx.x & 7) * xcd_span + i;
+    const int t = static_cast<int>(item / n_groups);
+    if (i >= xcd_span || t >= tps) return;
+    const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * L;
+    if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
-    topk_short_latent<WT, GT, RT, VEC>(
-        slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(D) * sizeof(typename Traits<RT>::store_t), scale,
-        dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f, b0, static_cast<int>(n), d0, D);
+    topk_short_latents<WT, GT, RT, VEC, L>(
+        begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(D) * sizeof(typename Traits<RT>::store_t), scale,
+        dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, F, col0 + t * (kWave * VEC) + lane * VEC, D,
+        pieces[wave_in_block()]);
     return;
   }
   const uint32_t n_long = long_ctrl[kLongCount];
   if (n_long == 0) return;
   const uint32_t n_chunks = long_ctrl[kLongChunks];
   const int64_t total = static_cast<int64_t>(n_chunks) * tps;
-  const int64_t n_waves = static_cast<int64_t>(n_long_blocks) * gridDim.y * (blockDim.x >> 6);
-  for (int64_t wk = (static_cast<int64_t>(blockIdx.y) * n_long_blocks + blockIdx.x) * (blockDim.x >> 6) +
-                    wave_in_block();
+  const int64_t n_waves = static_cast<int64_t>(n_long_blocks) * (blockDim.x >> 6);
+  for (int64_t wk = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
        wk < total; wk += n_waves) {
     // tile-major over the work list as well
     const int t = static_cast<int>(wk / n_chunks);

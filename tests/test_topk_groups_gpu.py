@@ -1,0 +1,51 @@
+"""TopK backward, groups of neighbouring latents per wavefront: latents without pairs, with the most a group takes, and
+with more than that (reduced apart) side by side; groups cut short by F, streams of more than 64 pairs; against float64."""
+import pytest
+import torch
+
+from tests import abi
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+
+
+@pytest.mark.parametrize("D", [8, 520, 1030, 77])
+@pytest.mark.parametrize("dtype,vals_dtype,dw_dtype", [
+    (torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16, torch.bfloat16),
+    (torch.bfloat16, torch.float32, torch.float32), (torch.float16, torch.float16, torch.float16)], ids=str)
+@pytest.mark.parametrize("counts", [
+    [0, 64, 65, 1, 0, 0, 130, 64, 64, 64, 64, 64, 64, 64, 64, 64, 0, 0, 0, 0, 0, 0, 0, 0, 3],
+    [5], [0, 0, 7, 66, 0, 8, 9, 1, 0], [66] * 8 + [2] * 33 + [0] * 7], ids=["edges", "one", "short", "runs"])
+def test_groups(counts, dtype, vals_dtype, dw_dtype, D):
+    print("[case]", counts[:4], dtype, vals_dtype, dw_dtype, D, flush=True)
+    F = len(counts)
+    K = 4
+    pairs = torch.cat([torch.full((c,), f, dtype=torch.long) for f, c in enumerate(counts)])
+    B = -(-len(pairs) // K)
+    g = torch.Generator().manual_seed(len(pairs) + D)
+    pairs = torch.cat([pairs, torch.full((B * K - len(pairs),), F - 1)])
+    idx = pairs[torch.randperm(B * K, generator=g)].view(B, K)
+    W = torch.randn(F, D, generator=g).to(dtype)
+    v = torch.randn(B, K, generator=g).to(vals_dtype)
+    resid = torch.randn(B, D, generator=g)
+    grad = 1.5
+    rc, dW, dv, db = abi.topk_backward(idx.to(DEV), W.to(DEV), v.to(DEV), resid.to(DEV), grad, dw_dtype=dw_dtype)
+    torch.cuda.synchronize()
+    assert rc == 0
+    gathered = resid.to(torch.bfloat16) if dtype == torch.bfloat16 else resid  # what the call gathers
+    scale = grad * 2.0 / (B * D)
+    rows = gathered.double().repeat_interleave(K, 0)
+    flat = idx.reshape(-1)
+    terms = v.double().reshape(-1, 1) * scale * rows
+    exact = torch.zeros(F, D, dtype=torch.double).index_add_(0, flat, terms)
+    size = torch.zeros(F, D, dtype=torch.double).index_add_(0, flat, terms.abs())
+    # a rounding per pair and a few for the scale and the chunks' sums, then the one to dW's type
+    n = torch.tensor(counts).double().max() + K + 8
+    half_ulp = {  # of numbers of 8 and 11 significant bits
+        torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dw_dtype]
+    floor = 2.0 ** -25 if dw_dtype == torch.float16 else 0.0  # half of fp16's smallest number
+    assert ((dW.cpu().double() - exact).abs() <= n * 2.0 ** -24 * size + 1.001 * half_ulp * exact.abs() + floor).all()
+    prods = rows * W.double()[flat] * scale
+    bound = (D + 8) * 2.0 ** -24 * prods.abs().sum(1)
+    assert ((dv.cpu().double().reshape(-1) - prods.sum(1)).abs() <= bound).all()
