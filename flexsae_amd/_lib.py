@@ -39,6 +39,7 @@ BWD_REUSE_HOT_TABLES = 1024
 BWD_DENSE_LATENTS = 2048
 BWD_HOT_BLOCKS_64 = 4096
 BWD_HOT_BLOCKS_32 = 8192
+BWD_RAGGED_ROWS = 16384
 TOPK_BWD_FP32_RESIDUAL = 256
 
 

@@ -709,6 +709,12 @@ inline bool piece_reduce_ok(const flexsae_shape *s, const HierBwdPlan &p, const 
          (dW == nullptr || aligned(dW, static_cast<size_t>(ev) * dtype_size(dW_dtype)));
 }
 
+// The same for the training step: rows that allow no 8- or 16-byte access of their own elements are reduced by pieces, which
+// are read 16 bytes per lane whatever D is and written in dword-aligned vectors or by elements.
+inline bool train_piece_ok(const flexsae_shape *s, const HierBwdPlan &p, const void *dW, int dW_dtype) {
+  return p.vec < 4 ? train_tile_cols(s) % piece_cols(p) == 0 : piece_reduce_ok(s, p, dW, dW_dtype);
+}
+
 // Columns the slice loop works on: D rounded up to whole reduction tiles, or to whole training tiles
 // when the piece reduction lets slices end there.
 inline int64_t hier_cols_used(const flexsae_shape *s, const HierBwdPlan &p, bool train, bool piece) {
@@ -731,7 +737,12 @@ inline bool solo_marks(const flexsae_shape *s) { return s->B * s->K < (1LL << 30
 inline uint32_t slot_mask(const flexsae_shape *s) { return solo_marks(s) ? kSoloSlotBit - 1u : 0xffffffffu; }
 
 // largest K the training-step kernel holds in registers
-inline bool train_supported(const flexsae_shape *s) { return s->D % 4 == 0 && s->K <= 256; }
+inline bool train_supported(const flexsae_shape *s, int flags = 0) {
+  if (s->K > 256) return false;
+  // FLEXSAE_BWD_RAGGED_ROWS: any row that a lane's columns divide (two, or one for fp32 rows of more than 64 steps)
+  if (flags & FLEXSAE_BWD_RAGGED_ROWS) return s->D % 2 == 0 || train_tile_cols(s) == kWave;
+  return s->D % 4 == 0;
+}
 
 // Row pieces the training-step kernel keeps in the LDS instead of registers (one dword per lane
 // and row: 16-bit weights with two columns per lane, fp32 with one), chosen so that one more
@@ -1435,10 +1446,10 @@ size_t flexsae_hier_bwd_workspace_bytes(const flexsae_shape *s, int64_t slice_co
 }
 
 size_t flexsae_hier_fwd_bwd_workspace_bytes_flags(const flexsae_shape *s, int64_t slice_cols, int flags) {
-  if (check_shape(s) != FLEXSAE_OK || !train_supported(s)) return 0;
+  if (check_shape(s) != FLEXSAE_OK || !train_supported(s, flags)) return 0;
   const bool hot = (flags & FLEXSAE_BWD_HOT_LATENTS) && hot_supported(s);
   const HierBwdPlan pl = plan_hier_bwd(s, hot, flags);
-  const int64_t granule = piece_reduce_ok(s, pl, nullptr, s->weight_dtype) ? train_tile_cols(s) : pl.tile;
+  const int64_t granule = train_piece_ok(s, pl, nullptr, s->weight_dtype) ? train_tile_cols(s) : pl.tile;
   int64_t sw = slice_cols <= 0 ? granule : ceil_div(slice_cols, granule) * granule;
   if (sw > pl.d_pad) sw = pl.d_pad;
   return hier_bwd_bytes(pl, sw);
@@ -1596,12 +1607,13 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   if (!indices || !weight || !vals || !bias || !target || !loss || !dvals || !dbias ||
       (!defer_reduce && !no_dw && (!dW || !valid_dtype(dW_dtype))))
     return FLEXSAE_ERR_INVALID_ARGUMENT;
-  if (!train_supported(s)) return FLEXSAE_ERR_UNSUPPORTED;
+  if (!train_supported(s, flags)) return FLEXSAE_ERR_UNSUPPORTED;
+  if (s->D % 4 != 0 && defer_reduce) return FLEXSAE_ERR_UNSUPPORTED;
   // hot-latent accumulators: a hint, taken where the shape allows them, the reductions run in this
   // call and every pointer is aligned for the piece reduction (the workspace layout depends on it)
   const bool hot = (flags & FLEXSAE_BWD_HOT_LATENTS) && hot_supported(s) && !defer_reduce &&
                    piece_reduce_ok(s, plan_hier_bwd(s), (defer_reduce || no_dw) ? nullptr : dW, dW_dtype);
-  const HierBwdPlan pl = plan_hier_bwd(s, hot, flags);  // D % 4 == 0 here, so tiles are 256 columns
+  const HierBwdPlan pl = plan_hier_bwd(s, hot, flags);
   if (!aligned(indices, 8) || !aligned(weight, 4 * dtype_size(s->weight_dtype)) ||
       !aligned(vals, dtype_size(s->vals_dtype)) || !aligned(bias, 2 * dtype_size(s->bias_dtype)) ||
       !aligned(target, 2 * dtype_size(s->target_dtype)) || !aligned(loss, 4) ||
@@ -1610,7 +1622,7 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
     return FLEXSAE_ERR_ALIGNMENT;
   // slices are whole training tiles when the reduction can work on 256-byte pieces, else whole
   // reduction tiles
-  const bool piece = piece_reduce_ok(s, pl, (defer_reduce || no_dw) ? nullptr : dW, dW_dtype);
+  const bool piece = train_piece_ok(s, pl, (defer_reduce || no_dw) ? nullptr : dW, dW_dtype);
   if (sgd_step && !piece) return FLEXSAE_ERR_UNSUPPORTED;  // only the piece reduction updates in place
   const int64_t granule = piece ? train_tile_cols(s) : pl.tile;
   if (!workspace || !aligned(workspace, kAlign) || workspace_bytes < hier_bwd_bytes(pl, granule))
@@ -1639,13 +1651,14 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   const TrainArgs ta = {bias, target, loss, s->B * (hier_cols_used(s, pl, true, piece) / train_tile_cols(s)),
                         1.0 / count};
   // without dW the reductions are left out like in the deferred case (dW_dtype only selects a template then)
-  launch_hier_slices_w<4>(s, pl, slice_w, indices, weight, vals, nullptr, sgd_step, coef, dW,
-                          no_dw ? s->weight_dtype : dW_dtype, dvals, dbias, ws,
-                          (flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE |
-                                    FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS)) |
-                              (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : 0) | (hot ? kBwdHot : 0) |
-                              (solo ? kBwdSolo : 0),
-                          status_flag, st, &ta, piece ? static_cast<int>(piece_cols(pl)) : 0);
+  const auto slices = pl.vec == 4 ? launch_hier_slices_w<4> : pl.vec == 2 ? launch_hier_slices_w<2> : launch_hier_slices_w<1>;
+  slices(s, pl, slice_w, indices, weight, vals, nullptr, sgd_step, coef, dW,
+         no_dw ? s->weight_dtype : dW_dtype, dvals, dbias, ws,
+         (flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE |
+                   FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS)) |
+             (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : 0) | (hot ? kBwdHot : 0) |
+             (solo ? kBwdSolo : 0),
+         status_flag, st, &ta, piece ? static_cast<int>(piece_cols(pl)) : 0);
   return launch_status();
 }
 

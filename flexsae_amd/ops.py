@@ -633,6 +633,15 @@ def _train_supported(weight: Tensor, K: int) -> bool:
     return D % 4 == 0 and K <= 256
 
 
+def _train_ragged(weight: Tensor, K: int) -> bool:
+    """Rows that the training-step kernel takes by its lanes' columns though no vector of four divides them
+    (FLEXSAE_BWD_RAGGED_ROWS; not staged): one gather instead of one in the forward and one in the sweep, the same bits
+    (B = 1777, K = 50, F = 24571, D = 1538 bf16: the step 298 -> 266 us; B = 4096, K = 128, F = 65536, D = 2306:
+    1892 -> 1486)."""
+    D = weight.shape[1]
+    return D % 4 != 0 and K <= 256 and (D % 2 == 0 or (weight.dtype == torch.float32 and K > 64))
+
+
 def _stage_fits(indices: Tensor, weight: Tensor) -> bool:
     """Staging keeps one contribution per (b, k, d) alive until the backward; it is chosen only
     when the stage budget covers that."""
@@ -767,7 +776,8 @@ def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tenso
         hot_flag = _hot_flags(B, K, D, dev) if (hot and need_dw) else 0
         if hot_flag:
             slice_cols = _hot_slice_cols(B, slice_cols, dev)
-        ws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(shape), slice_cols, hot_flag)
+        ragged = _lib.BWD_RAGGED_ROWS if _train_ragged(weight, K) else 0
+        ws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(shape), slice_cols, hot_flag | ragged)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)
         dw_dtype = _unit_dw_dtype(weight.dtype)
@@ -779,7 +789,7 @@ def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tenso
         if cached is not None:
             _pair_import(lib, shape, workspace, cached)
         flags = ((_lib.BWD_REUSE_PAIR_LIST if cached is not None else 0) | (0 if need_dw else _lib.BWD_NO_DW) |
-                 hot_flag | (_lib.BWD_DENSE_LATENTS if dense else 0))
+                 hot_flag | (_lib.BWD_DENSE_LATENTS if dense else 0) | ragged)
         rc = lib.flexsae_hier_fwd_bwd(ctypes.byref(shape), _ptr(indices), _ptr(weight), _ptr(vals), _ptr(bias),
                                       _ptr(target), _ptr(loss), _ptr(dW) if need_dw else None,
                                       _DTYPES[dw_dtype], _ptr(dvals),
@@ -1042,10 +1052,10 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
         indices = indices.to(torch.int64)
     needs_grad = torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad)
     if (needs_grad and _fused_training and weight.dim() == 2 and indices.dim() == 2
-            and _train_supported(weight, indices.shape[1])):
+            and (_train_supported(weight, indices.shape[1]) or _train_ragged(weight, indices.shape[1]))):
         # (a compiler trace cannot follow the stage's size query: traced calls take the sliced step,
         # which gives the same bits)
-        if _stage_fits(indices, weight) and not _is_traced(weight):
+        if _train_supported(weight, indices.shape[1]) and _stage_fits(indices, weight) and not _is_traced(weight):
             return _HierTrainStaged.apply(indices, weight, vals, bias, target)
         # (fp16 weights: the step's unit-gradient dW is fp32, of magnitude 2/(B*K*D), and is scaled by the
         # upstream gradient before its only rounding, like reference hierarchical_kernels.py:294-299)

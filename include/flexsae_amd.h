@@ -97,6 +97,10 @@ enum {
   FLEXSAE_BWD_HOT_BLOCKS_32 = 8192,  /* of 32, or with both flags of 16: for batches whose blocks */
                                      /* of 128 rows are fewer than the compute units.  The same */
                                      /* flags in the workspace query and in every call on it    */
+  FLEXSAE_BWD_RAGGED_ROWS = 16384,   /* flexsae_hier_fwd_bwd: also take rows that no vector of   */
+                                     /* four columns divides: D % 2 == 0, or any D for fp32     */
+                                     /* weights with K > 64 (not with SWEEP_ONLY).  The same    */
+                                     /* flag in the workspace query                             */
   FLEXSAE_BWD_HOT_NO_HEADROOM = 512, /* NOT PART OF THE STABLE ABI (a test aid): the block      */
                                      /* exponent of the hot-latent accumulators is set 8 bits   */
                                      /* lower than usual, so that most rows take the deferred   */
@@ -211,7 +215,7 @@ int flexsae_hier_bwd(const flexsae_shape *shape, const int64_t *indices, const v
  * the real one afterwards (flexsae_scale for dW; dvals/dbias are small).  Same workspace, same
  * slicing and the same segment reduction as flexsae_hier_bwd (use
  * flexsae_hier_bwd_workspace_bytes).
- * Supported when D % 4 == 0 and K <= 256 (the row pieces of a tile are kept on chip: in registers
+ * Supported when D % 4 == 0 (FLEXSAE_BWD_RAGGED_ROWS: see there) and K <= 256 (the row pieces of a tile are kept on chip: in registers
  * and, for K = 64, 128 or 256, a quarter of them in the LDS):
  * flexsae_hier_fwd_bwd_supported() tells; otherwise FLEXSAE_ERR_UNSUPPORTED (use
  * flexsae_hier_fwd + flexsae_hier_bwd).
