@@ -196,6 +196,7 @@ topk_fwd.register_fake(_fwd_fake)
 # None (the default) sizes it from the problem, see _hier_scratch_budget.
 _hier_scratch_bytes = (int(os.environ["FLEXSAE_HIER_SCRATCH_MB"]) << 20) if "FLEXSAE_HIER_SCRATCH_MB" in os.environ else None
 _HIER_SCRATCH_CAP = 256 << 20
+_HIER_SCRATCH_LEAST = 128 << 20
 
 
 # Narrowest slice the scratch budget may lead to on its own; a budget that gives fewer columns is
@@ -226,11 +227,16 @@ def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype) -> int:
     matrix, at most 256 MiB -- memory above the inputs then stays within about 1.25 of the TopK
     loss's (whose peak is the dense gradient plus the residual) whatever K is, at 4-5 % of the step
     time where that is less than the 256 MiB that measured fastest (B = 4096, F = 65536, D = 2304,
-    bf16: K = 32 0.483 instead of 0.463 ms, K = 64 0.751 instead of 0.717 ms; K = 128 unchanged)."""
+    bf16: K = 32 0.483 instead of 0.463 ms, K = 64 0.751 instead of 0.717 ms; K = 128 unchanged) --
+    and at least 128 MiB: weights small enough to give less have batches whose slices, launch by
+    launch, leave compute units idle (us with 0.45 of the weights, 64 and 128 MiB: B = 1777, K = 50,
+    F = 24571, D = 1538 bf16 284, 277, 246; B = 512, K = 128, F = 16384, D = 8192 bf16 730, 697, 675;
+    B = 1024, K = 256, F = 16384, D = 2048 fp32 1260, 1261, 1035; B = 200, K = 250, F = 8000,
+    D = 2048 fp32 679, 364, 350)."""
     if _hier_scratch_bytes is not None:
         return _hier_scratch_bytes
     sw = 4 if weight_dtype == torch.float32 else 2
-    return min(_HIER_SCRATCH_CAP, int(0.45 * F * D * sw))
+    return min(_HIER_SCRATCH_CAP, max(_HIER_SCRATCH_LEAST, int(0.45 * F * D * sw)))
 
 
 def _hier_slice_cols(B: int, K: int, F: int, D: int, weight_dtype) -> int:
@@ -247,7 +253,7 @@ def set_hier_scratch_bytes(nbytes) -> None:
     """Upper bound on the scratch of the hierarchical backward (bytes): the per-pair contributions
     of one slice of columns.  0 = use the atomic scatter fallback, which needs no scratch but an
     fp32 [F,D] accumulator.  ``None`` (the default) sizes it from the problem: 0.45 of the weight
-    matrix, at most 256 MiB.  A slice is never narrower than ``set_hier_min_slice_cols``, so with
+    matrix, at least 128 and at most 256 MiB.  A slice is never narrower than ``set_hier_min_slice_cols``, so with
     many pairs the scratch can exceed the bound by a large factor (B*K*256 contributions).  Slices
     of 256 columns measured fastest at B*K = 2^19 pairs; wider ones are not faster."""
     global _hier_scratch_bytes
