@@ -89,6 +89,7 @@ SIGNATURES = {
     "flexsae_topk_bwd_workspace_bytes": (_sz, [_shape_p, _i64]),
     "flexsae_cast_from_f32": (_int, [_p, _int, _p, _i64, _p]),
     "flexsae_scale_from_f32": (_int, [_p, _int, _p, _i64, _p, _p]),
+    "flexsae_finish_grads": (_int, [_p, _int, _p, _int, _i64, _p, _int, _p, _i64, _p, _int, _p, _i64, _p, _p]),
     "flexsae_hier_hot_latents_supported": (_int, [_shape_p]),
     "flexsae_hier_hot_stats": (_int, [_shape_p, _p, _p, _p]),
     "flexsae_hier_pair_stats": (_int, [_shape_p, _p, _p, _p]),

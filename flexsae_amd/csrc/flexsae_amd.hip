@@ -1821,6 +1821,39 @@ int flexsae_scale_from_f32(void *dst, int dst_dtype, const float *src, int64_t n
   return launch_status();
 }
 
+int flexsae_finish_grads(void *dW, int dW_dtype, const void *dW_unit, int dW_unit_dtype, int64_t n_dw, void *dvals,
+                         int dvals_dtype, const float *dvals_unit, int64_t n_dvals, void *dbias, int dbias_dtype,
+                         const float *dbias_unit, int64_t n_dbias, const float *scale, void *stream) {
+  if (n_dw < 0 || n_dvals < 0 || n_dbias < 0 || (n_dw > 0 && (!dW || !dW_unit)) || (n_dvals > 0 && (!dvals || !dvals_unit)) ||
+      (n_dbias > 0 && (!dbias || !dbias_unit)) || !valid_dtype(dW_dtype) || !valid_dtype(dW_unit_dtype) ||
+      !valid_dtype(dvals_dtype) || !valid_dtype(dbias_dtype) ||
+      (dW_unit_dtype != dW_dtype && (dW_unit_dtype != FLEXSAE_F32 || dW == dW_unit)))
+    return FLEXSAE_ERR_INVALID_ARGUMENT;
+  if ((n_dw > 0 && (!aligned(dW, 4 * dtype_size(dW_dtype)) || !aligned(dW_unit, 4 * dtype_size(dW_unit_dtype)))) ||
+      (n_dvals > 0 && (!aligned(dvals, 4 * dtype_size(dvals_dtype)) || !aligned(dvals_unit, 16))) ||
+      (n_dbias > 0 && (!aligned(dbias, 4 * dtype_size(dbias_dtype)) || !aligned(dbias_unit, 16))) || !aligned(scale, 4))
+    return FLEXSAE_ERR_ALIGNMENT;
+  if (n_dw + n_dvals + n_dbias == 0) return FLEXSAE_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const unsigned n_small = 1 + grid_for(ceil_div(n_dvals, 4), 256, 1024);
+  // in place: few blocks, since by one they all return at once
+  const unsigned n_large = n_dw == 0 ? 0 : grid_for(ceil_div(n_dw, 4), 256, dW == dW_unit ? 2048 : 1 << 16);
+#define FLEXSAE_FINISH(UT, GT)                                                                                             \
+  hipLaunchKernelGGL((finish_grads_kernel<UT, GT>), dim3(n_small + n_large), dim3(256), 0, st, dW, dW_unit, n_dw, dvals,   \
+                     dvals_dtype, dvals_unit, n_dvals, dbias, dbias_dtype, dbias_unit, n_dbias, scale, n_small)
+  if (dW_unit_dtype == FLEXSAE_F32) {
+    if (dW_dtype == FLEXSAE_F32) FLEXSAE_FINISH(float, float);
+    else if (dW_dtype == FLEXSAE_BF16) FLEXSAE_FINISH(float, bf16_t);
+    else FLEXSAE_FINISH(float, f16_t);
+  } else if (dW_unit_dtype == FLEXSAE_BF16) {
+    FLEXSAE_FINISH(bf16_t, bf16_t);
+  } else {
+    FLEXSAE_FINISH(f16_t, f16_t);
+  }
+#undef FLEXSAE_FINISH
+  return launch_status();
+}
+
 int flexsae_cast_from_f32(void *dst, int dst_dtype, const float *src, int64_t n, void *stream) {
   return flexsae_scale_from_f32(dst, dst_dtype, src, n, nullptr, stream);
 }

@@ -501,9 +501,8 @@ def _pair_export(lib, shape, workspace: Tensor, indices: Tensor, F: int) -> None
     _pair_store(indices, F, begin, pair_map)
 
 
-@torch.library.custom_op("flexsae_amd::hier_bwd", mutates_args=())
-def hier_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
-             resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+def _hier_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
+                   resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
     lib = _lib.load()
     B, K = indices.shape
     F, D = weight.shape
@@ -545,6 +544,9 @@ def hier_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
     return dW, dvals, dbias
 
 
+hier_bwd = torch.library.custom_op("flexsae_amd::hier_bwd", mutates_args=())(_hier_bwd_impl)
+
+
 # With bf16 weights the TopK backward gathers a bf16 copy of the residual (half the cache footprint;
 # the reference's backward also receives the residual gradient in the weight dtype, reference
 # torch-ext/flex_sae/topk_kernels.py:52).  That rounding shows in `vals.grad` (about 4e-3 normwise
@@ -559,9 +561,8 @@ def set_topk_residual_bf16(enabled: bool) -> None:
     _topk_residual_bf16 = bool(enabled)
 
 
-@torch.library.custom_op("flexsae_amd::topk_bwd", mutates_args=())
-def topk_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
-             resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
+                   resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
     lib = _lib.load()
     B, K = indices.shape
     F, D = weight.shape
@@ -596,6 +597,9 @@ def topk_bwd(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
                                   0 if _topk_residual_bf16 else _lib.TOPK_BWD_FP32_RESIDUAL, _stream())
         _lib.check(rc, "flexsae_topk_bwd")
     return dW, dvals, dbias
+
+
+topk_bwd = torch.library.custom_op("flexsae_amd::topk_bwd", mutates_args=())(_topk_bwd_impl)
 
 
 def _bwd_fake(grad_out, indices, weight, vals, resid):
@@ -760,10 +764,9 @@ class _HierTrainStaged(torch.autograd.Function):
         return None, dW, (dvals * g).to(vdt), (dbias * g).to(bdt), None
 
 
-@torch.library.custom_op("flexsae_amd::hier_train_sliced", mutates_args=())
-def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
-                      target: Tensor, need_dw: bool = True, hot: bool = False,
-                      dense: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
+def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
+                            target: Tensor, need_dw: bool = True, hot: bool = False,
+                            dense: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """Fused forward + reverse walk in column slices, each reduced right away (flat memory).
 
     Used when the contributions of a whole step do not fit the stage budget: the scratch is one
@@ -810,6 +813,9 @@ def hier_train_sliced(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tenso
     return loss, dvals, dbias, dW
 
 
+hier_train_sliced = torch.library.custom_op("flexsae_amd::hier_train_sliced", mutates_args=())(_hier_train_sliced_impl)
+
+
 def _unit_dw_dtype(weight_dtype):
     """dtype of the unit-gradient dW of the sliced step: the weight's, but fp32 for fp16 weights."""
     return torch.float32 if weight_dtype == torch.float16 else weight_dtype
@@ -824,9 +830,8 @@ def _(indices, weight, vals, bias, target, need_dw=True, hot=False, dense=False)
             else weight.new_empty((0, weight.shape[1]), dtype=dw_dtype))
 
 
-@torch.library.custom_op("flexsae_amd::hier_sgd_step", mutates_args=("weight",))
-def hier_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, target: Tensor,
-                  step: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+def _hier_sgd_step_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, target: Tensor,
+                        step: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
     """HierarchicalTopK training step with the plain-SGD decoder update fused in.
 
     ``weight[f] -= step * dL/dW[f]`` for every latent f that ``indices`` touches, in place (fp32
@@ -883,6 +888,9 @@ def hier_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, t
     return loss, dvals, dbias
 
 
+hier_sgd_step = torch.library.custom_op("flexsae_amd::hier_sgd_step", mutates_args=("weight",))(_hier_sgd_step_impl)
+
+
 @hier_sgd_step.register_fake
 def _(indices, weight, vals, bias, target, step):
     return (weight.new_empty((), dtype=torch.float32), vals.new_empty(vals.shape, dtype=torch.float32),
@@ -898,7 +906,11 @@ def hierarchical_sae_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bia
         if isinstance(grad_out, Tensor):
             step = (grad_out.detach().to(device=weight.device, dtype=torch.float32) * lr).reshape(())
         else:
-            step = torch.tensor(float(lr) * float(grad_out), dtype=torch.float32, device=weight.device)
+            # (a fill: a copy from host memory would wait for the work queued so far)
+            step = torch.full((), float(lr) * float(grad_out), dtype=torch.float32, device=weight.device)
+        if _plain_call(indices, weight, vals, bias, target):
+            torch.autograd.graph.increment_version(weight)  # what the op's schema says of its weight
+            return _hier_sgd_step_impl(indices, weight, vals.detach(), bias.detach(), target, step)
         return hier_sgd_step(indices, weight, vals.detach(), bias.detach(), target, step)
 
 
@@ -1020,32 +1032,148 @@ def _train_sliced_backward(ctx, grad_loss, grad_dvals, grad_dbias, grad_dw):
 hier_train_sliced.register_autograd(_train_sliced_backward, setup_context=_train_sliced_setup_context)
 
 
-def _hier_backward(ctx, grad_loss, grad_resid):
+def _leaf_grads(weight, dvals, vals_dtype, dbias, bias_dtype, plain):
+    """dvals and dbias in the leaves' types: one launch for both in an ordinary eager call."""
+    if plain and (vals_dtype != torch.float32 or bias_dtype != torch.float32):
+        return _finish_grads(None, weight, None, dvals, vals_dtype, dbias, bias_dtype)[1:]
+    return dvals.to(vals_dtype), dbias.to(bias_dtype)
+
+
+def _hier_backward(ctx, grad_loss, grad_resid, impl=None):
     indices, weight, vals, resid = ctx.saved_tensors
     if grad_loss is None:
         return None, None, None, None, None
-    dW, dvals, dbias = hier_bwd(grad_loss, indices, weight, vals, resid)
+    dW, dvals, dbias = (impl or hier_bwd)(grad_loss, indices, weight, vals, resid)
     vdt, bdt, _ = ctx.leaf_dtypes
     # no gradient for target on this path (reference hierarchical_kernels.py:299)
-    return None, dW, dvals.to(vdt), dbias.to(bdt), None
+    return None, dW, *_leaf_grads(weight, dvals, vdt, dbias, bdt, impl is not None), None
 
 
-def _topk_backward(ctx, grad_loss, grad_resid):
+def _topk_backward(ctx, grad_loss, grad_resid, impl=None):
     indices, weight, vals, resid = ctx.saved_tensors
     if grad_loss is None:
         return None, None, None, None, None
-    dW, dvals, dbias = topk_bwd(grad_loss, indices, weight, vals, resid)
+    dW, dvals, dbias = (impl or topk_bwd)(grad_loss, indices, weight, vals, resid)
     vdt, bdt, tdt = ctx.leaf_dtypes
+    dvals, dbias = _leaf_grads(weight, dvals, vdt, dbias, bdt, impl is not None)
     dtarget = None
     if ctx.needs_input_grad[4]:
         # the reference's eager loss tail is differentiable w.r.t. target (topk_kernels.py:221)
         B, D = resid.shape
         dtarget = (resid * (grad_loss.to(torch.float32) * (-2.0 / (B * D)))).to(tdt)
-    return None, dW, dvals.to(vdt), dbias.to(bdt), dtarget
+    return None, dW, dvals, dbias, dtarget
 
 
 hier_fwd.register_autograd(_hier_backward, setup_context=_setup_context)
 topk_fwd.register_autograd(_topk_backward, setup_context=_setup_context)
+
+
+# ---- ordinary eager calls ------------------------------------------------------------------
+# A call on plain tensors with no tracer, mode or transform around it does without the dispatcher: the same functions as the
+# ops run, under an autograd.Function that saves the same tensors.  The wrappers of torch.library.custom_op around forward
+# and backward cost as much as the launches of a small step (us a step with them and without: B = 64, K = 32, F = 4096,
+# D = 256 fp32 TopK 197, 168, hierarchical 233, 188, of which about 70 are the hand-over to autograd's device thread;
+# B = 1024, K = 64, F = 32768, D = 1024 bf16 Zipf, SGD step 179, 127).  Everything else goes through the ops, which tracers,
+# modes and transforms see.
+_PLAIN_TYPES = (Tensor, torch.nn.Parameter)
+_C = torch._C
+_can_tell_plain = (all(hasattr(_C, n) for n in ("_len_torch_dispatch_stack", "_len_torch_function_stack", "_get_tracing_state"))
+                   and hasattr(getattr(_C, "_functorch", None), "peek_interpreter_stack")
+                   and hasattr(torch.autograd.forward_ad, "_current_level"))
+
+
+def _plain_call(*tensors: Tensor) -> bool:
+    """Ordinary tensors on the GPU, and nothing around the call that would have to see the ops."""
+    if torch.compiler.is_compiling() or not _can_tell_plain:
+        return False
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+            return False
+    return (_C._len_torch_dispatch_stack() == 0 and _C._len_torch_function_stack() == 0
+            and _C._functorch.peek_interpreter_stack() is None and _C._get_tracing_state() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
+
+def _finish_grads(grad_out, weight: Tensor, dW_unit, dvals: Tensor, vals_dtype, dbias: Tensor, bias_dtype):
+    """(dW, dvals, dbias) of a backward in the leaves' types, in one launch: the fp32 dvals and dbias times ``grad_out``
+    (None: one), and ``dW_unit`` (None: no weight gradient) times it, in place where it has the weight's type."""
+    lib = _lib.load()
+    dev = weight.device
+    with _on_device(dev):
+        g = None if grad_out is None else _grad_scalar(grad_out, dev)
+        dW = None
+        if dW_unit is not None:
+            dW = dW_unit if dW_unit.dtype == weight.dtype else torch.empty(dW_unit.shape, dtype=weight.dtype, device=dev)
+        out_v = torch.empty(dvals.shape, dtype=vals_dtype, device=dev)
+        out_b = torch.empty(dbias.shape, dtype=bias_dtype, device=dev)
+        unit_dtype = _DTYPES[weight.dtype] if dW_unit is None else _DTYPES[dW_unit.dtype]
+        rc = lib.flexsae_finish_grads(
+            None if dW is None else _ptr(dW), _DTYPES[weight.dtype], None if dW is None else _ptr(dW_unit), unit_dtype,
+            0 if dW is None else dW.numel(), _ptr(out_v), _DTYPES[vals_dtype], _ptr(dvals), dvals.numel(), _ptr(out_b),
+            _DTYPES[bias_dtype], _ptr(dbias), dbias.numel(), None if g is None else _ptr(g), _stream())
+        _lib.check(rc, "flexsae_finish_grads")
+    return dW, out_v, out_b
+
+
+class _TopkLoss(torch.autograd.Function):
+    """topk_fwd and its backward for ordinary eager calls."""
+
+    @staticmethod
+    def forward(ctx, indices, weight, vals, bias, target):
+        loss, resid = _forward("flexsae_topk_fwd", indices, weight, vals, bias, target)
+        _setup_context(ctx, (indices, weight, vals, bias, target), (loss, resid))
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_loss):
+        if grad_loss is None or torch.is_grad_enabled():  # (a graph of the backward is built by the ops)
+            return _topk_backward(ctx, grad_loss, None)
+        return _topk_backward(ctx, grad_loss, None, _topk_bwd_impl)
+
+
+class _HierLoss(torch.autograd.Function):
+    """hier_fwd and its backward for ordinary eager calls."""
+
+    @staticmethod
+    def forward(ctx, indices, weight, vals, bias, target):
+        loss, resid = _forward("flexsae_hier_fwd", indices, weight, vals, bias, target)
+        _setup_context(ctx, (indices, weight, vals, bias, target), (loss, resid))
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_loss):
+        if grad_loss is None or torch.is_grad_enabled():
+            return _hier_backward(ctx, grad_loss, None)
+        return _hier_backward(ctx, grad_loss, None, _hier_bwd_impl)
+
+
+class _HierTrainSliced(torch.autograd.Function):
+    """hier_train_sliced and its backward for ordinary eager calls."""
+
+    @staticmethod
+    def forward(ctx, indices, weight, vals, bias, target, need_dw, hot, dense):
+        loss, dvals, dbias, dW = _hier_train_sliced_impl(indices, weight, vals, bias, target, need_dw, hot, dense)
+        ctx.need_dw, ctx.hot, ctx.dense = need_dw, hot, dense
+        ctx.leaf_dtypes = (vals.dtype, bias.dtype)
+        ctx.set_materialize_grads(False)
+        ctx.dw_in_place = True
+        ctx.save_for_backward(indices, weight, vals, bias, target, dvals, dbias)
+        ctx.dw_unit = dW if ctx.needs_input_grad[1] else None
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_loss):
+        if grad_loss is None or torch.is_grad_enabled():
+            return _train_sliced_backward(ctx, grad_loss, None, None, None)
+        indices, weight, vals, bias, target, dvals, dbias = ctx.saved_tensors
+        dW = None
+        if ctx.needs_input_grad[1]:
+            dW = ctx.dw_unit
+            ctx.dw_unit = None  # the buffer now belongs to whoever receives the gradient
+            if dW is None:  # a second backward through a retained graph: the buffer went with the first one
+                _, dvals, dbias, dW = _hier_train_sliced_impl(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense)
+        dW, dvals, dbias = _finish_grads(grad_loss, weight, dW, dvals, ctx.leaf_dtypes[0], dbias, ctx.leaf_dtypes[1])
+        return None, dW, dvals, dbias, None, None, None, None
 
 
 def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
@@ -1072,7 +1200,13 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
                                                                    _is_traced(weight))
             dense = bool(weight.requires_grad) and _use_dense_latents(B, K, F, D, weight.dtype, weight.device,
                                                                        _is_traced(weight))
+            if _plain_call(indices, weight, vals, bias, target):
+                return _HierTrainSliced.apply(indices, weight, vals, bias, target, bool(weight.requires_grad), hot, dense)
             return hier_train_sliced(indices, weight, vals, bias, target, bool(weight.requires_grad), hot, dense)[0]
+    if _plain_call(indices, weight, vals, bias, target):
+        if needs_grad or (torch.is_grad_enabled() and target.requires_grad):
+            return _HierLoss.apply(indices, weight, vals, bias, target)
+        return _forward("flexsae_hier_fwd", indices, weight, vals, bias, target)[0]
     return hier_fwd(indices, weight, vals, bias, target)[0]
 
 
@@ -1084,4 +1218,8 @@ def triton_topk_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Te
     (torch-ext/flex_sae/topk_kernels.py:213-223); the kernels underneath are HIP."""
     if indices.dtype == torch.int32:
         indices = indices.to(torch.int64)
+    if _plain_call(indices, weight, vals, bias, target):
+        if torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad or target.requires_grad):
+            return _TopkLoss.apply(indices, weight, vals, bias, target)
+        return _forward("flexsae_topk_fwd", indices, weight, vals, bias, target)[0]
     return topk_fwd(indices, weight, vals, bias, target)[0]

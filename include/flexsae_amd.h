@@ -423,6 +423,17 @@ int flexsae_cast_from_f32(void *dst, int dst_dtype, const float *src, int64_t n,
 int flexsae_scale_from_f32(void *dst, int dst_dtype, const float *src, int64_t n, const float *scale,
                            void *stream);
 
+/*
+ * The end of a step's backward in one launch: dvals and dbias = their fp32 values * scale[0], rounded to the leaves' types;
+ * dW = dW_unit * scale[0], rounded once (dW_unit of dW's type, in place if it is dW itself, or fp32).  scale: a device
+ * fp32 scalar, NULL = 1.  A count of zero leaves that output out (its pointers may be NULL).  Vectors of four elements
+ * are read and written: every pointer aligned to four of its elements.
+ * replaces: the mul_(grad) passes and the engine's casts to the leaf dtypes (hierarchical_kernels.py:294-299).
+ */
+int flexsae_finish_grads(void *dW, int dW_dtype, const void *dW_unit, int dW_unit_dtype, int64_t n_dw, void *dvals,
+                         int dvals_dtype, const float *dvals_unit, int64_t n_dvals, void *dbias, int dbias_dtype,
+                         const float *dbias_unit, int64_t n_dbias, const float *scale, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,124 @@
+"""Ordinary eager calls go past the dispatcher: the same bits as through the ops, and the ops wherever something has to see
+them (modes, transforms, a graph of the backward)."""
+import ctypes
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+import flexsae_amd as flex
+from flexsae_amd import _lib, ops
+from tests import abi
+from tests.helpers import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+LOSS = {"hier": flex.triton_hierarchical_sae_loss, "topk": flex.triton_topk_sae_loss}
+
+
+class _Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.ops = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.ops.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def _step(loss, args, upstream, needs=(True, True, True), seen=None):
+    idx, W, v, b, t = args
+    leaves = [x.clone().requires_grad_(n) for x, n in zip((W, v, b), needs)]
+    out = LOSS[loss](idx, *leaves, t)
+    (out * upstream).backward()
+    return [out.detach()] + [x.grad for x in leaves]
+
+
+@pytest.mark.parametrize("loss,fused", [("topk", True), ("hier", True), ("hier", False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("B,K,F,D", [(7, 9, 40, 132), (64, 32, 300, 256), (5, 3, 11, 35)])
+def test_same_bits_as_through_the_ops(loss, fused, dtype, B, K, F, D):
+    print("[case]", loss, fused, dtype, B, K, F, D, flush=True)
+    args = [x.to(DEV) for x in make_inputs(B, K, F, D, dtype, seed=B + D)]
+    flex.set_fused_training(fused)
+    try:
+        for upstream in (1.0, 3.25):
+            for needs in ((True, True, True), (False, True, True), (True, False, False)):
+                with _Seen() as seen:
+                    want = _step(loss, args, upstream, needs)
+                assert any("flexsae_amd" in o for o in seen.ops)
+                got = _step(loss, args, upstream, needs)
+                for x, y in zip(got, want):
+                    assert (x is None and y is None) or torch.equal(x, y)
+        with torch.no_grad():
+            quiet = LOSS[loss](*args)
+            with _Seen() as seen:
+                assert torch.equal(quiet, LOSS[loss](*args))
+            assert any("flexsae_amd" in o for o in seen.ops) and not quiet.requires_grad
+    finally:
+        flex.set_fused_training(True)
+
+
+@pytest.mark.parametrize("loss", ["topk", "hier"])
+def test_graphs_hooks_and_transforms(loss):
+    args = [x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=4)]
+    idx, W, v, b, t = args
+    want = _step(loss, args, 2.0)
+    # twice through a retained graph, and with a graph of the backward
+    leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+    out = LOSS[loss](idx, *leaves, t) * 2.0
+    for kw in ({"retain_graph": True}, {"retain_graph": True}, {"create_graph": True}):
+        for x, y in zip(torch.autograd.grad(out, leaves, **kw), want[1:]):
+            assert torch.equal(x.detach(), y)
+    # what is saved passes the hooks: as many tensors as the op saves, and the gradients are those of what they give back
+    counts = []
+    for mode in (None, _Seen()):
+        packed = []
+        leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: packed.append(1) or x.cpu(), lambda x: x.to(DEV)):
+            if mode is None:
+                out = LOSS[loss](idx, *leaves, t)
+            else:
+                with mode:
+                    out = LOSS[loss](idx, *leaves, t)
+        (out * 2.0).backward()
+        counts.append(len(packed))
+        for x, y in zip(leaves, want[1:]):
+            assert torch.equal(x.grad, y)
+    assert counts[0] == counts[1]
+    # a weight changed between forward and backward is refused
+    leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+    out = LOSS[loss](idx, *leaves, t)
+    with torch.no_grad():
+        leaves[0].add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward()
+    # functional transforms are the ops' business, which refuse them
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.grad(lambda w: LOSS[loss](idx, w, v, b, t) * 2.0)(W)
+
+
+def test_the_fused_update_marks_the_weight():
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=4))
+    W2 = W.clone()
+    before = W._version
+    got = flex.hierarchical_sae_sgd_step(idx, W, v, b, t, 0.5)
+    assert W._version > before
+    with _Seen():
+        want = flex.hierarchical_sae_sgd_step(idx, W2, v, b, t, 0.5)
+    assert torch.equal(W, W2) and all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_finish_grads_checks_its_arguments():
+    fn = _lib.load().flexsae_finish_grads
+    x = torch.zeros(64, device=DEV)
+    p = abi.ptr(x)
+    odd = ctypes.c_void_p(x.data_ptr() + 4)
+    none = ctypes.c_void_p(0)
+    assert fn(none, 0, none, 0, 0, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == 0
+    assert fn(none, 0, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT
+    assert fn(p, 1, p, 2, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT
+    assert fn(p, 1, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT  # in place
+    assert fn(odd, 0, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_ALIGNMENT
+    assert fn(p, 7, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT
