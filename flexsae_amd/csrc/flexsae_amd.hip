@@ -50,6 +50,7 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr size_t kAlign = 256;
 constexpr int kBwdSgdUpdate = 1 << 20;  // internal flag of the slice loop: dW is the weight matrix, updated in place
 constexpr int kBwdSolo = 1 << 22;       // internal flag of the slice loop: slot[] marks the only pairs of their latents
+constexpr int kBwdScaled = 1 << 23;  // internal flag of the slice loop: dW is multiplied by grad_out[0] before it is rounded
 constexpr int kBwdHot = 1 << 21;        // internal flag of the slice loop: hot latents are accumulated in the LDS
 constexpr unsigned kLongBlocks = 1024;    // leading blocks of a reduction launch that serve hot latents
 constexpr int64_t kListBlocks = 8192;     // blocks of a reduction launch that work from the lists of latents
@@ -893,7 +894,7 @@ void launch_seg_reduce(bool narrow, const uint32_t *begin, const LongList &ll, c
   // the second step of the hot latents: launched here, or handed back through `defer` for the next
   // training-step launch to carry
   auto finalize = [&](int mode, int units) {
-    HotFinalize h = {ll.ctrl, ll.list, ll.chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, dwords, 256u};
+    HotFinalize h = {ll.ctrl, ll.list, ll.chunk_begin, partial, dW, dw_scale, mode, units, col0, sw, D, update, dwords, 0, 256u};
     if (defer) {
       h.n_blocks = 64u;  // riding along with a long launch: few blocks, so that they cost little where there is nothing to do
       *defer = h;
@@ -963,7 +964,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   const bool do_reduce = !(flags & FLEXSAE_BWD_SWEEP_ONLY);
   // in-place weight update: `grad_out` is the step size and dW the weight matrix (piece reduction only)
   const int update = (flags & kBwdSgdUpdate) ? 1 : 0;
-  const float *dw_scale = (flags & (FLEXSAE_BWD_SCALE_BY_GRAD_OUT | kBwdSgdUpdate)) ? grad_out : nullptr;
+  const float *dw_scale = (flags & (FLEXSAE_BWD_SCALE_BY_GRAD_OUT | kBwdSgdUpdate | kBwdScaled)) ? grad_out : nullptr;
   const uint32_t *begin = reinterpret_cast<const uint32_t *>(ws + pl.off_begin);
   const uint32_t *slot = reinterpret_cast<const uint32_t *>(ws + pl.off_slot);
   const CsrScratch sc = carve_hier_lists(s, pl, ws);
@@ -1011,13 +1012,14 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     hipLaunchKernelGGL((seg_zero_rows_kernel<GT>), dim3(static_cast<unsigned>(ceil_div(s->F, kZeroRows * kWavesPerBlock))), dim3(kBlock), 0, st, sc.lists.ctrl,
                        sc.lists.empty_list, dW, D, rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t)));
   // In the training step the second step of a slice's hot latents travels with the next slice's
-  // training-step launch (a gradient of CarriedGrad's type or the in-place update only: that is what that kernel
+  // training-step launch (a gradient of CarriedGrad's type; by pieces, the weight's: that is what that kernel
   // writes; a launch of its own costs 4.7 us a slice); the last slice's gets one.
   HotFinalize pending = {};
   HotBlockFinalize pending_hot = {};
   // (the sweep of the plain backward carries it for a gradient of the weight's type)
-  const bool fold = (train && !update ? std::is_same<GT, typename CarriedGrad<WT>::type>::value : std::is_same<GT, WT>::value) &&
-                    do_sweep && do_reduce;
+  constexpr bool carried = std::is_same<GT, typename CarriedGrad<WT>::type>::value;
+  constexpr bool weight_typed = std::is_same<GT, WT>::value && !carried;
+  const bool fold = (train && !update ? carried || weight_typed : std::is_same<GT, WT>::value) && do_sweep && do_reduce;
   // Only pairs of their latents write dW themselves where its type is the contributions' own.
   void *const dW_solo = (flags & kBwdSolo) && std::is_same<GT, PT>::value && train != nullptr && do_sweep && do_reduce &&
                                 !update && !dw_scale
@@ -1071,13 +1073,14 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
         piece != 0 && (update || pl.vec < 4 || cols % pl.tile != 0 || sparse_latents(s, flags) || cache_sized);
     launch_seg_reduce<PT, GT, VEC>(narrow_reduce, begin, reduce_long, sc.lists, P, partial, dW, dw_scale, s->F, tps,
                                    static_cast<int>(col0), sw, D, st, by_pieces ? piece : 0, cols, s->B * s->K, update,
-                                   sparse, fold ? &pending : nullptr, dW_solo != nullptr);
+                                   sparse, fold && (!train || carried || by_pieces) ? &pending : nullptr, dW_solo != nullptr);
+    pending.weight_typed = weight_typed;
     if (hot) {
       // the block partials of the slice's hot latents are added up by the next training-step launch
       // (they live in the buffer that launch does not write), or here
       const HotBlockFinalize h = {hot_ctrl, hot_list, hot_partial[slice_no & 1], dW, dw_scale,
                                   static_cast<int>(cols / kHotCols), static_cast<int>(pl.n_row_blocks),
-                                  static_cast<int>(col0), D, update};
+                                  static_cast<int>(col0), D, update, weight_typed};
       if (fold)
         pending_hot = h;
       else
@@ -1594,13 +1597,13 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
                       const void *vals, const void *bias, const void *target, float *loss,
                       void *dW, int dW_dtype, float *dvals, float *dbias, void *workspace,
                       size_t workspace_bytes, int flags, int *status_flag, void *stream,
-                      const float *sgd_step) {
+                      const float *sgd_step, const float *dw_scale = nullptr) {
   int rc = check_shape(s);
   if (rc != FLEXSAE_OK) return rc;
-  if (sgd_step) {
+  if (sgd_step || dw_scale) {
     if (flags & (FLEXSAE_BWD_NO_DW | FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE))
       return FLEXSAE_ERR_INVALID_ARGUMENT;
-    if (!aligned(sgd_step, 4)) return FLEXSAE_ERR_ALIGNMENT;
+    if (!aligned(sgd_step, 4) || !aligned(dw_scale, 4)) return FLEXSAE_ERR_ALIGNMENT;
   }
   const bool no_dw = (flags & FLEXSAE_BWD_NO_DW) != 0;
   const bool defer_reduce = (flags & FLEXSAE_BWD_SWEEP_ONLY) != 0 && !no_dw;
@@ -1652,12 +1655,12 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
                         1.0 / count};
   // without dW the reductions are left out like in the deferred case (dW_dtype only selects a template then)
   const auto slices = pl.vec == 4 ? launch_hier_slices_w<4> : pl.vec == 2 ? launch_hier_slices_w<2> : launch_hier_slices_w<1>;
-  slices(s, pl, slice_w, indices, weight, vals, nullptr, sgd_step, coef, dW,
+  slices(s, pl, slice_w, indices, weight, vals, nullptr, sgd_step ? sgd_step : dw_scale, coef, dW,
          no_dw ? s->weight_dtype : dW_dtype, dvals, dbias, ws,
          (flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE |
                    FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS)) |
-             (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : 0) | (hot ? kBwdHot : 0) |
-             (solo ? kBwdSolo : 0),
+             (no_dw ? FLEXSAE_BWD_SWEEP_ONLY : 0) | (sgd_step ? kBwdSgdUpdate : dw_scale ? kBwdScaled : 0) |
+             (hot ? kBwdHot : 0) | (solo ? kBwdSolo : 0),
          status_flag, st, &ta, piece ? static_cast<int>(piece_cols(pl)) : 0);
   return launch_status();
 }
@@ -1671,7 +1674,17 @@ int flexsae_hier_fwd_bwd(const flexsae_shape *s, const int64_t *indices, const v
                          void *dW, int dW_dtype, float *dvals, float *dbias, void *workspace,
                          size_t workspace_bytes, int flags, int *status_flag, void *stream) {
   return hier_fwd_bwd_impl(s, indices, weight, vals, bias, target, loss, dW, dW_dtype, dvals, dbias, workspace,
-                           workspace_bytes, flags & ~(kBwdSgdUpdate | kBwdHot | kBwdSolo), status_flag, stream, nullptr);
+                           workspace_bytes, flags & ~(kBwdSgdUpdate | kBwdHot | kBwdSolo | kBwdScaled), status_flag, stream, nullptr);
+}
+
+int flexsae_hier_fwd_bwd_scaled(const flexsae_shape *s, const int64_t *indices, const void *weight, const void *vals,
+                                const void *bias, const void *target, const float *grad_out, float *loss, void *dW,
+                                int dW_dtype, float *dvals, float *dbias, void *workspace, size_t workspace_bytes,
+                                int flags, int *status_flag, void *stream) {
+  if (!grad_out) return FLEXSAE_ERR_INVALID_ARGUMENT;
+  return hier_fwd_bwd_impl(s, indices, weight, vals, bias, target, loss, dW, dW_dtype, dvals, dbias, workspace,
+                           workspace_bytes, flags & ~(kBwdSgdUpdate | kBwdHot | kBwdSolo | kBwdScaled), status_flag, stream,
+                           nullptr, grad_out);
 }
 
 int flexsae_hier_sgd_step(const flexsae_shape *s, const int64_t *indices, void *weight, const void *vals,

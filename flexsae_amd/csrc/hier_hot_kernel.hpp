@@ -240,6 +240,7 @@ struct HotBlockFinalize {
   void *out;
   const float *scale;
   int n_tiles, n_row_blocks, col0, D, update;
+  int weight_typed;  // as in HotFinalize
 };
 
 template <typename GT>
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
   // this block's share of the previous slice's second steps
   hot_finalize_carried<WT>(fin, blockIdx.x);
   if constexpr (!std::is_same<WT, typename CarriedGrad<WT>::type>::value) {
-    if (hfin.update) hot_block_finalize_run<WT>(hfin, blockIdx.x, gridDim.x);
+    if (hfin.weight_typed) hot_block_finalize_run<WT>(hfin, blockIdx.x, gridDim.x);
     else hot_block_finalize_run<typename CarriedGrad<WT>::type>(hfin, blockIdx.x, gridDim.x);
   } else {
     hot_block_finalize_run<WT>(hfin, blockIdx.x, gridDim.x);

@@ -530,6 +530,7 @@ struct HotFinalize {
   int units;  // pieces or tiles per slice
   int col0, slice_w, D, update;
   int dwords;  // rows of `out` start at multiples of four bytes (mode 1)
+  int weight_typed;  // `out` has the weight's type where CarriedGrad's is another (mode 1; so it does with update)
   unsigned n_blocks;  // blocks of 256 threads that share it
 };
 
@@ -546,8 +547,9 @@ __device__ __forceinline__ void hot_finalize_run(const HotFinalize &h, unsigned 
                                      h.col0, h.slice_w, h.D, block, h.n_blocks);
 }
 
-// Gradient type of the finalize work that a training-step launch carries: the type the package asks for, the
-// weight's own, or fp32 for fp16 weights (whose unit gradient would underflow).  The in-place update writes the weights.
+// Gradient type of the finalize work that a training-step launch carries: the weight's own, or fp32 for fp16 weights (whose
+// unit gradient would underflow); by pieces also the weight's type there: the in-place update, and a gradient that is
+// scaled before its only rounding.
 template <typename WT>
 struct CarriedGrad {
   using type = WT;
@@ -560,11 +562,10 @@ struct CarriedGrad<f16_t> {
 template <typename WT>
 __device__ __forceinline__ void hot_finalize_carried(const HotFinalize &h, unsigned block) {
   if constexpr (!std::is_same<WT, typename CarriedGrad<WT>::type>::value) {
-    if (h.update) {
-      // (by pieces, the only reduction that updates in place)
+    if (h.weight_typed) {
       if (h.mode == 1)
         seg_piece_finalize_body<WT>(h.long_ctrl, h.long_list, h.chunk_begin, h.partial, h.out, h.scale, h.units, h.col0,
-                                    h.slice_w, h.D, 1, h.dwords, block, h.n_blocks);
+                                    h.slice_w, h.D, h.update, h.dwords, block, h.n_blocks);
       return;
     }
   }

@@ -764,17 +764,9 @@ class _HierTrainStaged(torch.autograd.Function):
         return None, dW, (dvals * g).to(vdt), (dbias * g).to(bdt), None
 
 
-def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
-                            target: Tensor, need_dw: bool = True, hot: bool = False,
-                            dense: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
-    """Fused forward + reverse walk in column slices, each reduced right away (flat memory).
-
-    Used when the contributions of a whole step do not fit the stage budget: the scratch is one
-    slice of them (``set_hier_scratch_bytes``), and every slice gathers its weight-row pieces once
-    for both walks.  Returns (loss, dvals, dbias, dW), the gradients for a unit upstream gradient;
-    the backward scales them.  With ``need_dw`` false (a decoder whose weight takes no gradient)
-    the segment reductions are left out and the returned dW is empty.  ``hot`` and ``dense`` are the
-    library's FLEXSAE_BWD_HOT_LATENTS and FLEXSAE_BWD_DENSE_LATENTS hints."""
+def _hier_sliced_step(indices, weight, vals, bias, target, need_dw, hot, dense, grad_out=None):
+    """The step of ``hier_train_sliced``; with ``grad_out`` (then need_dw) dW is the gradient for that upstream gradient
+    in the weight's type, loss, dvals and dbias as without."""
     B, K, F, D = _validate(indices, weight, vals, bias, target)
     lib = _lib.load()
     indices, weight, vals, bias, target = (_prep(t) for t in (indices, weight, vals, bias, target))
@@ -789,7 +781,7 @@ def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias:
         ws_bytes = lib.flexsae_hier_fwd_bwd_workspace_bytes_flags(ctypes.byref(shape), slice_cols, hot_flag | ragged)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)
-        dw_dtype = _unit_dw_dtype(weight.dtype)
+        dw_dtype = _unit_dw_dtype(weight.dtype) if grad_out is None else weight.dtype
         dW = torch.empty((F, D), dtype=dw_dtype, device=dev) if need_dw else weight.new_empty((0, D), dtype=dw_dtype)
         dvals = torch.empty((B, K), dtype=torch.float32, device=dev)
         dbias = torch.empty((D,), dtype=torch.float32, device=dev)
@@ -799,10 +791,16 @@ def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias:
             _pair_import(lib, shape, workspace, cached)
         flags = ((_lib.BWD_REUSE_PAIR_LIST if cached is not None else 0) | (0 if need_dw else _lib.BWD_NO_DW) |
                  hot_flag | (_lib.BWD_DENSE_LATENTS if dense else 0) | ragged)
-        rc = lib.flexsae_hier_fwd_bwd(ctypes.byref(shape), _ptr(indices), _ptr(weight), _ptr(vals), _ptr(bias),
-                                      _ptr(target), _ptr(loss), _ptr(dW) if need_dw else None,
-                                      _DTYPES[dw_dtype], _ptr(dvals),
-                                      _ptr(dbias), _ptr(workspace), ws_bytes, flags, _ptr(flag), _stream())
+        if grad_out is None:
+            rc = lib.flexsae_hier_fwd_bwd(ctypes.byref(shape), _ptr(indices), _ptr(weight), _ptr(vals), _ptr(bias),
+                                          _ptr(target), _ptr(loss), _ptr(dW) if need_dw else None,
+                                          _DTYPES[dw_dtype], _ptr(dvals),
+                                          _ptr(dbias), _ptr(workspace), ws_bytes, flags, _ptr(flag), _stream())
+        else:
+            g = _grad_scalar(grad_out, dev)
+            rc = lib.flexsae_hier_fwd_bwd_scaled(ctypes.byref(shape), _ptr(indices), _ptr(weight), _ptr(vals), _ptr(bias),
+                                                 _ptr(target), _ptr(g), _ptr(loss), _ptr(dW), _DTYPES[dw_dtype], _ptr(dvals),
+                                                 _ptr(dbias), _ptr(workspace), ws_bytes, flags, _ptr(flag), _stream())
         _lib.check(rc, "flexsae_hier_fwd_bwd")
         if cached is None:
             _pair_export(lib, shape, workspace, indices, F)
@@ -811,6 +809,20 @@ def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias:
         if _check_indices:
             check_index_flag(dev)
     return loss, dvals, dbias, dW
+
+
+def _hier_train_sliced_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
+                            target: Tensor, need_dw: bool = True, hot: bool = False,
+                            dense: bool = False) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
+    """Fused forward + reverse walk in column slices, each reduced right away (flat memory).
+
+    Used when the contributions of a whole step do not fit the stage budget: the scratch is one
+    slice of them (``set_hier_scratch_bytes``), and every slice gathers its weight-row pieces once
+    for both walks.  Returns (loss, dvals, dbias, dW), the gradients for a unit upstream gradient;
+    the backward scales them.  With ``need_dw`` false (a decoder whose weight takes no gradient)
+    the segment reductions are left out and the returned dW is empty.  ``hot`` and ``dense`` are the
+    library's FLEXSAE_BWD_HOT_LATENTS and FLEXSAE_BWD_DENSE_LATENTS hints."""
+    return _hier_sliced_step(indices, weight, vals, bias, target, need_dw, hot, dense)
 
 
 hier_train_sliced = torch.library.custom_op("flexsae_amd::hier_train_sliced", mutates_args=())(_hier_train_sliced_impl)
@@ -1176,6 +1188,44 @@ class _HierTrainSliced(torch.autograd.Function):
         return None, dW, dvals, dbias, None, None, None, None
 
 
+def _late_step(weight: Tensor, B: int, K: int) -> bool:
+    """fp16 weights of few pairs per latent: loss alone in the forward, the step in the backward, where the upstream
+    gradient is known and dW is written once in fp16, instead of an fp32 unit gradient written, read back, scaled and
+    rounded.  A second gather (2*B*K*D bytes, partly out of the L2s) for 6*F*D bytes less: us with it / without, uniform
+    and Zipf indices, B = 4096, F = 65536, D = 2304: K = 16 469 / 538, 409 / 566; K = 32 723 / 765, 595 / 697; K = 64
+    1252 / 1284, 1059 / 1081; K = 128 2369 / 2279; B = 8192, K = 64, F = 262144, D = 4096 4878 / 5786, 3526 / 4518; B = 256,
+    K = 64, F = 65536, D = 2048 171 / 332.  Not below 16 million weights, where two launches more show (F = 16384, D = 512
+    161 / 148; F = 32768, D = 1024 182 / 202)."""
+    F, D = weight.shape
+    return weight.dtype == torch.float16 and B * K <= 4 * F and F * D >= 1 << 24
+
+
+class _HierLateStep(torch.autograd.Function):
+    """The loss in the forward, ``_hier_sliced_step`` with the upstream gradient in the backward (``_late_step``)."""
+
+    @staticmethod
+    def forward(ctx, indices, weight, vals, bias, target, hot, dense):
+        loss, _ = _forward("flexsae_hier_fwd", indices, weight, vals, bias, target)
+        ctx.hot, ctx.dense = hot, dense
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(indices, weight, vals, bias, target)
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_loss):
+        if grad_loss is None:
+            return None, None, None, None, None, None, None
+        indices, weight, vals, bias, target = ctx.saved_tensors
+        if torch.is_grad_enabled():  # (a graph of the backward is built by the ops)
+            with torch.no_grad():
+                _, dvals, dbias, dW = hier_train_sliced(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense)
+            g = grad_loss.to(torch.float32)
+            return None, scale_to(dW, g, weight.dtype), (dvals * g).to(vals.dtype), (dbias * g).to(bias.dtype), None, None, None
+        _, dvals, dbias, dW = _hier_sliced_step(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense, grad_loss)
+        _, dvals, dbias = _finish_grads(grad_loss, weight, None, dvals, vals.dtype, dbias, bias.dtype)
+        return None, dW, dvals, dbias, None, None, None
+
+
 def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
                                  target: Tensor) -> Tensor:
     """Fused HierarchicalTopK decoder loss (0-dim fp32), differentiable w.r.t. weight, vals, bias.
@@ -1201,6 +1251,8 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
             dense = bool(weight.requires_grad) and _use_dense_latents(B, K, F, D, weight.dtype, weight.device,
                                                                        _is_traced(weight))
             if _plain_call(indices, weight, vals, bias, target):
+                if weight.requires_grad and _late_step(weight, B, K):
+                    return _HierLateStep.apply(indices, weight, vals, bias, target, hot, dense)
                 return _HierTrainSliced.apply(indices, weight, vals, bias, target, bool(weight.requires_grad), hot, dense)
             return hier_train_sliced(indices, weight, vals, bias, target, bool(weight.requires_grad), hot, dense)[0]
     if _plain_call(indices, weight, vals, bias, target):

@@ -289,6 +289,17 @@ int flexsae_hier_fwd_bwd(const flexsae_shape *shape, const int64_t *indices, con
                          size_t workspace_bytes, int flags, int *status_flag, void *stream);
 
 /*
+ * flexsae_hier_fwd_bwd with dW multiplied by grad_out[0] (a device fp32 scalar) in fp32 before its only rounding, for
+ * callers that know the upstream gradient: a dW of 16 bits then is the gradient itself, where a unit gradient of fp16
+ * weights (2/(B*K*D) and below) needs 32.  loss, dvals and dbias are those of a unit upstream gradient.  Flags as there,
+ * without NO_DW, SWEEP_ONLY, REDUCE_ONLY and SKIP_EPILOGUE (FLEXSAE_ERR_INVALID_ARGUMENT).
+ */
+int flexsae_hier_fwd_bwd_scaled(const flexsae_shape *shape, const int64_t *indices, const void *weight, const void *vals,
+                                const void *bias, const void *target, const float *grad_out, float *loss, void *dW,
+                                int dW_dtype, float *dvals, float *dbias, void *workspace, size_t workspace_bytes,
+                                int flags, int *status_flag, void *stream);
+
+/*
  * HierarchicalTopK training step with the plain-SGD weight update fused in: the same pass as
  * flexsae_hier_fwd_bwd, but the segment reduction, instead of writing a dense dW[F,D], subtracts
  * step[0] * (unit-gradient row) from every weight row that the batch touches, in place, in the
