@@ -11,6 +11,7 @@
 #include "hier_bwd_kernels.hpp"
 #include "hier_train_kernel.hpp"
 #include "hier_hot_kernel.hpp"
+#include "hier_epilogue_kernel.hpp"
 #include "segment_kernels.hpp"
 #include "topk_bwd_kernels.hpp"
 
@@ -971,7 +972,6 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   float *s_final = reinterpret_cast<float *>(ws + pl.off_sfinal);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   float *colsum_part = reinterpret_cast<float *>(ws + pl.off_colsum);
-  const int n_chunks = static_cast<int>(ceil_div(s->B, kColsumRows));
   const int d_pad = static_cast<int>(pl.d_pad);
   const int K = static_cast<int>(s->K), D = static_cast<int>(s->D);
   const int sw = static_cast<int>(slice_w);
@@ -1087,32 +1087,37 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
         hipLaunchKernelGGL((hot_block_finalize_kernel<GT>), dim3(256), dim3(kBlock), 0, st, h);
     }
   }
-  if (pending.n_blocks != 0) {
-    pending.n_blocks = 256u;
-    hipLaunchKernelGGL((hot_finalize_kernel<GT>), dim3(pending.n_blocks), dim3(kBlock), 0, st, pending);
+  // What is left goes into one launch, unless this call ends with its reductions.
+  const bool with_epilogue = do_sweep && (do_reduce || train) && !(flags & FLEXSAE_BWD_SKIP_EPILOGUE);
+  if (!with_epilogue) {
+    if (pending.n_blocks != 0) {
+      pending.n_blocks = 256u;
+      hipLaunchKernelGGL((hot_finalize_kernel<GT>), dim3(pending.n_blocks), dim3(kBlock), 0, st, pending);
+    }
+    if (pending_hot.ctrl != nullptr)
+      hipLaunchKernelGGL((hot_block_finalize_kernel<GT>), dim3(256), dim3(kBlock), 0, st, pending_hot);
+    return;  // (with !do_reduce && !train a measurement aid of the plain backward: sweep kernels only)
   }
-  if (pending_hot.ctrl != nullptr)
-    hipLaunchKernelGGL((hot_block_finalize_kernel<GT>), dim3(256), dim3(kBlock), 0, st, pending_hot);
-  if (!do_sweep) return;
-  if (!do_reduce && !train) return;  // measurement aid of the plain backward: sweep kernels only
-  if (flags & FLEXSAE_BWD_SKIP_EPILOGUE) return;
-  // one launch: dvals = its per-tile shares added in tile order; stage 1 of dbias = column sums of
-  // s_final over the rows, in a fixed order; the loss of the training step from its partials
-  {
-    // (the hot-latent training step has formed stage 1 of the column sums on chip)
-    const unsigned n_colsum_blocks = hot ? 0u : static_cast<unsigned>(ceil_div(D, 256) * ceil_div(n_chunks, 4));
-    const unsigned n_dvals_blocks = grid_for(s->B * s->K, 1024, 2048);
-    hipLaunchKernelGGL(hier_epilogue_kernel, dim3(1 + n_colsum_blocks + n_dvals_blocks), dim3(1024), 0, st,
-                       train ? reinterpret_cast<const float *>(ws + pl.off_loss) : static_cast<const float *>(nullptr),
-                       train ? train->n_loss_partials : 0, train ? train->inv_count : 0.0,
-                       train ? train->loss : static_cast<float *>(nullptr), s_final, s->B,
-                       static_cast<int64_t>(d_pad), D, colsum_part, n_colsum_blocks, dv_part,
-                       static_cast<int>(d_used / (train ? train_tile_cols(s) : kWave * sweep_vec)), s->B * s->K, dvals);
-  }
-  // (one partial per row block of the hot-latent step, else per chunk of kColsumRows)
-  hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(D, 256))), dim3(256), 0, st,
-                     colsum_part, hot ? static_cast<int>(pl.n_row_blocks) : n_chunks, D,
-                     static_cast<const float *>(nullptr), 1.0f, dbias);
+  if (pending.n_blocks != 0) pending.n_blocks = 64u;  // of 1024 threads
+  const unsigned n_hot_blocks = pending_hot.ctrl != nullptr ? 64u : 0u;
+  // (the hot-latent training step has formed stage 1 of the column sums on chip, one partial per row block)
+  const int n_chunks = static_cast<int>(ceil_div(s->B, kColsumRows));
+  const bool two_launches = !hot && s->B > kEndRows;
+  const unsigned n_col_blocks =
+      hot ? static_cast<unsigned>(ceil_div(D, 1024))
+          : static_cast<unsigned>(two_launches ? ceil_div(D, 256) * ceil_div(n_chunks, 4) : ceil_div(D, 16 * kEndCols) * 16);
+  const unsigned n_dvals_blocks = grid_for(s->B * s->K, 1024, 2048);
+  hipLaunchKernelGGL((hier_epilogue_kernel<GT>), dim3(1 + pending.n_blocks + n_hot_blocks + n_col_blocks + n_dvals_blocks),
+                     dim3(1024), 0, st,
+                     train ? reinterpret_cast<const float *>(ws + pl.off_loss) : static_cast<const float *>(nullptr),
+                     train ? train->n_loss_partials : 0, train ? train->inv_count : 0.0,
+                     train ? train->loss : static_cast<float *>(nullptr), pending, pending_hot, n_hot_blocks,
+                     s_final, s->B, static_cast<int64_t>(d_pad), D, colsum_part,
+                     hot ? static_cast<int>(pl.n_row_blocks) : two_launches ? -1 : 0, dbias, n_col_blocks, dv_part,
+                     static_cast<int>(d_used / (train ? train_tile_cols(s) : kWave * sweep_vec)), s->B * s->K, dvals);
+  if (two_launches)
+    hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(D, 256))), dim3(256), 0, st, colsum_part,
+                       n_chunks, D, static_cast<const float *>(nullptr), 1.0f, dbias);
 }
 
 template <typename WT, typename PT, int VEC>

@@ -590,7 +590,7 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
       }
       // the row's final S (the gradient of its reconstruction) is only needed summed over the rows,
       // for dbias: summed here per wavefront in row order, the wavefronts' sums added in order at
-      // the end of the block, the blocks' sums in order by colsum_final_kernel -- a fixed order that
+      // the end of the block, the blocks' sums in order by hier_epilogue_kernel -- a fixed order that
       // does not depend on the slice width (a deferred row is walked twice with the same S: counted
       // in the first pass).  The plain step sums the same values in another fixed order (runs of 64
       // rows), so dbias may differ from its in the last bits.
