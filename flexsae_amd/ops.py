@@ -920,7 +920,7 @@ def hierarchical_sae_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bia
         else:
             # (a fill: a copy from host memory would wait for the work queued so far)
             step = torch.full((), float(lr) * float(grad_out), dtype=torch.float32, device=weight.device)
-        if _plain_call(indices, weight, vals, bias, target):
+        if _plain_call(indices, weight, vals, bias, target, step):
             torch.autograd.graph.increment_version(weight)  # what the op's schema says of its weight
             return _hier_sgd_step_impl(indices, weight, vals.detach(), bias.detach(), target, step)
         return hier_sgd_step(indices, weight, vals.detach(), bias.detach(), target, step)
@@ -1090,20 +1090,29 @@ topk_fwd.register_autograd(_topk_backward, setup_context=_setup_context)
 _PLAIN_TYPES = (Tensor, torch.nn.Parameter)
 _C = torch._C
 _can_tell_plain = (all(hasattr(_C, n) for n in ("_len_torch_dispatch_stack", "_len_torch_function_stack", "_get_tracing_state"))
-                   and hasattr(getattr(_C, "_functorch", None), "peek_interpreter_stack")
+                   and all(hasattr(getattr(_C, "_functorch", None), n)
+                           for n in ("peek_interpreter_stack", "is_functorch_wrapped_tensor", "is_legacy_batchedtensor"))
                    and hasattr(torch.autograd.forward_ad, "_current_level"))
 
 
 def _plain_call(*tensors: Tensor) -> bool:
-    """Ordinary tensors on the GPU, and nothing around the call that would have to see the ops."""
+    """Ordinary tensors on the GPU, and nothing around the call that would have to see the ops.  (The tensors of
+    ``torch.autograd.grad(..., is_grads_batched=True)`` are of type Tensor and have no memory of their own.)"""
     if torch.compiler.is_compiling() or not _can_tell_plain:
         return False
     for t in tensors:
-        if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+        if (type(t) not in _PLAIN_TYPES or not t.is_cuda or _C._functorch.is_legacy_batchedtensor(t)
+                or _C._functorch.is_functorch_wrapped_tensor(t)):
             return False
     return (_C._len_torch_dispatch_stack() == 0 and _C._len_torch_function_stack() == 0
             and _C._functorch.peek_interpreter_stack() is None and _C._get_tracing_state() is None
             and torch.autograd.forward_ad._current_level < 0)
+
+
+def _plain_backward(grad_loss: Tensor) -> bool:
+    """The same of a backward, whose surroundings and gradient need not be those of its forward; the ops build a graph of
+    the backward."""
+    return not torch.is_grad_enabled() and _plain_call(grad_loss)
 
 
 def _finish_grads(grad_out, weight: Tensor, dW_unit, dvals: Tensor, vals_dtype, dbias: Tensor, bias_dtype):
@@ -1138,7 +1147,7 @@ class _TopkLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_loss):
-        if grad_loss is None or torch.is_grad_enabled():  # (a graph of the backward is built by the ops)
+        if grad_loss is None or not _plain_backward(grad_loss):
             return _topk_backward(ctx, grad_loss, None)
         return _topk_backward(ctx, grad_loss, None, _topk_bwd_impl)
 
@@ -1154,7 +1163,7 @@ class _HierLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_loss):
-        if grad_loss is None or torch.is_grad_enabled():
+        if grad_loss is None or not _plain_backward(grad_loss):
             return _hier_backward(ctx, grad_loss, None)
         return _hier_backward(ctx, grad_loss, None, _hier_bwd_impl)
 
@@ -1175,7 +1184,7 @@ class _HierTrainSliced(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_loss):
-        if grad_loss is None or torch.is_grad_enabled():
+        if grad_loss is None or not _plain_backward(grad_loss):
             return _train_sliced_backward(ctx, grad_loss, None, None, None)
         indices, weight, vals, bias, target, dvals, dbias = ctx.saved_tensors
         dW = None
@@ -1216,7 +1225,7 @@ class _HierLateStep(torch.autograd.Function):
         if grad_loss is None:
             return None, None, None, None, None, None, None
         indices, weight, vals, bias, target = ctx.saved_tensors
-        if torch.is_grad_enabled():  # (a graph of the backward is built by the ops)
+        if not _plain_backward(grad_loss):
             with torch.no_grad():
                 _, dvals, dbias, dW = hier_train_sliced(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense)
             g = grad_loss.to(torch.float32)

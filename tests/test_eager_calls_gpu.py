@@ -100,6 +100,29 @@ def test_graphs_hooks_and_transforms(loss):
         torch.func.grad(lambda w: LOSS[loss](idx, w, v, b, t) * 2.0)(W)
 
 
+@pytest.mark.parametrize("loss,fused,dtype,size", [
+    ("topk", True, torch.float32, (16, 8, 60, 128)), ("hier", False, torch.bfloat16, (16, 8, 60, 128)),
+    ("hier", True, torch.float16, (16, 8, 60, 128)), ("hier", True, torch.float16, (16, 8, 8192, 2048))])
+def test_the_surroundings_of_the_backward_count(loss, fused, dtype, size):
+    """A backward over batched upstream gradients, and one under a mode that its forward did not see, go through the ops."""
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(*size, dtype, seed=6))
+    flex.set_fused_training(fused)
+    try:
+        leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+        out = LOSS[loss](idx, *leaves, t)
+        ups = torch.tensor([1.0, 2.0, -0.5], device=DEV)
+        want = [torch.autograd.grad(out, leaves, u, retain_graph=True) for u in ups]
+        got = torch.autograd.grad(out, leaves, ups, retain_graph=True, is_grads_batched=True)
+        for i, grads in enumerate(want):
+            assert all(torch.equal(x, y[i]) for x, y in zip(grads, got))
+        with _Seen() as seen:
+            again = torch.autograd.grad(out, leaves, ups[1])
+        assert any("flexsae_amd" in o for o in seen.ops)
+        assert all(torch.equal(x, y) for x, y in zip(again, want[1]))
+    finally:
+        flex.set_fused_training(True)
+
+
 def test_the_fused_update_marks_the_weight():
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=4))
     W2 = W.clone()
