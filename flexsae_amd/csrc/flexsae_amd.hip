@@ -1193,6 +1193,8 @@ void build_hot_tables(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws
 
 struct TopkBwdPlan {
   int vec, tile;
+  int row_vec;      // elements of a vector that divides the rows of W and dW: vec, or less where the residual copy is padded
+  int resid_ld;     // elements from one gathered row to the next
   int64_t d_pad;
   size_t n_pairs, n_partial_rows;
   size_t off_colsum, off_ctrl, off_long_list, off_lists, off_resid16, off_dvpart, off_slotbv, off_partial, fixed_bytes;
@@ -1207,8 +1209,19 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   // shares: flexsae_topk_bwd_workspace_bytes returns the larger of the two layouts).
   p.resid16 = FLEXSAE_TOPK_RESID16 && s->weight_dtype == FLEXSAE_BF16 && !(flags & FLEXSAE_TOPK_BWD_FP32_RESIDUAL);
   p.vec = (s->D % 4 == 0) ? 4 : (s->D % 2 == 0) ? 2 : 1;
+  p.row_vec = p.vec;
+  p.resid_ld = static_cast<int>(s->D);
   // all-bf16: 16 bytes per lane (512-column tiles) halve the per-tile overheads
-  if (FLEXSAE_TOPK_VEC8 && p.resid16 && s->D % 8 == 0) p.vec = 8;
+  if (FLEXSAE_TOPK_VEC8 && p.resid16 && s->D % 8 == 0) p.vec = p.row_vec = 8;
+  // Rows that eight does not divide: the copy's rows are padded, so that its gathers are as wide (the step, us, with
+  // vectors that divide the row / padded; B=4096, F=65536, K=128: D=2305 1146 / 829, 2306 879 / 759, 2308 756 / 718; K=32:
+  // D=2305 563 / 405, 2306 399 / 346; B=8192, F=262144, K=64, D=1026 687 / 660; B=300, F=400000, K=16, D=4097 3281 / 1812,
+  // D=4098 2253 / 1580; B=16384, F=65536, K=64: D=129 246 / 234, 130 216 / 216).  Not where one narrow tile holds the row:
+  // as many gathers either way, and the wide ones leave most lanes without columns.
+  if (FLEXSAE_TOPK_VEC8 && p.resid16 && p.vec != 8 && s->D > kWave * p.vec) {
+    p.vec = 8;
+    p.resid_ld = static_cast<int>(round_up(static_cast<size_t>(s->D), 8));
+  }
   p.tile = kWave * p.vec;
   p.d_pad = ceil_div(s->D, p.tile) * p.tile;
   p.n_pairs = static_cast<size_t>(s->B) * static_cast<size_t>(s->K);
@@ -1223,7 +1236,7 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   p.off_lists = off;
   off += carve_pair_lists(p.n_pairs, static_cast<size_t>(s->F), false, nullptr, nullptr);
   p.off_resid16 = off;
-  if (p.resid16) off += round_up(static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 2, kAlign);
+  if (p.resid16) off += round_up(static_cast<size_t>(s->B) * static_cast<size_t>(p.resid_ld) * 2, kAlign);
   p.off_dvpart = off;  // per-tile shares of dvals: [d_pad / tile, B*K] fp32
   off += round_up(static_cast<size_t>(p.d_pad / p.tile) * p.n_pairs * 4, kAlign);
   p.off_slotbv = off;  // (batch row, val) of every pair in pair-list order
@@ -1245,7 +1258,7 @@ size_t topk_bwd_bytes(const TopkBwdPlan &p, int64_t slice_w) {
   return p.fixed_bytes + round_up(p.n_partial_rows * static_cast<size_t>(slice_w) * 4, kAlign);
 }
 
-template <typename WT, typename GT, typename RT, int VEC>
+template <typename WT, typename GT, typename RT, int VEC, int EV>
 void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                         const uint32_t *begin, const uint32_t *map, const void *weight,
                         const void *vals, const void *resid, const float *grad_out, float coef,
@@ -1266,46 +1279,47 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
     const int64_t xcd_span = ceil_div(n_groups * tps, 8);
     const unsigned n_long = kLongBlocks * static_cast<unsigned>(tps);
     const size_t resid_bytes =
-        static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * sizeof(typename Traits<RT>::store_t);
-    hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC>),
+        static_cast<size_t>(s->B) * static_cast<size_t>(pl.resid_ld) * sizeof(typename Traits<RT>::store_t);
+    constexpr int kEndTiles = VEC / EV;  // tiles of the long latents' second step per tile
+    hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC, EV>),
                        dim3(n_long + static_cast<unsigned>(xcd_span * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
                        s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, tps,
-                       static_cast<int>(col0), sw, s->F, K, D, static_cast<uint32_t>(resid_bytes));
+                       static_cast<int>(col0), sw, s->F, K, D, pl.resid_ld, static_cast<uint32_t>(resid_bytes));
     if (col0 + slice_w < s->D) {
-      hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, VEC, 8>), dim3(256), dim3(kBlock), 0, st,
-                         long_ctrl, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps,
+      hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, EV, 8>), dim3(256), dim3(kBlock), 0, st,
+                         long_ctrl, long_list, chunk_begin, partial, dW, static_cast<const float *>(nullptr), tps * kEndTiles,
                          static_cast<int>(col0), sw, D);
       continue;
     }
     constexpr unsigned n_long_blocks = 256;
     const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(D, kBlock));
-    hipLaunchKernelGGL((topk_epilogue_kernel<GT, VEC>),
+    hipLaunchKernelGGL((topk_epilogue_kernel<GT, EV>),
                        dim3(n_long_blocks + n_col_blocks + grid_for(n_pairs, kBlock, 8192)), dim3(kBlock), 0, st, long_ctrl,
-                       long_list, chunk_begin, partial, dW, tps, static_cast<int>(col0), sw, D, n_long_blocks,
+                       long_list, chunk_begin, partial, dW, tps * kEndTiles, static_cast<int>(col0), sw, D, n_long_blocks,
                        reinterpret_cast<const float *>(ws + pl.off_colsum), static_cast<int>(ceil_div(s->B, kColsumRows)),
                        grad_out, coef, dbias, n_col_blocks, map, dv_part, static_cast<int>(pl.d_pad / pl.tile), n_pairs,
                        dvals);
   }
 }
 
-template <typename WT, typename RT, int VEC>
+template <typename WT, typename RT, int VEC, int EV = VEC>
 void launch_topk_slices_g(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                           const uint32_t *begin, const uint32_t *map, const void *weight,
                           const void *vals, const void *resid, const float *grad_out, float coef,
                           void *dW, int dW_dtype, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
   switch (dW_dtype) {
     case FLEXSAE_F32:
-      launch_topk_slices<WT, float, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
+      launch_topk_slices<WT, float, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
                                              coef, dW, dvals, dbias, ws, st);
       break;
     case FLEXSAE_BF16:
-      launch_topk_slices<WT, bf16_t, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
+      launch_topk_slices<WT, bf16_t, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
                                               coef, dW, dvals, dbias, ws, st);
       break;
     default:
-      launch_topk_slices<WT, f16_t, RT, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
+      launch_topk_slices<WT, f16_t, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
                                              coef, dW, dvals, dbias, ws, st);
   }
 }
@@ -1774,9 +1788,9 @@ int flexsae_topk_bwd(const flexsae_shape *s, const uint32_t *begin, const uint32
   if (static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 4 > 0xffffffffull) return FLEXSAE_ERR_UNSUPPORTED;
   const TopkBwdPlan pl = plan_topk_bwd(s, flags);
   if (!aligned(begin, 4) || !aligned(map, 4) || (indices && !aligned(indices, 8)) ||
-      !aligned(weight, pl.vec * dtype_size(s->weight_dtype)) ||
+      !aligned(weight, pl.row_vec * dtype_size(s->weight_dtype)) ||
       !aligned(vals, dtype_size(s->vals_dtype)) || !aligned(resid, pl.resid16 ? 16 : pl.vec * 4) ||
-      !aligned(grad_out, 4) || !aligned(dW, pl.vec * dtype_size(dW_dtype)) || !aligned(dvals, 16) ||
+      !aligned(grad_out, 4) || !aligned(dW, pl.row_vec * dtype_size(dW_dtype)) || !aligned(dvals, 16) ||
       !aligned(dbias, 4))
     return FLEXSAE_ERR_ALIGNMENT;
   if (!workspace || !aligned(workspace, kAlign) || workspace_bytes < topk_bwd_bytes(pl, pl.tile))
@@ -1793,19 +1807,22 @@ int flexsae_topk_bwd(const flexsae_shape *s, const uint32_t *begin, const uint32
   // per-pair records, for bf16 weights the bf16 copy of the residual, and stage 1 of dbias: one launch
   const void *gather_src = pl.resid16 ? static_cast<const void *>(ws + pl.off_resid16) : resid;
   {
-    const int64_t n_resid = pl.resid16 ? s->B * s->D : 0;
+    const int64_t n_resid = pl.resid16 ? s->B * pl.resid_ld : 0;
     const int64_t work = s->B * s->K > ceil_div(n_resid, 4) ? s->B * s->K : ceil_div(n_resid, 4);
     const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(s->D, 256) * ceil_div(s->B, kColsumRows));
     hipLaunchKernelGGL(topk_prepare_kernel, dim3(n_col_blocks + grid_for(work, 256, 1 << 16)), dim3(256), 0, st, map, indices,
                        s->F, vals, s->vals_dtype, s->B * s->K, static_cast<int>(s->K),
                        reinterpret_cast<vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), resid, n_resid,
                        pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr, lists.ctrl, s->B,
-                       static_cast<int>(s->D), reinterpret_cast<float *>(ws + pl.off_colsum), n_col_blocks);
+                       static_cast<int>(s->D), pl.resid_ld, reinterpret_cast<float *>(ws + pl.off_colsum), n_col_blocks);
   }
   launch_pair_lists(begin, s->F, lists, st, true);
   if (pl.vec == 8) {
-    launch_topk_slices_g<bf16_t, bf16_t, 8>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef,
-                                            dW, dW_dtype, dvals, dbias, ws, st);
+    const auto slices = pl.row_vec == 8   ? launch_topk_slices_g<bf16_t, bf16_t, 8>
+                        : pl.row_vec == 4 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 4>
+                        : pl.row_vec == 2 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 2>
+                                          : launch_topk_slices_g<bf16_t, bf16_t, 8, 1>;
+    slices(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW, dW_dtype, dvals, dbias, ws, st);
   } else if (pl.vec == 4) {
     launch_topk_slices_w<4>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
                             dW_dtype, dvals, dbias, ws, st);

@@ -98,7 +98,11 @@ constexpr int topk_group() {
 // the W and dW streams.  Against one latent per wavefront (us; the kernel there 265 -> 245) the whole backward: K=128 340 ->
 // 320, K=64 247 -> 224, K=32 214 -> 180; F=262144, K=64 650 -> 463; B=2048, K=64, F=131072, D=1024 fp32 241 -> 192; two or four
 // latents, or two batches in flight (fewer wavefronts per SIMD): 2-20 % slower.
-template <typename WT, typename GT, typename RT, int VEC, int L>
+//
+// EV < VEC: rows of W and dW that only vectors of EV elements divide (the residual copy's rows are padded to VEC with zeros).
+// They pass through the LDS in such vectors, neighbouring lanes on neighbouring ones, so that every access is one run of
+// lines as with narrow tiles, while the gathers keep their 16 bytes per lane.
+template <typename WT, typename GT, typename RT, int VEC, int EV, int L>
 __device__ __forceinline__ void topk_short_latents(
     const uint32_t *__restrict__ begin, const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight,
     int vals_dtype, const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
@@ -144,16 +148,43 @@ __device__ __forceinline__ void topk_short_latents(
   };
   uint32_t slot = slot_of(lane);
   // W rows: for a latent without pairs here a descriptor of no bytes, which reads zeros and no memory (so do lanes beyond D)
-  raw_vec_t<WT, VEC> wraw[L];
-#pragma unroll
-  for (int l = 0; l < L; ++l) {
+  constexpr int kParts = VEC / EV;
+  auto w_row = [&](int l) {
     const uint32_t bytes = bcast_i32(static_cast<int>(n_mine), l) != 0 ? static_cast<uint32_t>(D) * sizeof(S_w) : 0u;
-    const GatherSource row = make_gather_source(static_cast<const S_w *>(weight) + (f0 + l) * D, bytes);
-    wraw[l] = gather_raw<WT, VEC, FLEXSAE_TOPK_NT>(row, static_cast<uint32_t>(d0) * sizeof(S_w), 0u);
-  }
-  if (lane < M) bv = __builtin_nontemporal_load(slot_bv + slot);
+    return make_gather_source(static_cast<const S_w *>(weight) + (f0 + l) * D, bytes);
+  };
+  if constexpr (kParts == 1) {
+    raw_vec_t<WT, VEC> wraw[L];
 #pragma unroll
-  for (int l = 0; l < L; ++l) pieces[l * kWave + lane].w = wraw[l];
+    for (int l = 0; l < L; ++l)
+      wraw[l] = gather_raw<WT, VEC, FLEXSAE_TOPK_NT>(w_row(l), static_cast<uint32_t>(d0) * sizeof(S_w), 0u);
+    if (lane < M) bv = __builtin_nontemporal_load(slot_bv + slot);
+#pragma unroll
+    for (int l = 0; l < L; ++l) pieces[l * kWave + lane].w = wraw[l];
+  } else {
+    const int tile0 = d0 - lane * VEC;
+    if (lane < M) bv = __builtin_nontemporal_load(slot_bv + slot);
+    constexpr int kAtOnce = kParts == 8 && L == 8 ? L / 2 : L;  // 32 registers
+#pragma unroll
+    for (int l0 = 0; l0 < L; l0 += kAtOnce) {
+      raw_vec_t<WT, EV> part[kAtOnce][kParts];
+#pragma unroll
+      for (int l = 0; l < kAtOnce; ++l) {
+        const GatherSource row = w_row(l0 + l);
+#pragma unroll
+        for (int k = 0; k < kParts; ++k)
+          part[l][k] = gather_raw<WT, EV>(row, static_cast<uint32_t>(tile0 + (k * kWave + lane) * EV) * sizeof(S_w), 0u);
+      }
+#pragma unroll
+      for (int l = 0; l < kAtOnce; ++l)
+#pragma unroll
+        for (int k = 0; k < kParts; ++k) {
+          const int c = (k * kWave + lane) * EV;
+          auto *const w_at = reinterpret_cast<S_w *>(&pieces[(l0 + l) * kWave + c / VEC].w) + c % VEC;
+          *reinterpret_cast<raw_vec_t<WT, EV> *>(w_at) = part[l][k];
+        }
+    }
+  }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 
@@ -265,17 +296,27 @@ __device__ __forceinline__ void topk_short_latents(
     walk(std::false_type{});
   }
   if (M > 0) flush();
+  if constexpr (kParts > 1) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
 #pragma unroll
   for (int l = 0; l < L; ++l) {
     const uint32_t n = static_cast<uint32_t>(bcast_i32(static_cast<int>(n_all), l));
     if (f0 + l < F && n <= static_cast<uint32_t>(kSegChunk)) {  // uniform
       using G = typename Traits<GT>::store_t;
-      raw_vec_t<GT, VEC> x = pieces[l * kWave + lane].g;
-      if (n == 0) x = raw_vec_t<GT, VEC>{};
-      if (active) {
-        auto *const to = reinterpret_cast<raw_vec_t<GT, VEC> *>(static_cast<G *>(dW) + (f0 + l) * D + d0);
-        if constexpr (FLEXSAE_TOPK_NT) __builtin_nontemporal_store(x, to);
-        else *to = x;
+#pragma unroll
+      for (int k = 0; k < kParts; ++k) {
+        const int c = kParts == 1 ? lane * VEC : (k * kWave + lane) * EV;  // column in the tile
+        const int d = d0 - lane * VEC + c;
+        raw_vec_t<GT, EV> x =
+            *reinterpret_cast<const raw_vec_t<GT, EV> *>(reinterpret_cast<const G *>(&pieces[l * kWave + c / VEC].g) + c % VEC);
+        if (n == 0) x = raw_vec_t<GT, EV>{};
+        if (d < D) {
+          auto *const to = reinterpret_cast<raw_vec_t<GT, EV> *>(static_cast<G *>(dW) + (f0 + l) * D + d);
+          if constexpr (FLEXSAE_TOPK_NT) __builtin_nontemporal_store(x, to);
+          else *to = x;
+        }
       }
     }
   }
@@ -292,7 +333,8 @@ __device__ __forceinline__ void topk_short_latents(
 // backward, K=64 249 -> 192; bf16 the same either way).
 // dW[f, tile] is written exactly once, in the gradient's final dtype; latents without pairs
 // get zeros.
-template <typename WT, typename GT, typename RT, int VEC>
+// resid_ld: elements from one row of resid to the next.  EV: elements of a vector that divides the rows of W and dW.
+template <typename WT, typename GT, typename RT, int VEC, int EV>
 __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const uint32_t *__restrict__ begin, const uint32_t *__restrict__ map,
     const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
@@ -301,7 +343,7 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
     unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int tps, int col0, int slice_w, int64_t F, int K, int D,
-    uint32_t resid_bytes) {
+    int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
   constexpr int L = topk_group<WT, GT, VEC>();
@@ -314,8 +356,8 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * L;
     if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
-    topk_short_latents<WT, GT, RT, VEC, L>(
-        begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(D) * sizeof(typename Traits<RT>::store_t), scale,
+    topk_short_latents<WT, GT, RT, VEC, EV, L>(
+        begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
         dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, F, col0 + t * (kWave * VEC) + lane * VEC, D,
         pieces[wave_in_block()]);
     return;
@@ -336,14 +378,19 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const bool active = d0 < D;
     const int dsafe = active ? d0 : 0;
     float w[VEC], acc[VEC];
-    load_vec<WT, VEC>(weight, c.f * D + dsafe, w);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      acc[i] = 0.f;
-      if (!active) w[i] = 0.f;
+    for (int i = 0; i < VEC; i += EV) {
+      float part[EV];
+      const int d = d0 + i < D ? d0 + i : 0;
+      load_vec<WT, EV>(weight, c.f * D + d, part);
+#pragma unroll
+      for (int k = 0; k < EV; ++k) {
+        acc[i + k] = 0.f;
+        w[i + k] = d0 + i < D ? part[k] : 0.f;
+      }
     }
     topk_accumulate_slots<RT, VEC>(slot_bv, resid, scale, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, w, c.s0,
-                                   c.s1, D, dsafe, acc);
+                                   c.s1, resid_ld, dsafe, acc);
     store_vec<float, VEC>(partial, static_cast<int64_t>(chunk) * slice_w + pc, acc);
   }
 }
@@ -387,7 +434,8 @@ __global__ __launch_bounds__(256) void topk_epilogue_kernel(
 //     the backward reads per pair, contiguous per latent instead of scattered over vals; a pair
 //     whose index lies outside [0, F) gets a val of zero, as in the forward (the pair list files it
 //     under latent 0), so that it adds nothing to dW (`indices` may be null: every val is kept);
-//   resid16[i] = bf16(resid[i]) for i < n_resid (n_resid = 0: no copy wanted);
+//   resid16[b, d] = bf16(resid[b, d]), rows of ld16 >= cols elements with zeros past cols (ld16 a multiple of four, or
+//     cols; n_resid = rows * ld16, 0: no copy wanted);
 //   ctrl[] = 0: the control words of the lists that the next launch fills;
 //   in the first n_col_blocks blocks, stage 1 of the column sums of resid (for dbias).
 __global__ __launch_bounds__(256) void topk_prepare_kernel(const uint32_t *__restrict__ map, const int64_t *__restrict__ indices,
@@ -395,7 +443,7 @@ __global__ __launch_bounds__(256) void topk_prepare_kernel(const uint32_t *__res
                                     int vals_dtype, int64_t n_pairs, int K,
                                     vec_t<uint32_t, 2> *__restrict__ slot_bv, const float *__restrict__ resid,
                                     int64_t n_resid, void *__restrict__ resid16, uint32_t *__restrict__ ctrl,
-                                    int64_t rows, int cols, float *__restrict__ colsum_part, unsigned n_col_blocks) {
+                                    int64_t rows, int cols, int ld16, float *__restrict__ colsum_part, unsigned n_col_blocks) {
   if (blockIdx.x < n_col_blocks) {
     const unsigned across = static_cast<unsigned>((cols + 255) / 256);
     colsum_partial_one(resid, rows, cols, cols, colsum_part, static_cast<int>(blockIdx.x % across * 256 + threadIdx.x),
@@ -415,6 +463,19 @@ __global__ __launch_bounds__(256) void topk_prepare_kernel(const uint32_t *__res
     slot_bv[s] = r;
   }
   const int64_t n4 = n_resid >> 2;
+  if (ld16 != cols) {
+    const uint32_t per_row = static_cast<uint32_t>(ld16) >> 2;
+    for (int64_t i = tid; i < n4; i += stride) {
+      const uint32_t row = static_cast<uint32_t>(i) / per_row;
+      const int c = static_cast<int>((static_cast<uint32_t>(i) - row * per_row) * 4);
+      const float *const from = resid + static_cast<int64_t>(row) * cols;
+      float x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = c + k < cols ? from[c + k] : 0.f;
+      store_vec<bf16_t, 4>(resid16, i * 4, x);
+    }
+    return;
+  }
   for (int64_t i = tid; i < n4; i += stride) {
     float x[4];
     load_vec<float, 4>(resid, i * 4, x);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
 
 
-@pytest.mark.parametrize("D", [8, 520, 1030, 77])
+@pytest.mark.parametrize("D", [8, 64, 65, 77, 130, 260, 515, 520, 1028, 1030])
 @pytest.mark.parametrize("dtype,vals_dtype,dw_dtype", [
     (torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16, torch.bfloat16),
     (torch.bfloat16, torch.float32, torch.float32), (torch.float16, torch.float16, torch.float16)], ids=str)
