@@ -645,11 +645,30 @@ def _train_supported(weight: Tensor, K: int) -> bool:
 
 def _train_ragged(weight: Tensor, K: int) -> bool:
     """Rows that the training-step kernel takes by its lanes' columns though no vector of four divides them
-    (FLEXSAE_BWD_RAGGED_ROWS; not staged): one gather instead of one in the forward and one in the sweep, the same bits
-    (B = 1777, K = 50, F = 24571, D = 1538 bf16: the step 298 -> 266 us; B = 4096, K = 128, F = 65536, D = 2306:
-    1892 -> 1486)."""
+    (FLEXSAE_BWD_RAGGED_ROWS; not staged): one gather instead of one in the forward and one in the sweep, the same bits."""
     D = weight.shape[1]
     return D % 4 != 0 and K <= 256 and (D % 2 == 0 or (weight.dtype == torch.float32 and K > 64))
+
+
+def _ragged_pays(weight: Tensor, B: int, K: int) -> bool:
+    """Whether the training step is the faster one for such rows.  Against forward and sweep, uniform and Zipf:
+    bf16, D = 2306, B = 1662, F = 97114: K = 16 1.19 and 1.17 times as fast, K = 50 1.23 and 1.11, K = 128 1.21 and 1.15,
+    K = 256 1.17 and 1.15 (fp32 1.11 to 1.30).  Not with 129 to 255 steps (K = 160 and 200 0.80 to 0.83, B = 1777, F = 24571
+    0.73 to 0.82; fp32 0.77 to 1.0), and for fp16 weights, whose unit gradient is written in fp32 and scaled in a pass of its
+    own, from six pairs per latent on (B = 1777, F = 24571, K = 64 1.02 and 0.94, K = 100 1.06 and 1.06; B = 6000, F = 8192
+    1.1; B = 300, F = 65536, K = 16 to 64 0.84 to 0.97)."""
+    if 128 < K < 256:
+        return False
+    return weight.dtype != torch.float16 or not weight.requires_grad or B * K > 6 * weight.shape[0]
+
+
+def _step_pays(weight: Tensor, K: int) -> bool:
+    """Not 129 to 255 steps, for which the training-step kernel is the one built for 256 and tests every step: forward and
+    sweep, two gathers, are faster where the weight takes a gradient.  Time of forward and sweep over that of the training
+    step, K = 136 to 240, uniform and Zipf: B = 1777, F = 24571, D = 2304 bf16 0.71 to 0.74, fp16 0.86 to 0.94, fp32 0.69
+    to 0.81; B = 1662, F = 97114 0.79 to 0.88, 0.86 to 0.91, 0.85 to 1.0; B = 300, F = 65536 0.80 to 1.09, 0.74 to 1.04,
+    0.93 to 1.02; K = 128 and 256 1.1 to 1.3."""
+    return not 128 < K < 256 or not weight.requires_grad
 
 
 def _stage_fits(indices: Tensor, weight: Tensor) -> bool:
@@ -1203,10 +1222,11 @@ def _late_step(weight: Tensor, B: int, K: int) -> bool:
     rounded.  A second gather (2*B*K*D bytes, partly out of the L2s) for 6*F*D bytes less: us with it / without, uniform
     and Zipf indices, B = 4096, F = 65536, D = 2304: K = 16 469 / 538, 409 / 566; K = 32 723 / 765, 595 / 697; K = 64
     1252 / 1284, 1059 / 1081; K = 128 2369 / 2279; B = 8192, K = 64, F = 262144, D = 4096 4878 / 5786, 3526 / 4518; B = 256,
-    K = 64, F = 65536, D = 2048 171 / 332.  Not below 16 million weights, where two launches more show (F = 16384, D = 512
-    161 / 148; F = 32768, D = 1024 182 / 202)."""
+    K = 64, F = 65536, D = 2048 171 / 332.  Not below 96 million weights, where more launches and their host work show (F = 65536,
+    K = 32, B = 410 and 2048: D = 1544 282 / 338 and 362 / 414, D = 1024 258 / 221 and 266 / 262, D = 900 256 / 219 and
+    269 / 257, D = 512 249 / 219 and 252 / 215)."""
     F, D = weight.shape
-    return weight.dtype == torch.float16 and B * K <= 4 * F and F * D >= 1 << 24
+    return weight.dtype == torch.float16 and B * K <= 4 * F and F * D >= 96 << 20
 
 
 class _HierLateStep(torch.autograd.Function):
@@ -1245,14 +1265,15 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
         indices = indices.to(torch.int64)
     needs_grad = torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad)
     if (needs_grad and _fused_training and weight.dim() == 2 and indices.dim() == 2
-            and (_train_supported(weight, indices.shape[1]) or _train_ragged(weight, indices.shape[1]))):
+            and (_train_supported(weight, indices.shape[1])
+                 or (_train_ragged(weight, indices.shape[1]) and _ragged_pays(weight, *indices.shape)))):
         # (a compiler trace cannot follow the stage's size query: traced calls take the sliced step,
         # which gives the same bits)
         if _train_supported(weight, indices.shape[1]) and _stage_fits(indices, weight) and not _is_traced(weight):
             return _HierTrainStaged.apply(indices, weight, vals, bias, target)
         # (fp16 weights: the step's unit-gradient dW is fp32, of magnitude 2/(B*K*D), and is scaled by the
         # upstream gradient before its only rounding, like reference hierarchical_kernels.py:294-299)
-        if _hier_scratch_bytes != 0:
+        if _hier_scratch_bytes != 0 and _step_pays(weight, indices.shape[1]):
             B, K = indices.shape
             F, D = weight.shape
             hot = bool(weight.requires_grad) and _use_hot_latents(B, K, F, D, weight.dtype, weight.device,

@@ -102,10 +102,12 @@ def test_graphs_hooks_and_transforms(loss):
 
 @pytest.mark.parametrize("loss,fused,dtype,size", [
     ("topk", True, torch.float32, (16, 8, 60, 128)), ("hier", False, torch.bfloat16, (16, 8, 60, 128)),
-    ("hier", True, torch.float16, (16, 8, 60, 128)), ("hier", True, torch.float16, (16, 8, 8192, 2048))])
-def test_the_surroundings_of_the_backward_count(loss, fused, dtype, size):
+    ("hier", True, torch.float16, (16, 8, 60, 128)), ("hier", True, torch.float16, (16, 8, 200, 256))])
+@pytest.mark.parametrize("late", [False, True])
+def test_the_surroundings_of_the_backward_count(loss, fused, dtype, size, late, monkeypatch):
     """A backward over batched upstream gradients, and one under a mode that its forward did not see, go through the ops."""
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(*size, dtype, seed=6))
+    monkeypatch.setattr(ops, "_late_step", lambda *_: late)
     flex.set_fused_training(fused)
     try:
         leaves = [x.clone().requires_grad_() for x in (W, v, b)]

@@ -21,12 +21,14 @@ DEV = torch.device("cuda", 0)
     (torch.float32, 65, 1), (torch.float32, 100, 63), (torch.float32, 128, 129), (torch.float32, 200, 1026),
     (torch.float32, 256, 321)], ids=str)
 @pytest.mark.parametrize("F", [70, 4000])
-def test_ragged_rows(F, dtype, K, D):
+def test_ragged_rows(F, dtype, K, D, monkeypatch):
     print("[case]", F, dtype, K, D, flush=True)
     args = make_inputs(150, K, F, D, dtype, seed=K + D)
     args[0][:, 0] = 3
     idx, W, v, b, t = (x.to(DEV) for x in args)
     assert flex.ops._train_ragged(W, K)
+    monkeypatch.setattr(flex.ops, "_ragged_pays", lambda *_: True)  # (whatever is faster)
+    monkeypatch.setattr(flex.ops, "_step_pays", lambda *_: True)
     grads = []
     for fused in (True, False):
         leaves = [x.clone().requires_grad_() for x in (W, v, b)]
@@ -54,3 +56,35 @@ def test_ragged_rows_want_the_flag():
                           flags=_lib.BWD_RAGGED_ROWS | _lib.BWD_SWEEP_ONLY)[0] == _lib.ERR_UNSUPPORTED
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(8, 8, 32, 7, seed=3))
     assert abi.hier_train(idx, W, v, b, t, flags=_lib.BWD_RAGGED_ROWS)[0] == _lib.ERR_UNSUPPORTED
+
+
+def test_which_ragged_rows_take_the_training_step():
+    def pays(dtype, B, K, F, D=390):
+        return flex.ops._ragged_pays(torch.empty(F, D, dtype=dtype, device="meta", requires_grad=True), B, K)
+
+    for dtype in (torch.float32, torch.bfloat16):
+        assert all(pays(dtype, 64, K, 4000) for K in (1, 128, 256)) and not any(pays(dtype, 64, K, 4000) for K in (129, 255))
+    assert pays(torch.float16, 601, 10, 1000) and not pays(torch.float16, 600, 10, 1000)
+    assert not pays(torch.float16, 6000, 200, 1000)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("K,D", [(128, 132), (129, 132), (129, 130), (255, 64), (256, 64)])
+@pytest.mark.parametrize("needs", [(True, True, True), (False, True, True)])
+def test_steps_between_the_kernels(needs, K, D, dtype, monkeypatch):
+    """129 to 255 steps go by forward and sweep where the weight takes a gradient: the training step's gradients."""
+    print("[case]", needs, K, D, dtype, flush=True)
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(70, K, 500, D, dtype, seed=K + D))
+    grads = []
+    for forced in (False, True):
+        if forced:
+            monkeypatch.setattr(flex.ops, "_step_pays", lambda *_: True)
+            monkeypatch.setattr(flex.ops, "_ragged_pays", lambda *_: True)
+        leaves = [x.clone().requires_grad_(n) for x, n in zip((W, v, b), needs)]
+        assert flex.ops._step_pays(leaves[0], K) == (forced or K in (128, 256) or not needs[0])
+        loss = flex.triton_hierarchical_sae_loss(idx, *leaves, t)
+        loss.backward()
+        grads.append([loss.detach()] + [x.grad for x in leaves])
+    assert rel_err(grads[0][0].cpu(), grads[1][0].cpu()) < 1e-6  # other partial sums, all beyond a column in double
+    for x, y in zip(grads[0][1:], grads[1][1:]):
+        assert (x is None and y is None) or torch.equal(x, y)
