@@ -1011,6 +1011,12 @@ def _is_traced(t: Tensor) -> bool:
     return type(t) is not torch.Tensor or torch.compiler.is_compiling()
 
 
+def _is_batched(t: Tensor) -> bool:
+    """A batch of tensors that looks like one of them: under vmap, and in ``autograd.grad(..., is_grads_batched=True)``."""
+    ask = getattr(torch._C, "_functorch", None)
+    return any(getattr(ask, name)(t) for name in ("is_batchedtensor", "is_legacy_batchedtensor") if hasattr(ask, name))
+
+
 def _train_sliced_setup_context(ctx, inputs, output):
     indices, weight, vals, bias, target, need_dw, hot, dense = inputs
     ctx.need_dw = need_dw
@@ -1048,15 +1054,21 @@ def _train_sliced_backward(ctx, grad_loss, grad_dvals, grad_dbias, grad_dw):
         dW = None
         if ctx.needs_input_grad[1]:
             dW = ctx.dw_unit
-            ctx.dw_unit = None  # the buffer now belongs to whoever receives the gradient
+            # Several upstream gradients at once, or a graph of the backward, get gradients of their own: the buffer stays.
+            own = torch.is_grad_enabled() or _is_batched(g)
+            if not own:
+                ctx.dw_unit = None  # the buffer now belongs to whoever receives the gradient
             if dW is None:
                 # a second backward through a retained graph: the buffer went with the first one
                 with torch.no_grad():
                     _, dvals, dbias, dW = hier_train_sliced(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense)
-            if dW.dtype == weight.dtype:
-                scale_(dW, g)
-            else:  # fp16 weights: the fp32 unit gradient meets the upstream gradient before its only rounding
+            if dW.dtype != weight.dtype:
+                # fp16 weights: the fp32 unit gradient meets the upstream gradient before its only rounding
                 dW = scale_to(dW, g, weight.dtype)
+            elif own:
+                dW = scale_by(dW, g)
+            else:
+                scale_(dW, g)
     return None, dW, (dvals * g).to(vdt), (dbias * g).to(bdt), None, None, None, None
 
 

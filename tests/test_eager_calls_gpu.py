@@ -148,3 +148,27 @@ def test_finish_grads_checks_its_arguments():
     assert fn(p, 1, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT  # in place
     assert fn(odd, 0, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_ALIGNMENT
     assert fn(p, 7, p, 0, 4, none, 0, none, 0, none, 0, none, 0, none, abi.stream()) == _lib.ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("through_ops", [False, True])
+def test_batched_upstream_gradients_of_the_fused_step(dtype, through_ops):
+    """Each gets a weight gradient of its own, and the step's buffer stays for the backward after them: the same with a graph
+    of the backward."""
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, dtype, seed=6))
+    leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+    if through_ops:
+        with _Seen():
+            out = flex.triton_hierarchical_sae_loss(idx, *leaves, t)
+    else:
+        out = flex.triton_hierarchical_sae_loss(idx, *leaves, t)
+    ups = torch.tensor([1.0, 2.0, -0.5], device=DEV)
+    got = torch.autograd.grad(out, leaves, ups, retain_graph=True, is_grads_batched=True)
+    graph = torch.autograd.grad(out, leaves, ups[1], create_graph=True)
+    with _Seen() as seen:
+        want = [torch.autograd.grad(out, leaves, ups[0], retain_graph=True)]
+    assert not any("train_sliced" in o for o in seen.ops)  # from the buffer, not computed again
+    want += [torch.autograd.grad(out, leaves, u, retain_graph=True) for u in ups[1:]]
+    for i, grads in enumerate(want):
+        assert all(torch.equal(x, y[i]) for x, y in zip(grads, got))
+    assert all(torch.equal(x, y) for x, y in zip(want[1], graph))
