@@ -1128,12 +1128,13 @@ _can_tell_plain = (all(hasattr(_C, n) for n in ("_len_torch_dispatch_stack", "_l
 
 def _plain_call(*tensors: Tensor) -> bool:
     """Ordinary tensors on the GPU, and nothing around the call that would have to see the ops.  (The tensors of
-    ``torch.autograd.grad(..., is_grads_batched=True)`` are of type Tensor and have no memory of their own.)"""
+    ``torch.autograd.grad(..., is_grads_batched=True)`` are of type Tensor and have no memory of their own; nor have zero
+    tensors, and the memory of a negative view holds the values with the other sign: the dispatcher sees to both.)"""
     if torch.compiler.is_compiling() or not _can_tell_plain:
         return False
     for t in tensors:
-        if (type(t) not in _PLAIN_TYPES or not t.is_cuda or _C._functorch.is_legacy_batchedtensor(t)
-                or _C._functorch.is_functorch_wrapped_tensor(t)):
+        if (type(t) not in _PLAIN_TYPES or not t.is_cuda or t.is_neg() or t._is_zerotensor()
+                or _C._functorch.is_legacy_batchedtensor(t) or _C._functorch.is_functorch_wrapped_tensor(t)):
             return False
     return (_C._len_torch_dispatch_stack() == 0 and _C._len_torch_function_stack() == 0
             and _C._functorch.peek_interpreter_stack() is None and _C._get_tracing_state() is None

@@ -172,3 +172,26 @@ def test_batched_upstream_gradients_of_the_fused_step(dtype, through_ops):
     for i, grads in enumerate(want):
         assert all(torch.equal(x, y[i]) for x, y in zip(grads, got))
     assert all(torch.equal(x, y) for x, y in zip(want[1], graph))
+
+
+@pytest.mark.parametrize("loss", ["topk", "hier"])
+def test_tensors_whose_memory_is_not_their_values(loss):
+    """Negative views and zero tensors are resolved by the dispatcher: such calls go through the ops."""
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=7))
+    for i in range(1, 5):
+        args = [idx, W, v, b, t]
+        plain = list(args)
+        plain[i] = -plain[i]
+        args[i] = torch._neg_view(args[i])
+        assert torch.equal(LOSS[loss](*args), LOSS[loss](*plain))
+    leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+    out = LOSS[loss](idx, *leaves, t)
+    grads = torch.autograd.grad(out, leaves, torch._efficientzerotensor((), device=DEV), retain_graph=True)
+    assert not any(x.any() for x in grads)
+    grads = torch.autograd.grad(out, leaves, torch._neg_view(torch.ones((), device=DEV)), retain_graph=True)
+    want = torch.autograd.grad(out, leaves, -torch.ones((), device=DEV))
+    assert all(torch.equal(x, y) for x, y in zip(grads, want))
+    W2 = W.clone()
+    got = flex.hierarchical_sae_sgd_step(idx, W, torch._neg_view(v), b, t, 0.5)
+    want = flex.hierarchical_sae_sgd_step(idx, W2, -v, b, t, 0.5)
+    assert torch.equal(W, W2) and all(torch.equal(x, y) for x, y in zip(got, want))
