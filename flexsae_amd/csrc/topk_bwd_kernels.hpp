@@ -115,7 +115,10 @@ __device__ __forceinline__ void topk_short_latents(
   const int dsafe = active ? d0 : 0;
   const uint32_t lane_off = static_cast<uint32_t>(dsafe) * sizeof(S);
   constexpr bool kDot2 = Traits<WT>::dtype == FLEXSAE_BF16 && Traits<RT>::dtype == FLEXSAE_BF16 && VEC % 2 == 0;
-  const bool late_scale = kDot2 && vals_dtype == FLEXSAE_BF16;  // vals enter the dot2 as they are
+  // bf16 vals enter the dot2 as they are, beside a zero for the pair's other column.  Not in rows of odd length: a residual
+  // that is infinite or NaN stays in its own column of dW there, as with the narrow tiles (and the products in fp32 are the
+  // faster ones: the backward at B=4096, K=128, F=65536, D=2305 394 -> 377 us; at D=2304 302 -> 311).
+  const bool late_scale = kDot2 && EV != 1 && vals_dtype == FLEXSAE_BF16;
 
   // lane l: first slot of latent f0 + l (of the one after the last for l = L, and wherever F cuts the group short)
   const int64_t fl = f0 + (lane < L ? lane : L);
@@ -289,7 +292,7 @@ __device__ __forceinline__ void topk_short_latents(
       if (lane < n) dv_tile[slot] = my_dot * scale;
     }
   };
-  if constexpr (kDot2) {
+  if constexpr (kDot2 && EV != 1) {
     if (late_scale) walk(std::true_type{});
     else walk(std::false_type{});
   } else {
