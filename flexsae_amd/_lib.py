@@ -41,6 +41,7 @@ BWD_HOT_BLOCKS_64 = 4096
 BWD_HOT_BLOCKS_32 = 8192
 BWD_RAGGED_ROWS = 16384
 TOPK_BWD_FP32_RESIDUAL = 256
+TOPK_BWD_AS_LARGE = 32768
 
 
 class Shape(ctypes.Structure):

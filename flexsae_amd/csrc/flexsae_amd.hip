@@ -1199,6 +1199,7 @@ struct TopkBwdPlan {
   size_t n_pairs, n_partial_rows;
   size_t off_colsum, off_ctrl, off_long_list, off_lists, off_resid16, off_dvpart, off_slotbv, off_partial, fixed_bytes;
   bool resid16;  // gather a bf16 copy of the residual (bf16 weights): half the cache footprint
+  bool whole_groups;  // as many latents per wavefront as it takes, whatever the size
 };
 
 TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
@@ -1208,6 +1209,7 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   // the caller asks for the fp32 residual (no copy, but narrower tiles and so more per-tile dvals
   // shares: flexsae_topk_bwd_workspace_bytes returns the larger of the two layouts).
   p.resid16 = FLEXSAE_TOPK_RESID16 && s->weight_dtype == FLEXSAE_BF16 && !(flags & FLEXSAE_TOPK_BWD_FP32_RESIDUAL);
+  p.whole_groups = (flags & FLEXSAE_TOPK_BWD_AS_LARGE) != 0;
   p.vec = (s->D % 4 == 0) ? 4 : (s->D % 2 == 0) ? 2 : 1;
   p.row_vec = p.vec;
   p.resid_ld = static_cast<int>(s->D);
@@ -1254,6 +1256,23 @@ PairLists carve_topk_lists(const flexsae_shape *s, const TopkBwdPlan &pl, uint8_
   return ls;
 }
 
+// Neighbouring latents per wavefront, a power of two up to `most`: a wavefront walks their pairs one after the other, so
+// groups pay while there are wavefronts enough with them.  The fewest wavefronts (the chip holds 5120), by pairs per latent;
+// us of the backward with eight / four / two / one latents per wavefront, uniform and skewed (Zipf 1.1) indices:
+//   from 12 pairs on 8192: the walk is long and wants wavefronts to spread over
+//          B=2048, K=109, F=4096, D=336 bf16 108 / 88 / 73 / 67, 92 / 81 / 78 / 76;  8192 to 16384 wavefronts with eight, 16 to
+//          48 pairs: 1.01 / 1.00 / 0.93 and 1.00 / 0.97 / 0.88 times as fast with four / two / one
+//   from 2 on 3072, below 1024: what a wavefront waits for is the head of a latent (its bounds, its records, its W row), and
+//          a group pays it once: 4096 to 6144 wavefronts with eight, 1 to 4 pairs: 0.96 / 0.85 / 0.68, 0.96 / 0.87 / 0.75
+// Over 320 shapes (F 4096 to 131072) 0.6 % behind the best of the four on average, and 5 % at most behind eight.
+int latents_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl, int most) {
+  const int64_t tiles = pl.d_pad / pl.tile, pairs = s->B * s->K;
+  const int64_t least = pairs >= 12 * s->F ? 8192 : pairs >= 2 * s->F ? 3072 : 1024;
+  int n = most;
+  while (n > 1 && ceil_div(s->F, static_cast<int64_t>(n)) * tiles < least) n /= 2;
+  return n;
+}
+
 size_t topk_bwd_bytes(const TopkBwdPlan &p, int64_t slice_w) {
   return p.fixed_bytes + round_up(p.n_partial_rows * static_cast<size_t>(slice_w) * 4, kAlign);
 }
@@ -1268,7 +1287,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   const int64_t n_pairs = static_cast<int64_t>(pl.n_pairs);
-  const int64_t n_groups = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock) * topk_group<WT, GT, VEC>());
+  const int per_wave = pl.whole_groups ? topk_group<WT, GT, VEC>() : latents_per_wave(s, pl, topk_group<WT, GT, VEC>());
+  const int64_t n_groups = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock) * per_wave);
   // a launch holds fewer than 2^32 threads, 2^24 blocks: narrower slices where all tiles would be more
   const int64_t most_tiles = (int64_t{1} << 23) / (n_groups + kLongBlocks);
   if (slice_w / pl.tile > most_tiles) slice_w = (most_tiles < 1 ? 1 : most_tiles) * pl.tile;
@@ -1285,7 +1305,7 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
                        dim3(n_long + static_cast<unsigned>(xcd_span * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
-                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, tps,
+                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, per_wave, tps,
                        static_cast<int>(col0), sw, s->F, K, D, pl.resid_ld, static_cast<uint32_t>(resid_bytes));
     if (col0 + slice_w < s->D) {
       hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, EV, 8>), dim3(256), dim3(kBlock), 0, st,
@@ -1765,7 +1785,7 @@ size_t flexsae_topk_bwd_workspace_bytes(const flexsae_shape *s, int64_t slice_co
   // tiles plus the bf16 copy of the residual) and the FLEXSAE_TOPK_BWD_FP32_RESIDUAL one (narrower
   // tiles: twice the per-tile dvals shares, which outweighs the copy once K exceeds 256).
   size_t need = 0;
-  for (const int flags : {0, static_cast<int>(FLEXSAE_TOPK_BWD_FP32_RESIDUAL)}) {
+  for (const int flags : {0, static_cast<int>(FLEXSAE_TOPK_BWD_FP32_RESIDUAL), static_cast<int>(FLEXSAE_TOPK_BWD_AS_LARGE)}) {
     const TopkBwdPlan pl = plan_topk_bwd(s, flags);
     int64_t sw = slice_cols <= 0 ? pl.tile : ceil_div(slice_cols, pl.tile) * pl.tile;
     if (sw > pl.d_pad) sw = pl.d_pad;

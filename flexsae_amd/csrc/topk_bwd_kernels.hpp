@@ -106,7 +106,8 @@ template <typename WT, typename GT, typename RT, int VEC, int EV, int L>
 __device__ __forceinline__ void topk_short_latents(
     const uint32_t *__restrict__ begin, const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight,
     int vals_dtype, const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
-    float *__restrict__ dv_tile, int64_t f0, int64_t F, int d0, int D, LatentPiece<WT, GT, VEC> *__restrict__ pieces) {
+    float *__restrict__ dv_tile, int64_t f0, int per_wave, int64_t F, int d0, int D,
+    LatentPiece<WT, GT, VEC> *__restrict__ pieces) {
   using S = typename Traits<RT>::store_t;
   using S_w = typename Traits<WT>::store_t;
   static_assert(L <= 8, "the counts of a wavefront's latents are scanned inside eight lanes");
@@ -120,11 +121,11 @@ __device__ __forceinline__ void topk_short_latents(
   // faster ones: the backward at B=4096, K=128, F=65536, D=2305 394 -> 377 us; at D=2304 302 -> 311).
   const bool late_scale = kDot2 && EV != 1 && vals_dtype == FLEXSAE_BF16;
 
-  // lane l: first slot of latent f0 + l (of the one after the last for l = L, and wherever F cuts the group short)
-  const int64_t fl = f0 + (lane < L ? lane : L);
+  // lane l: first slot of latent f0 + l (of the one after the last for l >= per_wave, and wherever F cuts the group short)
+  const int64_t fl = f0 + (lane < per_wave ? lane : per_wave);
   const uint32_t first = begin[fl < F ? fl : F];
   const uint32_t past = static_cast<uint32_t>(__shfl_down(static_cast<int>(first), 1));  // (of all lanes: lane L is read)
-  const uint32_t n_all = lane < L ? past - first : 0u;
+  const uint32_t n_all = lane < per_wave ? past - first : 0u;
   const bool is_long = n_all > static_cast<uint32_t>(kSegChunk);  // chunk role
   const uint32_t n_mine = is_long ? 0u : n_all;
   uint32_t upto = n_mine;  // pairs of latents f0 .. f0 + lane
@@ -306,7 +307,7 @@ __device__ __forceinline__ void topk_short_latents(
 #pragma unroll
   for (int l = 0; l < L; ++l) {
     const uint32_t n = static_cast<uint32_t>(bcast_i32(static_cast<int>(n_all), l));
-    if (f0 + l < F && n <= static_cast<uint32_t>(kSegChunk)) {  // uniform
+    if (l < per_wave && f0 + l < F && n <= static_cast<uint32_t>(kSegChunk)) {  // uniform
       using G = typename Traits<GT>::store_t;
 #pragma unroll
       for (int k = 0; k < kParts; ++k) {
@@ -345,8 +346,8 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
-    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int tps, int col0, int slice_w, int64_t F, int K, int D,
-    int resid_ld, uint32_t resid_bytes) {
+    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int per_wave, int tps, int col0, int slice_w, int64_t F, int K,
+    int D, int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
   constexpr int L = topk_group<WT, GT, VEC>();
@@ -356,12 +357,12 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const int64_t item = (blockIdx.x & 7) * xcd_span + i;
     const int t = static_cast<int>(item / n_groups);
     if (i >= xcd_span || t >= tps) return;
-    const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * L;
+    const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * per_wave;
     if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
     topk_short_latents<WT, GT, RT, VEC, EV, L>(
         begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
-        dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, F, col0 + t * (kWave * VEC) + lane * VEC, D,
+        dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F, col0 + t * (kWave * VEC) + lane * VEC, D,
         pieces[wave_in_block()]);
     return;
   }

@@ -105,6 +105,9 @@ enum {
                                      /* exponent of the hot-latent accumulators is set 8 bits   */
                                      /* lower than usual, so that most rows take the deferred   */
                                      /* second pass; results stay valid                         */
+  FLEXSAE_TOPK_BWD_AS_LARGE = 32768, /* NOT PART OF THE STABLE ABI (a test aid): flexsae_topk_bwd */
+                                     /* launches as for a problem that fills the chip whatever  */
+                                     /* its size; results stay valid                            */
   FLEXSAE_BWD_SKIP_EPILOGUE = 64     /* NOT PART OF THE STABLE ABI (a measurement aid of this   */
                                      /* library's own benchmark, with no counterpart in the     */
                                      /* reference; may change or go without an ABI bump).       */

@@ -3,6 +3,7 @@ with more than that (reduced apart) side by side; groups cut short by F, streams
 import pytest
 import torch
 
+from flexsae_amd import _lib
 from tests import abi
 
 pytestmark = pytest.mark.gpu
@@ -17,8 +18,9 @@ DEV = torch.device("cuda", 0)
 @pytest.mark.parametrize("counts", [
     [0, 64, 65, 1, 0, 0, 130, 64, 64, 64, 64, 64, 64, 64, 64, 64, 0, 0, 0, 0, 0, 0, 0, 0, 3],
     [5], [0, 0, 7, 66, 0, 8, 9, 1, 0], [66] * 8 + [2] * 33 + [0] * 7], ids=["edges", "one", "short", "runs"])
-def test_groups(counts, dtype, vals_dtype, dw_dtype, D):
-    print("[case]", counts[:4], dtype, vals_dtype, dw_dtype, D, flush=True)
+@pytest.mark.parametrize("flags", [0, _lib.TOPK_BWD_AS_LARGE], ids=["as_small", "whole_groups"])
+def test_groups(flags, counts, dtype, vals_dtype, dw_dtype, D):
+    print("[case]", flags, counts[:4], dtype, vals_dtype, dw_dtype, D, flush=True)
     F = len(counts)
     K = 4
     pairs = torch.cat([torch.full((c,), f, dtype=torch.long) for f, c in enumerate(counts)])
@@ -30,7 +32,8 @@ def test_groups(counts, dtype, vals_dtype, dw_dtype, D):
     v = torch.randn(B, K, generator=g).to(vals_dtype)
     resid = torch.randn(B, D, generator=g)
     grad = 1.5
-    rc, dW, dv, db = abi.topk_backward(idx.to(DEV), W.to(DEV), v.to(DEV), resid.to(DEV), grad, dw_dtype=dw_dtype)
+    rc, dW, dv, db = abi.topk_backward(idx.to(DEV), W.to(DEV), v.to(DEV), resid.to(DEV), grad, dw_dtype=dw_dtype,
+                                       flags=flags)
     torch.cuda.synchronize()
     assert rc == 0
     gathered = resid.to(torch.bfloat16) if dtype == torch.bfloat16 else resid  # what the call gathers
@@ -49,3 +52,19 @@ def test_groups(counts, dtype, vals_dtype, dw_dtype, D):
     prods = rows * W.double()[flat] * scale
     bound = (D + 8) * 2.0 ** -24 * prods.abs().sum(1)
     assert ((dv.cpu().double().reshape(-1) - prods.sum(1)).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("B,K,F,D", [(40, 30, 100, 264), (500, 4, 1001, 520), (300, 5, 12293, 72), (2048, 52, 8195, 264)])
+def test_groups_of_any_size_give_the_same_bits(B, K, F, D, dtype):
+    """One, two, four or eight latents per wavefront, by size: as with whole groups."""
+    print("[case]", B, K, F, D, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(B + D)
+    idx = torch.randint(0, F, (B, K), generator=g, device=DEV)
+    W = torch.randn(F, D, generator=g, device=DEV).to(dtype)
+    v = torch.randn(B, K, generator=g, device=DEV).to(dtype)
+    resid = torch.randn(B, D, generator=g, device=DEV)
+    small, large = (abi.topk_backward(idx, W, v, resid, 1.5, flags=f) for f in (0, _lib.TOPK_BWD_AS_LARGE))
+    torch.cuda.synchronize()
+    assert small[0] == 0 and large[0] == 0
+    assert all(torch.equal(x, y) for x, y in zip(small[1:], large[1:]))
