@@ -1296,16 +1296,23 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
   for (int64_t col0 = 0; col0 < s->D; col0 += slice_w) {
     const int64_t cols = (pl.d_pad - col0) < slice_w ? (pl.d_pad - col0) : slice_w;
     const int tps = static_cast<int>(cols / pl.tile);
-    const int64_t xcd_span = ceil_div(n_groups * tps, 8);
+    // A last tile of less than two thirds of the columns apart from the others (us with it among them / apart, uniform
+    // indices: D=296 of 256-column tiles, B=11147, K=62, F=50975 fp32 227 / 192; D=2304 of 512, B=4096, K=128, F=65536 bf16
+    // 296 / 289; with more columns it fetches its slice into all L2s for little: D=1992, B=2048, K=44, F=32768 bf16 102 / 106).
+    const int64_t last_cols = s->D - (col0 + cols - pl.tile);
+    const int n_full = 3 * last_cols < 2 * static_cast<int64_t>(pl.tile) ? tps - 1 : tps;
+    const int64_t xcd_span = ceil_div(n_groups * n_full, 8);
+    const int64_t last_span = n_full < tps ? ceil_div(n_groups, 8) : 0;
     const unsigned n_long = kLongBlocks * static_cast<unsigned>(tps);
     const size_t resid_bytes =
         static_cast<size_t>(s->B) * static_cast<size_t>(pl.resid_ld) * sizeof(typename Traits<RT>::store_t);
     constexpr int kEndTiles = VEC / EV;  // tiles of the long latents' second step per tile
     hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC, EV>),
-                       dim3(n_long + static_cast<unsigned>(xcd_span * 8)),
+                       dim3(n_long + static_cast<unsigned>((xcd_span + last_span) * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
-                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, per_wave, tps,
+                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, n_full,
+                       per_wave, tps,
                        static_cast<int>(col0), sw, s->F, K, D, pl.resid_ld, static_cast<uint32_t>(resid_bytes));
     if (col0 + slice_w < s->D) {
       hipLaunchKernelGGL((seg_reduce_long_finalize_kernel<GT, EV, 8>), dim3(256), dim3(kBlock), 0, st,

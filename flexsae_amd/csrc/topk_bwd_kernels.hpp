@@ -331,10 +331,11 @@ __device__ __forceinline__ void topk_short_latents(
 // dvals shares, leaves its dW contribution in partial[chunk, slice column] (fp32) for
 // seg_reduce_long_finalize_kernel (next launch).  They come first so hot latents start at once.
 // Remaining blocks: one wavefront per (tile of the slice, group of latents), see topk_short_latents; tile = 64*VEC columns,
-// lane l owning VEC consecutive columns.  The n_groups blocks of each of the tps tiles, tiles outermost, are cut into eight runs of
-// xcd_span, one per XCD (blocks go round the XCDs): an L2 holds the B x tile slice of resid that its own wavefronts
-// gather from, instead of every L2 fetching every slice (B=2048, K=256, F=131072, D=1024 fp32 327 -> 301 us for the whole
-// backward, K=64 249 -> 192; bf16 the same either way).
+// lane l owning VEC consecutive columns.  The n_groups blocks of each of the first n_full tiles, tiles
+// outermost, are cut into eight runs of xcd_span, one per XCD (blocks go round the XCDs): an L2 holds the B x tile slice of
+// resid that its own wavefronts gather from, instead of every L2 fetching every slice (B=2048, K=256, F=131072, D=1024 fp32
+// 327 -> 301 us for the whole backward, K=64 249 -> 192; bf16 the same either way).  A last tile with few columns follows in
+// eight runs of its own: among the others' it leaves the XCDs that hold it idle for much of the time.
 // dW[f, tile] is written exactly once, in the gradient's final dtype; latents without pairs
 // get zeros.
 // resid_ld: elements from one row of resid to the next.  EV: elements of a vector that divides the rows of W and dW.
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
-    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int per_wave, int tps, int col0, int slice_w, int64_t F, int K,
+    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int n_full, int per_wave, int tps, int col0, int slice_w, int64_t F, int K,
     int D, int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
@@ -354,9 +355,11 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
   __shared__ LatentPiece<WT, GT, VEC> pieces[256 / kWave][L * kWave];
   if (blockIdx.x >= n_long_blocks) {
     const int64_t i = (blockIdx.x - n_long_blocks) >> 3;
-    const int64_t item = (blockIdx.x & 7) * xcd_span + i;
+    const bool in_full = i < xcd_span;
+    const int64_t item = in_full ? (blockIdx.x & 7) * xcd_span + i
+                                 : n_groups * n_full + (blockIdx.x & 7) * ((n_groups + 7) >> 3) + i - xcd_span;
     const int t = static_cast<int>(item / n_groups);
-    if (i >= xcd_span || t >= tps) return;
+    if (t >= (in_full ? n_full : tps)) return;
     const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * per_wave;
     if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
