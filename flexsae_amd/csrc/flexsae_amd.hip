@@ -1273,6 +1273,18 @@ int latents_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl, int most) {
   return n;
 }
 
+// The kernel of one latent per wavefront (topk_short_latent): 54 to 73 registers against 92 to 117 leave two or three more
+// wavefronts per SIMD to gather with, and a head per latent, which a group pays once.  Times as fast as the groups, geometric
+// mean over 300 shapes, uniform and skewed indices: 12 to 72 pairs per latent 1.04 and 1.04 (B=8192, K=63, F=16384, D=296
+// fp16 126 -> 117 us), with more than 140000 latents in all tiles 0.96; 8 to 12 1.04 and 1.03 with fewer than 65536, 0.99 and
+// 0.97 with more; 4 to 8 0.98 and 0.97; below 4 0.87 and 0.91; above 72 (nearly all pairs in chunks of long latents) 1.00 and
+// 1.01.
+bool one_latent_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl) {
+  const int64_t pairs = s->B * s->K;
+  const int64_t latents = s->F * (pl.d_pad / pl.tile);  // of all tiles
+  return !pl.whole_groups && latents < 140000 && pairs >= (latents < 65536 ? 8 : 12) * s->F && pairs < 72 * s->F;
+}
+
 size_t topk_bwd_bytes(const TopkBwdPlan &p, int64_t slice_w) {
   return p.fixed_bytes + round_up(p.n_partial_rows * static_cast<size_t>(slice_w) * 4, kAlign);
 }
@@ -1287,7 +1299,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   const int64_t n_pairs = static_cast<int64_t>(pl.n_pairs);
-  const int per_wave = pl.whole_groups ? topk_group<WT, GT, VEC>() : latents_per_wave(s, pl, topk_group<WT, GT, VEC>());
+  const bool one = EV == VEC && one_latent_per_wave(s, pl);
+  const int per_wave = one ? 1 : pl.whole_groups ? topk_group<WT, GT, VEC>() : latents_per_wave(s, pl, topk_group<WT, GT, VEC>());
   const int64_t n_groups = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock) * per_wave);
   // a launch holds fewer than 2^32 threads, 2^24 blocks: narrower slices where all tiles would be more
   const int64_t most_tiles = (int64_t{1} << 23) / (n_groups + kLongBlocks);
@@ -1307,7 +1320,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
     const size_t resid_bytes =
         static_cast<size_t>(s->B) * static_cast<size_t>(pl.resid_ld) * sizeof(typename Traits<RT>::store_t);
     constexpr int kEndTiles = VEC / EV;  // tiles of the long latents' second step per tile
-    hipLaunchKernelGGL((topk_bwd_kernel<WT, GT, RT, VEC, EV>),
+    const auto kernel = one ? topk_bwd_kernel<WT, GT, RT, VEC, EV, EV == VEC> : topk_bwd_kernel<WT, GT, RT, VEC, EV, false>;
+    hipLaunchKernelGGL(kernel,
                        dim3(n_long + static_cast<unsigned>((xcd_span + last_span) * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,

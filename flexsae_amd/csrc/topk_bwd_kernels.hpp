@@ -326,11 +326,147 @@ __device__ __forceinline__ void topk_short_latents(
   }
 }
 
+// One short latent (1 to kSegChunk pairs) for one tile, the fewer registers where latents have many pairs (which sizes take
+// it: one_latent_per_wave): the pair records of the latent are one
+// contiguous load, the residual rows are gathered through a buffer descriptor (no vector ALU work
+// for addresses) eight at a time (with the next eight already requested when registers allow),
+// and each group of eight shares one transposed wave reduction for the dvals dot products.  Inside a
+// group, rows are requested and consumed two at a time under one uniform test, so a latent with
+// nine pairs costs ten rows, not sixteen (a test per row costs more than it saves; the odd slot
+// past the end re-reads the last row, a cache hit, with a val of zero).  With bf16 weights and a
+// bf16 residual copy the products run on packed pairs (dot2) without unpacking.
+template <typename WT, typename GT, typename RT, int VEC>
+__device__ __forceinline__ void topk_short_latent(
+    const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight, int vals_dtype,
+    const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
+    float *__restrict__ dv_tile, int64_t f, uint32_t b0, int n, int d0, int D) {
+  using S = typename Traits<RT>::store_t;
+  const int lane = lane_id();
+  const bool active = d0 < D;
+  const uint32_t lane_off = static_cast<uint32_t>(active ? d0 : 0) * sizeof(S);
+  constexpr bool kDot2 = Traits<WT>::dtype == FLEXSAE_BF16 && Traits<RT>::dtype == FLEXSAE_BF16 && VEC % 2 == 0;
+  const bool late_scale = kDot2 && vals_dtype == FLEXSAE_BF16;  // vals enter the dot2 as they are
+
+  const raw_vec_t<WT, VEC> wraw = load_raw<WT, VEC, FLEXSAE_TOPK_NT>(weight, f * D + (active ? d0 : 0));
+  // lanes past the end hold row 0 and a val of zero
+  const vec_t<uint32_t, 2> bv = lane < n ? __builtin_nontemporal_load(slot_bv + b0 + lane) : vec_t<uint32_t, 2>{0u, 0u};
+  const int my_b = static_cast<int>(bv[0]);
+  const uint32_t vbits = bv[1];
+
+  // two groups of eight rows in flight, or one when a group alone takes 32 registers: the
+  // kernel gains more from another wavefront per SIMD than from the deeper prefetch
+  constexpr int kRowsPerTest = 2;  // rows of a group of eight that share one uniform "are there rows left" test
+  constexpr bool kTwoGroups = sizeof(raw_vec_t<RT, VEC>) * 8 <= 64;
+  raw_vec_t<RT, VEC> buf_a[8], buf_b[kTwoGroups ? 8 : 1];
+  auto issue = [&](raw_vec_t<RT, VEC>(&buf)[8], int j) {
+#pragma unroll
+    for (int h = 0; h < 8; h += kRowsPerTest) {
+      if (h == 0 || j + h < n) {  // uniform: the second half of a group only when it has rows
+#pragma unroll
+        for (int u = h; u < h + kRowsPerTest; ++u) {
+          const int jj = (j + u) < n ? (j + u) : (n - 1);
+          buf[u] = gather_raw<RT, VEC>(rows_src, lane_off, static_cast<uint32_t>(bcast_i32(my_b, jj)) * row_stride);
+        }
+      }
+    }
+  };
+  issue(buf_a, 0);
+  if constexpr (kTwoGroups) {
+    if (n > 8) issue(buf_b, 8);
+  }
+
+  float w[VEC], acc[VEC];
+  unpack_raw<WT, VEC>(wraw, w);
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) {
+    acc[i] = 0.f;
+    if (!active) w[i] = 0.f;
+  }
+  uint32_t ww[(VEC + 1) / 2] = {};  // the W piece as packed pairs (dot2 path)
+  if constexpr (kDot2) {
+    __builtin_memcpy(ww, &wraw, sizeof(raw_vec_t<WT, VEC>));
+#pragma unroll
+    for (int i = 0; i < VEC / 2; ++i)
+      if (!active) ww[i] = 0u;
+  }
+  const float v = __uint_as_float(vbits) * (late_scale ? 1.f : scale);
+  float my_dot = 0.f;
+  auto consume = [&](const raw_vec_t<RT, VEC>(&rows)[8], int j) {  // slots j .. j+7 of the latent
+    float dots[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) dots[u] = 0.f;
+#pragma unroll
+    for (int h = 0; h < 8; h += kRowsPerTest) {
+      if (h != 0 && j + h >= n) continue;  // uniform
+#pragma unroll
+      for (int u = h; u < h + kRowsPerTest; ++u) {
+        float dot = 0.f;
+        if constexpr (kDot2) {
+          uint32_t xw[VEC / 2];
+          __builtin_memcpy(xw, &rows[u], sizeof(xw));
+#pragma unroll
+          for (int i = 0; i < VEC / 2; ++i) dot = dot2_bf16(xw[i], ww[i], dot);
+          if (late_scale) {  // uniform
+            // a bf16 val widened to fp32 keeps its 16 bits in the upper half
+            const uint32_t v_hi = static_cast<uint32_t>(bcast_i32(static_cast<int>(vbits), j + u));
+            const uint32_t v_lo = v_hi >> 16;
+#pragma unroll
+            for (int i = 0; i < VEC / 2; ++i) {
+              acc[2 * i] = dot2_bf16(xw[i], v_lo, acc[2 * i]);
+              acc[2 * i + 1] = dot2_bf16(xw[i], v_hi, acc[2 * i + 1]);
+            }
+          } else {
+            float x[VEC];
+            unpack_raw<RT, VEC>(rows[u], x);
+            const float vj = bcast_f32(v, j + u);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) acc[i] = fmaf(vj, x[i], acc[i]);
+          }
+        } else {
+          float x[VEC];
+          unpack_raw<RT, VEC>(rows[u], x);
+          const float vj = bcast_f32(v, j + u);
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            acc[i] = fmaf(vj, x[i], acc[i]);
+            dot = fmaf(x[i], w[i], dot);
+          }
+        }
+        dots[u] = dot;
+      }
+    }
+    const float tot = wave_sum8_transposed(dots);  // lane L: total of slot j + (L & 7)
+    if ((lane >> 3) == (j >> 3)) my_dot = tot;
+  };
+  if constexpr (kTwoGroups) {
+    for (int j = 0; j < n; j += 16) {
+      consume(buf_a, j);
+      if (j + 16 < n) issue(buf_a, j + 16);
+      if (j + 8 < n) {
+        consume(buf_b, j + 8);
+        if (j + 24 < n) issue(buf_b, j + 24);
+      }
+    }
+  } else {
+    for (int j = 0; j < n; j += 8) {
+      consume(buf_a, j);
+      if (j + 8 < n) issue(buf_a, j + 8);
+    }
+  }
+  if (late_scale) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) acc[i] *= scale;
+  }
+  if (active) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f * D + d0, acc);
+  if (lane < n) dv_tile[b0 + lane] = my_dot * scale;
+}
+
 // TopK backward of one slice.  scale = grad_out * 2/(B*D).
 // Blocks [0, n_long_blocks), a multiple of eight: long latents, one wavefront per (64-pair chunk, tile): stores its
 // dvals shares, leaves its dW contribution in partial[chunk, slice column] (fp32) for
 // seg_reduce_long_finalize_kernel (next launch).  They come first so hot latents start at once.
-// Remaining blocks: one wavefront per (tile of the slice, group of latents), see topk_short_latents; tile = 64*VEC columns,
+// Remaining blocks: one wavefront per (tile of the slice, group of per_wave latents), see topk_short_latents, or with ONE per
+// (tile, latent), see topk_short_latent; tile = 64*VEC columns,
 // lane l owning VEC consecutive columns.  The n_groups blocks of each of the first n_full tiles, tiles
 // outermost, are cut into eight runs of xcd_span, one per XCD (blocks go round the XCDs): an L2 holds the B x tile slice of
 // resid that its own wavefronts gather from, instead of every L2 fetching every slice (B=2048, K=256, F=131072, D=1024 fp32
@@ -339,7 +475,7 @@ __device__ __forceinline__ void topk_short_latents(
 // dW[f, tile] is written exactly once, in the gradient's final dtype; latents without pairs
 // get zeros.
 // resid_ld: elements from one row of resid to the next.  EV: elements of a vector that divides the rows of W and dW.
-template <typename WT, typename GT, typename RT, int VEC, int EV>
+template <typename WT, typename GT, typename RT, int VEC, int EV, bool ONE>
 __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const uint32_t *__restrict__ begin, const uint32_t *__restrict__ map,
     const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
@@ -351,8 +487,6 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     int D, int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
-  constexpr int L = topk_group<WT, GT, VEC>();
-  __shared__ LatentPiece<WT, GT, VEC> pieces[256 / kWave][L * kWave];
   if (blockIdx.x >= n_long_blocks) {
     const int64_t i = (blockIdx.x - n_long_blocks) >> 3;
     const bool in_full = i < xcd_span;
@@ -363,10 +497,27 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * per_wave;
     if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
-    topk_short_latents<WT, GT, RT, VEC, EV, L>(
-        begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
-        dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F, col0 + t * (kWave * VEC) + lane * VEC, D,
-        pieces[wave_in_block()]);
+    if constexpr (ONE) {
+      const uint32_t b0 = begin[f0];
+      const uint32_t n = begin[f0 + 1] - b0;
+      if (n > static_cast<uint32_t>(kSegChunk)) return;  // chunk role
+      const int d0 = col0 + t * (kWave * VEC) + lane * VEC;
+      if (n == 0) {  // unused latent: zeros
+        const float zero[VEC] = {};
+        if (d0 < D) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f0 * D + d0, zero);
+        return;
+      }
+      topk_short_latent<WT, GT, RT, VEC>(
+          slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
+          dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, b0, static_cast<int>(n), d0, D);
+    } else {
+      constexpr int L = topk_group<WT, GT, VEC>();
+      __shared__ LatentPiece<WT, GT, VEC> pieces[256 / kWave][L * kWave];
+      topk_short_latents<WT, GT, RT, VEC, EV, L>(
+          begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
+          dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F, col0 + t * (kWave * VEC) + lane * VEC, D,
+          pieces[wave_in_block()]);
+    }
     return;
   }
   const uint32_t n_long = long_ctrl[kLongCount];
