@@ -1202,6 +1202,24 @@ struct TopkBwdPlan {
   bool whole_groups;  // as many latents per wavefront as it takes, whatever the size
 };
 
+// Whether a bf16 copy of the residual with padded rows (16 bytes per lane, tiles of 512 columns) beats one whose rows are read
+// in the vectors of `vec` elements that divide them (tiles of 64 * vec), by 740 shapes of both kinds of indices; the backward
+// in us with narrow / padded rows, uniform and skewed:
+//   vec 1, 160 columns and more, or more than 128 and at least 65536 latents: B=4096, K=128, F=65536, D=2305 695 / 374,
+//       834 / 477, D=129 101 / 94, 135 / 134;  B=1024, K=64, F=32768, D=129 44 / 43, 58 / 60
+//   vec 2, more than 256 columns, where the padded tile of the copy (1 KB per row) is no more than 8 MiB, two L2s, or the only
+//       tile: B=8192, K=64, F=262144, D=1026 491 / 440, 551 / 490;  B=12288, K=32, F=16384 187 / 224, 243 / 251
+//   vec 4, the same with 4 MiB (B=8192, K=64, F=16384, D=1028 186 / 239, 237 / 272), and where there is enough to do for half
+//       the wavefronts (B=3072, K=16, F=8192, D=1028 54 / 57, 76 / 79; B=64, K=39, F=32768, D=364 37 / 40, 39 / 41)
+// At the sizes it takes, padded rows are at most 6 % behind (shapes of 40 us, mostly the launches), on average 30 % ahead.
+bool padding_pays(const flexsae_shape *s, int vec) {
+  const int64_t tiles = ceil_div(s->D, kWave * 8);
+  if (vec == 1) return s->D >= 160 || (s->D > 128 && s->F >= 65536);
+  if (s->D <= 256) return false;
+  if (tiles == 1) return vec == 2 || s->B >= 1024;
+  return vec == 2 ? s->B <= 8192 : s->B <= 4096 && s->F * tiles >= 40000;
+}
+
 TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   TopkBwdPlan p;
   // The reference hands its backward the residual gradient in the weight dtype
@@ -1215,12 +1233,9 @@ TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
   p.resid_ld = static_cast<int>(s->D);
   // all-bf16: 16 bytes per lane (512-column tiles) halve the per-tile overheads
   if (FLEXSAE_TOPK_VEC8 && p.resid16 && s->D % 8 == 0) p.vec = p.row_vec = 8;
-  // Rows that eight does not divide: the copy's rows are padded, so that its gathers are as wide (the step, us, with
-  // vectors that divide the row / padded; B=4096, F=65536, K=128: D=2305 1146 / 829, 2306 879 / 759, 2308 756 / 718; K=32:
-  // D=2305 563 / 405, 2306 399 / 346; B=8192, F=262144, K=64, D=1026 687 / 660; B=300, F=400000, K=16, D=4097 3281 / 1812,
-  // D=4098 2253 / 1580; B=16384, F=65536, K=64: D=129 246 / 234, 130 216 / 216).  Not where one narrow tile holds the row:
-  // as many gathers either way, and the wide ones leave most lanes without columns.
-  if (FLEXSAE_TOPK_VEC8 && p.resid16 && p.vec != 8 && s->D > kWave * p.vec) {
+  // Rows that eight does not divide: the copy's rows are padded, so that its gathers are as wide.
+  if (FLEXSAE_TOPK_VEC8 && p.resid16 && p.vec != 8 &&
+      ((flags & FLEXSAE_TOPK_BWD_AS_LARGE) ? s->D > kWave * p.vec : padding_pays(s, p.vec))) {
     p.vec = 8;
     p.resid_ld = static_cast<int>(round_up(static_cast<size_t>(s->D), 8));
   }
