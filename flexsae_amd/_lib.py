@@ -71,6 +71,7 @@ SIGNATURES = {
     "flexsae_status_string": (ctypes.c_char_p, [_int]),
     "flexsae_fwd_workspace_bytes": (_sz, [_shape_p]),
     "flexsae_topk_fwd_workspace_bytes": (_sz, [_shape_p]),
+    "flexsae_topk_fwd_best_workspace_bytes": (_sz, [_shape_p]),
     "flexsae_hier_fwd": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _p]),
     "flexsae_hier_fwd_static": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "flexsae_topk_fwd": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _p]),

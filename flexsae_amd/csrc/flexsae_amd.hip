@@ -242,19 +242,10 @@ struct OrderedPlan {
   size_t steps_bytes;  // (row, val) of every pair, after the loss partials
 };
 
-// By sizes alone; forward_ordered() also asks for rows of whole 16-byte vectors and room for the steps.
-// us without / with the ordering, uniform and skewed (Zipf 1.1) indices:
-//   bf16, K=128  B=4096, D=2304: F=65536 286 / 188, 150 / 149; F=131072 323 / 229, 168 / 164;  B=1024, D=2048, F=32768
-//                63 / 36, 33 / 33;   K=256  B=1024, D=1024, F=65536 65 / 48, 40 / 43;  B=512, D=4096 148 / 114, 73 / 69
-//   bf16, K=64   B=4096, D=2304: F=32768 96 / 76, 68 / 71; F=65536 151 / 116, 70 / 76;  B=16384, D=768 192 / 133, 89 / 96
-//   bf16, K=32   B=4096, D=2304, F=65536 84 / 77, 41 / 48;  B=16384, D=768 107 / 94, 51 / 63
-//   fp32, K=128  B=4096, D=2304, F=65536 553 / 338, 301 / 275;  K=64 286 / 219, 161 / 156;  K=32 156 / 153, 84 / 91;
-//                K=64, B=1024, D=1024, F=65536 36 / 33, 19 / 21;   K=256, B=2048, D=1024, F=131072 275 / 181, 144 / 133
-// So: rows of 64 pairs and more (with fewer, the latents at one position of two rows are too far apart); where the pieces of
-// one tile do not fit an L2 (4 MB; B=4096, K=64, D=2304, F=16384 72 / 71); gathers of a quarter of a GiB and more, half a
-// GiB below 128 steps (the ordering is a launch of 5-6 us); and, like the tiles per XCD that it walks, rows that start on a
-// line and at most 131072 latents (262144: B=8192, K=64, D=4096 614 / 658) and 512 batch rows or more (B=300, K=200,
-// F=40000, D=4096 72 / 65, 38 / 45; B=128, K=256, F=65536, D=2048 25 / 49).
+// What the ordered walk takes (whether it pays: order_pays): 64 to 512 pairs per row and 512 batch rows or more, rows that
+// start on a line, pieces of one tile that do not fit an L2 (4 MB), gathers of 128 MiB and more, half a GiB below 128 pairs per
+// row; forward_ordered() also asks for whole 16-byte vectors and room for the steps.  Fewer than 2^20 latents: a latent and
+// a position in its row fit a dword.
 // 128-byte pieces (16-bit weights, eight rows per wavefront) beat 256-byte ones from more than 2048 rows on (B=4096, K=64,
 // D=2304, F=131072 149 / 161; at B=2048, K=256, D=1024 96 / 87, at B=512 143 / 114).  As many wavefronts per block as
 // leave 32 blocks, one per compute unit of an XCD, for a tile: fp32, K=256, D=4096, F=65536, B=512 blocks of 16 / 8 / 4
@@ -265,7 +256,7 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
   const size_t es = dtype_size(s->weight_dtype);
   const uint64_t row_bytes = static_cast<uint64_t>(s->D) * es;
   const uint64_t F = static_cast<uint64_t>(s->F);
-  if (s->K < 64 || s->K > 512 || s->B < 512 || F > 131072 || row_bytes % 128 != 0) return p;
+  if (s->K < 64 || s->K > 512 || s->B < 512 || F >= (uint64_t{1} << 20) || row_bytes % 128 != 0) return p;
   if (static_cast<uint64_t>(s->B) * s->K * row_bytes < (s->K < 128 ? uint64_t{512} << 20 : uint64_t{128} << 20)) return p;
   const bool narrow = es == 2 && s->B > 2048;
   const uint64_t piece_bytes = narrow ? 128 : 256;
@@ -281,16 +272,47 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
   return p;
 }
 
+// Whether it is the faster walk of such a shape.  Two things decide, and uniform indices gain by them what skewed ones (Zipf
+// 1.1, most of whose gathers hit an L2 either way) lose without them:
+//   reuse   pairs per latent among the rows that an XCD walks at a time (32 compute units of sixteen wavefronts): what a
+//           piece fetched once is used for.  Below 1.25 with 256-byte pieces uniform indices gain nothing, below three with
+//           128-byte ones skewed indices lose 5 to 14 %.
+//   work    the sort is a launch of 5-6 us, and blocks of up to sixteen wavefronts leave a last round that is not full: with
+//           0.88 of the rounds full, 80 pairs per row are enough (75: 0.97 as fast on skewed indices); with less, 2350 MiB
+//           of gathers, or rows of 5632 bytes and K times the gathered MiB of 75 * 1024.
+// us without / with the ordering, uniform and skewed indices:
+//   bf16, 128 B   B=4096, D=2304: K=128, F=65536 286 / 188, 150 / 149; K=256, F=262144 673 / 487, 359 / 315;  K=64, F=131072
+//                 169 / 149, 83 / 90 (not taken);  B=8192, K=192, D=1024, F=262144 449 / 369, 214 / 236 (not taken)
+//   bf16, 256 B   B=2048, D=4096: K=128, F=32768 264 / 149, 127 / 120; K=256, F=262144 604 / 510, 364 / 298;  B=1024, K=128,
+//                 D=2304, F=131072 93 / 96, 43 / 53 and K=256, D=1024, F=65536 65 / 48, 40 / 43 (not taken)
+//   fp32, 256 B   B=2048, D=1024: K=256, F=131072 275 / 181, 144 / 133; K=96, F=65536 100 / 66, 45 / 44; K=64, F=65536 69 / 50,
+//                 32 / 34 (not taken);  B=1024, K=192, D=1152, F=32768 103 / 72, 52 / 59 (not taken)
+// Over 1319 shapes (F 16384 to 1048576, many of them near the lines): of the 578 that it takes 13 are 5 % slower or more on one
+// kind of indices (the most B=512, K=192, D=4096, F=16384 bf16: 89 / 55, 44 / 54); uniform ones are 1.44 times as fast, skewed
+// ones 1.06.
+bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
+  const size_t es = dtype_size(s->weight_dtype);
+  const uint64_t B = static_cast<uint64_t>(s->B), K = static_cast<uint64_t>(s->K), F = static_cast<uint64_t>(s->F);
+  const uint64_t row_bytes = static_cast<uint64_t>(s->D) * es, mib = B * K * row_bytes >> 20;
+  const bool narrow = p.lpr == 8;
+  const uint64_t at_a_time = 32 * 16 * (narrow ? 8 : 4);
+  const uint64_t reused = (B < at_a_time ? B : at_a_time) * K;
+  if (narrow)
+    return (reused >= 3 * F && row_bytes >= 2560 && K * mib >= 200 * 1024) || (reused >= 6 * F && mib >= 2000) ||
+           (reused >= 8 * F && K * mib >= 100 * 1024);
+  if (4 * reused < 5 * F) return false;
+  const int64_t round = 32 * 16 / p.waves;  // blocks of an XCD at a time
+  const bool full = 100 * p.xcd_span >= 88 * round * ceil_div(p.xcd_span, round);
+  return full ? K >= 80 : mib >= 2350 || (row_bytes >= 5632 && K * mib >= 75 * 1024);
+}
+
 void launch_order(const flexsae_shape *s, const int64_t *indices, const void *vals, vec_t<uint32_t, 2> *steps,
                   int *status_flag, hipStream_t st) {
   const int K = static_cast<int>(s->K);
   const int C = K <= 64 ? 1 : K <= 128 ? 2 : K <= 256 ? 4 : 8;
-  // latents that share a key, so that the keys stay below the one of the elements past a row's end
-  int shift = 0;
-  while ((static_cast<uint64_t>(s->F - 1) >> shift) + 1 >= (uint64_t{1} << (32 - order_pos_bits(C)))) ++shift;
   const dim3 grid(static_cast<unsigned>(ceil_div(s->B, kWavesPerBlock)));
   const auto kernel = C == 1 ? topk_order_kernel<1> : C == 2 ? topk_order_kernel<2> : C == 4 ? topk_order_kernel<4> : topk_order_kernel<8>;
-  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, indices, vals, s->vals_dtype, s->B, K, s->F, shift, steps, status_flag);
+  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, indices, vals, s->vals_dtype, s->B, K, s->F, steps, status_flag);
 }
 
 template <typename WT>
@@ -321,7 +343,7 @@ void launch_ordered_fwd(const flexsae_shape *s, const OrderedPlan &p, const vec_
 #undef FLEXSAE_ORDERED
 }
 
-// The TopK forward in latent order, where it pays, the rows allow it and the workspace has room behind the partials
+// The TopK forward in latent order, where the shape and the rows allow it and the workspace has room behind the partials
 // (flexsae_topk_fwd_workspace_bytes).  Returns the number of loss partials, 0 if nothing was launched.
 int64_t forward_ordered(const flexsae_shape *s, const int64_t *indices, const void *weight, const void *vals,
                         const void *bias, const void *target, float *resid, void *workspace, size_t workspace_bytes,
@@ -1446,6 +1468,13 @@ size_t flexsae_fwd_workspace_bytes(const flexsae_shape *s) {
 size_t flexsae_topk_fwd_workspace_bytes(const flexsae_shape *s) {
   const size_t base = flexsae_fwd_workspace_bytes(s);
   return base == 0 ? 0 : base + plan_ordered(s).steps_bytes;
+}
+
+size_t flexsae_topk_fwd_best_workspace_bytes(const flexsae_shape *s) {
+  const size_t base = flexsae_fwd_workspace_bytes(s);
+  if (base == 0) return 0;
+  const OrderedPlan p = plan_ordered(s);
+  return base + (p.waves != 0 && order_pays(s, p) ? p.steps_bytes : 0);
 }
 
 int flexsae_hier_fwd(const flexsae_shape *shape, const int64_t *indices, const void *weight,

@@ -211,13 +211,12 @@ __global__ __launch_bounds__(256) void sae_fwd_kernel(
 
 // (row of the weight matrix, val bits) of every pair, each row's pairs by ascending latent (and by position where two are
 // equal: the order, and so every sum, is the same on every run).  One wavefront per row of at most 64 * C pairs: a bitonic
-// sort of one key per pair, the latent's upper bits over the pair's position.  `shift` latent bits are left out where both
-// do not fit a dword, which costs locality within that few latents and nothing else.  An index outside [0, F) becomes
+// sort of one key per pair, the latent over the pair's position (fewer than 2^20 latents).  An index outside [0, F) becomes
 // latent 0 with a val of zero, as in the kernels that read indices themselves.  5-6 us for half a million pairs, most of it
 // the launch (ranks by counting, a comparison per pair of pairs: 9 us at K=128, 19 at K=256).
 template <int C>
 __global__ __launch_bounds__(256) void topk_order_kernel(const int64_t *__restrict__ indices, const void *__restrict__ vals,
-                                                         int vals_dtype, int64_t B, int K, int64_t F, int shift,
+                                                         int vals_dtype, int64_t B, int K, int64_t F,
                                                          vec_t<uint32_t, 2> *__restrict__ steps, int *status_flag) {
   constexpr int N = kWave * C;
   constexpr int kPosBits = order_pos_bits(C);
@@ -250,8 +249,8 @@ __global__ __launch_bounds__(256) void topk_order_kernel(const int64_t *__restri
     s[0] = static_cast<uint32_t>(idx[c]);
     s[1] = __float_as_uint(v);
     mine[k] = s;
-    // elements past the row's end sort behind all others (the host leaves the largest key free)
-    key[c] = k < K ? (static_cast<uint32_t>(idx[c]) >> shift) << kPosBits | static_cast<uint32_t>(k) : 0xffffffffu;
+    // elements past the row's end sort behind all others
+    key[c] = k < K ? static_cast<uint32_t>(idx[c]) << kPosBits | static_cast<uint32_t>(k) : 0xffffffffu;
   }
 #pragma unroll
   for (int size = 2; size <= N; size *= 2) {
@@ -282,7 +281,7 @@ __global__ __launch_bounds__(256) void topk_order_kernel(const int64_t *__restri
 }
 
 // sae_fwd_kernel for rows in latent order: NW wavefronts per block, the tiles cut into runs, one per XCD.
-// At most four wavefronts per SIMD and eight gathers in flight (16-byte lanes): with more of either the wavefronts of a
+// At most four wavefronts per SIMD and eight gathers in flight, sixteen of 256-byte pieces (16-byte lanes): with more of either the wavefronts of a
 // tile drift further apart than the L2 covers, and those of the next tile join them.  What bounds it: the L2s, at 13-14 of
 // the 18 TB/s they give to row gathers, and the misses beside them (5-6 TB/s).  Ordering included: B=4096, K=128, F=65536,
 // D=2304 bf16 286 -> 188 us (128-byte pieces), B=2048, K=256, F=131072, D=1024 fp32 275 -> 181 us (256-byte pieces).

@@ -150,7 +150,7 @@ def _forward(entry: str, indices, weight, vals, bias, target) -> Tuple[Tensor, T
     dev = weight.device
     with _on_device(dev):
         shape = _shape(B, K, F, D, weight, vals, bias.dtype, target.dtype)
-        ws_bytes = (lib.flexsae_topk_fwd_workspace_bytes if entry == "flexsae_topk_fwd"
+        ws_bytes = (lib.flexsae_topk_fwd_best_workspace_bytes if entry == "flexsae_topk_fwd"
                     else lib.flexsae_fwd_workspace_bytes)(ctypes.byref(shape))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)

@@ -132,10 +132,14 @@ const char *flexsae_status_string(int status);
 /* Bytes of workspace the two forward entry points need for `shape`. */
 size_t flexsae_fwd_workspace_bytes(const flexsae_shape *shape);
 
-/* Bytes of workspace with which flexsae_topk_fwd walks the pairs of every row by ascending latent where that is faster:
+/* Bytes of workspace with which flexsae_topk_fwd walks the pairs of every row by ascending latent where it can:
  * flexsae_fwd_workspace_bytes, plus eight bytes per pair for such shapes.  With the smaller workspace it walks them in
  * the order given: the same sums in another order, equal to fp32 rounding. */
 size_t flexsae_topk_fwd_workspace_bytes(const flexsae_shape *shape);
+
+/* The one of the two with which flexsae_topk_fwd is the faster one: by ascending latent where uniform indices gain by it and
+ * skewed ones (a few latents in most rows) do not lose. */
+size_t flexsae_topk_fwd_best_workspace_bytes(const flexsae_shape *shape);
 
 /*
  * HierarchicalTopK forward.

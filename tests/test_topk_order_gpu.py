@@ -92,3 +92,43 @@ def test_infinite_weights_stay_out_of_other_steps():
     assert torch.isposinf(resid[5]).all()
     keep = torch.arange(B, device=DEV) != 5
     assert torch.isfinite(resid[keep]).all()
+
+
+@pytest.mark.parametrize("shape,dtype,pays", [
+    ((4096, 128, 65536, 2304), torch.bfloat16, True), ((4096, 256, 262144, 2304), torch.bfloat16, True),
+    ((4096, 64, 131072, 2304), torch.bfloat16, False),
+    ((8192, 192, 262144, 1024), torch.bfloat16, False), ((1024, 256, 65536, 1024), torch.bfloat16, False),
+    ((1024, 128, 131072, 2304), torch.bfloat16, False), ((2048, 256, 262144, 4096), torch.float16, True),
+    ((2048, 256, 131072, 1024), torch.float32, True), ((2048, 64, 65536, 1024), torch.float32, False),
+    ((2048, 96, 65536, 1024), torch.float32, True), ((1024, 192, 32768, 1152), torch.float32, False),
+    ((2048, 192, 524288, 1024), torch.float32, False), ((4096, 512, (1 << 20) - 1, 2304), torch.bfloat16, False),
+    ((300, 128, 65536, 2304), torch.bfloat16, False)], ids=str)
+def test_which_shapes_are_walked_in_latent_order(shape, dtype, pays):
+    lib = _lib.load()
+    sh = ctypes.byref(_lib.Shape(*shape, *[abi.DT[dtype]] * 4))
+    small, large = lib.flexsae_fwd_workspace_bytes(sh), lib.flexsae_topk_fwd_workspace_bytes(sh)
+    assert lib.flexsae_topk_fwd_best_workspace_bytes(sh) == (large if pays else small)
+    assert (large > small) == (shape[0] >= 512)
+
+
+def test_more_latents_than_seventeen_bits():
+    """Keys of twenty latent bits over nine position bits: the last latents come last."""
+    B, K, F, D = 512, 500, (1 << 20) - 1, 160
+    g = torch.Generator(device=DEV).manual_seed(9)
+    idx = torch.randint(F - 4000, F, (B, K), generator=g, device=DEV)
+    W = torch.zeros(F, D, device=DEV)
+    W[F - 4000:] = torch.randn(4000, D, generator=g, device=DEV)
+    v = torch.randn(B, K, generator=g, device=DEV)
+    b, t = torch.randn(D, generator=g, device=DEV), torch.randn(B, D, generator=g, device=DEV)
+    sh = ctypes.byref(abi.shape_of(idx, W, v, b.dtype, t.dtype))
+    large = _lib.load().flexsae_topk_fwd_workspace_bytes(sh)
+    assert large >= 8 * B * K
+    _, resid = _forward(large, idx, W, v, b, t)
+    at, order = torch.sort(idx, dim=1, stable=True)
+    want = (b - t).double()
+    size = b.double().abs() + t.double().abs()
+    for k in range(K):
+        term = W[at[:, k]].double() * v.gather(1, order[:, k:k + 1]).double()
+        want += term
+        size += term.abs()
+    assert ((resid.double() - want).abs() <= (K + 2) * 2.0 ** -24 * size).all()
