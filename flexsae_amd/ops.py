@@ -653,11 +653,12 @@ def _train_ragged(weight: Tensor, K: int) -> bool:
 def _ragged_pays(weight: Tensor, B: int, K: int) -> bool:
     """Whether the training step is the faster one for such rows.  Against forward and sweep, uniform and Zipf:
     bf16, D = 2306, B = 1662, F = 97114: K = 16 1.19 and 1.17 times as fast, K = 50 1.23 and 1.11, K = 128 1.21 and 1.15,
-    K = 256 1.17 and 1.15 (fp32 1.11 to 1.30).  Not with 129 to 255 steps (K = 160 and 200 0.80 to 0.83, B = 1777, F = 24571
-    0.73 to 0.82; fp32 0.77 to 1.0), and for fp16 weights, whose unit gradient is written in fp32 and scaled in a pass of its
-    own, from six pairs per latent on (B = 1777, F = 24571, K = 64 1.02 and 0.94, K = 100 1.06 and 1.06; B = 6000, F = 8192
-    1.1; B = 300, F = 65536, K = 16 to 64 0.84 to 0.97)."""
-    if 128 < K < 256:
+    K = 256 1.17 and 1.15 (fp32 1.11 to 1.30).  Not with 129 to 255 steps where the weight takes a gradient (K = 160 and 200
+    0.80 to 0.83, B = 1777, F = 24571 0.73 to 0.82; fp32 0.77 to 1.0; without, D = 2306, B = 300, F = 65536, K = 176 1.44 bf16,
+    1.60 fp16, 1.56 fp32; D = 1538, B = 1777, F = 24571 0.96 to 1.0, 1.3, 1.1 to 1.2), and for fp16 weights, whose unit
+    gradient is written in fp32 and scaled in a pass of its own, from six pairs per latent on (B = 1777, F = 24571, K = 64 1.02
+    and 0.94, K = 100 1.06 and 1.06; B = 6000, F = 8192 1.1; B = 300, F = 65536, K = 16 to 64 0.84 to 0.97)."""
+    if not _step_pays(weight, K):
         return False
     return weight.dtype != torch.float16 or not weight.requires_grad or B * K > 6 * weight.shape[0]
 
@@ -669,6 +670,24 @@ def _step_pays(weight: Tensor, K: int) -> bool:
     to 0.81; B = 1662, F = 97114 0.79 to 0.88, 0.86 to 0.91, 0.85 to 1.0; B = 300, F = 65536 0.80 to 1.09, 0.74 to 1.04,
     0.93 to 1.02; K = 128 and 256 1.1 to 1.3."""
     return not 128 < K < 256 or not weight.requires_grad
+
+
+def _one_gather_pays(weight: Tensor, B: int, K: int) -> bool:
+    """Where the training step is the faster one with 129 to 255 steps all the same.  Time of forward and sweep over that of the
+    training step, uniform and Zipf, over 634 shapes: 1.09 and 1.07 on average where this says so, 0.89 and 0.84 elsewhere.
+    Small steps of 16-bit weights are bound by the host, and forward and sweep are more launches (B = 512, K = 160, F = 16384,
+    D = 512 bf16 184 and 164 us; not where two pairs per latent or fewer are measured for the list of latents, which costs the
+    step as much).  Weights of several times the memory-side cache of which few latents repeat come out of memory with every
+    gather (B = 412, K = 150, F = 478747, D = 4944 bf16 2037 and 1424 us, Zipf 1847 and 1490; B = 488, K = 254, F = 407482,
+    D = 1632 fp32 1257 and 986, 1209 and 1043; B = 182, K = 200, F = 221872, D = 5240 fp16 1183 and 1058, 1118 and 975)."""
+    F, D = weight.shape
+    pairs, es = B * K, weight.element_size()
+    gathered, size = pairs * D * es, F * D * es
+    if weight.dtype == torch.float32:
+        return pairs <= 2 * F and size >= 600 << 20 and gathered >= 200 << 20
+    if pairs > 2 * F:
+        return gathered <= (128 if weight.dtype == torch.bfloat16 else 64) << 20
+    return pairs <= F and size >= 400 << 20 if weight.dtype == torch.bfloat16 else 5 * pairs <= 2 * F and size >= 1500 << 20
 
 
 def _stage_fits(indices: Tensor, weight: Tensor) -> bool:
@@ -1286,7 +1305,7 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
             return _HierTrainStaged.apply(indices, weight, vals, bias, target)
         # (fp16 weights: the step's unit-gradient dW is fp32, of magnitude 2/(B*K*D), and is scaled by the
         # upstream gradient before its only rounding, like reference hierarchical_kernels.py:294-299)
-        if _hier_scratch_bytes != 0 and _step_pays(weight, indices.shape[1]):
+        if _hier_scratch_bytes != 0 and (_step_pays(weight, indices.shape[1]) or _one_gather_pays(weight, *indices.shape)):
             B, K = indices.shape
             F, D = weight.shape
             hot = bool(weight.requires_grad) and _use_hot_latents(B, K, F, D, weight.dtype, weight.device,

@@ -75,6 +75,7 @@ def test_steps_between_the_kernels(needs, K, D, dtype, monkeypatch):
     """129 to 255 steps go by forward and sweep where the weight takes a gradient: the training step's gradients."""
     print("[case]", needs, K, D, dtype, flush=True)
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(70, K, 500, D, dtype, seed=K + D))
+    monkeypatch.setattr(flex.ops, "_one_gather_pays", lambda *_: False)  # (whatever is faster)
     grads = []
     for forced in (False, True):
         if forced:
@@ -88,3 +89,24 @@ def test_steps_between_the_kernels(needs, K, D, dtype, monkeypatch):
     assert rel_err(grads[0][0].cpu(), grads[1][0].cpu()) < 1e-6  # other partial sums, all beyond a column in double
     for x, y in zip(grads[0][1:], grads[1][1:]):
         assert (x is None and y is None) or torch.equal(x, y)
+
+
+def test_which_steps_between_the_kernels_gather_once():
+    def pays(dtype, B, K, F, D):
+        return flex.ops._one_gather_pays(torch.empty(F, D, dtype=dtype, device="meta", requires_grad=True), B, K)
+
+    bf16, fp16, fp32 = torch.bfloat16, torch.float16, torch.float32
+    assert pays(bf16, 512, 160, 16384, 512) and pays(fp16, 192, 160, 8192, 512) and not pays(fp32, 512, 160, 16384, 512)
+    assert not pays(bf16, 2048, 160, 65536, 1024) and not pays(fp16, 224, 168, 17816, 1160) and not pays(bf16, 64, 160, 8192, 512)
+    assert pays(bf16, 412, 150, 478747, 4944) and pays(fp32, 488, 254, 407482, 1632) and pays(fp16, 182, 200, 221872, 5240)
+    assert not pays(bf16, 2734, 168, 233249, 1768) and not pays(fp32, 200, 150, 202656, 736) and not pays(fp16, 531, 168, 85672, 7264)
+
+
+@pytest.mark.parametrize("D", [128, 130])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+def test_frozen_weights_gather_once(dtype, D):
+    """129 to 255 steps without a weight gradient take the training step, whether or not vectors of four divide the rows."""
+    W = torch.empty(500, D, dtype=dtype, device="meta")
+    assert flex.ops._step_pays(W, 150) and flex.ops._ragged_pays(W, 70, 150)
+    W.requires_grad_()
+    assert not flex.ops._step_pays(W, 150) and not flex.ops._ragged_pays(W, 70, 150)
