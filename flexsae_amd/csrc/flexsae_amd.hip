@@ -278,8 +278,9 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
 //           piece fetched once is used for.  Below 1.25 with 256-byte pieces uniform indices gain nothing, below three with
 //           128-byte ones skewed indices lose 5 to 14 %.
 //   work    the sort is a launch of 5-6 us, and blocks of up to sixteen wavefronts leave a last round that is not full: with
-//           0.88 of the rounds full, 80 pairs per row are enough (75: 0.97 as fast on skewed indices); with less, 2350 MiB
-//           of gathers, or rows of 5632 bytes and K times the gathered MiB of 75 * 1024.
+//           0.88 of the rounds full, 80 pairs per row or 2500 MiB of gathers are enough; with less, 2350 MiB, or rows of 5632
+//           bytes and K times the gathered MiB of 75 * 1024.  128-byte pieces, whose waves last longer, by the reuse alone:
+//           1500 MiB with five, K times the MiB of 100 * 1024 with seven, of 150 * 1024 and rows of 2560 bytes with three.
 // us without / with the ordering, uniform and skewed indices:
 //   bf16, 128 B   B=4096, D=2304: K=128, F=65536 286 / 188, 150 / 149; K=256, F=262144 673 / 487, 359 / 315;  K=64, F=131072
 //                 169 / 149, 83 / 90 (not taken);  B=8192, K=192, D=1024, F=262144 449 / 369, 214 / 236 (not taken)
@@ -287,8 +288,8 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
 //                 D=2304, F=131072 93 / 96, 43 / 53 and K=256, D=1024, F=65536 65 / 48, 40 / 43 (not taken)
 //   fp32, 256 B   B=2048, D=1024: K=256, F=131072 275 / 181, 144 / 133; K=96, F=65536 100 / 66, 45 / 44; K=64, F=65536 69 / 50,
 //                 32 / 34 (not taken);  B=1024, K=192, D=1152, F=32768 103 / 72, 52 / 59 (not taken)
-// Over 1319 shapes (F 16384 to 1048576, many of them near the lines): of the 578 that it takes 13 are 5 % slower or more on one
-// kind of indices (the most B=512, K=192, D=4096, F=16384 bf16: 89 / 55, 44 / 54); uniform ones are 1.44 times as fast, skewed
+// Over 1319 shapes (F 16384 to 1048576, many of them near the lines): of the 609 that it takes 22 are 5 % slower or more on one
+// kind of indices (the most B=512, K=192, D=4096, F=16384 bf16: 89 / 55, 44 / 54); uniform ones are 1.43 times as fast, skewed
 // ones 1.06.
 bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
   const size_t es = dtype_size(s->weight_dtype);
@@ -298,12 +299,12 @@ bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
   const uint64_t at_a_time = 32 * 16 * (narrow ? 8 : 4);
   const uint64_t reused = (B < at_a_time ? B : at_a_time) * K;
   if (narrow)
-    return (reused >= 3 * F && row_bytes >= 2560 && K * mib >= 200 * 1024) || (reused >= 6 * F && mib >= 2000) ||
-           (reused >= 8 * F && K * mib >= 100 * 1024);
+    return (reused >= 3 * F && row_bytes >= 2560 && K * mib >= 150 * 1024) || (reused >= 5 * F && mib >= 1500) ||
+           (reused >= 7 * F && K * mib >= 100 * 1024);
   if (4 * reused < 5 * F) return false;
   const int64_t round = 32 * 16 / p.waves;  // blocks of an XCD at a time
   const bool full = 100 * p.xcd_span >= 88 * round * ceil_div(p.xcd_span, round);
-  return full ? K >= 80 : mib >= 2350 || (row_bytes >= 5632 && K * mib >= 75 * 1024);
+  return full ? K >= 80 || mib >= 2500 : mib >= 2350 || (row_bytes >= 5632 && K * mib >= 75 * 1024);
 }
 
 void launch_order(const flexsae_shape *s, const int64_t *indices, const void *vals, vec_t<uint32_t, 2> *steps,
