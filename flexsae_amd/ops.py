@@ -112,9 +112,13 @@ def _shape(B, K, F, D, weight: Tensor, vals: Tensor, bias_dtype, target_dtype) -
 
 def _prep(t: Tensor) -> Tensor:
     """Contiguous and 16-byte aligned, as the vector accesses of the kernels need: a view into a
-    larger buffer that starts at an odd element (``flat[1:1 + D]``) is copied."""
+    larger buffer that starts at an odd element (``flat[1:1 + D]``) is copied.  A zero tensor, which
+    has no memory, gets some."""
     t = t.contiguous()
-    return t.clone() if t.data_ptr() % 16 else t
+    at = t.data_ptr()
+    if at == 0:
+        return torch.zeros(t.shape, dtype=t.dtype, device=t.device)
+    return t.clone() if at % 16 else t
 
 
 def _ptr(t: Tensor) -> int:
@@ -166,7 +170,8 @@ def _forward(entry: str, indices, weight, vals, bias, target) -> Tuple[Tensor, T
 
 
 def _grad_scalar(grad_out: Tensor, dev) -> Tensor:
-    return grad_out.detach().to(device=dev, dtype=torch.float32).reshape(1).contiguous()
+    g = grad_out.detach().to(device=dev, dtype=torch.float32).reshape(1).contiguous()
+    return g if g.data_ptr() else torch.zeros(1, dtype=torch.float32, device=dev)  # (a zero tensor has no memory)
 
 
 @torch.library.custom_op("flexsae_amd::hier_fwd", mutates_args=())
@@ -896,7 +901,7 @@ def _hier_sgd_step_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Ten
     ``weight`` must be contiguous and 16-byte aligned, D a multiple of 8 (16-bit) or 4 (fp32),
     K <= 256."""
     B, K, F, D = _validate(indices, weight, vals, bias, target)
-    if not weight.is_contiguous() or weight.data_ptr() % 16:
+    if not weight.is_contiguous() or weight.data_ptr() % 16 or not weight.data_ptr():
         raise ValueError("hier_sgd_step updates weight in place: it must be contiguous and 16-byte aligned")
     if not _train_supported(weight, K):
         raise ValueError("hier_sgd_step needs D % 4 == 0 and K <= 256")
@@ -1147,13 +1152,14 @@ _can_tell_plain = (all(hasattr(_C, n) for n in ("_len_torch_dispatch_stack", "_l
 
 def _plain_call(*tensors: Tensor) -> bool:
     """Ordinary tensors on the GPU, and nothing around the call that would have to see the ops.  (The tensors of
-    ``torch.autograd.grad(..., is_grads_batched=True)`` are of type Tensor and have no memory of their own; nor have zero
-    tensors, and the memory of a negative view holds the values with the other sign: the dispatcher sees to both.)"""
-    if torch.compiler.is_compiling() or not _can_tell_plain:
+    ``torch.autograd.grad(..., is_grads_batched=True)`` are of type Tensor and have no memory of their own; that of a negative
+    view holds the values with the other sign, which the dispatcher sees to.  Zero tensors have none either: see _prep.
+    Devices are compared later.)"""
+    if torch.compiler.is_compiling() or not _can_tell_plain or not tensors[0].is_cuda:
         return False
     for t in tensors:
-        if (type(t) not in _PLAIN_TYPES or not t.is_cuda or t.is_neg() or t._is_zerotensor()
-                or _C._functorch.is_legacy_batchedtensor(t) or _C._functorch.is_functorch_wrapped_tensor(t)):
+        if (type(t) not in _PLAIN_TYPES or t.is_neg() or _C._functorch.is_legacy_batchedtensor(t)
+                or _C._functorch.is_functorch_wrapped_tensor(t)):
             return False
     return (_C._len_torch_dispatch_stack() == 0 and _C._len_torch_function_stack() == 0
             and _C._functorch.peek_interpreter_stack() is None and _C._get_tracing_state() is None

@@ -176,13 +176,16 @@ def test_batched_upstream_gradients_of_the_fused_step(dtype, through_ops):
 
 @pytest.mark.parametrize("loss", ["topk", "hier"])
 def test_tensors_whose_memory_is_not_their_values(loss):
-    """Negative views and zero tensors are resolved by the dispatcher: such calls go through the ops."""
+    """Negative views, which the dispatcher resolves, go through the ops; zero tensors are given memory."""
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=7))
     for i in range(1, 5):
         args = [idx, W, v, b, t]
         plain = list(args)
         plain[i] = -plain[i]
         args[i] = torch._neg_view(args[i])
+        assert torch.equal(LOSS[loss](*args), LOSS[loss](*plain))
+        args[i] = torch._efficientzerotensor(plain[i].shape, dtype=plain[i].dtype, device=DEV)
+        plain[i] = torch.zeros_like(plain[i])
         assert torch.equal(LOSS[loss](*args), LOSS[loss](*plain))
     leaves = [x.clone().requires_grad_() for x in (W, v, b)]
     out = LOSS[loss](idx, *leaves, t)
@@ -195,3 +198,5 @@ def test_tensors_whose_memory_is_not_their_values(loss):
     got = flex.hierarchical_sae_sgd_step(idx, W, torch._neg_view(v), b, t, 0.5)
     want = flex.hierarchical_sae_sgd_step(idx, W2, -v, b, t, 0.5)
     assert torch.equal(W, W2) and all(torch.equal(x, y) for x, y in zip(got, want))
+    with pytest.raises((ValueError, RuntimeError)):
+        flex.hierarchical_sae_sgd_step(idx, torch._efficientzerotensor(W.shape, device=DEV), v, b, t, 0.5)
