@@ -1128,7 +1128,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   const bool two_launches = !hot && s->B > kEndRows;
   const unsigned n_col_blocks =
       hot ? static_cast<unsigned>(ceil_div(D, 1024))
-          : static_cast<unsigned>(two_launches ? ceil_div(D, 256) * ceil_div(n_chunks, 4) : ceil_div(D, 16 * kEndCols) * 16);
+          : static_cast<unsigned>(two_launches ? ceil_div(D, 256) * ceil_div(n_chunks, 4) : ceil_div(D, kEndCols));
   const unsigned n_dvals_blocks = grid_for(s->B * s->K, 1024, 2048);
   hipLaunchKernelGGL((hier_epilogue_kernel<GT>), dim3(1 + pending.n_blocks + n_hot_blocks + n_col_blocks + n_dvals_blocks),
                      dim3(1024), 0, st,
@@ -1235,6 +1235,8 @@ struct TopkBwdPlan {
 //   vec 4, the same with 4 MiB (B=8192, K=64, F=16384, D=1028 186 / 239, 237 / 272), and where there is enough to do for half
 //       the wavefronts (B=3072, K=16, F=8192, D=1028 54 / 57, 76 / 79; B=64, K=39, F=32768, D=364 37 / 40, 39 / 41)
 // At the sizes it takes, padded rows are at most 6 % behind (shapes of 40 us, mostly the launches), on average 30 % ahead.
+// (Pairs in chunks of long latents, most of them with skewed indices, load their W piece in vectors of `vec` elements either way;
+// that is in the figures.)
 bool padding_pays(const flexsae_shape *s, int vec) {
   const int64_t tiles = ceil_div(s->D, kWave * 8);
   if (vec == 1) return s->D >= 160 || (s->D > 128 && s->F >= 65536);

@@ -281,10 +281,11 @@ __global__ __launch_bounds__(256) void topk_order_kernel(const int64_t *__restri
 }
 
 // sae_fwd_kernel for rows in latent order: NW wavefronts per block, the tiles cut into runs, one per XCD.
-// At most four wavefronts per SIMD and eight gathers in flight, sixteen of 256-byte pieces (16-byte lanes): with more of either the wavefronts of a
-// tile drift further apart than the L2 covers, and those of the next tile join them.  What bounds it: the L2s, at 13-14 of
-// the 18 TB/s they give to row gathers, and the misses beside them (5-6 TB/s).  Ordering included: B=4096, K=128, F=65536,
-// D=2304 bf16 286 -> 188 us (128-byte pieces), B=2048, K=256, F=131072, D=1024 fp32 275 -> 181 us (256-byte pieces).
+// At most four wavefronts per SIMD and eight gathers in flight, sixteen of 256-byte pieces (16-byte lanes): with more of either
+// the wavefronts of a tile drift further apart than the L2 covers, and those of the next tile join them.  What bounds it: the
+// L2s, at 13-14 of the 18 TB/s they give to row gathers, and the misses beside them (5-6 TB/s).  Ordering included: B=4096,
+// K=128, F=65536, D=2304 bf16 286 -> 188 us (128-byte pieces), B=2048, K=256, F=131072, D=1024 fp32 275 -> 181 us (256-byte
+// pieces).
 template <typename WT, int VEC, int LPR, int U, int NW>
 __global__ __launch_bounds__(NW *kWave) __attribute__((amdgpu_waves_per_eu(1, 4))) void topk_ordered_fwd_kernel(
     const vec_t<uint32_t, 2> *__restrict__ ordered, const void *__restrict__ weight, const void *__restrict__ bias,

@@ -483,8 +483,8 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
-    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int n_full, int per_wave, int tps, int col0, int slice_w, int64_t F, int K,
-    int D, int resid_ld, uint32_t resid_bytes) {
+    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int n_full, int per_wave, int tps, int col0, int slice_w,
+    int64_t F, int K, int D, int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
   if (blockIdx.x >= n_long_blocks) {

@@ -1260,7 +1260,7 @@ def _late_step(weight: Tensor, B: int, K: int) -> bool:
     rounded.  A second gather (2*B*K*D bytes, partly out of the L2s) for 6*F*D bytes less: us with it / without, uniform
     and Zipf indices, B = 4096, F = 65536, D = 2304: K = 16 469 / 538, 409 / 566; K = 32 723 / 765, 595 / 697; K = 64
     1252 / 1284, 1059 / 1081; K = 128 2369 / 2279; B = 8192, K = 64, F = 262144, D = 4096 4878 / 5786, 3526 / 4518; B = 256,
-    K = 64, F = 65536, D = 2048 171 / 332.  Not below 96 million weights, where more launches and their host work show (F = 65536,
+    K = 64, F = 65536, D = 2048 171 / 332.  Not below 96 * 2^20 weights, where more launches and their host work show (F = 65536,
     K = 32, B = 410 and 2048: D = 1544 282 / 338 and 362 / 414, D = 1024 258 / 221 and 266 / 262, D = 900 256 / 219 and
     269 / 257, D = 512 249 / 219 and 252 / 215)."""
     F, D = weight.shape

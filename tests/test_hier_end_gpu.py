@@ -1,5 +1,5 @@
 """dbias of the hierarchical step at the edges of its column sums: one block of rows or many, columns that no block of
-sixteen (or of 256) divides, and the most rows that are summed in one launch."""
+32 (or of 256) divides, and the most rows that are summed in one launch."""
 import pytest
 import torch
 
