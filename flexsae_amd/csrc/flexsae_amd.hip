@@ -1352,8 +1352,13 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
     // A last tile of less than two thirds of the columns apart from the others (us with it among them / apart, uniform
     // indices: D=296 of 256-column tiles, B=11147, K=62, F=50975 fp32 227 / 192; D=2304 of 512, B=4096, K=128, F=65536 bf16
     // 296 / 289; with more columns it fetches its slice into all L2s for little: D=1992, B=2048, K=44, F=32768 bf16 102 / 106).
+    // Not of an even number of tiles, four or more, with less than two pairs per latent, where W and dW are what moves: the runs
+    // of several XCDs then begin at the same latents and write a row's pieces at one time (four tiles, B=1721, K=23, F=343189,
+    // D=1576 bf16 354 / 369, skewed 341 / 398; sixteen, B=1458, K=55, F=89752, D=3844 fp32 557 / 591; an odd number has no such
+    // order to lose: nine, B=388, K=167, F=159036, D=2084 478 / 459).
     const int64_t last_cols = s->D - (col0 + cols - pl.tile);
-    const int n_full = 3 * last_cols < 2 * static_cast<int64_t>(pl.tile) ? tps - 1 : tps;
+    const bool in_step = tps >= 4 && tps % 2 == 0 && n_pairs < 2 * s->F;
+    const int n_full = 3 * last_cols < 2 * static_cast<int64_t>(pl.tile) && !in_step ? tps - 1 : tps;
     const int64_t xcd_span = ceil_div(n_groups * n_full, 8);
     const int64_t last_span = n_full < tps ? ceil_div(n_groups, 8) : 0;
     const unsigned n_long = kLongBlocks * static_cast<unsigned>(tps);

@@ -68,3 +68,26 @@ def test_groups_of_any_size_give_the_same_bits(B, K, F, D, dtype):
     torch.cuda.synchronize()
     assert small[0] == 0 and large[0] == 0
     assert all(torch.equal(x, y) for x, y in zip(small[1:], large[1:]))
+
+
+@pytest.mark.parametrize("K", [20, 40])
+@pytest.mark.parametrize("D", [1028, 1284, 1524])
+def test_last_tile_of_few_columns(D, K):
+    """Five and six tiles of 256 columns, the last one of four or of most: apart from the others or in step with them, by the
+    number of tiles, its columns and the pairs per latent."""
+    print("[case]", D, K, flush=True)
+    B, F = 64, 1001
+    g = torch.Generator().manual_seed(D + K)
+    idx = torch.randint(0, F, (B, K), generator=g)
+    W, v, resid = torch.randn(F, D, generator=g), torch.randn(B, K, generator=g), torch.randn(B, D, generator=g)
+    rc, dW, dv, db = abi.topk_backward(idx.to(DEV), W.to(DEV), v.to(DEV), resid.to(DEV), 1.5)
+    torch.cuda.synchronize()
+    assert rc == 0
+    scale = 1.5 * 2.0 / (B * D)
+    rows, flat = resid.double().repeat_interleave(K, 0), idx.reshape(-1)
+    terms = v.double().reshape(-1, 1) * scale * rows
+    exact, size = (torch.zeros(F, D, dtype=torch.double).index_add_(0, flat, t) for t in (terms, terms.abs()))
+    n = torch.bincount(flat, minlength=F).max() + 8  # a rounding per pair and a few for the scale
+    assert ((dW.cpu().double() - exact).abs() <= n * 2.0 ** -24 * size).all()
+    prods = rows * W.double()[flat] * scale
+    assert ((dv.cpu().double().reshape(-1) - prods.sum(1)).abs() <= (D + 8) * 2.0 ** -24 * prods.abs().sum(1)).all()
