@@ -1226,23 +1226,30 @@ struct TopkBwdPlan {
 };
 
 // Whether a bf16 copy of the residual with padded rows (16 bytes per lane, tiles of 512 columns) beats one whose rows are read
-// in the vectors of `vec` elements that divide them (tiles of 64 * vec), by 740 shapes of both kinds of indices; the backward
+// in the vectors of `vec` elements that divide them (tiles of 64 * vec).  By 1120 shapes of both kinds of indices; the backward
 // in us with narrow / padded rows, uniform and skewed:
 //   vec 1, 160 columns and more, or more than 128 and at least 65536 latents: B=4096, K=128, F=65536, D=2305 695 / 374,
 //       834 / 477, D=129 101 / 94, 135 / 134;  B=1024, K=64, F=32768, D=129 44 / 43, 58 / 60
-//   vec 2, more than 256 columns, where the padded tile of the copy (1 KB per row) is no more than 8 MiB, two L2s, or the only
-//       tile: B=8192, K=64, F=262144, D=1026 491 / 440, 551 / 490;  B=12288, K=32, F=16384 187 / 224, 243 / 251
-//   vec 4, the same with 4 MiB (B=8192, K=64, F=16384, D=1028 186 / 239, 237 / 272), and where there is enough to do for half
-//       the wavefronts (B=3072, K=16, F=8192, D=1028 54 / 57, 76 / 79; B=64, K=39, F=32768, D=364 37 / 40, 39 / 41)
-// At the sizes it takes, padded rows are at most 6 % behind (shapes of 40 us, mostly the launches), on average 30 % ahead.
+//   vec 2, more than 256 columns: B=8192, K=64, F=262144, D=1026 491 / 440, 551 / 490.  From 12000 batch rows on, whose tile of
+//       the copy is three L2s (1 KB per row), only where the tiles are full to 0.68: B=14886, K=43, F=73564, D=2154 607 / 587,
+//       776 / 685; not B=12288, K=32, F=16384, D=1026 187 / 224, 243 / 251
+//   vec 4, more than 256 columns in one tile and 1024 batch rows; in several tiles where there is enough to do for half the
+//       wavefronts (38000 latents in all tiles, four tiles, or three and 100000 pairs: B=2716, K=123, F=8124, D=1324 144 / 127,
+//       170 / 160; not B=700, K=159, F=7689, D=556 58 / 64, 75 / 85), and beyond 4096 batch rows, an L2, where few pairs gather
+//       from it: five per latent, or thirteen up to 6144 rows (B=6189, K=89, F=256085, D=828 345 / 321, 366 / 325; not B=8192,
+//       K=64, F=16384, D=1028 186 / 239, 237 / 272)
+// Where it takes them, padded rows are on average 60 % ahead with vec 1 and 12 % with the others, at most 6 % behind on one kind
+// of indices.
 // (Pairs in chunks of long latents, most of them with skewed indices, load their W piece in vectors of `vec` elements either way;
 // that is in the figures.)
 bool padding_pays(const flexsae_shape *s, int vec) {
-  const int64_t tiles = ceil_div(s->D, kWave * 8);
+  const int64_t tiles = ceil_div(s->D, kWave * 8), pairs = s->B * s->K;
   if (vec == 1) return s->D >= 160 || (s->D > 128 && s->F >= 65536);
   if (s->D <= 256) return false;
-  if (tiles == 1) return vec == 2 || s->B >= 1024;
-  return vec == 2 ? s->B <= 8192 : s->B <= 4096 && s->F * tiles >= 40000;
+  if (vec == 2) return tiles == 1 || s->B <= 12000 || 100 * s->D >= 68 * kWave * 8 * tiles;
+  if (tiles == 1) return s->B >= 1024;
+  if (s->F * tiles < 38000 && tiles < 4 && !(tiles == 3 && pairs >= 100000)) return false;
+  return s->B <= 4096 || pairs <= 5 * s->F || (s->B <= 6144 && pairs <= 13 * s->F);
 }
 
 TopkBwdPlan plan_topk_bwd(const flexsae_shape *s, int flags = 0) {
