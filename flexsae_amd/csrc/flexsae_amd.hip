@@ -272,39 +272,35 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
   return p;
 }
 
-// Whether it is the faster walk of such a shape.  Two things decide, and uniform indices gain by them what skewed ones (Zipf
-// 1.1, most of whose gathers hit an L2 either way) lose without them:
-//   reuse   pairs per latent among the rows that an XCD walks at a time (32 compute units of sixteen wavefronts): what a
-//           piece fetched once is used for.  Below 1.25 with 256-byte pieces uniform indices gain nothing, below three with
-//           128-byte ones skewed indices lose 5 to 14 %.
-//   work    the sort is a launch of 5-6 us, and blocks of up to sixteen wavefronts leave a last round that is not full: with
-//           0.88 of the rounds full, 80 pairs per row or 2500 MiB of gathers are enough; with less, 2350 MiB, or rows of 5632
-//           bytes and K times the gathered MiB of 75 * 1024.  128-byte pieces, whose waves last longer, by the reuse alone:
-//           1500 MiB with five, K times the MiB of 100 * 1024 with seven, of 150 * 1024 and rows of 2560 bytes with three.
+// Whether it is the better walk of such a shape.  A call does not know how its indices repeat: uniform ones gain by the order,
+// skewed ones (Zipf 1.1), most of whose gathers hit an L2 either way, pay a sort of 5-6 us and mostly gain little.  The lines lie
+// where the gain of the first is most, a loss of the second counted three times; two things decide:
+//   reuse   pairs per latent among the rows that an XCD walks at a time (32 compute units of sixteen wavefronts): what a piece
+//           fetched once is used for.  From two with 128-byte pieces, one with 256-byte ones, with more and with fewer latents
+//           than 131072 alike.
+//   work    the gathered MiB: 800 with 128-byte pieces; with 256-byte ones 1200, or 500 where the last round of blocks (up to
+//           sixteen wavefronts each) leaves no more than a quarter of the rounds empty, and 80 pairs per row or 1000 MiB.
 // us without / with the ordering, uniform and skewed indices:
-//   bf16, 128 B   B=4096, D=2304: K=128, F=65536 286 / 188, 150 / 149; K=256, F=262144 673 / 487, 359 / 315;  K=64, F=131072
-//                 169 / 149, 83 / 90 (not taken);  B=8192, K=192, D=1024, F=262144 449 / 369, 214 / 236 (not taken)
-//   bf16, 256 B   B=2048, D=4096: K=128, F=32768 264 / 149, 127 / 120; K=256, F=262144 604 / 510, 364 / 298;  B=1024, K=128,
-//                 D=2304, F=131072 93 / 96, 43 / 53 and K=256, D=1024, F=65536 65 / 48, 40 / 43 (not taken)
-//   fp32, 256 B   B=2048, D=1024: K=256, F=131072 275 / 181, 144 / 133; K=96, F=65536 100 / 66, 45 / 44; K=64, F=65536 69 / 50,
-//                 32 / 34 (not taken);  B=1024, K=192, D=1152, F=32768 103 / 72, 52 / 59 (not taken)
-// Over 1319 shapes (F 16384 to 1048576, many of them near the lines): of the 609 that it takes 22 are 5 % slower or more on one
-// kind of indices (the most B=512, K=192, D=4096, F=16384 bf16: 89 / 55, 44 / 54); uniform ones are 1.43 times as fast, skewed
-// ones 1.06.
+//   bf16, 128 B   B=4096, D=2304: K=128, F=65536 286 / 188, 150 / 149; K=64, F=65536 150 / 116, 69 / 77, F=131072 169 / 149,
+//                 83 / 90; K=256, F=262144 673 / 487, 359 / 315;  B=16384, K=64, F=52516, D=1024 247 / 158, 116 / 125;  not
+//                 B=8041, K=128, F=524288, D=512 153 / 183, 72 / 88 (fp16), nor B=4096, K=134, F=131072, D=256 41 / 36, 24 / 32
+//   bf16, 256 B   B=2048, D=4096: K=128, F=32768 264 / 149, 127 / 120; K=256, F=262144 604 / 510, 364 / 298;  B=1016, K=195,
+//                 F=65536, D=2048 108 / 83, 51 / 61;  not B=1024, K=128, D=2304, F=131072 93 / 96, 43 / 53
+//   fp32, 256 B   B=2048, D=1024: K=256, F=131072 275 / 181, 144 / 133; K=96, F=65536 100 / 66, 45 / 44;  B=8192, K=109,
+//                 F=65536, D=704 293 / 166, 121 / 125;  not B=2048, K=64, F=65536, D=1024 69 / 50, 32 / 34, B=1024, K=192,
+//                 D=1152, F=32768 103 / 72, 52 / 59 or B=512, K=256, F=65536, D=256 24 / 26, 22 / 22
+// Of 230 shapes (F 16384 to 524288) it takes 155: uniform indices are 1.35 times as fast there, none slower by 5 %, skewed ones 1.01,
+// 30 of them 5 % slower or more (the most B=8192, K=66, F=32768, D=672 fp32: 139 / 104, 74 / 89).
 bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
-  const size_t es = dtype_size(s->weight_dtype);
   const uint64_t B = static_cast<uint64_t>(s->B), K = static_cast<uint64_t>(s->K), F = static_cast<uint64_t>(s->F);
-  const uint64_t row_bytes = static_cast<uint64_t>(s->D) * es, mib = B * K * row_bytes >> 20;
+  const uint64_t mib = B * K * static_cast<uint64_t>(s->D) * dtype_size(s->weight_dtype) >> 20;
   const bool narrow = p.lpr == 8;
   const uint64_t at_a_time = 32 * 16 * (narrow ? 8 : 4);
   const uint64_t reused = (B < at_a_time ? B : at_a_time) * K;
-  if (narrow)
-    return (reused >= 3 * F && row_bytes >= 2560 && K * mib >= 150 * 1024) || (reused >= 5 * F && mib >= 1500) ||
-           (reused >= 7 * F && K * mib >= 100 * 1024);
-  if (4 * reused < 5 * F) return false;
+  if (narrow) return reused >= 2 * F && mib >= 800;
+  if (reused < F || (K < 80 && mib < 1000)) return false;
   const int64_t round = 32 * 16 / p.waves;  // blocks of an XCD at a time
-  const bool full = 100 * p.xcd_span >= 88 * round * ceil_div(p.xcd_span, round);
-  return full ? K >= 80 || mib >= 2500 : mib >= 2350 || (row_bytes >= 5632 && K * mib >= 75 * 1024);
+  return mib >= 1200 || (mib >= 500 && 4 * p.xcd_span >= 3 * round * ceil_div(p.xcd_span, round));
 }
 
 void launch_order(const flexsae_shape *s, const int64_t *indices, const void *vals, vec_t<uint32_t, 2> *steps,

@@ -137,8 +137,8 @@ size_t flexsae_fwd_workspace_bytes(const flexsae_shape *shape);
  * the order given: the same sums in another order, equal to fp32 rounding. */
 size_t flexsae_topk_fwd_workspace_bytes(const flexsae_shape *shape);
 
-/* The one of the two with which flexsae_topk_fwd is the faster one: by ascending latent where uniform indices gain by it and
- * skewed ones (a few latents in most rows) do not lose. */
+/* The one of the two to ask for without knowing the indices: by ascending latent where uniform ones gain more by it than
+ * skewed ones (a few latents in most rows) may lose. */
 size_t flexsae_topk_fwd_best_workspace_bytes(const flexsae_shape *shape);
 
 /*

@@ -96,12 +96,13 @@ def test_infinite_weights_stay_out_of_other_steps():
 
 @pytest.mark.parametrize("shape,dtype,pays", [
     ((4096, 128, 65536, 2304), torch.bfloat16, True), ((4096, 256, 262144, 2304), torch.bfloat16, True),
-    ((4096, 64, 131072, 2304), torch.bfloat16, False),
-    ((8192, 192, 262144, 1024), torch.bfloat16, False), ((1024, 256, 65536, 1024), torch.bfloat16, False),
+    ((4096, 64, 131072, 2304), torch.bfloat16, True),
+    ((8192, 192, 262144, 1024), torch.bfloat16, True), ((1024, 256, 65536, 1024), torch.bfloat16, False),
     ((1024, 128, 131072, 2304), torch.bfloat16, False), ((2048, 256, 262144, 4096), torch.float16, True),
     ((2048, 256, 131072, 1024), torch.float32, True), ((2048, 64, 65536, 1024), torch.float32, False),
     ((2048, 96, 65536, 1024), torch.float32, True), ((1024, 192, 32768, 1152), torch.float32, False),
-    ((2048, 192, 524288, 1024), torch.float32, False), ((4096, 512, (1 << 20) - 1, 2304), torch.bfloat16, False),
+    ((2048, 192, 524288, 1024), torch.float32, False),
+    ((4096, 64, 65536, 2304), torch.bfloat16, True), ((8041, 128, 524288, 512), torch.float16, False), ((4096, 512, (1 << 20) - 1, 2304), torch.bfloat16, True),
     ((300, 128, 65536, 2304), torch.bfloat16, False)], ids=str)
 def test_which_shapes_are_walked_in_latent_order(shape, dtype, pays):
     lib = _lib.load()
