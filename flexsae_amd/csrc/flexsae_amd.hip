@@ -1652,7 +1652,16 @@ int flexsae_hier_bwd(const flexsae_shape *s, const int64_t *indices, const void 
   } else {
     // rows that allow no more than 8 bytes of their own elements at a time are reduced by pieces where a slice is
     // whole pieces
-    const int piece = slice_w % piece_cols(pl) == 0 ? static_cast<int>(piece_cols(pl)) : 0;
+    const int64_t pc = piece_cols(pl);
+    if (slice_w % pc != 0 && slice_w > pc && s->F * s->D >= (6 << 20) &&
+        !(flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY))) {
+      // as many slices of whole pieces as are needed, of about the same width (bf16 rows of odd length; us of the step in one
+      // slice by elements / in two by pieces: B=287, K=32, F=14239, D=4099 237 / 187, B=4096, K=64, F=65536, D=129 171 / 144;
+      // small dW only pays for the launches: B=300, K=20, F=8000, D=513 61 / 73)
+      const int64_t n_slices = ceil_div(pl.d_pad, slice_w - slice_w % pc);
+      slice_w = ceil_div(ceil_div(pl.d_pad, n_slices), pc) * pc;
+    }
+    const int piece = slice_w % pc == 0 ? static_cast<int>(pc) : 0;
     if (pl.vec == 2)
       launch_hier_slices_w<2>(s, pl, slice_w, indices, weight, vals, resid, grad_out, coef, dW, dW_dtype,
                               dvals, dbias, ws, flags, status_flag, st, nullptr, piece);

@@ -110,3 +110,31 @@ def test_frozen_weights_gather_once(dtype, D):
     assert flex.ops._step_pays(W, 150) and flex.ops._ragged_pays(W, 70, 150)
     W.requires_grad_()
     assert not flex.ops._step_pays(W, 150) and not flex.ops._ragged_pays(W, 70, 150)
+
+
+@pytest.mark.parametrize("D", [65, 129, 321, 705])
+def test_odd_bf16_rows_give_the_same_bits_in_any_slices(D):
+    """Rows whose whole width is no whole number of pieces: cut into slices of whole pieces."""
+    print("[case] odd rows in slices", D, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(D)
+    B, K, F = 70, 20, 301
+    idx = torch.randint(0, F, (B, K), generator=g, device=DEV)
+    got = []
+    for least, scratch in ((None, None), (64, 1)):
+        W, v, b = (torch.randn(*s, generator=g.manual_seed(7), device=DEV).to(torch.bfloat16).requires_grad_()
+                   for s in ((F, D), (B, K), (D,)))
+        t = torch.randn(B, D, generator=g, device=DEV).to(torch.bfloat16)
+        try:
+            flex.set_hier_scratch_bytes(scratch)
+            if least:
+                flex.set_hier_min_slice_cols(least)
+            flex.triton_hierarchical_sae_loss(idx, W, v, b, t).backward()
+        finally:
+            flex.set_hier_scratch_bytes(None)
+            flex.set_hier_min_slice_cols(None)
+        got.append((W.grad, v.grad, b.grad))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    W, v, b, t = (x.detach().double().cpu() for x in (W, v, b, t))
+    W.requires_grad_()
+    flex.hierarchical_sae_loss(idx.cpu(), W, v, b, t).backward()
+    assert (got[0][0].double().cpu() - W.grad).norm() < 1e-2 * W.grad.norm()
