@@ -1322,10 +1322,15 @@ int latents_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl, int most) {
 // fp16 126 -> 117 us), with more than 140000 latents in all tiles 0.96; 8 to 12 1.04 and 1.03 with fewer than 65536, 0.99 and
 // 0.97 with more; 4 to 8 0.98 and 0.97; below 4 0.87 and 0.91; above 72 (nearly all pairs in chunks of long latents) 1.00 and
 // 1.01.
-bool one_latent_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl) {
+// And with less than one pair for 32 latents, pieces of 16 bytes per lane (`wide`): all but zero rows of dW, which a group
+// stores a row apart (groups / one, us, uniform and skewed: B=64, K=16, F=131072, fp32 D=8192 861 / 759, 866 / 722, D=4096
+// 446 / 388, 438 / 369, bf16 D=8192 469 / 420, 462 / 397; fp16, 8 bytes, 550 / 629, 468 / 615).
+bool one_latent_per_wave(const flexsae_shape *s, const TopkBwdPlan &pl, bool wide) {
   const int64_t pairs = s->B * s->K;
   const int64_t latents = s->F * (pl.d_pad / pl.tile);  // of all tiles
-  return !pl.whole_groups && latents < 140000 && pairs >= (latents < 65536 ? 8 : 12) * s->F && pairs < 72 * s->F;
+  if (pl.whole_groups) return false;
+  if (wide && 32 * pairs < s->F) return true;
+  return latents < 140000 && pairs >= (latents < 65536 ? 8 : 12) * s->F && pairs < 72 * s->F;
 }
 
 size_t topk_bwd_bytes(const TopkBwdPlan &p, int64_t slice_w) {
@@ -1342,7 +1347,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
   float *dv_part = reinterpret_cast<float *>(ws + pl.off_dvpart);
   const int64_t n_pairs = static_cast<int64_t>(pl.n_pairs);
-  const bool one = EV == VEC && one_latent_per_wave(s, pl);
+  const bool one = EV == VEC && one_latent_per_wave(s, pl, sizeof(LatentPiece<WT, GT, VEC>) == 16 &&
+                                                               sizeof(raw_vec_t<WT, VEC>) == sizeof(raw_vec_t<GT, VEC>));
   const int per_wave = one ? 1 : pl.whole_groups ? topk_group<WT, GT, VEC>() : latents_per_wave(s, pl, topk_group<WT, GT, VEC>());
   const int64_t n_groups = ceil_div(s->F, static_cast<int64_t>(kWavesPerBlock) * per_wave);
   // a launch holds fewer than 2^32 threads, 2^24 blocks: narrower slices where all tiles would be more
@@ -1364,7 +1370,10 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
     const int n_full = 3 * last_cols < 2 * static_cast<int64_t>(pl.tile) && !in_step ? tps - 1 : tps;
     const int64_t xcd_span = ceil_div(n_groups * n_full, 8);
     const int64_t last_span = n_full < tps ? ceil_div(n_groups, 8) : 0;
-    const unsigned n_long = kLongBlocks * static_cast<unsigned>(tps);
+    // no more leading blocks than chunks of long latents there can be (a multiple of eight)
+    const int64_t most_long = (ceil_div(static_cast<int64_t>(pl.n_partial_rows) * tps, kWavesPerBlock) + 7) & ~int64_t{7};
+    const int64_t all_long = static_cast<int64_t>(kLongBlocks) * tps;
+    const unsigned n_long = static_cast<unsigned>(most_long < all_long ? most_long : all_long);
     const size_t resid_bytes =
         static_cast<size_t>(s->B) * static_cast<size_t>(pl.resid_ld) * sizeof(typename Traits<RT>::store_t);
     constexpr int kEndTiles = VEC / EV;  // tiles of the long latents' second step per tile
@@ -1373,7 +1382,8 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
                        dim3(n_long + static_cast<unsigned>((xcd_span + last_span) * 8)),
                        dim3(kBlock), 0, st, begin, map, long_ctrl, long_list, chunk_begin,
                        reinterpret_cast<const vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), weight, vals,
-                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, n_groups, xcd_span, n_full,
+                       s->vals_dtype, resid, grad_out, coef, dW, dv_part, n_pairs, partial, n_long, static_cast<uint32_t>(n_groups),
+                       static_cast<uint32_t>(xcd_span), static_cast<uint32_t>(n_full),
                        per_wave, tps,
                        static_cast<int>(col0), sw, s->F, K, D, pl.resid_ld, static_cast<uint32_t>(resid_bytes));
     if (col0 + slice_w < s->D) {

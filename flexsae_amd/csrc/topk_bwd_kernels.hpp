@@ -483,25 +483,26 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
     const void *__restrict__ weight, const void *__restrict__ vals, int vals_dtype,
     const void *__restrict__ resid, const float *__restrict__ grad_out, float coef,
     void *__restrict__ dW, float *__restrict__ dv_part, int64_t n_pairs, float *__restrict__ partial,
-    unsigned n_long_blocks, int64_t n_groups, int64_t xcd_span, int n_full, int per_wave, int tps, int col0, int slice_w,
+    unsigned n_long_blocks, uint32_t n_groups, uint32_t xcd_span, uint32_t n_full, int per_wave, int tps, int col0, int slice_w,
     int64_t F, int K, int D, int resid_ld, uint32_t resid_bytes) {
   const int lane = lane_id();
   const float scale = coef * grad_out[0];
   if (blockIdx.x >= n_long_blocks) {
-    const int64_t i = (blockIdx.x - n_long_blocks) >> 3;
+    // (in 32 bits: a launch holds fewer than 2^24 blocks)
+    const uint32_t i = (blockIdx.x - n_long_blocks) >> 3;
     const bool in_full = i < xcd_span;
-    const int64_t item = in_full ? (blockIdx.x & 7) * xcd_span + i
-                                 : n_groups * n_full + (blockIdx.x & 7) * ((n_groups + 7) >> 3) + i - xcd_span;
-    const int t = static_cast<int>(item / n_groups);
-    if (t >= (in_full ? n_full : tps)) return;
-    const int64_t f0 = ((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * per_wave;
+    const uint32_t item = in_full ? (blockIdx.x & 7) * xcd_span + i
+                                  : n_groups * n_full + (blockIdx.x & 7) * ((n_groups + 7) >> 3) + i - xcd_span;
+    const uint32_t t = item / n_groups;
+    if (t >= (in_full ? n_full : static_cast<uint32_t>(tps))) return;
+    const int64_t f0 = static_cast<int64_t>((item - t * n_groups) * (blockDim.x >> 6) + wave_in_block()) * per_wave;
     if (f0 >= F) return;  // uniform per wavefront
     const GatherSource rows_src = make_gather_source(resid, resid_bytes);
     if constexpr (ONE) {
       const uint32_t b0 = begin[f0];
       const uint32_t n = begin[f0 + 1] - b0;
       if (n > static_cast<uint32_t>(kSegChunk)) return;  // chunk role
-      const int d0 = col0 + t * (kWave * VEC) + lane * VEC;
+      const int d0 = col0 + static_cast<int>(t) * (kWave * VEC) + lane * VEC;
       if (n == 0) {  // unused latent: zeros
         const float zero[VEC] = {};
         if (d0 < D) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f0 * D + d0, zero);
@@ -515,8 +516,8 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
       __shared__ LatentPiece<WT, GT, VEC> pieces[256 / kWave][L * kWave];
       topk_short_latents<WT, GT, RT, VEC, EV, L>(
           begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
-          dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F, col0 + t * (kWave * VEC) + lane * VEC, D,
-          pieces[wave_in_block()]);
+          dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F,
+          col0 + static_cast<int>(t) * (kWave * VEC) + lane * VEC, D, pieces[wave_in_block()]);
     }
     return;
   }
