@@ -276,8 +276,8 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
 // skewed ones (Zipf 1.1), most of whose gathers hit an L2 either way, pay a sort of 5-6 us and mostly gain little.  The lines lie
 // where the gain of the first is most, a loss of the second counted three times; two things decide:
 //   reuse   pairs per latent among the rows that an XCD walks at a time (32 compute units of sixteen wavefronts): what a piece
-//           fetched once is used for.  From two with 128-byte pieces, one with 256-byte ones, with more and with fewer latents
-//           than 131072 alike.
+//           fetched once is used for.  From two with 128-byte pieces, more than 0.75 with 256-byte ones, with more and with fewer
+//           latents than 131072 alike.
 //   work    the gathered MiB: 800 with 128-byte pieces; with 256-byte ones 1200, or 500 where the last round of blocks (up to
 //           sixteen wavefronts each) leaves no more than a quarter of the rounds empty, and 80 pairs per row or 1000 MiB.
 // us without / with the ordering, uniform and skewed indices:
@@ -289,7 +289,7 @@ OrderedPlan plan_ordered(const flexsae_shape *s) {
 //   fp32, 256 B   B=2048, D=1024: K=256, F=131072 275 / 181, 144 / 133; K=96, F=65536 100 / 66, 45 / 44;  B=8192, K=109,
 //                 F=65536, D=704 293 / 166, 121 / 125;  not B=2048, K=64, F=65536, D=1024 69 / 50, 32 / 34, B=1024, K=192,
 //                 D=1152, F=32768 103 / 72, 52 / 59 or B=512, K=256, F=65536, D=256 24 / 26, 22 / 22
-// Of 230 shapes (F 16384 to 524288) it takes 155: uniform indices are 1.35 times as fast there, none slower by 5 %, skewed ones 1.01,
+// Of 230 shapes (F 16384 to 524288) it takes 157: uniform indices are 1.34 times as fast there, none slower by 5 %, skewed ones 1.01,
 // 30 of them 5 % slower or more (the most B=8192, K=66, F=32768, D=672 fp32: 139 / 104, 74 / 89).
 bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
   const uint64_t B = static_cast<uint64_t>(s->B), K = static_cast<uint64_t>(s->K), F = static_cast<uint64_t>(s->F);
@@ -298,7 +298,7 @@ bool order_pays(const flexsae_shape *s, const OrderedPlan &p) {
   const uint64_t at_a_time = 32 * 16 * (narrow ? 8 : 4);
   const uint64_t reused = (B < at_a_time ? B : at_a_time) * K;
   if (narrow) return reused >= 2 * F && mib >= 800;
-  if (reused < F || (K < 80 && mib < 1000)) return false;
+  if (4 * reused <= 3 * F || (K < 80 && mib < 1000)) return false;
   const int64_t round = 32 * 16 / p.waves;  // blocks of an XCD at a time
   return mib >= 1200 || (mib >= 500 && 4 * p.xcd_span >= 3 * round * ceil_div(p.xcd_span, round));
 }
