@@ -55,7 +55,8 @@ def test_groups(flags, counts, dtype, vals_dtype, dw_dtype, D):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
-@pytest.mark.parametrize("B,K,F,D", [(40, 30, 100, 264), (500, 4, 1001, 520), (300, 5, 12293, 72), (2048, 52, 8195, 264)])
+@pytest.mark.parametrize("B,K,F,D", [(40, 30, 100, 264), (500, 4, 1001, 520), (300, 5, 12293, 72), (2048, 52, 8195, 264),
+                                     (10, 4, 4097, 264)])
 def test_groups_of_any_size_give_the_same_bits(B, K, F, D, dtype):
     """One, two, four or eight latents per wavefront, by size: as with whole groups."""
     print("[case]", B, K, F, D, dtype, flush=True)
