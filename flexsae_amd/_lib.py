@@ -90,6 +90,8 @@ SIGNATURES = {
     "flexsae_hier_import_pair_list": (_int, [_shape_p, _p, _p, _p, _sz, _p]),
     "flexsae_topk_bwd": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p, _p, _sz, _int, _p]),
     "flexsae_topk_bwd_workspace_bytes": (_sz, [_shape_p, _i64]),
+    "flexsae_topk_bwd_from_indices": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _int, _p, _int, _p, _int, _p, _sz, _int, _p, _p]),
+    "flexsae_topk_bwd_from_indices_workspace_bytes": (_sz, [_shape_p, _i64]),
     "flexsae_cast_from_f32": (_int, [_p, _int, _p, _i64, _p]),
     "flexsae_scale_from_f32": (_int, [_p, _int, _p, _i64, _p, _p]),
     "flexsae_finish_grads": (_int, [_p, _int, _p, _int, _i64, _p, _int, _p, _i64, _p, _int, _p, _i64, _p, _p]),

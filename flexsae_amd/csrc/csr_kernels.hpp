@@ -460,8 +460,8 @@ constexpr int64_t kBucketBlocks = 512;  // blocks of the bucket kernel on the ch
 // A pair inside its chunk is one word: latent within its bucket << pack_shift | place in the chunk.
 inline int csr_pack_shift(int shift) { return 32 - (shift > 11 ? shift : 11); }
 
-// Dynamic LDS: (n_buckets rounded up to four + 1) * kChunkWaves words.  n_bits: bits of a bucket number.
-__global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
+// Chunk blockIdx.x.  Dynamic LDS: (n_buckets rounded up to four + 1) * kChunkWaves words.  n_bits: bits of a bucket number.
+__device__ __forceinline__ void chunk_sort_block(
     const int64_t *__restrict__ indices, int64_t n_pairs, int64_t F, int shift, int pack_shift, uint32_t n_buckets, int n_bits,
     int64_t chunk, uint32_t n_chunks, uint32_t *__restrict__ table, uint32_t *__restrict__ tmp,
     uint32_t *__restrict__ ctrl, int *status_flag) {
@@ -573,6 +573,24 @@ __global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
   }
 }
 
+__global__ __launch_bounds__(kChunkThreads) void csr_chunk_sort_kernel(
+    const int64_t *__restrict__ indices, int64_t n_pairs, int64_t F, int shift, int pack_shift, uint32_t n_buckets, int n_bits,
+    int64_t chunk, uint32_t n_chunks, uint32_t *__restrict__ table, uint32_t *__restrict__ tmp,
+    uint32_t *__restrict__ ctrl, int *status_flag) {
+  chunk_sort_block(indices, n_pairs, F, shift, pack_shift, n_buckets, n_bits, chunk, n_chunks, table, tmp, ctrl, status_flag);
+}
+
+// Records of the pairs in the order of the list: out[place] = (batch row, val as fp32 bits), what a backward reads per pair,
+// contiguous per latent instead of scattered over vals.  A pair whose index lies outside [0, F) gets a val of zero, as in the
+// forward (the list files it under latent 0, so only that latent's pairs are looked up in indices).
+struct PairRecords {
+  const void *vals;
+  const int64_t *indices;
+  vec_t<uint32_t, 2> *out;
+  int vals_dtype;
+  uint32_t K;
+};
+
 // counter[at] += 1 for every lane with `have`, in the LDS.  The lanes that agree with the first one add up
 // beforehand (ROUNDS times over): adds to one address are served one lane after the other, and a frequent latent
 // is most of its bucket.
@@ -593,7 +611,7 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
 }
 
 // One block per bucket.  hslot: a second copy of slot[] (null: none).  solo_bit: marks in both the only pair of
-// its latent (0: no marks).
+// its latent (0: no marks).  RECORDS: writes the pairs' records (rec) instead of slot[] and hslot[].
 // The pieces of a bucket, one from every chunk, hold its pairs in pair order: pair i of the bucket is found by a search
 // for its chunk in first[].
 //   Up to kSortCap pairs: four to a thread, kept in registers.  Groups of up to kListLong pairs are gathered in the LDS in
@@ -608,10 +626,14 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
 // batches that fit the LDS: 524288 pairs of 65536 latents, uniform: 21 (24); 262144 of 262144, skewed, latents in any
 // order: 75 (96), latents by frequency: 298 (3336), half of the pairs on the first 32 latents: 144 (317); 64 latents in
 // every one of 16384 rows: 1329 (2584).
-__global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
+// WAVES: wavefronts per SIMD that its registers leave room for: eight, two blocks per compute unit, spill 13 (with records 30)
+// registers; four do not, where there is no second block (with records, us: 26.9 -> 18.8 for 524288 pairs of 65536 latents,
+// 13.7 -> 9.5 for 2048 of 4096; without 11.1 -> 10.2 there and the same for the former).
+template <bool RECORDS, int WAVES>
+__global__ __launch_bounds__(kSortThreads, WAVES) void csr_bucket_sort_kernel(
     const uint32_t *__restrict__ tmp, const uint32_t *__restrict__ table, uint32_t n_chunks, int64_t chunk, int shift,
     int pack_shift, int64_t F, uint32_t *__restrict__ begin, uint32_t *__restrict__ map, uint32_t *__restrict__ slot,
-    uint32_t *__restrict__ hslot, uint32_t solo_bit, PairLists ls) {
+    uint32_t *__restrict__ hslot, uint32_t solo_bit, PairLists ls, PairRecords rec) {
   constexpr int kWaves = kSortThreads / kWave;
   constexpr int PER = kSortMaxLatents / kSortThreads;  // latents per thread
   constexpr int kPairs = kSortCap / kSortThreads;      // pairs per thread
@@ -699,10 +721,22 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
     for (uint32_t step = probes >> 1; step > 0; step >>= 1) c += first[c + step] <= i ? step : 0u;
     return c;
   };
-  auto put = [&](uint32_t place, uint32_t id, uint32_t mark) {
+  // the bits of a pair's val, where records are written
+  auto val_bits = [&](uint32_t id) {
+    uint32_t bits = 0;
+    if constexpr (RECORDS) bits = load_scalar_bits(rec.vals, rec.vals_dtype, id);
+    return bits;
+  };
+  auto put = [&](uint32_t place, uint32_t key, uint32_t id, uint32_t mark, uint32_t bits) {
     map[place] = id;
-    if (slot) slot[id] = place | mark;
-    if (hslot) hslot[id] = place | mark;
+    if constexpr (RECORDS) {
+      float v = scalar_from_bits(bits, rec.vals_dtype);
+      if (f0 + key == 0 && static_cast<uint64_t>(rec.indices[id]) >= static_cast<uint64_t>(F)) v = 0.f;
+      rec.out[place] = vec_t<uint32_t, 2>{id / rec.K, __float_as_uint(v)};
+    } else {
+      if (slot) slot[id] = place | mark;
+      if (hslot) hslot[id] = place | mark;
+    }
   };
   // the lanes (of those with `have`, at least one) that agree with this one in the low `bits` bits of key: the first
   // lane's followers by a ballot (a frequent latent), the others by their marks in the LDS under the key's low six bits
@@ -739,7 +773,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
       if (ls.chunk_begin) append_latents(ls, f0 + my_k, my_n, x, sh);
       return;
     }
-    uint32_t key[kPairs], id[kPairs];
+    uint32_t key[kPairs], id[kPairs], bits_of[kPairs];
     const int rounds = static_cast<int>((n + kSortThreads - 1) / kSortThreads);
     {
       uint32_t c[kPairs], v[kPairs];
@@ -754,10 +788,11 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
       }
 #pragma unroll
       for (int u = 0; u < kPairs; ++u) {
-        key[u] = id[u] = 0;
+        key[u] = id[u] = bits_of[u] = 0;
         if (u < rounds) {
           key[u] = v[u] >> pack_shift;
           id[u] = c[u] * chunk_w + (v[u] & place_mask);
+          bits_of[u] = val_bits(id[u]);
           count_in_lds<2>(cnt, key[u], static_cast<uint32_t>(tid) + u * kSortThreads < n);
         }
       }
@@ -831,7 +866,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
           if (!__any(have)) continue;
           const uint32_t l = have ? lid[key[u]] : 0u;
           const unsigned long long same = agreeing(l, have, bits);
-          if (have) put(base + cnt[key[u]] + ids[l * kRounds + u * kWaves + wv] + lanes_before(same), id[u], 0u);
+          if (have) put(base + cnt[key[u]] + ids[l * kRounds + u * kWaves + wv] + lanes_before(same), key[u], id[u], 0u, bits_of[u]);
         }
       __syncthreads();
     }
@@ -856,15 +891,16 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
         for (int w = 0; w < 8; ++w) rank += (y[w] < id[u]) ? 1u : 0u;
       }
       for (; j < len; ++j) rank += (group[j] < id[u]) ? 1u : 0u;
-      put(base + start + rank, id[u], len == 1 ? solo_bit : 0u);
+      put(base + start + rank, key[u], id[u], len == 1 ? solo_bit : 0u, bits_of[u]);
     }
     if (ls.chunk_begin) append_latents(ls, f0 + my_k, my_n, x, sh);
   } else {
     uint32_t run = (n + kWaves - 1) / kWaves;
     run = (run + kWave - 1) / kWave * kWave;
     const uint32_t r0 = wv * run, r1 = (r0 + run) < n ? (r0 + run) : n;
-    // body(key, id, valid) for the wavefront's pairs in order, 64 at a time
-    auto walk = [&](auto body) {
+    // body(key, id, valid, fetch(key, id, valid)) for the wavefront's pairs in order, 64 at a time; what is fetched for several
+    // of them is in flight together
+    auto walk = [&](auto fetch, auto body) {
       constexpr int U = 8;
       uint32_t hi = 0, off = 0, id0 = 0;  // pairs from the last one looked at to hi lie in one piece
       for (uint32_t i0 = r0; i0 < r1; i0 += U * kWave) {
@@ -888,10 +924,16 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
             id0 = last * chunk_w;
           }
         }
+        uint32_t x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          idb[u] += v[u] & place_mask;
+          x[u] = fetch(v[u] >> pack_shift, idb[u], i0 + u * kWave + lane < r1);
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const uint32_t at = i0 + u * kWave;
-          if (at < r1) body(v[u] >> pack_shift, idb[u] + (v[u] & place_mask), at + lane < r1);
+          if (at < r1) body(v[u] >> pack_shift, idb[u], at + lane < r1, x[u]);
         }
       }
     };
@@ -903,7 +945,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
       for (uint32_t l = tid; l < kWaves * kRunLatents; l += kSortThreads) ids[l] = 0u;
       __syncthreads();
       uint32_t before = 0;  // this lane's pairs of the latents before the batch
-      walk([&](uint32_t key, uint32_t, bool valid) {
+      walk([](uint32_t, uint32_t, bool) { return 0u; }, [&](uint32_t key, uint32_t, bool valid, uint32_t) {
         before += valid && key < k0 ? 1u : 0u;
         count_in_lds<1>(mine, key - k0, valid && key - k0 < batch);
       });
@@ -942,7 +984,8 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
       if (mine_too) begin[f0 + k0 + tid] = base + start;
       if (ls.chunk_begin) append_latents(ls, f0 + k0 + tid, mine_too ? 1 : 0, total, sh);
       __syncthreads();
-      walk([&](uint32_t key, uint32_t id, bool valid) {
+      walk([&](uint32_t key, uint32_t id, bool valid) { return valid && key - k0 < batch ? val_bits(id) : 0u; },
+           [&](uint32_t key, uint32_t id, bool valid, uint32_t bits_of) {
         const uint32_t l = key - k0;
         const bool have = valid && l < batch;
         if (!__any(have)) return;
@@ -950,7 +993,7 @@ __global__ __launch_bounds__(kSortThreads, 8) void csr_bucket_sort_kernel(
         const uint32_t rank = lanes_before(same);
         if (have) {
           const uint32_t place = mine[l] + rank, at = cnt[l];
-          put(base + at + place, id, cnt[l + 1] - at == 1u ? solo_bit : 0u);
+          put(base + at + place, key, id, cnt[l + 1] - at == 1u ? solo_bit : 0u, bits_of);
           // (LDS accesses of a wavefront are served in order: all lanes have read the cursor)
           if (rank == 0) mine[l] = place + static_cast<uint32_t>(__popcll(same));
         }
@@ -1005,11 +1048,9 @@ __device__ __forceinline__ void colsum_partial_one(const float *__restrict__ x, 
   partial[chunk * cols + c] = s;
 }
 
-// stage 2 for column c
-__device__ __forceinline__ void colsum_final_one(const float *__restrict__ partial, int n_chunks, int cols,
-                                                 const float *__restrict__ grad_out, float coef,
-                                                 float *__restrict__ out, int c) {
-  if (c >= cols) return;
+// stage 2 for column c < cols
+__device__ __forceinline__ float colsum_final_value(const float *__restrict__ partial, int n_chunks, int cols,
+                                                    const float *__restrict__ grad_out, float coef, int c) {
   float s = 0.f;
   int k = 0;
   for (; k + 8 <= n_chunks; k += 8) {
@@ -1020,7 +1061,13 @@ __device__ __forceinline__ void colsum_final_one(const float *__restrict__ parti
     for (int u = 0; u < 8; ++u) s += v[u];
   }
   for (; k < n_chunks; ++k) s += partial[static_cast<int64_t>(k) * cols + c];
-  out[c] = s * coef * (grad_out ? grad_out[0] : 1.f);
+  return s * coef * (grad_out ? grad_out[0] : 1.f);
+}
+
+__device__ __forceinline__ void colsum_final_one(const float *__restrict__ partial, int n_chunks, int cols,
+                                                 const float *__restrict__ grad_out, float coef,
+                                                 float *__restrict__ out, int c) {
+  if (c < cols) out[c] = colsum_final_value(partial, n_chunks, cols, grad_out, coef, c);
 }
 
 __global__ __launch_bounds__(256) void colsum_final_kernel(const float *__restrict__ partial,

@@ -544,6 +544,16 @@ void launch_pair_lists(const uint32_t *begin, int64_t F, const PairLists &lists,
                      F, lists);
 }
 
+template <bool RECORDS>
+void launch_bucket_sort(const CsrScratch &sc, int64_t F, uint32_t *begin, uint32_t *map, uint32_t *slot, uint32_t *hslot,
+                        uint32_t solo_bit, const PairLists &lists, const PairRecords &rec, hipStream_t st) {
+  const CsrPlan &pl = sc.plan;
+  const auto kernel = static_cast<int64_t>(pl.n_buckets) * pl.n_batches <= kBucketBlocks / 2 ? csr_bucket_sort_kernel<RECORDS, 4>
+                                                                                             : csr_bucket_sort_kernel<RECORDS, 8>;
+  hipLaunchKernelGGL(kernel, dim3(pl.n_buckets, pl.n_batches), dim3(kSortThreads), 0, st, sc.tmp, sc.table, pl.n_chunks,
+                     pl.chunk, pl.shift, pl.pack_shift, F, begin, map, slot, hslot, solo_bit, lists, rec);
+}
+
 // begin[F+1], map[B*K] and, when `slot` is given, its inverse slot[B*K] (and a second copy of it in
 // `hslot`); fills the lists of sc.lists.
 void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, uint32_t *begin,
@@ -556,8 +566,7 @@ void csr_build_launch(const int64_t *indices, int64_t B, int64_t K, int64_t F, u
     hipLaunchKernelGGL(csr_chunk_sort_kernel, dim3(pl.n_chunks), dim3(kChunkThreads), lds, st, indices, n_pairs, F,
                        pl.shift, pl.pack_shift, pl.n_buckets, pl.n_bits, pl.chunk, pl.n_chunks, sc.table, sc.tmp, sc.lists.ctrl,
                        status_flag);
-    hipLaunchKernelGGL(csr_bucket_sort_kernel, dim3(pl.n_buckets, pl.n_batches), dim3(kSortThreads), 0, st, sc.tmp, sc.table,
-                       pl.n_chunks, pl.chunk, pl.shift, pl.pack_shift, F, begin, map, slot, hslot, solo_bit, sc.lists);
+    launch_bucket_sort<false>(sc, F, begin, map, slot, hslot, solo_bit, sc.lists, PairRecords{}, st);
     return;
   }
   hipLaunchKernelGGL(csr_init_kernel, dim3(grid_for(F + 1, 256, 4096)), dim3(256), 0, st, begin, F + 1,
@@ -1341,7 +1350,7 @@ template <typename WT, typename GT, typename RT, int VEC, int EV>
 void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                         const uint32_t *begin, const uint32_t *map, const void *weight,
                         const void *vals, const void *resid, const float *grad_out, float coef,
-                        void *dW, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
+                        void *dW, const LeafGrads &leaf, uint8_t *ws, hipStream_t st) {
   const PairLists ls = carve_topk_lists(s, pl, ws);
   const uint32_t *long_ctrl = ls.ctrl, *long_list = ls.long_list, *chunk_begin = ls.chunk_begin;
   float *partial = reinterpret_cast<float *>(ws + pl.off_partial);
@@ -1398,8 +1407,7 @@ void launch_topk_slices(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t s
                        dim3(n_long_blocks + n_col_blocks + grid_for(n_pairs, kBlock, 8192)), dim3(kBlock), 0, st, long_ctrl,
                        long_list, chunk_begin, partial, dW, tps * kEndTiles, static_cast<int>(col0), sw, D, n_long_blocks,
                        reinterpret_cast<const float *>(ws + pl.off_colsum), static_cast<int>(ceil_div(s->B, kColsumRows)),
-                       grad_out, coef, dbias, n_col_blocks, map, dv_part, static_cast<int>(pl.d_pad / pl.tile), n_pairs,
-                       dvals);
+                       grad_out, coef, n_col_blocks, map, dv_part, static_cast<int>(pl.d_pad / pl.tile), n_pairs, leaf);
   }
 }
 
@@ -1407,19 +1415,19 @@ template <typename WT, typename RT, int VEC, int EV = VEC>
 void launch_topk_slices_g(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                           const uint32_t *begin, const uint32_t *map, const void *weight,
                           const void *vals, const void *resid, const float *grad_out, float coef,
-                          void *dW, int dW_dtype, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
+                          void *dW, int dW_dtype, const LeafGrads &leaf, uint8_t *ws, hipStream_t st) {
   switch (dW_dtype) {
     case FLEXSAE_F32:
       launch_topk_slices<WT, float, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                             coef, dW, dvals, dbias, ws, st);
+                                             coef, dW, leaf, ws, st);
       break;
     case FLEXSAE_BF16:
       launch_topk_slices<WT, bf16_t, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dvals, dbias, ws, st);
+                                              coef, dW, leaf, ws, st);
       break;
     default:
       launch_topk_slices<WT, f16_t, RT, VEC, EV>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                             coef, dW, dvals, dbias, ws, st);
+                                             coef, dW, leaf, ws, st);
   }
 }
 
@@ -1428,24 +1436,85 @@ template <int VEC>
 void launch_topk_slices_w(const flexsae_shape *s, const TopkBwdPlan &pl, int64_t slice_w,
                           const uint32_t *begin, const uint32_t *map, const void *weight,
                           const void *vals, const void *resid, const float *grad_out, float coef,
-                          void *dW, int dW_dtype, float *dvals, float *dbias, uint8_t *ws, hipStream_t st) {
+                          void *dW, int dW_dtype, const LeafGrads &leaf, uint8_t *ws, hipStream_t st) {
   switch (s->weight_dtype) {
     case FLEXSAE_F32:
       launch_topk_slices_g<float, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dW_dtype, dvals, dbias, ws, st);
+                                              coef, dW, dW_dtype, leaf, ws, st);
       break;
     case FLEXSAE_BF16:
       if (pl.resid16)
         launch_topk_slices_g<bf16_t, bf16_t, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                                  coef, dW, dW_dtype, dvals, dbias, ws, st);
+                                                  coef, dW, dW_dtype, leaf, ws, st);
       else
         launch_topk_slices_g<bf16_t, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                                 coef, dW, dW_dtype, dvals, dbias, ws, st);
+                                                 coef, dW, dW_dtype, leaf, ws, st);
       break;
     default:
       launch_topk_slices_g<f16_t, float, VEC>(s, pl, slice_w, begin, map, weight, vals, resid, grad_out,
-                                              coef, dW, dW_dtype, dvals, dbias, ws, st);
+                                              coef, dW, dW_dtype, leaf, ws, st);
   }
+}
+
+size_t least_topk_bwd_bytes(const TopkBwdPlan &pl) { return topk_bwd_bytes(pl, pl.tile); }
+
+// What a backward checks besides the pair list.
+int check_topk_bwd(const flexsae_shape *s, const TopkBwdPlan &pl, const int64_t *indices, const void *weight, const void *vals,
+                   const float *resid, const float *grad_out, const void *dW, int dW_dtype) {
+  if ((indices && !aligned(indices, 8)) || !aligned(weight, pl.row_vec * dtype_size(s->weight_dtype)) ||
+      !aligned(vals, dtype_size(s->vals_dtype)) || !aligned(resid, pl.resid16 ? 16 : pl.vec * 4) || !aligned(grad_out, 4) ||
+      !aligned(dW, pl.row_vec * dtype_size(dW_dtype)))
+    return FLEXSAE_ERR_ALIGNMENT;
+  return FLEXSAE_OK;
+}
+
+// The backward proper, with the records, the lists, the copy of the residual and stage 1 of dbias in the workspace.
+void launch_topk_bwd(const flexsae_shape *s, const TopkBwdPlan &pl, const uint32_t *begin, const uint32_t *map,
+                     const void *weight, const void *vals, const float *resid, const float *grad_out, void *dW, int dW_dtype,
+                     const LeafGrads &leaf, uint8_t *ws, size_t ws_bytes, hipStream_t st) {
+  int64_t slice_w = pl.tile;
+  while (slice_w + pl.tile <= pl.d_pad && topk_bwd_bytes(pl, slice_w + pl.tile) <= ws_bytes) slice_w += pl.tile;
+  const float coef =
+      static_cast<float>(2.0 / (static_cast<double>(s->B) * static_cast<double>(s->D)));
+  const void *gather_src = pl.resid16 ? static_cast<const void *>(ws + pl.off_resid16) : resid;
+  if (pl.vec == 8) {
+    const auto slices = pl.row_vec == 8   ? launch_topk_slices_g<bf16_t, bf16_t, 8>
+                        : pl.row_vec == 4 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 4>
+                        : pl.row_vec == 2 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 2>
+                                          : launch_topk_slices_g<bf16_t, bf16_t, 8, 1>;
+    slices(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW, dW_dtype, leaf, ws, st);
+    return;
+  }
+  const auto slices = pl.vec == 4 ? launch_topk_slices_w<4> : pl.vec == 2 ? launch_topk_slices_w<2> : launch_topk_slices_w<1>;
+  slices(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW, dW_dtype, leaf, ws, st);
+}
+
+// The preparation on a given pair list (topk_prepare_kernel) and the lists of its long latents.
+void launch_topk_prepare(const flexsae_shape *s, const TopkBwdPlan &pl, const uint32_t *begin, const uint32_t *map,
+                         const int64_t *indices, const void *vals, const float *resid, uint8_t *ws, hipStream_t st) {
+  const PairLists lists = carve_topk_lists(s, pl, ws);
+  const int64_t n_resid = pl.resid16 ? s->B * pl.resid_ld : 0;
+  const int64_t work = s->B * s->K > ceil_div(n_resid, 4) ? s->B * s->K : ceil_div(n_resid, 4);
+  const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(s->D, 256) * ceil_div(s->B, kColsumRows));
+  hipLaunchKernelGGL(topk_prepare_kernel, dim3(n_col_blocks + grid_for(work, 256, 1 << 16)), dim3(256), 0, st, map, indices,
+                     s->F, vals, s->vals_dtype, s->B * s->K, static_cast<int>(s->K),
+                     reinterpret_cast<vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), resid, n_resid,
+                     pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr, lists.ctrl, s->B,
+                     static_cast<int>(s->D), pl.resid_ld, reinterpret_cast<float *>(ws + pl.off_colsum), n_col_blocks);
+  launch_pair_lists(begin, s->F, lists, st, true);
+}
+
+// A pair list made for one TopK backward, in front of its workspace: begin[F+1] | map[B*K] | scratch.
+struct TopkListPlan {
+  size_t off_map, off_csr, bytes;
+};
+
+TopkListPlan plan_topk_list(const flexsae_shape *s) {
+  TopkListPlan p;
+  p.off_map = round_up(static_cast<size_t>(s->F + 1) * 4, kAlign);
+  p.off_csr = p.off_map + round_up(static_cast<size_t>(s->B) * static_cast<size_t>(s->K) * 4, kAlign);
+  p.bytes = p.off_csr + round_up(flexsae_csr_workspace_bytes(s->B, s->K, s->F), kAlign);
+  return p;
 }
 
 }  // namespace
@@ -1902,52 +1971,67 @@ int flexsae_topk_bwd(const flexsae_shape *s, const uint32_t *begin, const uint32
   // the residual rows are gathered through a 32-bit buffer descriptor
   if (static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 4 > 0xffffffffull) return FLEXSAE_ERR_UNSUPPORTED;
   const TopkBwdPlan pl = plan_topk_bwd(s, flags);
-  if (!aligned(begin, 4) || !aligned(map, 4) || (indices && !aligned(indices, 8)) ||
-      !aligned(weight, pl.row_vec * dtype_size(s->weight_dtype)) ||
-      !aligned(vals, dtype_size(s->vals_dtype)) || !aligned(resid, pl.resid16 ? 16 : pl.vec * 4) ||
-      !aligned(grad_out, 4) || !aligned(dW, pl.row_vec * dtype_size(dW_dtype)) || !aligned(dvals, 16) ||
-      !aligned(dbias, 4))
-    return FLEXSAE_ERR_ALIGNMENT;
-  if (!workspace || !aligned(workspace, kAlign) || workspace_bytes < topk_bwd_bytes(pl, pl.tile))
-    return FLEXSAE_ERR_WORKSPACE;
-  int64_t slice_w = pl.tile;
-  while (slice_w + pl.tile <= pl.d_pad && topk_bwd_bytes(pl, slice_w + pl.tile) <= workspace_bytes)
-    slice_w += pl.tile;
+  if (!aligned(begin, 4) || !aligned(map, 4) || !aligned(dvals, 16) || !aligned(dbias, 4)) return FLEXSAE_ERR_ALIGNMENT;
+  rc = check_topk_bwd(s, pl, indices, weight, vals, resid, grad_out, dW, dW_dtype);
+  if (rc != FLEXSAE_OK) return rc;
+  if (!workspace || !aligned(workspace, kAlign) || workspace_bytes < least_topk_bwd_bytes(pl)) return FLEXSAE_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   // (every output element is written exactly once: nothing needs a zero-fill, whatever `flags` says)
-  const PairLists lists = carve_topk_lists(s, pl, ws);
-  const float coef =
-      static_cast<float>(2.0 / (static_cast<double>(s->B) * static_cast<double>(s->D)));
-  // per-pair records, for bf16 weights the bf16 copy of the residual, and stage 1 of dbias: one launch
-  const void *gather_src = pl.resid16 ? static_cast<const void *>(ws + pl.off_resid16) : resid;
-  {
-    const int64_t n_resid = pl.resid16 ? s->B * pl.resid_ld : 0;
-    const int64_t work = s->B * s->K > ceil_div(n_resid, 4) ? s->B * s->K : ceil_div(n_resid, 4);
-    const unsigned n_col_blocks = static_cast<unsigned>(ceil_div(s->D, 256) * ceil_div(s->B, kColsumRows));
-    hipLaunchKernelGGL(topk_prepare_kernel, dim3(n_col_blocks + grid_for(work, 256, 1 << 16)), dim3(256), 0, st, map, indices,
-                       s->F, vals, s->vals_dtype, s->B * s->K, static_cast<int>(s->K),
-                       reinterpret_cast<vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), resid, n_resid,
-                       pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr, lists.ctrl, s->B,
-                       static_cast<int>(s->D), pl.resid_ld, reinterpret_cast<float *>(ws + pl.off_colsum), n_col_blocks);
-  }
-  launch_pair_lists(begin, s->F, lists, st, true);
-  if (pl.vec == 8) {
-    const auto slices = pl.row_vec == 8   ? launch_topk_slices_g<bf16_t, bf16_t, 8>
-                        : pl.row_vec == 4 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 4>
-                        : pl.row_vec == 2 ? launch_topk_slices_g<bf16_t, bf16_t, 8, 2>
-                                          : launch_topk_slices_g<bf16_t, bf16_t, 8, 1>;
-    slices(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW, dW_dtype, dvals, dbias, ws, st);
-  } else if (pl.vec == 4) {
-    launch_topk_slices_w<4>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, dbias, ws, st);
-  } else if (pl.vec == 2) {
-    launch_topk_slices_w<2>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, dbias, ws, st);
+  launch_topk_prepare(s, pl, begin, map, indices, vals, resid, ws, st);
+  launch_topk_bwd(s, pl, begin, map, weight, vals, resid, grad_out, dW, dW_dtype,
+                  LeafGrads{dvals, dbias, FLEXSAE_F32, FLEXSAE_F32}, ws, workspace_bytes, st);
+  return launch_status();
+}
+
+size_t flexsae_topk_bwd_from_indices_workspace_bytes(const flexsae_shape *s, int64_t slice_cols) {
+  if (check_shape(s) != FLEXSAE_OK) return 0;
+  return plan_topk_list(s).bytes + flexsae_topk_bwd_workspace_bytes(s, slice_cols);
+}
+
+int flexsae_topk_bwd_from_indices(const flexsae_shape *s, const int64_t *indices, const void *weight, const void *vals,
+                                  const float *resid, const float *grad_out, void *dW, int dW_dtype, void *dvals,
+                                  int dvals_dtype, void *dbias, int dbias_dtype, void *workspace, size_t workspace_bytes,
+                                  int flags, int *status_flag, void *stream) {
+  int rc = check_shape(s);
+  if (rc != FLEXSAE_OK) return rc;
+  if (!indices || !weight || !vals || !resid || !grad_out || !dW || !dvals || !dbias || !valid_dtype(dW_dtype) ||
+      !valid_dtype(dvals_dtype) || !valid_dtype(dbias_dtype))
+    return FLEXSAE_ERR_INVALID_ARGUMENT;
+  if (static_cast<size_t>(s->B) * static_cast<size_t>(s->D) * 4 > 0xffffffffull) return FLEXSAE_ERR_UNSUPPORTED;
+  const TopkBwdPlan pl = plan_topk_bwd(s, flags);
+  if (!aligned(dvals, dtype_size(dvals_dtype)) || !aligned(dbias, dtype_size(dbias_dtype)) || !aligned(status_flag, 4))
+    return FLEXSAE_ERR_ALIGNMENT;
+  rc = check_topk_bwd(s, pl, indices, weight, vals, resid, grad_out, dW, dW_dtype);
+  if (rc != FLEXSAE_OK) return rc;
+  const TopkListPlan lp = plan_topk_list(s);
+  if (!workspace || !aligned(workspace, kAlign) || workspace_bytes < lp.bytes + least_topk_bwd_bytes(pl))
+    return FLEXSAE_ERR_WORKSPACE;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  uint32_t *begin = static_cast<uint32_t *>(workspace);
+  uint32_t *map = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(workspace) + lp.off_map);
+  uint8_t *ws = static_cast<uint8_t *>(workspace) + lp.bytes;
+  CsrScratch sc = carve_csr_scratch(static_cast<uint8_t *>(workspace) + lp.off_csr, s->F, s->B * s->K);
+  const CsrPlan &cp = sc.plan;
+  if (cp.bucketed) {
+    const size_t lds = (round_up(cp.n_buckets, 4) + 1) * kChunkWaves * 4;
+    const int cols = static_cast<int>(s->D);
+    const int64_t n_resid_blocks = resid_blocks(s->B, cols, pl.resid16 ? pl.resid_ld : cols);
+    const PairLists lists = carve_topk_lists(s, pl, ws);
+    hipLaunchKernelGGL(topk_front_kernel, dim3(cp.n_chunks + static_cast<unsigned>(n_resid_blocks)),
+                       dim3(kChunkThreads), lds, st, indices, s->B * s->K, s->F, cp.shift, cp.pack_shift, cp.n_buckets,
+                       cp.n_bits, cp.chunk, cp.n_chunks, sc.table, sc.tmp, lists.ctrl, status_flag, resid, s->B, cols,
+                       pl.resid_ld, pl.resid16 ? static_cast<void *>(ws + pl.off_resid16) : nullptr,
+                       reinterpret_cast<float *>(ws + pl.off_colsum));
+    const PairRecords rec = {vals, indices, reinterpret_cast<vec_t<uint32_t, 2> *>(ws + pl.off_slotbv), s->vals_dtype,
+                             static_cast<uint32_t>(s->K)};
+    launch_bucket_sort<true>(sc, s->F, begin, map, nullptr, nullptr, 0u, lists, rec, st);
   } else {
-    launch_topk_slices_w<1>(s, pl, slice_w, begin, map, weight, vals, gather_src, grad_out, coef, dW,
-                            dW_dtype, dvals, dbias, ws, st);
+    csr_build_launch(indices, s->B, s->K, s->F, begin, map, nullptr, nullptr, sc, status_flag, st);
+    launch_topk_prepare(s, pl, begin, map, indices, vals, resid, ws, st);
   }
+  launch_topk_bwd(s, pl, begin, map, weight, vals, resid, grad_out, dW, dW_dtype,
+                  LeafGrads{dvals, dbias, dvals_dtype, dbias_dtype}, ws, workspace_bytes - lp.bytes, st);
   return launch_status();
 }
 

@@ -554,6 +554,20 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
   }
 }
 
+// x (fp32) rounded to run-time type `dtype`
+__device__ __forceinline__ void store_scalar(void *base, int dtype, int64_t i, float x) {
+  const float v[1] = {x};
+  if (dtype == FLEXSAE_F32) store_vec<float, 1>(base, i, v);
+  else if (dtype == FLEXSAE_BF16) store_vec<bf16_t, 1>(base, i, v);
+  else store_vec<f16_t, 1>(base, i, v);
+}
+
+// Gradients of vals and bias in the leaves' types.
+struct LeafGrads {
+  void *dvals, *dbias;
+  int dvals_dtype, dbias_dtype;
+};
+
 // What follows the (last) slice of a TopK backward, in one launch of 256-thread blocks; the parts are independent:
 //   the first n_long_blocks  second step of the slice's long latents (seg_long_finalize_body);
 //   the next n_col_blocks    dbias = coef * grad_out * column sums of resid: stage 2 (colsum_final_one);
@@ -566,9 +580,8 @@ __global__ __launch_bounds__(256) void topk_epilogue_kernel(
     const uint32_t *__restrict__ long_ctrl, const uint32_t *__restrict__ long_list,
     const uint32_t *__restrict__ chunk_begin, const float *__restrict__ partial, void *__restrict__ dW, int tps, int col0,
     int slice_w, int D, unsigned n_long_blocks, const float *__restrict__ colsum_part, int n_chunks,
-    const float *__restrict__ grad_out, float coef, float *__restrict__ dbias, unsigned n_col_blocks,
-    const uint32_t *__restrict__ map, const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs,
-    float *__restrict__ dvals) {
+    const float *__restrict__ grad_out, float coef, unsigned n_col_blocks,
+    const uint32_t *__restrict__ map, const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs, LeafGrads leaf) {
   if (blockIdx.x < n_long_blocks) {
     seg_long_finalize_body<GT, VEC, 8>(long_ctrl, long_list, chunk_begin, partial, dW, nullptr, tps, col0, slice_w, D,
                                        blockIdx.x, n_long_blocks);
@@ -576,7 +589,8 @@ __global__ __launch_bounds__(256) void topk_epilogue_kernel(
   }
   unsigned blk = blockIdx.x - n_long_blocks;
   if (blk < n_col_blocks) {
-    colsum_final_one(colsum_part, n_chunks, D, grad_out, coef, dbias, static_cast<int>(blk * blockDim.x + threadIdx.x));
+    const int c = static_cast<int>(blk * blockDim.x + threadIdx.x);
+    if (c < D) store_scalar(leaf.dbias, leaf.dbias_dtype, c, colsum_final_value(colsum_part, n_chunks, D, grad_out, coef, c));
     return;
   }
   blk -= n_col_blocks;
@@ -584,11 +598,85 @@ __global__ __launch_bounds__(256) void topk_epilogue_kernel(
   for (int64_t s = static_cast<int64_t>(blk) * blockDim.x + threadIdx.x; s < n_pairs; s += stride) {
     float acc = 0.f;
     for (int t = 0; t < n_tiles; ++t) acc += dv_part[t * n_pairs + s];
-    dvals[map[s]] = acc;
+    store_scalar(leaf.dvals, leaf.dvals_dtype, map[s], acc);
   }
 }
 
-// Preparation of a TopK backward, one launch:
+// For the kColsumRows rows of a chunk and 64 * V columns, by one block of four wavefronts: resid16[b, c] = bf16(resid[b, c])
+// (resid16 null: no copy; ld16 >= cols elements a row, zeros past cols; V divides cols and ld16) and stage 1 of the column sums
+// of resid, both from one read.  A wavefront has sixteen rows, all in flight at once; the sums are colsum_partial_one's: a
+// wavefront adds its rows to the sums of the rows before.
+template <int V>
+__device__ __forceinline__ void resid_block(const float *__restrict__ resid, int64_t rows, int cols, int ld16,
+                                            void *__restrict__ resid16, float *__restrict__ colsum_part, unsigned block,
+                                            float *__restrict__ sums) {
+  constexpr int kBlockWaves = kChunkThreads / kWave, U = kColsumRows / kBlockWaves;
+  const int width = resid16 ? ld16 : cols;
+  const unsigned across = static_cast<unsigned>((width + kWave * V - 1) / (kWave * V));
+  const unsigned chunk = block / across;
+  const int lane = lane_id(), wv = wave_in_block();
+  const int c = static_cast<int>((block - chunk * across) * (kWave * V)) + lane * V;
+  const int64_t r0 = static_cast<int64_t>(chunk) * kColsumRows + wv * U;
+  const bool inside = c < cols;
+  float x[U][V];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) x[u][i] = 0.f;
+    if (inside && r0 + u < rows) load_vec<float, V>(resid, (r0 + u) * cols + c, x[u]);
+  }
+  for (int w = 0; w < kBlockWaves; ++w) {
+    if (w == wv) {  // uniform
+      float s[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) s[i] = w == 0 ? 0.f : sums[lane * V + i];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (r0 + u < rows) {  // uniform
+#pragma unroll
+          for (int i = 0; i < V; ++i) s[i] += x[u][i];
+        }
+#pragma unroll
+      for (int i = 0; i < V; ++i) sums[lane * V + i] = s[i];
+      if (w == kBlockWaves - 1 && inside) store_vec<float, V>(colsum_part, static_cast<int64_t>(chunk) * cols + c, s);
+    }
+    __syncthreads();
+  }
+  if (!resid16 || c >= ld16) return;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (r0 + u < rows) store_vec<bf16_t, V>(resid16, (r0 + u) * ld16 + c, x[u]);
+}
+
+// Blocks of resid_block for a residual of `cols` columns
+inline int64_t resid_blocks(int64_t rows, int cols, int width) {
+  const int v = cols % 4 == 0 ? 4 : cols % 2 == 0 ? 2 : 1;
+  return ((rows + kColsumRows - 1) / kColsumRows) * ((width + kWave * v - 1) / (kWave * v));
+}
+
+// First launch of a TopK backward that makes its own pair list: the first n_chunks blocks order the list's chunks
+// (csr_chunk_sort_kernel), the others are resid_block; the records come with the second launch (csr_bucket_sort_kernel).
+// The chunks are a chain of trips to memory on a few wavefronts per compute unit and the residual streams beside them.  B=4096,
+// K=128, F=65536, D=2304 bf16: the two launches take 15.7 + 18.8 us; chunks, buckets, topk_prepare_kernel and pair_lists_kernel
+// 9.4 + 12.6 + 23.2 + 4.7 (fp32 B=2048, K=256, F=131072, D=1024 9.7 + 19.2 against 9.2 + 13.0 + 13.3 + 4.7; B=64, K=32, F=4096,
+// D=256 5.3 + 9.5 against 5.2 + 7.6 + 4.0 + 2.9).
+__global__ __launch_bounds__(kChunkThreads) void topk_front_kernel(
+    const int64_t *__restrict__ indices, int64_t n_pairs, int64_t F, int shift, int pack_shift, uint32_t n_buckets, int n_bits,
+    int64_t chunk, uint32_t n_chunks, uint32_t *__restrict__ table, uint32_t *__restrict__ tmp, uint32_t *__restrict__ ctrl,
+    int *status_flag, const float *__restrict__ resid, int64_t rows, int cols, int ld16, void *__restrict__ resid16,
+    float *__restrict__ colsum_part) {
+  if (blockIdx.x < n_chunks) {
+    chunk_sort_block(indices, n_pairs, F, shift, pack_shift, n_buckets, n_bits, chunk, n_chunks, table, tmp, ctrl, status_flag);
+    return;
+  }
+  __shared__ float sums[kWave * 4];
+  const unsigned block = blockIdx.x - n_chunks;
+  if (cols % 4 == 0) resid_block<4>(resid, rows, cols, ld16, resid16, colsum_part, block, sums);
+  else if (cols % 2 == 0) resid_block<2>(resid, rows, cols, ld16, resid16, colsum_part, block, sums);
+  else resid_block<1>(resid, rows, cols, ld16, resid16, colsum_part, block, sums);
+}
+
+// Preparation of a TopK backward on a given pair list, one launch:
 //   slot_bv[s] = (batch row, val as fp32 bits) of the pair in slot s of the latent-major list: what
 //     the backward reads per pair, contiguous per latent instead of scattered over vals; a pair
 //     whose index lies outside [0, F) gets a val of zero, as in the forward (the pair list files it

@@ -566,8 +566,13 @@ def set_topk_residual_bf16(enabled: bool) -> None:
     _topk_residual_bf16 = bool(enabled)
 
 
-def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
-                   resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor, resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+    return _topk_bwd_typed(grad_out, indices, weight, vals, resid, torch.float32, torch.float32)
+
+
+def _topk_bwd_typed(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor, resid: Tensor, dvals_dtype,
+                    dbias_dtype) -> Tuple[Tensor, Tensor, Tensor]:
+    """(dW, dvals, dbias), dvals and dbias in the types asked for."""
     lib = _lib.load()
     B, K = indices.shape
     F, D = weight.shape
@@ -576,6 +581,22 @@ def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tens
     with _on_device(dev):
         g = _grad_scalar(grad_out, dev)
         shape = _shape(B, K, F, D, weight, vals, torch.float32, torch.float32)
+        flags = 0 if _topk_residual_bf16 else _lib.TOPK_BWD_FP32_RESIDUAL
+        dW = torch.empty_like(weight)
+        # the slice width only sizes the partial sums of hot latents; one launch over all of D is
+        # fastest, so allow them 256 MiB before slicing
+        slice_cols = max(1, (256 << 20) // max(1, (B * K // 32) * 4))
+        if _pair_cache is None:
+            dvals = torch.empty((B, K), dtype=dvals_dtype, device=dev)
+            dbias = torch.empty((D,), dtype=dbias_dtype, device=dev)
+            ws_bytes = lib.flexsae_topk_bwd_from_indices_workspace_bytes(ctypes.byref(shape), slice_cols)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            rc = lib.flexsae_topk_bwd_from_indices(
+                ctypes.byref(shape), _ptr(indices), _ptr(weight), _ptr(vals), _ptr(resid), _ptr(g), _ptr(dW),
+                _DTYPES[weight.dtype], _ptr(dvals), _DTYPES[dvals_dtype], _ptr(dbias), _DTYPES[dbias_dtype], _ptr(ws), ws_bytes,
+                flags, _ptr(_flag_for(dev)), _stream())
+            _lib.check(rc, "flexsae_topk_bwd_from_indices")
+            return dW, dvals, dbias
         cached = _pair_lookup(indices, F)
         if cached is not None:
             begin, pair_map = cached
@@ -588,20 +609,15 @@ def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tens
                                        ws_bytes, _ptr(_flag_for(dev)), _stream())
             _lib.check(rc, "flexsae_csr_build")
             _pair_store(indices, F, begin, pair_map)
-        dW = torch.empty_like(weight)
         dvals = torch.empty((B, K), dtype=torch.float32, device=dev)
         dbias = torch.empty((D,), dtype=torch.float32, device=dev)
-        # the slice width only sizes the partial sums of hot latents; one launch over all of D is
-        # fastest, so allow them 256 MiB before slicing
-        slice_cols = max(1, (256 << 20) // max(1, (B * K // 32) * 4))
         bws_bytes = lib.flexsae_topk_bwd_workspace_bytes(ctypes.byref(shape), slice_cols)
         bws = torch.empty(bws_bytes, dtype=torch.uint8, device=dev)
         rc = lib.flexsae_topk_bwd(ctypes.byref(shape), _ptr(begin), _ptr(pair_map), _ptr(indices), _ptr(weight),
                                   _ptr(vals), _ptr(resid), _ptr(g), _ptr(dW), _DTYPES[weight.dtype], _ptr(dvals),
-                                  _ptr(dbias), _ptr(bws), bws_bytes,
-                                  0 if _topk_residual_bf16 else _lib.TOPK_BWD_FP32_RESIDUAL, _stream())
+                                  _ptr(dbias), _ptr(bws), bws_bytes, flags, _stream())
         _lib.check(rc, "flexsae_topk_bwd")
-    return dW, dvals, dbias
+    return (dW, *_leaf_grads(weight, dvals, dvals_dtype, dbias, dbias_dtype, True))
 
 
 topk_bwd = torch.library.custom_op("flexsae_amd::topk_bwd", mutates_args=())(_topk_bwd_impl)
@@ -1116,13 +1132,16 @@ def _hier_backward(ctx, grad_loss, grad_resid, impl=None):
     return None, dW, *_leaf_grads(weight, dvals, vdt, dbias, bdt, impl is not None), None
 
 
-def _topk_backward(ctx, grad_loss, grad_resid, impl=None):
+def _topk_backward(ctx, grad_loss, grad_resid, plain=False):
     indices, weight, vals, resid = ctx.saved_tensors
     if grad_loss is None:
         return None, None, None, None, None
-    dW, dvals, dbias = (impl or topk_bwd)(grad_loss, indices, weight, vals, resid)
     vdt, bdt, tdt = ctx.leaf_dtypes
-    dvals, dbias = _leaf_grads(weight, dvals, vdt, dbias, bdt, impl is not None)
+    if plain:
+        dW, dvals, dbias = _topk_bwd_typed(grad_loss, indices, weight, vals, resid, vdt, bdt)
+    else:
+        dW, dvals, dbias = topk_bwd(grad_loss, indices, weight, vals, resid)
+        dvals, dbias = dvals.to(vdt), dbias.to(bdt)
     dtarget = None
     if ctx.needs_input_grad[4]:
         # the reference's eager loss tail is differentiable w.r.t. target (topk_kernels.py:221)
@@ -1206,7 +1225,7 @@ class _TopkLoss(torch.autograd.Function):
     def backward(ctx, grad_loss):
         if grad_loss is None or not _plain_backward(grad_loss):
             return _topk_backward(ctx, grad_loss, None)
-        return _topk_backward(ctx, grad_loss, None, _topk_bwd_impl)
+        return _topk_backward(ctx, grad_loss, None, True)
 
 
 class _HierLoss(torch.autograd.Function):

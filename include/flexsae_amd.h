@@ -423,6 +423,19 @@ int flexsae_topk_bwd(const flexsae_shape *shape, const uint32_t *begin, const ui
 size_t flexsae_topk_bwd_workspace_bytes(const flexsae_shape *shape, int64_t slice_cols);
 
 /*
+ * flexsae_topk_bwd for a pair list of one call: builds the list of `indices` in the workspace (as flexsae_csr_build, with
+ * `status_flag` as there; fewer launches and passes than the two calls) and writes dvals and dbias rounded once to
+ * `dvals_dtype` and `dbias_dtype`.  Everything else as flexsae_topk_bwd, and the same values.
+ * replaces: additionally the engine's casts to the leaf dtypes (topk_kernels.py:188-223)
+ */
+int flexsae_topk_bwd_from_indices(const flexsae_shape *shape, const int64_t *indices, const void *weight, const void *vals,
+                                  const float *resid, const float *grad_out, void *dW, int dW_dtype, void *dvals,
+                                  int dvals_dtype, void *dbias, int dbias_dtype, void *workspace, size_t workspace_bytes,
+                                  int flags, int *status_flag, void *stream);
+/* Bytes of its workspace; `slice_cols` as in flexsae_topk_bwd_workspace_bytes. */
+size_t flexsae_topk_bwd_from_indices_workspace_bytes(const flexsae_shape *shape, int64_t slice_cols);
+
+/*
  * dst[n] (dtype) = src[n] (fp32), round-to-nearest-even.  Used to hand the fp32
  * scatter accumulator of the hierarchical backward over in the weight's dtype.
  * replaces: the autograd engine's implicit cast of the fp32 gradients returned at
