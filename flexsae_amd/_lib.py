@@ -131,6 +131,25 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_eager = None
+
+
+def eager(general_backward):
+    """The extension module of ordinary eager calls, bound to the library once; ``general_backward`` takes the backwards that
+    are not plain."""
+    global _eager
+    if _eager is None:
+        load()
+        try:
+            from . import _eager as module
+        except ImportError as exc:
+            raise FlexSAELibraryError(f"cannot load flexsae_amd/_eager.so ({exc}): build it with "
+                                      "`python -m flexsae_amd.build` against this torch") from exc
+        module.init(LIB_PATH, general_backward, check)
+        _eager = module
+    return _eager
+
+
 def build_id() -> str:
     """Hash of the sources and flags the loaded library was built from (flexsae_amd/build.py)."""
     return load().flexsae_build_id().decode()

@@ -1,4 +1,5 @@
-"""Builds libflexsae_amd.so (the C-ABI library of HIP kernels) in-tree with hipcc for gfx950.
+"""Builds libflexsae_amd.so (the C-ABI library of HIP kernels) with hipcc for gfx950 and _eager.so (the extension module that
+calls it for ordinary eager calls, over torch's C++ interface) with g++, both in-tree.
 
 Usage: python -m flexsae_amd.build
 """
@@ -9,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libflexsae_amd.so")
+EAGER_PATH = os.path.join(HERE, "_eager.so")
 
 # gfx950 only: some kernels use more LDS per workgroup than the 64 KiB of earlier gfx9 parts
 # (csr_sort_long_kernel 65 600 bytes, the hot-latent variant of the training-step kernel more), the
@@ -44,7 +46,32 @@ def source_id(extra_flags=()) -> str:
     return h.hexdigest()[:16]
 
 
+def build_eager(verbose: bool = False) -> str:
+    import sysconfig
+
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    include = [os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    # (the macros are what torch's own headers ask for; the libraries are loaded by torch, found by name)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in include), os.path.join(CSRC, "eager.cpp"), "-o", EAGER_PATH,
+           "-L" + os.path.join(base, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ltorch"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        sys.stderr.write(proc.stdout + proc.stderr)
+        raise RuntimeError("g++ failed building _eager.so")
+    if verbose and proc.stderr:
+        sys.stderr.write(proc.stderr)
+    return EAGER_PATH
+
+
 def build(verbose: bool = False, extra_flags=()) -> str:
+    build_eager(verbose)
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     cmd = [hipcc, *HIPCC_FLAGS, *extra_flags, f'-DFLEXSAE_BUILD_ID="{source_id(extra_flags)}"', "-o", LIB_PATH,
            os.path.join(CSRC, "flexsae_amd.hip")]

@@ -38,6 +38,8 @@ from . import _lib
 
 _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 
+_eager = None  # the extension module of ordinary eager calls, once one has been made (see _native)
+
 # device index -> int32[1] status flag the kernels OR error bits into (never reset by the ops)
 _status_flags = {}
 _check_indices = os.environ.get("FLEXSAE_CHECK_INDICES", "0") not in ("", "0")
@@ -59,6 +61,8 @@ def _flag_for(device: torch.device) -> Tensor:
     if flag is None:
         flag = torch.zeros(1, dtype=torch.int32, device=device)
         _status_flags[key] = flag
+        if _eager is not None:
+            _eager.set_flag(key, flag)
     return flag
 
 
@@ -369,6 +373,13 @@ def _index_stats(key, B, K, F):
     return st
 
 
+def _new_stats(key):
+    pinned = torch.zeros(3, dtype=torch.int32, pin_memory=True)
+    st = _hot_auto[key] = {"hot": False, "dense": False, "pinned": pinned, "pinned_at": pinned.data_ptr(), "event": None,
+                           "spare": torch.cuda.Event()}
+    return st
+
+
 def _hot_measure(lib, shape, workspace: Tensor, B, K, F, D, weight_dtype) -> None:
     """Leave the skew of this step's indices where the next step of the shape finds it."""
     wanted = ((_hot_latents == "auto" and _hot_latents_supported(B, K, F, D, weight_dtype))
@@ -376,11 +387,7 @@ def _hot_measure(lib, shape, workspace: Tensor, B, K, F, D, weight_dtype) -> Non
     if not wanted or torch.cuda.is_current_stream_capturing():
         return
     key = _hot_key(workspace.device, B, K, F, D, weight_dtype)
-    st = _hot_auto.get(key)
-    if st is None:
-        st = _hot_auto[key] = {"hot": False, "dense": False,
-                               "pinned": torch.zeros(3, dtype=torch.int32, pin_memory=True), "event": None,
-                               "spare": torch.cuda.Event()}
+    st = _hot_auto.get(key) or _new_stats(key)
     if st["event"] is not None:
         return  # a measurement is still on its way
     rc = lib.flexsae_hier_pair_stats(ctypes.byref(shape), _ptr(workspace), _ptr(st["pinned"]), _stream())
@@ -464,10 +471,12 @@ def shared_pair_list():
     outer = _pair_cache
     if outer is None:
         _pair_cache = {}
+        _tell_native()
     try:
         yield
     finally:
         _pair_cache = outer
+        _tell_native()
 
 
 def _pair_key(indices: Tensor, F: int):
@@ -564,6 +573,7 @@ def set_topk_residual_bf16(enabled: bool) -> None:
     faster) or the fp32 residual itself (``vals.grad`` then carries fp32 rounding only)."""
     global _topk_residual_bf16
     _topk_residual_bf16 = bool(enabled)
+    _tell_native()
 
 
 def _topk_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor, resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
@@ -979,6 +989,18 @@ def hierarchical_sae_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bia
         else:
             # (a fill: a copy from host memory would wait for the work queued so far)
             step = torch.full((), float(lr) * float(grad_out), dtype=torch.float32, device=weight.device)
+        native = _native(weight)
+        if native is not None and weight.dim() == 2 and indices.dim() == 2 and weight.dtype in _DTYPES:
+            B, K = indices.shape
+            F, D = weight.shape
+            if B * K * F * D:
+                route = _route(B, K, F, D, weight, True)
+                cols, flags, ws_flags, pinned = route.decide(B, K, F)
+                out = native.hier_sgd(indices, weight, vals, bias, target, step, cols, flags, ws_flags, pinned)
+                if out is not None:
+                    if pinned:
+                        route.measured()
+                    return out
         if _plain_call(indices, weight, vals, bias, target, step):
             torch.autograd.graph.increment_version(weight)  # what the op's schema says of its weight
             return _hier_sgd_step_impl(indices, weight, vals.detach(), bias.detach(), target, step)
@@ -1155,12 +1177,13 @@ topk_fwd.register_autograd(_topk_backward, setup_context=_setup_context)
 
 
 # ---- ordinary eager calls ------------------------------------------------------------------
-# A call on plain tensors with no tracer, mode or transform around it does without the dispatcher: the same functions as the
-# ops run, under an autograd.Function that saves the same tensors.  The wrappers of torch.library.custom_op around forward
-# and backward cost as much as the launches of a small step (us a step with them and without: B = 64, K = 32, F = 4096,
-# D = 256 fp32 TopK 197, 168, hierarchical 233, 188, of which about 70 are the hand-over to autograd's device thread;
-# B = 1024, K = 64, F = 32768, D = 1024 bf16 Zipf, SGD step 179, 127).  Everything else goes through the ops, which tracers,
-# modes and transforms see.
+# A call on plain tensors with no tracer, mode or transform around it does without the dispatcher and, but for what is decided
+# here, without Python: csrc/eager.cpp checks, allocates, launches and has the autograd nodes, which save the tensors that the
+# ops save.  Calls that share a pair list or check their indices, and the late fp16 step, run the ops' functions under an
+# autograd.Function.  Everything else goes through the ops, which tracers, modes and transforms see.
+# us a step with the functions under an autograd.Function and with eager.cpp: B = 64, K = 32, F = 4096, D = 256 fp32 TopK 160
+# and 79, hierarchical 195 and 99 (through the ops 40 to 45 more; the least that torch's engine takes for a forward and a
+# backward of any kind is 45); the host's share of an SGD step 62 and 35.
 _PLAIN_TYPES = (Tensor, torch.nn.Parameter)
 _C = torch._C
 _can_tell_plain = (all(hasattr(_C, n) for n in ("_len_torch_dispatch_stack", "_len_torch_function_stack", "_get_tracing_state"))
@@ -1213,7 +1236,7 @@ def _finish_grads(grad_out, weight: Tensor, dW_unit, dvals: Tensor, vals_dtype, 
 
 
 class _TopkLoss(torch.autograd.Function):
-    """topk_fwd and its backward for ordinary eager calls."""
+    """topk_fwd and its backward on plain tensors."""
 
     @staticmethod
     def forward(ctx, indices, weight, vals, bias, target):
@@ -1229,7 +1252,7 @@ class _TopkLoss(torch.autograd.Function):
 
 
 class _HierLoss(torch.autograd.Function):
-    """hier_fwd and its backward for ordinary eager calls."""
+    """hier_fwd and its backward on plain tensors."""
 
     @staticmethod
     def forward(ctx, indices, weight, vals, bias, target):
@@ -1245,7 +1268,7 @@ class _HierLoss(torch.autograd.Function):
 
 
 class _HierTrainSliced(torch.autograd.Function):
-    """hier_train_sliced and its backward for ordinary eager calls."""
+    """hier_train_sliced and its backward on plain tensors."""
 
     @staticmethod
     def forward(ctx, indices, weight, vals, bias, target, need_dw, hot, dense):
@@ -1312,6 +1335,158 @@ class _HierLateStep(torch.autograd.Function):
         return None, dW, dvals, dbias, None, None, None
 
 
+class _Saved:
+    """What a backward of eager.cpp hands over, as the context the functions above read."""
+
+    def __init__(self, saved, needs):
+        self.saved_tensors = saved
+        self.needs_input_grad = needs
+
+
+_TYPES = {code: dtype for dtype, code in _DTYPES.items()}
+
+
+def _general_backward(kind, grad, saved, needs, numbers, dw_unit):
+    """The backwards of eager.cpp that are not plain, or that a shared pair list may serve: (gradients, unit gradient left)."""
+    ctx = _Saved(saved, needs)
+    plain = _plain_backward(grad)
+    if kind == 0:
+        ctx.leaf_dtypes = (saved[2].dtype, _TYPES[numbers[0]], _TYPES[numbers[1]])
+        return _topk_backward(ctx, grad, None, plain), None
+    if kind == 1:
+        ctx.leaf_dtypes = (saved[2].dtype, _TYPES[numbers[0]], None)
+        return _hier_backward(ctx, grad, None, _hier_bwd_impl if plain else None), None
+    ctx.leaf_dtypes = (saved[2].dtype, saved[3].dtype)
+    ctx.need_dw, ctx.dw_in_place, ctx.dw_unit = bool(numbers[0]), True, dw_unit
+    ctx.hot, ctx.dense = bool(numbers[1] & _lib.BWD_HOT_LATENTS), bool(numbers[1] & _lib.BWD_DENSE_LATENTS)
+    grads = _HierTrainSliced.backward(ctx, grad) if plain else _train_sliced_backward(ctx, grad, None, None, None)
+    return tuple(grads[:5]), ctx.dw_unit
+
+
+def _tell_native() -> None:
+    if _eager is not None:
+        _eager.settings(0 if _topk_residual_bf16 else _lib.TOPK_BWD_FP32_RESIDUAL, int(_pair_cache is not None))
+
+
+def _native(weight: Tensor):
+    """eager.cpp's module, where a call may be its business (it looks at the tensors itself), else None."""
+    global _eager
+    if (torch.compiler.is_compiling() or type(weight) not in _PLAIN_TYPES or not weight.is_cuda or not _can_tell_plain
+            or _check_indices or _pair_cache is not None or torch.autograd.forward_ad._current_level >= 0):
+        return None
+    if _eager is None:
+        _eager = _lib.eager(_general_backward)
+        for index, flag in _status_flags.items():
+            _eager.set_flag(index, flag)
+        _tell_native()
+    if weight.device.index not in _status_flags:
+        _flag_for(weight.device)
+    return _eager
+
+
+# Shapes, types and settings -> _Route: what is decided from them alone.  Bounded: cleared when full.
+_routes = {}
+_ROUTES_MOST = 1024
+
+
+class _Route:
+    """How a hierarchical call with gradients runs: ``train`` the step of hier_train_sliced, else forward and sweep; ``here`` by
+    the functions of this module (the late step, the staged one, the atomic backward); the slices' width plain and with hot
+    latents; what is measured for the next step of the shape."""
+
+    def __init__(self, B, K, F, D, weight, device):
+        dtype, need_dw = weight.dtype, weight.requires_grad
+        takes = _fused_training and (_train_supported(weight, K) or (_train_ragged(weight, K) and _ragged_pays(weight, B, K)))
+        stage = takes and _train_supported(weight, K) and hier_stage_bytes(device) > 0
+        self.train = takes and _hier_scratch_bytes != 0 and (_step_pays(weight, K) or _one_gather_pays(weight, B, K))
+        late = self.train and need_dw and _late_step(weight, B, K)
+        # by the functions of this module
+        self.here = stage or late or _hier_scratch_budget(B, K, F, D, dtype) <= 0
+        self._step(B, K, F, D, dtype, device, need_dw, _lib.BWD_RAGGED_ROWS if _train_ragged(weight, K) else 0)
+
+    def _step(self, B, K, F, D, dtype, device, need_dw, ragged):
+        self.device = device
+        self.key = _hot_key(device, B, K, F, D, dtype)
+        self.ragged = ragged
+        self.cols = _hier_slice_cols(B, K, F, D, dtype)
+        hot_can = need_dw and _hot_latents != "off" and _hot_latents_supported(B, K, F, D, dtype)
+        dense_can = need_dw and _dense_latents != "off" and B * K <= 2 * F
+        self.hot = _hot_latents if hot_can else "off"
+        self.dense = _dense_latents if dense_can else "off"
+        self.asks = self.hot == "auto" or self.dense == "auto"
+        self.measures = need_dw and ((_hot_latents == "auto" and _hot_latents_supported(B, K, F, D, dtype))
+                                     or (_dense_latents == "auto" and B * K <= 2 * F))
+        if hot_can:
+            self.hot_flags = _hot_flags(B, K, D, device)
+            self.hot_cols = _hot_slice_cols(B, self.cols, device)
+
+    def decide(self, B, K, F):
+        """(slice width, flags of the call, flags of the workspace query, pinned memory for the measurement or 0)"""
+        hot, dense = self.hot == "on", self.dense == "on"
+        pinned = 0
+        if self.asks or self.measures:
+            if not torch.cuda.is_current_stream_capturing():
+                st = _index_stats(self.key, B, K, F)
+                if st is not None:
+                    hot = hot or (self.hot == "auto" and st["hot"])
+                    dense = dense or (self.dense == "auto" and st["dense"])
+                if self.measures and (st is None or st["event"] is None):
+                    if st is None:
+                        st = _new_stats(self.key)
+                    pinned = st["pinned_at"]
+        hot_flags = self.hot_flags if hot else 0
+        return (self.hot_cols if hot else self.cols, hot_flags | self.ragged | (_lib.BWD_DENSE_LATENTS if dense else 0),
+                hot_flags | self.ragged, pinned)
+
+    def measured(self):
+        """The measurement that `decide` asked for is on its way."""
+        st = _hot_auto.get(self.key)
+        if st is not None:
+            with _on_device(self.device):
+                st["spare"].record()
+            st["event"] = st["spare"]
+
+
+def _route(B, K, F, D, weight, sgd=False):
+    key = (B, K, F, D, weight.dtype, weight.requires_grad, weight.device.index, sgd, _fused_training, _hier_scratch_bytes,
+           _hier_min_slice_cols, _hier_stage_bytes, _hot_latents, _dense_latents, _ragged_pays, _step_pays, _one_gather_pays,
+           _late_step)
+    route = _routes.get(key)
+    if route is None:
+        if len(_routes) >= _ROUTES_MOST:
+            _routes.clear()
+        if sgd:
+            route = _Route.__new__(_Route)
+            route._step(B, K, F, D, weight.dtype, weight.device, True, 0)
+        else:
+            route = _Route(B, K, F, D, weight, weight.device)
+        _routes[key] = route
+    return route
+
+
+def _native_hier(native, indices, weight, vals, bias, target):
+    """The hierarchical loss by eager.cpp; None: not its business."""
+    if weight.dim() != 2 or indices.dim() != 2 or weight.numel() == 0 or indices.numel() == 0:
+        return None
+    if not (torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad)):
+        # (target alone may take part: it gets no gradient)
+        return native.hier_loss(indices, weight, vals, bias, target, 0) if not target.requires_grad else None
+    if weight.dtype not in _DTYPES:
+        return None
+    B, K = indices.shape
+    F, D = weight.shape
+    route = _route(B, K, F, D, weight)
+    if route.here:
+        return None
+    if not route.train:
+        return native.hier_loss(indices, weight, vals, bias, target, route.cols)
+    cols, flags, ws_flags, pinned = route.decide(B, K, F)
+    loss = native.hier_sliced(indices, weight, vals, bias, target, weight.requires_grad, cols, flags, ws_flags, pinned)
+    if pinned and loss is not None:
+        route.measured()
+    return loss
+
+
 def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,
                                  target: Tensor) -> Tensor:
     """Fused HierarchicalTopK decoder loss (0-dim fp32), differentiable w.r.t. weight, vals, bias.
@@ -1320,6 +1495,11 @@ def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, 
     (torch-ext/flex_sae/hierarchical_kernels.py:302-309); the kernels underneath are HIP."""
     if indices.dtype == torch.int32:
         indices = indices.to(torch.int64)
+    native = _native(weight)
+    if native is not None:
+        loss = _native_hier(native, indices, weight, vals, bias, target)
+        if loss is not None:
+            return loss
     needs_grad = torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad)
     if (needs_grad and _fused_training and weight.dim() == 2 and indices.dim() == 2
             and (_train_supported(weight, indices.shape[1])
@@ -1357,6 +1537,11 @@ def triton_topk_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Te
     (torch-ext/flex_sae/topk_kernels.py:213-223); the kernels underneath are HIP."""
     if indices.dtype == torch.int32:
         indices = indices.to(torch.int64)
+    native = _native(weight)
+    if native is not None:
+        loss = native.topk_loss(indices, weight, vals, bias, target)
+        if loss is not None:
+            return loss
     if _plain_call(indices, weight, vals, bias, target):
         if torch.is_grad_enabled() and (weight.requires_grad or vals.requires_grad or bias.requires_grad or target.requires_grad):
             return _TopkLoss.apply(indices, weight, vals, bias, target)

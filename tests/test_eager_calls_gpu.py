@@ -200,3 +200,63 @@ def test_tensors_whose_memory_is_not_their_values(loss):
     assert torch.equal(W, W2) and all(torch.equal(x, y) for x, y in zip(got, want))
     with pytest.raises((ValueError, RuntimeError)):
         flex.hierarchical_sae_sgd_step(idx, torch._efficientzerotensor(W.shape, device=DEV), v, b, t, 0.5)
+
+
+@pytest.mark.parametrize("entry", ["topk_loss", "hier_loss", "hier_sliced"])
+def test_what_the_extension_module_takes(entry):
+    """Plain tensors of fitting shapes, contiguous or not; the rest it leaves to the ops, which see it or say what is wrong."""
+    args = [x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=8)]
+    idx, W, v, b, t = args
+    LOSS["topk"](*args)
+    fn = getattr(ops._native(W), entry)
+    more = {"topk_loss": (), "hier_loss": (128,), "hier_sliced": (True, 128, 0, 0, 0)}[entry]
+    want = fn(*args, *more)
+    assert torch.equal(want, LOSS["topk" if entry == "topk_loss" else "hier"](*args))
+    strided = [x.repeat_interleave(2, -1)[..., ::2] for x in args]
+    assert not strided[1].is_contiguous() and torch.equal(fn(*strided, *more), want)
+    odd = W.new_empty(W.numel() + 1)[1:].view_as(W).copy_(W)
+    assert odd.data_ptr() % 16 and torch.equal(fn(idx, odd, v, b, t, *more), want)
+
+    class Sub(torch.Tensor):
+        pass
+
+    refused = [(idx, W.as_subclass(Sub), v, b, t), (idx, W, v, b, t.cpu()), (idx.int(), W, v, b, t), (idx, W.double(), v, b, t),
+               (idx, W, v[:, :4], b, t), (idx, W, v, b[:64], t), (idx[:0], W, v[:0], b, t[:0]), (idx, W[0], v, b, t),
+               (idx, torch._neg_view(W), v, b, t), (idx, torch._efficientzerotensor(W.shape, device=DEV), v, b, t)]
+    for wrong in refused:
+        assert fn(*wrong, *more) is None
+    with _Seen():
+        assert fn(*args, *more) is None
+    with pytest.raises(TypeError):
+        fn(*args)[0] if more else fn(*args, 1)
+    seen = []
+    torch.func.vmap(lambda x: seen.append(fn(idx, W, x, b, t, *more)) or x)(torch.stack([v, v]))
+    assert seen == [None]
+
+
+@pytest.mark.parametrize("loss", ["topk", "hier"])
+def test_other_threads_and_streams(loss):
+    """Forward and backward on a stream and a thread of their own, several at once: each the same bits."""
+    import threading
+
+    args = [x.to(DEV) for x in make_inputs(64, 16, 300, 256, torch.bfloat16, seed=9)]
+    want = _step(loss, args, 2.0)
+    got = [None] * 4
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            for _ in range(5):
+                got[i] = _step(loss, args, 2.0)
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    torch.cuda.synchronize()
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    for grads in got:
+        assert all(torch.equal(x, y) for x, y in zip(grads, want))
