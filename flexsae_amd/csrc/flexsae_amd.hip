@@ -804,6 +804,12 @@ void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int6
   // K == KMAX (the usual powers of two) runs the variant without per-step bound tests, part of its
   // row pieces in the LDS
   const bool stream = slice_w >= d_pad;  // all of P in one launch: streaming stores
+  // Tiles of a row one after the other where there are too few rows for the wavefronts on the chip (4096) to share the pieces
+  // of one tile anyway: what is gathered and stored of a row then lies side by side.  us of the step by tile / by row: B=1024,
+  // K=64, F=65536, D=4096 bf16 407 / 387, B=128, K=128, F=16384, D=2048 73 / 66, B=512, K=64, F=65536, D=2048 fp32 274 / 255,
+  // B=207, K=90, F=68238, D=2348 fp16 228 / 224, B=1777, K=50, F=24571, D=1538 193 / 187; not B=2048, K=64, F=32768, D=1024 bf16
+  // 165 / 167, B=4096, K=128, F=65536, D=2304 1224 / 1257.
+  const int row_tiles = s->B < 2048 ? static_cast<int>(cols / (kWave * VEC)) : 0;
   const auto kernel = s->K == KMAX
                           ? (stream ? hier_train_kernel<WT, PT, KMAX, true, true, VEC, LDSROWS>
                                     : hier_train_kernel<WT, PT, KMAX, true, false, VEC, LDSROWS>)
@@ -811,7 +817,7 @@ void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int6
                                     : hier_train_kernel<WT, PT, KMAX, false, false, VEC, 0>);
   hipLaunchKernelGGL(kernel, dim3(fin.n_blocks + static_cast<unsigned>(ceil_div(n_items, kWavesPerBlock))), dim3(kBlock),
                      0, st, indices, weight, vals, s->vals_dtype, ta.bias, s->bias_dtype, ta.target, s->target_dtype,
-                     coef, slot, P, dvals, s_final, d_pad, loss_partial, status_flag, n_items, s->B, col0,
+                     coef, slot, P, dvals, s_final, d_pad, loss_partial, status_flag, n_items, s->B, row_tiles, col0,
                      slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), slot_mask(s), dW_solo, fin);
 }
 

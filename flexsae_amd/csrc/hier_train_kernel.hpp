@@ -68,6 +68,7 @@ struct RowPiece<f16_t, 2> {
 // back with plain LDS loads.  bias - target is fetched before the gathers are issued: the memory
 // counter retires in order, so anything issued after them can only be waited for together with
 // all of them, and the forward walk could not start while rows are still arriving.
+// row_tiles: 0: the items are all rows of one tile after the other; else so many tiles of one row after the other.
 // fin: the second step of the previous slice's hot latents (see HotFinalize), run by the leading blocks
 // of the launch into a gradient of CarriedGrad's type, or into the weights.
 // STREAM: the contributions are stored with the non-temporal hint.  That is the faster choice
@@ -89,7 +90,7 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
     const void *__restrict__ target, int target_dtype, float coef,
     const uint32_t *__restrict__ slot, void *__restrict__ P, float *__restrict__ dv_part,
     float *__restrict__ s_final, int s_final_ld, float *__restrict__ loss_partial,
-    int *status_flag, int64_t n_items, int64_t B, int col0, int slice_w, int K, int64_t F, int D, uint32_t slot_mask,
+    int *status_flag, int64_t n_items, int64_t B, int row_tiles, int col0, int slice_w, int K, int64_t F, int D, uint32_t slot_mask,
     void *__restrict__ dW, HotFinalize fin) {
   using Piece = RowPiece<WT, VEC>;
   using raw_t = typename Piece::raw_t;
@@ -108,8 +109,15 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
   }
   const int64_t item = static_cast<int64_t>(blockIdx.x - fin.n_blocks) * (blockDim.x >> 6) + wave_in_block();
   if (item >= n_items) return;  // uniform per wavefront
-  const int t = static_cast<int>(item / B);
-  const int64_t b = item - static_cast<int64_t>(t) * B;
+  int t;
+  int64_t b;
+  if (row_tiles > 0) {  // uniform
+    b = item / row_tiles;
+    t = static_cast<int>(item - b * row_tiles);
+  } else {
+    t = static_cast<int>(item / B);
+    b = item - static_cast<int64_t>(t) * B;
+  }
   const int pc = t * (kWave * VEC) + lane * VEC;  // column inside the slice
   const int d0 = col0 + pc;
   const bool active = d0 < D;

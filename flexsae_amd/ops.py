@@ -206,6 +206,7 @@ topk_fwd.register_fake(_fwd_fake)
 _hier_scratch_bytes = (int(os.environ["FLEXSAE_HIER_SCRATCH_MB"]) << 20) if "FLEXSAE_HIER_SCRATCH_MB" in os.environ else None
 _HIER_SCRATCH_CAP = 256 << 20
 _HIER_SCRATCH_LEAST = 128 << 20
+_HIER_SCRATCH_WHOLE = 384 << 20
 
 
 # Narrowest slice the scratch budget may lead to on its own; a budget that gives fewer columns is
@@ -241,11 +242,20 @@ def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype) -> int:
     launch, leave compute units idle (us with 0.45 of the weights, 64 and 128 MiB: B = 1777, K = 50,
     F = 24571, D = 1538 bf16 284, 277, 246; B = 512, K = 128, F = 16384, D = 8192 bf16 730, 697, 675;
     B = 1024, K = 256, F = 16384, D = 2048 fp32 1260, 1261, 1035; B = 200, K = 250, F = 8000,
-    D = 2048 fp32 679, 364, 350)."""
+    D = 2048 fp32 679, 364, 350).  With such weights all contributions at once where they take at most 384 MiB (us with
+    128 MiB / all: B = 1500, K = 40, F = 24571, D = 2328 bf16 208 / 189, fp32 D = 1160 206 / 183, fp16 205 / 192; B = 512,
+    K = 64, F = 16384, D = 5488 bf16 248 / 219; B = 400, K = 100, F = 60000, D = 1872 166 / 144; over 64 shapes 4 % less on
+    average, one more than 4 % more: B = 1900, K = 128, F = 8192, D = 152 fp32 124 / 131)."""
     if _hier_scratch_bytes is not None:
         return _hier_scratch_bytes
     sw = 4 if weight_dtype == torch.float32 else 2
-    return min(_HIER_SCRATCH_CAP, max(_HIER_SCRATCH_LEAST, int(0.45 * F * D * sw)))
+    budget = min(_HIER_SCRATCH_CAP, max(_HIER_SCRATCH_LEAST, int(0.45 * F * D * sw)))
+    if budget == _HIER_SCRATCH_LEAST:
+        tile = _train_tile_cols(K, weight_dtype)
+        whole = B * K * (-(-D // tile) * tile) * (2 if weight_dtype == torch.bfloat16 else 4)
+        if whole <= _HIER_SCRATCH_WHOLE:
+            return max(budget, whole)
+    return budget
 
 
 def _hier_slice_cols(B: int, K: int, F: int, D: int, weight_dtype) -> int:
@@ -262,7 +272,7 @@ def set_hier_scratch_bytes(nbytes) -> None:
     """Upper bound on the scratch of the hierarchical backward (bytes): the per-pair contributions
     of one slice of columns.  0 = use the atomic scatter fallback, which needs no scratch but an
     fp32 [F,D] accumulator.  ``None`` (the default) sizes it from the problem: 0.45 of the weight
-    matrix, at least 128 and at most 256 MiB.  A slice is never narrower than ``set_hier_min_slice_cols``, so with
+    matrix, at least 128 and at most 256 MiB, or, of weights for which that is 128 MiB, all contributions up to 384 MiB.  A slice is never narrower than ``set_hier_min_slice_cols``, so with
     many pairs the scratch can exceed the bound by a large factor (B*K*256 contributions).  Slices
     of 256 columns measured fastest at B*K = 2^19 pairs; wider ones are not faster."""
     global _hier_scratch_bytes
