@@ -82,6 +82,8 @@ SIGNATURES = {
     "flexsae_hier_fwd_bwd": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p, _p, _sz, _int, _p, _p]),
     "flexsae_hier_fwd_bwd_scaled": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p, _p, _sz, _int, _p, _p]),
     "flexsae_hier_sgd_step": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _int, _p, _p]),
+    "flexsae_hier_step": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p, _p, _sz, _int, _p, ctypes.c_uint32, _p,
+                                 _p]),
     "flexsae_scale": (_int, [_p, _p, _int, _i64, _p, _p]),
     "flexsae_hier_bwd_atomic": (_int, [_shape_p, _p, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p]),
     "flexsae_csr_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -36,7 +36,7 @@ using torch::autograd::variable_list;
 #define FLEXSAE_ENTRIES(X)                                                                                              \
   X(abi_version) X(fwd_workspace_bytes) X(topk_fwd_best_workspace_bytes) X(topk_fwd) X(hier_fwd)                        \
   X(topk_bwd_from_indices_workspace_bytes) X(topk_bwd_from_indices) X(hier_bwd_workspace_bytes) X(hier_bwd)             \
-  X(hier_fwd_bwd_workspace_bytes_flags) X(hier_fwd_bwd) X(hier_sgd_step) X(hier_pair_stats) X(finish_grads)
+  X(hier_fwd_bwd_workspace_bytes_flags) X(hier_step) X(finish_grads)
 struct Library {
 #define X(name) decltype(&flexsae_##name) name = nullptr;
   FLEXSAE_ENTRIES(X)
@@ -204,38 +204,55 @@ struct StepPlan {
   int64_t slice_cols;
   int64_t flags;     // of the call
   int64_t ws_flags;  // of the workspace query
+  Tensor stats;      // pinned memory for what the pair list says about the indices (undefined: not wanted) ...
+  int64_t tag;       // ... and the mark that it has arrived
 };
 
 struct Step {
   Tensor loss, dvals, dbias, dW;
 };
 
-Step hier_step(const Inputs &given, const StepPlan &p, void *stats) {
+// grad (undefined: the unit gradient, of fp16 weights in fp32): dW is the gradient for it in the weight's type.
+// step: dW is not formed, the weights move by it.
+Step hier_step(const Inputs &given, const StepPlan &p, const Tensor &grad = Tensor(), const Tensor &step = Tensor()) {
   const c10::DeviceGuard guard(given.weight.device());
   const Inputs in = prepared(given);
   const flexsae_shape s = shape_of(in);
   const size_t bytes = lib.hier_fwd_bwd_workspace_bytes_flags(&s, p.slice_cols, static_cast<int>(p.ws_flags));
   const Tensor workspace = make_workspace(in.weight, bytes);
-  const auto type = in.weight.scalar_type() == c10::ScalarType::Half ? c10::ScalarType::Float : in.weight.scalar_type();
+  const bool half = in.weight.scalar_type() == c10::ScalarType::Half;
+  const auto type = half && !grad.defined() ? c10::ScalarType::Float : in.weight.scalar_type();
   Step r;
   r.loss = make(in.weight, {}, c10::ScalarType::Float);
-  if (p.need_dw) r.dW = make(in.weight, {s.F, s.D}, type);
+  if (p.need_dw && !step.defined()) r.dW = make(in.weight, {s.F, s.D}, type);
   r.dvals = make(in.weight, {s.B, s.K}, c10::ScalarType::Float);
   r.dbias = make(in.weight, {s.D}, c10::ScalarType::Float);
-  check(lib.hier_fwd_bwd(&s, index_ptr(in.indices), in.weight.data_ptr(), in.vals.data_ptr(), in.bias.data_ptr(),
-                         in.target.data_ptr(), f32(r.loss), p.need_dw ? r.dW.data_ptr() : nullptr, dtype_of(type),
-                         f32(r.dvals), f32(r.dbias), workspace.data_ptr(), bytes,
-                         static_cast<int>(p.flags) | (p.need_dw ? 0 : FLEXSAE_BWD_NO_DW), flag_of(in.weight),
-                         stream_of(in.weight)),
-        "flexsae_hier_fwd_bwd");
-  if (stats)
-    check(lib.hier_pair_stats(&s, workspace.data_ptr(), static_cast<uint32_t *>(stats), stream_of(in.weight)),
-          "flexsae_hier_pair_stats");
+  const Tensor g = grad.defined() ? grad_scalar(grad, in.weight.device()) : Tensor();
+  const Tensor by = step.defined() ? grad_scalar(step, in.weight.device()) : Tensor();
+  check(lib.hier_step(&s, index_ptr(in.indices), in.weight.data_ptr(), in.vals.data_ptr(), in.bias.data_ptr(),
+                      in.target.data_ptr(), g.defined() ? f32(g) : nullptr, by.defined() ? f32(by) : nullptr, f32(r.loss),
+                      r.dW.defined() ? r.dW.data_ptr() : nullptr, dtype_of(type), f32(r.dvals), f32(r.dbias),
+                      workspace.data_ptr(), bytes, static_cast<int>(p.flags) | (p.need_dw ? 0 : FLEXSAE_BWD_NO_DW),
+                      p.stats.defined() ? static_cast<uint32_t *>(p.stats.data_ptr()) : nullptr,
+                      static_cast<uint32_t>(p.tag), flag_of(in.weight), stream_of(in.weight)),
+        "flexsae_hier_step");
   return r;
 }
 
 // ---- autograd ------------------------------------------------------------------------------
-enum Kind { kTopk = 0, kHier = 1, kSliced = 2 };
+enum Kind { kTopk = 0, kHier = 1, kSliced = 2, kLate = 3 };
+
+void save_plan(AutogradContext *ctx, const StepPlan &plan) {
+  ctx->saved_data["need_dw"] = static_cast<int64_t>(plan.need_dw);
+  ctx->saved_data["cols"] = plan.slice_cols;
+  ctx->saved_data["flags"] = plan.flags;
+  ctx->saved_data["ws_flags"] = plan.ws_flags;
+}
+
+StepPlan saved_plan(AutogradContext *ctx) {
+  return {ctx->saved_data["need_dw"].toInt() != 0, ctx->saved_data["cols"].toInt(), ctx->saved_data["flags"].toInt(),
+          ctx->saved_data["ws_flags"].toInt(), Tensor(), 0};
+}
 
 // A backward that is not plain, by ops.py; dW: the unit gradient, which it may take or leave.
 variable_list backward_in_python(AutogradContext *ctx, Kind kind, const Tensor &grad, const variable_list &saved,
@@ -350,29 +367,25 @@ struct HierLoss : torch::autograd::Function<HierLoss> {
 
 struct SlicedLoss : torch::autograd::Function<SlicedLoss> {
   static Variable forward(AutogradContext *ctx, const Variable &indices, const Variable &weight, const Variable &vals,
-                          const Variable &bias, const Variable &target, const StepPlan &plan, void *stats) {
-    Step r = hier_step({indices, weight, vals, bias, target}, plan, stats);
+                          const Variable &bias, const Variable &target, const StepPlan &plan) {
+    Step r = hier_step({indices, weight, vals, bias, target}, plan);
     ctx->save_for_backward({indices, weight, vals, bias, target, r.dvals, r.dbias});
     ctx->set_materialize_grads(false);
     // the unit gradient is no saved tensor: the backward scales it in place and hands the very buffer on
     if (plan.need_dw) ctx->saved_data["dW"] = r.dW;
-    ctx->saved_data["need_dw"] = static_cast<int64_t>(plan.need_dw);
-    ctx->saved_data["cols"] = plan.slice_cols;
-    ctx->saved_data["flags"] = plan.flags;
-    ctx->saved_data["ws_flags"] = plan.ws_flags;
+    save_plan(ctx, plan);
     return r.loss;
   }
 
   static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
     auto saved = ctx->get_saved_variables();
     const Tensor &grad = grads[0];
-    if (!grad.defined()) return variable_list(7);
+    if (!grad.defined()) return variable_list(6);
     const auto at = ctx->saved_data.find("dW");
     Tensor dW = at != ctx->saved_data.end() ? at->second.toTensor() : Tensor();
-    const StepPlan plan = {ctx->saved_data["need_dw"].toInt() != 0, ctx->saved_data["cols"].toInt(),
-                           ctx->saved_data["flags"].toInt(), ctx->saved_data["ws_flags"].toInt()};
+    const StepPlan plan = saved_plan(ctx);
     if (!plain_backward(grad) || (lists_in_python && !dW.defined())) {
-      auto out = backward_in_python(ctx, kSliced, grad, saved, {plan.need_dw, plan.flags}, &dW, 7);
+      auto out = backward_in_python(ctx, kSliced, grad, saved, {plan.need_dw, plan.flags}, &dW, 6);
       if (dW.defined()) ctx->saved_data["dW"] = dW;
       else ctx->saved_data.erase("dW");
       return out;
@@ -382,7 +395,7 @@ struct SlicedLoss : torch::autograd::Function<SlicedLoss> {
       TORCH_CHECK(plan.need_dw, "the step ran without dW but weight requires a gradient");
       ctx->saved_data.erase("dW");  // the buffer now belongs to whoever receives the gradient
       if (!dW.defined()) {          // a second backward through a retained graph: the buffer went with the first one
-        Step again = hier_step({saved[0], saved[1], saved[2], saved[3], saved[4]}, plan, nullptr);
+        Step again = hier_step({saved[0], saved[1], saved[2], saved[3], saved[4]}, plan);
         dW = again.dW;
         dvals = again.dvals;
         dbias = again.dbias;
@@ -392,7 +405,40 @@ struct SlicedLoss : torch::autograd::Function<SlicedLoss> {
     }
     const c10::DeviceGuard guard(saved[1].device());
     auto [w, v, b] = finish(grad, saved[1], dW, dvals, saved[2].scalar_type(), dbias, saved[3].scalar_type());
-    return {Tensor(), w, v, b, Tensor(), Tensor(), Tensor()};
+    return {Tensor(), w, v, b, Tensor(), Tensor()};
+  }
+};
+
+// The loss alone in the forward, the step with the upstream gradient in the backward (_late_step in ops.py).
+struct LateLoss : torch::autograd::Function<LateLoss> {
+  static Variable forward(AutogradContext *ctx, const Variable &indices, const Variable &weight, const Variable &vals,
+                          const Variable &bias, const Variable &target, const StepPlan &plan) {
+    auto [loss, resid] = ::forward(false, {indices, weight, vals, bias, target});
+    ctx->save_for_backward({indices, weight, vals, bias, target});
+    ctx->set_materialize_grads(false);
+    save_plan(ctx, plan);
+    if (plan.stats.defined()) ctx->saved_data["stats"] = plan.stats;
+    ctx->saved_data["tag"] = plan.tag;
+    return loss;
+  }
+
+  static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &grad = grads[0];
+    if (!grad.defined()) return variable_list(6);
+    StepPlan plan = saved_plan(ctx);
+    if (!plain_backward(grad) || lists_in_python)
+      return backward_in_python(ctx, kLate, grad, saved, {plan.need_dw, plan.flags}, nullptr, 6);
+    const auto at = ctx->saved_data.find("stats");
+    if (at != ctx->saved_data.end()) {
+      plan.stats = at->second.toTensor();
+      plan.tag = ctx->saved_data["tag"].toInt();
+      ctx->saved_data.erase("stats");
+    }
+    const Step r = hier_step({saved[0], saved[1], saved[2], saved[3], saved[4]}, plan, grad);
+    const c10::DeviceGuard guard(saved[1].device());
+    auto [w, v, b] = finish(grad, saved[1], Tensor(), r.dvals, saved[2].scalar_type(), r.dbias, saved[3].scalar_type());
+    return {Tensor(), r.dW, v, b, Tensor(), Tensor()};
   }
 };
 
@@ -453,59 +499,56 @@ PyObject *py_hier_loss(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// hier_sliced(indices, weight, vals, bias, target, need_dw, slice_cols, flags, ws_flags, stats) -> loss: the training step
-PyObject *py_hier_sliced(PyObject *, PyObject *const *args, Py_ssize_t n) {
+// need_dw (or the step of an update), slice_cols, flags, ws_flags, stats, tag
+constexpr Py_ssize_t kPlanArguments = 6;
+StepPlan take_plan(PyObject *const *args, bool need_dw) {
+  StepPlan plan = {need_dw, number(args[1]), number(args[2]), number(args[3]), Tensor(), number(args[5])};
+  if (THPVariable_Check(args[4])) plan.stats = THPVariable_Unpack(args[4]);
+  return plan;
+}
+
+template <typename Loss>
+PyObject *step_loss(PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Inputs in;
-  if (!arguments(n, 10)) return nullptr;
+  if (!arguments(n, 5 + kPlanArguments)) return nullptr;
   if (!take_inputs(args, in)) Py_RETURN_NONE;
-  const StepPlan plan = {number(args[5]) != 0, number(args[6]), number(args[7]), number(args[8])};
-  void *const stats = reinterpret_cast<void *>(number(args[9]));
+  const StepPlan plan = take_plan(args + 5, number(args[5]) != 0);
   Tensor loss;
   {
     pybind11::gil_scoped_release no_gil;
-    loss = SlicedLoss::apply(in.indices, in.weight, in.vals, in.bias, in.target, plan, stats);
+    loss = Loss::apply(in.indices, in.weight, in.vals, in.bias, in.target, plan);
   }
   return THPVariable_Wrap(loss);
   END_HANDLE_TH_ERRORS
 }
 
-// hier_sgd(indices, weight, vals, bias, target, step, slice_cols, flags, ws_flags, stats) -> (loss, dvals, dbias)
+// hier_sliced(indices, weight, vals, bias, target, need_dw, slice_cols, flags, ws_flags, stats, tag) -> loss: the training step
+PyObject *py_hier_sliced(PyObject *, PyObject *const *args, Py_ssize_t n) { return step_loss<SlicedLoss>(args, n); }
+// hier_late(the same): the loss, and the step in the backward
+PyObject *py_hier_late(PyObject *, PyObject *const *args, Py_ssize_t n) { return step_loss<LateLoss>(args, n); }
+
+// hier_sgd(indices, weight, vals, bias, target, step, slice_cols, flags, ws_flags, stats, tag) -> (loss, dvals, dbias)
 PyObject *py_hier_sgd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Inputs in;
-  if (!arguments(n, 10)) return nullptr;
+  if (!arguments(n, 5 + kPlanArguments)) return nullptr;
   if (!take_inputs(args, in) || !THPVariable_CheckExact(args[5])) Py_RETURN_NONE;
   const Tensor step = THPVariable_Unpack(args[5]);
   if (!plain_tensor(step) || in.weight.is_inference() || !in.weight.is_contiguous() ||
       reinterpret_cast<uintptr_t>(in.weight.data_ptr()) % 16 || in.weight.size(1) % 4 || in.indices.size(1) > 256)
     Py_RETURN_NONE;
-  const int64_t cols = number(args[6]), flags = number(args[7]), ws_flags = number(args[8]);
-  void *const stats = reinterpret_cast<void *>(number(args[9]));
-  Tensor loss, dvals, dbias;
+  const StepPlan plan = take_plan(args + 5, true);
+  Step r;
   {
     pybind11::gil_scoped_release no_gil;
     const c10::AutoGradMode no_grad(false);
-    const c10::DeviceGuard guard(in.weight.device());
     torch::autograd::impl::bump_version(in.weight);
-    const Tensor indices = prepared(in.indices), vals = prepared(in.vals.detach()), bias = prepared(in.bias.detach()),
-                 target = prepared(in.target);
-    const flexsae_shape s = shape_of(in);
-    const size_t bytes = lib.hier_fwd_bwd_workspace_bytes_flags(&s, cols, static_cast<int>(ws_flags));
-    const Tensor workspace = make_workspace(in.weight, bytes);
-    loss = make(in.weight, {}, c10::ScalarType::Float);
-    dvals = make(in.weight, {s.B, s.K}, c10::ScalarType::Float);
-    dbias = make(in.weight, {s.D}, c10::ScalarType::Float);
-    const Tensor g = grad_scalar(step, in.weight.device());
-    check(lib.hier_sgd_step(&s, index_ptr(indices), in.weight.data_ptr(), vals.data_ptr(), bias.data_ptr(), target.data_ptr(),
-                            f32(g), f32(loss), f32(dvals), f32(dbias), workspace.data_ptr(), bytes, static_cast<int>(flags),
-                            flag_of(in.weight), stream_of(in.weight)),
-          "flexsae_hier_sgd_step");
-    if (stats)
-      check(lib.hier_pair_stats(&s, workspace.data_ptr(), static_cast<uint32_t *>(stats), stream_of(in.weight)),
-            "flexsae_hier_pair_stats");
+    in.vals = in.vals.detach();
+    in.bias = in.bias.detach();
+    r = hier_step(in, plan, Tensor(), step);
   }
-  return Py_BuildValue("NNN", THPVariable_Wrap(loss), THPVariable_Wrap(dvals), THPVariable_Wrap(dbias));
+  return Py_BuildValue("NNN", THPVariable_Wrap(r.loss), THPVariable_Wrap(r.dvals), THPVariable_Wrap(r.dbias));
   END_HANDLE_TH_ERRORS
 }
 
@@ -554,7 +597,7 @@ PyObject *py_init(PyObject *, PyObject *const *args, Py_ssize_t n) {
 #define FLEXSAE_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {FLEXSAE_METHOD(init),       FLEXSAE_METHOD(set_flag),    FLEXSAE_METHOD(settings),
                          FLEXSAE_METHOD(topk_loss),  FLEXSAE_METHOD(hier_loss),   FLEXSAE_METHOD(hier_sliced),
-                         FLEXSAE_METHOD(hier_sgd),   {nullptr, nullptr, 0, nullptr}};
+                         FLEXSAE_METHOD(hier_late),  FLEXSAE_METHOD(hier_sgd),    {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_eager", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

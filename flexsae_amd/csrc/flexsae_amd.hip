@@ -645,7 +645,7 @@ struct HierBwdPlan {
   // latents, the candidates and what became of them, the long latents that stayed cold and their
   // chunk table
   bool hot;
-  size_t off_hslot, off_hot_ctrl, off_hot_list, off_cand_list, off_cand_state, off_long_cand, off_long2, off_chunk2;
+  size_t off_hslot, off_hot_ctrl, off_hot_list, off_cand_list, off_long2, off_chunk2;
   int hot_rows;            // rows per block of the accumulator kernel
   size_t n_row_blocks;     // blocks of that many rows
 };
@@ -705,10 +705,6 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 
     off += round_up(kHotMax * 4, kAlign);
     p.off_cand_list = off;
     off += round_up(kHotMax * 4, kAlign);
-    p.off_cand_state = off;
-    off += round_up(kHotMax * 4, kAlign);
-    p.off_long_cand = off;
-    off += round_up(n_long_max * 4, kAlign);
     p.off_long2 = off;
     off += round_up(n_long_max * 4, kAlign);
     p.off_chunk2 = off;
@@ -760,6 +756,7 @@ struct TrainArgs {
   float *loss;              // finished by the epilogue from the per-(tile, row) partials
   int64_t n_loss_partials;
   double inv_count;         // 1 / (B*K*D)
+  PairStats stats;          // likewise
 };
 
 // what of slot[] is the slot: all of it, or all but the mark of a latent's only pair
@@ -798,7 +795,8 @@ template <typename WT, typename PT, int KMAX, int VEC = 2>
 void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int64_t *indices,
                          const void *weight, const void *vals, float coef, const uint32_t *slot, void *P,
                          float *dvals, float *s_final, int d_pad, float *loss_partial, int *status_flag,
-                         int64_t cols, int col0, int slice_w, hipStream_t st, const HotFinalize &fin, void *dW_solo) {
+                         int64_t cols, int col0, int slice_w, hipStream_t st, const HotFinalize &fin, void *dW_solo,
+                         const ZeroRows &zero) {
   constexpr int LDSROWS = train_lds_rows<WT, KMAX, VEC>();
   const int64_t n_items = s->B * (cols / (kWave * VEC));
   // K == KMAX (the usual powers of two) runs the variant without per-step bound tests, part of its
@@ -815,10 +813,10 @@ void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int6
                                     : hier_train_kernel<WT, PT, KMAX, true, false, VEC, LDSROWS>)
                           : (stream ? hier_train_kernel<WT, PT, KMAX, false, true, VEC, 0>
                                     : hier_train_kernel<WT, PT, KMAX, false, false, VEC, 0>);
-  hipLaunchKernelGGL(kernel, dim3(fin.n_blocks + static_cast<unsigned>(ceil_div(n_items, kWavesPerBlock))), dim3(kBlock),
-                     0, st, indices, weight, vals, s->vals_dtype, ta.bias, s->bias_dtype, ta.target, s->target_dtype,
+  hipLaunchKernelGGL(kernel, dim3(fin.n_blocks + static_cast<unsigned>(ceil_div(n_items, kWavesPerBlock)) + zero.n_blocks),
+                     dim3(kBlock), 0, st, indices, weight, vals, s->vals_dtype, ta.bias, s->bias_dtype, ta.target, s->target_dtype,
                      coef, slot, P, dvals, s_final, d_pad, loss_partial, status_flag, n_items, s->B, row_tiles, col0,
-                     slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), slot_mask(s), dW_solo, fin);
+                     slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), slot_mask(s), dW_solo, fin, zero);
 }
 
 template <typename WT, typename PT>
@@ -826,10 +824,10 @@ void launch_train_kernel_k(const flexsae_shape *s, const TrainArgs &ta, const in
                            const void *weight, const void *vals, float coef, const uint32_t *slot, void *P,
                            float *dvals, float *s_final, int d_pad, float *loss_partial,
                            int *status_flag, int64_t cols, int col0, int slice_w, hipStream_t st,
-                           const HotFinalize &fin, void *dW_solo) {
+                           const HotFinalize &fin, void *dW_solo, const ZeroRows &zero) {
 #define FLEXSAE_TRAIN(KM)                                                                              \
   launch_train_kernel<WT, PT, KM>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,  \
-                                  loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo)
+                                  loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo, zero)
   // (the fp32 16-step instantiation allocates registers badly; 32 covers it)
   if (s->K <= 16 && sizeof(typename Traits<WT>::store_t) == 2) {
     FLEXSAE_TRAIN(16);
@@ -845,10 +843,10 @@ void launch_train_kernel_k(const flexsae_shape *s, const TrainArgs &ta, const in
     }
   } else if (s->K <= 128) {  // fp32 rows of 65..128 steps: one column per lane
     launch_train_kernel<WT, PT, 128, 1>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,
-                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo);
+                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo, zero);
   } else {
     launch_train_kernel<WT, PT, 256, 1>(s, ta, indices, weight, vals, coef, slot, P, dvals, s_final, d_pad,
-                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo);
+                                        loss_partial, status_flag, cols, col0, slice_w, st, fin, dW_solo, zero);
   }
 #undef FLEXSAE_TRAIN
 }
@@ -1042,9 +1040,17 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   // rows of latents without pairs are zeroed here, whole rows in one pass (the in-place update leaves
   // them alone).
   const bool sparse = piece != 0 && sparse_latents(s, flags);
-  if (sparse && do_reduce && !update)
-    hipLaunchKernelGGL((seg_zero_rows_kernel<GT>), dim3(static_cast<unsigned>(ceil_div(s->F, kZeroRows * kWavesPerBlock))), dim3(kBlock), 0, st, sc.lists.ctrl,
-                       sc.lists.empty_list, dW, D, rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t)));
+  // (by the last blocks of the first walk, where that is hier_train_kernel)
+  ZeroRows zero = {};
+  if (sparse && do_reduce && !update) {
+    const unsigned n_zero_blocks = static_cast<unsigned>(ceil_div(s->F, kZeroRows * kWavesPerBlock));
+    const int dwords = rows_on_dwords(dW, D, sizeof(typename Traits<GT>::store_t));
+    if (train && do_sweep && !hot)
+      zero = {sc.lists.ctrl, sc.lists.empty_list, dW, sizeof(typename Traits<GT>::store_t) == 4, dwords, n_zero_blocks};
+    else
+      hipLaunchKernelGGL((seg_zero_rows_kernel<GT>), dim3(n_zero_blocks), dim3(kBlock), 0, st, sc.lists.ctrl,
+                         sc.lists.empty_list, dW, D, dwords);
+  }
   // In the training step the second step of a slice's hot latents travels with the next slice's
   // training-step launch (a gradient of CarriedGrad's type; by pieces, the weight's: that is what that kernel
   // writes; a launch of its own costs 4.7 us a slice); the last slice's gets one.
@@ -1075,8 +1081,9 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
     } else if (train && do_sweep) {
       launch_train_kernel_k<WT, PT>(s, *train, indices, weight, vals, coef, slot, P, dv_part, s_final, d_pad,
                                     reinterpret_cast<float *>(ws + pl.off_loss), status_flag, cols,
-                                    static_cast<int>(col0), sw, st, pending, dW_solo);
+                                    static_cast<int>(col0), sw, st, pending, dW_solo, zero);
       pending = HotFinalize{};
+      zero = ZeroRows{};
     } else if (do_sweep) {
 #define FLEXSAE_SWEEP(SV)                                                                                      \
   hipLaunchKernelGGL((hier_sweep_kernel<WT, PT, SV, FLEXSAE_SWEEP_U>),                                         \
@@ -1148,7 +1155,8 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                      train ? train->loss : static_cast<float *>(nullptr), pending, pending_hot, n_hot_blocks,
                      s_final, s->B, static_cast<int64_t>(d_pad), D, colsum_part,
                      hot ? static_cast<int>(pl.n_row_blocks) : two_launches ? -1 : 0, dbias, n_col_blocks, dv_part,
-                     static_cast<int>(d_used / (train ? train_tile_cols(s) : kWave * sweep_vec)), s->B * s->K, dvals);
+                     static_cast<int>(d_used / (train ? train_tile_cols(s) : kWave * sweep_vec)), s->B * s->K, dvals,
+                     train ? train->stats : PairStats{});
   if (two_launches)
     hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(D, 256))), dim3(256), 0, st, colsum_part,
                        n_chunks, D, static_cast<const float *>(nullptr), 1.0f, dbias);
@@ -1207,20 +1215,17 @@ void build_hot_tables(const flexsae_shape *s, const HierBwdPlan &pl, uint8_t *ws
   uint32_t *ctrl = reinterpret_cast<uint32_t *>(ws + pl.off_hot_ctrl);
   uint32_t *hot_list = reinterpret_cast<uint32_t *>(ws + pl.off_hot_list);
   uint32_t *cand_list = reinterpret_cast<uint32_t *>(ws + pl.off_cand_list);
-  uint32_t *cand_state = reinterpret_cast<uint32_t *>(ws + pl.off_cand_state);
-  uint32_t *long_cand = reinterpret_cast<uint32_t *>(ws + pl.off_long_cand);
   uint32_t *long2 = reinterpret_cast<uint32_t *>(ws + pl.off_long2);
   if (!have_hslot) {
     const int64_t n_pairs = s->B * s->K;
     hipLaunchKernelGGL(copy_u32_kernel, dim3(grid_for(n_pairs, 256, 8192)), dim3(256), 0, st, hslot,
                        reinterpret_cast<const uint32_t *>(ws + pl.off_slot), n_pairs);
   }
+  uint32_t *chunk2 = reinterpret_cast<uint32_t *>(ws + pl.off_chunk2);
   hipLaunchKernelGGL(hot_select_kernel, dim3(1), dim3(1024), 0, st, begin, sc.lists.ctrl, sc.lists.long_list, ctrl,
-                     cand_list, long_cand, static_cast<uint32_t>(kHotMax));
-  hipLaunchKernelGGL(hot_mark_kernel, dim3(kHotMax), dim3(1024), 0, st, begin, map, ctrl, cand_list, cand_state,
-                     hot_list, hslot, static_cast<uint32_t>(s->K));
-  hipLaunchKernelGGL(hot_cold_long_kernel, dim3(64), dim3(256), 0, st, begin, sc.lists.ctrl, sc.lists.long_list,
-                     long_cand, cand_state, ctrl, long2, reinterpret_cast<uint32_t *>(ws + pl.off_chunk2));
+                     cand_list, long2, chunk2, static_cast<uint32_t>(kHotMax));
+  hipLaunchKernelGGL(hot_mark_kernel, dim3(kHotMax), dim3(1024), 0, st, begin, map, ctrl, cand_list, hot_list, hslot,
+                     static_cast<uint32_t>(s->K), long2, chunk2);
 }
 
 // ---- TopK backward: workspace plan and slice loop ---------------------------------------
@@ -1674,7 +1679,8 @@ int flexsae_hier_pair_stats(const flexsae_shape *s, const void *workspace, uint3
   const HierBwdPlan pl = plan_hier_bwd(s);  // the part of the layout every hierarchical workspace shares
   uint8_t *ws = static_cast<uint8_t *>(const_cast<void *>(workspace));
   const CsrScratch sc = carve_hier_lists(s, pl, ws);
-  hipLaunchKernelGGL(pair_stats_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), sc.lists.ctrl, stats);
+  hipLaunchKernelGGL(pair_stats_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
+                     PairStats{sc.lists.ctrl, stats, 0u, 0});
   return launch_status();
 }
 
@@ -1806,7 +1812,8 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
                       const void *vals, const void *bias, const void *target, float *loss,
                       void *dW, int dW_dtype, float *dvals, float *dbias, void *workspace,
                       size_t workspace_bytes, int flags, int *status_flag, void *stream,
-                      const float *sgd_step, const float *dw_scale = nullptr) {
+                      const float *sgd_step, const float *dw_scale = nullptr, uint32_t *stats = nullptr,
+                      uint32_t stats_tag = 0) {
   int rc = check_shape(s);
   if (rc != FLEXSAE_OK) return rc;
   if (sgd_step || dw_scale) {
@@ -1861,7 +1868,7 @@ int hier_fwd_bwd_impl(const flexsae_shape *s, const int64_t *indices, const void
   const double count = static_cast<double>(s->B) * static_cast<double>(s->K) * static_cast<double>(s->D);
   const float coef = static_cast<float>(2.0 / count);
   const TrainArgs ta = {bias, target, loss, s->B * (hier_cols_used(s, pl, true, piece) / train_tile_cols(s)),
-                        1.0 / count};
+                        1.0 / count, PairStats{sc.lists.ctrl, stats, stats_tag, 1}};
   // without dW the reductions are left out like in the deferred case (dW_dtype only selects a template then)
   const auto slices = pl.vec == 4 ? launch_hier_slices_w<4> : pl.vec == 2 ? launch_hier_slices_w<2> : launch_hier_slices_w<1>;
   slices(s, pl, slice_w, indices, weight, vals, nullptr, sgd_step ? sgd_step : dw_scale, coef, dW,
@@ -1907,6 +1914,20 @@ int flexsae_hier_sgd_step(const flexsae_shape *s, const int64_t *indices, void *
                                     FLEXSAE_BWD_HOT_NO_HEADROOM | FLEXSAE_BWD_DENSE_LATENTS | FLEXSAE_BWD_HOT_BLOCKS_64 |
                                     FLEXSAE_BWD_HOT_BLOCKS_32),
                            status_flag, stream, step);
+}
+
+int flexsae_hier_step(const flexsae_shape *s, const int64_t *indices, void *weight, const void *vals, const void *bias,
+                      const void *target, const float *grad_out, const float *step, float *loss, void *dW, int dW_dtype,
+                      float *dvals, float *dbias, void *workspace, size_t workspace_bytes, int flags, uint32_t *stats,
+                      uint32_t stats_tag, int *status_flag, void *stream) {
+  if (!s || (step && (grad_out || dW)) ||
+      (flags & (FLEXSAE_BWD_SWEEP_ONLY | FLEXSAE_BWD_REDUCE_ONLY | FLEXSAE_BWD_SKIP_EPILOGUE)))
+    return FLEXSAE_ERR_INVALID_ARGUMENT;
+  if (!aligned(stats, 4)) return FLEXSAE_ERR_ALIGNMENT;
+  return hier_fwd_bwd_impl(s, indices, weight, vals, bias, target, loss, step ? weight : dW, step ? s->weight_dtype : dW_dtype,
+                           dvals, dbias, workspace, workspace_bytes,
+                           flags & ~(kBwdSgdUpdate | kBwdHot | kBwdSolo | kBwdScaled | (step ? FLEXSAE_BWD_RAGGED_ROWS : 0)),
+                           status_flag, stream, step, grad_out, stats, stats_tag);
 }
 
 int flexsae_scale(void *dst, const void *src, int dtype, int64_t n, const float *scale, void *stream) {

@@ -48,7 +48,8 @@ __device__ __forceinline__ void colsum_whole_block(const float *__restrict__ x, 
 }
 
 // What follows the slices of a hierarchical step, in one launch of 1024-thread blocks.  The parts are independent:
-//   block 0                   the loss from the per-(tile, row) partials (loss_finalize_kernel), when loss_partial is given;
+//   block 0                   the loss from the per-(tile, row) partials (loss_finalize_kernel), when loss_partial is given, and
+//                             what the pair list says about the indices, where that is wanted;
 //   the next fin.n_blocks     the second step of the last slice's frequent latents (hot_finalize_run);
 //   the next n_hot_blocks     the last slice's accumulator rows (hot_block_finalize_run);
 //   the next n_col_blocks     dbias: column sums of s_final, kEndCols columns per block (n_parts = 0), or of more than kEndRows
@@ -65,10 +66,12 @@ __global__ __launch_bounds__(1024) void hier_epilogue_kernel(
     const float *__restrict__ loss_partial, int64_t n_loss_partials, double inv_count, float *__restrict__ loss,
     HotFinalize fin, HotBlockFinalize hfin, unsigned n_hot_blocks, const float *__restrict__ s_final, int64_t rows,
     int64_t ld, int cols, float *__restrict__ colsum_part, int n_parts, float *__restrict__ dbias,
-    unsigned n_col_blocks, const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs, float *__restrict__ dvals) {
+    unsigned n_col_blocks, const float *__restrict__ dv_part, int n_tiles, int64_t n_pairs, float *__restrict__ dvals,
+    PairStats stats) {
   __shared__ double red[1024];
   unsigned blk = blockIdx.x;
   if (blk == 0) {
+    if (stats.out && threadIdx.x == 0) write_pair_stats(stats);
     if (loss_partial) loss_finalize_block(loss_partial, n_loss_partials, inv_count, loss, red);
     return;
   }

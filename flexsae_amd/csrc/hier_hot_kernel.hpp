@@ -62,18 +62,30 @@ __device__ __forceinline__ float wave_max_bcast(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// long2_list = the latents with more than kSegChunk pairs that do not become hot (any order), with their chunk table: what
+// the chunked part of the segment reduction still serves.
+__device__ __forceinline__ void append_cold_long(uint32_t f, uint32_t pairs, uint32_t *__restrict__ ctrl,
+                                                 uint32_t *__restrict__ long2_list, uint32_t *__restrict__ chunk2_begin) {
+  const uint32_t chunks = (pairs + kSegChunk - 1) / kSegChunk;
+  const unsigned long long at = atomicAdd(reinterpret_cast<unsigned long long *>(ctrl + kHotLong2), (1ull << 32) | chunks);
+  long2_list[at >> 32] = f;
+  chunk2_begin[at >> 32] = static_cast<uint32_t>(at);
+  atomicAdd(&ctrl[kHotLong2Count], 1u);  // a statistic
+}
+
 // ---- which latents are hot -----------------------------------------------------------------
 // Candidates: the latents with the most pairs, at most kHotMax of them, taken from the list of
 // latents with more than kSegChunk pairs: all with a pair count above T, T the (kHotMax+1)-th
 // largest count (found by a radix select over four 8-bit digits), so the choice does not depend on
-// the order of that list.  Single block.  cand_list[c] = latent, long_cand[i] = candidate number of
-// long_list[i] or kHotNone; clears the counters that the kernels after it advance.
+// the order of that list.  Single block.  cand_list[c] = latent; clears the counters that it and the kernel after it
+// advance, and hands the long latents that are no candidates on (append_cold_long).
 __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__restrict__ begin,
                                                           const uint32_t *__restrict__ long_ctrl,
                                                           const uint32_t *__restrict__ long_list,
                                                           uint32_t *__restrict__ ctrl,
                                                           uint32_t *__restrict__ cand_list,
-                                                          uint32_t *__restrict__ long_cand, uint32_t max_hot) {
+                                                          uint32_t *__restrict__ long2_list,
+                                                          uint32_t *__restrict__ chunk2_begin, uint32_t max_hot) {
   constexpr uint32_t kCached = 8192;  // pair counts kept in the LDS (each costs two dependent loads from memory)
   __shared__ uint32_t hist[256];
   __shared__ uint32_t cnt_lds[kCached];
@@ -152,12 +164,11 @@ __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__rest
   __syncthreads();
   for (uint32_t i = tid; i < n_long; i += 1024) {
     const uint32_t c = count_of(i);
-    uint32_t cand = kHotNone;
     if (max_hot > 0 && c > T) {
-      cand = atomicAdd(&n_cand_s, 1u);  // at most max_hot by the choice of T
-      cand_list[cand] = long_list[i];
+      cand_list[atomicAdd(&n_cand_s, 1u)] = long_list[i];  // at most max_hot by the choice of T
+    } else {
+      append_cold_long(long_list[i], c, ctrl, long2_list, chunk2_begin);
     }
-    long_cand[i] = cand;
   }
   __syncthreads();
   if (tid == 0) ctrl[kHotNCand] = n_cand_s;
@@ -165,15 +176,16 @@ __global__ __launch_bounds__(1024) void hot_select_kernel(const uint32_t *__rest
 
 // One block per candidate: a candidate none of whose rows holds it twice becomes a hot latent (an
 // accumulator then takes at most one addition per row, which the bound on its sums counts on); it
-// gets an accumulator row h and its pairs are marked in hslot[].  cand_state[c] = h or kHotNone.
+// gets an accumulator row h and its pairs are marked in hslot[]; the others join the cold long latents.
 // hslot must hold a copy of slot[] on entry.
 __global__ __launch_bounds__(1024) void hot_mark_kernel(const uint32_t *__restrict__ begin,
                                                        const uint32_t *__restrict__ map,
                                                        uint32_t *__restrict__ ctrl,
                                                        const uint32_t *__restrict__ cand_list,
-                                                       uint32_t *__restrict__ cand_state,
                                                        uint32_t *__restrict__ hot_list,
-                                                       uint32_t *__restrict__ hslot, uint32_t K) {
+                                                       uint32_t *__restrict__ hslot, uint32_t K,
+                                                       uint32_t *__restrict__ long2_list,
+                                                       uint32_t *__restrict__ chunk2_begin) {
   __shared__ uint32_t h_s;
   const uint32_t c = blockIdx.x;
   if (c >= ctrl[kHotNCand]) return;  // uniform per block
@@ -186,7 +198,7 @@ __global__ __launch_bounds__(1024) void hot_mark_kernel(const uint32_t *__restri
   if (threadIdx.x == 0) {
     const uint32_t h = dup ? kHotNone : atomicAdd(&ctrl[kHotNHot], 1u);
     if (!dup) hot_list[h] = f;
-    cand_state[c] = h;
+    else append_cold_long(f, s1 - s0, ctrl, long2_list, chunk2_begin);
     h_s = h;
   }
   __syncthreads();
@@ -195,38 +207,25 @@ __global__ __launch_bounds__(1024) void hot_mark_kernel(const uint32_t *__restri
   for (uint32_t i = s0 + threadIdx.x; i < s1; i += blockDim.x) hslot[map[i]] = kHotSlotBit | h;
 }
 
-// long2_list = the latents with more than kSegChunk pairs that did not become hot (any order), with
-// their chunk table: what the chunked part of the segment reduction still serves.
-__global__ void hot_cold_long_kernel(const uint32_t *__restrict__ begin, const uint32_t *__restrict__ long_ctrl,
-                                     const uint32_t *__restrict__ long_list,
-                                     const uint32_t *__restrict__ long_cand,
-                                     const uint32_t *__restrict__ cand_state, uint32_t *__restrict__ ctrl,
-                                     uint32_t *__restrict__ long2_list, uint32_t *__restrict__ chunk2_begin) {
-  const uint32_t n_long = long_ctrl[kLongCount];
-  const uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_long; i += stride) {
-    const uint32_t c = long_cand[i];
-    const bool hot = c != kHotNone && cand_state[c] != kHotNone;
-    if (hot) continue;
-    const uint32_t f = long_list[i];
-    const uint32_t chunks = (begin[f + 1] - begin[f] + kSegChunk - 1) / kSegChunk;
-    const unsigned long long at =
-        atomicAdd(reinterpret_cast<unsigned long long *>(ctrl + kHotLong2), (1ull << 32) | chunks);
-    long2_list[at >> 32] = f;
-    chunk2_begin[at >> 32] = static_cast<uint32_t>(at);
-    atomicAdd(&ctrl[kHotLong2Count], 1u);  // a statistic
-  }
-}
-
 // What a pair list's control words say about the indices: out[0] = latents with more than kSegChunk
 // pairs, out[1] = their pairs in chunks of kSegChunk, out[2] = latents without a pair.  `out` may be
-// pinned host memory.
-__global__ void pair_stats_kernel(const uint32_t *__restrict__ ctrl, uint32_t *__restrict__ out) {
-  if (threadIdx.x == 0) {
-    out[0] = ctrl[kLongCount];
-    out[1] = ctrl[kLongChunks];
-    out[2] = ctrl[kEmptyCount];
-  }
+// pinned host memory.  tagged: out[3] = tag once the others can be read.
+struct PairStats {
+  const uint32_t *ctrl;
+  uint32_t *out;  // null: not wanted
+  uint32_t tag;
+  int tagged;
+};
+
+__device__ __forceinline__ void write_pair_stats(const PairStats &p) {
+  p.out[0] = p.ctrl[kLongCount];
+  p.out[1] = p.ctrl[kLongChunks];
+  p.out[2] = p.ctrl[kEmptyCount];
+  if (p.tagged) __hip_atomic_store(p.out + 3, p.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void pair_stats_kernel(PairStats p) {
+  if (threadIdx.x == 0) write_pair_stats(p);
 }
 
 // ---- second step of the hot latents ---------------------------------------------------------

@@ -68,6 +68,7 @@ struct RowPiece<f16_t, 2> {
 // back with plain LDS loads.  bias - target is fetched before the gathers are issued: the memory
 // counter retires in order, so anything issued after them can only be waited for together with
 // all of them, and the forward walk could not start while rows are still arriving.
+// zero: rows of dW to clear, by the last blocks; a launch of its own costs 4-5 us on the device and as much on the host.
 // row_tiles: 0: the items are all rows of one tile after the other; else so many tiles of one row after the other.
 // fin: the second step of the previous slice's hot latents (see HotFinalize), run by the leading blocks
 // of the launch into a gradient of CarriedGrad's type, or into the weights.
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
     const uint32_t *__restrict__ slot, void *__restrict__ P, float *__restrict__ dv_part,
     float *__restrict__ s_final, int s_final_ld, float *__restrict__ loss_partial,
     int *status_flag, int64_t n_items, int64_t B, int row_tiles, int col0, int slice_w, int K, int64_t F, int D, uint32_t slot_mask,
-    void *__restrict__ dW, HotFinalize fin) {
+    void *__restrict__ dW, HotFinalize fin, ZeroRows zero) {
   using Piece = RowPiece<WT, VEC>;
   using raw_t = typename Piece::raw_t;
   using S_t = typename Traits<WT>::store_t;
@@ -105,6 +106,12 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
   // the leading blocks finish the hot latents of the previous slice (fin.n_blocks of them; none at the first slice)
   if (blockIdx.x < fin.n_blocks) {
     hot_finalize_carried<WT>(fin, blockIdx.x);
+    return;
+  }
+  // the last ones clear the rows of latents without pairs (the first slice's launch, where they are listed)
+  const unsigned n_walk = gridDim.x - zero.n_blocks;
+  if (blockIdx.x >= n_walk) {
+    zero_rows_carried(zero, D, blockIdx.x - n_walk);
     return;
   }
   const int64_t item = static_cast<int64_t>(blockIdx.x - fin.n_blocks) * (blockDim.x >> 6) + wave_in_block();

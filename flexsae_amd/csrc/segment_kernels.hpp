@@ -585,13 +585,12 @@ __global__ __launch_bounds__(256) void hot_finalize_kernel(HotFinalize h) {
 // columns: 295 and 257 with and without.
 constexpr int kZeroRows = 8;
 template <typename GT>
-__global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__restrict__ ctrl,
-                                                            const uint32_t *__restrict__ empty_list,
-                                                            void *__restrict__ out, int D, int dwords) {
+__device__ __forceinline__ void zero_rows_block(const uint32_t *__restrict__ ctrl, const uint32_t *__restrict__ empty_list,
+                                                void *__restrict__ out, int D, int dwords, unsigned block) {
   constexpr int EV = 16 / static_cast<int>(sizeof(typename Traits<GT>::store_t));
   const uint32_t n = ctrl[kListed] ? ctrl[kEmptyCount] : 0u;
   const int lane = lane_id();
-  const int64_t w0 = (static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block()) * kZeroRows;
+  const int64_t w0 = (static_cast<int64_t>(block) * (blockDim.x >> 6) + wave_in_block()) * kZeroRows;
   if (w0 >= n) return;  // uniform per wavefront
   const int rows = static_cast<int>((n - w0) < kZeroRows ? (n - w0) : kZeroRows);
   const int mine = lane < rows ? static_cast<int>(empty_list[w0 + lane]) : 0;
@@ -602,6 +601,28 @@ __global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__re
     const int64_t row = static_cast<int64_t>(static_cast<uint32_t>(bcast_i32(mine, r))) * D;
     for (int d = lane * EV; d < D; d += kWave * EV) store_vec_upto<GT, EV>(out, row + d, zero, D - d, dwords);
   }
+}
+
+template <typename GT>
+__global__ __launch_bounds__(256) void seg_zero_rows_kernel(const uint32_t *__restrict__ ctrl,
+                                                            const uint32_t *__restrict__ empty_list,
+                                                            void *__restrict__ out, int D, int dwords) {
+  zero_rows_block<GT>(ctrl, empty_list, out, D, dwords, blockIdx.x);
+}
+
+// The same for blocks of another launch (n_blocks of them; 0: none): zero is zero in every type, so rows of 16-bit elements
+// are bf16 here.
+struct ZeroRows {
+  const uint32_t *ctrl, *empty_list;
+  void *out;
+  int wide;  // 32-bit elements
+  int dwords;
+  unsigned n_blocks;
+};
+
+__device__ __forceinline__ void zero_rows_carried(const ZeroRows &z, int D, unsigned block) {
+  if (z.wide) zero_rows_block<float>(z.ctrl, z.empty_list, z.out, D, z.dwords, block);
+  else zero_rows_block<bf16_t>(z.ctrl, z.empty_list, z.out, D, z.dwords, block);
 }
 
 }  // namespace flexsae

@@ -285,7 +285,7 @@ def set_hier_scratch_bytes(nbytes) -> None:
 # where they are not (its blocks hold the LDS of a whole compute unit: half the wavefronts of the
 # plain kernel), and only the device knows which it is.  "auto" therefore measures: every sliced step
 # leaves, in pinned host memory, how many of its pairs belong to latents with more than 64 pairs
-# (flexsae_hier_pair_stats; no synchronisation: an event is polled), and the next step of the same
+# (no synchronisation: a tag beside them or an event is polled), and the next step of the same
 # shape on the same device takes the accumulators when that was a quarter of the pairs or more.  The
 # first step of a shape, and steps traced by a compiler, run the plain kernel.
 # "on" takes them wherever the shape is supported (16-bit weights, K <= 64); "off" never.
@@ -375,18 +375,21 @@ def _index_stats(key, B, K, F):
     st = _hot_auto.get(key)
     if st is None:
         return None
-    if st["event"] is not None and st["event"].query():  # the previous step's measurement has arrived
-        long_pairs = int(st["pinned"][1]) * 64
-        st["hot"] = long_pairs >= _HOT_AUTO_FRACTION * B * K
-        st["dense"] = int(st["pinned"][2]) < _DENSE_AUTO_FRACTION * F
+    words = st["words"]
+    # the previous step's measurement has arrived: its event, or its tag in the last word
+    if (st["event"] is not None and st["event"].query()) or words[3] != st["seen"]:
+        st["seen"] = words[3]
+        st["hot"] = words[1] * 64 >= _HOT_AUTO_FRACTION * B * K
+        st["dense"] = words[2] < _DENSE_AUTO_FRACTION * F
         st["event"] = None
     return st
 
 
 def _new_stats(key):
-    pinned = torch.zeros(3, dtype=torch.int32, pin_memory=True)
-    st = _hot_auto[key] = {"hot": False, "dense": False, "pinned": pinned, "pinned_at": pinned.data_ptr(), "event": None,
-                           "spare": torch.cuda.Event()}
+    # four words: what flexsae_hier_pair_stats writes, and the tag of the step that wrote it (flexsae_hier_step)
+    pinned = torch.zeros(4, dtype=torch.int32, pin_memory=True)
+    st = _hot_auto[key] = {"hot": False, "dense": False, "pinned": pinned, "event": None, "spare": torch.cuda.Event(),
+                           "words": (ctypes.c_uint32 * 4).from_address(pinned.data_ptr()), "seen": 0, "asked": 0}
     return st
 
 
@@ -398,7 +401,7 @@ def _hot_measure(lib, shape, workspace: Tensor, B, K, F, D, weight_dtype) -> Non
         return
     key = _hot_key(workspace.device, B, K, F, D, weight_dtype)
     st = _hot_auto.get(key) or _new_stats(key)
-    if st["event"] is not None:
+    if st["event"] is not None or st["seen"] != st["asked"]:
         return  # a measurement is still on its way
     rc = lib.flexsae_hier_pair_stats(ctypes.byref(shape), _ptr(workspace), _ptr(st["pinned"]), _stream())
     _lib.check(rc, "flexsae_hier_pair_stats")
@@ -1005,11 +1008,8 @@ def hierarchical_sae_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bia
             F, D = weight.shape
             if B * K * F * D:
                 route = _route(B, K, F, D, weight, True)
-                cols, flags, ws_flags, pinned = route.decide(B, K, F)
-                out = native.hier_sgd(indices, weight, vals, bias, target, step, cols, flags, ws_flags, pinned)
+                out = native.hier_sgd(indices, weight, vals, bias, target, step, *route.decide(B, K, F))
                 if out is not None:
-                    if pinned:
-                        route.measured()
                     return out
         if _plain_call(indices, weight, vals, bias, target, step):
             torch.autograd.graph.increment_version(weight)  # what the op's schema says of its weight
@@ -1189,8 +1189,7 @@ topk_fwd.register_autograd(_topk_backward, setup_context=_setup_context)
 # ---- ordinary eager calls ------------------------------------------------------------------
 # A call on plain tensors with no tracer, mode or transform around it does without the dispatcher and, but for what is decided
 # here, without Python: csrc/eager.cpp checks, allocates, launches and has the autograd nodes, which save the tensors that the
-# ops save.  Calls that share a pair list or check their indices, and the late fp16 step, run the ops' functions under an
-# autograd.Function.  Everything else goes through the ops, which tracers, modes and transforms see.
+# ops save.  Calls that share a pair list or check their indices run the ops' functions under an autograd.Function.  Everything else goes through the ops, which tracers, modes and transforms see.
 # us a step with the functions under an autograd.Function and with eager.cpp: B = 64, K = 32, F = 4096, D = 256 fp32 TopK 160
 # and 79, hierarchical 195 and 99 (through the ops 40 to 45 more; the least that torch's engine takes for a forward and a
 # backward of any kind is 45); the host's share of an SGD step 62 and 35.
@@ -1320,7 +1319,7 @@ def _late_step(weight: Tensor, B: int, K: int) -> bool:
 
 
 class _HierLateStep(torch.autograd.Function):
-    """The loss in the forward, ``_hier_sliced_step`` with the upstream gradient in the backward (``_late_step``)."""
+    """On plain tensors the loss in the forward, ``_hier_sliced_step`` with the upstream gradient in the backward (``_late_step``)."""
 
     @staticmethod
     def forward(ctx, indices, weight, vals, bias, target, hot, dense):
@@ -1366,6 +1365,9 @@ def _general_backward(kind, grad, saved, needs, numbers, dw_unit):
     if kind == 1:
         ctx.leaf_dtypes = (saved[2].dtype, _TYPES[numbers[0]], None)
         return _hier_backward(ctx, grad, None, _hier_bwd_impl if plain else None), None
+    if kind == 3:
+        ctx.hot, ctx.dense = bool(numbers[1] & _lib.BWD_HOT_LATENTS), bool(numbers[1] & _lib.BWD_DENSE_LATENTS)
+        return tuple(_HierLateStep.backward(ctx, grad)[:5]), None
     ctx.leaf_dtypes = (saved[2].dtype, saved[3].dtype)
     ctx.need_dw, ctx.dw_in_place, ctx.dw_unit = bool(numbers[0]), True, dw_unit
     ctx.hot, ctx.dense = bool(numbers[1] & _lib.BWD_HOT_LATENTS), bool(numbers[1] & _lib.BWD_DENSE_LATENTS)
@@ -1400,8 +1402,8 @@ _ROUTES_MOST = 1024
 
 
 class _Route:
-    """How a hierarchical call with gradients runs: ``train`` the step of hier_train_sliced, else forward and sweep; ``here`` by
-    the functions of this module (the late step, the staged one, the atomic backward); the slices' width plain and with hot
+    """How a hierarchical call with gradients runs: ``train`` the step of hier_train_sliced, ``late`` in the backward, else forward
+    and sweep; ``here`` by the functions of this module (the staged step, the atomic backward); the slices' width plain and with hot
     latents; what is measured for the next step of the shape."""
 
     def __init__(self, B, K, F, D, weight, device):
@@ -1409,13 +1411,13 @@ class _Route:
         takes = _fused_training and (_train_supported(weight, K) or (_train_ragged(weight, K) and _ragged_pays(weight, B, K)))
         stage = takes and _train_supported(weight, K) and hier_stage_bytes(device) > 0
         self.train = takes and _hier_scratch_bytes != 0 and (_step_pays(weight, K) or _one_gather_pays(weight, B, K))
-        late = self.train and need_dw and _late_step(weight, B, K)
         # by the functions of this module
-        self.here = stage or late or _hier_scratch_budget(B, K, F, D, dtype) <= 0
+        self.here = stage or _hier_scratch_budget(B, K, F, D, dtype) <= 0
         self._step(B, K, F, D, dtype, device, need_dw, _lib.BWD_RAGGED_ROWS if _train_ragged(weight, K) else 0)
+        self.late = self.train and need_dw and _late_step(weight, B, K)
 
     def _step(self, B, K, F, D, dtype, device, need_dw, ragged):
-        self.device = device
+        self.late = False
         self.key = _hot_key(device, B, K, F, D, dtype)
         self.ragged = ragged
         self.cols = _hier_slice_cols(B, K, F, D, dtype)
@@ -1431,30 +1433,22 @@ class _Route:
             self.hot_cols = _hot_slice_cols(B, self.cols, device)
 
     def decide(self, B, K, F):
-        """(slice width, flags of the call, flags of the workspace query, pinned memory for the measurement or 0)"""
+        """(slice width, flags of the call, flags of the workspace query, pinned memory for a measurement or None, its tag)"""
         hot, dense = self.hot == "on", self.dense == "on"
-        pinned = 0
-        if self.asks or self.measures:
-            if not torch.cuda.is_current_stream_capturing():
-                st = _index_stats(self.key, B, K, F)
-                if st is not None:
-                    hot = hot or (self.hot == "auto" and st["hot"])
-                    dense = dense or (self.dense == "auto" and st["dense"])
-                if self.measures and (st is None or st["event"] is None):
-                    if st is None:
-                        st = _new_stats(self.key)
-                    pinned = st["pinned_at"]
+        pinned, tag = None, 0
+        if (self.asks or self.measures) and not torch.cuda.is_current_stream_capturing():
+            st = _index_stats(self.key, B, K, F)
+            if st is not None:
+                hot = hot or (self.hot == "auto" and st["hot"])
+                dense = dense or (self.dense == "auto" and st["dense"])
+            # (a late step that is never asked for its gradients measures nothing: the next one does not wait for it)
+            if self.measures and (st is None or (st["event"] is None and (self.late or st["seen"] == st["asked"]))):
+                st = st or _new_stats(self.key)
+                tag = st["asked"] = st["asked"] % 0xffffffff + 1
+                pinned = st["pinned"]
         hot_flags = self.hot_flags if hot else 0
         return (self.hot_cols if hot else self.cols, hot_flags | self.ragged | (_lib.BWD_DENSE_LATENTS if dense else 0),
-                hot_flags | self.ragged, pinned)
-
-    def measured(self):
-        """The measurement that `decide` asked for is on its way."""
-        st = _hot_auto.get(self.key)
-        if st is not None:
-            with _on_device(self.device):
-                st["spare"].record()
-            st["event"] = st["spare"]
+                hot_flags | self.ragged, pinned, tag)
 
 
 def _route(B, K, F, D, weight, sgd=False):
@@ -1490,11 +1484,8 @@ def _native_hier(native, indices, weight, vals, bias, target):
         return None
     if not route.train:
         return native.hier_loss(indices, weight, vals, bias, target, route.cols)
-    cols, flags, ws_flags, pinned = route.decide(B, K, F)
-    loss = native.hier_sliced(indices, weight, vals, bias, target, weight.requires_grad, cols, flags, ws_flags, pinned)
-    if pinned and loss is not None:
-        route.measured()
-    return loss
+    step = native.hier_late if route.late else native.hier_sliced
+    return step(indices, weight, vals, bias, target, weight.requires_grad, *route.decide(B, K, F))
 
 
 def triton_hierarchical_sae_loss(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor,

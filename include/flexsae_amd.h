@@ -336,6 +336,17 @@ int flexsae_hier_sgd_step(const flexsae_shape *shape, const int64_t *indices, vo
                           int flags, int *status_flag, void *stream);
 
 /*
+ * The three entry points above in one, with what flexsae_hier_pair_stats tells: without `grad_out` and `step`
+ * flexsae_hier_fwd_bwd, with `grad_out` flexsae_hier_fwd_bwd_scaled, with `step` flexsae_hier_sgd_step (dW NULL then); not for
+ * SWEEP_ONLY, REDUCE_ONLY and SKIP_EPILOGUE.  stats (NULL: not wanted) may be pinned host memory of four words: the last
+ * launch writes the three numbers and then `stats_tag` into the fourth, so that the host need not wait for anything.
+ */
+int flexsae_hier_step(const flexsae_shape *shape, const int64_t *indices, void *weight, const void *vals, const void *bias,
+                      const void *target, const float *grad_out, const float *step, float *loss, void *dW, int dW_dtype,
+                      float *dvals, float *dbias, void *workspace, size_t workspace_bytes, int flags, uint32_t *stats,
+                      uint32_t stats_tag, int *status_flag, void *stream);
+
+/*
  * dst[n] = src[n] * scale[0]  (same dtype in and out; `scale` is a device fp32 scalar).  dst may
  * be src (in place); then a scale of exactly 1 costs one empty launch.
  * replaces: the dW.mul_(grad) pass of HierarchicalSAELossFunction.backward

@@ -209,7 +209,7 @@ def test_what_the_extension_module_takes(entry):
     idx, W, v, b, t = args
     LOSS["topk"](*args)
     fn = getattr(ops._native(W), entry)
-    more = {"topk_loss": (), "hier_loss": (128,), "hier_sliced": (True, 128, 0, 0, 0)}[entry]
+    more = {"topk_loss": (), "hier_loss": (128,), "hier_sliced": (True, 128, 0, 0, None, 0)}[entry]
     want = fn(*args, *more)
     assert torch.equal(want, LOSS["topk" if entry == "topk_loss" else "hier"](*args))
     strided = [x.repeat_interleave(2, -1)[..., ::2] for x in args]
