@@ -1310,12 +1310,15 @@ def _late_step(weight: Tensor, B: int, K: int) -> bool:
     gradient is known and dW is written once in fp16, instead of an fp32 unit gradient written, read back, scaled and
     rounded.  A second gather (2*B*K*D bytes, partly out of the L2s) for 6*F*D bytes less: us with it / without, uniform
     and Zipf indices, B = 4096, F = 65536, D = 2304: K = 16 469 / 538, 409 / 566; K = 32 723 / 765, 595 / 697; K = 64
-    1252 / 1284, 1059 / 1081; K = 128 2369 / 2279; B = 8192, K = 64, F = 262144, D = 4096 4878 / 5786, 3526 / 4518; B = 256,
-    K = 64, F = 65536, D = 2048 171 / 332.  Not below 96 * 2^20 weights, where more launches and their host work show (F = 65536,
-    K = 32, B = 410 and 2048: D = 1544 282 / 338 and 362 / 414, D = 1024 258 / 221 and 266 / 262, D = 900 256 / 219 and
-    269 / 257, D = 512 249 / 219 and 252 / 215)."""
+    1252 / 1284, 1059 / 1081; K = 128 2369 / 2279; B = 8192, K = 64, F = 262144, D = 4096 4878 / 5786, 3526 / 4518; B = 207,
+    K = 256, F = 131072, D = 448 123 / 153, 131 / 174; B = 2048, K = 32, F = 65536, D = 512 119 / 132, 145 / 182; B = 410, D = 1024
+    84 / 155, 105 / 187; B = 300, K = 90, F = 9000, D = 2348 166 / 176, 173 / 183; B = 1500, K = 20, F = 30000, D = 1002
+    120 / 120, 117 / 117.  Not below 24 * 2^20 weights, where two launches more show, on the host too (B = 64, K = 64, F = 65536,
+    D = 256 109 / 102, B = 500, K = 64, F = 32768, D = 512 109 / 103), nor, below 96 * 2^20, for odd rows, which the step does
+    not take."""
     F, D = weight.shape
-    return weight.dtype == torch.float16 and B * K <= 4 * F and F * D >= 96 << 20
+    return (weight.dtype == torch.float16 and B * K <= 4 * F and F * D >= 24 << 20
+            and (D % 2 == 0 or F * D >= 96 << 20))
 
 
 class _HierLateStep(torch.autograd.Function):
