@@ -627,8 +627,9 @@ __device__ __forceinline__ void count_in_lds(uint32_t *counter, uint32_t at, boo
 // order: 75 (96), latents by frequency: 298 (3336), half of the pairs on the first 32 latents: 144 (317); 64 latents in
 // every one of 16384 rows: 1329 (2584).
 // WAVES: wavefronts per SIMD that its registers leave room for: eight, two blocks per compute unit, spill 13 (with records 30)
-// registers; four do not, where there is no second block (with records, us: 26.9 -> 18.8 for 524288 pairs of 65536 latents,
-// 13.7 -> 9.5 for 2048 of 4096; without 11.1 -> 10.2 there and the same for the former).
+// registers; four do not, where there are no more buckets than compute units (with records, us: 26.9 -> 18.8 for 524288 pairs of
+// 65536 latents, 13.7 -> 9.5 for 2048 of 4096, 19.5 -> 10.7 for 4710 of 262144; without 11.1 -> 10.2 for the second and the same
+// for the first).
 template <bool RECORDS, int WAVES>
 __global__ __launch_bounds__(kSortThreads, WAVES) void csr_bucket_sort_kernel(
     const uint32_t *__restrict__ tmp, const uint32_t *__restrict__ table, uint32_t n_chunks, int64_t chunk, int shift,

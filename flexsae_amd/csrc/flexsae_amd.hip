@@ -548,8 +548,9 @@ template <bool RECORDS>
 void launch_bucket_sort(const CsrScratch &sc, int64_t F, uint32_t *begin, uint32_t *map, uint32_t *slot, uint32_t *hslot,
                         uint32_t solo_bit, const PairLists &lists, const PairRecords &rec, hipStream_t st) {
   const CsrPlan &pl = sc.plan;
-  const auto kernel = static_cast<int64_t>(pl.n_buckets) * pl.n_batches <= kBucketBlocks / 2 ? csr_bucket_sort_kernel<RECORDS, 4>
-                                                                                             : csr_bucket_sort_kernel<RECORDS, 8>;
+  // (of the blocks that share a bucket most return at once)
+  const auto kernel =
+      pl.n_buckets <= kBucketBlocks / 2 ? csr_bucket_sort_kernel<RECORDS, 4> : csr_bucket_sort_kernel<RECORDS, 8>;
   hipLaunchKernelGGL(kernel, dim3(pl.n_buckets, pl.n_batches), dim3(kSortThreads), 0, st, sc.tmp, sc.table, pl.n_chunks,
                      pl.chunk, pl.shift, pl.pack_shift, F, begin, map, slot, hslot, solo_bit, lists, rec);
 }
