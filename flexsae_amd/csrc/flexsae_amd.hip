@@ -646,7 +646,7 @@ struct HierBwdPlan {
   // latents, the candidates and what became of them, the long latents that stayed cold and their
   // chunk table
   bool hot;
-  size_t off_hslot, off_hot_ctrl, off_hot_list, off_cand_list, off_long2, off_chunk2;
+  size_t off_hslot, off_hot_steps, off_hot_ctrl, off_hot_list, off_cand_list, off_long2, off_chunk2;
   int hot_rows;            // rows per block of the accumulator kernel
   size_t n_row_blocks;     // blocks of that many rows
 };
@@ -700,6 +700,8 @@ HierBwdPlan plan_hier_bwd(const flexsae_shape *s, bool hot = false, int flags = 
     const size_t n_long_max = p.n_pairs / 65 + 2;
     p.off_hslot = off;
     off += round_up(p.n_pairs * 4, kAlign);
+    p.off_hot_steps = off;  // what the walk reads of a row: hot_row_words words
+    off += round_up(p.n_rows * hot_row_words(hot_kmax(s->K)) * 4, kAlign);
     p.off_hot_ctrl = off;
     off += round_up(kHotCtrlWords * 4, kAlign);
     p.off_hot_list = off;
@@ -855,9 +857,8 @@ void launch_train_kernel_k(const flexsae_shape *s, const TrainArgs &ta, const in
 // The training-step kernel with hot-latent accumulators (16-bit weights, K <= 64): one block per
 // (row block, 128-column tile); every block first takes its share of the previous slice's second steps.
 template <typename WT, typename PT>
-void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const int64_t *indices,
-                             const void *weight, const void *vals, float coef, const uint32_t *hslot, void *P,
-                             float *dvals, float *colsum_part, float *loss_partial, int *status_flag,
+void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const uint32_t *steps, bool off32,
+                             const void *weight, float coef, void *P, float *dvals, float *colsum_part, float *loss_partial,
                              int64_t cols, int col0, int slice_w, hipStream_t st, HotFinalize fin,
                              const HotBlockFinalize &hfin, uint32_t *ctrl, float *hot_partial,
                              int hot_rows, int n_row_blocks, int headroom, void *dW_solo) {
@@ -865,21 +866,16 @@ void launch_train_hot_kernel(const flexsae_shape *s, const TrainArgs &ta, const 
     const int n_tiles = static_cast<int>(cols / kHotCols);
     const unsigned grid = static_cast<unsigned>(n_tiles) * static_cast<unsigned>(n_row_blocks);
     if (fin.mode != 0) fin.n_blocks = grid;  // every block takes a share
-    // 32-bit byte offsets from one descriptor per matrix where the matrices allow it
-    const bool off32 = s->D % kHotCols == 0 &&
-                       static_cast<uint64_t>(s->F) * s->D * sizeof(typename Traits<WT>::store_t) < (uint64_t{1} << 32) &&
-                       static_cast<uint64_t>(s->B) * s->K * slice_w * sizeof(typename Traits<PT>::store_t) < (uint64_t{1} << 31);
 #define FLEXSAE_TRAIN_HOT(KM)                                                                                   \
   do {                                                                                                          \
     const auto kernel = s->K == KM ? (off32 ? hier_train_hot_kernel<WT, PT, KM, true, true>                     \
                                             : hier_train_hot_kernel<WT, PT, KM, true, false>)                   \
                                    : (off32 ? hier_train_hot_kernel<WT, PT, KM, false, true>                    \
                                             : hier_train_hot_kernel<WT, PT, KM, false, false>);                 \
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHotThreads), 0, st, indices, weight, vals, s->vals_dtype, ta.bias, \
-                       s->bias_dtype, ta.target, s->target_dtype, coef, hslot, P, dvals, colsum_part,           \
-                       loss_partial, status_flag, s->B, n_tiles, n_row_blocks, col0, slice_w,                   \
-                       static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, hot_rows / kHotWaves, slot_mask(s), \
-                       dW_solo, fin, hfin); \
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHotThreads), 0, st, steps, weight, ta.bias, s->bias_dtype, ta.target, \
+                       s->target_dtype, coef, P, dvals, colsum_part, loss_partial, s->B, n_tiles, n_row_blocks, col0, \
+                       slice_w, static_cast<int>(s->K), s->F, static_cast<int>(s->D), ctrl, hot_partial, headroom, \
+                       hot_rows / kHotWaves, dW_solo, fin, hfin);                                               \
   } while (0)
     if (s->K <= 16) {
       FLEXSAE_TRAIN_HOT(16);
@@ -1066,14 +1062,24 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
                                 !update && !dw_scale
                             ? dW
                             : nullptr;
+  // 32-bit byte offsets from one descriptor per matrix where the matrices allow it
+  const bool hot_off32 = s->D % kHotCols == 0 && sw % kHotCols == 0 &&
+                         static_cast<uint64_t>(s->F) * s->D * sizeof(typename Traits<WT>::store_t) < (uint64_t{1} << 32) &&
+                         static_cast<uint64_t>(s->B) * s->K * slice_w * sizeof(typename Traits<PT>::store_t) < (uint64_t{1} << 31);
+  if (hot && do_sweep)
+    hipLaunchKernelGGL(hot_steps_kernel, dim3(static_cast<unsigned>(ceil_div(s->B, kWavesPerBlock))), dim3(kBlock), 0, st, indices,
+                       vals, s->vals_dtype, reinterpret_cast<const uint32_t *>(ws + pl.off_hslot), s->B, K, hot_kmax(s->K), s->F,
+                       slot_mask(s), dW_solo != nullptr, hot_off32,
+                       static_cast<uint32_t>(s->D * sizeof(typename Traits<WT>::store_t)),
+                       static_cast<uint32_t>(slice_w * sizeof(typename Traits<PT>::store_t)),
+                       reinterpret_cast<uint32_t *>(ws + pl.off_hot_steps), status_flag);
   int slice_no = 0;
   for (int64_t col0 = 0; col0 < s->D; col0 += slice_w, ++slice_no) {
     const int64_t cols = (d_used - col0) < slice_w ? (d_used - col0) : slice_w;
     const int tps = static_cast<int>(cols / pl.tile);
     if (train && do_sweep && hot) {
-      launch_train_hot_kernel<WT, PT>(s, *train, indices, weight, vals, coef,
-                                      reinterpret_cast<const uint32_t *>(ws + pl.off_hslot), P, dv_part, colsum_part,
-                                      reinterpret_cast<float *>(ws + pl.off_loss), status_flag, cols,
+      launch_train_hot_kernel<WT, PT>(s, *train, reinterpret_cast<const uint32_t *>(ws + pl.off_hot_steps), hot_off32, weight,
+                                      coef, P, dv_part, colsum_part, reinterpret_cast<float *>(ws + pl.off_loss), cols,
                                       static_cast<int>(col0), sw, st, pending, pending_hot, hot_ctrl,
                                       hot_partial[slice_no & 1], pl.hot_rows, static_cast<int>(pl.n_row_blocks), hot_headroom,
                                       dW_solo);

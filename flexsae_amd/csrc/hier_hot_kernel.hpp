@@ -300,6 +300,63 @@ __global__ __launch_bounds__(256) void hot_block_finalize_kernel(HotBlockFinaliz
   hot_block_finalize_run<GT>(h, blockIdx.x, gridDim.x);
 }
 
+// ---- what the walk reads of a row ------------------------------------------------------------
+// Per batch row four runs of KMAX words, read by the walk's scalar unit (a lane read is a vector instruction, which is what
+// binds it most: B=8192, K=64, F=262144, D=4096 bf16 Zipf 170.5 -> 162.3 us a launch, 6.7 us once for the words): where the step's weight row begins, where its contribution goes, its val as fp32 bits; steps from K on are
+// zero, and the last run begins with the row's largest |val|.  A pair whose index is out of range gets row 0 and a val of 0.
+// OFF32 (see the walk): byte offsets of the weight row and of the contribution row (multiples of 256), for a hot pair
+// kHotSlotBit and the byte offset of its accumulator row, for a latent's only pair that goes to dW the offset of the weight
+// row >> 7 (even) plus one.  Else row, slot, kHotSlotBit with the accumulator, kSoloSlotBit.
+constexpr int kStepRuns = 3;
+__host__ __device__ constexpr int hot_row_words(int kmax) { return kStepRuns * kmax + 16; }
+constexpr int hot_kmax(int64_t K) { return K <= 16 ? 16 : K <= 32 ? 32 : 64; }
+
+__global__ __launch_bounds__(256) void hot_steps_kernel(const int64_t *__restrict__ indices, const void *__restrict__ vals,
+                                                        int vals_dtype, const uint32_t *__restrict__ hslot, int64_t B, int K,
+                                                        int kmax, int64_t F, uint32_t slot_mask, int solo, int off32,
+                                                        uint32_t w_row_bytes, uint32_t p_row_bytes,
+                                                        uint32_t *__restrict__ steps, int *status_flag) {
+  const int lane = lane_id();
+  const int64_t b = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
+  if (b >= B) return;  // uniform per wavefront
+  const bool have = lane < K;
+  const int64_t mine = b * K + (have ? lane : 0);
+  int64_t idx = indices[mine];
+  float v = load_scalar(vals, vals_dtype, mine);
+  uint32_t sl = hslot[mine];
+  if (static_cast<uint64_t>(idx) >= static_cast<uint64_t>(F)) {
+    if (status_flag && have) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);
+    idx = 0;
+    v = 0.f;
+  }
+  if (!have) v = 0.f;
+  const float v_max = wave_max_bcast(fabsf(v));
+  uint32_t row = static_cast<uint32_t>(idx), word;
+  if (off32) row *= w_row_bytes;
+  if (sl & kHotSlotBit) {
+    word = off32 ? kHotSlotBit | ((sl & ~kHotSlotBit) * (kHotCols * 4u)) : sl;
+  } else if (solo && (sl & kSoloSlotBit)) {
+    word = off32 ? (row >> 7) | 1u : kSoloSlotBit;
+  } else {
+    sl &= slot_mask;
+    word = off32 ? sl * p_row_bytes : sl;
+  }
+  uint32_t *const to = steps + b * hot_row_words(kmax);
+  if (lane < kmax) {
+    to[lane] = have ? row : 0u;
+    to[kmax + lane] = have ? word : 0u;
+    to[2 * kmax + lane] = __float_as_uint(v);
+  }
+  if (lane == 0) to[kStepRuns * kmax] = __float_as_uint(v_max);
+}
+
+// N words at a wave-uniform address of memory that the kernel does not write, into scalar registers
+template <int N>
+__device__ __forceinline__ vec_t<uint32_t, N> scalar_words(const uint32_t *p) {
+  typedef const __attribute__((address_space(4))) vec_t<uint32_t, N> *from_t;
+  return *(from_t)(reinterpret_cast<uintptr_t>(p));
+}
+
 // ---- the training-step kernel with hot-latent accumulators ---------------------------------
 // One block of kHotThreads per (row block of 16 * rows_per_wave rows, 128-column tile of the slice):
 // blockIdx = row block * n_tiles + tile, so that with the usual round-robin placement the blocks
@@ -309,24 +366,24 @@ __global__ __launch_bounds__(256) void hot_block_finalize_kernel(HotBlockFinaliz
 // of storing it.  The leading work of every block is its share of the previous slice's second
 // steps (fin, hfin); the last is the flush of its accumulators to
 // hot_partial[tile][row block][accumulator row][2][64].
+// What it reads of a row's steps comes through the scalar unit (hot_steps_kernel); with lane reads instead, four a step, a
+// launch of B=8192, K=64, F=262144, D=4096 bf16 Zipf takes 170.5 us, without 162.3, and 158.3 with the turns below.  What
+// binds it then is what its rounds of rows do one after the other: gathers, 25 vector instructions a step, and stores that
+// the next row's loads are counted behind.
 // OFF32: the weight matrix is smaller than 4 GiB, the slice of contributions smaller than 2 GiB
 // and D a whole number of tiles.  Rows and contribution rows are then addressed through one
-// descriptor each plus a 32-bit byte offset that the lanes compute for all steps of a row at once
-// (lane k: step k), so a step's gather and store need one lane read each and no scalar address
-// arithmetic; for a hot pair the same word carries the hot bit and the byte offset of its
-// accumulator row.  This kernel is bound by the instructions it issues, not by its bytes.
+// descriptor each plus a 32-bit byte offset, so a step's gather and store need no address arithmetic; for a hot pair the
+// same word carries the hot bit and the byte offset of its accumulator row.
 // dW_solo (of PT's type, or null): a pair that is its latent's only one stores its contribution into the latent's
 // row of dW instead of P (see kSoloSlotBit; a fifth of the pairs that are not hot in a trained dictionary:
 // B=8192, K=64, F=262144, D=4096 bf16 Zipf: the step 2253 -> 2149 us).
 template <typename WT, typename PT, int KMAX, bool FULL, bool OFF32>
 __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
-    const int64_t *__restrict__ indices, const void *__restrict__ weight,
-    const void *__restrict__ vals, int vals_dtype, const void *__restrict__ bias, int bias_dtype,
-    const void *__restrict__ target, int target_dtype, float coef,
-    const uint32_t *__restrict__ hslot, void *__restrict__ P, float *__restrict__ dv_part,
+    const uint32_t *__restrict__ steps, const void *__restrict__ weight, const void *__restrict__ bias, int bias_dtype,
+    const void *__restrict__ target, int target_dtype, float coef, void *__restrict__ P, float *__restrict__ dv_part,
     float *__restrict__ colsum_part, float *__restrict__ loss_partial,
-    int *status_flag, int64_t B, int n_tiles, int n_row_blocks, int col0, int slice_w, int K, int64_t F, int D,
-    uint32_t *__restrict__ ctrl, float *__restrict__ hot_partial, int headroom, int rows_per_wave, uint32_t slot_mask,
+    int64_t B, int n_tiles, int n_row_blocks, int col0, int slice_w, int K, int64_t F, int D,
+    uint32_t *__restrict__ ctrl, float *__restrict__ hot_partial, int headroom, int rows_per_wave,
     void *__restrict__ dW_solo, HotFinalize fin,
     HotBlockFinalize hfin) {
   constexpr int VEC = 2;
@@ -334,7 +391,7 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
   using raw_t = typename Piece::raw_t;
   using S_t = typename Traits<WT>::store_t;
   static_assert(sizeof(raw_t) == 4 && KMAX <= kWave && KMAX % 8 == 0, "16-bit weights, at most 64 steps");
-  // an only pair in the word of a step: offsets of contribution rows are multiples of 256, slots are below 2^30
+  // an only pair that goes to dW in the word of a step: offsets of contribution rows are even, slots are below 2^30
   constexpr uint32_t kSoloWord = OFF32 ? 1u : kSoloSlotBit;
   __shared__ int acc_lds[kHotMax * kHotCols];
   __shared__ int exp_lds[kHotWaves];
@@ -398,43 +455,21 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
       const bool valid = b < B;  // uniform
       const int64_t pair0 = b * K;
 
-      int my_row = 0, my_slot = 0;
-      float my_val = 0.f, my_dval = 0.f;
+      float my_dval = 0.f;
       float e[VEC], acc[VEC];
       raw_t raw[KMAX];
       int exp_row = kHotExpMin;
+      // (uniform; the addresses of each phase are formed anew: what is read for one is not kept for the next)
+      auto run_of = [&](int run) {
+        const uint32_t *p = steps + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(b))) * hot_row_words(KMAX) +
+                            run * KMAX;
+        asm volatile("" : "+s"(p));
+        return p;
+      };
       if (valid) {
-        // everything the row needs before its gathers, requested at once and waited for once: a load
-        // issued after the stores of the row before it returns after them, so every separate wait here
-        // would cost a trip to memory of its own
-        const int64_t mine = pair0 + (lane < K ? lane : 0);
-        int64_t idx = indices[mine];
-        const uint32_t val_bits = load_scalar_bits(vals, vals_dtype, mine);
-        my_slot = static_cast<int>(hslot[mine]);
-        if (!dW_solo && my_slot >= 0) my_slot &= static_cast<int>(slot_mask);  // (bit 31 set: hot)
+        // bias and target before the gathers: the memory counter retires in order
         const PairBits bias_bits = load_pair_bits(bias, bias_dtype, dsafe);
         const PairBits target_bits = load_pair_bits(target, target_dtype, b * D + dsafe);
-        my_val = scalar_from_bits(val_bits, vals_dtype);
-        if (lane >= K) {
-          idx = 0;
-          my_val = 0.f;
-          my_slot = 0;
-        }
-        if (static_cast<uint64_t>(idx) >= static_cast<uint64_t>(F)) {
-          if (status_flag) atomicOr(status_flag, FLEXSAE_FLAG_INDEX_RANGE);
-          idx = 0;
-          my_val = 0.f;
-        }
-        my_row = static_cast<int>(idx);
-        if constexpr (OFF32) {
-          // byte offsets instead of row numbers: of the weight row, and of the contribution row or
-          // (hot bit kept) of the accumulator row
-          my_row = static_cast<int>(static_cast<uint32_t>(my_row) * w_row_bytes);
-          const uint32_t sl = static_cast<uint32_t>(my_slot);
-          my_slot = static_cast<int>((sl & kHotSlotBit) ? (kHotSlotBit | ((sl & ~kHotSlotBit) * (kHotCols * 4u)))
-                        : (dW_solo && (sl & kSoloSlotBit))  ? kSoloWord
-                                                            : sl * p_row_bytes);
-        }
         float tt[VEC];
         pair_from_bits(bias_bits, bias_dtype, e);
         pair_from_bits(target_bits, target_dtype, tt);
@@ -445,10 +480,13 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
         }
         {
           const int kb = k_bound();
+          const uint32_t *const rows = run_of(0);
+          vec_t<uint32_t, 16> part = {};
 #pragma unroll
           for (int k = 0; k < KMAX; ++k) {
+            if (k % 16 == 0) part = scalar_words<16>(rows + k);
             if (FULL || k < kb) {  // uniform
-              const uint32_t row = static_cast<uint32_t>(bcast_i32(my_row, k));
+              const uint32_t row = part[k % 16];
               const auto dw = OFF32 ? descriptor_load_at<sizeof(raw_t)>(w_all, w_lane_bytes, row)
                                     : descriptor_load<sizeof(raw_t)>(row_descriptor(weight, row, w_row_bytes), w_lane_bytes);
               __builtin_memcpy(&raw[k], &dw, sizeof(raw_t));
@@ -458,12 +496,23 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
           // the scheduler starts the walk's first step between the first two gathers
           __builtin_amdgcn_sched_barrier(0);
         }
+        // The four wavefronts of a SIMD start together and stay in step, all gathering or all computing, unless one goes
+        // ahead: each is the first in turn (B=8192, K=64, F=262144, D=4096 Zipf 163.6 -> 158.3 us; a fixed order 164.2).
+        switch (((wv >> 2) + i) & 3) {  // uniform; the builtin takes constants
+          case 0: __builtin_amdgcn_s_setprio(0); break;
+          case 1: __builtin_amdgcn_s_setprio(1); break;
+          case 2: __builtin_amdgcn_s_setprio(2); break;
+          default: __builtin_amdgcn_s_setprio(3);
+        }
         // forward walk
         const int kb_fwd = k_bound();
+        const uint32_t *const fwd_vals = run_of(2);
+        vec_t<uint32_t, 16> v_bits = {};
 #pragma unroll
         for (int k = 0; k < KMAX; ++k) {
+          if (k % 16 == 0) v_bits = scalar_words<16>(fwd_vals + k);
           if (FULL || k < kb_fwd) {  // uniform
-            const float v = bcast_f32(my_val, k);
+            const float v = __uint_as_float(v_bits[k % 16]);
             float w[VEC];
             Piece::unpack(raw[k], w);
 #pragma unroll
@@ -480,14 +529,18 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
         if (lane == kWave - 1) loss_partial[(static_cast<int64_t>(col0 / kHotCols) + t) * B + b] = lsum;
         // the row's bound on its contributions: max |v| * c * sqrt(K * max over the columns of sum_k e_k^2)
         const float acc_max = wave_max_bcast(fmaxf(acc[0], acc[1]));
-        const float v_max = wave_max_bcast(fabsf(my_val));
+        const float v_max = __uint_as_float(scalar_words<1>(run_of(kStepRuns))[0]);
         const float bound = v_max * coef * __builtin_sqrtf(static_cast<float>(K) * acc_max);
         if (!(bound <= 3.0e38f)) {  // infinity or NaN in the inputs: the block's partial sums are made NaN
           if (lane == 0) bad_lds = 1;
-        } else if (bound > 0.f) {
+        } else {
           int ex;
-          (void)__builtin_frexpf(bound, &ex);  // bound < 2^ex
-          exp_row = ex < kHotExpMin ? kHotExpMin : ex;
+          if (bound > 0.f) {
+            (void)__builtin_frexpf(bound, &ex);  // bound < 2^ex
+            exp_row = ex < kHotExpMin ? kHotExpMin : ex;
+          }
+          (void)__builtin_frexpf(v_max, &ex);  // no val times 2^(22 - E) overflows
+          exp_row = ex - 104 > exp_row ? ex - 104 : exp_row;
         }
       }
       if (calibrate) {  // the first row of every wavefront of the block sets the block's exponent
@@ -508,14 +561,24 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
         ask = exp_row > ask ? exp_row : ask;
       }
       if (!valid) continue;
+      // (a row that is walked again adds nothing yet: cheaper than a test at every step)
+      const float row_scale = hot_ok ? qscale : 0.f;
 
       // reverse walk, eight steps per dvals reduction
       float S[VEC];
 #pragma unroll
       for (int c = 0; c < VEC; ++c) S[c] = 0.f;
       const int kb_rev = k_bound();
+      const uint32_t *const rev = run_of(0);
+      // the words of eight steps, requested while the eight before them are walked
+      vec_t<uint32_t, 8> next_v = scalar_words<8>(rev + 2 * KMAX + KMAX - 8), next_w = scalar_words<8>(rev + KMAX + KMAX - 8);
 #pragma unroll
       for (int k8 = KMAX - 8; k8 >= 0; k8 -= 8) {
+        const vec_t<uint32_t, 8> v_of = next_v, w_of = next_w;
+        if (k8 > 0) {
+          next_v = scalar_words<8>(rev + 2 * KMAX + k8 - 8);
+          next_w = scalar_words<8>(rev + KMAX + k8 - 8);
+        }
         if (FULL || k8 < kb_rev) {  // uniform
           float dots[8];
 #pragma unroll
@@ -523,33 +586,35 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
             const int k = k8 + u;
             dots[u] = 0.f;
             if (FULL || k < kb_rev) {  // uniform
-              const float v = bcast_f32(my_val, k);
-              const uint32_t prow = static_cast<uint32_t>(bcast_i32(my_slot, k));
+              const float v = __uint_as_float(v_of[u]);
+              const uint32_t prow = w_of[u];
               // (laundered in place, its last use: keeps the unpacked values of the forward walk from
               // being kept alive across the two walks, at no copy)
               Piece::launder(raw[k]);
-              float w[VEC], contrib[VEC];
+              float w[VEC];
               Piece::unpack(raw[k], w);
               float dot = 0.f;
 #pragma unroll
               for (int c = 0; c < VEC; ++c) {
                 S[c] = fmaf(coef, e[c], S[c]);
-                contrib[c] = S[c] * v;
                 dot = fmaf(w[c], S[c], dot);
                 e[c] = fmaf(-w[c], v, e[c]);
               }
-              const bool is_hot = (prow & kHotSlotBit) != 0;  // uniform: a pair of a hot latent
-              if (is_hot && hot_ok) {
+              if (static_cast<int32_t>(prow) < 0) {  // uniform: a pair of a hot latent
                 int *a = OFF32 ? reinterpret_cast<int *>(reinterpret_cast<char *>(my_acc) + (prow & ~kHotSlotBit))
                                : my_acc + (prow & ~kHotSlotBit) * kHotCols;
+                const float vq = v * row_scale;
 #pragma unroll
                 for (int c = 0; c < VEC; ++c) {
-                  // round(contrib * 2^(22 - E)) as an integer: |.| <= 2^22, so adding 1.5 * 2^23 leaves it in
+                  // round(S v 2^(22 - E)) as an integer: |.| <= 2^22, so adding 1.5 * 2^23 leaves it in
                   // the low mantissa bits (round to nearest even), one instruction instead of three
-                  const int q = __float_as_int(fmaf(contrib[c], qscale, 12582912.0f)) - 0x4B400000;
+                  const int q = __float_as_int(fmaf(S[c], vq, 12582912.0f)) - 0x4B400000;
                   __hip_atomic_fetch_add(a + c * kWave, q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
-              } else if (!is_hot) {
+              } else {
+                float contrib[VEC];
+#pragma unroll
+                for (int c = 0; c < VEC; ++c) contrib[c] = S[c] * v;
                 vec_t<uint32_t, VEC * sizeof(typename Traits<PT>::store_t) / 4> packed;
                 if constexpr (Traits<PT>::dtype == FLEXSAE_BF16) {
                   packed[0] = f32x2_to_bf16x2_bits(contrib[0], contrib[1]);
@@ -558,17 +623,19 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
 #pragma unroll
                   for (int c = 0; c < VEC; ++c) packed[c] = __float_as_uint(contrib[c]);
                 }
-                if (prow & kSoloWord) {  // uniform; (OFF32: my_row holds byte offsets of weight rows)
-                  const uint32_t row = static_cast<uint32_t>(bcast_i32(my_row, k));
+                if (prow & kSoloWord) {
                   constexpr uint32_t kElem = sizeof(typename Traits<PT>::store_t);
-                  char *const dst = static_cast<char *>(dW_solo) +
-                                    (OFF32 ? static_cast<uint64_t>(row) * (kElem / sizeof(S_t))
-                                           : static_cast<uint64_t>(row) * static_cast<uint32_t>(D) * kElem);
+                  const uint64_t at = OFF32 ? static_cast<uint64_t>((prow & ~1u) << 7) * (kElem / sizeof(S_t))
+                                            : static_cast<uint64_t>(scalar_words<1>(rev + k)[0]) * static_cast<uint32_t>(D) * kElem;
+                  char *const dst = static_cast<char *>(dW_solo) + at;
                   descriptor_store<sizeof(packed), true>(
                       __builtin_amdgcn_make_buffer_rsrc(dst, 0, static_cast<int>(static_cast<uint32_t>(D) * kElem), 0x00020000),
                       static_cast<uint32_t>(d0) * kElem, packed);
-                } else if constexpr (OFF32) descriptor_store_at<sizeof(packed), false>(p_all, p_lane_bytes, prow, packed);
-                else descriptor_store<sizeof(packed), false>(row_descriptor(P, prow, p_row_bytes), p_lane_bytes, packed);
+                } else if constexpr (OFF32) {
+                  descriptor_store_at<sizeof(packed), false>(p_all, p_lane_bytes, prow, packed);
+                } else {
+                  descriptor_store<sizeof(packed), false>(row_descriptor(P, prow, p_row_bytes), p_lane_bytes, packed);
+                }
               }
               dots[u] = dot;  // zero where the lane is beyond column D: its w is zero
             }
