@@ -108,23 +108,18 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
     hot_finalize_carried<WT>(fin, blockIdx.x);
     return;
   }
-  // the last ones clear the rows of latents without pairs (the first slice's launch, where they are listed)
-  const unsigned n_walk = gridDim.x - zero.n_blocks;
-  if (blockIdx.x >= n_walk) {
-    zero_rows_carried(zero, D, blockIdx.x - n_walk);
+  // (a launch holds fewer than 2^26 wavefronts, and a row number has 32 bits)
+  const uint32_t item = (blockIdx.x - fin.n_blocks) * (256 / kWave) + wave_in_block();
+  if (item >= static_cast<uint64_t>(n_items)) {  // uniform per wavefront
+    // the last blocks clear the rows of latents without pairs (the first slice's launch, where they are listed)
+    const unsigned n_walk = gridDim.x - zero.n_blocks;
+    if (blockIdx.x >= n_walk) zero_rows_carried(zero, D, blockIdx.x - n_walk);
     return;
   }
-  const int64_t item = static_cast<int64_t>(blockIdx.x - fin.n_blocks) * (blockDim.x >> 6) + wave_in_block();
-  if (item >= n_items) return;  // uniform per wavefront
-  int t;
-  int64_t b;
-  if (row_tiles > 0) {  // uniform
-    b = item / row_tiles;
-    t = static_cast<int>(item - b * row_tiles);
-  } else {
-    t = static_cast<int>(item / B);
-    b = item - static_cast<int64_t>(t) * B;
-  }
+  const uint32_t per = row_tiles > 0 ? static_cast<uint32_t>(row_tiles) : static_cast<uint32_t>(B);
+  const uint32_t quot = item / per, rest = item - quot * per;
+  const int t = static_cast<int>(row_tiles > 0 ? rest : quot);
+  const int64_t b = row_tiles > 0 ? quot : rest;
   const int pc = t * (kWave * VEC) + lane * VEC;  // column inside the slice
   const int d0 = col0 + pc;
   const bool active = d0 < D;
