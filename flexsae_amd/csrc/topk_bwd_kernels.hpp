@@ -86,6 +86,25 @@ constexpr int topk_group() {
   return sizeof(LatentPiece<WT, GT, VEC>) > 16 ? 4 : 8;
 }
 
+// Stores of dW take the streaming hint but for rows stored two bytes per lane, whose runs of 128 bytes begin and end inside lines,
+// and, where nearly all rows are zeros (`plain`), for rows stored four bytes per lane.  us with / without it, uniform and skewed
+// indices: D=1001 bf16 B=128, K=32, F=131072 159 / 113, 160 / 113, B=1024 169 / 155, 182 / 145; D=1938 B=128 239 / 207, 239 / 187,
+// D=778 fp16 156 / 130, 156 / 121; not B=1024 D=1938 252 / 273, 257 / 271, B=4096, F=65536 266 / 268, 268 / 306, and
+// not with eight bytes and more (B=1024, F=131072, D=1764 bf16 189 / 271, D=2304 215 / 274).
+template <bool STREAM, typename V>
+__device__ __forceinline__ void store_dw(V *to, V x, bool plain) {
+  if constexpr (STREAM && sizeof(V) == 4) {
+    if (plain) {  // uniform
+      asm volatile("");  // (two stores that differ in the hint alone would become one without it)
+      *to = x;
+      asm volatile("");
+      return;
+    }
+  }
+  if constexpr (STREAM && sizeof(V) >= 4) __builtin_nontemporal_store(x, to);
+  else *to = x;
+}
+
 // The short latents (at most kSegChunk pairs) of a group of L neighbours, one tile: their pairs are one run of slots but for
 // the long latents among them, so a wavefront walks them as one stream.  The chain of trips to memory at the head of a
 // latent (its bounds, its records and W row, the first residual rows) is paid once per group, and the batches of eight rows
@@ -107,7 +126,7 @@ __device__ __forceinline__ void topk_short_latents(
     const uint32_t *__restrict__ begin, const vec_t<uint32_t, 2> *__restrict__ slot_bv, const void *__restrict__ weight,
     int vals_dtype, const GatherSource &rows_src, uint32_t row_stride, float scale, void *__restrict__ dW,
     float *__restrict__ dv_tile, int64_t f0, int per_wave, int64_t F, int d0, int D,
-    LatentPiece<WT, GT, VEC> *__restrict__ pieces) {
+    LatentPiece<WT, GT, VEC> *__restrict__ pieces, bool plain) {
   using S = typename Traits<RT>::store_t;
   using S_w = typename Traits<WT>::store_t;
   static_assert(L <= 8, "the counts of a wavefront's latents are scanned inside eight lanes");
@@ -318,8 +337,7 @@ __device__ __forceinline__ void topk_short_latents(
         if (n == 0) x = raw_vec_t<GT, EV>{};
         if (d < D) {
           auto *const to = reinterpret_cast<raw_vec_t<GT, EV> *>(static_cast<G *>(dW) + (f0 + l) * D + d);
-          if constexpr (FLEXSAE_TOPK_NT) __builtin_nontemporal_store(x, to);
-          else *to = x;
+          store_dw<FLEXSAE_TOPK_NT>(to, x, plain);
         }
       }
     }
@@ -457,7 +475,7 @@ __device__ __forceinline__ void topk_short_latent(
 #pragma unroll
     for (int i = 0; i < VEC; ++i) acc[i] *= scale;
   }
-  if (active) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f * D + d0, acc);
+  if (active) store_vec<GT, VEC, FLEXSAE_TOPK_NT && sizeof(raw_vec_t<GT, VEC>) >= 4>(dW, f * D + d0, acc);
   if (lane < n) dv_tile[b0 + lane] = my_dot * scale;
 }
 
@@ -505,7 +523,7 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
       const int d0 = col0 + static_cast<int>(t) * (kWave * VEC) + lane * VEC;
       if (n == 0) {  // unused latent: zeros
         const float zero[VEC] = {};
-        if (d0 < D) store_vec<GT, VEC, FLEXSAE_TOPK_NT>(dW, f0 * D + d0, zero);
+        if (d0 < D) store_vec<GT, VEC, FLEXSAE_TOPK_NT && sizeof(raw_vec_t<GT, VEC>) >= 4>(dW, f0 * D + d0, zero);
         return;
       }
       topk_short_latent<WT, GT, RT, VEC>(
@@ -517,7 +535,8 @@ __global__ __launch_bounds__(256) void topk_bwd_kernel(
       topk_short_latents<WT, GT, RT, VEC, EV, L>(
           begin, slot_bv, weight, vals_dtype, rows_src, static_cast<uint32_t>(resid_ld) * sizeof(typename Traits<RT>::store_t), scale,
           dW, dv_part + (col0 / (kWave * VEC) + t) * n_pairs, f0, per_wave, F,
-          col0 + static_cast<int>(t) * (kWave * VEC) + lane * VEC, D, pieces[wave_in_block()]);
+          col0 + static_cast<int>(t) * (kWave * VEC) + lane * VEC, D, pieces[wave_in_block()],
+          16 * n_pairs < F);
     }
     return;
   }
