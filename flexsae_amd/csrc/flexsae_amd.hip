@@ -809,8 +809,10 @@ void launch_train_kernel(const flexsae_shape *s, const TrainArgs &ta, const int6
   // of one tile anyway: what is gathered and stored of a row then lies side by side.  us of the step by tile / by row: B=1024,
   // K=64, F=65536, D=4096 bf16 407 / 387, B=128, K=128, F=16384, D=2048 73 / 66, B=512, K=64, F=65536, D=2048 fp32 274 / 255,
   // B=207, K=90, F=68238, D=2348 fp16 228 / 224, B=1777, K=50, F=24571, D=1538 193 / 187; not B=2048, K=64, F=32768, D=1024 bf16
-  // 165 / 167, B=4096, K=128, F=65536, D=2304 1224 / 1257.
-  const int row_tiles = s->B < 2048 ? static_cast<int>(cols / (kWave * VEC)) : 0;
+  // 165 / 167, B=4096, K=128, F=65536, D=2304 1224 / 1257, nor in slices where latents repeat, B=1024, K=100, F=40000, D=2304
+  // 318 / 323.
+  const bool by_row = s->B < 2048 && (slice_w >= s->D || s->B * s->K <= s->F);
+  const int row_tiles = by_row ? static_cast<int>(cols / (kWave * VEC)) : 0;
   const auto kernel = s->K == KMAX
                           ? (stream ? hier_train_kernel<WT, PT, KMAX, true, true, VEC, LDSROWS>
                                     : hier_train_kernel<WT, PT, KMAX, true, false, VEC, LDSROWS>)
@@ -1037,7 +1039,7 @@ void launch_hier_slices(const flexsae_shape *s, const HierBwdPlan &pl, int64_t s
   // rows of latents without pairs are zeroed here, whole rows in one pass (the in-place update leaves
   // them alone).
   const bool sparse = piece != 0 && sparse_latents(s, flags);
-  // (by the last blocks of the first walk, where that is hier_train_kernel)
+  // (by the first blocks of the first walk, where that is hier_train_kernel)
   ZeroRows zero = {};
   if (sparse && do_reduce && !update) {
     const unsigned n_zero_blocks = static_cast<unsigned>(ceil_div(s->F, kZeroRows * kWavesPerBlock));

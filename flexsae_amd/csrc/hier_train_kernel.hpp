@@ -68,7 +68,9 @@ struct RowPiece<f16_t, 2> {
 // back with plain LDS loads.  bias - target is fetched before the gathers are issued: the memory
 // counter retires in order, so anything issued after them can only be waited for together with
 // all of them, and the forward walk could not start while rows are still arriving.
-// zero: rows of dW to clear, by the last blocks; a launch of its own costs 4-5 us on the device and as much on the host.
+// zero: rows of dW to clear; a launch of its own costs 4-5 us on the device and as much on the host.  By the first blocks:
+// cleared last they would take the place of the slice's contributions in the memory-side cache (B=4096, K=32, F=65536, D=1538
+// fp32 Zipf 612 -> 631 us).
 // row_tiles: 0: the items are all rows of one tile after the other; else so many tiles of one row after the other.
 // fin: the second step of the previous slice's hot latents (see HotFinalize), run by the leading blocks
 // of the launch into a gradient of CarriedGrad's type, or into the weights.
@@ -103,19 +105,17 @@ __global__ __launch_bounds__(256) void hier_train_kernel(
   __shared__ uint32_t lds_rows[LDSROWS > 0 ? (256 / kWave) * LDSROWS * kWave : 1];
   uint32_t *const my_lds = lds_rows + wave_in_block() * (LDSROWS * kWave);
   const int lane = lane_id();
-  // the leading blocks finish the hot latents of the previous slice (fin.n_blocks of them; none at the first slice)
-  if (blockIdx.x < fin.n_blocks) {
-    hot_finalize_carried<WT>(fin, blockIdx.x);
+  // the leading blocks finish the hot latents of the previous slice (fin.n_blocks of them; none at the first slice) and clear
+  // the rows of latents without pairs (the first slice's launch, where they are listed)
+  const unsigned n_lead = fin.n_blocks + zero.n_blocks;
+  if (blockIdx.x < n_lead) {
+    if (blockIdx.x < fin.n_blocks) hot_finalize_carried<WT>(fin, blockIdx.x);
+    else zero_rows_carried(zero, D, blockIdx.x - fin.n_blocks);
     return;
   }
   // (a launch holds fewer than 2^26 wavefronts, and a row number has 32 bits)
-  const uint32_t item = (blockIdx.x - fin.n_blocks) * (256 / kWave) + wave_in_block();
-  if (item >= static_cast<uint64_t>(n_items)) {  // uniform per wavefront
-    // the last blocks clear the rows of latents without pairs (the first slice's launch, where they are listed)
-    const unsigned n_walk = gridDim.x - zero.n_blocks;
-    if (blockIdx.x >= n_walk) zero_rows_carried(zero, D, blockIdx.x - n_walk);
-    return;
-  }
+  const uint32_t item = (blockIdx.x - n_lead) * (256 / kWave) + wave_in_block();
+  if (item >= static_cast<uint64_t>(n_items)) return;  // uniform per wavefront
   const uint32_t per = row_tiles > 0 ? static_cast<uint32_t>(row_tiles) : static_cast<uint32_t>(B);
   const uint32_t quot = item / per, rest = item - quot * per;
   const int t = static_cast<int>(row_tiles > 0 ? rest : quot);

@@ -232,7 +232,7 @@ def _train_tile_cols(K: int, weight_dtype) -> int:
     return 64 if (weight_dtype == torch.float32 and K > 64) else 128
 
 
-def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype) -> int:
+def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype, step: bool = True) -> int:
     """Bytes the contributions of one slice may take.  Unless set explicitly: 0.45 of the weight
     matrix, at most 256 MiB -- memory above the inputs then stays within about 1.25 of the TopK
     loss's (whose peak is the dense gradient plus the residual) whatever K is, at 4-5 % of the step
@@ -245,12 +245,13 @@ def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype) -> int:
     D = 2048 fp32 679, 364, 350).  With such weights all contributions at once where they take at most 384 MiB (us with
     128 MiB / all: B = 1500, K = 40, F = 24571, D = 2328 bf16 208 / 189, fp32 D = 1160 206 / 183, fp16 205 / 192; B = 512,
     K = 64, F = 16384, D = 5488 bf16 248 / 219; B = 400, K = 100, F = 60000, D = 1872 166 / 144; over 64 shapes 4 % less on
-    average, one more than 4 % more: B = 1900, K = 128, F = 8192, D = 152 fp32 124 / 131)."""
+    average, one more than 4 % more: B = 1900, K = 128, F = 8192, D = 152 fp32 124 / 131); ``step`` false, forward and sweep, not
+    (B = 512, K = 150, F = 30000, Zipf, D = 2304 bf16 278 / 293, D = 1024 fp32 218 / 235)."""
     if _hier_scratch_bytes is not None:
         return _hier_scratch_bytes
     sw = 4 if weight_dtype == torch.float32 else 2
     budget = min(_HIER_SCRATCH_CAP, max(_HIER_SCRATCH_LEAST, int(0.45 * F * D * sw)))
-    if budget == _HIER_SCRATCH_LEAST:
+    if step and budget == _HIER_SCRATCH_LEAST:
         tile = _train_tile_cols(K, weight_dtype)
         whole = B * K * (-(-D // tile) * tile) * (2 if weight_dtype == torch.bfloat16 else 4)
         if whole <= _HIER_SCRATCH_WHOLE:
@@ -258,11 +259,11 @@ def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype) -> int:
     return budget
 
 
-def _hier_slice_cols(B: int, K: int, F: int, D: int, weight_dtype) -> int:
+def _hier_slice_cols(B: int, K: int, F: int, D: int, weight_dtype, step: bool = True) -> int:
     p_size = 2 if weight_dtype == torch.bfloat16 else 4
     tile = _train_tile_cols(K, weight_dtype)
     floor = _hier_min_slice_cols if _hier_min_slice_cols is not None else (64 if tile == 64 else 256)
-    cols = _hier_scratch_budget(B, K, F, D, weight_dtype) // (B * K * p_size)
+    cols = _hier_scratch_budget(B, K, F, D, weight_dtype, step) // (B * K * p_size)
     if cols >= tile:
         cols -= cols % tile  # whole tiles: the library rounds up, the budget is an upper bound
     return max(floor, cols, 1)
@@ -541,7 +542,7 @@ def _hier_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tens
         dvals = torch.empty((B, K), dtype=torch.float32, device=dev)
         dbias = torch.empty((D,), dtype=torch.float32, device=dev)
         if _hier_scratch_budget(B, K, F, D, weight.dtype) > 0:
-            slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype)
+            slice_cols = _hier_slice_cols(B, K, F, D, weight.dtype, False)
             ws_bytes = lib.flexsae_hier_bwd_workspace_bytes(ctypes.byref(shape), slice_cols)
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
             dW = torch.empty_like(weight)
@@ -1416,14 +1417,14 @@ class _Route:
         self.train = takes and _hier_scratch_bytes != 0 and (_step_pays(weight, K) or _one_gather_pays(weight, B, K))
         # by the functions of this module
         self.here = stage or _hier_scratch_budget(B, K, F, D, dtype) <= 0
-        self._step(B, K, F, D, dtype, device, need_dw, _lib.BWD_RAGGED_ROWS if _train_ragged(weight, K) else 0)
+        self._step(B, K, F, D, dtype, device, need_dw, _lib.BWD_RAGGED_ROWS if _train_ragged(weight, K) else 0, self.train)
         self.late = self.train and need_dw and _late_step(weight, B, K)
 
-    def _step(self, B, K, F, D, dtype, device, need_dw, ragged):
+    def _step(self, B, K, F, D, dtype, device, need_dw, ragged, step=True):
         self.late = False
         self.key = _hot_key(device, B, K, F, D, dtype)
         self.ragged = ragged
-        self.cols = _hier_slice_cols(B, K, F, D, dtype)
+        self.cols = _hier_slice_cols(B, K, F, D, dtype, step)
         hot_can = need_dw and _hot_latents != "off" and _hot_latents_supported(B, K, F, D, dtype)
         dense_can = need_dw and _dense_latents != "off" and B * K <= 2 * F
         self.hot = _hot_latents if hot_can else "off"
