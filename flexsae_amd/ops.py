@@ -26,6 +26,7 @@ index checking is switched on.
 """
 from __future__ import annotations
 
+import collections
 import contextlib
 import ctypes
 import os
@@ -304,7 +305,13 @@ _dense_latents = os.environ.get("FLEXSAE_DENSE_LATENTS", "auto").lower()
 _HOT_ROWS_PER_BLOCK = 128   # kHotRowsPerBlock of the library
 _HOT_AUTO_FRACTION = 0.25   # of the pairs in latents with more than 64 pairs
 _DENSE_AUTO_FRACTION = 0.40  # of the latents without a pair
-_hot_auto = {}              # (device index, B, K, F, D, dtype) -> {"hot", "dense", "pinned", "event"}
+_hot_auto = {}              # (device index, B, K, F, D, dtype) -> {"hot", "dense", "pinned", "event", ...} (_new_stats)
+_hot_retired = collections.deque(maxlen=1024)  # buffers of forgotten shapes: a step under way may still write its words
+
+
+def _forget_stats() -> None:
+    _hot_retired.extend(st["pinned"] for st in _hot_auto.values())
+    _hot_auto.clear()
 
 
 def set_hot_latents(mode) -> None:
@@ -319,7 +326,7 @@ def set_hot_latents(mode) -> None:
     if mode not in ("auto", "on", "off"):
         raise ValueError("set_hot_latents: expected 'auto', 'on' or 'off'")
     _hot_latents = mode
-    _hot_auto.clear()
+    _forget_stats()
 
 
 def set_dense_latents(mode) -> None:
@@ -334,7 +341,7 @@ def set_dense_latents(mode) -> None:
     if mode not in ("auto", "on", "off"):
         raise ValueError("set_dense_latents: expected 'auto', 'on' or 'off'")
     _dense_latents = mode
-    _hot_auto.clear()
+    _forget_stats()
 
 
 def _hot_latents_supported(B: int, K: int, F: int, D: int, weight_dtype) -> bool:

@@ -2,6 +2,7 @@
 eager torch definitions, and that nothing in the package touches the oracle."""
 import os
 import re
+import weakref
 
 import pytest
 import torch
@@ -88,3 +89,15 @@ def test_rows_per_block_of_the_hot_latent_step(B, K, D, want):
     assert got == want
     blocks = -(-B // (128 >> got)) * -(-D // 128)
     assert got == 0 or blocks <= 256
+
+
+@pytest.mark.parametrize("forget", [lambda: flex.set_hot_latents("auto"), lambda: flex.set_dense_latents("auto")])
+def test_forgotten_index_statistics_keep_their_buffer(forget):
+    """A step under way may still write the words of a shape whose statistics were dropped."""
+    words = torch.zeros(4, dtype=torch.int32)
+    alive = weakref.ref(words)
+    ops._hot_auto["a shape"] = {"pinned": words}
+    del words
+    forget()
+    assert "a shape" not in ops._hot_auto and alive() is not None
+    ops._hot_retired.pop()
