@@ -463,7 +463,7 @@ struct CsrPlan {
 
 CsrPlan plan_csr(int64_t n_pairs, int64_t F) {
   CsrPlan p;
-  // latents per bucket: about 2048 pairs per bucket on average, a power of two; more than 2048 latents only where buckets
+  // latents per bucket: about 2048 pairs per bucket on average, a power of two (see below for fewer); more than 2048 latents only where buckets
   // of 2048 are more than the chip holds at once (2097152 latents, 262144 pairs: 29 us that way and 21 with 4096 latents;
   // 1048576 latents fit and are as fast either way)
   int shift = 0;
@@ -471,6 +471,15 @@ CsrPlan plan_csr(int64_t n_pairs, int64_t F) {
          (shift < 11 || ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketBlocks))
     ++shift;
   while (shift < kSortMaxShift && ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketMaxBuckets) ++shift;
+  // Half as many where every compute unit still has at most one block (with the batches below): a block with fewer pairs is done
+  // sooner, one with frequent latents above all.  us of the pair list, uniform and skewed (distinct in a row), before / with this:
+  // B=1024, K=64, F=32768 18.1 / 17.1, 27.6 / 25.6; B=4096, K=64, F=65536 22.5 / 22.8, 33.8 / 31.5; B=404, K=50, F=12953 16.9 /
+  // 15.9, 23.8 / 21.3; not with more blocks than that: B=2435, K=128, F=24332 in 381 buckets 23.1 / 24.5, 31.3 / 36.2, B=2048,
+  // K=64, F=262144 in 256 of two batches 21.4 / 24.5; nor a quarter, whose chunks take longer to order (B=1777, K=50, F=24571,
+  // D=1538 bf16, the step: 183.6 us with 2048 pairs, 181.9 with 1024, 186.7 with 512).
+  while (shift > 0 && (n_pairs << shift) > 1024 * F &&
+         ceil_div(F, int64_t{1} << (shift - 1)) * ceil_div(int64_t{1} << (shift - 1), kRunLatents) <= kBucketBlocks / 2)
+    --shift;
   p.shift = shift;
   p.pack_shift = csr_pack_shift(shift);
   const int64_t n_buckets = ceil_div(F, static_cast<int64_t>(1) << shift);
