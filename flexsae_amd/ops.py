@@ -409,7 +409,7 @@ def _hot_measure(lib, shape, workspace: Tensor, B, K, F, D, weight_dtype) -> Non
         return
     key = _hot_key(workspace.device, B, K, F, D, weight_dtype)
     st = _hot_auto.get(key) or _new_stats(key)
-    if st["event"] is not None or st["seen"] != st["asked"]:
+    if st["event"] is not None:
         return  # a measurement is still on its way
     rc = lib.flexsae_hier_pair_stats(ctypes.byref(shape), _ptr(workspace), _ptr(st["pinned"]), _stream())
     _lib.check(rc, "flexsae_hier_pair_stats")
@@ -1452,8 +1452,10 @@ class _Route:
             if st is not None:
                 hot = hot or (self.hot == "auto" and st["hot"])
                 dense = dense or (self.dense == "auto" and st["dense"])
-            # (a late step that is never asked for its gradients measures nothing: the next one does not wait for it)
-            if self.measures and (st is None or (st["event"] is None and (self.late or st["seen"] == st["asked"]))):
+            # Every step is asked, whether or not those before it have answered: one that is refused, fails or, late, is never
+            # asked for its gradients answers nothing.  (The steps under way write whole words, and each word is read for one
+            # decision alone.)
+            if self.measures:
                 st = st or _new_stats(self.key)
                 tag = st["asked"] = st["asked"] % 0xffffffff + 1
                 pinned = st["pinned"]

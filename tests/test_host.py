@@ -1,5 +1,6 @@
 """Host-side logic of the python layer (no GPU): validation, public names, fake kernels, the
 eager torch definitions, and that nothing in the package touches the oracle."""
+import ctypes
 import os
 import re
 import weakref
@@ -101,3 +102,48 @@ def test_forgotten_index_statistics_keep_their_buffer(forget):
     forget()
     assert "a shape" not in ops._hot_auto and alive() is not None
     ops._hot_retired.pop()
+
+
+@pytest.mark.parametrize("late", [False, True])
+def test_a_step_that_was_not_taken_leaves_the_measurement_alive(late, monkeypatch):
+    """The extension module may refuse a call, or raise, after the call has been given its measurement to leave: the next step
+    of the shape asks again, and what arrives is read."""
+    words = torch.zeros(4, dtype=torch.int32)
+
+    def new_stats(key):
+        st = ops._hot_auto[key] = {"hot": False, "dense": False, "pinned": words, "event": None, "spare": None,
+                                   "words": (ctypes.c_uint32 * 4).from_address(words.data_ptr()), "seen": 0, "asked": 0}
+        return st
+
+    monkeypatch.setattr(ops, "_new_stats", new_stats)
+    monkeypatch.setattr(ops, "_hot_auto", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    B, K, F, D = 64, 32, 4096, 256
+    route = ops._Route.__new__(ops._Route)
+    route._step(B, K, F, D, torch.float32, torch.device("cuda", 0), True, 0)
+    route.late = late
+    monkeypatch.setattr(ops, "_route", lambda *_: route)
+    route.here, route.train = False, True
+    args = make_inputs(B, K, F, D)
+    args = (args[0], *(x.requires_grad_() for x in args[1:4]), args[4])
+    asked = []
+
+    class Module:
+        def hier_sliced(self, *a):
+            asked.append(a[-2:])
+            if len(asked) == 1:
+                return None
+            if len(asked) == 2:
+                raise RuntimeError("no memory")
+            return torch.zeros(())
+
+        hier_late = hier_sliced
+
+    assert ops._native_hier(Module(), *args) is None
+    with pytest.raises(RuntimeError):
+        ops._native_hier(Module(), *args)
+    ops._native_hier(Module(), *args)
+    assert len({tag for _, tag in asked}) == 3 and 0 not in {tag for _, tag in asked}
+    assert all(pinned is words for pinned, _ in asked)
+    words[:] = torch.tensor([0, 0, 100, asked[-1][1]], dtype=torch.int32)  # (few latents without a pair)
+    assert ops._index_stats(route.key, B, K, F)["dense"] is True
