@@ -229,13 +229,17 @@ Step hier_step(const Inputs &given, const StepPlan &p, const Tensor &grad = Tens
   r.dbias = make(in.weight, {s.D}, c10::ScalarType::Float);
   const Tensor g = grad.defined() ? grad_scalar(grad, in.weight.device()) : Tensor();
   const Tensor by = step.defined() ? grad_scalar(step, in.weight.device()) : Tensor();
-  check(lib.hier_step(&s, index_ptr(in.indices), in.weight.data_ptr(), in.vals.data_ptr(), in.bias.data_ptr(),
-                      in.target.data_ptr(), g.defined() ? f32(g) : nullptr, by.defined() ? f32(by) : nullptr, f32(r.loss),
-                      r.dW.defined() ? r.dW.data_ptr() : nullptr, dtype_of(type), f32(r.dvals), f32(r.dbias),
-                      workspace.data_ptr(), bytes, static_cast<int>(p.flags) | (p.need_dw ? 0 : FLEXSAE_BWD_NO_DW),
-                      p.stats.defined() ? static_cast<uint32_t *>(p.stats.data_ptr()) : nullptr,
-                      static_cast<uint32_t>(p.tag), flag_of(in.weight), stream_of(in.weight)),
-        "flexsae_hier_step");
+  const int status = lib.hier_step(
+      &s, index_ptr(in.indices), in.weight.data_ptr(), in.vals.data_ptr(), in.bias.data_ptr(), in.target.data_ptr(),
+      g.defined() ? f32(g) : nullptr, by.defined() ? f32(by) : nullptr, f32(r.loss),
+      r.dW.defined() ? r.dW.data_ptr() : nullptr, dtype_of(type), f32(r.dvals), f32(r.dbias), workspace.data_ptr(), bytes,
+      static_cast<int>(p.flags) | (p.need_dw ? 0 : FLEXSAE_BWD_NO_DW),
+      p.stats.defined() ? static_cast<uint32_t *>(p.stats.data_ptr()) : nullptr, static_cast<uint32_t>(p.tag),
+      flag_of(in.weight), stream_of(in.weight));
+  // (a call that was refused, here or by an allocation above, has left the weights alone)
+  if (step.defined() && (status == FLEXSAE_OK || status == FLEXSAE_ERR_LAUNCH))
+    torch::autograd::impl::bump_version(given.weight);
+  check(status, "flexsae_hier_step");
   return r;
 }
 
@@ -543,7 +547,6 @@ PyObject *py_hier_sgd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   {
     pybind11::gil_scoped_release no_gil;
     const c10::AutoGradMode no_grad(false);
-    torch::autograd::impl::bump_version(in.weight);
     in.vals = in.vals.detach();
     in.bias = in.bias.detach();
     r = hier_step(in, plan, Tensor(), step);

@@ -947,6 +947,11 @@ def _hier_sgd_step_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Ten
     too, and the dense gradient of ``triton_hierarchical_sae_loss`` is the interface to use.
     ``weight`` must be contiguous and 16-byte aligned, D a multiple of 8 (16-bit) or 4 (fp32),
     K <= 256."""
+    return _sgd_step(indices, weight, vals, bias, target, step)
+
+
+def _sgd_step(indices, weight, vals, bias, target, step, changed=None):
+    """``hier_sgd_step``; ``changed`` is called once the weights may have changed (not where the call is refused)."""
     B, K, F, D = _validate(indices, weight, vals, bias, target)
     if not weight.is_contiguous() or weight.data_ptr() % 16 or not weight.data_ptr():
         raise ValueError("hier_sgd_step updates weight in place: it must be contiguous and 16-byte aligned")
@@ -980,6 +985,8 @@ def _hier_sgd_step_impl(indices: Tensor, weight: Tensor, vals: Tensor, bias: Ten
                                        (_lib.BWD_REUSE_PAIR_LIST if cached is not None else 0) | hot_flag | dense_flag,
                                        _ptr(flag),
                                        _stream())
+        if changed is not None and rc in (_lib.OK, _lib.ERR_LAUNCH):
+            changed()
         _lib.check(rc, "flexsae_hier_sgd_step")
         if cached is None:
             _pair_export(lib, shape, workspace, indices, F)
@@ -1020,8 +1027,8 @@ def hierarchical_sae_sgd_step(indices: Tensor, weight: Tensor, vals: Tensor, bia
                 if out is not None:
                     return out
         if _plain_call(indices, weight, vals, bias, target, step):
-            torch.autograd.graph.increment_version(weight)  # what the op's schema says of its weight
-            return _hier_sgd_step_impl(indices, weight, vals.detach(), bias.detach(), target, step)
+            return _sgd_step(indices, weight, vals.detach(), bias.detach(), target, step,
+                             lambda: torch.autograd.graph.increment_version(weight))  # what the op's schema says of its weight
         return hier_sgd_step(indices, weight, vals.detach(), bias.detach(), target, step)
 
 

@@ -1,5 +1,6 @@
 """Ordinary eager calls go past the dispatcher: the same bits as through the ops, and the ops wherever something has to see
 them (modes, transforms, a graph of the backward)."""
+import contextlib
 import ctypes
 
 import pytest
@@ -134,6 +135,20 @@ def test_the_fused_update_marks_the_weight():
     with _Seen():
         want = flex.hierarchical_sae_sgd_step(idx, W2, v, b, t, 0.5)
     assert torch.equal(W, W2) and all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_a_refused_update_leaves_the_weight_as_it_was(shared):
+    """Rows that the update does not take: the weight keeps its values and its version, and a graph that saved it its backward."""
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 132, torch.bfloat16, seed=4))
+    before, version = W.clone(), W._version
+    vals = v.clone().requires_grad_()
+    loss = flex.triton_topk_sae_loss(idx, W, vals, b, t)
+    with flex.shared_pair_list() if shared else contextlib.nullcontext():
+        with pytest.raises(_lib.FlexSAELibraryError):
+            flex.hierarchical_sae_sgd_step(idx, W, v, b, t, 0.5)
+    assert W._version == version and torch.equal(W, before)
+    loss.backward()
 
 
 def test_finish_grads_checks_its_arguments():
