@@ -52,14 +52,20 @@ constexpr int kHotExpMin = -96;         // exponents are clamped to [kHotExpMin,
 // the long latents that stayed cold.
 enum { kHotNHot = 0, kHotNCand = 1, kHotLong2Count = 2, kHotThreshold = 3, kHotDeferred = 4, kHotLong2 = 6, kHotCtrlWords = 64 };
 
+// The largest value of the wavefront, of values >= 0 and NaNs, which count as larger than infinity: fmaxf would drop them, their
+// bits compared as whole numbers are above all others.
+__device__ __forceinline__ uint32_t max_bits(uint32_t a, uint32_t b) { return a > b ? a : b; }
+
 __device__ __forceinline__ float wave_max_bcast(float v) {
-  v = fmaxf(v, dpp_move<0xB1>(v));       // lanes whose source does not exist receive 0: the values are >= 0
-  v = fmaxf(v, dpp_move<0x4E>(v));
-  v = fmaxf(v, dpp_move<0x141>(v));
-  v = fmaxf(v, dpp_move<0x140>(v));
-  v = fmaxf(v, dpp_move<0x142, 0xa>(v));
-  v = fmaxf(v, dpp_move<0x143, 0xc>(v));
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+  uint32_t x = __float_as_uint(v);
+  // (lanes whose source does not exist receive 0)
+  x = max_bits(x, __float_as_uint(dpp_move<0xB1>(__uint_as_float(x))));
+  x = max_bits(x, __float_as_uint(dpp_move<0x4E>(__uint_as_float(x))));
+  x = max_bits(x, __float_as_uint(dpp_move<0x141>(__uint_as_float(x))));
+  x = max_bits(x, __float_as_uint(dpp_move<0x140>(__uint_as_float(x))));
+  x = max_bits(x, __float_as_uint(dpp_move<0x142, 0xa>(__uint_as_float(x))));
+  x = max_bits(x, __float_as_uint(dpp_move<0x143, 0xc>(__uint_as_float(x))));
+  return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63)));
 }
 
 // long2_list = the latents with more than kSegChunk pairs that do not become hot (any order), with their chunk table: what
@@ -528,7 +534,9 @@ __global__ __launch_bounds__(kHotThreads) void hier_train_hot_kernel(
         lsum = wave_sum_lane63(lsum);
         if (lane == kWave - 1) loss_partial[(static_cast<int64_t>(col0 / kHotCols) + t) * B + b] = lsum;
         // the row's bound on its contributions: max |v| * c * sqrt(K * max over the columns of sum_k e_k^2)
-        const float acc_max = wave_max_bcast(fmaxf(acc[0], acc[1]));
+        // (lanes beyond column D hold a residual of another tile's columns)
+        const float acc_max =
+            wave_max_bcast(__uint_as_float(active ? max_bits(__float_as_uint(acc[0]), __float_as_uint(acc[1])) : 0u));
         const float v_max = __uint_as_float(scalar_words<1>(run_of(kStepRuns))[0]);
         const float bound = v_max * coef * __builtin_sqrtf(static_cast<float>(K) * acc_max);
         if (!(bound <= 3.0e38f)) {  // infinity or NaN in the inputs: the block's partial sums are made NaN

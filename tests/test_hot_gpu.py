@@ -153,6 +153,33 @@ def test_deferred_rows_and_reproducibility():
         _check_vs_oracle(cpu_args, outs[0], dv, db, loss, 1e-2)
 
 
+@pytest.mark.parametrize("value", [float("nan"), -float("nan"), float("inf")])
+@pytest.mark.parametrize("where,col", [("target", 0), ("target", 131), ("weight", 5), ("vals", None)])
+def test_inputs_that_are_not_finite(where, col, value):
+    """One NaN or infinity: what is not finite in the plain step's dW is not finite with the accumulators either, and nothing
+    outside its tile of 128 columns is (the last tile, of 8, has lanes without a column)."""
+    print("[case] hot", where, col, value, flush=True)
+    idx, W, v, b, t = make_inputs(300, 64, 2000, 264, torch.bfloat16, seed=38, zipf_s=1.1, sort_vals=True, w_std=0.3)
+    frequent = int(np.bincount(idx.numpy().ravel()).argmax())
+    if where == "target":
+        t[257, col] = value
+    elif where == "weight":
+        W[frequent, col] = value
+    else:
+        v[257, 7] = value
+    args = _dev((idx, W, v, b, t))
+    rc0, loss0, dW0, dv0, _ = abi.hier_train(*args, dw_dtype=torch.bfloat16, slice_cols=128)
+    rc, loss, dW, dv, _, ws = abi.hier_train(*args, dw_dtype=torch.bfloat16, slice_cols=128, flags=HOT, keep_workspace=True)
+    assert rc0 == 0 and rc == 0 and abi.hot_stats(*args, ws)[0] > 0
+    assert not torch.isfinite(loss) and not torch.isfinite(loss0)
+    assert torch.equal(torch.isfinite(dv), torch.isfinite(dv0))
+    bad, bad0 = ~torch.isfinite(dW), ~torch.isfinite(dW0)
+    assert bool(bad0[frequent].any()) and bool(bad[bad0].all())
+    if col is not None:
+        elsewhere = torch.arange(264, device=DEV) // 128 != col // 128
+        assert not bool(bad[:, elsewhere].any())
+
+
 def test_pair_list_and_hot_tables_reused():
     """A second call on the same workspace may keep the pair list (FLEXSAE_BWD_REUSE_PAIR_LIST: the hot
     tables are rebuilt from it) and the hot tables too (FLEXSAE_BWD_REUSE_HOT_TABLES): the same bits
