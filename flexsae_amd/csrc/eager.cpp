@@ -105,24 +105,37 @@ struct Inputs {
   Tensor indices, weight, vals, bias, target;
 };
 
-// The checks of _validate in ops.py (which says what is wrong with what fails here).
+// The checks of _validate in ops.py (which says what is wrong with what fails here).  A bias that is not defined is not asked for.
 bool usable(const Inputs &in) {
   for (const Tensor *t : {&in.indices, &in.weight, &in.vals, &in.bias, &in.target})
-    if (!plain_tensor(*t) || t->device() != in.weight.device()) return false;
-  if (in.indices.dim() != 2 || in.weight.dim() != 2 || in.vals.dim() != 2 || in.bias.dim() != 1 || in.target.dim() != 2)
-    return false;
+    if (t->defined() || t != &in.bias)
+      if (!plain_tensor(*t) || t->device() != in.weight.device() || t->dim() != (t == &in.bias ? 1 : 2)) return false;
   const int64_t B = in.indices.size(0), K = in.indices.size(1), F = in.weight.size(0), D = in.weight.size(1);
-  if (in.vals.size(0) != B || in.vals.size(1) != K || in.bias.size(0) != D || in.target.size(0) != B || in.target.size(1) != D)
+  if (in.vals.size(0) != B || in.vals.size(1) != K || (in.bias.defined() && in.bias.size(0) != D) || in.target.size(0) != B ||
+      in.target.size(1) != D)
     return false;
   if (B < 1 || K < 1 || F < 1 || D < 1 || F >= (int64_t{1} << 31) || D >= (int64_t{1} << 29) ||
       B > ((int64_t{1} << 32) - 1) / K)
     return false;
   if (in.indices.scalar_type() != c10::ScalarType::Long) return false;
   for (const Tensor *t : {&in.weight, &in.vals, &in.bias, &in.target})
-    if (dtype_of(t->scalar_type()) < 0) return false;
+    if (t->defined() && dtype_of(t->scalar_type()) < 0) return false;
   const int device = in.weight.device().index();
   return device >= 0 && device < kMaxDevices && status_flags[device].defined();
 }
+
+// What hooks have handed back for the saved tensors of a backward may be anything.
+bool usable_fp32(const Tensor &t, const Tensor &weight, at::IntArrayRef sizes) {
+  return plain_tensor(t) && t.device() == weight.device() && t.sizes() == sizes && t.scalar_type() == c10::ScalarType::Float;
+}
+
+// ... of a backward of its own: indices, weight, vals, resid
+bool usable_saved(const variable_list &saved) {
+  return usable({saved[0], saved[1], saved[2], Tensor(), saved[3]}) && saved[3].scalar_type() == c10::ScalarType::Float;
+}
+
+// ... of a step: its inputs
+bool usable_inputs(const variable_list &saved) { return usable({saved[0], saved[1], saved[2], saved[3], saved[4]}); }
 
 flexsae_shape shape_of(const Tensor &indices, const Tensor &weight, const Tensor &vals, int bias_dtype, int target_dtype) {
   return {indices.size(0), indices.size(1), weight.size(0), weight.size(1), dtype_of(weight.scalar_type()),
@@ -304,12 +317,12 @@ struct TopkLoss : torch::autograd::Function<TopkLoss> {
     const Tensor &grad = grads[0];
     if (!grad.defined()) return variable_list(5);
     const int64_t bias_type = ctx->saved_data["bias"].toInt(), target_type = ctx->saved_data["target"].toInt();
-    if (!plain_backward(grad) || lists_in_python)
+    if (!plain_backward(grad) || lists_in_python || !usable_saved(saved))
       return backward_in_python(ctx, kTopk, grad, saved,
                                 {dtype_of(static_cast<c10::ScalarType>(bias_type)),
                                  dtype_of(static_cast<c10::ScalarType>(target_type))},
                                 nullptr, 5);
-    const Tensor indices = prepared(saved[0]), weight = prepared(saved[1]), vals = prepared(saved[2]), resid = saved[3];
+    const Tensor indices = prepared(saved[0]), weight = prepared(saved[1]), vals = prepared(saved[2]), resid = prepared(saved[3]);
     const c10::DeviceGuard guard(weight.device());
     const Tensor g = grad_scalar(grad, weight.device());
     const flexsae_shape s = shape_of(indices, weight, vals, FLEXSAE_F32, FLEXSAE_F32);
@@ -349,9 +362,9 @@ struct HierLoss : torch::autograd::Function<HierLoss> {
     const Tensor &grad = grads[0];
     if (!grad.defined()) return variable_list(6);
     const auto leaf_bias = static_cast<c10::ScalarType>(ctx->saved_data["bias"].toInt());
-    if (!plain_backward(grad) || lists_in_python)
+    if (!plain_backward(grad) || lists_in_python || !usable_saved(saved))
       return backward_in_python(ctx, kHier, grad, saved, {dtype_of(leaf_bias)}, nullptr, 6);
-    const Tensor indices = prepared(saved[0]), weight = prepared(saved[1]), vals = prepared(saved[2]), resid = saved[3];
+    const Tensor indices = prepared(saved[0]), weight = prepared(saved[1]), vals = prepared(saved[2]), resid = prepared(saved[3]);
     const c10::DeviceGuard guard(weight.device());
     const Tensor g = grad_scalar(grad, weight.device());
     const flexsae_shape s = shape_of(indices, weight, vals, FLEXSAE_F32, FLEXSAE_F32);
@@ -388,13 +401,15 @@ struct SlicedLoss : torch::autograd::Function<SlicedLoss> {
     const auto at = ctx->saved_data.find("dW");
     Tensor dW = at != ctx->saved_data.end() ? at->second.toTensor() : Tensor();
     const StepPlan plan = saved_plan(ctx);
-    if (!plain_backward(grad) || (lists_in_python && !dW.defined())) {
+    if (!plain_backward(grad) || (lists_in_python && !dW.defined()) || !usable_inputs(saved) ||
+        !usable_fp32(saved[5], saved[1], saved[2].sizes()) || !usable_fp32(saved[6], saved[1], saved[3].sizes()) ||
+        (dW.defined() && dW.device() != saved[1].device())) {
       auto out = backward_in_python(ctx, kSliced, grad, saved, {plan.need_dw, plan.flags}, &dW, 6);
       if (dW.defined()) ctx->saved_data["dW"] = dW;
       else ctx->saved_data.erase("dW");
       return out;
     }
-    Tensor dvals = saved[5], dbias = saved[6];
+    Tensor dvals = prepared(saved[5]), dbias = prepared(saved[6]);
     if (ctx->needs_input_grad(1)) {
       TORCH_CHECK(plan.need_dw, "the step ran without dW but weight requires a gradient");
       ctx->saved_data.erase("dW");  // the buffer now belongs to whoever receives the gradient
@@ -431,7 +446,7 @@ struct LateLoss : torch::autograd::Function<LateLoss> {
     const Tensor &grad = grads[0];
     if (!grad.defined()) return variable_list(6);
     StepPlan plan = saved_plan(ctx);
-    if (!plain_backward(grad) || lists_in_python)
+    if (!plain_backward(grad) || lists_in_python || !usable_inputs(saved))
       return backward_in_python(ctx, kLate, grad, saved, {plan.need_dw, plan.flags}, nullptr, 6);
     const auto at = ctx->saved_data.find("stats");
     if (at != ctx->saved_data.end()) {

@@ -110,6 +110,13 @@ def _validate(indices: Tensor, weight: Tensor, vals: Tensor, bias: Tensor, targe
     return B, K, F, D
 
 
+def _validate_saved(indices: Tensor, weight: Tensor, vals: Tensor, resid: Tensor):
+    """The same of a backward: saved tensors are whatever a hook (``torch.autograd.graph.saved_tensors_hooks``) hands back."""
+    if resid.dim() != 2 or resid.dtype != torch.float32:
+        raise ValueError(f"expected resid[B,D] in float32, got {resid.dtype} of {tuple(resid.shape)}")
+    return _validate(indices, weight, vals, resid[0] if resid.shape[0] else resid.new_empty(weight.shape[-1:]), resid)
+
+
 def _shape(B, K, F, D, weight: Tensor, vals: Tensor, bias_dtype, target_dtype) -> _lib.Shape:
     return _lib.Shape(B, K, F, D, _DTYPES[weight.dtype], _DTYPES[vals.dtype], _DTYPES[bias_dtype],
                       _DTYPES[target_dtype])
@@ -539,8 +546,7 @@ def _pair_export(lib, shape, workspace: Tensor, indices: Tensor, F: int) -> None
 def _hier_bwd_impl(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Tensor,
                    resid: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
     lib = _lib.load()
-    B, K = indices.shape
-    F, D = weight.shape
+    B, K, F, D = _validate_saved(indices, weight, vals, resid)
     dev = weight.device
     indices, weight, vals, resid = (_prep(t) for t in (indices, weight, vals, resid))
     with _on_device(dev):
@@ -605,8 +611,7 @@ def _topk_bwd_typed(grad_out: Tensor, indices: Tensor, weight: Tensor, vals: Ten
                     dbias_dtype) -> Tuple[Tensor, Tensor, Tensor]:
     """(dW, dvals, dbias), dvals and dbias in the types asked for."""
     lib = _lib.load()
-    B, K = indices.shape
-    F, D = weight.shape
+    B, K, F, D = _validate_saved(indices, weight, vals, resid)
     dev = weight.device
     indices, weight, vals, resid = (_prep(t) for t in (indices, weight, vals, resid))
     with _on_device(dev):
@@ -1232,10 +1237,10 @@ def _plain_call(*tensors: Tensor) -> bool:
             and torch.autograd.forward_ad._current_level < 0)
 
 
-def _plain_backward(grad_loss: Tensor) -> bool:
-    """The same of a backward, whose surroundings and gradient need not be those of its forward; the ops build a graph of
-    the backward."""
-    return not torch.is_grad_enabled() and _plain_call(grad_loss)
+def _plain_backward(grad_loss: Tensor, *saved: Tensor) -> bool:
+    """The same of a backward, whose surroundings and gradient need not be those of its forward, nor its saved tensors, where
+    hooks hand them back; the ops build a graph of the backward."""
+    return not torch.is_grad_enabled() and _plain_call(grad_loss, *saved)
 
 
 def _finish_grads(grad_out, weight: Tensor, dW_unit, dvals: Tensor, vals_dtype, dbias: Tensor, bias_dtype):
@@ -1243,6 +1248,12 @@ def _finish_grads(grad_out, weight: Tensor, dW_unit, dvals: Tensor, vals_dtype, 
     (None: one), and ``dW_unit`` (None: no weight gradient) times it, in place where it has the weight's type."""
     lib = _lib.load()
     dev = weight.device
+    for t in (dvals, dbias) if dW_unit is None else (dvals, dbias, dW_unit):  # (saved tensors: see _validate_saved)
+        if t.device != dev or not t.is_cuda:
+            raise RuntimeError(f"a saved tensor is on {t.device}, weight on {dev}")
+    if dvals.dtype != torch.float32 or dbias.dtype != torch.float32:
+        raise ValueError(f"expected float32 gradients of vals and bias, got {dvals.dtype} and {dbias.dtype}")
+    dvals, dbias = _prep(dvals), _prep(dbias)
     with _on_device(dev):
         g = None if grad_out is None else _grad_scalar(grad_out, dev)
         dW = None
@@ -1352,7 +1363,7 @@ class _HierLateStep(torch.autograd.Function):
         if grad_loss is None:
             return None, None, None, None, None, None, None
         indices, weight, vals, bias, target = ctx.saved_tensors
-        if not _plain_backward(grad_loss):
+        if not _plain_backward(grad_loss, indices, weight, vals, bias, target):
             with torch.no_grad():
                 _, dvals, dbias, dW = hier_train_sliced(indices, weight, vals, bias, target, True, ctx.hot, ctx.dense)
             g = grad_loss.to(torch.float32)
@@ -1376,7 +1387,7 @@ _TYPES = {code: dtype for dtype, code in _DTYPES.items()}
 def _general_backward(kind, grad, saved, needs, numbers, dw_unit):
     """The backwards of eager.cpp that are not plain, or that a shared pair list may serve: (gradients, unit gradient left)."""
     ctx = _Saved(saved, needs)
-    plain = _plain_backward(grad)
+    plain = _plain_backward(grad, *saved)
     if kind == 0:
         ctx.leaf_dtypes = (saved[2].dtype, _TYPES[numbers[0]], _TYPES[numbers[1]])
         return _topk_backward(ctx, grad, None, plain), None

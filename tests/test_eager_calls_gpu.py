@@ -126,6 +126,42 @@ def test_the_surroundings_of_the_backward_count(loss, fused, dtype, size, late, 
         flex.set_fused_training(True)
 
 
+def _transposed(x):  # the same values in another order in memory
+    return x.t().contiguous().t() if x.dim() == 2 else x.repeat_interleave(2)[::2]
+
+
+def _odd(x):  # ... behind one element of another buffer
+    return x.new_empty(x.numel() + 1)[1:].view_as(x).copy_(x)
+
+
+@pytest.mark.parametrize("loss,fused,dtype,late", [
+    ("topk", True, torch.float32, False), ("topk", True, torch.bfloat16, False), ("hier", False, torch.bfloat16, False),
+    ("hier", True, torch.bfloat16, False), ("hier", True, torch.float16, True)])
+@pytest.mark.parametrize("lists", [False, True])
+def test_saved_tensors_are_what_hooks_hand_back(loss, fused, dtype, late, lists, monkeypatch):
+    """Of another layout or alignment: the same gradients.  On the host, or of another shape: refused before any launch."""
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, dtype, seed=7))
+    monkeypatch.setattr(ops, "_late_step", lambda *_: late)
+    flex.set_fused_training(fused)
+
+    def grads(unpack):
+        leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: x, unpack):
+            out = LOSS[loss](idx, *leaves, t)
+        with flex.shared_pair_list() if lists else contextlib.nullcontext():
+            return torch.autograd.grad(out * 2.0, leaves)
+
+    try:
+        want = grads(lambda x: x)
+        for other in (_transposed, _odd):
+            assert all(torch.equal(x, y) for x, y in zip(grads(other), want))
+        for other in (lambda x: x.cpu(), lambda x: x[:, :-1] if x.dim() == 2 and x.is_floating_point() else x):
+            with pytest.raises((RuntimeError, ValueError)):
+                grads(other)
+    finally:
+        flex.set_fused_training(True)
+
+
 def test_the_fused_update_marks_the_weight():
     idx, W, v, b, t = (x.to(DEV) for x in make_inputs(16, 8, 60, 128, seed=4))
     W2 = W.clone()

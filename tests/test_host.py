@@ -46,6 +46,19 @@ def test_validation_errors():
         ops._validate(idx.flatten(), W, v, b, t)
 
 
+@pytest.mark.parametrize("fn", [ops._topk_bwd_impl, ops._hier_bwd_impl])
+def test_a_backward_refuses_saved_tensors_that_do_not_fit(fn, monkeypatch):
+    """... before it asks for anything on the device."""
+    monkeypatch.setattr(ops._lib, "load", lambda: None)
+    idx, W, v, b, t = make_inputs(4, 8, 16, 64)
+    for saved in ((idx, W, v, t), (idx, W, v[:, :7], t), (idx, W[:, :63], v, t), (idx, W, v, t.half()), (idx, W, v, t[0]),
+                  (idx[:0], W, v[:0], t[:0])):
+        with pytest.raises((RuntimeError, ValueError), match="AMD GPU only|shape mismatch|expected resid|empty"):
+            fn(torch.ones(()), *saved)
+    with pytest.raises(RuntimeError, match="a saved tensor is on cpu"):
+        ops._finish_grads(None, W, None, v, v.dtype, b, b.dtype)
+
+
 @pytest.mark.parametrize("mode,fn", [(oracle.TOPK, flex.topk_sae_loss), (oracle.HIER, flex.hierarchical_sae_loss)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_eager_definitions_agree_with_oracle(mode, fn, dtype):
