@@ -17,6 +17,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -166,6 +167,10 @@ Tensor make_workspace(const Tensor &like, size_t bytes) {
 
 int *flag_of(const Tensor &t) { return status_flags[t.device().index()].data_ptr<int>(); }
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+bool capturing(const Tensor &t) {
+  const c10::DeviceGuard guard(t.device());
+  return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
 const int64_t *index_ptr(const Tensor &t) { return t.const_data_ptr<int64_t>(); }
 float *f32(const Tensor &t) { return t.data_ptr<float>(); }
 
@@ -449,7 +454,8 @@ struct LateLoss : torch::autograd::Function<LateLoss> {
     if (!plain_backward(grad) || lists_in_python || !usable_inputs(saved))
       return backward_in_python(ctx, kLate, grad, saved, {plan.need_dw, plan.flags}, nullptr, 6);
     const auto at = ctx->saved_data.find("stats");
-    if (at != ctx->saved_data.end()) {
+    // (a graph under capture would write them again at every replay, as those of the forward's step)
+    if (at != ctx->saved_data.end() && !capturing(saved[1])) {
       plan.stats = at->second.toTensor();
       plan.tag = ctx->saved_data["tag"].toInt();
       ctx->saved_data.erase("stats");

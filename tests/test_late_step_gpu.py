@@ -88,3 +88,34 @@ def test_which_shapes_take_it():
     assert late(torch.float16, 4096, 32, 65536, 2304) and late(torch.float16, 4096, 64, 65536, 1536)
     assert not late(torch.float16, 4097, 64, 65536, 1536) and not late(torch.float16, 64, 32, 65536, 1535)
     assert not late(torch.bfloat16, 4096, 32, 65536, 2304) and not late(torch.float32, 4096, 32, 65536, 2304)
+
+
+def test_a_captured_backward_leaves_no_measurement(monkeypatch):
+    """The forward runs before the capture, the step inside it: no replay writes what the pair list says about its indices, which
+    would pass for that of a later step."""
+    monkeypatch.setattr(ops, "_late_step", lambda *_: True)
+    B, K, F, D = 40, 16, 411, 256
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(B, K, F, D, torch.float16, seed=6))
+    up = torch.tensor(2.0, device=DEV)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    leaves = [x.clone().requires_grad_() for x in (W, v, b)]
+    with torch.cuda.stream(stream):
+        want = torch.autograd.grad(flex.triton_hierarchical_sae_loss(idx, *leaves, t), leaves, up)
+        torch.cuda.synchronize()
+        st = ops._hot_auto[ops._hot_key(DEV, B, K, F, D, torch.float16)]
+        assert st["words"][3] == st["asked"]
+        loss = flex.triton_hierarchical_sae_loss(idx, *leaves, t)
+        torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = torch.autograd.grad(loss, leaves, up)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
+        assert st["words"][3] == st["asked"] - 1
+        st["pinned"][3] = 0  # (eager work between the replays)
+        torch.zeros(8, device=DEV).add_(1)
+        torch.cuda.synchronize()
+        st["pinned"][3] = st["asked"] - 1
