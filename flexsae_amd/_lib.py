@@ -138,15 +138,21 @@ _eager = None
 
 def eager(general_backward):
     """The extension module of ordinary eager calls, bound to the library once; ``general_backward`` takes the backwards that
-    are not plain."""
+    are not plain.  Absent, or built from other sources than the library or against another torch: FlexSAELibraryError."""
     global _eager
     if _eager is None:
+        import torch
+
         load()
         try:
             from . import _eager as module
         except ImportError as exc:
             raise FlexSAELibraryError(f"cannot load flexsae_amd/_eager.so ({exc}): build it with "
                                       "`python -m flexsae_amd.build` against this torch") from exc
+        have = (getattr(module, "build_id", None), getattr(module, "torch_version", None))
+        if have != (build_id(), torch.__version__):
+            raise FlexSAELibraryError(f"flexsae_amd/_eager.so is of build {have[0]} for torch {have[1]}, the library of build "
+                                      f"{build_id()}, torch is {torch.__version__}: rebuild with `python -m flexsae_amd.build`")
         module.init(LIB_PATH, general_backward, check)
         _eager = module
     return _eager

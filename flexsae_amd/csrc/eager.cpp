@@ -626,4 +626,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_eager", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__eager() { return PyModule_Create(&module); }
+// build_id, torch_version: what the module was built from and against, for whoever loads it to compare
+PyMODINIT_FUNC PyInit__eager() {
+  PyObject *const m = PyModule_Create(&module);
+  if (m && (PyModule_AddStringConstant(m, "build_id", FLEXSAE_BUILD_ID) < 0 ||
+            PyModule_AddStringConstant(m, "torch_version", FLEXSAE_TORCH_VERSION) < 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -3,6 +3,7 @@ eager torch definitions, and that nothing in the package touches the oracle."""
 import ctypes
 import os
 import re
+import shutil
 import weakref
 
 import pytest
@@ -10,7 +11,7 @@ import torch
 
 import flexsae_amd as flex
 import oracle
-from flexsae_amd import ops
+from flexsae_amd import _lib, build, ops
 from helpers import make_inputs
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -82,6 +83,43 @@ def test_fake_kernels_give_shapes_and_dtypes(name):
     assert dW.shape == (100, 256) and dW.dtype == torch.bfloat16
     assert dv.shape == (32, 8) and dv.dtype == torch.float32
     assert db.shape == (256,) and db.dtype == torch.float32
+
+
+def test_the_build_id_covers_the_extension_module(tmp_path, monkeypatch):
+    for f in os.listdir(build.CSRC):
+        shutil.copy(os.path.join(build.CSRC, f), tmp_path)
+    here = build.source_id()
+    monkeypatch.setattr(build, "CSRC", str(tmp_path))
+    assert build.source_id() == here
+    with open(tmp_path / "eager.cpp", "a") as fh:
+        fh.write("// another source\n")
+    changed = build.source_id()
+    monkeypatch.setattr(build, "EAGER_FLAGS", [*build.EAGER_FLAGS, "-DX"])
+    assert len({here, changed, build.source_id()}) == 3
+
+
+@pytest.mark.parametrize("build_id,torch_version,fits", [
+    ("this", torch.__version__, True), ("another", torch.__version__, False), ("this", "1.0", False), (None, None, False)])
+def test_a_stale_extension_module_is_refused(build_id, torch_version, fits, monkeypatch):
+    class Module:
+        bound = False
+
+        def init(self, *args):
+            self.bound = True
+
+    module = Module()
+    if build_id is not None:
+        module.build_id, module.torch_version = build_id, torch_version
+    monkeypatch.setattr(flex, "_eager", module, raising=False)
+    monkeypatch.setattr(_lib, "_eager", None)
+    monkeypatch.setattr(_lib, "load", lambda: None)
+    monkeypatch.setattr(_lib, "build_id", lambda: "this")
+    if fits:
+        assert _lib.eager(None) is module and module.bound
+    else:
+        with pytest.raises(_lib.FlexSAELibraryError, match="rebuild"):
+            _lib.eager(None)
+        assert not module.bound
 
 
 def test_package_never_imports_the_oracle():
