@@ -285,6 +285,95 @@ def test_what_the_extension_module_takes(entry):
     assert seen == [None]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("entry", ["hier_sliced", "hier_late", "hier_sgd"])
+def test_what_the_steps_of_the_extension_module_take(entry, dtype):
+    """The step leaves its measurement, tagged, in pinned memory; a call that it does not take leaves the words and the weight."""
+    print("[case]", entry, dtype, flush=True)
+    B, K, F, D = 100, 8, 900, 128
+    idx, W, v, b, t = make_inputs(B, K, F, D, dtype, seed=8)
+    idx[:, 0] = 3  # a latent with more than 64 pairs
+    counts = torch.bincount(idx.flatten(), minlength=F)
+    long = counts[counts > 64]
+    want = [long.numel(), int(((long + 63) // 64).sum()), int((counts == 0).sum()), 77]
+    idx, W, v, b, t = (x.to(DEV) for x in (idx, W, v, b, t))
+    LOSS["topk"](idx, W, v, b, t)
+    fn = getattr(ops._native(W), entry)
+    words = torch.full((4,), -5, dtype=torch.int32, pin_memory=True)
+    first = torch.full((), 0.5, device=DEV) if entry == "hier_sgd" else True
+    more = (first, 128, 0, 0, words, 77)
+
+    def taken(args):
+        words.fill_(-5)
+        got = fn(*args, *more)
+        if got is not None and entry == "hier_late":
+            torch.cuda.synchronize()
+            assert words.tolist() == [-5] * 4  # (the step comes with the backward)
+            torch.autograd.grad(got, args[1])
+        torch.cuda.synchronize()
+        assert words.tolist() == ([-5] * 4 if got is None else want)
+        return got is not None
+
+    def fresh(x=W):
+        return x.clone().requires_grad_(entry != "hier_sgd")
+
+    old = fresh()
+    assert taken((idx, old, v, b, t))
+    changed = not torch.equal(old.detach(), W)
+    assert changed == (entry == "hier_sgd")
+
+    class Sub(torch.Tensor):
+        pass
+
+    weight = fresh()
+    refused = [(idx, W.as_subclass(Sub), v, b, t), (idx, weight, v, b, t.cpu()), (idx.int(), weight, v, b, t),
+               (idx, weight.double(), v, b, t), (idx, weight, v[:, :4], b, t), (idx, weight, v, b[:64], t),
+               (idx[:0], weight, v[:0], b, t[:0]), (idx, torch._neg_view(W), v, b, t)]
+    strided = W.repeat_interleave(2, -1)[..., ::2]
+    odd = W.new_empty(W.numel() + 1)[1:].view_as(W).copy_(W)
+    narrow = (idx, W[:, :126].contiguous(), v, b[:126], t[:, :126])
+    deep = (idx.repeat(1, 33), W, v.repeat(1, 33), b, t)  # 264 steps
+    if entry == "hier_sgd":  # in place: whole rows on whole vectors
+        refused += [(idx, strided, v, b, t), (idx, odd, v, b, t), narrow, deep]
+    else:
+        for w in (strided, odd):
+            assert taken((idx, w.detach().requires_grad_(), v, b, t))
+    for args in refused:
+        assert not taken(args)
+    with _Seen():
+        assert not taken((idx, weight, v, b, t))
+    assert torch.equal(weight.detach(), W) and weight._version == 0
+    with pytest.raises(TypeError):
+        fn(idx, W, v, b, t)
+
+
+@pytest.mark.parametrize("sgd", [False, True])
+def test_a_call_that_the_module_left_to_the_ops_does_not_end_the_measurement(sgd):
+    B, K, F, D = 24, 8, 613, 132
+    idx, W, v, b, t = (x.to(DEV) for x in make_inputs(B, K, F, D, seed=9))
+
+    def step():
+        w = W.clone().requires_grad_(not sgd)
+        if sgd:
+            flex.hierarchical_sae_sgd_step(idx, w, v, b, t, 0.5)
+        else:
+            flex.triton_hierarchical_sae_loss(idx, w, v, b, t).backward()
+        torch.cuda.synchronize()
+
+    key = ops._hot_key(DEV, B, K, F, D, torch.float32)
+    for _ in range(2):
+        with _Seen():
+            step()
+        step()
+        st = ops._hot_auto[key]
+        assert st["words"][3] == st["asked"] != 0
+        st["words"][2] = F  # (as if no latent had a pair)
+        with _Seen():
+            step()
+        step()
+        assert st["words"][3] == st["asked"] and st["words"][2] == F - idx.unique().numel()
+
+
 @pytest.mark.parametrize("loss", ["topk", "hier"])
 def test_other_threads_and_streams(loss):
     """Forward and backward on a stream and a thread of their own, several at once: each the same bits."""
