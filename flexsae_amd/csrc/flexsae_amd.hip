@@ -471,8 +471,9 @@ CsrPlan plan_csr(int64_t n_pairs, int64_t F) {
          (shift < 11 || ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketBlocks))
     ++shift;
   while (shift < kSortMaxShift && ceil_div(F, static_cast<int64_t>(1) << shift) > kBucketMaxBuckets) ++shift;
-  // Half as many where every compute unit still has at most one block (with the batches below): a block with fewer pairs is done
-  // sooner, one with frequent latents above all.  us of the pair list, uniform and skewed (distinct in a row), before / with this:
+  // Half as many where every compute unit still has at most one block (kBucketBlocks is two for each; with the batches below): a
+  // block with fewer pairs is done sooner, one with frequent latents above all, which is what the rule is for: uniform indices gain
+  // less or, once, lose 1 %.  us of the pair list, uniform and skewed (distinct in a row), before / with this:
   // B=1024, K=64, F=32768 18.1 / 17.1, 27.6 / 25.6; B=4096, K=64, F=65536 22.5 / 22.8, 33.8 / 31.5; B=404, K=50, F=12953 16.9 /
   // 15.9, 23.8 / 21.3; not with more blocks than that: B=2435, K=128, F=24332 in 381 buckets 23.1 / 24.5, 31.3 / 36.2, B=2048,
   // K=64, F=262144 in 256 of two batches 21.4 / 24.5; nor a quarter, whose chunks take longer to order (B=1777, K=50, F=24571,

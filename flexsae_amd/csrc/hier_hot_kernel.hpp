@@ -307,9 +307,10 @@ __global__ __launch_bounds__(256) void hot_block_finalize_kernel(HotBlockFinaliz
 }
 
 // ---- what the walk reads of a row ------------------------------------------------------------
-// Per batch row four runs of KMAX words, read by the walk's scalar unit (a lane read is a vector instruction, which is what
-// binds it most: B=8192, K=64, F=262144, D=4096 bf16 Zipf 170.5 -> 162.3 us a launch, 6.7 us once for the words): where the step's weight row begins, where its contribution goes, its val as fp32 bits; steps from K on are
-// zero, and the last run begins with the row's largest |val|.  A pair whose index is out of range gets row 0 and a val of 0.
+// Per batch row three runs of KMAX words and sixteen more, read by the walk's scalar unit (a lane read is a vector instruction,
+// which is what binds it most: B=8192, K=64, F=262144, D=4096 bf16 Zipf 170.5 -> 162.3 us a launch when it was made, 6.7 us once
+// for the words): where the step's weight row begins, where its contribution goes, its val as fp32 bits; steps from K on are zero,
+// and the sixteen begin with the row's largest |val|.  A pair whose index is out of range gets row 0 and a val of 0.
 // OFF32 (see the walk): byte offsets of the weight row and of the contribution row (multiples of 256), for a hot pair
 // kHotSlotBit and the byte offset of its accumulator row, for a latent's only pair that goes to dW the offset of the weight
 // row >> 7 (even) plus one.  Else row, slot, kHotSlotBit with the accumulator, kSoloSlotBit.
@@ -373,7 +374,8 @@ __device__ __forceinline__ vec_t<uint32_t, N> scalar_words(const uint32_t *p) {
 // steps (fin, hfin); the last is the flush of its accumulators to
 // hot_partial[tile][row block][accumulator row][2][64].
 // What it reads of a row's steps comes through the scalar unit (hot_steps_kernel); with lane reads instead, four a step, a
-// launch of B=8192, K=64, F=262144, D=4096 bf16 Zipf takes 170.5 us, without 162.3, and 158.3 with the turns below.  What
+// launch of B=8192, K=64, F=262144, D=4096 bf16 Zipf took 170.5 us, without 162.3, and 158.3 with the turns below (one run
+// on one box; boxes differ: 154 in a trace on another).  What
 // binds it then is what its rounds of rows do one after the other: gathers, 25 vector instructions a step, and stores that
 // the next row's loads are counted behind.
 // OFF32: the weight matrix is smaller than 4 GiB, the slice of contributions smaller than 2 GiB

@@ -243,7 +243,8 @@ def _train_tile_cols(K: int, weight_dtype) -> int:
 def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype, step: bool = True) -> int:
     """Bytes the contributions of one slice may take.  Unless set explicitly: 0.45 of the weight
     matrix, at most 256 MiB -- memory above the inputs then stays within about 1.25 of the TopK
-    loss's (whose peak is the dense gradient plus the residual) whatever K is, at 4-5 % of the step
+    loss's (whose peak is the dense gradient plus the residual) whatever K is, for K <= 256, bf16 or fp32 and weights of
+    285 MiB and more (smaller ones: below), at 4-5 % of the step
     time where that is less than the 256 MiB that measured fastest (B = 4096, F = 65536, D = 2304,
     bf16: K = 32 0.483 instead of 0.463 ms, K = 64 0.751 instead of 0.717 ms; K = 128 unchanged) --
     and at least 128 MiB: weights small enough to give less have batches whose slices, launch by
@@ -253,7 +254,9 @@ def _hier_scratch_budget(B: int, K: int, F: int, D: int, weight_dtype, step: boo
     D = 2048 fp32 679, 364, 350).  With such weights all contributions at once where they take at most 384 MiB (us with
     128 MiB / all: B = 1500, K = 40, F = 24571, D = 2328 bf16 208 / 189, fp32 D = 1160 206 / 183, fp16 205 / 192; B = 512,
     K = 64, F = 16384, D = 5488 bf16 248 / 219; B = 400, K = 100, F = 60000, D = 1872 166 / 144; over 64 shapes 4 % less on
-    average, one more than 4 % more: B = 1900, K = 128, F = 8192, D = 152 fp32 124 / 131); ``step`` false, forward and sweep, not
+    average, one more than 4 % more: B = 1900, K = 128, F = 8192, D = 152 fp32 124 / 131; MiB above the inputs, this step and TopK's:
+    B = 1777, K = 50, F = 24571, D = 1538 bf16 389 and 112, B = 512, K = 64, F = 16384, D = 5488 555 and 212;
+    ``set_hier_scratch_bytes`` bounds it); ``step`` false, forward and sweep, not
     (B = 512, K = 150, F = 30000, Zipf, D = 2304 bf16 278 / 293, D = 1024 fp32 218 / 235)."""
     if _hier_scratch_bytes is not None:
         return _hier_scratch_bytes
@@ -278,7 +281,7 @@ def _hier_slice_cols(B: int, K: int, F: int, D: int, weight_dtype, step: bool = 
 
 
 def set_hier_scratch_bytes(nbytes) -> None:
-    """Upper bound on the scratch of the hierarchical backward (bytes): the per-pair contributions
+    """Upper bound on the scratch of the hierarchical step and backward (bytes): the per-pair contributions
     of one slice of columns.  0 = use the atomic scatter fallback, which needs no scratch but an
     fp32 [F,D] accumulator.  ``None`` (the default) sizes it from the problem: 0.45 of the weight
     matrix, at least 128 and at most 256 MiB, or, of weights for which that is 128 MiB, all contributions up to 384 MiB.  A slice is never narrower than ``set_hier_min_slice_cols``, so with
@@ -1209,7 +1212,8 @@ topk_fwd.register_autograd(_topk_backward, setup_context=_setup_context)
 # ---- ordinary eager calls ------------------------------------------------------------------
 # A call on plain tensors with no tracer, mode or transform around it does without the dispatcher and, but for what is decided
 # here, without Python: csrc/eager.cpp checks, allocates, launches and has the autograd nodes, which save the tensors that the
-# ops save.  Calls that share a pair list or check their indices run the ops' functions under an autograd.Function.  Everything else goes through the ops, which tracers, modes and transforms see.
+# ops save.  Calls that share a pair list or check their indices run the ops' functions under an autograd.Function.  Everything
+# else goes through the ops, which tracers, modes and transforms see.
 # us a step with the functions under an autograd.Function and with eager.cpp: B = 64, K = 32, F = 4096, D = 256 fp32 TopK 160
 # and 79, hierarchical 195 and 99 (through the ops 40 to 45 more; the least that torch's engine takes for a forward and a
 # backward of any kind is 45); the host's share of an SGD step 62 and 35.

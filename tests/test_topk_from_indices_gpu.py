@@ -63,8 +63,8 @@ def test_same_values(B, K, F, D, kind, dtype, leaf_dtypes, flags):
         assert torch.equal(a, b)
 
 
-def test_more_latents_than_buckets_take():
-    F = (1 << 25) + 1
+@pytest.mark.parametrize("F", [1 << 25, (1 << 25) + 1])  # 8192 buckets of 4096 latents, and one latent more
+def test_more_latents_than_buckets_take(F):
     idx = torch.tensor([[0, F - 1, 5], [F - 1, 7, F]], device=DEV)
     W = torch.ones(F, 1, device=DEV)
     v = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
