@@ -163,7 +163,8 @@ def test_a_step_that_was_not_taken_leaves_the_measurement_alive(late, monkeypatc
 
     def new_stats(key):
         st = ops._hot_auto[key] = {"hot": False, "dense": False, "pinned": words, "event": None, "spare": None,
-                                   "words": (ctypes.c_uint32 * 4).from_address(words.data_ptr()), "seen": 0, "asked": 0}
+                                   "words": (ctypes.c_uint32 * 4).from_address(words.data_ptr()), "seen": 0, "asked": 0,
+                                   "pending": False}
         return st
 
     monkeypatch.setattr(ops, "_new_stats", new_stats)
@@ -196,5 +197,15 @@ def test_a_step_that_was_not_taken_leaves_the_measurement_alive(late, monkeypatc
     ops._native_hier(Module(), *args)
     assert len({tag for _, tag in asked}) == 3 and 0 not in {tag for _, tag in asked}
     assert all(pinned is words for pinned, _ in asked)
-    words[:] = torch.tensor([0, 0, 100, asked[-1][1]], dtype=torch.int32)  # (few latents without a pair)
+    # the third was taken: the next is asked only if that one may never answer
+    ops._native_hier(Module(), *args)
+    assert asked[3] == ((words, 4) if late else (None, 0))
+    words[:] = torch.tensor([0, 0, 100, asked[2][1]], dtype=torch.int32)  # (few latents without a pair)
     assert ops._index_stats(route.key, B, K, F)["dense"] is True
+    ops._native_hier(Module(), *args)  # answered: asked again
+    assert asked[4][0] is words and asked[4][1] not in {tag for _, tag in asked[:4]}
+    # a shape that is forgotten while its step is refused
+    Module.hier_sliced = Module.hier_late = lambda *_: ops._forget_stats()
+    words[3] = asked[4][1]
+    assert ops._native_hier(Module(), *args) is None and not ops._hot_auto
+    ops._hot_retired.pop()
